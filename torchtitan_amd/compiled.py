@@ -64,7 +64,7 @@ def mx_linear_fwd(x: torch.Tensor, weight: torch.Tensor, mode: int, need_dx: boo
         xq0, xq1 = ops.to_mx_dim0_dim1(x2, name, MX_SCALES_MFMA)
     else:
         xq0, xq1 = ops.to_mx_dim0(x2, name, MX_SCALES_MFMA), None
-    wq0, wq1 = _cast_weight(weight, name, need_dx, _block_cfg(mode, cache_w))
+    wq0, wq1 = _cast_weight(weight, name, need_dx, _block_cfg(mode, cache_w), whole_blocks=False)
     y = ops.mx_gemm_nt(xq0, wq0).view(*x.shape[:-1], N)
     if cache_w and wq1 is not None:  # an operator's outputs are its own: not the cache's tensors
         wq1 = MXData(wq1.codes.clone(), wq1.scales.clone(), MX_SCALES_MFMA)

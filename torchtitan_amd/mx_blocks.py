@@ -11,9 +11,8 @@ import torch
 import torch.nn.functional as F
 
 from . import ops
-from .mx_tensor import (MXFP8Config, MXFP8TrainingWeight, _cast_activation, _cast_cache, _cast_cols_padded,
-                        _cast_into_groups, _cast_rows_padded, _cast_weight, _grouped_2d3d_padded,
-                        _pad_plan, _unwrap)
+from .mx_tensor import (MXFP8Config, MXFP8TrainingWeight, _cast_activation, _cast_cache, _cast_into_groups,
+                        _cast_weight, _grouped_2d3d_padded, _pad_plan, _unwrap)
 from .ops import MX_SCALES_MFMA, MX_SCALES_ROWMAJOR, MXData
 
 # ----------------------------------------------------------------------------- SwiGLU + linear
@@ -27,18 +26,16 @@ class _MXSwiGLULinear(torch.autograd.Function):
     def forward(ctx, h1, h3, weight, cfg: MXFP8Config):
         mode = cfg.scale_mode
         H, N = h1.shape[-1], weight.shape[0]
-        a, b = h1.reshape(-1, H), h3.reshape(-1, H)
-        w = weight if weight.dtype == torch.bfloat16 else weight.to(torch.bfloat16)
-        gq0, gq1, _ = ops.swiglu_to_mx_dim0_dim1(a, b, mode, MX_SCALES_MFMA)
-        need_dh = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
+        need_dh, need_dw = ctx.needs_input_grad[0] or ctx.needs_input_grad[1], ctx.needs_input_grad[2]
+        gq0, gq1 = ops.swiglu_to_operands(h1.reshape(-1, H), h3.reshape(-1, H), mode, need_dw)
         wq0, wq1 = _cast_weight(weight, mode, need_dh, cfg)
         y = ops.mx_gemm_nt(gq0, wq0)
-        ctx.cfg, ctx.w_dtype, ctx.have_wq1 = cfg, weight.dtype, wq1 is not None
+        ctx.cfg, ctx.w_dtype = cfg, weight.dtype
         saved = [h1, h3]
-        if ctx.needs_input_grad[2]:
+        if need_dw:
             saved += [gq1.codes, gq1.scales]
         if need_dh:
-            saved += [wq1.codes, wq1.scales] if wq1 is not None else [w]
+            saved += [wq1.codes, wq1.scales]
         ctx.save_for_backward(*saved)
         return y.view(*h1.shape[:-1], N)
 
@@ -47,42 +44,26 @@ class _MXSwiGLULinear(torch.autograd.Function):
         mode = ctx.cfg.scale_mode
         need_dh = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
         need_dw = ctx.needs_input_grad[2]
-        saved = list(ctx.saved_tensors)
-        h1, h3 = saved.pop(0), saved.pop(0)
-        N = dy.shape[-1]
-        dy2 = dy.reshape(-1, N)
-        if dy2.dtype != torch.bfloat16:
-            dy2 = dy2.to(torch.bfloat16)
-        dy2 = dy2.contiguous()
-        gq1 = MXData(saved.pop(0), saved.pop(0), MX_SCALES_MFMA) if need_dw else None
-        wq1 = None
-        if need_dh:
-            if ctx.have_wq1:
-                wq1 = MXData(saved.pop(0), saved.pop(0), MX_SCALES_MFMA)
-            else:
-                wq1 = _cast_cols_padded(saved.pop(0), mode)
-        if need_dh and need_dw and N % ops.BLOCK == 0:
-            dyq0, dyq1 = ops.to_mx_dim0_dim1(dy2, mode, MX_SCALES_MFMA)
-        else:
-            dyq0 = _cast_rows_padded(dy2, mode) if need_dh else None
-            dyq1 = ops.to_mx_dim1(dy2, mode, MX_SCALES_MFMA) if need_dw else None
+        saved = ctx.saved_tensors
+        h1, h3 = saved[0], saved[1]
+        dyq0, dyq1 = ops.to_operands(_bf16(dy.reshape(-1, dy.shape[-1])), mode, need_dh, need_dw)
         dh1 = dh3 = dw = None
         if need_dh:
-            dg = ops.mx_gemm_nt(dyq0, wq1).view(h1.shape)
+            dg = ops.mx_gemm_nt(dyq0, MXData(saved[-2], saved[-1], MX_SCALES_MFMA)).view(h1.shape)
             if ctx.needs_input_grad[1]:
                 dh3 = dg * F.silu(h1)
             if ctx.needs_input_grad[0]:
                 dh1 = torch.ops.aten.silu_backward(dg * h3, h1)
         if need_dw:
-            dw = ops.mx_gemm_nt(dyq1, gq1)
+            dw = ops.mx_gemm_nt(dyq1, MXData(saved[2], saved[3], MX_SCALES_MFMA))
             if dw.dtype != ctx.w_dtype:
                 dw = dw.to(ctx.w_dtype)
         return dh1, dh3, dw, None
 
 
 def swiglu_fusable(h1: torch.Tensor, h3: torch.Tensor, weight: torch.Tensor) -> bool:
-    """The fused gate + cast needs bf16 row-contiguous inputs of one shape with 32-aligned token
-    and hidden counts (what a converted SwiGLU block produces) and a converted weight."""
+    """The fused gate + cast needs bf16 row-contiguous inputs of one shape with a 32-aligned hidden
+    size (what a converted SwiGLU block produces) and a converted weight; any number of tokens."""
     if torch.compiler.is_compiling():  # the fused block functions are eager-only
         return False
     if not isinstance(weight, MXFP8TrainingWeight) or not weight.mx_config.fuse_swiglu_cast:
@@ -90,8 +71,7 @@ def swiglu_fusable(h1: torch.Tensor, h3: torch.Tensor, weight: torch.Tensor) -> 
     if h1.dtype != torch.bfloat16 or h3.dtype != torch.bfloat16 or h1.shape != h3.shape:
         return False
     H = h1.shape[-1]
-    return (h1.is_contiguous() and h3.is_contiguous() and h1.is_cuda and H % ops.BLOCK == 0
-            and h1.numel() // max(H, 1) % ops.BLOCK == 0 and h1.numel() > 0)
+    return h1.is_contiguous() and h3.is_contiguous() and h1.is_cuda and H % ops.BLOCK == 0 and h1.numel() > 0
 
 
 def mx_swiglu_linear(h1: torch.Tensor, h3: torch.Tensor, weight: torch.Tensor,
@@ -122,33 +102,67 @@ FFN_SAVED = 14
 
 def block_pitch_pad(cfg: MXFP8Config, need_dx: bool, need_dw: bool) -> int:
     """Bytes the eager SwiGLU block leaves between the rows of its MXFP8 codes: ops.CODE_PITCH_PAD
-    in a training step (every operand is then cast both ways by the kernels that know pitches);
-    none with cached weight casts, whose entries other callers read as dense codes."""
+    in a training step; none with cached weight casts, whose entries other callers read as dense
+    codes."""
     return ops.CODE_PITCH_PAD if need_dx and need_dw and not cfg.cache_weight_casts else 0
 
 
+class _FFNCasts:
+    """The casts of the SwiGLU block in the form its caller runs: GEMM operands over any number of
+    tokens, contractions in whole 128-deep blocks (`ops.to_operands`: the eager block), or dense ones
+    over exactly the sizes, which must be multiples of 32 (the traced operator, whose saved tensors
+    have the shapes its fake kernel announces)."""
+
+    def __init__(self, cfg: MXFP8Config, whole_blocks: bool, pad: int):
+        self.cfg, self.mode, self.whole, self.pad = cfg, cfg.scale_mode, whole_blocks, pad
+
+    def plain(self, t, cols: bool):
+        if self.whole:
+            return ops.to_operands(t, self.mode, True, cols, self.pad)
+        t = t.contiguous()
+        return (ops.to_mx_dim0_dim1(t, self.mode, MX_SCALES_MFMA) if cols
+                else (ops.to_mx_dim0(t, self.mode, MX_SCALES_MFMA), None))
+
+    def weight(self, w, cols: bool):
+        return _cast_weight(w, self.mode, cols, self.cfg, self.pad, self.whole)
+
+    def gate(self, h13, cols: bool):
+        if self.whole:
+            return ops.swiglu_to_operands(h13[0], h13[1], self.mode, cols, self.pad)
+        return ops.swiglu_to_mx_dim0_dim1(h13[0], h13[1], self.mode, MX_SCALES_MFMA)[:2]
+
+    def gate_backward(self, dg, h13):
+        if self.whole:
+            return ops.swiglu_bwd_to_operands(dg, h13[0], h13[1], self.mode, self.pad)
+        return ops.swiglu_bwd_to_mx_dim0_dim1(dg, h13[0], h13[1], self.mode, MX_SCALES_MFMA)[:2]
+
+    def norm(self, x2, weight, eps):
+        if self.whole:
+            return ops.rms_norm_to_operands(x2, _bf16(weight), eps, self.mode, self.pad)
+        return ops.rms_norm_to_mx(x2, _bf16(weight), eps, self.mode, MX_SCALES_MFMA)[:3]
+
+
 def ffn_forward(x2, x_src, w1, w2, w3, cfg: MXFP8Config, need_dx: bool, need_dw: bool, norm_weight=None,
-                eps: float = 0.0, pad: int = 0):
+                eps: float = 0.0, pad: int = 0, whole_blocks: bool = False):
     """Forward of the SwiGLU block on a 2-D bf16 activation: (y [M, out], the FFN_SAVED slots).
     `x_src` is the tensor the activation-cast cache is keyed on (None: no sharing of x's cast
     with sibling linears); `pad`: the row pitch padding of every code matrix (the saved ones
-    carry it into the backward).  The eager autograd function and the traced operator both run this."""
-    mode = cfg.scale_mode
+    carry it into the backward); `whole_blocks`: see `_FFNCasts`.  The eager autograd function and
+    the traced operator both run this."""
+    cast = _FFNCasts(cfg, whole_blocks, pad)
     rstd = None
     if norm_weight is not None:  # RMSNorm in front: normalised inside the cast, rstd kept for its backward
         x2 = x2.contiguous()
-        xq0, xq1, rstd, _ = ops.rms_norm_to_mx(x2, _bf16(norm_weight), eps, mode, MX_SCALES_MFMA, pitch_pad=pad)
+        xq0, xq1, rstd = cast.norm(x2, norm_weight, eps)
     elif x_src is not None:
-        xq0, xq1 = _cast_activation(x2, x_src, mode, need_cols=need_dw, pitch_pad=pad)
-    elif need_dw:
-        xq0, xq1 = ops.to_mx_dim0_dim1(x2.contiguous(), mode, MX_SCALES_MFMA, pitch_pad=pad)
+        xq0, xq1 = _cast_activation(x2, x_src, cfg.scale_mode, need_cols=need_dw, pitch_pad=pad)
     else:
-        xq0, xq1 = ops.to_mx_dim0(x2.contiguous(), mode, MX_SCALES_MFMA), None
-    w1q0, w1q1 = _cast_weight(w1, mode, need_dx, cfg, pitch_pad=pad)
-    w3q0, w3q1 = _cast_weight(w3, mode, need_dx, cfg, pitch_pad=pad)
-    w2q0, w2q1 = _cast_weight(w2, mode, need_dx or need_dw, cfg, pitch_pad=pad)
+        xq0, xq1 = cast.plain(x2, need_dw)
+    w1q0, w1q1 = cast.weight(w1, need_dx)
+    w3q0, w3q1 = cast.weight(w3, need_dx)
+    w2q0, w2q1 = cast.weight(w2, need_dx or need_dw)
     h13 = ops.mx_gemm_nt_shared_a(xq0, w1q0, w3q0)  # one launch: x's panels fetched once for both
-    gq0, gq1, _ = ops.swiglu_to_mx_dim0_dim1(h13[0], h13[1], mode, MX_SCALES_MFMA, pitch_pad=pad)
+    gq0, gq1 = cast.gate(h13, need_dw)
     y = ops.mx_gemm_nt(gq0, w2q0)
     saved = [None] * FFN_SAVED
     if need_dx or need_dw:
@@ -163,18 +177,15 @@ def ffn_forward(x2, x_src, w1, w2, w3, cfg: MXFP8Config, need_dx: bool, need_dw:
 
 
 def ffn_backward(dy2, saved, cfg: MXFP8Config, need_x: bool, need_dw1: bool, need_dw2: bool, need_dw3: bool,
-                 need_dnw: bool = False, pad: int = 0):
-    """(dx [M, in], dW1, dW2, dW3, d norm weight), bf16, None where not asked for; `pad` as the
-    forward's."""
-    mode = cfg.scale_mode
+                 need_dnw: bool = False, pad: int = 0, whole_blocks: bool = False):
+    """(dx [M, in], dW1, dW2, dW3, d norm weight), bf16, None where not asked for; `pad` and
+    `whole_blocks` as the forward's."""
+    cast = _FFNCasts(cfg, whole_blocks, pad)
     h13 = saved[0]
     w2q1 = _take(saved, 1)
-    if need_dw2:
-        dyq0, dyq1 = ops.to_mx_dim0_dim1(dy2, mode, MX_SCALES_MFMA, pitch_pad=pad)
-    else:
-        dyq0, dyq1 = ops.to_mx_dim0(dy2, mode, MX_SCALES_MFMA), None
+    dyq0, dyq1 = cast.plain(dy2, need_dw2)
     dg = ops.mx_gemm_nt(dyq0, w2q1)
-    (da0, da1), (db0, db1), _ = ops.swiglu_bwd_to_mx_dim0_dim1(dg, h13[0], h13[1], mode, MX_SCALES_MFMA, pitch_pad=pad)
+    (da0, da1), (db0, db1) = cast.gate_backward(dg, h13)
     dx = dw1 = dw2 = dw3 = dnw = None
     if need_dw1 or need_dw2 or need_dw3:
         xq1, gq1 = _take(saved, 3), _take(saved, 5)
@@ -209,7 +220,7 @@ class _MXFeedForward(torch.autograd.Function):
         need_dw = any(ctx.needs_input_grad[1:4])
         ctx.pad = block_pitch_pad(cfg, need_dx, need_dw)
         y, saved = ffn_forward(x.reshape(-1, x.shape[-1]), x, w1, w2, w3, cfg, need_dx, need_dw, norm_weight, eps,
-                               pad=ctx.pad)
+                               pad=ctx.pad, whole_blocks=True)
         ctx.cfg, ctx.x_shape = cfg, x.shape
         ctx.w_dtypes = (w1.dtype, w2.dtype, w3.dtype)
         ctx.save_for_backward(*saved)
@@ -221,7 +232,7 @@ class _MXFeedForward(torch.autograd.Function):
         need = ctx.needs_input_grad
         dy2 = _bf16(dy.reshape(-1, dy.shape[-1])).contiguous()
         dx, dw1, dw2, dw3, dnw = ffn_backward(dy2, list(ctx.saved_tensors), ctx.cfg, need[0], need[1], need[2],
-                                              need[3], need[5], pad=ctx.pad)
+                                              need[3], need[5], pad=ctx.pad, whole_blocks=True)
         cast_back = lambda g, dt: g if g is None or g.dtype == dt else g.to(dt)
         if dx is not None:
             dx = dx.view(ctx.x_shape)
@@ -231,7 +242,7 @@ class _MXFeedForward(torch.autograd.Function):
 
 def feed_forward_fusable(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, w3: torch.Tensor) -> bool:
     """The whole-block function needs all three weights converted with gate fusion on, a bf16
-    GPU activation and 32-aligned token, model and hidden sizes."""
+    GPU activation and 32-aligned model and hidden sizes (traced: a multiple of 32 tokens, too)."""
     ws = (w1, w2, w3)
     if not all(isinstance(w, MXFP8TrainingWeight) and w.mx_config.fuse_swiglu_cast for w in ws):
         return False
@@ -240,7 +251,9 @@ def feed_forward_fusable(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, w3
     if x.dtype != torch.bfloat16 or not x.is_cuda or x.numel() == 0 or w1.shape != w3.shape:
         return False
     D, H = x.shape[-1], w1.shape[0]
-    return D % ops.BLOCK == 0 and H % ops.BLOCK == 0 and (x.numel() // D) % ops.BLOCK == 0
+    if torch.compiler.is_compiling() and (x.numel() // D) % ops.BLOCK:
+        return False
+    return D % ops.BLOCK == 0 and H % ops.BLOCK == 0
 
 
 def mx_feed_forward(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, w3: torch.Tensor,
@@ -279,7 +292,7 @@ class _MXNormLinears(torch.autograd.Function):
         mode = cfg.scale_mode
         D = x.shape[-1]
         x2 = x.reshape(-1, D).contiguous()
-        hq0, hq1, rstd, _ = ops.rms_norm_to_mx(x2, _bf16(norm_weight), eps, mode, MX_SCALES_MFMA)
+        hq0, hq1, rstd = ops.rms_norm_to_operands(x2, _bf16(norm_weight), eps, mode)
         need_dh = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
         outs, saved = [], [x2, rstd, norm_weight, hq1.codes, hq1.scales]
         for w in weights:
@@ -305,12 +318,7 @@ class _MXNormLinears(torch.autograd.Function):
             if dy is None or not (ctx.need_dh or need_dw):
                 dws.append(None)
                 continue
-            dy2 = _bf16(dy.reshape(-1, dy.shape[-1])).contiguous()
-            if ctx.need_dh and need_dw:
-                dyq0, dyq1 = ops.to_mx_dim0_dim1(dy2, mode, MX_SCALES_MFMA)
-            else:
-                dyq0 = ops.to_mx_dim0(dy2, mode, MX_SCALES_MFMA) if ctx.need_dh else None
-                dyq1 = ops.to_mx_dim1(dy2, mode, MX_SCALES_MFMA) if need_dw else None
+            dyq0, dyq1 = ops.to_operands(_bf16(dy.reshape(-1, dy.shape[-1])), mode, ctx.need_dh, need_dw)
             if ctx.need_dh:
                 part = ops.mx_gemm_nt(dyq0, MXData(rest[2 * i], rest[2 * i + 1], MX_SCALES_MFMA))
                 dh = part if dh is None else dh + part
@@ -332,7 +340,7 @@ def norm_fusable(x: torch.Tensor, norm_weight: torch.Tensor | None, *weights: to
                  for_feed_forward: bool = False) -> bool:
     """RMSNorm can move into the cast when the converter was built with `fuse_rmsnorm_cast`, the
     norm has a bf16 weight, every linear behind it is converted with in_features % 32 == 0 and
-    out_features % 32 == 0, and x is a bf16 GPU tensor with a multiple of 32 tokens.
+    out_features % 32 == 0, and x is a bf16 GPU tensor (traced: with a multiple of 32 tokens).
     `for_feed_forward`: the caller is about to use `mx_norm_feed_forward`, which also exists as a
     traced operator; `mx_norm_linears` is an eager function only."""
     if torch.compiler.is_compiling() and not for_feed_forward:
@@ -346,7 +354,9 @@ def norm_fusable(x: torch.Tensor, norm_weight: torch.Tensor | None, *weights: to
     D = x.shape[-1]
     if any(w.shape[1] != D or w.shape[0] % ops.BLOCK for w in weights):
         return False
-    return D % ops.BLOCK == 0 and (x.numel() // D) % ops.BLOCK == 0 and norm_weight.shape == (D,)
+    if torch.compiler.is_compiling() and (x.numel() // D) % ops.BLOCK:
+        return False
+    return D % ops.BLOCK == 0 and norm_weight.shape == (D,)
 
 
 def _norm_eps(x: torch.Tensor, eps: float | None) -> float:

@@ -103,18 +103,15 @@ def clear_cast_cache() -> None:
 
 
 def _cast_activation(x2: torch.Tensor, src: torch.Tensor, mode: str, need_cols: bool, pitch_pad: int = 0):
-    """(row-wise, column-wise or None) MXFP8 forms of the 2-D bf16 activation `x2`.  `pitch_pad`:
-    see `ops.to_mx_dim0_dim1`; callers that feed anything but `ops.mx_gemm_nt` leave it 0."""
+    """(row-wise, column-wise or None) GEMM operands of the 2-D bf16 activation `x2` (any number of
+    tokens), remembered for sibling linears that receive the same tensor `src`."""
     key = (mode, pitch_pad)
     hit = _cast_cache.get(src, key)
     if hit is not None and (hit[1] is not None or not need_cols):
         return hit
-    if need_cols and x2.shape[0] % ops.BLOCK == 0:
-        rows, cols = ops.to_mx_dim0_dim1(x2, mode, MX_SCALES_MFMA, pitch_pad)
-    else:
-        rows, cols = ops.to_mx_dim0(x2, mode, MX_SCALES_MFMA), None
-    _cast_cache.put(src, key, (rows, cols))
-    return rows, cols
+    q = ops.to_operands(x2, mode, True, need_cols, pitch_pad)
+    _cast_cache.put(src, key, q)
+    return q
 
 
 # ----------------------------------------------------------------------------- weight casts
@@ -132,10 +129,10 @@ class _WeightCastCache:
         self._entries = {}
 
     @staticmethod
-    def _key(w: torch.Tensor, mode: str):
+    def _key(w: torch.Tensor, mode):
         return (w.data_ptr(), tuple(w.shape), tuple(w.stride()), w.dtype, mode)
 
-    def get(self, w: torch.Tensor, mode: str):
+    def get(self, w: torch.Tensor, mode):
         e = self._entries.get(self._key(w, mode))
         if e is None:
             return None
@@ -144,7 +141,7 @@ class _WeightCastCache:
             return None
         return rows, cols
 
-    def put(self, w: torch.Tensor, mode: str, rows: MXData, cols):
+    def put(self, w: torch.Tensor, mode, rows: MXData, cols):
         from torch.multiprocessing.reductions import StorageWeakRef
 
         dead = [k for k, e in self._entries.items() if e[0].expired()]
@@ -162,26 +159,30 @@ class _WeightCastCache:
 _weight_cache = _WeightCastCache()
 
 
-def _cast_weight(w: torch.Tensor, mode: str, need_cols: bool, cfg: MXFP8Config, pitch_pad: int = 0):
+def _cast_weight(w: torch.Tensor, mode: str, need_cols: bool, cfg: MXFP8Config, pitch_pad: int = 0,
+                 whole_blocks: bool = True):
     """(row-wise, column-wise or None) MXFP8 forms of a weight [N, K] or stacked [G, N, K], MFMA
-    scale order.  The column-wise form exists when asked for and N is a multiple of 32.
-    `pitch_pad` (2-D weights, both forms asked for): see `ops.to_mx_dim0_dim1`."""
+    scale order.  2-D weights: GEMM operands as `ops.to_operands` makes them (the contraction in whole
+    128-deep blocks, `pitch_pad` bytes between the rows); with `whole_blocks` off the dense form
+    over exactly N and K.  The column-wise form of a stack or a dense form exists when asked for and
+    N is a multiple of 32."""
     cached = cfg.cache_weight_casts
-    mode_key = mode
-    if pitch_pad:
-        mode = (mode, pitch_pad)  # the cache keeps padded and dense casts apart
+    whole = whole_blocks and w.dim() == 2
+    # the cache keeps padded, rounded-up and dense casts apart (they coincide where nothing is rounded)
+    key = (mode, pitch_pad, whole and bool(w.shape[0] % ops.WHOLE_BLOCK or w.shape[1] % ops.WHOLE_BLOCK))
     if cached:
-        hit = _weight_cache.get(w, mode)
+        hit = _weight_cache.get(w, key)
         if hit is not None and (hit[1] is not None or not need_cols or w.shape[-2] % ops.BLOCK):
             return hit
         need_cols = True  # cast once in full, whoever asks first
-    key, mode = mode, mode_key
     wb = (w if w.dtype == torch.bfloat16 else w.to(torch.bfloat16)).contiguous()
-    both = need_cols and wb.shape[-2] % ops.BLOCK == 0
+    both = need_cols and (whole or wb.shape[-2] % ops.BLOCK == 0)
     if wb.dim() == 3:
         q = ops.to_mx_dim0_dim1_batched(wb, mode, MX_SCALES_MFMA) if both else (_cast_w_rows(wb, mode), None)
+    elif both:
+        q = ops.to_mx_dim0_dim1(wb, mode, MX_SCALES_MFMA, pitch_pad, whole)
     else:
-        q = (ops.to_mx_dim0_dim1(wb, mode, MX_SCALES_MFMA, pitch_pad) if both
+        q = (ops.to_operands(wb, mode, True, False, pitch_pad) if whole
              else (ops.to_mx_dim0(wb, mode, MX_SCALES_MFMA), None))
     if cached:
         _weight_cache.put(w, key, q[0], q[1])
@@ -189,99 +190,58 @@ def _cast_weight(w: torch.Tensor, mode: str, need_cols: bool, cfg: MXFP8Config, 
 
 
 # ----------------------------------------------------------------------------- dense linear
+def _linear_forward(x, weight, cfg: MXFP8Config, need_dx: bool, need_dw: bool):
+    """(y, column-wise x or None, column-wise W or None) of the converted linear."""
+    mode, K, N = cfg.scale_mode, x.shape[-1], weight.shape[0]
+    x2 = x.reshape(-1, K)
+    if x2.dtype != torch.bfloat16:
+        x2 = x2.to(torch.bfloat16)
+    # rows further apart than they are long, except with cached weight casts, which the fused
+    # blocks and the hand-over share without a pitch
+    pad = 0 if cfg.cache_weight_casts else ops.CODE_PITCH_PAD
+    xq0, xq1 = _cast_activation(x2, x, mode, need_cols=need_dw, pitch_pad=pad)
+    wq0, wq1 = _cast_weight(weight, mode, need_dx, cfg, pitch_pad=pad)
+    return ops.mx_gemm_nt(xq0, wq0).view(*x.shape[:-1], N), xq1, wq1
+
+
 class _MXLinear(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, cfg: MXFP8Config):
-        mode = cfg.scale_mode
-        K = x.shape[-1]
-        N = weight.shape[0]
-        x2 = x.reshape(-1, K)
-        if x2.dtype != torch.bfloat16:
-            x2 = x2.to(torch.bfloat16)
-        w = weight if weight.dtype == torch.bfloat16 else weight.to(torch.bfloat16)
-        needs_bwd = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
-        M = x2.shape[0]
-        # operands of mx_gemm_nt only: their rows may lie further apart than they are long (not with
-        # cached weight casts, which the fused blocks and the hand-over share in their dense form)
-        pad = 0 if cfg.cache_weight_casts else ops.CODE_PITCH_PAD
-        xq0, xq1 = _cast_activation(x2, x, mode, need_cols=ctx.needs_input_grad[1], pitch_pad=pad)
-        wq0, wq1 = _cast_weight(weight, mode, needs_bwd and ctx.needs_input_grad[0], cfg, pitch_pad=pad)
-        y = ops.mx_gemm_nt(xq0, wq0)
+        need_dx, need_dw = ctx.needs_input_grad[:2]
+        y, xq1, wq1 = _linear_forward(x, weight, cfg, need_dx, need_dw)
         ctx.cfg = cfg
         ctx.x_shape = x.shape
         ctx.x_dtype = x.dtype
         ctx.w_dtype = weight.dtype
-        ctx.have_xq1 = xq1 is not None
-        ctx.have_wq1 = wq1 is not None
         saved = []
-        if ctx.needs_input_grad[1]:
-            saved += [xq1.codes, xq1.scales] if xq1 is not None else [x2]
-        if ctx.needs_input_grad[0]:
-            saved += [wq1.codes, wq1.scales] if wq1 is not None else [w]
+        if need_dw:
+            saved += [xq1.codes, xq1.scales]
+        if need_dx:
+            saved += [wq1.codes, wq1.scales]
         ctx.save_for_backward(*saved)
-        return y.view(*x.shape[:-1], N)
+        return y
 
     @staticmethod
     def backward(ctx, dy):
         _cast_cache.clear()  # the forward whose sibling linears shared a cast is over
         mode = ctx.cfg.scale_mode
         need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
-        saved = list(ctx.saved_tensors)
-        N = dy.shape[-1]
-        dy2 = dy.reshape(-1, N)
+        saved = ctx.saved_tensors
+        dy2 = dy.reshape(-1, dy.shape[-1])
         if dy2.dtype != torch.bfloat16:
             dy2 = dy2.to(torch.bfloat16)
-        dy2 = dy2.contiguous()
-        M = dy2.shape[0]
-        xq1 = wq1 = None
-        if need_dw:
-            if ctx.have_xq1:
-                xq1 = MXData(saved.pop(0), saved.pop(0), MX_SCALES_MFMA)
-            else:  # M not a multiple of 32: pad the token dim with zero rows for the column cast
-                xq1 = _cast_cols_padded(saved.pop(0), mode)
-        if need_dx:
-            if ctx.have_wq1:
-                wq1 = MXData(saved.pop(0), saved.pop(0), MX_SCALES_MFMA)
-            else:
-                wq1 = _cast_cols_padded(saved.pop(0), mode)
-        dyq0 = dyq1 = None
-        if need_dx and need_dw and M % ops.BLOCK == 0 and N % ops.BLOCK == 0:
-            dyq0, dyq1 = ops.to_mx_dim0_dim1(dy2, mode, MX_SCALES_MFMA,
-                                             0 if ctx.cfg.cache_weight_casts else ops.CODE_PITCH_PAD)
-        else:
-            if need_dx:
-                dyq0 = _cast_rows_padded(dy2, mode)
-            if need_dw:
-                dyq1 = _cast_cols_padded(dy2, mode)
+        pad = 0 if ctx.cfg.cache_weight_casts else ops.CODE_PITCH_PAD
+        dyq0, dyq1 = ops.to_operands(dy2, mode, need_dx, need_dw, pad)
         dx = dw = None
         if need_dx:
-            dx = ops.mx_gemm_nt(dyq0, wq1).view(ctx.x_shape)
+            dx = ops.mx_gemm_nt(dyq0, MXData(saved[-2], saved[-1], MX_SCALES_MFMA)).view(ctx.x_shape)
             if dx.dtype != ctx.x_dtype:
                 dx = dx.to(ctx.x_dtype)
         if need_dw:
-            dw = ops.mx_gemm_nt(dyq1, xq1)
+            dw = ops.mx_gemm_nt(dyq1, MXData(saved[0], saved[1], MX_SCALES_MFMA))
             if dw.dtype != ctx.w_dtype:
                 dw = dw.to(ctx.w_dtype)
         return dx, dw, None
-
-
-def _cast_cols_padded(t: torch.Tensor, mode: str) -> MXData:
-    """Column-wise cast of t [R, C]; R is zero-padded up to a multiple of 32 (zeros add nothing
-    to a contraction over R)."""
-    R = t.shape[0]
-    pad = -R % ops.BLOCK
-    if pad:
-        t = torch.cat((t, t.new_zeros((pad, t.shape[1]))), dim=0)
-    return ops.to_mx_dim1(t.contiguous(), mode, MX_SCALES_MFMA)
-
-
-def _cast_rows_padded(t: torch.Tensor, mode: str) -> MXData:
-    """Row-wise cast of t [R, C]; C is zero-padded up to a multiple of 32."""
-    C = t.shape[1]
-    pad = -C % ops.BLOCK
-    if pad:
-        t = torch.cat((t, t.new_zeros((t.shape[0], pad))), dim=1)
-    return ops.to_mx_dim0(t.contiguous(), mode, MX_SCALES_MFMA)
 
 
 def mx_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, cfg: MXFP8Config):
@@ -291,7 +251,10 @@ def mx_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, 
     out_dtype = x.dtype
     if torch.is_autocast_enabled(x.device.type):
         out_dtype = torch.get_autocast_dtype(x.device.type)
-    y = _MXLinear.apply(x, weight, cfg)
+    if torch.is_grad_enabled():
+        y = _MXLinear.apply(x, weight, cfg)
+    else:
+        y = _linear_forward(x, weight, cfg, False, False)[0]
     if y.dtype != out_dtype:
         y = y.to(out_dtype)
     if bias is not None:

@@ -163,11 +163,111 @@ def _pitch_ok(pad: int) -> int:
     return pad if pad > 0 and pad % 16 == 0 else 0
 
 
-def to_mx_dim0_dim1(x: torch.Tensor, mode="floor", order: int = MX_SCALES_ROWMAJOR, pitch_pad: int = 0):
+WHOLE_BLOCK = 128  # depth of the persistent GEMM's K blocks
+
+
+def _whole_blocks(n: int) -> int:
+    return -(-n // WHOLE_BLOCK) * WHOLE_BLOCK
+
+
+def _operand_input(x: torch.Tensor) -> torch.Tensor:
+    """`x` as the tile casts read it: 16-byte aligned rows (a copy where they are not)."""
+    x = _check_hp(x)
+    cols = x.shape[1]
+    if cols % 8:
+        return torch.nn.functional.pad(x, (0, -cols % 8))
+    if x.stride(0) % 8 or x.data_ptr() % 16:
+        return x.clone(memory_format=torch.contiguous_format)
+    return x
+
+
+def _operand_buffers(rows: int, cols: int, pad: int, device):
+    """(codes, MFMA-order scales) of a GEMM operand [rows, cols]: the contraction rounded up to whole
+    128-deep blocks, rows `pad` bytes further apart than that."""
+    k = _whole_blocks(cols)
+    codes = torch.empty((rows, k + pad), dtype=torch.uint8, device=device)
+    if pad:
+        codes = codes[:, :k]
+    return codes, torch.empty((rows + 127) // 128 * 128 * (k // BLOCK), dtype=torch.uint8, device=device)
+
+
+def to_operands(x: torch.Tensor, mode="floor", rows: bool = True, cols: bool = True, pitch_pad: int = 0):
+    """GEMM operands of x [R, C], any R: (row-wise MXData or None, column-wise MXData or None), each
+    with its contraction rounded up to a multiple of 128 by zero codes (`mx_cast_pad`) -- codes
+    [R, C up to 128] and [C, R up to 128], MFMA-order scales, `pitch_pad` as for `to_mx_dim0_dim1`.
+    Both operands of a product come from here, so that they agree on the rounded contraction."""
+    C = x.shape[1]
+    x = _operand_input(x)
+    R, pad, dev = x.shape[0], _pitch_ok(pitch_pad), x.device
+    codes, scales = _operand_buffers(R, x.shape[1], pad, dev) if rows else (None, None)
+    codes_t, scales_t = _operand_buffers(x.shape[1], R, pad, dev) if cols else (None, None)
+    _call("mx_cast_pad", "cast_dim0_dim1" if rows and cols else "cast_dim0" if rows else "cast_dim1", dev, _ptr(x), R,
+          x.shape[1], x.stride(0), _ptr(codes) if rows else None, codes.stride(0) if rows else 0,
+          _ptr(scales) if rows else None, _ptr(codes_t) if cols else None, codes_t.stride(0) if cols else 0,
+          _ptr(scales_t) if cols else None, _mode(mode), _stream(x))
+    if cols and x.shape[1] != C:
+        codes_t = codes_t[:C]
+    return (MXData(codes, scales, MX_SCALES_MFMA) if rows else None,
+            MXData(codes_t, scales_t, MX_SCALES_MFMA) if cols else None)
+
+
+def swiglu_to_operands(a: torch.Tensor, b: torch.Tensor, mode="floor", cols: bool = True, pitch_pad: int = 0):
+    """`to_operands` of silu(a) * b (see `swiglu_to_mx_dim0_dim1`), any number of rows."""
+    a, b = _operand_input(a), _operand_input(b)
+    if a.shape != b.shape:
+        raise ValueError(f"shape mismatch: {tuple(a.shape)} vs {tuple(b.shape)}")
+    (R, C), pad, dev = a.shape, _pitch_ok(pitch_pad), a.device
+    codes, scales = _operand_buffers(R, C, pad, dev)
+    codes_t, scales_t = _operand_buffers(C, R, pad, dev) if cols else (None, None)
+    _call("mx_swiglu_cast_pad", "swiglu_cast_dim0_dim1", dev, _ptr(a), _ptr(b), R, C, a.stride(0), b.stride(0),
+          _ptr(codes), codes.stride(0), _ptr(scales), _ptr(codes_t) if cols else None,
+          codes_t.stride(0) if cols else 0, _ptr(scales_t) if cols else None, _mode(mode), _stream(a))
+    return MXData(codes, scales, MX_SCALES_MFMA), (MXData(codes_t, scales_t, MX_SCALES_MFMA) if cols else None)
+
+
+def swiglu_bwd_to_operands(dg: torch.Tensor, a: torch.Tensor, b: torch.Tensor, mode="floor", pitch_pad: int = 0):
+    """Both operand forms of both gradients of silu(a) * b (see `swiglu_bwd_to_mx_dim0_dim1`), any number
+    of rows: ((da row-wise, da column-wise), (db row-wise, db column-wise))."""
+    dg, a, b = _operand_input(dg), _operand_input(a), _operand_input(b)
+    if a.shape != b.shape or a.shape != dg.shape:
+        raise ValueError(f"shape mismatch: {tuple(dg.shape)}, {tuple(a.shape)}, {tuple(b.shape)}")
+    (R, C), pad, dev = a.shape, _pitch_ok(pitch_pad), a.device
+    ka, kt = _whole_blocks(C), _whole_blocks(R)
+    codes = torch.empty((2, R, ka + pad), dtype=torch.uint8, device=dev)[..., :ka]
+    codes_t = torch.empty((2, C, kt + pad), dtype=torch.uint8, device=dev)[..., :kt]
+    scales = torch.empty((2, mfma_scale_bytes(R, ka // BLOCK)), dtype=torch.uint8, device=dev)
+    scales_t = torch.empty((2, mfma_scale_bytes(C, kt // BLOCK)), dtype=torch.uint8, device=dev)
+    _call("mx_swiglu_bwd_cast_pad", "swiglu_bwd_cast_dim0_dim1", dev, _ptr(dg), _ptr(a), _ptr(b), R, C, dg.stride(0),
+          a.stride(0), b.stride(0), _ptr(codes), codes.stride(1), _ptr(scales), _ptr(codes_t), codes_t.stride(1),
+          _ptr(scales_t), _mode(mode), _stream(a))
+    return tuple((MXData(codes[i], scales[i], MX_SCALES_MFMA), MXData(codes_t[i], scales_t[i], MX_SCALES_MFMA))
+                 for i in range(2))
+
+
+def rms_norm_to_operands(x: torch.Tensor, weight: torch.Tensor, eps: float, mode="floor", pitch_pad: int = 0):
+    """(row-wise, column-wise, rstd) of rms_norm(x) * weight (see `rms_norm_to_mx`), any number of rows."""
+    x = _operand_input(x)
+    if weight.dtype != torch.bfloat16 or weight.shape != (x.shape[1],) or weight.device != x.device:
+        raise TypeError("the norm weight must be bf16 [cols] on x's device")
+    weight = weight.contiguous()
+    (R, C), pad, dev = x.shape, _pitch_ok(pitch_pad), x.device
+    codes, scales = _operand_buffers(R, C, pad, dev)
+    codes_t, scales_t = _operand_buffers(C, R, pad, dev)
+    rstd = torch.empty(R, dtype=torch.float32, device=dev)
+    _call("mx_rmsnorm_cast_pad", "rmsnorm_cast_dim0_dim1", dev, _ptr(x), _ptr(weight), ctypes.c_float(eps), R, C,
+          x.stride(0), _ptr(rstd), _ptr(codes), codes.stride(0), _ptr(scales), _ptr(codes_t), codes_t.stride(0),
+          _ptr(scales_t), _mode(mode), _stream(x))
+    return MXData(codes, scales, MX_SCALES_MFMA), MXData(codes_t, scales_t, MX_SCALES_MFMA), rstd
+
+
+def to_mx_dim0_dim1(x: torch.Tensor, mode="floor", order: int = MX_SCALES_ROWMAJOR, pitch_pad: int = 0,
+                    whole_blocks: bool = False):
     """Both casts from one read of x; returns (row-wise MXData, column-wise MXData).  With
     `pitch_pad` the rows of both code matrices lie that many bytes further apart than they are
     long (`codes.stride(0)` says so; only `mx_gemm_nt` takes such operands), where the tile kernel
-    takes the input; otherwise the codes are dense."""
+    takes the input; otherwise the codes are dense.  `whole_blocks`: as `to_operands` gives them."""
+    if whole_blocks:
+        return to_operands(x, mode, True, True, pitch_pad)
     x = _check_hp(x)
     R, C = x.shape
     if R % BLOCK or C % BLOCK:

@@ -208,18 +208,20 @@ def export_mxfp8_state_dict(model: nn.Module) -> dict:
         if p is None or not p.is_cuda or p.shape[-1] % 32:
             out[name] = t
             continue
+        lead, K = p.shape[:-1], p.shape[-1]
         with torch.no_grad():
-            rows, _ = _cast_weight(p.as_subclass(torch.Tensor), p.mx_config.scale_mode, False, p.mx_config)
-        lead = p.shape[:-1]
-        n_rows, nblk = int(torch.Size(lead).numel()), p.shape[-1] // 32
+            w = p.as_subclass(torch.Tensor)
+            rows, _ = _cast_weight(w, p.mx_config.scale_mode, False, p.mx_config)
+        codes = rows.codes
+        n_rows, nblk = int(torch.Size(lead).numel()), K // 32
         if p.dim() == 3 and p.shape[1] % 128:  # per-matrix scale blocks: undo them one by one
             per = ops.mfma_scale_bytes(p.shape[1], nblk)
             scales = torch.stack([ops.scale_unlayout(rows.scales[g * per:(g + 1) * per], p.shape[1], nblk)
                                   for g in range(p.shape[0])])
         else:
-            scales = ops.scale_unlayout(rows.scales, n_rows, nblk)
-        out[name] = {"format": MXFP8_PAYLOAD_FORMAT, "codes": rows.codes.view(*p.shape),
-                     "scales": scales.view(*lead, nblk), "dtype": p.dtype}
+            scales = ops.scale_unlayout(rows.scales, n_rows, codes.shape[-1] // 32)[:, :nblk]
+        codes, scales = codes[..., :K].contiguous(), scales.reshape(*lead, nblk)
+        out[name] = {"format": MXFP8_PAYLOAD_FORMAT, "codes": codes.view(*p.shape), "scales": scales, "dtype": p.dtype}
     return out
 
 

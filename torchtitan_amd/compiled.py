@@ -367,7 +367,25 @@ def mx_ffn_fwd(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, w3: torch.Te
     if x2.dtype != torch.bfloat16:
         x2 = x2.to(torch.bfloat16)
     y, saved = mx_blocks.ffn_forward(x2, None, w1, w2, w3, _block_cfg(mode, cache_w), need_dx, need_dw, norm_weight, eps)
-    return (y.view(*x.shape[:-1], w2.shape[0]), *_filled(saved, x.device, skip=(11, 13)))
+    return (y.view(*x.shape[:-1], w2.shape[0]), *_filled(_ffn_slots(saved), x.device, skip=(11, 13)))
+
+
+# mx_blocks.FFN_SAVED as the operator's 14 tensors: an MXData takes two slots, codes and scales
+_FFN_PAIRS = ("w2", "x", "g", "w1", "w3")
+
+
+def _ffn_slots(saved: dict) -> list:
+    slots = [saved["h13"]]
+    for name in _FFN_PAIRS:
+        q = saved[name]
+        slots += [None, None] if q is None else [q.codes, q.scales]
+    return slots + [saved["norm_x"], saved["rstd"], saved["norm_weight"]]
+
+
+def _ffn_saved(slots: list) -> dict:
+    saved = {name: None if slots[1 + 2 * i] is None else MXData(slots[1 + 2 * i], slots[2 + 2 * i], MX_SCALES_MFMA)
+             for i, name in enumerate(_FFN_PAIRS)}
+    return dict(saved, h13=slots[0], norm_x=slots[11], rstd=slots[12], norm_weight=slots[13])
 
 
 @mx_ffn_fwd.register_fake
@@ -401,8 +419,8 @@ def mx_ffn_bwd(dy: torch.Tensor, saved: list[torch.Tensor], x: torch.Tensor | No
     dy2 = dy.reshape(-1, dy.shape[-1])
     if dy2.dtype != torch.bfloat16:
         dy2 = dy2.to(torch.bfloat16)
-    dx, dw1, dw2, dw3, dnw = mx_blocks.ffn_backward(dy2.contiguous(), s, _block_cfg(mode, False), need_x, need_dw1,
-                                                    need_dw2, need_dw3, need_dnw)
+    dx, dw1, dw2, dw3, dnw = mx_blocks.ffn_backward(dy2.contiguous(), _ffn_saved(s), _block_cfg(mode, False), need_x,
+                                                    need_dw1, need_dw2, need_dw3, need_dnw)
     none = lambda: torch.empty((0,), dtype=torch.bfloat16, device=dy.device)
     return (dx if (dx is not None and need_x) else none(), _pack_pair(dw1, dw3, dy.device),
             dw2 if dw2 is not None else none(), dnw if dnw is not None else none())

@@ -31,12 +31,8 @@ class _MXSwiGLULinear(torch.autograd.Function):
         wq0, wq1 = _cast_weight(weight, mode, need_dh, cfg)
         y = ops.mx_gemm_nt(gq0, wq0)
         ctx.cfg, ctx.w_dtype = cfg, weight.dtype
-        saved = [h1, h3]
-        if need_dw:
-            saved += [gq1.codes, gq1.scales]
-        if need_dh:
-            saved += [wq1.codes, wq1.scales]
-        ctx.save_for_backward(*saved)
+        ctx.g_layout, ctx.w_layout = (gq1.layout if need_dw else None), (wq1.layout if need_dh else None)
+        ctx.save_for_backward(h1, h3, gq1.buf if need_dw else None, wq1.buf if need_dh else None)
         return y.view(*h1.shape[:-1], N)
 
     @staticmethod
@@ -44,18 +40,17 @@ class _MXSwiGLULinear(torch.autograd.Function):
         mode = ctx.cfg.scale_mode
         need_dh = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
         need_dw = ctx.needs_input_grad[2]
-        saved = ctx.saved_tensors
-        h1, h3 = saved[0], saved[1]
+        h1, h3, g_buf, w_buf = ctx.saved_tensors
         dyq0, dyq1 = ops.to_operands(_bf16(dy.reshape(-1, dy.shape[-1])), mode, need_dh, need_dw)
         dh1 = dh3 = dw = None
         if need_dh:
-            dg = ops.mx_gemm_nt(dyq0, MXData(saved[-2], saved[-1], MX_SCALES_MFMA)).view(h1.shape)
+            dg = ops.mx_gemm_nt(dyq0, ops.Operand(w_buf, ctx.w_layout)).view(h1.shape)
             if ctx.needs_input_grad[1]:
                 dh3 = dg * F.silu(h1)
             if ctx.needs_input_grad[0]:
                 dh1 = torch.ops.aten.silu_backward(dg * h3, h1)
         if need_dw:
-            dw = ops.mx_gemm_nt(dyq1, MXData(saved[2], saved[3], MX_SCALES_MFMA))
+            dw = ops.mx_gemm_nt(dyq1, ops.Operand(g_buf, ctx.g_layout))
             if dw.dtype != ctx.w_dtype:
                 dw = dw.to(ctx.w_dtype)
         return dh1, dh3, dw, None
@@ -85,6 +80,11 @@ def mx_swiglu_linear(h1: torch.Tensor, h3: torch.Tensor, weight: torch.Tensor,
 
 
 # ----------------------------------------------------------------------------- whole SwiGLU block
+def _rows_of(t: torch.Tensor) -> torch.Tensor:
+    """`t` as a matrix of its last dimension's rows."""
+    return t if t.dim() == 2 else t.reshape(-1, t.shape[-1])
+
+
 def _bf16(t: torch.Tensor) -> torch.Tensor:
     return t if t.dtype == torch.bfloat16 else t.to(torch.bfloat16)
 
@@ -94,10 +94,10 @@ def _take(saved, i):
     return MXData(saved[i], saved[i + 1], MX_SCALES_MFMA)
 
 
-# What the SwiGLU block keeps for its backward, by slot (None where a gradient is not needed):
-#   0 h1 and h3 stacked [2, M, H]    1, 2 column-wise W2       3, 4 column-wise x     5, 6 column-wise g
-#   7, 8 column-wise W1              9, 10 column-wise W3      11 x, 12 rstd, 13 norm weight (norm in front)
-FFN_SAVED = 14
+# What the SwiGLU block keeps for its backward (None where a gradient is not needed): h1 and h3 stacked
+# [2, M, H], the column-wise W2, x, g, W1, W3 (as `_FFNCasts` makes them), and with a norm in front x, its
+# rstd and the norm weight.
+FFN_SAVED = ("h13", "w2", "x", "g", "w1", "w3", "norm_x", "rstd", "norm_weight")
 
 
 def block_pitch_pad(cfg: MXFP8Config, need_dx: bool, need_dw: bool) -> int:
@@ -144,7 +144,7 @@ class _FFNCasts:
 
 def ffn_forward(x2, x_src, w1, w2, w3, cfg: MXFP8Config, need_dx: bool, need_dw: bool, norm_weight=None,
                 eps: float = 0.0, pad: int = 0, whole_blocks: bool = False):
-    """Forward of the SwiGLU block on a 2-D bf16 activation: (y [M, out], the FFN_SAVED slots).
+    """Forward of the SwiGLU block on a 2-D bf16 activation: (y [M, out], dict of what FFN_SAVED names).
     `x_src` is the tensor the activation-cast cache is keyed on (None: no sharing of x's cast
     with sibling linears); `pad`: the row pitch padding of every code matrix (the saved ones
     carry it into the backward); `whole_blocks`: see `_FFNCasts`.  The eager autograd function and
@@ -164,15 +164,15 @@ def ffn_forward(x2, x_src, w1, w2, w3, cfg: MXFP8Config, need_dx: bool, need_dw:
     h13 = ops.mx_gemm_nt_shared_a(xq0, w1q0, w3q0)  # one launch: x's panels fetched once for both
     gq0, gq1 = cast.gate(h13, need_dw)
     y = ops.mx_gemm_nt(gq0, w2q0)
-    saved = [None] * FFN_SAVED
+    saved = dict.fromkeys(FFN_SAVED)
     if need_dx or need_dw:
-        saved[0:3] = [h13, w2q1.codes, w2q1.scales]
+        saved.update(h13=h13, w2=w2q1)
     if need_dw:
-        saved[3:7] = [xq1.codes, xq1.scales, gq1.codes, gq1.scales]
+        saved.update(x=xq1, g=gq1)
     if need_dx:
-        saved[7:11] = [w1q1.codes, w1q1.scales, w3q1.codes, w3q1.scales]
+        saved.update(w1=w1q1, w3=w3q1)
         if norm_weight is not None:
-            saved[11:14] = [x2, rstd, norm_weight]
+            saved.update(norm_x=x2, rstd=rstd, norm_weight=norm_weight)
     return y, saved
 
 
@@ -181,27 +181,24 @@ def ffn_backward(dy2, saved, cfg: MXFP8Config, need_x: bool, need_dw1: bool, nee
     """(dx [M, in], dW1, dW2, dW3, d norm weight), bf16, None where not asked for; `pad` and
     `whole_blocks` as the forward's."""
     cast = _FFNCasts(cfg, whole_blocks, pad)
-    h13 = saved[0]
-    w2q1 = _take(saved, 1)
+    h13 = saved["h13"]
     dyq0, dyq1 = cast.plain(dy2, need_dw2)
-    dg = ops.mx_gemm_nt(dyq0, w2q1)
+    dg = ops.mx_gemm_nt(dyq0, saved["w2"])
     (da0, da1), (db0, db1) = cast.gate_backward(dg, h13)
     dx = dw1 = dw2 = dw3 = dnw = None
-    if need_dw1 or need_dw2 or need_dw3:
-        xq1, gq1 = _take(saved, 3), _take(saved, 5)
-        if need_dw1 and need_dw3:
-            dw1, dw3 = ops.mx_gemm_nt_shared_b(da1, db1, xq1).unbind(0)  # one launch over x's column-wise form
-        elif need_dw1:
-            dw1 = ops.mx_gemm_nt(da1, xq1)
-        elif need_dw3:
-            dw3 = ops.mx_gemm_nt(db1, xq1)
-        if need_dw2:
-            dw2 = ops.mx_gemm_nt(dyq1, gq1)
+    if need_dw1 and need_dw3:
+        dw1, dw3 = ops.mx_gemm_nt_shared_b(da1, db1, saved["x"]).unbind(0)  # one launch over x's column-wise form
+    elif need_dw1:
+        dw1 = ops.mx_gemm_nt(da1, saved["x"])
+    elif need_dw3:
+        dw3 = ops.mx_gemm_nt(db1, saved["x"])
+    if need_dw2:
+        dw2 = ops.mx_gemm_nt(dyq1, saved["g"])
     if need_x or need_dnw:
         # dx = d(h1) W1 + d(h3) W3 as one GEMM: summed in float32, rounded once
-        dx = ops.mx_gemm_nt_pair(da0, _take(saved, 7), db0, _take(saved, 9))
-        if saved[11] is not None:
-            dx, dnw = _rms_norm_backward(dx, saved[11], saved[12], saved[13], need_x, need_dnw)
+        dx = ops.mx_gemm_nt_pair(da0, saved["w1"], db0, saved["w3"])
+        if saved["norm_x"] is not None:
+            dx, dnw = _rms_norm_backward(dx, saved["norm_x"], saved["rstd"], saved["norm_weight"], need_x, need_dnw)
     return dx, dw1, dw2, dw3, dnw
 
 
@@ -219,22 +216,24 @@ class _MXFeedForward(torch.autograd.Function):
         need_dx = ctx.needs_input_grad[0] or ctx.needs_input_grad[5]
         need_dw = any(ctx.needs_input_grad[1:4])
         ctx.pad = block_pitch_pad(cfg, need_dx, need_dw)
-        y, saved = ffn_forward(x.reshape(-1, x.shape[-1]), x, w1, w2, w3, cfg, need_dx, need_dw, norm_weight, eps,
-                               pad=ctx.pad, whole_blocks=True)
+        y, saved = ffn_forward(_rows_of(x), x, w1, w2, w3, cfg, need_dx, need_dw, norm_weight, eps, pad=ctx.pad,
+                               whole_blocks=True)
         ctx.cfg, ctx.x_shape = cfg, x.shape
         ctx.w_dtypes = (w1.dtype, w2.dtype, w3.dtype)
-        ctx.save_for_backward(*saved)
-        return y.view(*x.shape[:-1], w2.shape[0])
+        ctx.layouts = [q.layout if isinstance(q, ops.Operand) else None for q in saved.values()]
+        ctx.save_for_backward(*[q.buf if isinstance(q, ops.Operand) else q for q in saved.values()])
+        return y if x.dim() == 2 else y.view(*x.shape[:-1], w2.shape[0])
 
     @staticmethod
     def backward(ctx, dy):
         _cast_cache.clear()  # the forward that shared x's cast with a sibling is over
         need = ctx.needs_input_grad
-        dy2 = _bf16(dy.reshape(-1, dy.shape[-1])).contiguous()
-        dx, dw1, dw2, dw3, dnw = ffn_backward(dy2, list(ctx.saved_tensors), ctx.cfg, need[0], need[1], need[2],
-                                              need[3], need[5], pad=ctx.pad, whole_blocks=True)
+        saved = {name: (t if layout is None else ops.Operand(t, layout))
+                 for name, t, layout in zip(FFN_SAVED, ctx.saved_tensors, ctx.layouts)}
+        dx, dw1, dw2, dw3, dnw = ffn_backward(_bf16(_rows_of(dy)), saved, ctx.cfg, need[0], need[1], need[2], need[3],
+                                              need[5], pad=ctx.pad, whole_blocks=True)
         cast_back = lambda g, dt: g if g is None or g.dtype == dt else g.to(dt)
-        if dx is not None:
+        if dx is not None and len(ctx.x_shape) != 2:
             dx = dx.view(ctx.x_shape)
         return (dx, cast_back(dw1, ctx.w_dtypes[0]), cast_back(dw2, ctx.w_dtypes[1]), cast_back(dw3, ctx.w_dtypes[2]),
                 None, dnw, None)
@@ -265,9 +264,19 @@ def mx_feed_forward(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, w3: tor
 
         with torch._C.DisableTorchFunctionSubclass():
             return mx_feed_forward_traced(x, w1, w2, w3, bias2)
-    y = _MXFeedForward.apply(x, _unwrap(w1), _unwrap(w2), _unwrap(w3), w2.mx_config, None, 0.0)
-    if bias2 is not None:
-        y = y + _unwrap(bias2).to(y.dtype)
+    return _feed_forward(x, w1, w2, w3, bias2, None, 0.0)
+
+
+def _feed_forward(x, w1, w2, w3, bias2, norm_weight, eps: float):
+    with torch._C.DisableTorchFunctionSubclass():
+        if torch.is_grad_enabled():
+            y = _MXFeedForward.apply(x, w1, w2, w3, w2.mx_config, norm_weight, eps)
+        else:  # nothing is kept for a backward
+            y, _ = ffn_forward(_rows_of(x), x, w1, w2, w3, w2.mx_config, False, False, norm_weight, eps,
+                               whole_blocks=True)
+            y = y if x.dim() == 2 else y.view(*x.shape[:-1], w2.shape[0])
+        if bias2 is not None:
+            y = y + bias2.to(y.dtype)
     return y
 
 
@@ -294,12 +303,13 @@ class _MXNormLinears(torch.autograd.Function):
         x2 = x.reshape(-1, D).contiguous()
         hq0, hq1, rstd = ops.rms_norm_to_operands(x2, _bf16(norm_weight), eps, mode)
         need_dh = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
-        outs, saved = [], [x2, rstd, norm_weight, hq1.codes, hq1.scales]
+        outs, saved, ctx.layouts = [], [x2, rstd, norm_weight, hq1.buf], [hq1.layout]
         for w in weights:
             wq0, wq1 = _cast_weight(w, mode, need_dh, cfg)
             outs.append(ops.mx_gemm_nt(hq0, wq0).view(*x.shape[:-1], w.shape[0]))
             if need_dh:
-                saved += [wq1.codes, wq1.scales]
+                saved.append(wq1.buf)
+                ctx.layouts.append(wq1.layout)
         ctx.cfg, ctx.x_shape, ctx.need_dh = cfg, x.shape, need_dh
         ctx.w_dtypes = tuple(w.dtype for w in weights)
         ctx.save_for_backward(*saved)
@@ -310,8 +320,7 @@ class _MXNormLinears(torch.autograd.Function):
         mode = ctx.cfg.scale_mode
         saved = list(ctx.saved_tensors)
         x2, rstd, norm_weight = saved[:3]
-        hq1 = MXData(saved[3], saved[4], MX_SCALES_MFMA)
-        rest = saved[5:]
+        hq1, *wqs = (ops.Operand(buf, layout) for buf, layout in zip(saved[3:], ctx.layouts))
         dh, dws = None, []
         for i, dy in enumerate(dys):
             need_dw = ctx.needs_input_grad[4 + i]
@@ -320,7 +329,7 @@ class _MXNormLinears(torch.autograd.Function):
                 continue
             dyq0, dyq1 = ops.to_operands(_bf16(dy.reshape(-1, dy.shape[-1])), mode, ctx.need_dh, need_dw)
             if ctx.need_dh:
-                part = ops.mx_gemm_nt(dyq0, MXData(rest[2 * i], rest[2 * i + 1], MX_SCALES_MFMA))
+                part = ops.mx_gemm_nt(dyq0, wqs[i])
                 dh = part if dh is None else dh + part
             dw = None
             if need_dw:
@@ -381,11 +390,7 @@ def mx_norm_feed_forward(x: torch.Tensor, norm_weight: torch.Tensor, eps: float 
 
         with torch._C.DisableTorchFunctionSubclass():
             return mx_feed_forward_traced(x, w1, w2, w3, bias2, norm_weight, _norm_eps(x, eps))
-    y = _MXFeedForward.apply(x, _unwrap(w1), _unwrap(w2), _unwrap(w3), w2.mx_config, norm_weight,
-                             _norm_eps(x, eps))
-    if bias2 is not None:
-        y = y + _unwrap(bias2).to(y.dtype)
-    return y
+    return _feed_forward(x, w1, w2, w3, bias2, norm_weight, _norm_eps(x, eps))
 
 
 def grouped_layout(D: int, H: int, G: int):

@@ -72,20 +72,19 @@ class _ActivationCastCache:
         self._value = None
         self._capturing = False
 
-    def _sync_capture_state(self):
-        capturing = torch.cuda.is_available() and torch.cuda.is_current_stream_capturing()
+    def _sync_capture_state(self, x: torch.Tensor):
+        capturing = x.is_cuda and torch.cuda.is_current_stream_capturing()
         if capturing != self._capturing:
             self.clear()
             self._capturing = capturing
 
-    def get(self, x: torch.Tensor, mode: str):
-        self._sync_capture_state()
+    def get(self, x: torch.Tensor, mode):
+        self._sync_capture_state(x)
         if self._ref is not None and self._ref() is x and self._key == (x._version, mode, x.data_ptr()):
             return self._value
         return None
 
-    def put(self, x: torch.Tensor, mode: str, value):
-        self._sync_capture_state()
+    def put(self, x: torch.Tensor, mode, value):
         self._ref = weakref.ref(x)
         self._key = (x._version, mode, x.data_ptr())
         self._value = value
@@ -193,7 +192,7 @@ def _cast_weight(w: torch.Tensor, mode: str, need_cols: bool, cfg: MXFP8Config, 
 def _linear_forward(x, weight, cfg: MXFP8Config, need_dx: bool, need_dw: bool):
     """(y, column-wise x or None, column-wise W or None) of the converted linear."""
     mode, K, N = cfg.scale_mode, x.shape[-1], weight.shape[0]
-    x2 = x.reshape(-1, K)
+    x2 = x if x.dim() == 2 else x.reshape(-1, K)
     if x2.dtype != torch.bfloat16:
         x2 = x2.to(torch.bfloat16)
     # rows further apart than they are long, except with cached weight casts, which the fused
@@ -201,7 +200,8 @@ def _linear_forward(x, weight, cfg: MXFP8Config, need_dx: bool, need_dw: bool):
     pad = 0 if cfg.cache_weight_casts else ops.CODE_PITCH_PAD
     xq0, xq1 = _cast_activation(x2, x, mode, need_cols=need_dw, pitch_pad=pad)
     wq0, wq1 = _cast_weight(weight, mode, need_dx, cfg, pitch_pad=pad)
-    return ops.mx_gemm_nt(xq0, wq0).view(*x.shape[:-1], N), xq1, wq1
+    y = ops.mx_gemm_nt(xq0, wq0)
+    return (y if x.dim() == 2 else y.view(*x.shape[:-1], N)), xq1, wq1
 
 
 class _MXLinear(torch.autograd.Function):
@@ -213,12 +213,8 @@ class _MXLinear(torch.autograd.Function):
         ctx.x_shape = x.shape
         ctx.x_dtype = x.dtype
         ctx.w_dtype = weight.dtype
-        saved = []
-        if need_dw:
-            saved += [xq1.codes, xq1.scales]
-        if need_dx:
-            saved += [wq1.codes, wq1.scales]
-        ctx.save_for_backward(*saved)
+        ctx.x_layout, ctx.w_layout = (xq1.layout if need_dw else None), (wq1.layout if need_dx else None)
+        ctx.save_for_backward(xq1.buf if need_dw else None, wq1.buf if need_dx else None)
         return y
 
     @staticmethod
@@ -226,19 +222,21 @@ class _MXLinear(torch.autograd.Function):
         _cast_cache.clear()  # the forward whose sibling linears shared a cast is over
         mode = ctx.cfg.scale_mode
         need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
-        saved = ctx.saved_tensors
-        dy2 = dy.reshape(-1, dy.shape[-1])
+        x_buf, w_buf = ctx.saved_tensors
+        dy2 = dy if dy.dim() == 2 else dy.reshape(-1, dy.shape[-1])
         if dy2.dtype != torch.bfloat16:
             dy2 = dy2.to(torch.bfloat16)
         pad = 0 if ctx.cfg.cache_weight_casts else ops.CODE_PITCH_PAD
         dyq0, dyq1 = ops.to_operands(dy2, mode, need_dx, need_dw, pad)
         dx = dw = None
         if need_dx:
-            dx = ops.mx_gemm_nt(dyq0, MXData(saved[-2], saved[-1], MX_SCALES_MFMA)).view(ctx.x_shape)
+            dx = ops.mx_gemm_nt(dyq0, ops.Operand(w_buf, ctx.w_layout))
+            if len(ctx.x_shape) != 2:
+                dx = dx.view(ctx.x_shape)
             if dx.dtype != ctx.x_dtype:
                 dx = dx.to(ctx.x_dtype)
         if need_dw:
-            dw = ops.mx_gemm_nt(dyq1, MXData(saved[0], saved[1], MX_SCALES_MFMA))
+            dw = ops.mx_gemm_nt(dyq1, ops.Operand(x_buf, ctx.x_layout))
             if dw.dtype != ctx.w_dtype:
                 dw = dw.to(ctx.w_dtype)
         return dx, dw, None

@@ -5,7 +5,6 @@ call into libmxfp8_gfx950.so.  There is no fallback path: CPU tensors are reject
 """
 from __future__ import annotations
 
-import ctypes
 import os
 from typing import NamedTuple
 
@@ -60,18 +59,27 @@ def set_kernel_timer(timer: KernelTimer | None) -> None:
     _timer = timer
 
 
+_entry_points: dict = {}  # C-ABI name -> bound function
+
+
 def _call(name: str, tag: str, device, *args) -> None:
     """Run one C-ABI entry point on `device`'s current stream and raise on a non-zero status."""
-    fn = getattr(_lib.load(), name)
-    with torch.cuda.device(device):
-        if _timer is None:
-            st = fn(*args)
-        else:
-            start, stop = _timer.bracket(tag, device)
-            start.record()
-            st = fn(*args)
-            stop.record()
-    _lib.check(st, name)
+    fn = _entry_points.get(name)
+    if fn is None:
+        fn = _entry_points[name] = getattr(_lib.load(), name)
+    if _timer is None and device.index == _current_device():
+        st = fn(*args)
+    else:
+        with torch.cuda.device(device):
+            if _timer is None:
+                st = fn(*args)
+            else:
+                start, stop = _timer.bracket(tag, device)
+                start.record()
+                st = fn(*args)
+                stop.record()
+    if st:
+        _lib.check(st, name)
 
 
 def _mode(mode) -> int:
@@ -82,12 +90,17 @@ def _mode(mode) -> int:
     return int(mode)
 
 
-def _stream(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+# (device ordinal -> current stream as an address, without a torch.cuda.Stream object around it)
+_current_device = getattr(torch._C, "_cuda_getDevice", lambda: -1)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
-def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr())
+def _stream(t: torch.Tensor) -> int:
+    return _raw_stream(t.device.index)
+
+
+def _ptr(t: torch.Tensor) -> int:
+    return t.data_ptr()
 
 
 def _wrote(out: torch.Tensor) -> torch.Tensor:
@@ -166,10 +179,6 @@ def _pitch_ok(pad: int) -> int:
 WHOLE_BLOCK = 128  # depth of the persistent GEMM's K blocks
 
 
-def _whole_blocks(n: int) -> int:
-    return -(-n // WHOLE_BLOCK) * WHOLE_BLOCK
-
-
 def _operand_input(x: torch.Tensor) -> torch.Tensor:
     """`x` as the tile casts read it: 16-byte aligned rows (a copy where they are not)."""
     x = _check_hp(x)
@@ -181,34 +190,85 @@ def _operand_input(x: torch.Tensor) -> torch.Tensor:
     return x
 
 
-def _operand_buffers(rows: int, cols: int, pad: int, device):
-    """(codes, MFMA-order scales) of a GEMM operand [rows, cols]: the contraction rounded up to whole
-    128-deep blocks, rows `pad` bytes further apart than that."""
-    k = _whole_blocks(cols)
-    codes = torch.empty((rows, k + pad), dtype=torch.uint8, device=device)
-    if pad:
-        codes = codes[:, :k]
-    return codes, torch.empty((rows + 127) // 128 * 128 * (k // BLOCK), dtype=torch.uint8, device=device)
+class Operand:
+    """One operand of the dense GEMMs, e4m3 codes [rows, k] and their MFMA-order scales, in one
+    allocation: rows `ld` bytes apart from byte `at` on, scales from byte `scales_at` on.  Reads as
+    an `MXData` (`codes`, `scales`, `scale_order`; views made when asked for).  One buffer and plain
+    numbers instead of two to four tensors and their views: at small sizes making those takes the
+    host longer than the GPU needs for the cast."""
+
+    __slots__ = ("buf", "rows", "k", "ld", "at", "scales_at")
+    scale_order = MX_SCALES_MFMA
+
+    def __init__(self, buf: torch.Tensor, layout):
+        self.buf = buf
+        self.rows, self.k, self.ld, self.at, self.scales_at = layout
+
+    @property
+    def layout(self):
+        """What, with the buffer, makes the operand: for a backward that gets the buffer back."""
+        return self.rows, self.k, self.ld, self.at, self.scales_at
+
+    @property
+    def codes(self) -> torch.Tensor:
+        return self.buf[self.at:self.at + self.rows * self.ld].view(self.rows, self.ld)[:, :self.k]
+
+    @property
+    def scales(self) -> torch.Tensor:
+        return self.buf[self.scales_at:self.scales_at + mfma_scale_bytes(self.rows, self.k // BLOCK)]
+
+    @property
+    def codes_ptr(self) -> int:
+        return self.buf.data_ptr() + self.at
+
+    @property
+    def scales_ptr(self) -> int:
+        return self.buf.data_ptr() + self.scales_at
+
+    def first_rows(self, n: int) -> "Operand":
+        """The operand's first n rows (n rounds up to the same multiple of 128)."""
+        return Operand(self.buf, (n, self.k, self.ld, self.at, self.scales_at))
+
+    def data(self) -> MXData:
+        return MXData(self.codes, self.scales, MX_SCALES_MFMA)
+
+
+def _new_operand(rows: int, cols: int, pad: int, device) -> Operand:
+    """An operand of `rows` rows with a contraction of `cols` rounded up to whole 128-deep blocks."""
+    k = -(-cols // WHOLE_BLOCK) * WHOLE_BLOCK
+    ld = k + pad
+    scales_at = (rows * ld + 255) & ~255
+    buf = torch.empty(scales_at + ((rows + 127) & ~127) * (k // BLOCK), dtype=torch.uint8, device=device)
+    return Operand(buf, (rows, k, ld, 0, scales_at))
+
+
+def _new_operand_pair(rows: int, cols: int, pad: int, device):
+    """Two operands of one shape in one buffer, codes and then scales stacked."""
+    k = -(-cols // WHOLE_BLOCK) * WHOLE_BLOCK
+    ld, scale_bytes = k + pad, ((rows + 127) & ~127) * (k // BLOCK)
+    scales_at = (2 * rows * ld + 255) & ~255
+    buf = torch.empty(scales_at + 2 * scale_bytes, dtype=torch.uint8, device=device)
+    return (Operand(buf, (rows, k, ld, 0, scales_at)),
+            Operand(buf, (rows, k, ld, rows * ld, scales_at + scale_bytes)))
 
 
 def to_operands(x: torch.Tensor, mode="floor", rows: bool = True, cols: bool = True, pitch_pad: int = 0):
-    """GEMM operands of x [R, C], any R: (row-wise MXData or None, column-wise MXData or None), each
+    """GEMM operands of x [R, C], any R: (row-wise `Operand` or None, column-wise `Operand` or None), each
     with its contraction rounded up to a multiple of 128 by zero codes (`mx_cast_pad`) -- codes
-    [R, C up to 128] and [C, R up to 128], MFMA-order scales, `pitch_pad` as for `to_mx_dim0_dim1`.
-    Both operands of a product come from here, so that they agree on the rounded contraction."""
+    [R, C up to 128] and [C, R up to 128], `pitch_pad` as for `to_mx_dim0_dim1`.  Both operands of a
+    product come from here, so that they agree on the rounded contraction."""
     C = x.shape[1]
     x = _operand_input(x)
-    R, pad, dev = x.shape[0], _pitch_ok(pitch_pad), x.device
-    codes, scales = _operand_buffers(R, x.shape[1], pad, dev) if rows else (None, None)
-    codes_t, scales_t = _operand_buffers(x.shape[1], R, pad, dev) if cols else (None, None)
-    _call("mx_cast_pad", "cast_dim0_dim1" if rows and cols else "cast_dim0" if rows else "cast_dim1", dev, _ptr(x), R,
-          x.shape[1], x.stride(0), _ptr(codes) if rows else None, codes.stride(0) if rows else 0,
-          _ptr(scales) if rows else None, _ptr(codes_t) if cols else None, codes_t.stride(0) if cols else 0,
-          _ptr(scales_t) if cols else None, _mode(mode), _stream(x))
-    if cols and x.shape[1] != C:
-        codes_t = codes_t[:C]
-    return (MXData(codes, scales, MX_SCALES_MFMA) if rows else None,
-            MXData(codes_t, scales_t, MX_SCALES_MFMA) if cols else None)
+    (R, Cx), dev, pad = x.shape, x.device, _pitch_ok(pitch_pad)
+    r = _new_operand(R, Cx, pad, dev) if rows else None
+    c = _new_operand(Cx, R, pad, dev) if cols else None
+    _call("mx_cast_pad", "cast_dim0_dim1" if rows and cols else "cast_dim0" if rows else "cast_dim1", dev,
+          x.data_ptr(), R, Cx, x.stride(0),
+          *((r.codes_ptr, r.ld, r.scales_ptr) if rows else (None, 0, None)),
+          *((c.codes_ptr, c.ld, c.scales_ptr) if cols else (None, 0, None)), _mode(mode), _stream(x))
+    if cols and Cx != C:
+        c = c.first_rows(C)
+    return r, c
 
 
 def swiglu_to_operands(a: torch.Tensor, b: torch.Tensor, mode="floor", cols: bool = True, pitch_pad: int = 0):
@@ -217,12 +277,12 @@ def swiglu_to_operands(a: torch.Tensor, b: torch.Tensor, mode="floor", cols: boo
     if a.shape != b.shape:
         raise ValueError(f"shape mismatch: {tuple(a.shape)} vs {tuple(b.shape)}")
     (R, C), pad, dev = a.shape, _pitch_ok(pitch_pad), a.device
-    codes, scales = _operand_buffers(R, C, pad, dev)
-    codes_t, scales_t = _operand_buffers(C, R, pad, dev) if cols else (None, None)
-    _call("mx_swiglu_cast_pad", "swiglu_cast_dim0_dim1", dev, _ptr(a), _ptr(b), R, C, a.stride(0), b.stride(0),
-          _ptr(codes), codes.stride(0), _ptr(scales), _ptr(codes_t) if cols else None,
-          codes_t.stride(0) if cols else 0, _ptr(scales_t) if cols else None, _mode(mode), _stream(a))
-    return MXData(codes, scales, MX_SCALES_MFMA), (MXData(codes_t, scales_t, MX_SCALES_MFMA) if cols else None)
+    r = _new_operand(R, C, pad, dev)
+    c = _new_operand(C, R, pad, dev) if cols else None
+    _call("mx_swiglu_cast_pad", "swiglu_cast_dim0_dim1", dev, a.data_ptr(), b.data_ptr(), R, C, a.stride(0), b.stride(0),
+          r.codes_ptr, r.ld, r.scales_ptr, *((c.codes_ptr, c.ld, c.scales_ptr) if cols else (None, 0, None)),
+          _mode(mode), _stream(a))
+    return r, c
 
 
 def swiglu_bwd_to_operands(dg: torch.Tensor, a: torch.Tensor, b: torch.Tensor, mode="floor", pitch_pad: int = 0):
@@ -232,16 +292,12 @@ def swiglu_bwd_to_operands(dg: torch.Tensor, a: torch.Tensor, b: torch.Tensor, m
     if a.shape != b.shape or a.shape != dg.shape:
         raise ValueError(f"shape mismatch: {tuple(dg.shape)}, {tuple(a.shape)}, {tuple(b.shape)}")
     (R, C), pad, dev = a.shape, _pitch_ok(pitch_pad), a.device
-    ka, kt = _whole_blocks(C), _whole_blocks(R)
-    codes = torch.empty((2, R, ka + pad), dtype=torch.uint8, device=dev)[..., :ka]
-    codes_t = torch.empty((2, C, kt + pad), dtype=torch.uint8, device=dev)[..., :kt]
-    scales = torch.empty((2, mfma_scale_bytes(R, ka // BLOCK)), dtype=torch.uint8, device=dev)
-    scales_t = torch.empty((2, mfma_scale_bytes(C, kt // BLOCK)), dtype=torch.uint8, device=dev)
-    _call("mx_swiglu_bwd_cast_pad", "swiglu_bwd_cast_dim0_dim1", dev, _ptr(dg), _ptr(a), _ptr(b), R, C, dg.stride(0),
-          a.stride(0), b.stride(0), _ptr(codes), codes.stride(1), _ptr(scales), _ptr(codes_t), codes_t.stride(1),
-          _ptr(scales_t), _mode(mode), _stream(a))
-    return tuple((MXData(codes[i], scales[i], MX_SCALES_MFMA), MXData(codes_t[i], scales_t[i], MX_SCALES_MFMA))
-                 for i in range(2))
+    ra, rb = _new_operand_pair(R, C, pad, dev)
+    ca, cb = _new_operand_pair(C, R, pad, dev)
+    _call("mx_swiglu_bwd_cast_pad", "swiglu_bwd_cast_dim0_dim1", dev, dg.data_ptr(), a.data_ptr(), b.data_ptr(), R, C,
+          dg.stride(0), a.stride(0), b.stride(0), ra.codes_ptr, ra.ld, ra.scales_ptr, ca.codes_ptr, ca.ld, ca.scales_ptr,
+          _mode(mode), _stream(a))
+    return (ra, ca), (rb, cb)
 
 
 def rms_norm_to_operands(x: torch.Tensor, weight: torch.Tensor, eps: float, mode="floor", pitch_pad: int = 0):
@@ -251,13 +307,11 @@ def rms_norm_to_operands(x: torch.Tensor, weight: torch.Tensor, eps: float, mode
         raise TypeError("the norm weight must be bf16 [cols] on x's device")
     weight = weight.contiguous()
     (R, C), pad, dev = x.shape, _pitch_ok(pitch_pad), x.device
-    codes, scales = _operand_buffers(R, C, pad, dev)
-    codes_t, scales_t = _operand_buffers(C, R, pad, dev)
+    r, c = _new_operand(R, C, pad, dev), _new_operand(C, R, pad, dev)
     rstd = torch.empty(R, dtype=torch.float32, device=dev)
-    _call("mx_rmsnorm_cast_pad", "rmsnorm_cast_dim0_dim1", dev, _ptr(x), _ptr(weight), ctypes.c_float(eps), R, C,
-          x.stride(0), _ptr(rstd), _ptr(codes), codes.stride(0), _ptr(scales), _ptr(codes_t), codes_t.stride(0),
-          _ptr(scales_t), _mode(mode), _stream(x))
-    return MXData(codes, scales, MX_SCALES_MFMA), MXData(codes_t, scales_t, MX_SCALES_MFMA), rstd
+    _call("mx_rmsnorm_cast_pad", "rmsnorm_cast_dim0_dim1", dev, x.data_ptr(), weight.data_ptr(), eps, R, C, x.stride(0),
+          rstd.data_ptr(), r.codes_ptr, r.ld, r.scales_ptr, c.codes_ptr, c.ld, c.scales_ptr, _mode(mode), _stream(x))
+    return r, c, rstd
 
 
 def to_mx_dim0_dim1(x: torch.Tensor, mode="floor", order: int = MX_SCALES_ROWMAJOR, pitch_pad: int = 0,
@@ -454,8 +508,14 @@ def token_logprob_bwd(logits: torch.Tensor, target: torch.Tensor, lse: torch.Ten
     rows, vocab = logits.shape
     g = grad_logprob.to(torch.float32).contiguous()
     lse, target = lse.contiguous(), target.contiguous()
-    out = torch.empty((rows, -(-vocab // 8) * 8), dtype=torch.bfloat16, device=logits.device)[:, :vocab]
+    out = torch.empty((rows, -(-vocab // 8) * 8), dtype=torch.bfloat16, device=logits.device)
+    if vocab % 8:
+        out = out[:, :vocab]
     step = 65535
+    if rows <= step:
+        _call("mx_token_logprob_bwd", "token_logprob_bwd", logits.device, _ptr(logits), rows, vocab, logits.stride(0),
+              _ptr(target), _ptr(lse), _ptr(g), _ptr(out), out.stride(0), _stream(logits))
+        return out
     for lo in range(0, rows, step):
         n = min(step, rows - lo)
         _call("mx_token_logprob_bwd", "token_logprob_bwd", logits.device, _ptr(logits[lo:]), n, vocab,
@@ -484,7 +544,7 @@ def rms_norm_to_mx(x: torch.Tensor, weight: torch.Tensor, eps: float, mode="floo
     rstd = torch.empty(R, dtype=torch.float32, device=x.device)
     y = torch.empty((R, C), dtype=torch.bfloat16, device=x.device) if want_y else None
     _call("mx_rmsnorm_cast_dim0_dim1_ld", "rmsnorm_cast_dim0_dim1", x.device, _ptr(x), _ptr(weight),
-          ctypes.c_float(eps), R, C, x.stride(0), _ptr(rstd), _ptr(y) if y is not None else None,
+          eps, R, C, x.stride(0), _ptr(rstd), _ptr(y) if y is not None else None,
           _ptr(codes), codes.stride(0), _ptr(scales), _ptr(codes_t), codes_t.stride(0), _ptr(scales_t),
           _mode(mode), order, _stream(x))
     return MXData(codes, scales, order), MXData(codes_t, scales_t, order), rstd, y
@@ -585,29 +645,55 @@ def _common_pitch(*codes, multiple: int = 128):
     return codes, pitch
 
 
+def _split_workspace(device, M: int, N: int, K: int):
+    """Float32 partial sums for the shapes whose contraction the library splits (few output tiles, long
+    contraction), else None."""
+    key = (device.index, M, N, K)
+    need = _gemm_workspace.get(key)
+    if need is None:
+        with torch.cuda.device(device):
+            need = _gemm_workspace[key] = int(_lib.load().mx_gemm_nt_workspace_bytes(M, N, K))
+    return torch.empty(need, dtype=torch.uint8, device=device) if need else None
+
+
 def _gemm_nt_into(a_codes, a_scales, b_codes, b_scales, out):
     M, K = a_codes.shape
     N = b_codes.shape[0]
     (a_codes, b_codes), ldk = _common_pitch(a_codes, b_codes, multiple=16)  # (the tile kernels take any such pitch)
-    key = (out.device.index, M, N, K)
-    need = _gemm_workspace.get(key)
-    if need is None:
-        with torch.cuda.device(out.device):
-            need = _gemm_workspace[key] = int(_lib.load().mx_gemm_nt_workspace_bytes(M, N, K))
-    ws = None
-    if need:  # few output tiles, long contraction: split over the CUs through float32 partial sums
-        ws = torch.empty(need, dtype=torch.uint8, device=out.device)
+    ws = _split_workspace(out.device, M, N, K)
     if ldk != K:
-        _call("mx_gemm_nt_ld", "gemm_nt_splitk" if need else "gemm_nt", out.device, _ptr(a_codes), _ptr(a_scales),
+        _call("mx_gemm_nt_ld", "gemm_nt" if ws is None else "gemm_nt_splitk", out.device, _ptr(a_codes), _ptr(a_scales),
               _ptr(b_codes), _ptr(b_scales), _ptr(out), M, N, K, ldk, out.stride(0),
-              _ptr(ws) if need else None, need, _stream(out))
+              None if ws is None else _ptr(ws), 0 if ws is None else ws.numel(), _stream(out))
         return out
-    if need:
+    if ws is not None:
         _call("mx_gemm_nt_ws", "gemm_nt_splitk", out.device, _ptr(a_codes), _ptr(a_scales), _ptr(b_codes),
-              _ptr(b_scales), _ptr(out), M, N, K, out.stride(0), _ptr(ws), need, _stream(out))
+              _ptr(b_scales), _ptr(out), M, N, K, out.stride(0), _ptr(ws), ws.numel(), _stream(out))
         return out
     _call("mx_gemm_nt", "gemm_nt", out.device, _ptr(a_codes), _ptr(a_scales), _ptr(b_codes),
           _ptr(b_scales), _ptr(out), M, N, K, out.stride(0), _stream(out))
+    return out
+
+
+def _operands(*qs) -> bool:
+    """All of them `Operand`s with one row pitch the persistent kernel takes: their pointers go to the
+    library as they are."""
+    ld = getattr(qs[0], "ld", 1)
+    if ld % 128:
+        return False
+    for q in qs:
+        if type(q) is not Operand or q.ld != ld:
+            return False
+    return True
+
+
+def _gemm_operands(a: Operand, b: Operand, out: torch.Tensor) -> torch.Tensor:
+    M, N, K = a.rows, b.rows, a.k
+    dev = out.device
+    ws = _split_workspace(dev, M, N, K)
+    _call("mx_gemm_nt_ld", "gemm_nt" if ws is None else "gemm_nt_splitk", dev, a.codes_ptr, a.scales_ptr, b.codes_ptr,
+          b.scales_ptr, out.data_ptr(), M, N, K, a.ld, out.stride(0), None if ws is None else ws.data_ptr(),
+          0 if ws is None else ws.numel(), _stream(out))
     return out
 
 
@@ -677,6 +763,10 @@ def op_sac_save_list() -> set:
 
 def mx_gemm_nt(a: MXData, b: MXData, out: torch.Tensor | None = None) -> torch.Tensor:
     """bf16 D[M,N] = deq(a)[M,K] @ deq(b)[N,K]^T with fp32 accumulation."""
+    if out is None and _operands(a, b) and not _watched():
+        if a.k != b.k:
+            raise ValueError(f"contraction mismatch: {a.k} vs {b.k}")
+        return _gemm_operands(a, b, torch.empty((a.rows, b.rows), dtype=torch.bfloat16, device=a.buf.device))
     M, K = a.codes.shape
     N, Kb = b.codes.shape
     if K != Kb:
@@ -695,11 +785,21 @@ def mx_gemm_nt_pair(a: MXData, b: MXData, a2: MXData, b2: MXData) -> torch.Tenso
     """bf16 deq(a) @ deq(b)^T + deq(a2) @ deq(b2)^T: one GEMM whose output tiles accumulate both
     products before they are rounded and written, where the persistent kernel takes the shape;
     otherwise two GEMMs and a bf16 add."""
+    if _operands(a, b, a2, b2):
+        M, N, K = a.rows, b.rows, a.k
+        if a2.rows != M or b2.rows != N or b.k != K or a2.k != K or b2.k != K:
+            raise ValueError("both operand sets must have the same shapes")
+        if not _persistent_shape(M, N, K):
+            return mx_gemm_nt(a, b) + mx_gemm_nt(a2, b2)
+        out = torch.empty((M, N), dtype=torch.bfloat16, device=a.buf.device)
+        _call("mx_gemm_nt_pair_ld", "gemm_nt_pair", out.device, a.codes_ptr, a.scales_ptr, b.codes_ptr, b.scales_ptr,
+              a2.codes_ptr, a2.scales_ptr, b2.codes_ptr, b2.scales_ptr, out.data_ptr(), M, N, K, a.ld, N, _stream(out))
+        return out
     M, K = a.codes.shape
     N = b.codes.shape[0]
     if a2.codes.shape != (M, K) or b2.codes.shape != (N, K) or b.codes.shape[1] != K:
         raise ValueError("both operand sets must have the same shapes")
-    if M <= 128 or N <= 128 or K % 128 or N % 8:
+    if not _persistent_shape(M, N, K):
         return mx_gemm_nt(a, b) + mx_gemm_nt(a2, b2)
     out = torch.empty((M, N), dtype=torch.bfloat16, device=a.codes.device)
     sa, sb, sa2, sb2 = _as_mfma(a), _as_mfma(b), _as_mfma(a2), _as_mfma(b2)  # kept alive over the launch
@@ -717,6 +817,19 @@ def mx_gemm_nt_shared_a(a: MXData, b: MXData, b2: MXData) -> torch.Tensor:
     """bf16 [2, M, N]: deq(a) @ deq(b)^T and deq(a) @ deq(b2)^T.  One launch in which the panels
     of `a` are fetched once for both products where the persistent kernel takes the shape,
     otherwise two GEMMs; bit-identical either way."""
+    if _operands(a, b, b2) and not _watched():
+        M, N, K = a.rows, b.rows, a.k
+        if b2.rows != N or b.k != K or b2.k != K:
+            raise ValueError("both second operands must have the same shape")
+        out = torch.empty((2, M, N), dtype=torch.bfloat16, device=a.buf.device)
+        if not _persistent_shape(M, N, K):
+            _gemm_operands(a, b, out[0])
+            _gemm_operands(a, b2, out[1])
+            return out
+        _call("mx_gemm_nt_shared_a_ld", "gemm_nt_shared_a", out.device, a.codes_ptr, a.scales_ptr, b.codes_ptr,
+              b.scales_ptr, b2.codes_ptr, b2.scales_ptr, out.data_ptr(), out.data_ptr() + 2 * M * N, M, N, K, a.ld, N,
+              _stream(out))
+        return out
     M, K = a.codes.shape
     N = b.codes.shape[0]
     if b2.codes.shape != b.codes.shape or b.codes.shape[1] != K:
@@ -738,6 +851,19 @@ def mx_gemm_nt_shared_a(a: MXData, b: MXData, b2: MXData) -> torch.Tensor:
 def mx_gemm_nt_shared_b(a: MXData, a2: MXData, b: MXData) -> torch.Tensor:
     """bf16 [2, M, N]: deq(a) @ deq(b)^T and deq(a2) @ deq(b)^T, as `mx_gemm_nt_shared_a` with the
     roles of the operands swapped."""
+    if _operands(a, a2, b):
+        M, N, K = a.rows, b.rows, a.k
+        if a2.rows != M or a2.k != K or b.k != K:
+            raise ValueError("both first operands must have the same shape")
+        out = torch.empty((2, M, N), dtype=torch.bfloat16, device=a.buf.device)
+        if not _persistent_shape(M, N, K):
+            _gemm_operands(a, b, out[0])
+            _gemm_operands(a2, b, out[1])
+            return out
+        _call("mx_gemm_nt_shared_b_ld", "gemm_nt_shared_b", out.device, a.codes_ptr, a.scales_ptr, a2.codes_ptr,
+              a2.scales_ptr, b.codes_ptr, b.scales_ptr, out.data_ptr(), out.data_ptr() + 2 * M * N, M, N, K, a.ld, N,
+              _stream(out))
+        return out
     M, K = a.codes.shape
     N = b.codes.shape[0]
     if a2.codes.shape != a.codes.shape or b.codes.shape[1] != K:

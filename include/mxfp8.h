@@ -270,6 +270,16 @@ int mx_token_logprob_bwd(const void* logits, int64_t rows, int64_t vocab, int64_
                          const int64_t* target, const float* lse, const float* grad_logprob,
                          void* dlogits, int64_t ldd, void* stream);
 
+/* The same without the alignment the two ask for (logits at any element, any row stride ld), the
+ * forward with every row cut into `splits` parts by as many workgroups: `partial` holds 2 * rows *
+ * splits floats (may be NULL for splits == 1).  For few rows, which alone do not fill the chip. */
+int mx_token_logprob_fwd_split(const void* logits, int64_t rows, int64_t vocab, int64_t ld,
+                               const int64_t* target, float* logprob, float* lse, int64_t splits,
+                               float* partial, void* stream);
+int mx_token_logprob_bwd_any(const void* logits, int64_t rows, int64_t vocab, int64_t ld,
+                             const int64_t* target, const float* lse, const float* grad_logprob,
+                             void* dlogits, int64_t ldd, void* stream);
+
 /* Re-order a row-major [rows, nblk] scale matrix into MX_SCALES_MFMA order
  * (the "blocked layout" step the reference leaves to torch._scaled_mm, docs/mxfp8.md:36). */
 int mx_scale_layout(const uint8_t* scales, int64_t rows, int64_t nblk, uint8_t* out, void* stream);

@@ -41,6 +41,8 @@ SIGNATURES = {
     "mx_cast_rows_gathered": (c_int, [_P, _P, _P, _I, _I, _I, _I, _P, _P, _P, _P, c_int, c_int, _P]),
     "mx_dequant": (c_int, [_P, _P, _I, _I, c_int, _P, _I, _P]),
     "mx_token_logprob_fwd": (c_int, [_P, _I, _I, _I, _P, _P, _P, _P]),
+    "mx_token_logprob_fwd_split": (c_int, [_P, _I, _I, _I, _P, _P, _P, _I, _P, _P]),
+    "mx_token_logprob_bwd_any": (c_int, [_P, _I, _I, _I, _P, _P, _P, _P, _I, _P]),
     "mx_token_logprob_bwd": (c_int, [_P, _I, _I, _I, _P, _P, _P, _P, _I, _P]),
     "mx_moe_route_plan": (c_int, [_P, _I, _P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P]),
     "mx_moe_combine": (c_int, [_P, _P, _I, _I, _P, _P, _I, _I, _I, _P, _I, _P]),

@@ -473,54 +473,47 @@ def mx_dequant(d: MXData, out: torch.Tensor | None = None) -> torch.Tensor:
     return out
 
 
+def _logprob_splits(rows: int, vocab: int) -> int:
+    """Parts that the forward cuts every row of logits into: enough for one workgroup per CU, none
+    of less than 12 288 logits (a workgroup asks for 16 384 at once; smaller parts cost more in
+    reductions than they spread).  Vocabulary 151 936, uncut against so cut: 16 rows 16.0 -> 7.0 us,
+    64 rows 16.6 -> 9.9, 200 rows 20.1 -> 17.8; 300 rows 25.7 -> 23.8 at best, 457 rows 28.7 -> 30.5."""
+    return max(1, min(-(-256 // rows), vocab // 12288))
+
+
 def token_logprob_fwd(logits: torch.Tensor, target: torch.Tensor):
     """(log-probability of target[r] under softmax(logits[r]), log-sum-exp of row r), float32
     [rows], from bf16 logits [rows, vocab] read once."""
     logits = _check_hp(logits)
     if target.dtype != torch.int64 or target.shape != (logits.shape[0],) or target.device != logits.device:
         raise TypeError("target must be int64 [rows] on the logits' device")
-    if logits.stride(0) % 8 or logits.data_ptr() % 16:
-        logits = logits.contiguous().clone() if logits.shape[1] % 8 == 0 else _pad_row_stride(logits)
     target = target.contiguous()
     rows, vocab = logits.shape
     lp = torch.empty(rows, dtype=torch.float32, device=logits.device)
     lse = torch.empty(rows, dtype=torch.float32, device=logits.device)
-    _call("mx_token_logprob_fwd", "token_logprob_fwd", logits.device, _ptr(logits), rows, vocab,
-          logits.stride(0), _ptr(target), _ptr(lp), _ptr(lse), _stream(logits))
+    splits = _logprob_splits(rows, vocab) if rows else 1
+    partial = torch.empty(2 * rows * splits, dtype=torch.float32, device=logits.device) if splits > 1 else None
+    _call("mx_token_logprob_fwd_split", "token_logprob_fwd", logits.device, _ptr(logits), rows, vocab,
+          logits.stride(0), _ptr(target), _ptr(lp), _ptr(lse), splits, _ptr(partial) if splits > 1 else None,
+          _stream(logits))
     return lp, lse
-
-
-def _pad_row_stride(x: torch.Tensor) -> torch.Tensor:
-    """Copy of x [rows, cols] whose row stride is a multiple of 8 elements (16-byte aligned rows)."""
-    rows, cols = x.shape
-    buf = torch.empty((rows, -(-cols // 8) * 8), dtype=x.dtype, device=x.device)
-    view = buf[:, :cols]
-    view.copy_(x)
-    return view
 
 
 def token_logprob_bwd(logits: torch.Tensor, target: torch.Tensor, lse: torch.Tensor,
                       grad_logprob: torch.Tensor) -> torch.Tensor:
     """Gradient of `token_logprob_fwd`'s first output with respect to the logits, bf16."""
     logits = _check_hp(logits)
-    if logits.stride(0) % 8 or logits.data_ptr() % 16:
-        logits = logits.contiguous().clone() if logits.shape[1] % 8 == 0 else _pad_row_stride(logits)
     rows, vocab = logits.shape
     g = grad_logprob.to(torch.float32).contiguous()
     lse, target = lse.contiguous(), target.contiguous()
     out = torch.empty((rows, -(-vocab // 8) * 8), dtype=torch.bfloat16, device=logits.device)
     if vocab % 8:
         out = out[:, :vocab]
-    step = 65535
-    if rows <= step:
-        _call("mx_token_logprob_bwd", "token_logprob_bwd", logits.device, _ptr(logits), rows, vocab, logits.stride(0),
-              _ptr(target), _ptr(lse), _ptr(g), _ptr(out), out.stride(0), _stream(logits))
-        return out
+    step, ld, ldo = 65535, logits.stride(0), out.stride(0)  # (one grid row per token row)
     for lo in range(0, rows, step):
-        n = min(step, rows - lo)
-        _call("mx_token_logprob_bwd", "token_logprob_bwd", logits.device, _ptr(logits[lo:]), n, vocab,
-              logits.stride(0), _ptr(target[lo:]), _ptr(lse[lo:]), _ptr(g[lo:]), _ptr(out[lo:]),
-              out.stride(0), _stream(logits))
+        _call("mx_token_logprob_bwd_any", "token_logprob_bwd", logits.device, _ptr(logits) + 2 * lo * ld,
+              min(step, rows - lo), vocab, ld, _ptr(target) + 8 * lo, _ptr(lse) + 4 * lo, _ptr(g) + 4 * lo,
+              _ptr(out) + 2 * lo * ldo, ldo, _stream(logits))
     return out
 
 

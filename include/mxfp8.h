@@ -163,6 +163,29 @@ int mx_moe_route_plan(const int32_t* counts, int64_t experts, const int64_t* ord
                       int64_t alignment, int32_t* m_offsets, int64_t* src_row, float* row_score,
                       int64_t* pos, void* stream);
 
+/* Token-choice routing from the router's float32 logits [tokens, experts], in two launches
+ * (torchtitan/models/common/moe/moe.py:137-315, the steps behind the gate).  Scores are the
+ * softmax (or sigmoid) of a token's logits in float32; the top_k experts of largest score + bias
+ * (bias float32 [experts], may be NULL; ties go to the lower number) are written to selected int64
+ * [tokens, top_k] in falling order, their scores -- with norm divided by (their sum + 1e-20) --
+ * times `scale` to top_scores float32 [tokens, top_k]; counts int64 [experts] = pairs per expert;
+ * block_counts int32 [experts * mx_route_blocks(tokens)] = pairs per expert of earlier token
+ * blocks, for mx_route_fill.  experts <= 512, top_k <= 16, else MX_ERR_UNSUPPORTED. */
+int64_t mx_route_blocks(int64_t tokens);
+int mx_route_topk(const float* logits, int64_t tokens, int64_t experts, const float* bias, int64_t top_k,
+                  int softmax, int norm, float scale, float* top_scores, int64_t* selected,
+                  int64_t* counts, int32_t* block_counts, void* stream);
+/* Gradient of top_scores with respect to the logits: dlogits float32 [tokens, experts]. */
+int mx_route_topk_bwd(const float* logits, int64_t tokens, int64_t experts, int64_t top_k, int softmax,
+                      int norm, float scale, const int64_t* selected, const float* dtop, float* dlogits,
+                      void* stream);
+/* The outputs of mx_moe_route_plan from mx_route_topk's, without a sort: within a group the pairs
+ * keep the order of their tokens, which is the order a stable sort by expert gives. */
+int mx_route_fill(const int64_t* selected, const float* scores, int64_t tokens, int64_t top_k,
+                  int64_t experts, const int32_t* block_counts, const int64_t* counts,
+                  int64_t max_len, int64_t alignment, int32_t* m_offsets, int64_t* src_row,
+                  float* row_score, int64_t* pos, void* stream);
+
 /* Combine of the routed expert outputs: out[t, :] = sum_j weights[t, j] * y[pos[t, j], :] for
  * j = 0 .. top_k-1 in that order, in float32 (product and sum rounded separately), result
  * rounded to bf16; weights == NULL gives the plain sum.  y: bf16 [y_rows, cols] (row stride

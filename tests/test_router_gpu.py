@@ -1,0 +1,69 @@
+"""The routing kernels: scores, top-k choice, weights and their gradient against torch in float64, the
+placement of the pairs against the plan from a stable sort."""
+import pytest
+import torch
+
+from torchtitan_amd import ops
+from torchtitan_amd.mx_blocks import mx_route_topk
+
+pytestmark = pytest.mark.gpu
+
+
+def _reference(logits, bias, k, softmax, norm, scale):
+    x = logits.double()
+    s = torch.softmax(x, dim=1) if softmax else torch.sigmoid(x)
+    choice = s if bias is None else s + bias.double()
+    selected = torch.topk(choice, k, dim=1).indices
+    w = s.gather(1, selected)
+    if norm:
+        w = w / (w.sum(dim=1, keepdim=True) + 1e-20)
+    return selected, w * scale, choice
+
+
+# tokens around a workgroup's 16 and a wave's share of it; experts around 64 per register; every k limit
+@pytest.mark.parametrize("tokens,experts,k", [(1, 2, 1), (15, 8, 2), (16, 64, 8), (17, 65, 6), (300, 128, 8),
+                                              (33, 129, 16), (70, 512, 16), (5, 16, 16)])
+@pytest.mark.parametrize("softmax,norm,with_bias", [(True, True, False), (True, False, True), (False, True, True),
+                                                    (False, False, False)])
+def test_routing_against_float64(device, tokens, experts, k, softmax, norm, with_bias):
+    """Weights within 2e-6 (float32 scores and sums of up to 512 terms), the same choice wherever the
+    float64 scores are further than 1e-6 apart, the gradient within 1e-5 of its row's norm."""
+    g = torch.Generator(device=device).manual_seed(tokens + experts + k)
+    logits = (torch.randn((tokens, experts), generator=g, device=device) * 2).requires_grad_(True)
+    bias = torch.randn(experts, generator=g, device=device) * 0.1 if with_bias else None
+    top, selected, counts, _ = mx_route_topk(logits, bias, k, softmax, norm, 1.5)
+    want_sel, want_top, choice = _reference(logits, bias, k, softmax, norm, 1.5)
+    picked = choice.gather(1, selected)
+    assert (picked - choice.gather(1, want_sel)).abs().max() <= 1e-6
+    assert bool((picked[:, :-1] >= picked[:, 1:] - 1e-6).all())
+    assert all(len(set(row)) == k for row in selected.tolist())
+    s = torch.softmax(logits.double(), 1) if softmax else torch.sigmoid(logits.double())
+    w = s.gather(1, selected)
+    w = (w / (w.sum(1, keepdim=True) + 1e-20) if norm else w) * 1.5
+    assert (top.double() - w).abs().max() <= 2e-6
+    assert torch.equal(counts, torch.bincount(selected.flatten(), minlength=experts))
+    dtop = torch.randn((tokens, k), generator=g, device=device)
+    (got,) = torch.autograd.grad(top, logits, dtop)
+    (want,) = torch.autograd.grad(w, logits, dtop.double())
+    assert (got.double() - want).norm() <= 1e-5 * want.norm() + 1e-7
+
+
+def test_equal_scores_go_to_the_lower_experts(device):
+    top, selected, counts, _ = ops.route_topk(torch.zeros((3, 130), device=device), None, 4, True, False, 1.0)
+    assert selected.tolist() == [[0, 1, 2, 3]] * 3 and counts.tolist() == [3] * 4 + [0] * 126
+    assert torch.allclose(top, torch.full((3, 4), 1 / 130, device=device))
+
+
+@pytest.mark.parametrize("tokens,experts,k", [(1, 2, 1), (17, 8, 2), (300, 65, 4), (1000, 128, 8), (40, 300, 16)])
+@pytest.mark.parametrize("alignment,multiple", [(32, 1), (32, 128), (8, 8)])
+def test_plan_equals_the_plan_from_a_stable_sort(device, tokens, experts, k, alignment, multiple):
+    g = torch.Generator(device=device).manual_seed(7 * tokens + experts)
+    # a skewed choice: some experts get most tokens, some none
+    logits = torch.randn((tokens, experts), generator=g, device=device)
+    logits += 2 * torch.randn((1, experts), generator=g, device=device)
+    top, selected, counts, block_counts = ops.route_topk(logits, None, k, False, False, 1.0)
+    got = ops.route_fill(selected, top, counts, block_counts, alignment, multiple)
+    order = torch.argsort(selected.flatten(), stable=True)
+    want = ops.moe_route_plan(counts, order, top.flatten(), k, alignment, multiple)
+    for a, b in zip(got, want):
+        assert torch.equal(a.flatten(), b)

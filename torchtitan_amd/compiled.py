@@ -288,6 +288,48 @@ def _(counts, experts_per_rank, num_ranks, max_len, alignment):
             torch.empty((experts_per_rank,), **i32), torch.empty((experts_per_rank,), **i32))
 
 
+# ----------------------------------------------------------------------------- routing
+@torch.library.custom_op("torchtitan_amd::route_topk", mutates_args=())
+def route_topk(logits: torch.Tensor, bias: torch.Tensor | None, top_k: int, softmax: bool, norm: bool,
+               scale: float) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
+    """``ops.route_topk`` (scores, choice and weights of token-choice routing) as a graph node."""
+    return ops.route_topk(logits, bias, top_k, softmax, norm, scale)
+
+
+@route_topk.register_fake
+def _(logits, bias, top_k, softmax, norm, scale):
+    T, E = logits.shape
+    i64 = dict(dtype=torch.int64, device=logits.device)
+    return (torch.empty((T, top_k), dtype=torch.float32, device=logits.device), torch.empty((T, top_k), **i64),
+            torch.empty((E,), **i64),
+            torch.empty((E * -(-T // ops._ROUTE_TOKENS),), dtype=torch.int32, device=logits.device))
+
+
+@torch.library.custom_op("torchtitan_amd::route_topk_bwd", mutates_args=())
+def route_topk_bwd(logits: torch.Tensor, selected: torch.Tensor, dtop: torch.Tensor, softmax: bool, norm: bool,
+                   scale: float) -> torch.Tensor:
+    return ops.route_topk_bwd(logits, selected, dtop, softmax, norm, scale)
+
+
+@route_topk_bwd.register_fake
+def _(logits, selected, dtop, softmax, norm, scale):
+    return torch.empty_like(logits)
+
+
+def _route_setup(ctx, inputs, output):
+    logits, _, _, softmax, norm, scale = inputs
+    ctx.save_for_backward(logits, output[1])
+    ctx.how = softmax, norm, scale
+
+
+def _route_backward(ctx, dtop, *unused):
+    logits, selected = ctx.saved_tensors
+    return (torch.ops.torchtitan_amd.route_topk_bwd(logits, selected, dtop, *ctx.how), None, None, None, None, None)
+
+
+route_topk.register_autograd(_route_backward, setup_context=_route_setup)
+
+
 # ----------------------------------------------------------------------------- fused blocks
 # The SwiGLU feed-forward block, the expert block and the routed half of an MoE layer as single
 # operators: their bodies are the very functions the eager autograd functions run

@@ -17,8 +17,8 @@ from torch import nn
 
 from dataclasses import dataclass
 
-from ..mx_blocks import (grouped_experts_align_themselves, grouped_feed_forward_fusable,
-                         mx_grouped_feed_forward, mx_routed_experts)
+from ..mx_blocks import (grouped_experts_align_themselves, grouped_feed_forward_fusable, mx_chosen_experts,
+                         mx_grouped_feed_forward, mx_route_topk, mx_routed_experts, route_fusable)
 from ..mx_tensor import grouped_mm
 from ..protocols import Module
 from .feed_forward import FeedForward
@@ -209,8 +209,18 @@ class TokenChoiceTopKRouter(Module):
     def forward(self, x: torch.Tensor, expert_bias: torch.Tensor | None = None):
         """x [tokens, dim] -> (top_scores [tokens, top_k] float32, expert indices [tokens, top_k],
         tokens per expert [num_experts])."""
+        return self.route(x, expert_bias)[:3]
+
+    def route(self, x: torch.Tensor, expert_bias: torch.Tensor | None = None):
+        """`forward`'s outputs and where the pairs of every token block start inside their experts'
+        groups (None unless the routing kernel ran: scores, choice, weights and counts in one)."""
         with torch.autocast(device_type=x.device.type, dtype=torch.float32):
             scores = self.gate(x)
+        if (self.num_expert_groups is None and not self._debug_force_load_balance
+                and self.score_func in ("sigmoid", "softmax") and route_fusable(scores, self.top_k)
+                and (expert_bias is None or expert_bias.dtype == torch.float32)):
+            return mx_route_topk(scores, expert_bias, self.top_k, self.score_func == "softmax", self.route_norm,
+                                 float(self.route_scale))
         if self.score_func == "sigmoid":
             scores = torch.sigmoid(scores)
         elif self.score_func == "softmax":
@@ -231,7 +241,7 @@ class TokenChoiceTopKRouter(Module):
             top_scores = top_scores / (top_scores.sum(dim=-1, keepdim=True) + 1e-20)
         top_scores = top_scores * self.route_scale
         counts = torch.histc(selected.view(-1), bins=self.num_experts, min=0, max=self.num_experts)
-        return top_scores, selected, counts
+        return top_scores, selected, counts, None
 
     def init_weights(self, **kwargs) -> None:
         init_std = kwargs.get("init_std")
@@ -253,6 +263,12 @@ class TokenReorderer(Module):
         counts = torch.histc(flat, bins=self.num_experts, min=0, max=self.num_experts)
         order = torch.argsort(flat, stable=True)
         return top_scores.view(-1)[order], order, counts
+
+
+def _stock(module: nn.Module, cls: type) -> bool:
+    """`module` is a `cls` as it comes, nobody listening to its calls: its work may be done elsewhere."""
+    return type(module) is cls and not (module._forward_hooks or module._forward_pre_hooks
+                                        or module._backward_hooks or module._backward_pre_hooks)
 
 
 class MoE(Module):
@@ -302,16 +318,32 @@ class MoE(Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         bs, slen, dim = x.shape
         x = x.view(-1, dim)
-        top_scores, selected, counts = self.router(x, self.expert_bias)
+        router = self.router
+        if _stock(router, TokenChoiceTopKRouter):
+            top_scores, selected, counts, block_counts = router.route(x, self.expert_bias)
+        else:
+            top_scores, selected, counts = router(x, self.expert_bias)
+            block_counts = None
         with torch.no_grad():
             self.tokens_per_expert.add_(counts)
-        scores_sorted, order, counts = self.reorderer(top_scores, selected)
-        top_k = self.router.top_k
+        top_k = router.top_k
         ex = self.experts
-        if (ex.use_grouped_mm and x.dtype == torch.bfloat16
-                and grouped_feed_forward_fusable(x, ex.w1, ex.w2, ex.w3)
-                and ex.w2.mx_config.pad_token_groups_for_grouped_mm):
-            # converted experts: gather, score, experts and combine as one fused function
+        fused = (ex.use_grouped_mm and x.dtype == torch.bfloat16
+                 and grouped_feed_forward_fusable(x, ex.w1, ex.w2, ex.w3)
+                 and ex.w2.mx_config.pad_token_groups_for_grouped_mm)
+        if (fused and block_counts is not None and _stock(self.reorderer, TokenReorderer)
+                and not torch.compiler.is_compiling()):
+            # converted experts behind the routing kernel: gather, score, experts and combine as one
+            # fused function that places the pairs by their counts
+            out_experts = mx_chosen_experts(x, top_scores, ex.w1, ex.w2, ex.w3, selected, counts, block_counts,
+                                            self.score_before_experts)
+            shared = self.shared_experts(x) if self.shared_experts is not None else None
+            if shared is None:
+                return out_experts.reshape(bs, slen, dim)
+            return (shared + out_experts).reshape(bs, slen, dim)
+        scores_sorted, order, counts = self.reorderer(top_scores, selected)
+        if fused:
+            # the same with the pairs in expert-sorted order
             out_experts = mx_routed_experts(x, top_scores, ex.w1, ex.w2, ex.w3, order, counts,
                                             self.score_before_experts)
             shared = self.shared_experts(x) if self.shared_experts is not None else None

@@ -538,8 +538,10 @@ ROUTED_SAVED = 17
 
 
 def routed_forward(x, top_scores, w1, w2, w3, tok_sorted, counts, score_before: bool, cfg: MXFP8Config,
-                   need_dx: bool, need_ds: bool, need_dw: bool):
-    """Forward of the routed half on x [T, D] (bf16 contiguous): (out [T, D], the ROUTED_SAVED slots)."""
+                   need_dx: bool, need_ds: bool, need_dw: bool, choices=None):
+    """Forward of the routed half on x [T, D] (bf16 contiguous): (out [T, D], the ROUTED_SAVED slots).
+    The pairs come in expert-sorted order (`tok_sorted`) or, with `choices` = (selected experts,
+    `ops.route_topk`'s block counts), as the router chose them."""
     mode = cfg.scale_mode
     T, D = x.shape
     k = top_scores.shape[1]
@@ -547,8 +549,11 @@ def routed_forward(x, top_scores, w1, w2, w3, tok_sorted, counts, score_before: 
     scores = top_scores.float().contiguous()
     order, multiple, _ = grouped_layout(D, H, G)
     # aligned group layout and the maps between padded rows, tokens and (token, j) pairs
-    offs_p, src_row, row_score, pos = ops.moe_route_plan(counts, tok_sorted, scores.view(-1), k, ops.BLOCK, multiple)
-    pos = pos.view(T, k)
+    if choices is not None:
+        offs_p, src_row, row_score, pos = ops.route_fill(choices[0], scores, counts, choices[1], ops.BLOCK, multiple)
+    else:
+        offs_p, src_row, row_score, pos = ops.moe_route_plan(counts, tok_sorted, scores.view(-1), k, ops.BLOCK, multiple)
+        pos = pos.view(T, k)
     xq0, xq1 = ops.to_mx_rows_gathered(x, src_row, mode, order, need_dw, row_score if score_before else None)
     need_dg = need_dx or need_ds or need_dw
     w1q0, w1q1 = _cast_weight(w1, mode, need_dx or need_ds, cfg)
@@ -624,11 +629,11 @@ class _MXRoutedExperts(torch.autograd.Function):
     backward the same two kernels swap roles and the score gradients are row dot products."""
 
     @staticmethod
-    def forward(ctx, x, top_scores, w1, w2, w3, tok_sorted, counts, score_before: bool, cfg: MXFP8Config):
+    def forward(ctx, x, top_scores, w1, w2, w3, tok_sorted, counts, score_before: bool, cfg: MXFP8Config, choices=None):
         need_dx, need_ds = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         need_dw = any(ctx.needs_input_grad[2:5])
         out, saved = routed_forward(_bf16(x).contiguous(), top_scores, w1, w2, w3, tok_sorted, counts, score_before,
-                                    cfg, need_dx, need_ds, need_dw)
+                                    cfg, need_dx, need_ds, need_dw, choices)
         ctx.cfg, ctx.score_before = cfg, score_before
         ctx.order = grouped_layout(x.shape[1], w1.shape[1], w1.shape[0])[0]
         ctx.dtypes = (x.dtype, top_scores.dtype, w1.dtype, w2.dtype, w3.dtype)
@@ -641,7 +646,7 @@ class _MXRoutedExperts(torch.autograd.Function):
         grads = routed_backward(_bf16(dout).contiguous(), list(ctx.saved_tensors), ctx.cfg, ctx.order,
                                 ctx.score_before, need[0], need[1], need[2], need[3], need[4])
         dx, ds, dw1, dw2, dw3 = (g if g is None or g.dtype == dt else g.to(dt) for g, dt in zip(grads, ctx.dtypes))
-        return dx, ds, dw1, dw2, dw3, None, None, None, None
+        return dx, ds, dw1, dw2, dw3, None, None, None, None, None
 
 
 def mx_routed_experts(x: torch.Tensor, top_scores: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor,
@@ -656,6 +661,56 @@ def mx_routed_experts(x: torch.Tensor, top_scores: torch.Tensor, w1: torch.Tenso
         with torch._C.DisableTorchFunctionSubclass():
             return mx_routed_experts_traced(x, top_scores, w1, w2, w3, token_indices_experts_sorted,
                                             num_tokens_per_expert, score_before_experts)
-    return _MXRoutedExperts.apply(x, top_scores, _unwrap(w1), _unwrap(w2), _unwrap(w3),
-                                  token_indices_experts_sorted, num_tokens_per_expert,
-                                  bool(score_before_experts), w2.mx_config)
+    return _routed_experts(x, top_scores, w1, w2, w3, token_indices_experts_sorted, num_tokens_per_expert,
+                           score_before_experts, None)
+
+
+def _routed_experts(x, top_scores, w1, w2, w3, tok_sorted, counts, score_before: bool, choices):
+    with torch._C.DisableTorchFunctionSubclass():
+        return _MXRoutedExperts.apply(x, top_scores, w1, w2, w3, tok_sorted, counts, bool(score_before), w2.mx_config,
+                                      choices)
+
+
+def mx_chosen_experts(x: torch.Tensor, top_scores: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, w3: torch.Tensor,
+                      selected: torch.Tensor, counts: torch.Tensor, block_counts: torch.Tensor,
+                      score_before_experts: bool) -> torch.Tensor:
+    """`mx_routed_experts` straight from the router's choices (`ops.route_topk`'s selected experts, counts
+    and block counts): nothing is sorted.  Eager only."""
+    return _routed_experts(x, top_scores, w1, w2, w3, None, counts, score_before_experts, (selected, block_counts))
+
+
+# ----------------------------------------------------------------------------- routing
+class _RouteTopK(torch.autograd.Function):
+    """(weights, chosen experts, pairs per expert, block counts) of `ops.route_topk`; the gradient of the
+    weights goes back to the logits in one launch."""
+
+    @staticmethod
+    def forward(ctx, logits, bias, top_k: int, softmax: bool, norm: bool, scale: float):
+        top, selected, counts, block_counts = ops.route_topk(logits, bias, top_k, softmax, norm, scale)
+        ctx.mark_non_differentiable(selected, counts, block_counts)
+        ctx.set_materialize_grads(False)
+        ctx.save_for_backward(logits, selected)
+        ctx.how = softmax, norm, scale
+        return top, selected, counts, block_counts
+
+    @staticmethod
+    def backward(ctx, dtop, *_):
+        if dtop is None:
+            return (None,) * 6
+        logits, selected = ctx.saved_tensors
+        return (ops.route_topk_bwd(logits, selected, dtop, *ctx.how), None, None, None, None, None)
+
+
+def route_fusable(logits: torch.Tensor, top_k: int) -> bool:
+    """Routing runs as one kernel for float32 logits on the GPU of at most 512 experts, 16 choices."""
+    return (logits.is_cuda and logits.dtype == torch.float32 and logits.dim() == 2
+            and logits.shape[1] <= ops.ROUTE_MAX_EXPERTS and top_k <= min(ops.ROUTE_MAX_TOP_K, logits.shape[1]))
+
+
+def mx_route_topk(logits: torch.Tensor, bias: torch.Tensor | None, top_k: int, softmax: bool, norm: bool, scale: float):
+    """Scores, choice and weights of token-choice routing.  Callers check `route_fusable` first."""
+    if torch.compiler.is_compiling():
+        from . import compiled
+
+        return torch.ops.torchtitan_amd.route_topk(logits, bias, top_k, softmax, norm, scale)
+    return _RouteTopK.apply(logits, bias, top_k, softmax, norm, scale)

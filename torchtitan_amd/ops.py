@@ -390,10 +390,7 @@ def moe_route_plan(counts: torch.Tensor, order: torch.Tensor, scores: torch.Tens
         if scores.dtype != torch.float32 or scores.numel() != R or scores.device != dev:
             raise TypeError("scores must be float32 with one entry per pair")
         scores = scores.contiguous()
-    step = max(alignment, length_multiple)
-    if step % alignment:
-        raise ValueError("length_multiple must be a multiple of the alignment")
-    max_len = -(-(R + alignment * E) // step) * step
+    max_len = _plan_length(R, E, alignment, length_multiple)
     offs = torch.empty(E, dtype=torch.int32, device=dev)
     src_row = torch.empty(max_len, dtype=torch.int64, device=dev)
     row_score = torch.empty(max_len, dtype=torch.float32, device=dev)
@@ -401,6 +398,67 @@ def moe_route_plan(counts: torch.Tensor, order: torch.Tensor, scores: torch.Tens
     _call("mx_moe_route_plan", "moe_route_plan", dev, _ptr(c32), E, _ptr(order),
           _ptr(scores) if scores is not None else None, R, top_k, max_len, alignment, _ptr(offs),
           _ptr(src_row), _ptr(row_score), _ptr(pos), _stream(counts))
+    return offs, src_row, row_score, pos
+
+
+ROUTE_MAX_EXPERTS = 512
+ROUTE_MAX_TOP_K = 16
+_ROUTE_TOKENS = 16  # tokens of one workgroup (mx_route_blocks)
+
+
+def route_topk(logits: torch.Tensor, bias: torch.Tensor | None, top_k: int, softmax: bool, norm: bool, scale: float):
+    """Token-choice routing from float32 logits [T, E] (`mx_route_topk`): (weights of the chosen experts
+    float32 [T, k], the experts int64 [T, k] in falling order of score + bias, pairs per expert int64
+    [E], and what `route_fill` needs to place the pairs)."""
+    T, E = logits.shape
+    dev = logits.device
+    if logits.dtype != torch.float32 or not logits.is_cuda:
+        raise TypeError("expected float32 logits on the GPU")
+    logits = logits.contiguous()
+    if bias is not None:
+        if bias.dtype != torch.float32 or bias.shape != (E,) or bias.device != dev:
+            raise TypeError("the routing bias must be float32 [experts] on the logits' device")
+        bias = bias.contiguous()
+    top = torch.empty((T, top_k), dtype=torch.float32, device=dev)
+    selected = torch.empty((T, top_k), dtype=torch.int64, device=dev)
+    counts = torch.empty(E, dtype=torch.int64, device=dev)
+    block_counts = torch.empty(E * -(-T // _ROUTE_TOKENS), dtype=torch.int32, device=dev)
+    _call("mx_route_topk", "route_topk", dev, _ptr(logits), T, E, None if bias is None else _ptr(bias), top_k,
+          int(softmax), int(norm), scale, _ptr(top), _ptr(selected), _ptr(counts), _ptr(block_counts), _stream(logits))
+    return top, selected, counts, block_counts
+
+
+def route_topk_bwd(logits: torch.Tensor, selected: torch.Tensor, dtop: torch.Tensor, softmax: bool, norm: bool,
+                   scale: float) -> torch.Tensor:
+    """Gradient of `route_topk`'s weights with respect to the logits, float32 [T, E]."""
+    T, E = logits.shape
+    logits, dtop = logits.contiguous(), dtop.contiguous()
+    out = torch.empty((T, E), dtype=torch.float32, device=logits.device)
+    _call("mx_route_topk_bwd", "route_topk_bwd", logits.device, _ptr(logits), T, E, selected.shape[1], int(softmax),
+          int(norm), scale, _ptr(selected), _ptr(dtop), _ptr(out), _stream(logits))
+    return out
+
+
+def _plan_length(pairs: int, experts: int, alignment: int, length_multiple: int) -> int:
+    step = max(alignment, length_multiple)
+    if step % alignment:
+        raise ValueError("length_multiple must be a multiple of the alignment")
+    return -(-(pairs + alignment * experts) // step) * step
+
+
+def route_fill(selected: torch.Tensor, scores: torch.Tensor, counts: torch.Tensor, block_counts: torch.Tensor,
+               alignment: int, length_multiple: int = 1):
+    """The plan of `moe_route_plan` (same outputs, pos [T, k]) from `route_topk`'s, without a sort."""
+    T, k = selected.shape
+    E, dev = counts.numel(), selected.device
+    max_len = _plan_length(T * k, E, alignment, length_multiple)
+    scores = scores.contiguous()
+    offs = torch.empty(E, dtype=torch.int32, device=dev)
+    src_row = torch.empty(max_len, dtype=torch.int64, device=dev)
+    row_score = torch.empty(max_len, dtype=torch.float32, device=dev)
+    pos = torch.empty((T, k), dtype=torch.int64, device=dev)
+    _call("mx_route_fill", "route_fill", dev, _ptr(selected), _ptr(scores), T, k, E, _ptr(block_counts), _ptr(counts),
+          max_len, alignment, _ptr(offs), _ptr(src_row), _ptr(row_score), _ptr(pos), _stream(selected))
     return offs, src_row, row_score, pos
 
 

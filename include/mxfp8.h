@@ -163,6 +163,17 @@ int mx_moe_route_plan(const int32_t* counts, int64_t experts, const int64_t* ord
                       int64_t alignment, int32_t* m_offsets, int64_t* src_row, float* row_score,
                       int64_t* pos, void* stream);
 
+/* Row-wise casts of n tensors in as few launches as a table of them takes (host arrays of n): tensor i
+ * has elems[i] values (bf16, or float32 rounded to bf16 first where is_f32[i]) in dense rows that are
+ * whole 32-element blocks; codes and row-major scales as mx_cast_dim0 writes them.  What a trainer
+ * hands over for every converted weight
+ * (torchtitan/experiments/rl/unified/actors/trainer.py:226-239).  mx_dequant_many is the way back
+ * (mx_dequant with row-major scales). */
+int mx_cast_rows_many(int64_t n, const void* const* x, const int64_t* elems, const int32_t* is_f32,
+                      uint8_t* const* codes, uint8_t* const* scales, int scale_mode, void* stream);
+int mx_dequant_many(int64_t n, const uint8_t* const* codes, const uint8_t* const* scales,
+                    const int64_t* elems, void* const* out, void* stream);
+
 /* Token-choice routing from the router's float32 logits [tokens, experts], in two launches
  * (torchtitan/models/common/moe/moe.py:137-315, the steps behind the gate).  Scores are the
  * softmax (or sigmoid) of a token's logits in float32; the top_k experts of largest score + bias

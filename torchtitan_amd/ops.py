@@ -6,6 +6,7 @@ call into libmxfp8_gfx950.so.  There is no fallback path: CPU tensors are reject
 from __future__ import annotations
 
 import os
+from ctypes import c_int32, c_int64
 from typing import NamedTuple
 
 import torch
@@ -528,6 +529,57 @@ def mx_dequant(d: MXData, out: torch.Tensor | None = None) -> torch.Tensor:
     scales = d.scales.contiguous()
     _call("mx_dequant", "dequant", codes.device, _ptr(codes), _ptr(scales), rows, cols, d.scale_order,
           _ptr(out), out.stride(0), _stream(codes))
+    return out
+
+
+def _host_table(values, kind):
+    """Host array of 64-bit (pointers, counts) or 32-bit entries for the library's list entry points."""
+    return (kind * len(values))(*values)
+
+
+def to_mx_rows_many(tensors, mode="floor"):
+    """Row-wise `MXData` (codes of the tensor's shape, row-major scales [..., last/32]) of every tensor in the
+    list -- bf16 or float32, one device, last dimension a multiple of 32 -- in one launch."""
+    tensors = [t.contiguous() if t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
+               for t in tensors]
+    if not tensors:
+        return []
+    dev = tensors[0].device
+    out = []
+    for t in tensors:
+        if not t.is_cuda or t.device != dev:
+            raise _lib.MXLibraryError("the MXFP8 kernels run on the GPU only, one device per call")
+        if t.dtype not in (torch.bfloat16, torch.float32):
+            raise TypeError(f"expected bfloat16 or float32, got {t.dtype}")
+        if t.shape[-1] % BLOCK:
+            raise ValueError(f"last dim {t.shape[-1]} is not a multiple of {BLOCK}")
+        out.append(MXData(torch.empty(t.shape, dtype=torch.uint8, device=dev),
+                          torch.empty((*t.shape[:-1], t.shape[-1] // BLOCK), dtype=torch.uint8, device=dev),
+                          MX_SCALES_ROWMAJOR))
+    _call("mx_cast_rows_many", "cast_rows_many", dev, len(out), _host_table([_ptr(t) for t in tensors], c_int64),
+          _host_table([t.numel() for t in tensors], c_int64),
+          _host_table([int(t.dtype == torch.float32) for t in tensors], c_int32),
+          _host_table([_ptr(q.codes) for q in out], c_int64), _host_table([_ptr(q.scales) for q in out], c_int64),
+          _mode(mode), _stream(tensors[0]))
+    return out
+
+
+def mx_dequant_many(data) -> list:
+    """bf16 values of every row-wise `MXData` with row-major scales in the list (any shapes), in one launch."""
+    data = [MXData(q.codes.contiguous(), q.scales.contiguous(), q.scale_order) for q in data]
+    if not data:
+        return []
+    dev = data[0].codes.device
+    for q in data:
+        if q.codes.dtype != torch.uint8 or not q.codes.is_cuda or q.codes.device != dev:
+            raise TypeError("expected uint8 codes on one GPU")
+        if (q.scale_order != MX_SCALES_ROWMAJOR or q.codes.shape[-1] % BLOCK
+                or q.scales.numel() * BLOCK != q.codes.numel()):
+            raise ValueError("expected row-major scales, one per 32 codes of a row")
+    out = [torch.empty(q.codes.shape, dtype=torch.bfloat16, device=dev) for q in data]
+    _call("mx_dequant_many", "dequant_many", dev, len(out), _host_table([_ptr(q.codes) for q in data], c_int64),
+          _host_table([_ptr(q.scales) for q in data], c_int64), _host_table([q.codes.numel() for q in data], c_int64),
+          _host_table([_ptr(t) for t in out], c_int64), _stream(out[0]))
     return out
 
 

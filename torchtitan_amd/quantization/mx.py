@@ -202,27 +202,45 @@ def export_mxfp8_state_dict(model: nn.Module) -> dict:
     from .. import ops
 
     converted = {name: p for name, p in model.named_parameters() if isinstance(p, MXFP8TrainingWeight)}
-    out = {}
-    for name, t in model.state_dict().items():
-        p = converted.get(name)
-        if p is None or not p.is_cuda or p.shape[-1] % 32:
-            out[name] = t
-            continue
-        lead, K = p.shape[:-1], p.shape[-1]
-        with torch.no_grad():
-            w = p.as_subclass(torch.Tensor)
-            rows, _ = _cast_weight(w, p.mx_config.scale_mode, False, p.mx_config)
-        codes = rows.codes
-        n_rows, nblk = int(torch.Size(lead).numel()), K // 32
-        if p.dim() == 3 and p.shape[1] % 128:  # per-matrix scale blocks: undo them one by one
-            per = ops.mfma_scale_bytes(p.shape[1], nblk)
-            scales = torch.stack([ops.scale_unlayout(rows.scales[g * per:(g + 1) * per], p.shape[1], nblk)
-                                  for g in range(p.shape[0])])
-        else:
-            scales = ops.scale_unlayout(rows.scales, n_rows, codes.shape[-1] // 32)[:, :nblk]
-        codes, scales = codes[..., :K].contiguous(), scales.reshape(*lead, nblk)
-        out[name] = {"format": MXFP8_PAYLOAD_FORMAT, "codes": codes.view(*p.shape), "scales": scales, "dtype": p.dtype}
+    with torch._C.DisableTorchFunctionSubclass(), torch.no_grad():
+        out = model.state_dict()
+        out = dict(out)
+        casts = {}
+        fresh: dict = {}  # (device, recipe) -> names of the weights to cast now
+        for name, p in converted.items():
+            if name not in out or not p.is_cuda or p.shape[-1] % 32:
+                continue
+            cfg = p.mx_config
+            if cfg.cache_weight_casts:
+                casts[name] = _rows_from_cache(p, cfg)
+            elif p.dtype in (torch.bfloat16, torch.float32):
+                fresh.setdefault((p.device, cfg.scale_mode), []).append(name)
+            else:
+                casts[name] = ops.to_mx_rows_many([p.to(torch.bfloat16)], cfg.scale_mode)[0]
+        for (_, mode), names in fresh.items():
+            casts.update(zip(names, ops.to_mx_rows_many([converted[n] for n in names], mode)))
+        for name, q in casts.items():
+            out[name] = {"format": MXFP8_PAYLOAD_FORMAT, "codes": q.codes, "scales": q.scales,
+                         "dtype": converted[name].dtype}
     return out
+
+
+def _rows_from_cache(p: torch.Tensor, cfg: MXFP8Config):
+    """Row-wise MXFP8 form of a weight, dense with row-major scales, from its cached cast (made now if there
+    is none)."""
+    from .. import ops
+
+    rows, _ = _cast_weight(p, cfg.scale_mode, False, cfg)
+    codes, laid = rows.codes, rows.scales
+    lead, K = p.shape[:-1], p.shape[-1]
+    nblk = K // 32
+    if p.dim() == 3 and p.shape[1] % 128:  # per-matrix scale blocks: undo them one by one
+        per = ops.mfma_scale_bytes(p.shape[1], nblk)
+        scales = torch.stack([ops.scale_unlayout(laid[g * per:(g + 1) * per], p.shape[1], nblk)
+                              for g in range(p.shape[0])])
+    else:
+        scales = ops.scale_unlayout(laid, int(torch.Size(lead).numel()), codes.shape[-1] // 32)[:, :nblk]
+    return ops.MXData(codes[..., :K].contiguous().view(p.shape), scales.reshape(*lead, nblk), ops.MX_SCALES_ROWMAJOR)
 
 
 def load_mxfp8_state_dict(payload: dict) -> dict:
@@ -232,13 +250,14 @@ def load_mxfp8_state_dict(payload: dict) -> dict:
     from .. import ops
     from ..ops import MX_SCALES_ROWMAJOR, MXData
 
-    out = {}
+    out = dict(payload)
+    here: dict = {}  # device -> names of the MXFP8 entries there
     for name, v in payload.items():
-        if not (isinstance(v, dict) and v.get("format") == MXFP8_PAYLOAD_FORMAT):
-            out[name] = v
-            continue
-        codes, scales = v["codes"], v["scales"]
-        flat = ops.mx_dequant(MXData(codes.reshape(-1, codes.shape[-1]),
-                                     scales.reshape(-1, scales.shape[-1]).contiguous(), MX_SCALES_ROWMAJOR))
-        out[name] = flat.view(codes.shape).to(v["dtype"])
+        if isinstance(v, dict) and v.get("format") == MXFP8_PAYLOAD_FORMAT:
+            here.setdefault(v["codes"].device, []).append(name)
+    for names in here.values():
+        values = ops.mx_dequant_many([MXData(payload[n]["codes"], payload[n]["scales"], MX_SCALES_ROWMAJOR)
+                                      for n in names])
+        for name, t in zip(names, values):
+            out[name] = t.to(payload[name]["dtype"])
     return out

@@ -98,7 +98,8 @@ int mx_cast_dim0_dim1_ld(const void* x, int64_t rows, int64_t cols, int64_t ldx,
  * them written (ld_codes at least that, a multiple of 16), scales in MFMA order for the rounded
  * width.  Column-wise: codes_t likewise over rows rounded up to 128 (rows beyond the matrix count
  * as zeros).  A pair (codes, scales) or (codes_t, scales_t) may be NULL where that form is not
- * needed.  Requires cols % 8 == 0, x 16-byte aligned, ldx % 8 == 0.  Where rows and cols are
+ * needed.  Requires cols % 8 == 0, x with 16-byte aligned rows.  mx_cast_pad takes x in bf16 or, with
+ * x_is_f32, in float32 rounded to bf16 first (nearest even).  Where rows and cols are
  * multiples of 128 the outputs equal mx_cast_dim0_dim1_ld's.  The reference pads activations it
  * cannot cast (torchtitan/models/common/moe/utils.py:65-89) before the cast; dense linears take
  * token counts as they come (torchtitan/models/common/feed_forward.py:61-62).
@@ -106,8 +107,8 @@ int mx_cast_dim0_dim1_ld(const void* x, int64_t rows, int64_t cols, int64_t ldx,
  *   mx_swiglu_bwd_cast_pad  casts of both its gradients    (mx_swiglu_bwd_cast_dim0_dim1_ld; stacked)
  *   mx_rmsnorm_cast_pad     casts of rms_norm(x) * weight  (mx_rmsnorm_cast_dim0_dim1_ld)
  * The last two need both forms, mx_swiglu_cast_pad the row-wise one. */
-int mx_cast_pad(const void* x, int64_t rows, int64_t cols, int64_t ldx, uint8_t* codes,
-                int64_t ld_codes, uint8_t* scales, uint8_t* codes_t, int64_t ld_codes_t,
+int mx_cast_pad(const void* x, int x_is_f32, int64_t rows, int64_t cols, int64_t ldx,
+                uint8_t* codes, int64_t ld_codes, uint8_t* scales, uint8_t* codes_t, int64_t ld_codes_t,
                 uint8_t* scales_t, int scale_mode, void* stream);
 int mx_swiglu_cast_pad(const void* a, const void* b, int64_t rows, int64_t cols, int64_t lda,
                        int64_t ldb, uint8_t* codes, int64_t ld_codes, uint8_t* scales,

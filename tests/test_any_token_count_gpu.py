@@ -60,6 +60,19 @@ def test_operands_hold_the_matrix_and_zeros(device, rows, cols, mode, pad):
     assert torch.equal(ops.to_operands(shifted, mode)[0].codes, by_row.codes)
 
 
+@pytest.mark.parametrize("rows,cols", SIZES)
+def test_float32_input_is_rounded_like_a_conversion(device, rows, cols):
+    x = _values(rows, cols, device, 3).float()
+    x += x.abs() * 2.0 ** -9 * torch.rand_like(x)  # off the bf16 grid, ties and NaN among them
+    x.view(-1)[::7] = x.view(-1)[::7].to(torch.bfloat16).float() * (1 + 2.0 ** -8)
+    if rows * cols > 200:
+        x.view(-1)[::97] = float("nan")
+    for want, got in zip(ops.to_operands(x.to(torch.bfloat16), "rceil"), ops.to_operands(x, "rceil")):
+        assert torch.equal(got.codes, want.codes) and torch.equal(got.scales, want.scales)
+    shifted = torch.zeros(rows * cols + 1, device=device)[1:].view(rows, cols).copy_(x)
+    assert torch.equal(ops.to_operands(shifted, "rceil")[1].codes, want.codes)
+
+
 @pytest.mark.parametrize("mode", ["rceil", "floor"])
 @pytest.mark.parametrize("rows,cols", SIZES)
 def test_gate_and_norm_operands_equal_the_casts_of_their_values(device, rows, cols, mode):

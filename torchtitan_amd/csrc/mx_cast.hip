@@ -507,6 +507,31 @@ __device__ __forceinline__ void load_patch(u32x4 (&v)[8], const uint16_t* src, i
   }
 }
 
+// The same from float32, rounded to bf16 on the way in as a tensor conversion rounds: to nearest even,
+// any NaN to the one quiet NaN.  (An activation or a master weight in float32 otherwise takes a pass of
+// its own, 4 bytes read and 2 written per element, in front of the cast's 2 read and 2 written.)
+__device__ __forceinline__ uint32_t pack_f32(uint32_t lo, uint32_t hi) {
+  const float a = __uint_as_float((lo & 0x7FFFFFFFu) > 0x7F800000u ? 0x7FC00000u : lo);
+  const float b = __uint_as_float((hi & 0x7FFFFFFFu) > 0x7F800000u ? 0x7FC00000u : hi);
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f_t{a, b}, v2bf_t));
+}
+__device__ __forceinline__ void load_patch_f32(u32x4 (&v)[8], const float* src, int64_t ld, bool col_ok,
+                                               int rows_left) {
+  u32x4 w[8][2];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    w[k][0] = w[k][1] = u32x4{0, 0, 0, 0};
+    if (col_ok && k < rows_left) {
+      w[k][0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src + k * ld));
+      w[k][1] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src + k * ld) + 1);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k)
+    v[k] = u32x4{pack_f32(w[k][0].x, w[k][0].y), pack_f32(w[k][0].z, w[k][0].w), pack_f32(w[k][1].x, w[k][1].y),
+                 pack_f32(w[k][1].z, w[k][1].w)};
+}
+
 // Second half of the tile kernel: block maxima, quantization and the stores of one 8 x 8 patch
 // per lane.  Ends with every wave past its reads of the shared staging buffers only after the
 // caller's next barrier.
@@ -667,7 +692,7 @@ struct TileExtras {
 };
 
 // The gate-backward variant is bound by vector ALU work: four workgroups per CU (128 VGPRs).
-template <int MODE, int ORDER, bool ROW, bool COL, int WAVES, int GATE, bool GATHER>
+template <int MODE, int ORDER, bool ROW, bool COL, int WAVES, int GATE, bool GATHER, bool F32 = false>
 __global__ __launch_bounds__(64 * WAVES, GATE == 2 ? 4 : 1) void cast_tile_kernel(
     const uint16_t* __restrict__ x, int64_t rows, int64_t cols, int64_t ldx,
     uint8_t* __restrict__ codes, uint8_t* __restrict__ scales, int64_t nblk, int64_t ks_n,
@@ -716,6 +741,8 @@ __global__ __launch_bounds__(64 * WAVES, GATE == 2 ? 4 : 1) void cast_tile_kerne
   if constexpr (GATHER)
     load_patch_rows(v, x, ldx, c, ex.row_idx + r0 + rl0, ex.src_rows,
                     ex.row_scale ? ex.row_scale + r0 + rl0 : nullptr, col_ok, rows_left);
+  else if constexpr (F32)
+    load_patch_f32(v, reinterpret_cast<const float*>(x) + (r0 + rl0) * ldx + c, ldx, col_ok, rows_left);
   else
     load_patch(v, x + (r0 + rl0) * ldx + c, ldx, col_ok, rows_left);
   if constexpr (GATE == 1) {  // x = gate input a, x3 = b: quantize g = silu(a) * b
@@ -1350,7 +1377,7 @@ int pad_plan(int64_t rows, int64_t cols, const PadOut& o, PadPlan& p) {
   return MX_OK;
 }
 
-template <bool ROW, bool COL, int GATE>
+template <bool ROW, bool COL, int GATE, bool F32 = false>
 int launch_pad(const void* x, int64_t rows, int64_t cols, int64_t ldx, const PadOut& o, const PadPlan& p,
                int scale_mode, hipStream_t st) {
   const int64_t s_b = mfma_scale_bytes(rows, p.nblk), st_b = mfma_scale_bytes(cols, p.nblk_t);
@@ -1360,9 +1387,9 @@ int launch_pad(const void* x, int64_t rows, int64_t cols, int64_t ldx, const Pad
                        (uint32_t)p.gy, p.ex);
   };
   if (scale_mode == MX_SCALE_FLOOR)
-    go(cast_tile_kernel<MX_SCALE_FLOOR, MX_SCALES_MFMA, ROW, COL, MX_CAST_WAVES, GATE, false>);
+    go(cast_tile_kernel<MX_SCALE_FLOOR, MX_SCALES_MFMA, ROW, COL, MX_CAST_WAVES, GATE, false, F32>);
   else
-    go(cast_tile_kernel<MX_SCALE_RCEIL, MX_SCALES_MFMA, ROW, COL, MX_CAST_WAVES, GATE, false>);
+    go(cast_tile_kernel<MX_SCALE_RCEIL, MX_SCALES_MFMA, ROW, COL, MX_CAST_WAVES, GATE, false, F32>);
   return launch_status();
 }
 
@@ -1370,7 +1397,7 @@ bool bad_input(const void* x, int64_t ld) { return ((uintptr_t)x & 15) || (ld & 
 
 }  // namespace
 
-extern "C" int mx_cast_pad(const void* x, int64_t rows, int64_t cols, int64_t ldx, uint8_t* codes,
+extern "C" int mx_cast_pad(const void* x, int x_is_f32, int64_t rows, int64_t cols, int64_t ldx, uint8_t* codes,
                            int64_t ld_codes, uint8_t* scales, uint8_t* codes_t, int64_t ld_codes_t,
                            uint8_t* scales_t, int scale_mode, void* stream) {
   if (rows < 0 || cols < 0 || ldx < cols || bad_enums(scale_mode, MX_SCALES_MFMA)) return MX_ERR_INVALID_ARG;
@@ -1379,8 +1406,13 @@ extern "C" int mx_cast_pad(const void* x, int64_t rows, int64_t cols, int64_t ld
   PadPlan p;
   if (!x) return MX_ERR_INVALID_ARG;
   if (const int rc = pad_plan(rows, cols, o, p)) return rc;
-  if (bad_input(x, ldx)) return MX_ERR_ALIGNMENT;
+  if (bad_input(x, x_is_f32 ? 2 * ldx : ldx)) return MX_ERR_ALIGNMENT;
   hipStream_t st = (hipStream_t)stream;
+  if (x_is_f32) {
+    if (codes && codes_t) return launch_pad<true, true, 0, true>(x, rows, cols, ldx, o, p, scale_mode, st);
+    if (codes) return launch_pad<true, false, 0, true>(x, rows, cols, ldx, o, p, scale_mode, st);
+    return launch_pad<false, true, 0, true>(x, rows, cols, ldx, o, p, scale_mode, st);
+  }
   if (codes && codes_t) return launch_pad<true, true, 0>(x, rows, cols, ldx, o, p, scale_mode, st);
   if (codes) return launch_pad<true, false, 0>(x, rows, cols, ldx, o, p, scale_mode, st);
   return launch_pad<false, true, 0>(x, rows, cols, ldx, o, p, scale_mode, st);

@@ -12,7 +12,7 @@ import torch.nn.functional as F
 
 from . import ops
 from .mx_tensor import (MXFP8Config, MXFP8TrainingWeight, _cast_activation, _cast_cache, _cast_into_groups,
-                        _cast_weight, _grouped_2d3d_padded, _pad_plan, _unwrap)
+                        _cast_weight, _castable, _grouped_2d3d_padded, _pad_plan, _unwrap)
 from .ops import MX_SCALES_MFMA, MX_SCALES_ROWMAJOR, MXData
 
 # ----------------------------------------------------------------------------- SwiGLU + linear
@@ -41,7 +41,7 @@ class _MXSwiGLULinear(torch.autograd.Function):
         need_dh = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
         need_dw = ctx.needs_input_grad[2]
         h1, h3, g_buf, w_buf = ctx.saved_tensors
-        dyq0, dyq1 = ops.to_operands(_bf16(dy.reshape(-1, dy.shape[-1])), mode, need_dh, need_dw)
+        dyq0, dyq1 = ops.to_operands(_castable(_rows_of(dy)), mode, need_dh, need_dw)
         dh1 = dh3 = dw = None
         if need_dh:
             dg = ops.mx_gemm_nt(dyq0, ops.Operand(w_buf, ctx.w_layout)).view(h1.shape)
@@ -230,7 +230,7 @@ class _MXFeedForward(torch.autograd.Function):
         need = ctx.needs_input_grad
         saved = {name: (t if layout is None else ops.Operand(t, layout))
                  for name, t, layout in zip(FFN_SAVED, ctx.saved_tensors, ctx.layouts)}
-        dx, dw1, dw2, dw3, dnw = ffn_backward(_bf16(_rows_of(dy)), saved, ctx.cfg, need[0], need[1], need[2], need[3],
+        dx, dw1, dw2, dw3, dnw = ffn_backward(_castable(_rows_of(dy)), saved, ctx.cfg, need[0], need[1], need[2], need[3],
                                               need[5], pad=ctx.pad, whole_blocks=True)
         cast_back = lambda g, dt: g if g is None or g.dtype == dt else g.to(dt)
         if dx is not None and len(ctx.x_shape) != 2:
@@ -327,7 +327,7 @@ class _MXNormLinears(torch.autograd.Function):
             if dy is None or not (ctx.need_dh or need_dw):
                 dws.append(None)
                 continue
-            dyq0, dyq1 = ops.to_operands(_bf16(dy.reshape(-1, dy.shape[-1])), mode, ctx.need_dh, need_dw)
+            dyq0, dyq1 = ops.to_operands(_castable(_rows_of(dy)), mode, ctx.need_dh, need_dw)
             if ctx.need_dh:
                 part = ops.mx_gemm_nt(dyq0, wqs[i])
                 dh = part if dh is None else dh + part

@@ -102,7 +102,7 @@ def clear_cast_cache() -> None:
 
 
 def _cast_activation(x2: torch.Tensor, src: torch.Tensor, mode: str, need_cols: bool, pitch_pad: int = 0):
-    """(row-wise, column-wise or None) GEMM operands of the 2-D bf16 activation `x2` (any number of
+    """(row-wise, column-wise or None) GEMM operands of the 2-D activation `x2` (any number of
     tokens), remembered for sibling linears that receive the same tensor `src`."""
     key = (mode, pitch_pad)
     hit = _cast_cache.get(src, key)
@@ -174,7 +174,7 @@ def _cast_weight(w: torch.Tensor, mode: str, need_cols: bool, cfg: MXFP8Config, 
         if hit is not None and (hit[1] is not None or not need_cols or w.shape[-2] % ops.BLOCK):
             return hit
         need_cols = True  # cast once in full, whoever asks first
-    wb = (w if w.dtype == torch.bfloat16 else w.to(torch.bfloat16)).contiguous()
+    wb = (_castable(w) if whole else w if w.dtype == torch.bfloat16 else w.to(torch.bfloat16)).contiguous()
     both = need_cols and (whole or wb.shape[-2] % ops.BLOCK == 0)
     if wb.dim() == 3:
         q = ops.to_mx_dim0_dim1_batched(wb, mode, MX_SCALES_MFMA) if both else (_cast_w_rows(wb, mode), None)
@@ -189,12 +189,15 @@ def _cast_weight(w: torch.Tensor, mode: str, need_cols: bool, cfg: MXFP8Config, 
 
 
 # ----------------------------------------------------------------------------- dense linear
+def _castable(t: torch.Tensor) -> torch.Tensor:
+    """`t` in a type the operand casts read: bf16, or float32 which they round to bf16 themselves."""
+    return t if t.dtype in (torch.bfloat16, torch.float32) else t.to(torch.bfloat16)
+
+
 def _linear_forward(x, weight, cfg: MXFP8Config, need_dx: bool, need_dw: bool):
     """(y, column-wise x or None, column-wise W or None) of the converted linear."""
     mode, K, N = cfg.scale_mode, x.shape[-1], weight.shape[0]
-    x2 = x if x.dim() == 2 else x.reshape(-1, K)
-    if x2.dtype != torch.bfloat16:
-        x2 = x2.to(torch.bfloat16)
+    x2 = _castable(x if x.dim() == 2 else x.reshape(-1, K))
     # rows further apart than they are long, except with cached weight casts, which the fused
     # blocks and the hand-over share without a pitch
     pad = 0 if cfg.cache_weight_casts else ops.CODE_PITCH_PAD
@@ -223,9 +226,7 @@ class _MXLinear(torch.autograd.Function):
         mode = ctx.cfg.scale_mode
         need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         x_buf, w_buf = ctx.saved_tensors
-        dy2 = dy if dy.dim() == 2 else dy.reshape(-1, dy.shape[-1])
-        if dy2.dtype != torch.bfloat16:
-            dy2 = dy2.to(torch.bfloat16)
+        dy2 = _castable(dy if dy.dim() == 2 else dy.reshape(-1, dy.shape[-1]))
         pad = 0 if ctx.cfg.cache_weight_casts else ops.CODE_PITCH_PAD
         dyq0, dyq1 = ops.to_operands(dy2, mode, need_dx, need_dw, pad)
         dx = dw = None

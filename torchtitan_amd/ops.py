@@ -180,13 +180,14 @@ def _pitch_ok(pad: int) -> int:
 WHOLE_BLOCK = 128  # depth of the persistent GEMM's K blocks
 
 
-def _operand_input(x: torch.Tensor) -> torch.Tensor:
-    """`x` as the tile casts read it: 16-byte aligned rows (a copy where they are not)."""
-    x = _check_hp(x)
-    cols = x.shape[1]
-    if cols % 8:
-        return torch.nn.functional.pad(x, (0, -cols % 8))
-    if x.stride(0) % 8 or x.data_ptr() % 16:
+def _operand_input(x: torch.Tensor, f32_ok: bool = False) -> torch.Tensor:
+    """`x` as the tile casts read it: 16-byte aligned rows (a copy where they are not); bf16, or float32
+    where the caller's kernel takes it."""
+    if not (f32_ok and x.dtype == torch.float32 and x.is_cuda and x.dim() == 2 and x.stride(1) == 1):
+        x = _check_hp(x)
+    if x.shape[1] % 8:
+        return torch.nn.functional.pad(x, (0, -x.shape[1] % 8))
+    if x.stride(0) * x.element_size() % 16 or x.data_ptr() % 16:
         return x.clone(memory_format=torch.contiguous_format)
     return x
 
@@ -254,17 +255,17 @@ def _new_operand_pair(rows: int, cols: int, pad: int, device):
 
 
 def to_operands(x: torch.Tensor, mode="floor", rows: bool = True, cols: bool = True, pitch_pad: int = 0):
-    """GEMM operands of x [R, C], any R: (row-wise `Operand` or None, column-wise `Operand` or None), each
+    """GEMM operands of x [R, C] (bf16; float32 is rounded to bf16 in the cast), any R: (row-wise `Operand` or None, column-wise `Operand` or None), each
     with its contraction rounded up to a multiple of 128 by zero codes (`mx_cast_pad`) -- codes
     [R, C up to 128] and [C, R up to 128], `pitch_pad` as for `to_mx_dim0_dim1`.  Both operands of a
     product come from here, so that they agree on the rounded contraction."""
     C = x.shape[1]
-    x = _operand_input(x)
+    x = _operand_input(x, f32_ok=True)
     (R, Cx), dev, pad = x.shape, x.device, _pitch_ok(pitch_pad)
     r = _new_operand(R, Cx, pad, dev) if rows else None
     c = _new_operand(Cx, R, pad, dev) if cols else None
     _call("mx_cast_pad", "cast_dim0_dim1" if rows and cols else "cast_dim0" if rows else "cast_dim1", dev,
-          x.data_ptr(), R, Cx, x.stride(0),
+          x.data_ptr(), x.dtype == torch.float32, R, Cx, x.stride(0),
           *((r.codes_ptr, r.ld, r.scales_ptr) if rows else (None, 0, None)),
           *((c.codes_ptr, c.ld, c.scales_ptr) if cols else (None, 0, None)), _mode(mode), _stream(x))
     if cols and Cx != C:

@@ -212,6 +212,14 @@ int mx_moe_combine(const void* y, const void* y2, int64_t y_rows, int64_t ldy, c
                    const float* weights, int64_t tokens, int64_t top_k, int64_t cols, void* out,
                    int64_t ldo, void* stream);
 
+/* mx_moe_combine without y2 and, from the same read of y, the dot products dots[t, j] =
+ * <y[pos[t, j], :], x[t, :]> (float32 [tokens, top_k]; 0 for a position outside y) with x bf16
+ * [tokens, cols] (row stride ldx): the gradients of a token's input and of its routing scores.
+ * out == NULL: the dot products alone.  1 <= top_k <= 16. */
+int mx_moe_combine_dot(const void* y, int64_t y_rows, int64_t ldy, const int64_t* pos, const float* weights,
+                       const void* x, int64_t ldx, int64_t tokens, int64_t top_k, int64_t cols, void* out,
+                       int64_t ldo, float* dots, void* stream);
+
 /* Row dot products out[i] = sum_d a[ia[i], d] * b[ib[i], d] in float32 over bf16 matrices
  * a [a_rows, cols], b [b_rows, cols]; an index outside its matrix gives 0; with a2 (a's shape,
  * may be NULL) a's rows are bf16(a + a2).  The gradient of the

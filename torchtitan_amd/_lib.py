@@ -52,6 +52,7 @@ SIGNATURES = {
     "mx_route_topk_bwd": (c_int, [_P, _I, _I, _I, c_int, c_int, ctypes.c_float, _P, _P, _P, _P]),
     "mx_route_fill": (c_int, [_P, _P, _I, _I, _I, _P, _P, _I, _I, _P, _P, _P, _P, _P]),
     "mx_moe_combine": (c_int, [_P, _P, _I, _I, _P, _P, _I, _I, _I, _P, _I, _P]),
+    "mx_moe_combine_dot": (c_int, [_P, _I, _I, _P, _P, _P, _I, _I, _I, _I, _P, _I, _P, _P]),
     "mx_moe_row_dot": (c_int, [_P, _P, _I, _I, _P, _P, _I, _I, _P, _I, _I, _P, _P]),
     "mx_rmsnorm_cast_dim0_dim1": (c_int, [_P, _P, ctypes.c_float, _I, _I, _I, _P, _P, _P, _P, _P, _P, c_int, c_int, _P]),
     "mx_rmsnorm_cast_dim0_dim1_ld": (c_int, [_P, _P, ctypes.c_float, _I, _I, _I, _P, _P, _P, _I, _P, _P, _I, _P, c_int, c_int, _P]),

@@ -604,16 +604,17 @@ def routed_backward(dout, saved, cfg: MXFP8Config, order: int, score_before: boo
             # gradient of the (scaled) routed inputs, padded layout: the halves from w1 and
             # w3 summed inside one grouped GEMM (float32, one rounding)
             dxp = ops.mx_grouped_gemm_2d3d_pair(da0, w1q1, db0, w3q1, offs_p)
-        if need_dx:
-            dx = ops.moe_combine(dxp, pos, scores if score_before else None)
-        if need_ds:
-            other = saved[16]  # x (scores in front of the experts) or the expert outputs
+        # scores' gradient: products of the rows summed into dx with x, or (scores behind the experts)
+        # of the expert outputs with dout
+        rows, other = (dxp, saved[16]) if score_before else (saved[16], dout)
+        if need_ds and k <= ops.MOE_DOT_MAX_TOP_K:
+            dx, ds = ops.moe_combine_dot(rows, pos, other, scores if score_before else None,
+                                         combine=need_dx and score_before)
+        elif need_ds:
             token = torch.arange(T * k, device=pos.device, dtype=torch.int64).div_(k, rounding_mode="floor")
-            if score_before:
-                ds = ops.moe_row_dot(dxp, pos.view(-1), other, token)
-            else:
-                ds = ops.moe_row_dot(other, pos.view(-1), dout, token)
-            ds = ds.view(T, k)
+            ds = ops.moe_row_dot(rows, pos.view(-1), other, token).view(T, k)
+        if need_dx and dx is None:
+            dx = ops.moe_combine(dxp, pos, scores if score_before else None)
     return dx, ds, dw1, dw2, dw3
 
 

@@ -490,6 +490,32 @@ def moe_combine(y: torch.Tensor, pos: torch.Tensor, weights: torch.Tensor | None
     return out
 
 
+MOE_DOT_MAX_TOP_K = 16  # choices per token whose dot products one wave keeps
+
+
+def moe_combine_dot(y: torch.Tensor, pos: torch.Tensor, x: torch.Tensor, weights: torch.Tensor | None = None,
+                    combine: bool = True):
+    """(`moe_combine(y, pos, weights)`, <y[pos[t, j]], x[t]> as float32 [tokens, top_k]) from one read of
+    y; x: bf16 [tokens, cols].  Without `combine` the first is None.  At most MOE_DOT_MAX_TOP_K choices."""
+    y, x = _check_hp(y), _check_hp(x)
+    if pos.dtype != torch.int64 or pos.dim() != 2 or pos.device != y.device or x.device != y.device:
+        raise TypeError("pos must be a 2-D int64 tensor, and x a tensor, on y's device")
+    T, k = pos.shape
+    if x.shape != (T, y.shape[1]):
+        raise ValueError(f"x must be [{T}, {y.shape[1]}], got {tuple(x.shape)}")
+    pos = pos.contiguous()
+    if weights is not None:
+        if weights.dtype != torch.float32 or weights.shape != pos.shape or weights.device != y.device:
+            raise TypeError("weights must be float32 of pos's shape on y's device")
+        weights = weights.contiguous()
+    out = torch.empty((T, y.shape[1]), dtype=torch.bfloat16, device=y.device) if combine else None
+    dots = torch.empty((T, k), dtype=torch.float32, device=y.device)
+    _call("mx_moe_combine_dot", "moe_combine_dot", y.device, _ptr(y), y.shape[0], y.stride(0), _ptr(pos),
+          _ptr(weights) if weights is not None else None, _ptr(x), x.stride(0), T, k, y.shape[1],
+          _ptr(out) if combine else None, out.stride(0) if combine else 0, _ptr(dots), _stream(y))
+    return out, dots
+
+
 def moe_row_dot(a: torch.Tensor, ia: torch.Tensor, b: torch.Tensor, ib: torch.Tensor,
                 a2: torch.Tensor | None = None) -> torch.Tensor:
     """out[i] = <a[ia[i]], b[ib[i]]> in float32 for bf16 matrices a, b with equal column counts;

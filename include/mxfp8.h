@@ -175,6 +175,21 @@ int mx_cast_rows_many(int64_t n, const void* const* x, const int64_t* elems, con
 int mx_dequant_many(int64_t n, const uint8_t* const* codes, const uint8_t* const* scales,
                     const int64_t* elems, void* const* out, void* stream);
 
+/* The router's gate (torchtitan/models/common/moe/moe.py:258-262, a linear in float32) for bf16 x [tokens,
+ * dim] (row stride ldx) and w [experts, dim] (row stride ldw): logits[t, e] = <x[t], w[e]>, float32 dense.
+ * mx_gate_dx: out = bf16(dlogits w), bf16 [tokens, dim] dense, or with base (bf16, row stride ldb, may be
+ * NULL) bf16(base + that): the sum of two bf16 gradients without a pass of its own.  mx_gate_dw: dw = bf16(dlogits^T x), bf16
+ * [experts, dim] dense, tokens >= 1, through a workspace of mx_gate_dw_workspace bytes.  The products are
+ * those of float32 operands (dlogits enters as three bf16 parts that add up to it).
+ * 8 <= experts <= 128, experts % 8 == 0, dim % 128 == 0, strides % 8 == 0, 16-byte aligned. */
+int mx_gate_logits(const void* x, int64_t ldx, const void* w, int64_t ldw, int64_t tokens, int64_t experts,
+                   int64_t dim, float* logits, void* stream);
+int mx_gate_dx(const float* dlogits, const void* w, int64_t ldw, const void* base, int64_t ldb, int64_t tokens,
+               int64_t experts, int64_t dim, void* out, void* stream);
+int64_t mx_gate_dw_workspace(int64_t tokens, int64_t experts, int64_t dim);
+int mx_gate_dw(const float* dlogits, const void* x, int64_t ldx, int64_t tokens, int64_t experts, int64_t dim,
+               void* workspace, void* dw, void* stream);
+
 /* Token-choice routing from the router's float32 logits [tokens, experts], in two launches
  * (torchtitan/models/common/moe/moe.py:137-315, the steps behind the gate).  Scores are the
  * softmax (or sigmoid) of a token's logits in float32; the top_k experts of largest score + bias

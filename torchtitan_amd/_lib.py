@@ -47,6 +47,10 @@ SIGNATURES = {
     "mx_moe_route_plan": (c_int, [_P, _I, _P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P]),
     "mx_cast_rows_many": (c_int, [_I, _P, _P, _P, _P, _P, c_int, _P]),
     "mx_dequant_many": (c_int, [_I, _P, _P, _P, _P, _P]),
+    "mx_gate_logits": (c_int, [_P, _I, _P, _I, _I, _I, _I, _P, _P]),
+    "mx_gate_dx": (c_int, [_P, _P, _I, _P, _I, _I, _I, _I, _P, _P]),
+    "mx_gate_dw_workspace": (_I, [_I, _I, _I]),
+    "mx_gate_dw": (c_int, [_P, _P, _I, _I, _I, _I, _P, _P, _P]),
     "mx_route_blocks": (_I, [_I]),
     "mx_route_topk": (c_int, [_P, _I, _I, _P, _I, c_int, c_int, ctypes.c_float, _P, _P, _P, _P, _P]),
     "mx_route_topk_bwd": (c_int, [_P, _I, _I, _I, c_int, c_int, ctypes.c_float, _P, _P, _P, _P]),

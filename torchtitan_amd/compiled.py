@@ -289,6 +289,51 @@ def _(counts, experts_per_rank, num_ranks, max_len, alignment):
 
 
 # ----------------------------------------------------------------------------- routing
+@torch.library.custom_op("torchtitan_amd::gate_logits", mutates_args=())
+def gate_logits(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """``ops.gate_logits`` (the router's gate in float32) as a graph node."""
+    return ops.gate_logits(x, weight)
+
+
+@gate_logits.register_fake
+def _(x, weight):
+    return torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float32, device=x.device)
+
+
+@torch.library.custom_op("torchtitan_amd::gate_dx", mutates_args=())
+def gate_dx(dlogits: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    return ops.gate_dx(dlogits, weight)
+
+
+@gate_dx.register_fake
+def _(dlogits, weight):
+    return torch.empty((dlogits.shape[0], weight.shape[1]), dtype=torch.bfloat16, device=weight.device)
+
+
+@torch.library.custom_op("torchtitan_amd::gate_dw", mutates_args=())
+def gate_dw(dlogits: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    return ops.gate_dw(dlogits, x)
+
+
+@gate_dw.register_fake
+def _(dlogits, x):
+    return torch.empty((dlogits.shape[1], x.shape[1]), dtype=torch.bfloat16, device=x.device)
+
+
+def _gate_setup(ctx, inputs, output):
+    ctx.save_for_backward(*inputs)
+
+
+def _gate_backward(ctx, dlogits):
+    x, weight = ctx.saved_tensors
+    dx = torch.ops.torchtitan_amd.gate_dx(dlogits, weight) if ctx.needs_input_grad[0] else None
+    dw = torch.ops.torchtitan_amd.gate_dw(dlogits, x) if ctx.needs_input_grad[1] else None
+    return dx, dw
+
+
+gate_logits.register_autograd(_gate_backward, setup_context=_gate_setup)
+
+
 @torch.library.custom_op("torchtitan_amd::route_topk", mutates_args=())
 def route_topk(logits: torch.Tensor, bias: torch.Tensor | None, top_k: int, softmax: bool, norm: bool,
                scale: float) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:

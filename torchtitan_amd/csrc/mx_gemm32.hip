@@ -1203,6 +1203,13 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   *reinterpret_cast<u32x4*>(d + r * ldd + c) = w;
 }
 
+int launch_splitk_reduce(const float* part, int slices, int64_t M, int64_t N, void* d, int64_t ldd, hipStream_t st) {
+  const int64_t threads = M * (N / 8);
+  hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, part, slices, M,
+                     N, (uint16_t*)d, ldd);
+  return hipGetLastError() == hipSuccess ? MX_OK : MX_ERR_LAUNCH;
+}
+
 // Number of K slices for a dense shape on the persistent kernel (1: no split), from a cost model
 // in microseconds fitted to measurements on MI355X:
 //   one 128-deep block of a 256x256 tile takes a CU 1.6 us with the whole chip busy (about 10 %
@@ -1253,10 +1260,7 @@ int launch_gemm_nt32_splitk(const uint8_t* a_codes, const uint8_t* a_scales, con
   p.ldk = ldk;
   const int rc = launch32<kSplitK, false>(p, tiles * slices, st);
   if (rc != MX_OK) return rc;
-  const int64_t threads = M * (N / 8);
-  hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st,
-                     (const float*)workspace, slices, M, N, (uint16_t*)d, ldd);
-  return hipGetLastError() == hipSuccess ? MX_OK : MX_ERR_LAUNCH;
+  return launch_splitk_reduce((const float*)workspace, slices, M, N, d, ldd, st);
 }
 
 // Grouped forms with every group end a multiple of 32 and all scales in MFMA order

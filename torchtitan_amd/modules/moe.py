@@ -17,8 +17,9 @@ from torch import nn
 
 from dataclasses import dataclass
 
-from ..mx_blocks import (grouped_experts_align_themselves, grouped_feed_forward_fusable, mx_chosen_experts,
-                         mx_grouped_feed_forward, mx_route_topk, mx_routed_experts, route_fusable)
+from ..mx_blocks import (gate_fusable, grouped_experts_align_themselves, grouped_feed_forward_fusable,
+                         mx_chosen_experts, mx_gate, mx_grouped_feed_forward, mx_route_topk, mx_routed_experts,
+                         route_fusable)
 from ..mx_tensor import grouped_mm
 from ..protocols import Module
 from .feed_forward import FeedForward
@@ -211,11 +212,14 @@ class TokenChoiceTopKRouter(Module):
         tokens per expert [num_experts])."""
         return self.route(x, expert_bias)[:3]
 
-    def route(self, x: torch.Tensor, expert_bias: torch.Tensor | None = None):
+    def route(self, x: torch.Tensor, expert_bias: torch.Tensor | None = None, logits: torch.Tensor | None = None):
         """`forward`'s outputs and where the pairs of every token block start inside their experts'
-        groups (None unless the routing kernel ran: scores, choice, weights and counts in one)."""
-        with torch.autocast(device_type=x.device.type, dtype=torch.float32):
-            scores = self.gate(x)
+        groups (None unless the routing kernel ran: scores, choice, weights and counts in one).
+        `logits`: the gate's output, where the caller has it."""
+        scores = logits
+        if scores is None:
+            with torch.autocast(device_type=x.device.type, dtype=torch.float32):
+                scores = self.gate(x)
         if (self.num_expert_groups is None and not self._debug_force_load_balance
                 and self.score_func in ("sigmoid", "softmax") and route_fusable(scores, self.top_k)
                 and (expert_bias is None or expert_bias.dtype == torch.float32)):
@@ -318,19 +322,21 @@ class MoE(Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         bs, slen, dim = x.shape
         x = x.view(-1, dim)
-        router = self.router
+        router, ex = self.router, self.experts
+        fused = (ex.use_grouped_mm and x.dtype == torch.bfloat16
+                 and grouped_feed_forward_fusable(x, ex.w1, ex.w2, ex.w3)
+                 and ex.w2.mx_config.pad_token_groups_for_grouped_mm)
         if _stock(router, TokenChoiceTopKRouter):
-            top_scores, selected, counts, block_counts = router.route(x, self.expert_bias)
+            logits, gate = None, router.gate
+            if fused and _stock(gate, Linear) and gate_fusable(x, gate.weight, gate.bias):
+                logits, x = mx_gate(x, gate.weight)
+            top_scores, selected, counts, block_counts = router.route(x, self.expert_bias, logits)
         else:
             top_scores, selected, counts = router(x, self.expert_bias)
             block_counts = None
         with torch.no_grad():
             self.tokens_per_expert.add_(counts)
         top_k = router.top_k
-        ex = self.experts
-        fused = (ex.use_grouped_mm and x.dtype == torch.bfloat16
-                 and grouped_feed_forward_fusable(x, ex.w1, ex.w2, ex.w3)
-                 and ex.w2.mx_config.pad_token_groups_for_grouped_mm)
         if (fused and block_counts is not None and _stock(self.reorderer, TokenReorderer)
                 and not torch.compiler.is_compiling()):
             # converted experts behind the routing kernel: gather, score, experts and combine as one

@@ -681,6 +681,52 @@ def mx_chosen_experts(x: torch.Tensor, top_scores: torch.Tensor, w1: torch.Tenso
 
 
 # ----------------------------------------------------------------------------- routing
+class _Gate(torch.autograd.Function):
+    """(x W^T in float32, x): the second output is x for whatever else reads the routed tokens, so that the
+    gradient from there comes through this backward and is added where the gate's own is written."""
+
+    @staticmethod
+    def forward(ctx, x, weight, pass_on: bool):
+        ctx.set_materialize_grads(False)
+        ctx.save_for_backward(x, weight)
+        logits = ops.gate_logits(x, weight)
+        return (logits, x) if pass_on else logits
+
+    @staticmethod
+    def backward(ctx, dlogits, dx=None):
+        x, weight = ctx.saved_tensors
+        dw = None
+        if dlogits is not None:
+            if ctx.needs_input_grad[1]:
+                dw = ops.gate_dw(dlogits, x)
+            if ctx.needs_input_grad[0]:
+                dx = ops.gate_dx(dlogits, weight, dx)
+        return dx, dw, None
+
+
+def gate_fusable(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> bool:
+    """The gate runs on its own kernels for plain bf16 tensors on one GPU, no bias, at most 128 experts in
+    whole eights and `dim` in whole 128s; not under a dispatch mode, which would not see them."""
+    return (bias is None and type(weight) in (torch.Tensor, torch.nn.Parameter) and type(x) is torch.Tensor
+            and x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.device == weight.device
+            and x.dim() == 2 and weight.dim() == 2 and x.is_contiguous() and weight.is_contiguous()
+            and x.shape[1] == weight.shape[1] and ops.gate_shape_ok(x.shape[0], weight.shape[0], x.shape[1])
+            and (torch.compiler.is_compiling() or not ops._watched()))
+
+
+def mx_gate(x: torch.Tensor, weight: torch.Tensor):
+    """(float32 logits x W^T, the x that everything behind the gate reads).  Callers check `gate_fusable`."""
+    if torch.compiler.is_compiling():
+        from . import compiled
+
+        return torch.ops.torchtitan_amd.gate_logits(x, weight), x
+    if not torch.is_grad_enabled() or not (x.requires_grad or weight.requires_grad):
+        return ops.gate_logits(x, weight), x
+    if x.requires_grad:
+        return _Gate.apply(x, weight, True)
+    return _Gate.apply(x, weight, False), x
+
+
 class _RouteTopK(torch.autograd.Function):
     """(weights, chosen experts, pairs per expert, block counts) of `ops.route_topk`; the gradient of the
     weights goes back to the logits in one launch."""

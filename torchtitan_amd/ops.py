@@ -408,6 +408,77 @@ ROUTE_MAX_TOP_K = 16
 _ROUTE_TOKENS = 16  # tokens of one workgroup (mx_route_blocks)
 
 
+GATE_MAX_EXPERTS = 128
+
+
+def gate_shape_ok(tokens: int, experts: int, dim: int) -> bool:
+    """The gate kernels' shapes: at most 128 experts in whole eights, `dim` in whole 128s."""
+    return tokens > 0 and 8 <= experts <= GATE_MAX_EXPERTS and experts % 8 == 0 and dim >= 128 and dim % 128 == 0
+
+
+def _gate_rows(t: torch.Tensor) -> torch.Tensor:
+    """bf16 [rows, dim] on the GPU with 16-byte aligned rows (a copy where they are not)."""
+    t = _check_hp(t)
+    return t.clone(memory_format=torch.contiguous_format) if t.stride(0) % 8 or t.data_ptr() % 16 else t
+
+
+def _gate_check(x: torch.Tensor, experts: int, *others: torch.Tensor) -> None:
+    if not gate_shape_ok(x.shape[0], experts, x.shape[1]):
+        raise ValueError(f"no gate kernel for {x.shape[0]} x {x.shape[1]}, {experts} experts")
+    if any(o.device != x.device for o in others):
+        raise ValueError("operands on different devices")
+
+
+def gate_logits(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """float32 [tokens, experts] = x w^T for bf16 x [tokens, dim], w [experts, dim], as a float32 matmul."""
+    x, w = _gate_rows(x), _gate_rows(w)
+    if w.shape[1] != x.shape[1]:
+        raise ValueError(f"column mismatch: {x.shape[1]} vs {w.shape[1]}")
+    _gate_check(x, w.shape[0], w)
+    (T, D), E = x.shape, w.shape[0]
+    logits = torch.empty((T, E), dtype=torch.float32, device=x.device)
+    _call("mx_gate_logits", "gate_logits", x.device, x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), T, E, D,
+          logits.data_ptr(), _stream(x))
+    return logits
+
+
+def _gate_grad(dlogits: torch.Tensor, T: int, E: int) -> torch.Tensor:
+    if dlogits.dtype != torch.float32 or dlogits.shape != (T, E):
+        raise TypeError(f"dlogits must be float32 [{T}, {E}]")
+    dlogits = dlogits.contiguous()
+    return dlogits.clone() if dlogits.data_ptr() % 16 else dlogits
+
+
+def gate_dx(dlogits: torch.Tensor, w: torch.Tensor, base: torch.Tensor | None = None) -> torch.Tensor:
+    """bf16 [tokens, dim] = dlogits w, summed in float32; with `base` (bf16 of that shape) the bf16 sum of both."""
+    w = _gate_rows(w)
+    (E, D), T = w.shape, dlogits.shape[0]
+    dlogits = _gate_grad(dlogits, T, E)
+    if base is not None:
+        base = _gate_rows(base)
+        if base.shape != (T, D):
+            raise ValueError(f"base must be [{T}, {D}]")
+    out = torch.empty((T, D), dtype=torch.bfloat16, device=w.device)
+    _gate_check(out, E, w, dlogits, *(() if base is None else (base,)))
+    _call("mx_gate_dx", "gate_dx", w.device, dlogits.data_ptr(), w.data_ptr(), w.stride(0),
+          None if base is None else base.data_ptr(), 0 if base is None else base.stride(0), T, E, D, out.data_ptr(),
+          _stream(w))
+    return out
+
+
+def gate_dw(dlogits: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """bf16 [experts, dim] = dlogits^T x, summed in float32."""
+    x = _gate_rows(x)
+    (T, D), E = x.shape, dlogits.shape[1]
+    dlogits = _gate_grad(dlogits, T, E)
+    _gate_check(x, E, dlogits)
+    work = torch.empty(_lib.load().mx_gate_dw_workspace(T, E, D), dtype=torch.uint8, device=x.device)
+    out = torch.empty((E, D), dtype=torch.bfloat16, device=x.device)
+    _call("mx_gate_dw", "gate_dw", x.device, dlogits.data_ptr(), x.data_ptr(), x.stride(0), T, E, D, work.data_ptr(),
+          out.data_ptr(), _stream(x))
+    return out
+
+
 def route_topk(logits: torch.Tensor, bias: torch.Tensor | None, top_k: int, softmax: bool, norm: bool, scale: float):
     """Token-choice routing from float32 logits [T, E] (`mx_route_topk`): (weights of the chosen experts
     float32 [T, k], the experts int64 [T, k] in falling order of score + bias, pairs per expert int64

@@ -651,26 +651,39 @@ __device__ __forceinline__ void emit_tile(
 // As load_patch, with the source row of output row r taken from row_idx[r]; an index outside
 // [0, src_rows) (the padding slots of a token-group layout hold -1) reads as a row of zeros.
 // With row_scale, every element of output row r is multiplied by row_scale[r] in float32 and
-// rounded back to bf16 first (the routing-score multiply in front of the experts).
+// rounded back to bf16 first (the routing-score multiply in front of the experts).  All indices and
+// scales are asked for together, then all rows (an index outside reads row 0 and is dropped); the
+// rows come again for every choice of a token, so they are read through the caches.
 __device__ __forceinline__ uint32_t scale2(uint32_t w, float s) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f_t{bf16_lo(w) * s, bf16_hi(w) * s}, v2bf_t));
 }
 __device__ __forceinline__ void load_patch_rows(u32x4 (&v)[8], const uint16_t* x, int64_t ld,
                                                 int64_t c, const int64_t* row_idx, int64_t src_rows,
                                                 const float* row_scale, bool col_ok, int rows_left) {
+  if (!col_ok || rows_left <= 0 || src_rows <= 0) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = u32x4{0, 0, 0, 0};
+    return;
+  }
+  int64_t r[8];
+  float s[8];
+  bool in[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    v[k] = u32x4{0, 0, 0, 0};
-    if (col_ok && k < rows_left) {
-      const int64_t r = row_idx[k];
-      if (r >= 0 && r < src_rows) {
-        v[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(x + r * ld + c));
-        if (row_scale) {
-          const float s = row_scale[k];
-          v[k] = u32x4{scale2(v[k].x, s), scale2(v[k].y, s), scale2(v[k].z, s), scale2(v[k].w, s)};
-        }
-      }
-    }
+    const int at = k < rows_left ? k : 0;
+    r[k] = row_idx[at];
+    s[k] = row_scale ? row_scale[at] : 1.0f;
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    in[k] = k < rows_left && r[k] >= 0 && r[k] < src_rows;
+    v[k] = *reinterpret_cast<const u32x4*>(x + (in[k] ? r[k] : 0) * ld + c);
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    if (row_scale)
+      v[k] = u32x4{scale2(v[k].x, s[k]), scale2(v[k].y, s[k]), scale2(v[k].z, s[k]), scale2(v[k].w, s[k])};
+    if (!in[k]) v[k] = u32x4{0, 0, 0, 0};
   }
 }
 

@@ -143,3 +143,15 @@ def test_feed_forward_over_any_number_of_tokens(device, tokens, dim, hidden):
     got = _step(ff, x, dy)
     for i, (g, w) in enumerate(zip(got, want)):
         assert torch.equal(g, w[:tokens] if i < 2 else w), i
+
+
+# tile counts around the walk's bands of 32 tile rows and strips of 2 (both forms) and of 2 and 32 (rows alone)
+@pytest.mark.parametrize("tile_rows,tile_cols", [(32, 2), (33, 1), (33, 3), (31, 33), (3, 65), (65, 5)])
+def test_every_tile_of_the_walk_is_cast_once(device, tile_rows, tile_cols):
+    rows, cols = 128 * tile_rows - 5, 128 * tile_cols - 32
+    x = _values(rows, cols, device, tile_rows)
+    by_row, by_col = ops.to_operands(x, "rceil")
+    _check(by_row, rows, _zero_padded(x, rows, _up(cols)), "rceil")
+    _check(by_col, cols, _zero_padded(x.t(), cols, _up(rows)).contiguous(), "rceil")
+    only_row, _ = ops.to_operands(x, "rceil", cols=False)
+    assert torch.equal(only_row.codes, by_row.codes) and torch.equal(only_row.scales, by_row.scales)

@@ -436,10 +436,24 @@ __device__ __forceinline__ void quantize_patch(u32x4 (&v)[8], const uint32_t (&m
 #define MX_CAST_COL_BX 2
 #define MX_CAST_COL_BY 32
 #endif
+//
+// Bands of BY tile rows, strips of BX tiles inside a band, down a strip's columns; the last band and
+// the last strip are as high and as wide as the matrix leaves them, so that every workgroup has a tile.
+// (Bands of full height throughout left 33 tile rows with 31 empty workgroups beside every one at
+// work, all of those on the one die that workgroup ids 0 mod 8 go to: both gradient casts of 4099 rows
+// of 6144 took 82 us and take 57 now, 5003 rows 92 and 71.)
 template <bool COL>
 struct TileWalk {
   static constexpr uint32_t BX = COL ? MX_CAST_COL_BX : MX_CAST_ROW_BX;
   static constexpr uint32_t BY = COL ? MX_CAST_COL_BY : MX_CAST_ROW_BY;
+  // tile (bx, by) of a gx x gy grid at place `id` of the walk; id < gx * gy, which fits 31 bits
+  static __device__ __forceinline__ void at(uint32_t id, uint32_t gx, uint32_t gy, uint32_t& bx, uint32_t& by) {
+    const uint32_t band = id / (gx * min(BY, gy));
+    const uint32_t in_band = id - band * (gx * min(BY, gy)), h = min(BY, gy - band * BY);
+    const uint32_t strip = in_band / (BX * h), in = in_band - strip * (BX * h);
+    bx = strip * BX + in / h;
+    by = band * BY + in % h;
+  }
 };
 
 // SwiGLU gate in front of the cast: g = bf16(bf16(silu(a)) * b) per element, each step rounded
@@ -724,13 +738,8 @@ __global__ __launch_bounds__(64 * WAVES, GATE == 2 ? 4 : 1) void cast_tile_kerne
   const int rl0 = wave * 32 + 8 * g;  // first tile-local row of this lane
 
   // a batch of independent [rows, cols] matrices is walked as one stack of gy * batch tile rows
-  constexpr uint32_t BX = TileWalk<COL>::BX, BY = TileWalk<COL>::BY;
-  const uint32_t gy_all = gy * ex.batch;
-  const uint32_t spr = (gx + BX - 1) / BX;
-  const uint32_t sup = blockIdx.x / (BX * BY), in = blockIdx.x % (BX * BY);
-  const uint32_t bx = (sup % spr) * BX + in / BY;
-  const uint32_t by_all = (sup / spr) * BY + in % BY;
-  if (bx >= gx || by_all >= gy_all) return;
+  uint32_t bx, by_all;
+  TileWalk<COL>::at(blockIdx.x, gx, gy * ex.batch, bx, by_all);
   const uint32_t bz = by_all / gy, by = by_all - bz * gy;
   const int64_t ldc = ex.ldc ? ex.ldc : cols, ldct = ex.ldct ? ex.ldct : rows;
   const int64_t cols_out = ex.cols_out ? ex.cols_out : cols, rows_out = ex.rows_out ? ex.rows_out : rows;
@@ -920,13 +929,10 @@ static inline bool tile_ok(const void* x, int64_t cols, int64_t ldx) {
   return ((uintptr_t)x & 15) == 0 && (ldx & 7) == 0 && (cols & 7) == 0;
 }
 constexpr int kTileRows = 32 * MX_CAST_WAVES;
-static inline int64_t tile_grid_x(int64_t gx, int64_t gy, bool col) {
-  const int64_t bx = col ? TileWalk<true>::BX : TileWalk<false>::BX;
-  const int64_t by = col ? TileWalk<true>::BY : TileWalk<false>::BY;
-  return ((gx + bx - 1) / bx) * ((gy + by - 1) / by) * (bx * by);
-}
-static inline dim3 tile_grid(int64_t gx, int64_t gy, int64_t batch, bool col) {
-  return dim3((unsigned)tile_grid_x(gx, gy * batch, col));
+// Workgroups of a tile kernel: one per tile.
+static inline int64_t tile_grid_x(int64_t gx, int64_t gy) { return gx * gy; }
+static inline dim3 tile_grid(int64_t gx, int64_t gy, int64_t batch) {
+  return dim3((unsigned)tile_grid_x(gx, gy * batch));
 }
 static inline TileExtras tile_batch(int64_t batch) {
   TileExtras ex;
@@ -973,9 +979,9 @@ extern "C" int mx_cast_dim0(const void* x, int64_t rows, int64_t cols, int64_t l
   hipStream_t st = (hipStream_t)stream;
   if (scale_order == MX_SCALES_MFMA && ((uintptr_t)scales & 3)) return MX_ERR_ALIGNMENT;
   const int64_t tgx = (cols + kT - 1) / kT, tgy = (rows + kTileRows - 1) / kTileRows;
-  if (scale_order == MX_SCALES_MFMA && tile_grid_x(tgx, tgy, false) <= 0x7FFFFFFF) {
+  if (scale_order == MX_SCALES_MFMA && tile_grid_x(tgx, tgy) <= 0x7FFFFFFF) {
     // scattered scale bytes cost more than the tiled read: stage them through LDS
-    dim3 grid = tile_grid(tgx, tgy, 1, false), block(64 * MX_CAST_WAVES);
+    dim3 grid = tile_grid(tgx, tgy, 1), block(64 * MX_CAST_WAVES);
     MX_DISPATCH_TILE(true, false, 0, false, (const uint16_t*)x, rows, cols, ldx, codes, scales, nblk,
                      ks_n, (uint8_t*)nullptr, (uint8_t*)nullptr, (int64_t)0, (int64_t)0, (int64_t)0,
                      (int64_t)0, (int64_t)0, (uint32_t)tgx, (uint32_t)tgy, TileExtras{});
@@ -1008,8 +1014,8 @@ extern "C" int mx_cast_dim1_batched(const void* x, int64_t batch, int64_t rows, 
   if (gy > 65535 || batch > 65535 || gx > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
   const int64_t tgy = (rows + kTileRows - 1) / kTileRows;
-  if (tile_ok(x, cols, ldx) && tile_grid_x(gx, tgy * batch, true) <= 0x7FFFFFFF) {
-    dim3 grid = tile_grid(gx, tgy, batch, true), block(64 * MX_CAST_WAVES);
+  if (tile_ok(x, cols, ldx) && tile_grid_x(gx, tgy * batch) <= 0x7FFFFFFF) {
+    dim3 grid = tile_grid(gx, tgy, batch), block(64 * MX_CAST_WAVES);
     MX_DISPATCH_TILE(false, true, 0, false, (const uint16_t*)x, rows, cols, ldx, (uint8_t*)nullptr,
                      (uint8_t*)nullptr, (int64_t)0, (int64_t)0, codes_t, scales_t, nblk_t, ks_n_t,
                      rows * ldx, (int64_t)0, st_b, (uint32_t)gx, (uint32_t)tgy,
@@ -1050,8 +1056,8 @@ extern "C" int mx_cast_dim0_dim1_batched(const void* x, int64_t batch, int64_t r
   if (scale_order == MX_SCALES_MFMA && ((uintptr_t)scales & 3)) return MX_ERR_ALIGNMENT;
   const int64_t tgy = (rows + kTileRows - 1) / kTileRows;
   if (tile_ok(x, cols, ldx) && ((uintptr_t)codes & 7) == 0 && ((uintptr_t)scales & 3) == 0 &&
-      tile_grid_x(gx, tgy * batch, true) <= 0x7FFFFFFF) {
-    dim3 grid = tile_grid(gx, tgy, batch, true), block(64 * MX_CAST_WAVES);
+      tile_grid_x(gx, tgy * batch) <= 0x7FFFFFFF) {
+    dim3 grid = tile_grid(gx, tgy, batch), block(64 * MX_CAST_WAVES);
     MX_DISPATCH_TILE(true, true, 0, false, (const uint16_t*)x, rows, cols, ldx, codes, scales, nblk,
                      ks_n, codes_t, scales_t, nblk_t, ks_n_t, rows * ldx, s_b, st_b, (uint32_t)gx,
                      (uint32_t)tgy, tile_batch(batch));
@@ -1091,9 +1097,9 @@ extern "C" int mx_cast_dim0_dim1_ld(const void* x, int64_t rows, int64_t cols, i
   const int64_t nblk_t = rows / 32, ks_n_t = (nblk_t + 1) / 2;
   const int64_t gx = (cols + kT - 1) / kT, tgy = (rows + kTileRows - 1) / kTileRows;
   // only the tile kernel knows pitches: inputs it does not take are the caller's dense cast
-  if (!tile_ok(x, cols, ldx) || tile_grid_x(gx, tgy, true) > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
+  if (!tile_ok(x, cols, ldx) || tile_grid_x(gx, tgy) > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
-  dim3 grid = tile_grid(gx, tgy, 1, true), block(64 * MX_CAST_WAVES);
+  dim3 grid = tile_grid(gx, tgy, 1), block(64 * MX_CAST_WAVES);
   TileExtras ex = tile_batch(1);
   ex.ldc = ld_codes;
   ex.ldct = ld_codes_t;
@@ -1158,9 +1164,9 @@ extern "C" int mx_cast_rows_gathered(const void* x, const int64_t* row_index,
   const int64_t nblk = cols / 32, ks_n = (nblk + 1) / 2;
   const int64_t nblk_t = rows / 32, ks_n_t = (nblk_t + 1) / 2;
   const int64_t gx = (cols + kT - 1) / kT, tgy = (rows + kTileRows - 1) / kTileRows;
-  if (tile_grid_x(gx, tgy, codes_t != nullptr) > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
+  if (tile_grid_x(gx, tgy) > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
-  dim3 grid = tile_grid(gx, tgy, 1, codes_t != nullptr), block(64 * MX_CAST_WAVES);
+  dim3 grid = tile_grid(gx, tgy, 1), block(64 * MX_CAST_WAVES);
   TileExtras ex;
   ex.row_idx = row_index;
   ex.src_rows = src_rows;
@@ -1229,11 +1235,11 @@ extern "C" int mx_rmsnorm_cast_dim0_dim1_ld(const void* x, const void* weight, f
   const int64_t nblk = cols / 32, ks_n = (nblk + 1) / 2;
   const int64_t nblk_t = rows / 32, ks_n_t = (nblk_t + 1) / 2;
   const int64_t gx = (cols + kT - 1) / kT, tgy = (rows + kTileRows - 1) / kTileRows;
-  if (tile_grid_x(gx, tgy, true) > 0x7FFFFFFF || (rows + 3) / 4 > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
+  if (tile_grid_x(gx, tgy) > 0x7FFFFFFF || (rows + 3) / 4 > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
   hipLaunchKernelGGL(rms_rstd_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st,
                      (const uint16_t*)x, rows, cols, ldx, eps, rstd);
-  dim3 grid = tile_grid(gx, tgy, 1, true), block(64 * MX_CAST_WAVES);
+  dim3 grid = tile_grid(gx, tgy, 1), block(64 * MX_CAST_WAVES);
   TileExtras ex;
   ex.x3 = (const uint16_t*)weight;
   ex.g_out = (uint16_t*)y;
@@ -1273,9 +1279,9 @@ extern "C" int mx_swiglu_cast_dim0_dim1_ld(const void* a, const void* b, int64_t
   const int64_t nblk = cols / 32, ks_n = (nblk + 1) / 2;
   const int64_t nblk_t = rows / 32, ks_n_t = (nblk_t + 1) / 2;
   const int64_t gx = (cols + kT - 1) / kT, tgy = (rows + kTileRows - 1) / kTileRows;
-  if (tile_grid_x(gx, tgy, true) > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
+  if (tile_grid_x(gx, tgy) > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
-  dim3 grid = tile_grid(gx, tgy, 1, true), block(64 * MX_CAST_WAVES);
+  dim3 grid = tile_grid(gx, tgy, 1), block(64 * MX_CAST_WAVES);
   TileExtras ex{(const uint16_t*)b, ldb, (uint16_t*)g, nullptr, 0, nullptr, 0};
   ex.ldc = ld_codes;
   ex.ldct = ld_codes_t;
@@ -1316,9 +1322,9 @@ extern "C" int mx_swiglu_bwd_cast_dim0_dim1_ld(const void* dg, const void* a, co
   const int64_t s_b = scale_bytes(rows, nblk, scale_order);
   const int64_t st_b = scale_bytes(cols, nblk_t, scale_order);
   const int64_t gx = (cols + kT - 1) / kT, tgy = (rows + kTileRows - 1) / kTileRows;
-  if (tile_grid_x(gx, tgy, true) > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
+  if (tile_grid_x(gx, tgy) > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
-  dim3 grid = tile_grid(gx, tgy, 1, true), block(64 * MX_CAST_WAVES);
+  dim3 grid = tile_grid(gx, tgy, 1), block(64 * MX_CAST_WAVES);
   TileExtras ex{(const uint16_t*)b, ldb, (uint16_t*)dab, (const uint16_t*)dg, lddg, nullptr, 0};
   ex.ldc = ld_codes;
   ex.ldct = ld_codes_t;
@@ -1379,8 +1385,8 @@ int pad_plan(int64_t rows, int64_t cols, const PadOut& o, PadPlan& p) {
   p.ks_n_t = p.nblk_t / 2;
   p.gx = cols_p / kT;
   p.gy = (rows + kTileRows - 1) / kTileRows;
-  if (tile_grid_x(p.gx, p.gy, o.codes_t != nullptr) > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
-  p.grid = tile_grid(p.gx, p.gy, 1, o.codes_t != nullptr);
+  if (tile_grid_x(p.gx, p.gy) > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
+  p.grid = tile_grid(p.gx, p.gy, 1);
   p.block = dim3(64 * MX_CAST_WAVES);
   p.ex = tile_batch(1);
   p.ex.ldc = o.ld;

@@ -110,6 +110,13 @@ int mx_cast_dim0_dim1_ld(const void* x, int64_t rows, int64_t cols, int64_t ldx,
 int mx_cast_pad(const void* x, int x_is_f32, int64_t rows, int64_t cols, int64_t ldx,
                 uint8_t* codes, int64_t ld_codes, uint8_t* scales, uint8_t* codes_t, int64_t ld_codes_t,
                 uint8_t* scales_t, int scale_mode, void* stream);
+/* Both forms of up to 8 matrices, or stacks of matrices, as mx_cast_pad makes them, in one launch.
+ * table (host memory): n times MX_CAST_PAD_MANY_FIELDS numbers -- x, x_is_f32, matrices in the stack,
+ * rows, cols, ldx, codes, ld_codes, scales, codes_t, ld_codes_t, scales_t.  Matrices of a stack follow
+ * one another without a gap: x after rows * ldx elements, codes after rows * ld_codes bytes, codes_t after
+ * cols * ld_codes_t, scales after the bytes of one matrix' scales in MFMA order. */
+#define MX_CAST_PAD_MANY_FIELDS 12
+int mx_cast_pad_many(int64_t n, const int64_t* table, int scale_mode, void* stream);
 int mx_swiglu_cast_pad(const void* a, const void* b, int64_t rows, int64_t cols, int64_t lda,
                        int64_t ldb, uint8_t* codes, int64_t ld_codes, uint8_t* scales,
                        uint8_t* codes_t, int64_t ld_codes_t, uint8_t* scales_t, int scale_mode,

@@ -155,3 +155,29 @@ def test_every_tile_of_the_walk_is_cast_once(device, tile_rows, tile_cols):
     _check(by_col, cols, _zero_padded(x.t(), cols, _up(rows)).contiguous(), "rceil")
     only_row, _ = ops.to_operands(x, "rceil", cols=False)
     assert torch.equal(only_row.codes, by_row.codes) and torch.equal(only_row.scales, by_row.scales)
+
+
+@pytest.mark.parametrize("mode", ["rceil", "floor"])
+@pytest.mark.parametrize("pad", [0, 128])
+def test_casts_of_a_list_equal_the_single_casts(device, mode, pad):
+    """Matrices of uneven sizes and both types, a stack and an unaligned view in one launch of eight."""
+    tensors = [_values(r, c, device, r) for r, c in [(1, 32), (129, 96), (4225, 128), (300, 264)]]
+    tensors += [_values(257, 160, device, 5).float(), _values(64, 72, device, 6)[:, 4:68]]
+    stacks = [_values(3 * 256, 128, device, 7).view(3, 256, 128), _values(2 * 128, 384, device, 8).view(2, 128, 384)]
+    casts = ops.CastList(mode)
+    got = [casts.add(t, pad) for t in tensors] + [casts.add_stack(t) for t in stacks]
+    assert len(got) == ops.CAST_LIST
+    with pytest.raises(ops._lib.MXLibraryError):
+        casts.add(tensors[0])
+    casts.launch()
+    for t, pair in zip(tensors, got):
+        for q, want in zip(pair, ops.to_operands(t, mode, pitch_pad=pad)):
+            assert torch.equal(q.codes, want.codes) and torch.equal(q.scales, want.scales)
+    for t, pair in zip(stacks, got[len(tensors):]):
+        for q, want in zip(pair, ops.to_mx_dim0_dim1_batched(t, mode)):
+            assert torch.equal(q.codes, want.codes) and torch.equal(q.scales, want.scales)
+    with pytest.raises(ValueError):
+        casts.add_stack(stacks[0][:, :32])
+    q, _ = casts.add_stack(stacks[0].float())
+    casts.launch()
+    assert torch.equal(q.codes, got[len(tensors)][0].codes)

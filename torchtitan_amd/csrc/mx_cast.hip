@@ -840,6 +840,57 @@ __global__ __launch_bounds__(64 * WAVES, GATE == 2 ? 4 : 1) void cast_tile_kerne
                                           rl0, rows_left, tid, wave, lane, ldc, ldct, cols_out, rows_out);
 }
 
+// Both casts of several matrices (stacks) in one launch, as the plain cast_tile_kernel makes them with
+// MFMA-order scales: workgroups from `first` on belong to an entry.  The operands of one product, or
+// the three weights of a SwiGLU block and its input, are independent and mostly small: a launch of its
+// own for each begins and drains the chip each time (2048 x 6144: 18 us where the bytes take 9).
+// HBM-bound, as the single cast.
+constexpr int kCastList = 8;
+struct CastListEntry {
+  const void* x;
+  uint8_t *codes, *scales, *codes_t, *scales_t;
+  int64_t rows, cols, ldx, ldc, ldct;       // per matrix of the stack
+  int64_t x_bstride, s_bstride, st_bstride; // elements / bytes between matrices of the stack
+  uint32_t first, gx, gy, batch, f32, pad;
+};
+struct CastList {
+  CastListEntry e[kCastList];
+};
+
+template <int MODE, bool F32, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void cast_list_kernel(CastList list, int n) {
+  constexpr int TR = 32 * WAVES, TC = 128, PITCH = TR + 16;
+  __shared__ __attribute__((aligned(16))) uint8_t lds_codes[TC * PITCH];
+  __shared__ __attribute__((aligned(16))) uint8_t lds_st[TC * WAVES];
+  __shared__ __attribute__((aligned(16))) uint8_t lds_sr[TR * 4];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, q = lane & 15;
+  const int rl0 = wave * 32 + 8 * g;
+  int at = 0;
+  for (int i = 1; i < n; ++i)
+    if (list.e[i].first <= blockIdx.x) at = i;
+  const CastListEntry& e = list.e[at];
+  uint32_t bx, by_all;
+  TileWalk<true>::at(blockIdx.x - e.first, e.gx, e.gy * e.batch, bx, by_all);
+  const uint32_t bz = by_all / e.gy, by = by_all - bz * e.gy;
+  const int64_t rows = e.rows, cols = e.cols, ldx = e.ldx;
+  const int64_t cols_out = (cols + 127) & ~(int64_t)127, rows_out = (rows + 127) & ~(int64_t)127;
+  const int64_t r0 = (int64_t)by * TR, c0 = (int64_t)bx * TC, c = c0 + 8 * q;
+  const bool col_ok = c < cols;
+  const int64_t left64 = rows - (r0 + rl0);
+  const int rows_left = left64 > 8 ? 8 : (left64 < 0 ? 0 : (int)left64);
+  const int64_t x_at = bz * e.x_bstride + (r0 + rl0) * ldx + c;
+  u32x4 v[8];
+  if (F32 && e.f32)
+    load_patch_f32(v, reinterpret_cast<const float*>(e.x) + x_at, ldx, col_ok, rows_left);
+  else
+    load_patch(v, reinterpret_cast<const uint16_t*>(e.x) + x_at, ldx, col_ok, rows_left);
+  const int64_t nblk = cols_out / 32, nblk_t = rows_out / 32;
+  emit_tile<MODE, MX_SCALES_MFMA, true, true, WAVES>(
+      v, e.codes + bz * rows * e.ldc, e.scales + bz * e.s_bstride, e.codes_t + bz * cols * e.ldct,
+      e.scales_t + bz * e.st_bstride, lds_codes, lds_st, lds_sr, rows, cols, nblk, nblk / 2, nblk_t, nblk_t / 2, r0, c0,
+      c, rl0, rows_left, tid, wave, lane, e.ldc, e.ldct, cols_out, rows_out);
+}
+
 // ------------------------------------------------------------------------------------
 // Scale re-layout (pure byte permutation) and its inverse.
 // ------------------------------------------------------------------------------------
@@ -1435,6 +1486,49 @@ extern "C" int mx_cast_pad(const void* x, int x_is_f32, int64_t rows, int64_t co
   if (codes && codes_t) return launch_pad<true, true, 0>(x, rows, cols, ldx, o, p, scale_mode, st);
   if (codes) return launch_pad<true, false, 0>(x, rows, cols, ldx, o, p, scale_mode, st);
   return launch_pad<false, true, 0>(x, rows, cols, ldx, o, p, scale_mode, st);
+}
+
+extern "C" int mx_cast_pad_many(int64_t n, const int64_t* table, int scale_mode, void* stream) {
+  if (n < 0 || n > kCastList || (n > 0 && !table) || bad_enums(scale_mode, MX_SCALES_MFMA)) return MX_ERR_INVALID_ARG;
+  CastList list;
+  int used = 0;
+  int64_t tiles = 0;
+  bool any_f32 = false;
+  for (int64_t i = 0; i < n; ++i) {
+    const int64_t* t = table + i * MX_CAST_PAD_MANY_FIELDS;
+    const int64_t batch = t[2], rows = t[3], cols = t[4], ldx = t[5];
+    const PadOut o{(uint8_t*)(uintptr_t)t[6], t[7], (uint8_t*)(uintptr_t)t[8],
+                   (uint8_t*)(uintptr_t)t[9], t[10], (uint8_t*)(uintptr_t)t[11]};
+    const void* x = (const void*)(uintptr_t)t[0];
+    const bool f32 = t[1] != 0;
+    if (batch < 0 || rows < 0 || cols < 0 || ldx < cols) return MX_ERR_INVALID_ARG;
+    if (batch == 0 || rows == 0 || cols == 0) continue;
+    if (!x || !o.codes || !o.codes_t) return MX_ERR_INVALID_ARG;
+    PadPlan p;
+    if (const int rc = pad_plan(rows, cols, o, p)) return rc;
+    if (bad_input(x, f32 ? 2 * ldx : ldx)) return MX_ERR_ALIGNMENT;
+    const int64_t mine = p.gx * p.gy;
+    // (32-bit workgroup numbers; the products stay far inside 64 bits)
+    if (mine > 0x7FFFFFFF || batch > 0x7FFFFFFF || mine * batch > 0x7FFFFFFF - tiles) return MX_ERR_UNSUPPORTED;
+    CastListEntry& e = list.e[used++];
+    e = CastListEntry{x, o.codes, o.scales, o.codes_t, o.scales_t, rows, cols, ldx, o.ld, o.ld_t, rows * ldx,
+                      mfma_scale_bytes(rows, p.nblk), mfma_scale_bytes(cols, p.nblk_t), (uint32_t)tiles, (uint32_t)p.gx,
+                      (uint32_t)p.gy, (uint32_t)batch, f32 ? 1u : 0u, 0u};
+    tiles += mine * batch;
+    any_f32 = any_f32 || f32;
+  }
+  if (tiles == 0) return MX_OK;
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(64 * MX_CAST_WAVES), 0, (hipStream_t)stream, list, used);
+  };
+  if (scale_mode == MX_SCALE_FLOOR) {
+    if (any_f32) go(cast_list_kernel<MX_SCALE_FLOOR, true, MX_CAST_WAVES>);
+    else go(cast_list_kernel<MX_SCALE_FLOOR, false, MX_CAST_WAVES>);
+  } else {
+    if (any_f32) go(cast_list_kernel<MX_SCALE_RCEIL, true, MX_CAST_WAVES>);
+    else go(cast_list_kernel<MX_SCALE_RCEIL, false, MX_CAST_WAVES>);
+  }
+  return launch_status();
 }
 
 extern "C" int mx_swiglu_cast_pad(const void* a, const void* b, int64_t rows, int64_t cols, int64_t lda,

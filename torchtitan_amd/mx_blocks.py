@@ -11,8 +11,9 @@ import torch
 import torch.nn.functional as F
 
 from . import ops
-from .mx_tensor import (MXFP8Config, MXFP8TrainingWeight, _cast_activation, _cast_cache, _cast_into_groups,
-                        _cast_weight, _castable, _grouped_2d3d_padded, _pad_plan, _unwrap)
+from .mx_tensor import (MXFP8Config, MXFP8TrainingWeight, _cast_activation, _cast_activation_and_weights,
+                        _cast_cache, _cast_into_groups, _cast_weight, _cast_weights, _castable,
+                        _grouped_2d3d_padded, _pad_plan, _unwrap)
 from .ops import MX_SCALES_MFMA, MX_SCALES_ROWMAJOR, MXData
 
 # ----------------------------------------------------------------------------- SwiGLU + linear
@@ -123,8 +124,8 @@ class _FFNCasts:
         return (ops.to_mx_dim0_dim1(t, self.mode, MX_SCALES_MFMA) if cols
                 else (ops.to_mx_dim0(t, self.mode, MX_SCALES_MFMA), None))
 
-    def weight(self, w, cols: bool):
-        return _cast_weight(w, self.mode, cols, self.cfg, self.pad, self.whole)
+    def weights(self, ws, cols):
+        return _cast_weights(ws, self.mode, cols, self.cfg, self.pad, self.whole)
 
     def gate(self, h13, cols: bool):
         if self.whole:
@@ -151,16 +152,18 @@ def ffn_forward(x2, x_src, w1, w2, w3, cfg: MXFP8Config, need_dx: bool, need_dw:
     the traced operator both run this."""
     cast = _FFNCasts(cfg, whole_blocks, pad)
     rstd = None
+    ws, ws_cols = (w1, w3, w2), (need_dx, need_dx, need_dx or need_dw)
     if norm_weight is not None:  # RMSNorm in front: normalised inside the cast, rstd kept for its backward
         x2 = x2.contiguous()
         xq0, xq1, rstd = cast.norm(x2, norm_weight, eps)
-    elif x_src is not None:
-        xq0, xq1 = _cast_activation(x2, x_src, cfg.scale_mode, need_cols=need_dw, pitch_pad=pad)
+        wqs = cast.weights(ws, ws_cols)
+    elif x_src is not None and need_dx:
+        (xq0, xq1), *wqs = _cast_activation_and_weights(x2, x_src, ws, cfg.scale_mode, need_dx, need_dw, cfg, pad)
     else:
-        xq0, xq1 = cast.plain(x2, need_dw)
-    w1q0, w1q1 = cast.weight(w1, need_dx)
-    w3q0, w3q1 = cast.weight(w3, need_dx)
-    w2q0, w2q1 = cast.weight(w2, need_dx or need_dw)
+        xq0, xq1 = (cast.plain(x2, need_dw) if x_src is None
+                    else _cast_activation(x2, x_src, cfg.scale_mode, need_cols=need_dw, pitch_pad=pad))
+        wqs = cast.weights(ws, ws_cols)
+    (w1q0, w1q1), (w3q0, w3q1), (w2q0, w2q1) = wqs
     h13 = ops.mx_gemm_nt_shared_a(xq0, w1q0, w3q0)  # one launch: x's panels fetched once for both
     gq0, gq1 = cast.gate(h13, need_dw)
     y = ops.mx_gemm_nt(gq0, w2q0)
@@ -423,9 +426,8 @@ def grouped_ffn_forward(x, w1, w2, w3, offs, cfg: MXFP8Config, need_dx: bool, ne
         if T % ops.BLOCK:
             raise ValueError("without padding the token dimension must be a multiple of 32")
     xq0, xq1 = _cast_into_groups(x.contiguous(), perm, mode, order, need_dw)
-    w1q0, w1q1 = _cast_weight(w1, mode, need_dx, cfg)
-    w3q0, w3q1 = _cast_weight(w3, mode, need_dx, cfg)
-    w2q0, w2q1 = _cast_weight(w2, mode, need_dx or need_dw, cfg)
+    (w1q0, w1q1), (w3q0, w3q1), (w2q0, w2q1) = _cast_weights((w1, w3, w2), mode, (need_dx, need_dx, need_dx or need_dw),
+                                                             cfg)
     h13 = ops.mx_grouped_gemm_2d3d_shared_a(xq0, w1q0, w3q0, offs_p)  # one pass over the routed tokens
     gq0, gq1, _ = ops.swiglu_to_mx_dim0_dim1(h13[0], h13[1], mode, order)
     y = _grouped_2d3d_padded(gq0, w2q0, offs_p, back, T)
@@ -556,9 +558,8 @@ def routed_forward(x, top_scores, w1, w2, w3, tok_sorted, counts, score_before: 
         pos = pos.view(T, k)
     xq0, xq1 = ops.to_mx_rows_gathered(x, src_row, mode, order, need_dw, row_score if score_before else None)
     need_dg = need_dx or need_ds or need_dw
-    w1q0, w1q1 = _cast_weight(w1, mode, need_dx or need_ds, cfg)
-    w3q0, w3q1 = _cast_weight(w3, mode, need_dx or need_ds, cfg)
-    w2q0, w2q1 = _cast_weight(w2, mode, need_dg, cfg)
+    need_w = need_dx or need_ds
+    (w1q0, w1q1), (w3q0, w3q1), (w2q0, w2q1) = _cast_weights((w1, w3, w2), mode, (need_w, need_w, need_dg), cfg)
     h13 = ops.mx_grouped_gemm_2d3d_shared_a(xq0, w1q0, w3q0, offs_p)  # one pass over the routed tokens
     gq0, gq1, _ = ops.swiglu_to_mx_dim0_dim1(h13[0], h13[1], mode, order)
     yp = ops.mx_grouped_gemm_2d3d(gq0, w2q0, offs_p)

@@ -188,6 +188,50 @@ def _cast_weight(w: torch.Tensor, mode: str, need_cols: bool, cfg: MXFP8Config, 
     return q
 
 
+def _one_launch(ws, cfg: MXFP8Config, whole_blocks: bool = True) -> bool:
+    """Both forms of all the weights can come from one launch (`ops.CastList`): nothing cached,
+    matrices as whole-block operands or stacks of whole tiles, on one GPU."""
+    if cfg.cache_weight_casts or len({w.device for w in ws}) != 1 or not ws[0].is_cuda:
+        return False
+    if all(w.dim() == 2 for w in ws):
+        return whole_blocks
+    return all(w.dim() == 3 and w.shape[1] % ops.WHOLE_BLOCK == 0 and w.shape[2] % ops.WHOLE_BLOCK == 0 for w in ws)
+
+
+def _list_weights(casts: ops.CastList, ws, mode: str, pitch_pad: int) -> list:
+    wbs = [_castable(w).contiguous() for w in ws]
+    return [casts.add_stack(w) if w.dim() == 3
+            else ops.to_mx_dim0_dim1(w, mode, MX_SCALES_MFMA, pitch_pad, True, cast_list=casts) for w in wbs]
+
+
+def _cast_weights(ws, mode: str, need_cols, cfg: MXFP8Config, pitch_pad: int = 0, whole_blocks: bool = True) -> list:
+    """`_cast_weight` of every weight, `need_cols[i]` for its column-wise form."""
+    if all(need_cols) and _one_launch(ws, cfg, whole_blocks):
+        casts = ops.CastList(mode)
+        q = _list_weights(casts, ws, mode, pitch_pad)
+        casts.launch()
+        return q
+    return [_cast_weight(w, mode, need, cfg, pitch_pad, whole_blocks) for w, need in zip(ws, need_cols)]
+
+
+def _cast_activation_and_weights(x2: torch.Tensor, src: torch.Tensor, ws, mode: str, need_dx: bool, need_dw: bool,
+                                 cfg: MXFP8Config, pitch_pad: int = 0) -> list:
+    """[`_cast_activation` of x2, then `_cast_weight` of every weight] (column-wise forms of the activation
+    with need_dw, of the weights with need_dx), in one launch where both forms of all are wanted."""
+    if need_dx and need_dw and x2.device == ws[0].device and x2.numel() and _one_launch(ws, cfg):
+        key = (mode, pitch_pad)
+        hit = _cast_cache.get(src, key)
+        if hit is None or hit[1] is None:
+            casts = ops.CastList(mode)
+            hit = casts.add(x2, pitch_pad)
+            rest = _list_weights(casts, ws, mode, pitch_pad)
+            casts.launch()
+            _cast_cache.put(src, key, hit)
+            return [hit, *rest]
+    return [_cast_activation(x2, src, mode, need_cols=need_dw, pitch_pad=pitch_pad),
+            *_cast_weights(ws, mode, [need_dx] * len(ws), cfg, pitch_pad)]
+
+
 # ----------------------------------------------------------------------------- dense linear
 def _castable(t: torch.Tensor) -> torch.Tensor:
     """`t` in a type the operand casts read: bf16, or float32 which they round to bf16 themselves."""
@@ -201,8 +245,7 @@ def _linear_forward(x, weight, cfg: MXFP8Config, need_dx: bool, need_dw: bool):
     # rows further apart than they are long, except with cached weight casts, which the fused
     # blocks and the hand-over share without a pitch
     pad = 0 if cfg.cache_weight_casts else ops.CODE_PITCH_PAD
-    xq0, xq1 = _cast_activation(x2, x, mode, need_cols=need_dw, pitch_pad=pad)
-    wq0, wq1 = _cast_weight(weight, mode, need_dx, cfg, pitch_pad=pad)
+    (xq0, xq1), (wq0, wq1) = _cast_activation_and_weights(x2, x, (weight,), mode, need_dx, need_dw, cfg, pad)
     y = ops.mx_gemm_nt(xq0, wq0)
     return (y if x.dim() == 2 else y.view(*x.shape[:-1], N)), xq1, wq1
 

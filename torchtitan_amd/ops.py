@@ -273,6 +273,60 @@ def to_operands(x: torch.Tensor, mode="floor", rows: bool = True, cols: bool = T
     return r, c
 
 
+CAST_LIST = 8  # matrices or stacks that one launch casts
+
+
+class CastList:
+    """Both forms of up to `CAST_LIST` tensors, written by one launch: `add` makes the outputs, `launch`
+    fills them.
+
+    The operands of a product are independent and mostly small, and a launch of its own for each has the
+    chip fill and drain every time."""
+
+    def __init__(self, mode="floor"):
+        self._mode, self._table, self._held, self._device = _mode(mode), [], [], None
+
+    def _entry(self, x, G, R, C, ldx, *outputs):
+        if len(self._held) == CAST_LIST:
+            raise _lib.MXLibraryError(f"a cast list holds {CAST_LIST} tensors")
+        if self._device is None:
+            self._device = x.device
+        elif x.device != self._device:
+            raise _lib.MXLibraryError("a cast list is of one device")
+        self._held.append(x)
+        self._table += (x.data_ptr(), x.dtype == torch.float32, G, R, C, ldx, *outputs)
+
+    def add(self, x: torch.Tensor, pitch_pad: int = 0):
+        """A matrix, bf16 or float32: (row-wise, column-wise) as `to_operands` gives them."""
+        pad, cols = _pitch_ok(pitch_pad), x.shape[1]
+        x = _operand_input(x, f32_ok=True)
+        R, C = x.shape
+        r, c = _new_operand(R, C, pad, x.device), _new_operand(C, R, pad, x.device)
+        self._entry(x, 1, R, C, x.stride(0), r.codes_ptr, r.ld, r.scales_ptr, c.codes_ptr, c.ld, c.scales_ptr)
+        return r, c if C == cols else c.first_rows(cols)
+
+    def add_stack(self, x: torch.Tensor):
+        """A contiguous stack [G, R, C], R and C multiples of 128: (row-wise, column-wise) as
+        `to_mx_dim0_dim1_batched` gives them; float32 is rounded to bf16 in the cast."""
+        if x.dim() != 3 or x.dtype not in (torch.bfloat16, torch.float32) or not x.is_cuda:
+            raise TypeError("expected a 3-D bf16 or float32 GPU tensor")
+        G, R, C = x.shape
+        if R % WHOLE_BLOCK or C % WHOLE_BLOCK or not x.is_contiguous():
+            raise ValueError(f"expected a contiguous stack of whole 128 x 128 tiles, got {tuple(x.shape)}")
+        x = x if x.data_ptr() % 16 == 0 else x.clone()
+        new = lambda *shape: torch.empty(shape, dtype=torch.uint8, device=x.device)
+        r = MXData(new(G, R, C), new(G * R * C // BLOCK), MX_SCALES_MFMA)
+        c = MXData(new(G, C, R), new(G * R * C // BLOCK), MX_SCALES_MFMA)
+        self._entry(x, G, R, C, C, r.codes.data_ptr(), C, r.scales.data_ptr(), c.codes.data_ptr(), R, c.scales.data_ptr())
+        return r, c
+
+    def launch(self) -> None:
+        if self._held:
+            _call("mx_cast_pad_many", "cast_dim0_dim1", self._device, len(self._held), _host_table(self._table, c_int64),
+                  self._mode, _stream(self._held[0]))
+            self._held, self._table, self._device = [], [], None
+
+
 def swiglu_to_operands(a: torch.Tensor, b: torch.Tensor, mode="floor", cols: bool = True, pitch_pad: int = 0):
     """`to_operands` of silu(a) * b (see `swiglu_to_mx_dim0_dim1`), any number of rows."""
     a, b = _operand_input(a), _operand_input(b)
@@ -317,11 +371,16 @@ def rms_norm_to_operands(x: torch.Tensor, weight: torch.Tensor, eps: float, mode
 
 
 def to_mx_dim0_dim1(x: torch.Tensor, mode="floor", order: int = MX_SCALES_ROWMAJOR, pitch_pad: int = 0,
-                    whole_blocks: bool = False):
+                    whole_blocks: bool = False, cast_list: CastList | None = None):
     """Both casts from one read of x; returns (row-wise MXData, column-wise MXData).  With
     `pitch_pad` the rows of both code matrices lie that many bytes further apart than they are
     long (`codes.stride(0)` says so; only `mx_gemm_nt` takes such operands), where the tile kernel
-    takes the input; otherwise the codes are dense.  `whole_blocks`: as `to_operands` gives them."""
+    takes the input; otherwise the codes are dense.  `whole_blocks`: as `to_operands` gives them, with
+    `cast_list` by that list's launch."""
+    if cast_list is not None:
+        if not whole_blocks:
+            raise ValueError("a cast list makes whole-block operands")
+        return cast_list.add(x, pitch_pad)
     if whole_blocks:
         return to_operands(x, mode, True, True, pitch_pad)
     x = _check_hp(x)

@@ -117,6 +117,13 @@ int mx_cast_pad(const void* x, int x_is_f32, int64_t rows, int64_t cols, int64_t
  * cols * ld_codes_t, scales after the bytes of one matrix' scales in MFMA order. */
 #define MX_CAST_PAD_MANY_FIELDS 12
 int mx_cast_pad_many(int64_t n, const int64_t* table, int scale_mode, void* stream);
+/* d[M, N] = mx(x)[M, K] deq(w)[N, K]^T for M <= 32 rows of bf16 x (row stride ldx elements, rows 16-byte
+ * aligned, K % 32 == 0), cast on the way in with the codes and scales of mx_cast_pad; w: codes [N, K rounded
+ * up to 128], rows ldw bytes apart, MFMA-order scales, as mx_cast_pad writes them.  With w2 (else NULL) a second
+ * product of x into d2.  bf16 results, row stride ldd elements. */
+int mx_few_rows(const void* x, int64_t M, int64_t K, int64_t ldx, const uint8_t* w_codes,
+                const uint8_t* w_scales, const uint8_t* w2_codes, const uint8_t* w2_scales, int64_t N,
+                int64_t ldw, void* d, void* d2, int64_t ldd, int scale_mode, void* stream);
 int mx_swiglu_cast_pad(const void* a, const void* b, int64_t rows, int64_t cols, int64_t lda,
                        int64_t ldb, uint8_t* codes, int64_t ld_codes, uint8_t* scales,
                        uint8_t* codes_t, int64_t ld_codes_t, uint8_t* scales_t, int scale_mode,

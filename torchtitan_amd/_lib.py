@@ -33,6 +33,7 @@ SIGNATURES = {
     "mx_cast_dim0_dim1": (c_int, [_P, _I, _I, _I, _P, _P, _P, _P, c_int, c_int, _P]),
     "mx_cast_dim0_dim1_ld": (c_int, [_P, _I, _I, _I, _P, _I, _P, _P, _I, _P, c_int, c_int, _P]),
     "mx_cast_pad_many": (c_int, [_I, _P, c_int, _P]),
+    "mx_few_rows": (c_int, [_P, _I, _I, _I, _P, _P, _P, _P, _I, _I, _P, _P, _I, c_int, _P]),
     "mx_cast_pad": (c_int, [_P, c_int, _I, _I, _I, _P, _I, _P, _P, _I, _P, c_int, _P]),
     "mx_swiglu_cast_pad": (c_int, [_P, _P, _I, _I, _I, _I, _P, _I, _P, _P, _I, _P, c_int, _P]),
     "mx_swiglu_bwd_cast_pad": (c_int, [_P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _P, _P, _I, _P, c_int, _P]),

@@ -245,6 +245,11 @@ def _linear_forward(x, weight, cfg: MXFP8Config, need_dx: bool, need_dw: bool):
     # rows further apart than they are long, except with cached weight casts, which the fused
     # blocks and the hand-over share without a pitch
     pad = 0 if cfg.cache_weight_casts else ops.CODE_PITCH_PAD
+    if not (need_dx or need_dw) and ops.few_rows_ok(x2):
+        wq0, _ = _cast_weight(weight, mode, False, cfg, pitch_pad=pad)
+        if type(wq0) is ops.Operand:  # (a cached cast of a traced forward is dense)
+            y = ops.mx_few_rows(x2, wq0, mode)
+            return (y if x.dim() == 2 else y.view(*x.shape[:-1], N)), None, None
     (xq0, xq1), (wq0, wq1) = _cast_activation_and_weights(x2, x, (weight,), mode, need_dx, need_dw, cfg, pad)
     y = ops.mx_gemm_nt(xq0, wq0)
     return (y if x.dim() == 2 else y.view(*x.shape[:-1], N)), xq1, wq1

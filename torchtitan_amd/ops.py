@@ -957,6 +957,36 @@ def _gemm_operands(a: Operand, b: Operand, out: torch.Tensor) -> torch.Tensor:
     return out
 
 
+FEW_ROWS = 32             # rows that `mx_few_rows` takes
+FEW_ROWS_VALUES = 65536   # values of x, rows counted in whole 16s, up to which it is chosen
+
+
+def few_rows_ok(x: torch.Tensor) -> bool:
+    """`mx_few_rows` runs the products of x: bf16 rows on the GPU in whole blocks of 32, few enough of them,
+    and no dispatch mode that would want to see the GEMM.  Every workgroup casts all of x, so the line is
+    where that costs more than the launch it saves (a cast of its own: 3.7 us on the GPU, about 10 on the
+    host): 16 x 4096 -> 4096 10.7 us in one launch, 3.7 + 7.5 in two; 32 x 2048 -> 6144 12.6, 3.7 + 7.4;
+    32 x 14336 -> 4096 42, 3.8 + 27."""
+    return (x.dtype == torch.bfloat16 and x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= FEW_ROWS
+            and (x.shape[0] + 15 & ~15) * x.shape[1] <= FEW_ROWS_VALUES and x.shape[1] % BLOCK == 0 and x.shape[1] > 0
+            and x.stride(1) == 1 and not _watched())
+
+
+def mx_few_rows(x: torch.Tensor, w: Operand, mode="floor", w2: Operand | None = None) -> torch.Tensor:
+    """bf16 mx(x) @ deq(w)^T with the cast of x inside the product's launch; with `w2` (of w's shape) both
+    products, stacked.  Callers check `few_rows_ok` first."""
+    x = _operand_input(x)
+    (M, K), N = x.shape, w.rows
+    if w.k != -(-K // WHOLE_BLOCK) * WHOLE_BLOCK:
+        raise ValueError(f"contraction mismatch: {K} vs {w.k}")
+    out = torch.empty((M, N) if w2 is None else (2, M, N), dtype=torch.bfloat16, device=x.device)
+    d = out.data_ptr()
+    _call("mx_few_rows", "few_rows", x.device, x.data_ptr(), M, K, x.stride(0), w.codes_ptr, w.scales_ptr,
+          *((None, None) if w2 is None else (w2.codes_ptr, w2.scales_ptr)), N, w.ld, d,
+          None if w2 is None else d + 2 * M * N, N, _mode(mode), _stream(x))
+    return out
+
+
 def _gemm_nt_op(a_codes, a_scales, b_codes, b_scales):
     out = torch.empty((a_codes.shape[0], b_codes.shape[0]), dtype=torch.bfloat16, device=a_codes.device)
     return _gemm_nt_into(a_codes, a_scales, b_codes, b_scales, out)

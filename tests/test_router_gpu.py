@@ -67,3 +67,38 @@ def test_plan_equals_the_plan_from_a_stable_sort(device, tokens, experts, k, ali
     want = ops.moe_route_plan(counts, order, top.flatten(), k, alignment, multiple)
     for a, b in zip(got, want):
         assert torch.equal(a.flatten(), b)
+
+
+@pytest.mark.parametrize("softmax,norm", [(True, True), (True, False), (False, True), (False, False)])
+def test_routing_twice_differentiated_and_transformed(device, softmax, norm):
+    """The gradient of the weights can be differentiated, and transforms take the tensor operations."""
+    from torchtitan_amd import mx_blocks
+
+    g = torch.Generator(device=device).manual_seed(5)
+    logits = torch.randn((7, 16), generator=g, device=device, requires_grad=True)
+    v, u = (torch.randn((7, n), generator=g, device=device) for n in (4, 16))
+    top, selected, *_ = mx_blocks.mx_route_topk(logits, None, 4, softmax, norm, 1.5)
+    plain = mx_blocks._route_weights(logits, selected, softmax, norm, 1.5)
+    second = []
+    for t in (top, plain):
+        (first,) = torch.autograd.grad(t, logits, v, create_graph=True)
+        second.append(torch.autograd.grad(first, logits, u)[0])
+    torch.testing.assert_close(second[0], second[1], rtol=1e-5, atol=1e-6)
+    assert mx_blocks.route_fusable(logits, 4)
+    seen = []
+    torch.func.vmap(lambda t: (seen.append(mx_blocks.route_fusable(t, 4)), t)[1])(logits.detach()[None])
+    with torch.autograd.forward_ad.dual_level():
+        seen.append(mx_blocks.route_fusable(logits, 4))
+    assert seen == [False, False]
+
+
+def test_forward_without_gradients_refuses_tangents(device):
+    """A converted linear has no forward-mode derivative: with gradients off it says so, too."""
+    from torchtitan_amd import mx_tensor
+
+    x = torch.randn((4, 64), device=device, dtype=torch.bfloat16)
+    w = torch.randn((32, 64), device=device, dtype=torch.bfloat16)
+    with torch.no_grad(), torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
+        with pytest.raises(Exception):
+            mx_tensor.mx_linear(dual, w, None, mx_tensor.MXFP8Config())

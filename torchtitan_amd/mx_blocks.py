@@ -277,7 +277,7 @@ def mx_feed_forward(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, w3: tor
 
 def _feed_forward(x, w1, w2, w3, bias2, norm_weight, eps: float):
     with torch._C.DisableTorchFunctionSubclass():
-        if torch.is_grad_enabled():
+        if torch.is_grad_enabled() or ops._transformed():
             y = _MXFeedForward.apply(x, w1, w2, w3, w2.mx_config, norm_weight, eps)
         else:  # nothing is kept for a backward
             y, _ = ffn_forward(_rows_of(x), x, w1, w2, w3, w2.mx_config, False, False, norm_weight, eps,
@@ -702,7 +702,13 @@ class _Gate(torch.autograd.Function):
     def backward(ctx, dlogits, dx=None):
         x, weight = ctx.saved_tensors
         dw = None
-        if dlogits is not None:
+        if dlogits is not None and torch.is_grad_enabled():  # the gradient itself is to be differentiated
+            if ctx.needs_input_grad[1]:
+                dw = (dlogits.t() @ x.float()).to(weight.dtype)
+            if ctx.needs_input_grad[0]:
+                own = (dlogits @ weight.float()).to(x.dtype)
+                dx = own if dx is None else dx + own
+        elif dlogits is not None:
             if ctx.needs_input_grad[1]:
                 dw = ops.gate_dw(dlogits, x)
             if ctx.needs_input_grad[0]:
@@ -717,7 +723,7 @@ def gate_fusable(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | Non
             and x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.device == weight.device
             and x.dim() == 2 and weight.dim() == 2 and x.is_contiguous() and weight.is_contiguous()
             and x.shape[1] == weight.shape[1] and ops.gate_shape_ok(x.shape[0], weight.shape[0], x.shape[1])
-            and (torch.compiler.is_compiling() or not ops._watched()))
+            and (torch.compiler.is_compiling() or not (ops._watched() or ops._transformed())))
 
 
 def mx_gate(x: torch.Tensor, weight: torch.Tensor):
@@ -731,6 +737,15 @@ def mx_gate(x: torch.Tensor, weight: torch.Tensor):
     if x.requires_grad:
         return _Gate.apply(x, weight, True)
     return _Gate.apply(x, weight, False), x
+
+
+def _route_weights(logits, selected, softmax: bool, norm: bool, scale: float):
+    """The weights of `ops.route_topk` for chosen experts, as tensor operations."""
+    scores = torch.softmax(logits, dim=1) if softmax else torch.sigmoid(logits)
+    top = scores.gather(1, selected)
+    if norm:
+        top = top / (top.sum(dim=-1, keepdim=True) + 1e-20)
+    return top * scale
 
 
 class _RouteTopK(torch.autograd.Function):
@@ -751,12 +766,16 @@ class _RouteTopK(torch.autograd.Function):
         if dtop is None:
             return (None,) * 6
         logits, selected = ctx.saved_tensors
+        if torch.is_grad_enabled():  # the gradient itself is to be differentiated
+            top = _route_weights(logits, selected, *ctx.how)
+            return (*torch.autograd.grad(top, logits, dtop, create_graph=True), *(None,) * 5)
         return (ops.route_topk_bwd(logits, selected, dtop, *ctx.how), None, None, None, None, None)
 
 
 def route_fusable(logits: torch.Tensor, top_k: int) -> bool:
-    """Routing runs as one kernel for float32 logits on the GPU of at most 512 experts, 16 choices."""
-    return (logits.is_cuda and logits.dtype == torch.float32 and logits.dim() == 2
+    """Routing runs as one kernel for float32 logits on the GPU of at most 512 experts, 16 choices; not under a
+    function transform or forward-mode AD, for which there are the tensor operations."""
+    return ((torch.compiler.is_compiling() or not ops._transformed()) and logits.is_cuda and logits.dtype == torch.float32 and logits.dim() == 2
             and logits.shape[1] <= ops.ROUTE_MAX_EXPERTS and top_k <= min(ops.ROUTE_MAX_TOP_K, logits.shape[1]))
 
 

@@ -298,7 +298,7 @@ def mx_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, 
     out_dtype = x.dtype
     if torch.is_autocast_enabled(x.device.type):
         out_dtype = torch.get_autocast_dtype(x.device.type)
-    if torch.is_grad_enabled():
+    if torch.is_grad_enabled() or ops._transformed():
         y = _MXLinear.apply(x, weight, cfg)
     else:
         y = _linear_forward(x, weight, cfg, False, False)[0]

@@ -1041,6 +1041,12 @@ def _watched() -> bool:
     return _dispatch_depth is not None and _dispatch_depth() > 0
 
 
+def _transformed() -> bool:
+    """True under a function transform (vmap, jvp, ...) or forward-mode AD: tensors may be wrappers or carry
+    tangents, which a library call would not see."""
+    return torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0
+
+
 def op_sac_save_list() -> set:
     """The dispatcher ops of this package whose outputs a per-op activation-checkpoint policy may
     save (the forward GEMMs): add them to the model's save list

@@ -145,6 +145,19 @@ def test_feed_forward_over_any_number_of_tokens(device, tokens, dim, hidden):
         assert torch.equal(g, w[:tokens] if i < 2 else w), i
 
 
+@pytest.mark.parametrize("tokens", [1, 45, 256])
+@pytest.mark.parametrize("block", ["linear", "ffn"])
+def test_gradients_whose_rows_are_one_expanded_row(device, tokens, block):
+    """The gradient behind a sum over tokens has stride 0 between its rows: the same as written out."""
+    module = Linear.Config().build(in_features=128, out_features=160) if block == "linear" else \
+        FeedForward.Config(hidden_dim=256).build(dim=128)
+    module = _converted(module, device)
+    x, row = _values(tokens, 128, device, 11), _values(1, 160 if block == "linear" else 128, device, 12)
+    dy = row.expand(tokens, -1) if tokens > 1 else row.as_strided(row.shape, (0, 1))
+    for got, want in zip(_step(module, x, dy), _step(module, x, dy.clone(memory_format=torch.contiguous_format))):
+        assert torch.equal(got, want)
+
+
 # tile counts around the walk's bands of 32 tile rows and strips of 2 (both forms) and of 2 and 32 (rows alone)
 @pytest.mark.parametrize("tile_rows,tile_cols", [(32, 2), (33, 1), (33, 3), (31, 33), (3, 65), (65, 5)])
 def test_every_tile_of_the_walk_is_cast_once(device, tile_rows, tile_cols):

@@ -54,6 +54,12 @@ def test_gate_keeps_infinite_gradients(device):
     assert not dx[:3].any() and not dx[4].any() and not dx[6:].any()
 
 
+def test_gate_gradient_onto_an_expanded_row(device):
+    dl, w = torch.randn((40, 8), device=device), torch.randn((8, 128), device=device).bfloat16()
+    base = torch.randn((1, 128), device=device).bfloat16().expand(40, -1)
+    assert torch.equal(ops.gate_dx(dl, w, base), ops.gate_dx(dl, w, base.contiguous()))
+
+
 @pytest.mark.parametrize("change", ["bias", "hook", "float32 weight", "experts", "dim"])
 def test_gate_leaves_other_gates_alone(device, change):
     """Calls that the kernels do not take, or that somebody listens to, go through the gate module."""

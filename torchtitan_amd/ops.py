@@ -187,7 +187,7 @@ def _operand_input(x: torch.Tensor, f32_ok: bool = False) -> torch.Tensor:
         x = _check_hp(x)
     if x.shape[1] % 8:
         return torch.nn.functional.pad(x, (0, -x.shape[1] % 8))
-    if x.stride(0) * x.element_size() % 16 or x.data_ptr() % 16:
+    if x.stride(0) * x.element_size() % 16 or x.data_ptr() % 16 or x.stride(0) < x.shape[1]:  # (expanded rows)
         return x.clone(memory_format=torch.contiguous_format)
     return x
 
@@ -478,7 +478,9 @@ def gate_shape_ok(tokens: int, experts: int, dim: int) -> bool:
 def _gate_rows(t: torch.Tensor) -> torch.Tensor:
     """bf16 [rows, dim] on the GPU with 16-byte aligned rows (a copy where they are not)."""
     t = _check_hp(t)
-    return t.clone(memory_format=torch.contiguous_format) if t.stride(0) % 8 or t.data_ptr() % 16 else t
+    if t.stride(0) % 8 or t.data_ptr() % 16 or t.stride(0) < t.shape[1]:
+        return t.clone(memory_format=torch.contiguous_format)
+    return t
 
 
 def _gate_check(x: torch.Tensor, experts: int, *others: torch.Tensor) -> None:

@@ -262,6 +262,34 @@ def test_permute_indices_host_reference_example():
                              6, 13, 14, 15, -1, -1, -1, -1, 7, 8, 9, 16, 17, 18, 19, -1]
 
 
+@pytest.mark.parametrize("listener", ["global hook", "global pre-hook", "own forward", "compiled call"])
+def test_router_calls_are_seen_by_whoever_listens(listener, monkeypatch):
+    """The router's work is done elsewhere only where nobody could notice: hooks on every module, a
+    replaced forward and a compiled call all still run."""
+    import torch.nn.modules.module as every
+
+    # (torch has no histogram of whole numbers on the CPU)
+    monkeypatch.setattr(torch, "histc", lambda t, bins, min, max: torch.bincount(t, minlength=bins))
+    moe = moe_mod.MoE(moe_mod.MoE.Config(num_experts=4, num_shared_experts=0, hidden_dim=32, top_k=2, use_grouped_mm=False), dim=32)
+    moe.init_weights(init_std=0.02, buffer_device=torch.device("cpu"))
+    router, seen, handle = moe.router, [], None
+    plain = router.forward
+    if listener == "global hook":
+        handle = every.register_module_forward_hook(lambda m, i, o: seen.append(m))
+    elif listener == "global pre-hook":
+        handle = every.register_module_forward_pre_hook(lambda m, i: seen.append(m))
+    elif listener == "own forward":
+        router.forward = lambda *a: (seen.append(router), plain(*a))[1]
+    else:
+        router._compiled_call_impl = lambda *a: (seen.append(router), plain(*a))[1]
+    try:
+        moe(torch.randn(1, 6, 32))
+    finally:
+        if handle is not None:
+            handle.remove()
+    assert any(m is router for m in seen)
+
+
 def test_alignment_switch():
     assert moe_mod.get_mxfp8_pad_multiple() is None
     moe_mod.set_token_group_alignment_size_m(32)

@@ -271,8 +271,11 @@ class TokenReorderer(Module):
 
 def _stock(module: nn.Module, cls: type) -> bool:
     """`module` is a `cls` as it comes, nobody listening to its calls: its work may be done elsewhere."""
-    return type(module) is cls and not (module._forward_hooks or module._forward_pre_hooks
-                                        or module._backward_hooks or module._backward_pre_hooks)
+    every = nn.modules.module
+    return type(module) is cls and "forward" not in vars(module) and module._compiled_call_impl is None and not (
+        module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+        or every._global_forward_hooks or every._global_forward_pre_hooks or every._global_backward_hooks
+        or every._global_backward_pre_hooks)
 
 
 class MoE(Module):

@@ -54,6 +54,17 @@ def test_equal_scores_go_to_the_lower_experts(device):
     assert torch.allclose(top, torch.full((3, 4), 1 / 130, device=device))
 
 
+@pytest.mark.parametrize("sign", [0x7FC00000, 0x7FC00000 - 2 ** 31])
+def test_nan_is_above_every_score(device, sign):
+    """Of either sign, as torch.topk orders it; the rest in falling order behind it."""
+    bias = torch.zeros(70, device=device)
+    bias.view(torch.int32)[66] = sign
+    logits = torch.arange(70, dtype=torch.float32, device=device).mul(0.1).expand(3, 70).contiguous()
+    _, selected, counts, _ = ops.route_topk(logits, bias, 3, False, False, 1.0)
+    assert selected.tolist() == [[66, 69, 68]] * 3 and counts.sum().item() == 9
+    assert torch.topk(torch.sigmoid(logits) + bias, 3, dim=1).indices.tolist() == selected.tolist()
+
+
 @pytest.mark.parametrize("tokens,experts,k", [(1, 2, 1), (17, 8, 2), (300, 65, 4), (1000, 128, 8), (40, 300, 16)])
 @pytest.mark.parametrize("alignment,multiple", [(32, 1), (32, 128), (8, 8)])
 def test_plan_equals_the_plan_from_a_stable_sort(device, tokens, experts, k, alignment, multiple):

@@ -39,8 +39,10 @@ __device__ __forceinline__ float wave_max(float v) {
   }));
 }
 
-// A float as an unsigned number of the same order; never 0, which marks a place that is taken.
+// A float as an unsigned number of the same order, a NaN of either sign above all as torch.topk has it; never 0,
+// which marks a place that is taken.
 __device__ __forceinline__ uint32_t order_key(float f) {
+  if (f != f) return 0xFFFFFFFFu;
   const uint32_t u = __float_as_uint(f);
   const uint32_t k = u ^ ((u >> 31) ? 0xFFFFFFFFu : 0x80000000u);
   return k ? k : 1u;

@@ -34,6 +34,20 @@ def test_log_probs_of_cut_and_unaligned_rows(device, vocab, splits, offset, monk
     assert ((d - exact).abs() <= exact.abs() * 2.0 ** -7 + 1e-6).all()
 
 
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("lo,hi", [(0, 8), (2400, 2408), (4096, 4104), (40000, 40008), (40008, 40011), (0, 40011)])
+def test_nan_logits_are_not_lost(device, lo, hi, splits, monkeypatch):
+    """A lane whose first piece is all NaN, in every place that reads one: the row is NaN, its neighbour
+    is not, and -inf beside the NaN changes nothing."""
+    logits = torch.randn((3, 40011), device=device).to(torch.bfloat16)
+    logits[2] = float("-inf")
+    logits[::2, lo:hi] = float("nan")
+    target = torch.full((3,), 17, device=device)
+    monkeypatch.setattr(ops, "_logprob_splits", lambda r, v: splits)
+    lp, lse = ops.token_logprob_fwd(logits, target)
+    assert lp.isnan().tolist() == [True, False, True] and lse.isnan().tolist() == [True, False, True]
+
+
 def test_parts_follow_the_number_of_rows():
     assert ops._logprob_splits(16, 151936) == 12 and ops._logprob_splits(64, 151936) == 4
     assert ops._logprob_splits(256, 151936) == 1 and ops._logprob_splits(16, 8192) == 1

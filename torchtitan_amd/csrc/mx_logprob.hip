@@ -20,12 +20,12 @@ __device__ __forceinline__ u32x4 lp_load8(const uint16_t* p) {
 }
 __device__ __forceinline__ float lp_bf16(uint32_t lo16) { return __uint_as_float(lo16 << 16); }
 
-// (max, sum of exp(x - max)) of two partial results.
+// (max, sum of exp(x - max)) of two partial results; one whose max is -inf has met no number yet, and its
+// sum is 0, or NaN if it has met a NaN.
 __device__ __forceinline__ void lse_merge(float& m, float& s, float m2, float s2) {
   const float mm = fmaxf(m, m2);
-  // exp(-inf - (-inf)) would be NaN: an empty partial result contributes nothing
-  const float a = m == -__builtin_inff() ? 0.f : s * __expf(m - mm);
-  const float b = m2 == -__builtin_inff() ? 0.f : s2 * __expf(m2 - mm);
+  const float a = m == -__builtin_inff() ? s : s * __expf(m - mm);  // (exp(-inf - (-inf)) would be NaN)
+  const float b = m2 == -__builtin_inff() ? s2 : s2 * __expf(m2 - mm);
   m = mm;
   s = a + b;
 }
@@ -76,17 +76,24 @@ __global__ __launch_bounds__(kLpFwdThreads) void token_logprob_fwd_kernel(
 #pragma unroll
       for (int e = 1; e < 8; ++e) cm = fmaxf(cm, x[e]);
       if (cm > m) {  // rescale the running sum to the new maximum
-        s = m == -__builtin_inff() ? 0.f : s * __expf(m - cm);
+        s = m == -__builtin_inff() ? s : s * __expf(m - cm);
         m = cm;
       }
       if (m != -__builtin_inff()) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) s += __expf(x[e] - m);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (x[e] != x[e]) s = x[e];
       }
     }
   }
   if (!SPLIT || part == splits - 1)
-    for (int64_t i = chunks * 8 + tid; i < vocab; i += kLpFwdThreads) lse_merge(m, s, lp_bf16(row[i]), 1.f);
+    for (int64_t i = chunks * 8 + tid; i < vocab; i += kLpFwdThreads) {
+      const float x = lp_bf16(row[i]);
+      lse_merge(m, s, x, x == -__builtin_inff() ? 0.f : 1.f);
+    }
   // across the workgroup: the maximum first, then one rescaling per lane and plain sums (merging
   // pairs step by step takes two exponentials a step: 2000 rows x 8192 12.5 us that way, 11.1 so)
   float top = m;
@@ -96,7 +103,7 @@ __global__ __launch_bounds__(kLpFwdThreads) void token_logprob_fwd_kernel(
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < kWaves; ++w) top = fmaxf(top, sm[w]);
-  s = m == -__builtin_inff() ? 0.f : s * __expf(m - top);
+  s = m == -__builtin_inff() ? s : s * __expf(m - top);
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
   if ((tid & 63) == 0) ss[tid >> 6] = s;

@@ -48,6 +48,19 @@ def test_routing_against_float64(device, tokens, experts, k, softmax, norm, with
     assert (got.double() - want).norm() <= 1e-5 * want.norm() + 1e-7
 
 
+@pytest.mark.parametrize("k", [1, 2, 3, 5, 8, 11, 16])
+@pytest.mark.parametrize("softmax", [True, False])
+def test_weights_are_normalised_by_a_tree_sum(device, k, softmax):
+    """Bit for bit the scores over their sum, pairs of neighbours added first: its error grows with the
+    logarithm of k, that of a running sum with k."""
+    logits = torch.randn((3000, 128), generator=torch.Generator(device=device).manual_seed(k), device=device) * 2
+    scores = ops.route_topk(logits, None, k, softmax, False, 1.0)[0]
+    total = torch.nn.functional.pad(scores, (0, 16 - k))
+    while total.shape[1] > 1:
+        total = total[:, 0::2] + total[:, 1::2]
+    assert torch.equal(ops.route_topk(logits, None, k, softmax, True, 1.0)[0], scores / (total + 1e-20))
+
+
 def test_equal_scores_go_to_the_lower_experts(device):
     top, selected, counts, _ = ops.route_topk(torch.zeros((3, 130), device=device), None, 4, True, False, 1.0)
     assert selected.tolist() == [[0, 1, 2, 3]] * 3 and counts.tolist() == [3] * 4 + [0] * 126

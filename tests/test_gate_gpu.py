@@ -45,6 +45,18 @@ def test_gate_against_float64(device, tokens, experts, dim):
     assert torch.equal(behind, base)
 
 
+@pytest.mark.parametrize("experts,dim", [(8, 2048), (32, 4096), (64, 2048), (72, 2048), (16, 1024), (128, 384)])
+@pytest.mark.parametrize("tokens", [300, 4100, 9001])
+def test_logits_do_not_depend_on_where_a_token_stands(device, tokens, experts, dim):
+    """Bit for bit the same anywhere in a batch and in a batch of another size, in every order of the
+    contraction that workgroups take."""
+    g = torch.Generator(device=device).manual_seed(experts + dim)
+    some = torch.randn((50, dim), generator=g, device=device).bfloat16()
+    w = (torch.randn((experts, dim), generator=g, device=device) * 0.02).bfloat16()
+    which = torch.randint(0, 50, (tokens,), generator=g, device=device)
+    assert torch.equal(ops.gate_logits(some[which], w), ops.gate_logits(some, w)[which])
+
+
 def test_gate_keeps_infinite_gradients(device):
     dl = torch.zeros((16, 8), device=device)
     dl[3, 2], dl[5, 1] = float("inf"), float("nan")

@@ -13,6 +13,8 @@
 // float32 matmuls around conversions of x, W and dx and a separate addition took 75 + 98 + 141 + 100 us.
 // With 8 experts 15, 34 and 28 us: the forward reads x at 4.5 TB/s, and what more experts add is W
 // coming from the L2 for every 32 tokens and the three-part products.
+#include <type_traits>
+
 #include "mx_gemm_tile.h"
 
 namespace mx {
@@ -65,12 +67,16 @@ __device__ __forceinline__ void three_parts(const float (&v)[8], u32x4 (&part)[3
 // up through LDS at the end: four times shorter chains, which is what counts for few tokens, and W
 // read once per 16 MT tokens from the L2.
 // Per wave: the next step's x and the next half step's W are in flight while one is multiplied.
-template <int MT, int NT>
+//
+// SEGS > 1: the contraction in that many equal parts with a sum of its own each; workgroups begin with
+// different parts, and the sums are added in one order, so that a token's logits do not depend on where it
+// stands.
+template <int MT, int NT, int SEGS>
 __global__ __launch_bounds__(256, 2) void gate_fwd_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                           const uint16_t* __restrict__ w, int64_t ldw,
                                                           int64_t tokens, int experts, int dim,
                                                           float* __restrict__ logits) {
-  __shared__ v4f sums[4][MT * NT][64];
+  __shared__ v4f sums[SEGS][4][MT * NT][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = lane & 15, j = lane >> 4;
   const int64_t t0 = (int64_t)blockIdx.x * 16 * MT;
@@ -90,8 +96,9 @@ __global__ __launch_bounds__(256, 2) void gate_fwd_kernel(const uint16_t* __rest
   for (int m = 0; m < MT; ++m)
 #pragma unroll
     for (int n = 0; n < NT; ++n) acc[m][n] = v4f{0.f, 0.f, 0.f, 0.f};
-  // rows a multiple of 4 KB apart lie on the same channels of the L2: workgroups start at different steps
-  const int steps = dim / 64, turn = (int)((blockIdx.x >> 3) * 4 % (unsigned)steps);
+  const int steps = dim / 64, per = steps / SEGS;  // (SEGS > 1: per is a multiple of 8)
+  int seg = SEGS > 1 ? (int)((blockIdx.x >> 3) % SEGS) : 0;
+  const int turn = seg * per;
   auto at = [&](int s) { return 64 * (s + turn < steps ? s + turn : s + turn - steps); };
   u32x4 xa[2][MT], xb[2][MT], w0[NT], w1[NT];
   auto load_x = [&](int k, u32x4 (&xp)[2][MT]) {
@@ -125,19 +132,34 @@ __global__ __launch_bounds__(256, 2) void gate_fwd_kernel(const uint16_t* __rest
     load_x(at(wave), xa);
     load_w(at(wave), w0);
   }
-  for (int s = wave; s < steps; s += 8) {
+  auto keep = [&]() {
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        sums[seg][wave][m * NT + n][lane] = acc[m][n];
+        acc[m][n] = v4f{0.f, 0.f, 0.f, 0.f};
+      }
+    seg = seg + 1 < SEGS ? seg + 1 : 0;
+  };
+  for (int s = wave, left = per; s < steps; s += 8) {
     step(s, xa, xb);
     if (s + 4 < steps) step(s + 4, xb, xa);
+    if (SEGS > 1 && (left -= 8) == 0) {
+      keep();
+      left = per;
+    }
   }
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int n = 0; n < NT; ++n) sums[wave][m * NT + n][lane] = acc[m][n];
+  if (SEGS == 1) keep();
   __syncthreads();
   // a lane holds experts 16n + 4j .. + 3 of token 16m + i
   for (int q = wave; q < MT * NT; q += 4) {
-    const v4f a = sums[0][q][lane], b = sums[1][q][lane], c = sums[2][q][lane], d = sums[3][q][lane];
-    const v4f s = (a + b) + (c + d);
+    v4f s = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int g = 0; g < SEGS; ++g) {
+      const v4f a = sums[g][0][q][lane], b = sums[g][1][q][lane], c = sums[g][2][q][lane], d = sums[g][3][q][lane];
+      s = g == 0 ? (a + b) + (c + d) : s + ((a + b) + (c + d));
+    }
     const int64_t t = t0 + 16 * (q / NT) + i;
     const int e = 16 * (q % NT) + 4 * j;
     if (t < tokens && e < experts) *reinterpret_cast<v4f*>(logits + t * experts + e) = s;
@@ -347,18 +369,23 @@ extern "C" int mx_gate_logits(const void* x, int64_t ldx, const void* w, int64_t
     hipLaunchKernelGGL(kernel, dim3((unsigned)((tokens + 16 * mt - 1) / (16 * mt))), dim3(256), 0, (hipStream_t)stream,
                        (const uint16_t*)x, ldx, (const uint16_t*)w, ldw, tokens, (int)experts, (int)dim, logits);
   };
-  // 32 tokens per workgroup halve the reads of W; 16 while that leaves CUs without work
-  if (tokens > 16 * 256) {
-    if (experts <= 16) launch(gate_fwd_kernel<2, 1>, 2);
-    else if (experts <= 32) launch(gate_fwd_kernel<2, 2>, 2);
-    else if (experts <= 64) launch(gate_fwd_kernel<2, 4>, 2);
-    else launch(gate_fwd_kernel<2, 8>, 2);
-  } else {
-    if (experts <= 16) launch(gate_fwd_kernel<1, 1>, 1);
-    else if (experts <= 32) launch(gate_fwd_kernel<1, 2>, 1);
-    else if (experts <= 64) launch(gate_fwd_kernel<1, 4>, 1);
-    else launch(gate_fwd_kernel<1, 8>, 1);
-  }
+  // 32 tokens per workgroup halve the reads of W; 16 while that leaves CUs without work.  Rows a multiple of
+  // 4 KB apart lie on the same channels of the L2: there half of the workgroups begin with the second half
+  // of the contraction.  16384 x 4096, us, in order / in halves: 8 experts 35.2 / 22.1, 32 38.8 / 31.5,
+  // 64 51.3 / 46.3; 128 76.9 / 76.9 and at 2048 41.5 / 42.5 (W's reads count for more, and a CU has room for one
+  // workgroup with twice the sums), so in order.
+  const bool halves = dim % 2048 == 0, few = tokens <= 16 * 256;
+  auto pick = [&](auto nt) {
+    constexpr int NT = decltype(nt)::value;
+    if constexpr (NT <= 4) {
+      if (halves) return few ? launch(gate_fwd_kernel<1, NT, 2>, 1) : launch(gate_fwd_kernel<2, NT, 2>, 2);
+    }
+    few ? launch(gate_fwd_kernel<1, NT, 1>, 1) : launch(gate_fwd_kernel<2, NT, 1>, 2);
+  };
+  if (experts <= 16) pick(std::integral_constant<int, 1>{});
+  else if (experts <= 32) pick(std::integral_constant<int, 2>{});
+  else if (experts <= 64) pick(std::integral_constant<int, 4>{});
+  else pick(std::integral_constant<int, 8>{});
   return hipGetLastError() == hipSuccess ? MX_OK : MX_ERR_LAUNCH;
 }
 

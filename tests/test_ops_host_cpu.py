@@ -73,3 +73,64 @@ def test_block_pitch_is_for_training_steps_without_cached_weight_casts():
     assert block_pitch_pad(cfg, True, False) == 0 and block_pitch_pad(cfg, False, True) == 0
     cached = MXFP8Config(cache_weight_casts=True)
     assert block_pitch_pad(cached, True, True) == 0
+
+
+@pytest.fixture
+def no_launches(monkeypatch):
+    """Everything around the library calls, on the CPU: no call is made and outputs keep what they held."""
+    from torchtitan_amd import mx_tensor
+
+    monkeypatch.setattr(ops, "_call", lambda *args: None)
+    monkeypatch.setattr(ops, "_stream", lambda t: 0)
+    monkeypatch.setattr(ops, "_operand_input", lambda x, f32_ok=False: x)
+    monkeypatch.setattr(ops, "_split_workspace", lambda *args: None)
+    mx_tensor._weight_cache.clear()
+    mx_tensor.clear_cast_cache()
+    yield
+    mx_tensor._weight_cache.clear()
+    mx_tensor.clear_cast_cache()
+
+
+def _bf16(*shape):
+    return torch.zeros(shape, dtype=torch.bfloat16)
+
+
+# contractions that round up to the same whole blocks, and the same ones
+@pytest.mark.parametrize("wrong,right", [(2016, 2048), (32, 128), (1920, 2016), (2048, 2048)])
+def test_products_compare_the_contraction_before_it_is_rounded_up(no_launches, wrong, right):
+    operand = lambda rows, depth, pad=128: ops.to_operands(_bf16(rows, depth), "rceil", True, False, pad)[0]
+    for M in (16, 200):
+        x, x2, w, w2 = operand(M, wrong), operand(M, wrong), operand(256, right), operand(256, right)
+        calls = [lambda: ops.mx_gemm_nt(x, w), lambda: ops.mx_gemm_nt(x, w, _bf16(M, 256)),
+                 lambda: ops.mx_gemm_nt(x, operand(256, right, 0)), lambda: ops.mx_gemm_nt_pair(x, w, x2, w2),
+                 lambda: ops.mx_gemm_nt_pair(w, w2, w, operand(256, wrong)),
+                 lambda: ops.mx_gemm_nt_shared_a(x, w, w2), lambda: ops.mx_gemm_nt_shared_a(x, operand(256, wrong), w),
+                 lambda: ops.mx_gemm_nt_shared_b(x, x2, w), lambda: ops.mx_gemm_nt_shared_b(w, operand(256, wrong), w2),
+                 lambda: ops.mx_few_rows(_bf16(16, wrong), w),
+                 lambda: ops.mx_few_rows(_bf16(16, right), w, "floor", operand(256, wrong))]
+        for call in calls:
+            if wrong == right:
+                call()
+            else:
+                with pytest.raises(ValueError):
+                    call()
+
+
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("tokens", [16, 200])
+def test_mismatched_modules_raise(no_launches, monkeypatch, grad, tokens):
+    from torchtitan_amd import mx_blocks, mx_tensor
+
+    cfg = mx_tensor.MXFP8Config()
+    x = _bf16(tokens, 2016)
+    monkeypatch.setattr(ops, "few_rows_ok", lambda t: t.shape[0] <= ops.FEW_ROWS)
+    weight = lambda *shape: mx_tensor.MXFP8TrainingWeight(_bf16(*shape).requires_grad_(grad), cfg)
+    mismatched = (lambda: mx_tensor.mx_linear(x, weight(512, 2048).as_subclass(torch.Tensor), None, cfg),
+                  lambda: mx_blocks.mx_feed_forward(x, weight(2048, 2048), weight(2016, 2048), weight(2048, 2048)),
+                  lambda: mx_blocks.mx_feed_forward(x, weight(2016, 2016), weight(2016, 2048), weight(2016, 2016)),
+                  lambda: mx_blocks.mx_swiglu_linear(x, x, weight(512, 2048)))
+    with torch.set_grad_enabled(grad):
+        for call in mismatched:
+            with pytest.raises(ValueError, match="contraction|same shape"):
+                call()
+        mx_blocks.mx_feed_forward(x, weight(2048, 2016), weight(2016, 2048), weight(2048, 2016))

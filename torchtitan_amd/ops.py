@@ -195,21 +195,23 @@ def _operand_input(x: torch.Tensor, f32_ok: bool = False) -> torch.Tensor:
 class Operand:
     """One operand of the dense GEMMs, e4m3 codes [rows, k] and their MFMA-order scales, in one
     allocation: rows `ld` bytes apart from byte `at` on, scales from byte `scales_at` on.  Reads as
-    an `MXData` (`codes`, `scales`, `scale_order`; views made when asked for).  One buffer and plain
+    an `MXData` (`codes`, `scales`, `scale_order`; views made when asked for).  `k` is the contraction in
+    whole 128-deep blocks, `depth` how much of it is not zero fill: what the other operand must agree
+    with.  One buffer and plain
     numbers instead of two to four tensors and their views: at small sizes making those takes the
     host longer than the GPU needs for the cast."""
 
-    __slots__ = ("buf", "rows", "k", "ld", "at", "scales_at")
+    __slots__ = ("buf", "rows", "k", "ld", "at", "scales_at", "depth")
     scale_order = MX_SCALES_MFMA
 
     def __init__(self, buf: torch.Tensor, layout):
         self.buf = buf
-        self.rows, self.k, self.ld, self.at, self.scales_at = layout
+        self.rows, self.k, self.ld, self.at, self.scales_at, self.depth = layout
 
     @property
     def layout(self):
         """What, with the buffer, makes the operand: for a backward that gets the buffer back."""
-        return self.rows, self.k, self.ld, self.at, self.scales_at
+        return self.rows, self.k, self.ld, self.at, self.scales_at, self.depth
 
     @property
     def codes(self) -> torch.Tensor:
@@ -229,7 +231,7 @@ class Operand:
 
     def first_rows(self, n: int) -> "Operand":
         """The operand's first n rows (n rounds up to the same multiple of 128)."""
-        return Operand(self.buf, (n, self.k, self.ld, self.at, self.scales_at))
+        return Operand(self.buf, (n, self.k, self.ld, self.at, self.scales_at, self.depth))
 
     def data(self) -> MXData:
         return MXData(self.codes, self.scales, MX_SCALES_MFMA)
@@ -241,7 +243,7 @@ def _new_operand(rows: int, cols: int, pad: int, device) -> Operand:
     ld = k + pad
     scales_at = (rows * ld + 255) & ~255
     buf = torch.empty(scales_at + ((rows + 127) & ~127) * (k // BLOCK), dtype=torch.uint8, device=device)
-    return Operand(buf, (rows, k, ld, 0, scales_at))
+    return Operand(buf, (rows, k, ld, 0, scales_at, cols))
 
 
 def _new_operand_pair(rows: int, cols: int, pad: int, device):
@@ -250,8 +252,8 @@ def _new_operand_pair(rows: int, cols: int, pad: int, device):
     ld, scale_bytes = k + pad, ((rows + 127) & ~127) * (k // BLOCK)
     scales_at = (2 * rows * ld + 255) & ~255
     buf = torch.empty(scales_at + 2 * scale_bytes, dtype=torch.uint8, device=device)
-    return (Operand(buf, (rows, k, ld, 0, scales_at)),
-            Operand(buf, (rows, k, ld, rows * ld, scales_at + scale_bytes)))
+    return (Operand(buf, (rows, k, ld, 0, scales_at, cols)),
+            Operand(buf, (rows, k, ld, rows * ld, scales_at + scale_bytes, cols)))
 
 
 def to_operands(x: torch.Tensor, mode="floor", rows: bool = True, cols: bool = True, pitch_pad: int = 0):
@@ -262,7 +264,7 @@ def to_operands(x: torch.Tensor, mode="floor", rows: bool = True, cols: bool = T
     C = x.shape[1]
     x = _operand_input(x, f32_ok=True)
     (R, Cx), dev, pad = x.shape, x.device, _pitch_ok(pitch_pad)
-    r = _new_operand(R, Cx, pad, dev) if rows else None
+    r = _new_operand(R, C, pad, dev) if rows else None
     c = _new_operand(Cx, R, pad, dev) if cols else None
     _call("mx_cast_pad", "cast_dim0_dim1" if rows and cols else "cast_dim0" if rows else "cast_dim1", dev,
           x.data_ptr(), x.dtype == torch.float32, R, Cx, x.stride(0),
@@ -301,7 +303,7 @@ class CastList:
         pad, cols = _pitch_ok(pitch_pad), x.shape[1]
         x = _operand_input(x, f32_ok=True)
         R, C = x.shape
-        r, c = _new_operand(R, C, pad, x.device), _new_operand(C, R, pad, x.device)
+        r, c = _new_operand(R, cols, pad, x.device), _new_operand(C, R, pad, x.device)
         self._entry(x, 1, R, C, x.stride(0), r.codes_ptr, r.ld, r.scales_ptr, c.codes_ptr, c.ld, c.scales_ptr)
         return r, c if C == cols else c.first_rows(cols)
 
@@ -949,6 +951,11 @@ def _operands(*qs) -> bool:
     return True
 
 
+def _depth(q) -> int:
+    """The contraction that `q` was cast from: its codes' row length but for the zero fill of an `Operand`."""
+    return q.depth if type(q) is Operand else q.codes.shape[-1]
+
+
 def _gemm_operands(a: Operand, b: Operand, out: torch.Tensor) -> torch.Tensor:
     M, N, K = a.rows, b.rows, a.k
     dev = out.device
@@ -979,8 +986,10 @@ def mx_few_rows(x: torch.Tensor, w: Operand, mode="floor", w2: Operand | None = 
     products, stacked.  Callers check `few_rows_ok` first."""
     x = _operand_input(x)
     (M, K), N = x.shape, w.rows
-    if w.k != -(-K // WHOLE_BLOCK) * WHOLE_BLOCK:
-        raise ValueError(f"contraction mismatch: {K} vs {w.k}")
+    if w.depth != K:
+        raise ValueError(f"contraction mismatch: {K} vs {w.depth}")
+    if w2 is not None and (w2.rows, w2.depth, w2.ld) != (N, K, w.ld):
+        raise ValueError("both weights must have the same shape and pitch")
     out = torch.empty((M, N) if w2 is None else (2, M, N), dtype=torch.bfloat16, device=x.device)
     d = out.data_ptr()
     _call("mx_few_rows", "few_rows", x.device, x.data_ptr(), M, K, x.stride(0), w.codes_ptr, w.scales_ptr,
@@ -1062,13 +1071,13 @@ def op_sac_save_list() -> set:
 def mx_gemm_nt(a: MXData, b: MXData, out: torch.Tensor | None = None) -> torch.Tensor:
     """bf16 D[M,N] = deq(a)[M,K] @ deq(b)[N,K]^T with fp32 accumulation."""
     if out is None and _operands(a, b) and not _watched():
-        if a.k != b.k:
-            raise ValueError(f"contraction mismatch: {a.k} vs {b.k}")
+        if a.depth != b.depth:
+            raise ValueError(f"contraction mismatch: {a.depth} vs {b.depth}")
         return _gemm_operands(a, b, torch.empty((a.rows, b.rows), dtype=torch.bfloat16, device=a.buf.device))
     M, K = a.codes.shape
     N, Kb = b.codes.shape
-    if K != Kb:
-        raise ValueError(f"contraction mismatch: {K} vs {Kb}")
+    if K != Kb or _depth(a) != _depth(b):
+        raise ValueError(f"contraction mismatch: {_depth(a)} vs {_depth(b)}")
     sa, sb = _as_mfma(a), _as_mfma(b)
     if out is None:
         if _watched():
@@ -1085,7 +1094,7 @@ def mx_gemm_nt_pair(a: MXData, b: MXData, a2: MXData, b2: MXData) -> torch.Tenso
     otherwise two GEMMs and a bf16 add."""
     if _operands(a, b, a2, b2):
         M, N, K = a.rows, b.rows, a.k
-        if a2.rows != M or b2.rows != N or b.k != K or a2.k != K or b2.k != K:
+        if a2.rows != M or b2.rows != N or not a.depth == b.depth == a2.depth == b2.depth:
             raise ValueError("both operand sets must have the same shapes")
         if not _persistent_shape(M, N, K):
             return mx_gemm_nt(a, b) + mx_gemm_nt(a2, b2)
@@ -1095,7 +1104,8 @@ def mx_gemm_nt_pair(a: MXData, b: MXData, a2: MXData, b2: MXData) -> torch.Tenso
         return out
     M, K = a.codes.shape
     N = b.codes.shape[0]
-    if a2.codes.shape != (M, K) or b2.codes.shape != (N, K) or b.codes.shape[1] != K:
+    if (a2.codes.shape != (M, K) or b2.codes.shape != (N, K) or b.codes.shape[1] != K
+            or not _depth(a) == _depth(b) == _depth(a2) == _depth(b2)):
         raise ValueError("both operand sets must have the same shapes")
     if not _persistent_shape(M, N, K):
         return mx_gemm_nt(a, b) + mx_gemm_nt(a2, b2)
@@ -1117,7 +1127,7 @@ def mx_gemm_nt_shared_a(a: MXData, b: MXData, b2: MXData) -> torch.Tensor:
     otherwise two GEMMs; bit-identical either way."""
     if _operands(a, b, b2) and not _watched():
         M, N, K = a.rows, b.rows, a.k
-        if b2.rows != N or b.k != K or b2.k != K:
+        if b2.rows != N or not a.depth == b.depth == b2.depth:
             raise ValueError("both second operands must have the same shape")
         out = torch.empty((2, M, N), dtype=torch.bfloat16, device=a.buf.device)
         if not _persistent_shape(M, N, K):
@@ -1130,7 +1140,7 @@ def mx_gemm_nt_shared_a(a: MXData, b: MXData, b2: MXData) -> torch.Tensor:
         return out
     M, K = a.codes.shape
     N = b.codes.shape[0]
-    if b2.codes.shape != b.codes.shape or b.codes.shape[1] != K:
+    if b2.codes.shape != b.codes.shape or b.codes.shape[1] != K or not _depth(a) == _depth(b) == _depth(b2):
         raise ValueError("both second operands must have the same shape")
     if _watched():  # as dispatcher ops, so that a per-op checkpoint policy can keep the outputs
         return torch.stack((mx_gemm_nt(a, b), mx_gemm_nt(a, b2)))
@@ -1151,7 +1161,7 @@ def mx_gemm_nt_shared_b(a: MXData, a2: MXData, b: MXData) -> torch.Tensor:
     roles of the operands swapped."""
     if _operands(a, a2, b):
         M, N, K = a.rows, b.rows, a.k
-        if a2.rows != M or a2.k != K or b.k != K:
+        if a2.rows != M or not a.depth == a2.depth == b.depth:
             raise ValueError("both first operands must have the same shape")
         out = torch.empty((2, M, N), dtype=torch.bfloat16, device=a.buf.device)
         if not _persistent_shape(M, N, K):
@@ -1164,7 +1174,7 @@ def mx_gemm_nt_shared_b(a: MXData, a2: MXData, b: MXData) -> torch.Tensor:
         return out
     M, K = a.codes.shape
     N = b.codes.shape[0]
-    if a2.codes.shape != a.codes.shape or b.codes.shape[1] != K:
+    if a2.codes.shape != a.codes.shape or b.codes.shape[1] != K or not _depth(a) == _depth(a2) == _depth(b):
         raise ValueError("both first operands must have the same shape")
     out = torch.empty((2, M, N), dtype=torch.bfloat16, device=a.codes.device)
     if not _persistent_shape(M, N, K):

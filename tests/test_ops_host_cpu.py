@@ -83,6 +83,7 @@ def no_launches(monkeypatch):
     monkeypatch.setattr(ops, "_call", lambda *args: None)
     monkeypatch.setattr(ops, "_stream", lambda t: 0)
     monkeypatch.setattr(ops, "_operand_input", lambda x, f32_ok=False: x)
+    monkeypatch.setattr(ops, "_check_hp", lambda x: x)
     monkeypatch.setattr(ops, "_split_workspace", lambda *args: None)
     mx_tensor._weight_cache.clear()
     mx_tensor.clear_cast_cache()
@@ -134,3 +135,23 @@ def test_mismatched_modules_raise(no_launches, monkeypatch, grad, tokens):
             with pytest.raises(ValueError, match="contraction|same shape"):
                 call()
         mx_blocks.mx_feed_forward(x, weight(2048, 2016), weight(2016, 2048), weight(2048, 2016))
+
+
+def test_a_cached_cast_is_given_in_the_form_its_caller_wants(no_launches):
+    from torchtitan_amd import mx_tensor
+
+    cfg = mx_tensor.MXFP8Config(cache_weight_casts=True)
+    w = _bf16(128, 384)
+    cast = lambda whole: mx_tensor._cast_weight(w, "rceil", True, cfg, whole_blocks=whole)
+    dense = cast(False)
+    for q in dense:
+        q.codes.random_(0, 255), q.scales.random_(0, 255)
+    whole = cast(True)  # a copy, which takes the dense entry's place
+    for q, d in zip(whole, dense):
+        assert type(q) is ops.Operand and type(d) is MXData and q.depth == d.codes.shape[1]
+        assert torch.equal(q.codes, d.codes) and torch.equal(q.scales, d.scales) and q.codes.is_contiguous()
+    assert cast(True)[0] is whole[0] and len(mx_tensor._weight_cache) == 1
+    for q, d in zip(cast(False), dense):  # and serves both
+        assert type(q) is MXData and torch.equal(q.codes, d.codes) and torch.equal(q.scales, d.scales)
+    with pytest.raises(ValueError):
+        ops.Operand.of(MXData(_codes(128, 160), torch.zeros(1280, dtype=torch.uint8), MX_SCALES_MFMA))

@@ -454,6 +454,10 @@ def mx_ffn_fwd(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, w3: torch.Te
     if x2.dtype != torch.bfloat16:
         x2 = x2.to(torch.bfloat16)
     y, saved = mx_blocks.ffn_forward(x2, None, w1, w2, w3, _block_cfg(mode, cache_w), need_dx, need_dw, norm_weight, eps)
+    if cache_w:  # an operator's outputs are its own: not the cache's tensors
+        for name in ("w1", "w2", "w3"):
+            q = saved[name]
+            saved[name] = None if q is None else MXData(q.codes.clone(), q.scales.clone(), MX_SCALES_MFMA)
     return (y.view(*x.shape[:-1], w2.shape[0]), *_filled(_ffn_slots(saved), x.device, skip=(11, 13)))
 
 

@@ -153,9 +153,8 @@ def ffn_forward(x2, x_src, w1, w2, w3, cfg: MXFP8Config, need_dx: bool, need_dw:
     cast = _FFNCasts(cfg, whole_blocks, pad)
     if whole_blocks and norm_weight is None and not (need_dx or need_dw) and ops.few_rows_ok(x2):
         (w1q0, _), (w3q0, _), (w2q0, _) = cast.weights((w1, w3, w2), (False, False, False))
-        if type(w1q0) is type(w3q0) is ops.Operand and w1q0.ld == w3q0.ld:  # (cached casts of a traced forward are dense)
-            h13 = ops.mx_few_rows(x2, w1q0, cfg.scale_mode, w3q0)
-            return ops.mx_gemm_nt(cast.gate(h13, False)[0], w2q0), dict.fromkeys(FFN_SAVED)
+        h13 = ops.mx_few_rows(x2, w1q0, cfg.scale_mode, w3q0)
+        return ops.mx_gemm_nt(cast.gate(h13, False)[0], w2q0), dict.fromkeys(FFN_SAVED)
     rstd = None
     ws, ws_cols = (w1, w3, w2), (need_dx, need_dx, need_dx or need_dw)
     if norm_weight is not None:  # RMSNorm in front: normalised inside the cast, rstd kept for its backward

@@ -167,12 +167,13 @@ def _cast_weight(w: torch.Tensor, mode: str, need_cols: bool, cfg: MXFP8Config, 
     N is a multiple of 32."""
     cached = cfg.cache_weight_casts
     whole = whole_blocks and w.dim() == 2
-    # the cache keeps padded, rounded-up and dense casts apart (they coincide where nothing is rounded)
+    # the cache keeps padded, rounded-up and dense casts apart; where nothing is rounded the last two have the
+    # same bytes, and one entry serves both
     key = (mode, pitch_pad, whole and bool(w.shape[0] % ops.WHOLE_BLOCK or w.shape[1] % ops.WHOLE_BLOCK))
     if cached:
         hit = _weight_cache.get(w, key)
         if hit is not None and (hit[1] is not None or not need_cols or w.shape[-2] % ops.BLOCK):
-            return hit
+            return _in_form(w, key, hit, whole)
         need_cols = True  # cast once in full, whoever asks first
     wb = (_castable(w) if whole else w if w.dtype == torch.bfloat16 else w.to(torch.bfloat16)).contiguous()
     both = need_cols and (whole or wb.shape[-2] % ops.BLOCK == 0)
@@ -186,6 +187,21 @@ def _cast_weight(w: torch.Tensor, mode: str, need_cols: bool, cfg: MXFP8Config, 
     if cached:
         _weight_cache.put(w, key, q[0], q[1])
     return q
+
+
+def _in_form(w: torch.Tensor, key, hit, whole: bool):
+    """A cached cast in the form its caller wants: operands, or dense `MXData` (views of an operand's buffer).
+    An operand made from a dense entry takes its place, except under graph capture, where it is filled
+    by the replay only."""
+    rows, cols = hit
+    if w.dim() != 2 or whole == (type(rows) is ops.Operand):
+        return hit
+    if not whole:
+        return rows.data(), (None if cols is None else cols.data())
+    hit = ops.Operand.of(rows), (None if cols is None else ops.Operand.of(cols))
+    if not (w.is_cuda and torch.cuda.is_current_stream_capturing()):
+        _weight_cache.put(w, key, *hit)
+    return hit
 
 
 def _one_launch(ws, cfg: MXFP8Config, whole_blocks: bool = True) -> bool:
@@ -247,9 +263,8 @@ def _linear_forward(x, weight, cfg: MXFP8Config, need_dx: bool, need_dw: bool):
     pad = 0 if cfg.cache_weight_casts else ops.CODE_PITCH_PAD
     if not (need_dx or need_dw) and ops.few_rows_ok(x2):
         wq0, _ = _cast_weight(weight, mode, False, cfg, pitch_pad=pad)
-        if type(wq0) is ops.Operand:  # (a cached cast of a traced forward is dense)
-            y = ops.mx_few_rows(x2, wq0, mode)
-            return (y if x.dim() == 2 else y.view(*x.shape[:-1], N)), None, None
+        y = ops.mx_few_rows(x2, wq0, mode)
+        return (y if x.dim() == 2 else y.view(*x.shape[:-1], N)), None, None
     (xq0, xq1), (wq0, wq1) = _cast_activation_and_weights(x2, x, (weight,), mode, need_dx, need_dw, cfg, pad)
     y = ops.mx_gemm_nt(xq0, wq0)
     return (y if x.dim() == 2 else y.view(*x.shape[:-1], N)), xq1, wq1

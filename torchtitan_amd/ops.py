@@ -233,6 +233,17 @@ class Operand:
         """The operand's first n rows (n rounds up to the same multiple of 128)."""
         return Operand(self.buf, (n, self.k, self.ld, self.at, self.scales_at, self.depth))
 
+    @classmethod
+    def of(cls, q: MXData) -> "Operand":
+        """A copy of dense codes in whole blocks with MFMA-order scales as an operand."""
+        rows, k = q.codes.shape
+        if k % WHOLE_BLOCK or q.scale_order != MX_SCALES_MFMA:
+            raise ValueError("an operand has whole blocks along its contraction and MFMA-order scales")
+        out = _new_operand(rows, k, 0, q.codes.device)
+        out.codes.copy_(q.codes)
+        out.scales.copy_(q.scales)
+        return out
+
     def data(self) -> MXData:
         return MXData(self.codes, self.scales, MX_SCALES_MFMA)
 

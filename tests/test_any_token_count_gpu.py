@@ -194,3 +194,32 @@ def test_casts_of_a_list_equal_the_single_casts(device, mode, pad):
     q, _ = casts.add_stack(stacks[0].float())
     casts.launch()
     assert torch.equal(q.codes, got[len(tensors)][0].codes)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_activations_in_any_order(device, dtype):
+    """Transposed and expanded inputs, as their contiguous copies: casts, lists of casts, and a converted linear
+    under autocast, forward and backward."""
+    from torchtitan_amd import mx_tensor
+
+    g = torch.Generator(device=device).manual_seed(3)
+    base = torch.randn((192, 96), generator=g, device=device).to(dtype)
+    for x in (base.t(), base[:, :1].expand(192, 64), base[None].transpose(1, 2)[0], base.t()[::2, 64:], base[:, :1]):
+        want = ops.to_operands(x.contiguous().clone(), "rceil")
+        casts = ops.CastList("rceil")
+        listed = casts.add(x)
+        casts.launch()
+        for q, p, w in zip(ops.to_operands(x, "rceil"), listed, want):
+            assert torch.equal(q.codes, w.codes) and torch.equal(p.codes, w.codes)
+    w = (torch.randn((64, 192), generator=g, device=device) * 0.05).to(dtype).requires_grad_(True)
+    for x in (base.t(), base[None].transpose(1, 2)):
+        out = []
+        for t in (x, x.contiguous()):
+            t = t.detach().requires_grad_(True)
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                y = mx_tensor.mx_linear(t, w, None, mx_tensor.MXFP8Config())
+            out.append([y, *torch.autograd.grad(y, (t, w), torch.ones_like(y))])
+            with torch.no_grad():
+                out[-1].append(mx_tensor.mx_linear(t, w, None, mx_tensor.MXFP8Config()))
+        for a, b in zip(*out):
+            assert torch.equal(a, b)

@@ -183,7 +183,9 @@ WHOLE_BLOCK = 128  # depth of the persistent GEMM's K blocks
 def _operand_input(x: torch.Tensor, f32_ok: bool = False) -> torch.Tensor:
     """`x` as the tile casts read it: 16-byte aligned rows (a copy where they are not); bf16, or float32
     where the caller's kernel takes it."""
-    if not (f32_ok and x.dtype == torch.float32 and x.is_cuda and x.dim() == 2 and x.stride(1) == 1):
+    if f32_ok and x.dtype == torch.float32 and x.is_cuda and x.dim() == 2:
+        x = x if x.stride(1) == 1 else x.contiguous()
+    else:
         x = _check_hp(x)
     if x.shape[1] % 8:
         return torch.nn.functional.pad(x, (0, -x.shape[1] % 8))

@@ -430,3 +430,20 @@ def test_optimizer_state_of_converted_weights_is_plain_and_pickling_keeps_parame
     assert isinstance(q, nn.Parameter) and isinstance(q, MXFP8TrainingWeight) and q.requires_grad
     assert q.mx_config.scale_mode == "floor" and torch.equal(q.detach().as_subclass(torch.Tensor),
                                                               lin.weight.detach().as_subclass(torch.Tensor))
+
+
+@pytest.mark.parametrize("inside", [True, False])
+def test_router_on_fake_gpu_tensors(inside):
+    """Shapes without memory (what a memory estimate runs on), under their mode and handed out of it: the tensor
+    operations, not a kernel that would want an address."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    router = moe_mod.MoE(moe_mod.MoE.Config(num_experts=8, num_shared_experts=0, hidden_dim=32, top_k=2), dim=64).router
+    mode = FakeTensorMode()
+    with mode:
+        x = torch.empty((48, 64), device="cuda")
+        router.gate.weight = nn.Parameter(torch.empty((8, 64), device="cuda"))
+        top, selected, counts = router(x) if inside else (None,) * 3
+    if not inside:
+        top, selected, counts = router(x)
+    assert top.shape == selected.shape == (48, 2) and counts.shape == (8,) and top.device.type == "cuda"

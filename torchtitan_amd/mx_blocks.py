@@ -772,10 +772,11 @@ class _RouteTopK(torch.autograd.Function):
 
 
 def route_fusable(logits: torch.Tensor, top_k: int) -> bool:
-    """Routing runs as one kernel for float32 logits on the GPU of at most 512 experts, 16 choices; not under a
-    function transform or forward-mode AD, for which there are the tensor operations."""
-    return ((torch.compiler.is_compiling() or not ops._transformed()) and logits.is_cuda and logits.dtype == torch.float32 and logits.dim() == 2
-            and logits.shape[1] <= ops.ROUTE_MAX_EXPERTS and top_k <= min(ops.ROUTE_MAX_TOP_K, logits.shape[1]))
+    """Routing runs as one kernel for plain float32 logits on the GPU of at most 512 experts, 16 choices; not under
+    a function transform, forward-mode AD or a dispatch mode, for which there are the tensor operations."""
+    return (type(logits) is torch.Tensor and logits.is_cuda and logits.dtype == torch.float32 and logits.dim() == 2
+            and logits.shape[1] <= ops.ROUTE_MAX_EXPERTS and top_k <= min(ops.ROUTE_MAX_TOP_K, logits.shape[1])
+            and (torch.compiler.is_compiling() or not (ops._watched() or ops._transformed())))
 
 
 def mx_route_topk(logits: torch.Tensor, bias: torch.Tensor | None, top_k: int, softmax: bool, norm: bool, scale: float):

@@ -126,3 +126,23 @@ def test_forward_without_gradients_refuses_tangents(device):
         dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
         with pytest.raises(Exception):
             mx_tensor.mx_linear(dual, w, None, mx_tensor.MXFP8Config())
+
+
+@pytest.mark.parametrize("bias", ["row", "one value", "per token", "one per token", "host value", "bf16"])
+def test_a_bias_that_broadcasts(device, bias):
+    """Whatever can be added to the scores steers the choice as the sum does."""
+    from torchtitan_amd.modules.moe import MoE
+
+    g = torch.Generator(device=device).manual_seed(2)
+    with torch.device(device):
+        router = MoE(MoE.Config(num_experts=16, num_shared_experts=0, hidden_dim=64, top_k=3, score_func="sigmoid"),
+                     dim=128).router
+    x = torch.randn((20, 128), generator=g, device=device)
+    rn = lambda *shape: torch.randn(shape, generator=g, device=device) * 0.3
+    b = {"row": rn(1, 16), "one value": rn(), "per token": rn(20, 16), "one per token": rn(20, 1),
+         "host value": torch.tensor(0.5), "bf16": rn(16).bfloat16()}[bias]
+    top, selected, counts = router(x, b)
+    scores = torch.sigmoid(x @ router.gate.weight.t())
+    want = torch.topk(scores + b, 3, dim=1).indices
+    assert torch.equal(selected.sort(dim=1).values, want.sort(dim=1).values)
+    assert counts.sum().item() == 60 and top.shape == (20, 3)

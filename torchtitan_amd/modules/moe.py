@@ -221,8 +221,7 @@ class TokenChoiceTopKRouter(Module):
             with torch.autocast(device_type=x.device.type, dtype=torch.float32):
                 scores = self.gate(x)
         if (self.num_expert_groups is None and not self._debug_force_load_balance
-                and self.score_func in ("sigmoid", "softmax") and route_fusable(scores, self.top_k)
-                and (expert_bias is None or expert_bias.dtype == torch.float32)):
+                and self.score_func in ("sigmoid", "softmax") and route_fusable(scores, self.top_k, expert_bias)):
             return mx_route_topk(scores, expert_bias, self.top_k, self.score_func == "softmax", self.route_norm,
                                  float(self.route_scale))
         if self.score_func == "sigmoid":

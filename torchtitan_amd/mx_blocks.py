@@ -771,11 +771,14 @@ class _RouteTopK(torch.autograd.Function):
         return (ops.route_topk_bwd(logits, selected, dtop, *ctx.how), None, None, None, None, None)
 
 
-def route_fusable(logits: torch.Tensor, top_k: int) -> bool:
-    """Routing runs as one kernel for plain float32 logits on the GPU of at most 512 experts, 16 choices; not under
-    a function transform, forward-mode AD or a dispatch mode, for which there are the tensor operations."""
+def route_fusable(logits: torch.Tensor, top_k: int, bias: torch.Tensor | None = None) -> bool:
+    """Routing runs as one kernel for plain float32 logits on the GPU of at most 512 experts, 16 choices, and a
+    float32 bias of one value per expert beside them; not under a function transform, forward-mode AD or a
+    dispatch mode, for which there are the tensor operations."""
     return (type(logits) is torch.Tensor and logits.is_cuda and logits.dtype == torch.float32 and logits.dim() == 2
             and logits.shape[1] <= ops.ROUTE_MAX_EXPERTS and top_k <= min(ops.ROUTE_MAX_TOP_K, logits.shape[1])
+            and (bias is None or (type(bias) in (torch.Tensor, torch.nn.Parameter) and bias.dtype == torch.float32
+                                  and bias.shape == logits.shape[1:] and bias.device == logits.device))
             and (torch.compiler.is_compiling() or not (ops._watched() or ops._transformed())))
 
 

@@ -178,15 +178,21 @@ static int launch_few_nt(const FewArgs& p, int products, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? MX_OK : MX_ERR_LAUNCH;
 }
 
-// 16 columns to a workgroup until two of them would still fill the chip: wider ones read x less often.  Codes,
-// 16 / 64 rows, us by columns per workgroup: 2048 x 6144 16: 7.1 / 12.8, 32: 6.4 / 9.1, 64: 9.3 / 12.6;
-// 4096 x 4096 16: 7.5 / 13.1, 32: 9.9 / 15.9; 4096 x 14336 16: 22 / 44, 32: 18 / 31, 64: 17 / 23.
+// The fewest columns that leave no more workgroups than CUs: a second round costs more than wider workgroups, which
+// read x less often, and narrower ones have the shorter chains.  us at 2048 deep (4096 deep moves alike) by columns
+// per workgroup 16 / 32 / 64, from codes of 16 and of 64 rows, from 16 rows of bf16:
+//    4096 columns    5.1 /  6.6 /  9.5     7.8 /  9.1 / 12.4     7.7 /  9.6 / 13.1
+//    5120            7.3 /  6.6 /  9.6    12.9 /  9.4 / 12.7    11.9 /  9.7 / 13.3
+//    8192            7.4 /  6.8 /  9.7    12.8 /  9.9 / 13.1    12.1 /  9.8 / 13.4
+//   10240            9.6 / 10.2 /  9.8    18.4 / 16.3 / 13.2    16.2 / 16.0 / 13.6
+//   16384           12.1 / 10.5 / 10.2    23.9 / 16.9 / 13.4    21.3 / 16.6 / 14.0
 template <int MODE, bool CODES>
 static int launch_few(const FewArgs& p, int products, hipStream_t st) {
+  constexpr int64_t kCus = 256;
   const int64_t columns = p.N * products;
-  if (columns >= 12288) return launch_few_nt<MODE, 4, CODES>(p, products, st);
-  if (columns >= 6144) return launch_few_nt<MODE, 2, CODES>(p, products, st);
-  return launch_few_nt<MODE, 1, CODES>(p, products, st);
+  if (columns <= 16 * kCus) return launch_few_nt<MODE, 1, CODES>(p, products, st);
+  if (columns <= 32 * kCus) return launch_few_nt<MODE, 2, CODES>(p, products, st);
+  return launch_few_nt<MODE, 4, CODES>(p, products, st);
 }
 
 // For mx_gemm_nt's dispatch: operands already checked, K and both pitches multiples of 128 and 16.

@@ -48,6 +48,19 @@ def test_nan_logits_are_not_lost(device, lo, hi, splits, monkeypatch):
     assert lp.isnan().tolist() == [True, False, True] and lse.isnan().tolist() == [True, False, True]
 
 
+@pytest.mark.parametrize("vocab", [8, 1001, 16384])
+def test_log_probs_of_rows_that_overlap(device, vocab):
+    """One row expanded to several, from any element, and a column seen as a row: as their contiguous copies."""
+    base = torch.randn(vocab + 1, device=device).to(torch.bfloat16)
+    for logits in (base[:vocab].expand(3, -1), base[1:].expand(3, -1), base[1:, None].t()):
+        target = torch.arange(logits.shape[0], device=device) % vocab
+        results = []
+        for t in (logits, logits.contiguous().view(-1).clone().view(logits.shape)):
+            lp, lse = ops.token_logprob_fwd(t, target)
+            results.append((lp, lse, ops.token_logprob_bwd(t, target, lse, torch.ones_like(lp))))
+        assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
 def test_parts_follow_the_number_of_rows():
     assert ops._logprob_splits(16, 151936) == 12 and ops._logprob_splits(64, 151936) == 4
     assert ops._logprob_splits(256, 151936) == 1 and ops._logprob_splits(16, 8192) == 1

@@ -765,10 +765,16 @@ def _logprob_splits(rows: int, vocab: int) -> int:
     return max(1, min(-(-256 // rows), vocab // 12288))
 
 
+def _logprob_rows(logits: torch.Tensor) -> torch.Tensor:
+    """bf16 logits [rows, vocab] whose rows follow one another (a copy of expanded ones)."""
+    logits = _check_hp(logits)
+    return logits if logits.stride(0) >= logits.shape[1] else logits.clone(memory_format=torch.contiguous_format)
+
+
 def token_logprob_fwd(logits: torch.Tensor, target: torch.Tensor):
     """(log-probability of target[r] under softmax(logits[r]), log-sum-exp of row r), float32
     [rows], from bf16 logits [rows, vocab] read once."""
-    logits = _check_hp(logits)
+    logits = _logprob_rows(logits)
     if target.dtype != torch.int64 or target.shape != (logits.shape[0],) or target.device != logits.device:
         raise TypeError("target must be int64 [rows] on the logits' device")
     target = target.contiguous()
@@ -786,7 +792,7 @@ def token_logprob_fwd(logits: torch.Tensor, target: torch.Tensor):
 def token_logprob_bwd(logits: torch.Tensor, target: torch.Tensor, lse: torch.Tensor,
                       grad_logprob: torch.Tensor) -> torch.Tensor:
     """Gradient of `token_logprob_fwd`'s first output with respect to the logits, bf16."""
-    logits = _check_hp(logits)
+    logits = _logprob_rows(logits)
     rows, vocab = logits.shape
     g = grad_logprob.to(torch.float32).contiguous()
     lse, target = lse.contiguous(), target.contiguous()

@@ -61,6 +61,23 @@ def test_log_probs_of_rows_that_overlap(device, vocab):
         assert all(torch.equal(a, b) for a, b in zip(*results))
 
 
+@pytest.mark.parametrize("vocab", [1, 7, 8, 1000, 2047, 8192, 8200, 12288, 12289])
+@pytest.mark.parametrize("rows", [512, 513])
+def test_log_probs_of_many_short_rows(device, rows, vocab):
+    """On either side of the rows that half a workgroup takes: as above, within 1e-5."""
+    g = torch.Generator(device=device).manual_seed(vocab)
+    logits = (torch.randn((rows, vocab), generator=g, device=device) * 4).to(torch.bfloat16)
+    logits[1], logits[3, 0] = float("-inf"), float("nan")
+    logits[1, -1] = 0.5
+    target = torch.randint(0, vocab, (rows,), generator=g, device=device)
+    target[1] = vocab - 1
+    lp, lse = ops.token_logprob_fwd(logits, target)
+    want = torch.log_softmax(logits.double(), dim=-1).gather(1, target[:, None])[:, 0]
+    fine = torch.arange(rows, device=device) != 3
+    assert lp[3].isnan() and lse[3].isnan() and (lp.double() - want)[fine].abs().max() <= 1e-5
+    assert (lse.double() - torch.logsumexp(logits.double(), dim=-1))[fine].abs().max() <= 1e-5
+
+
 def test_parts_follow_the_number_of_rows():
     assert ops._logprob_splits(16, 151936) == 12 and ops._logprob_splits(64, 151936) == 4
     assert ops._logprob_splits(256, 151936) == 1 and ops._logprob_splits(16, 8192) == 1

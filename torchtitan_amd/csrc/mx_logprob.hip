@@ -7,7 +7,7 @@
 namespace mx {
 
 constexpr int kLpThreads = 256;
-constexpr int kLpFwdThreads = 512;
+constexpr int kLpFwdThreads = 512, kLpFwdThreadsShort = 256;
 constexpr int kLpUnroll = 4;
 constexpr int kLpBwdUnroll = 2;
 
@@ -43,13 +43,13 @@ __device__ __forceinline__ void lp_finish(const uint16_t* row, int64_t vocab, in
 // for token_logprob_merge_kernel.  HBM-bound: what counts is bytes in flight, so a lane asks for
 // four 16-byte pieces before it uses the first, and rows are cut until the chip is full (a sample of
 // a few hundred generated tokens has fewer rows than the chip has room for workgroups).
-// 457 rows x 151 936: 53.7 us with one 256-lane workgroup per row and one piece in flight, 28.7 us now
-// (4.8 TB/s); 16 rows: 54 before, 7.0 us in 12 parts each (16.0 uncut).
-template <bool SPLIT>
-__global__ __launch_bounds__(kLpFwdThreads) void token_logprob_fwd_kernel(
+// 457 rows x 151 936: 52.6 us with one 256-lane workgroup per row and one piece in flight, 25.0 us now
+// (5.5 TB/s); 16 rows: 54 before, 6.7 us in 12 parts each (16.0 uncut).
+template <int THREADS, bool SPLIT>
+__global__ __launch_bounds__(THREADS) void token_logprob_fwd_kernel(
     const uint16_t* __restrict__ logits, int64_t ld, int64_t vocab, const int64_t* __restrict__ target,
     float* __restrict__ lp, float* __restrict__ lse, int splits, float2* __restrict__ partial) {
-  constexpr int kWaves = kLpFwdThreads / 64;
+  constexpr int kWaves = THREADS / 64;
   __shared__ float sm[kWaves], ss[kWaves];
   const int64_t r = SPLIT ? blockIdx.x / splits : blockIdx.x;
   const int part = SPLIT ? (int)(blockIdx.x - r * splits) : 0;
@@ -59,16 +59,16 @@ __global__ __launch_bounds__(kLpFwdThreads) void token_logprob_fwd_kernel(
   const int64_t chunks = vocab / 8;
   const int64_t per = SPLIT ? (chunks + splits - 1) / splits : chunks;
   const int64_t lo = part * per, hi = lo + per < chunks ? lo + per : chunks;
-  for (int64_t c = lo + tid; c < hi; c += kLpFwdThreads * kLpUnroll) {
+  for (int64_t c = lo + tid; c < hi; c += THREADS * kLpUnroll) {
     u32x4 v[kLpUnroll];
 #pragma unroll
     for (int u = 0; u < kLpUnroll; ++u) {
-      const int64_t cu = c + u * kLpFwdThreads;
-      v[u] = u32x4{0xFF80FF80u, 0xFF80FF80u, 0xFF80FF80u, 0xFF80FF80u};  // -inf: adds nothing
+      const int64_t cu = c + u * THREADS;
       if (cu < hi) v[u] = lp_load8(row + cu * 8);
     }
 #pragma unroll
     for (int u = 0; u < kLpUnroll; ++u) {
+      if (c + u * THREADS >= hi) break;  // (no exponentials of nothing: 16384 rows x 8192 67 us with them, 50 without)
       const float x[8] = {lp_bf16(v[u].x & 0xFFFFu), lp_bf16(v[u].x >> 16), lp_bf16(v[u].y & 0xFFFFu),
                           lp_bf16(v[u].y >> 16),     lp_bf16(v[u].z & 0xFFFFu), lp_bf16(v[u].z >> 16),
                           lp_bf16(v[u].w & 0xFFFFu), lp_bf16(v[u].w >> 16)};
@@ -90,7 +90,7 @@ __global__ __launch_bounds__(kLpFwdThreads) void token_logprob_fwd_kernel(
     }
   }
   if (!SPLIT || part == splits - 1)
-    for (int64_t i = chunks * 8 + tid; i < vocab; i += kLpFwdThreads) {
+    for (int64_t i = chunks * 8 + tid; i < vocab; i += THREADS) {
       const float x = lp_bf16(row[i]);
       lse_merge(m, s, x, x == -__builtin_inff() ? 0.f : 1.f);
     }
@@ -192,13 +192,19 @@ extern "C" int mx_token_logprob_fwd_split(const void* logits, int64_t rows, int6
     return MX_ERR_ALIGNMENT;
   if (rows > 0x7FFFFFFF || splits > 65535 || rows * splits > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
-  const dim3 grid((unsigned)(rows * splits)), block(kLpFwdThreads);
+  const dim3 grid((unsigned)(rows * splits)), block(kLpFwdThreads), small(kLpFwdThreadsShort);
+  auto whole_rows = [&](auto kernel, dim3 lanes) {
+    hipLaunchKernelGGL(kernel, grid, lanes, 0, st, (const uint16_t*)logits, ld, vocab, target, logprob, lse, 1, (float2*)nullptr);
+  };
   if (splits == 1) {
-    hipLaunchKernelGGL(token_logprob_fwd_kernel<false>, grid, block, 0, st, (const uint16_t*)logits, ld, vocab, target,
-                       logprob, lse, 1, (float2*)nullptr);
+    // Rows that 512 lanes read with four pieces in flight half empty, and more of them than the chip holds at
+    // once: half the lanes, us, 512 / 256: 16384 rows x 8192 49.7 / 39.2, 2000 rows x 1000 5.2 / 3.7, x 8192
+    // 8.4 / 7.6, x 12288 10.0 / 9.7; 4096 rows x 16000 21.3 / 22.6, x 32000 39.4 / 42.9; 16 rows x 8192 3.3 / 3.8
+    if (vocab <= 12288 && rows > 512) whole_rows(token_logprob_fwd_kernel<kLpFwdThreadsShort, false>, small);
+    else whole_rows(token_logprob_fwd_kernel<kLpFwdThreads, false>, block);
   } else {
-    hipLaunchKernelGGL(token_logprob_fwd_kernel<true>, grid, block, 0, st, (const uint16_t*)logits, ld, vocab, target,
-                       logprob, lse, (int)splits, (float2*)partial);
+    hipLaunchKernelGGL((token_logprob_fwd_kernel<kLpFwdThreads, true>), grid, block, 0, st, (const uint16_t*)logits, ld,
+                       vocab, target, logprob, lse, (int)splits, (float2*)partial);
     hipLaunchKernelGGL(token_logprob_merge_kernel, dim3((unsigned)((rows + 63) / 64)), dim3(64), 0, st,
                        (const uint16_t*)logits, ld, vocab, target, rows, (int)splits, (const float2*)partial, logprob, lse);
   }

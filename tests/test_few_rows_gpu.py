@@ -109,3 +109,16 @@ def test_cached_casts_of_another_form(device):
     got, _, _ = mx_tensor._linear_forward(x, w, cfg, False, False)
     mx_tensor._weight_cache.clear()
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("K", [256, 512])
+@pytest.mark.parametrize("N", [16384, 16400])
+def test_products_on_either_side_of_the_widest(device, N, K):
+    """Where few rows go to workgroups of their own or to tiles."""
+    w = _values(N, K, device, 1) * 0.1
+    wq, wd = ops.to_operands(w, "rceil", True, False, 128)[0], _dequantized(w, "rceil")
+    for M in (1, 16, 17, 64):
+        x = _values(M, K, device, M)
+        _check(ops.mx_gemm_nt(ops.to_operands(x, "rceil", True, False, 128)[0], wq), _dequantized(x, "rceil"), wd)
+        with torch.no_grad():
+            assert ops.few_rows_ok(x, N) == (M <= ops.FEW_ROWS and N <= 16384)

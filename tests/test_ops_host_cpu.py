@@ -124,7 +124,7 @@ def test_mismatched_modules_raise(no_launches, monkeypatch, grad, tokens):
 
     cfg = mx_tensor.MXFP8Config()
     x = _bf16(tokens, 2016)
-    monkeypatch.setattr(ops, "few_rows_ok", lambda t: t.shape[0] <= ops.FEW_ROWS)
+    monkeypatch.setattr(ops, "few_rows_ok", lambda t, columns: t.shape[0] <= ops.FEW_ROWS)
     weight = lambda *shape: mx_tensor.MXFP8TrainingWeight(_bf16(*shape).requires_grad_(grad), cfg)
     mismatched = (lambda: mx_tensor.mx_linear(x, weight(512, 2048).as_subclass(torch.Tensor), None, cfg),
                   lambda: mx_blocks.mx_feed_forward(x, weight(2048, 2048), weight(2016, 2048), weight(2048, 2048)),

@@ -106,9 +106,10 @@ static int gemm_nt_pitched(const uint8_t* a_codes, const uint8_t* a_scales, cons
   if (256 * ldk > 0x7FFFFFFFll) return MX_ERR_UNSUPPORTED;
   DenseArgs p{a_codes, a_scales, b_codes, b_scales, (uint16_t*)d, M, N, K, ldd, ldk};
   hipStream_t st = (hipStream_t)stream;
-  // few rows: a workgroup for every 16 columns and more, its waves along the contraction; faster than the
-  // tiles at every size measured up to here (64 rows 4096 x 14336: 23 vs 28 us; others in mx_few_rows.hip)
-  if (M <= 64 && K % 128 == 0 && force_kernel == 0)
+  // Few rows: a workgroup for every 16 columns and more, its waves along the contraction, while its widest
+  // workgroups fit the CUs in one round: 64 rows 2048 -> 16384 13.6 us, 16.4 on tiles; 20480 25.1 and 16.9,
+  // 151936 127.8 and 86.8.
+  if (M <= 64 && K % 128 == 0 && force_kernel == 0 && N <= 16384)
     return launch_few_rows_codes(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldk, ldd, st);
   if (M <= 128 || N <= 128 || force_kernel == 2) return launch_dense<128, 128>(p, st);
   // Few 256x256 tiles leave most CUs of the persistent kernel idle when the contraction is not

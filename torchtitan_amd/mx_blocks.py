@@ -151,7 +151,8 @@ def ffn_forward(x2, x_src, w1, w2, w3, cfg: MXFP8Config, need_dx: bool, need_dw:
     carry it into the backward); `whole_blocks`: see `_FFNCasts`.  The eager autograd function and
     the traced operator both run this."""
     cast = _FFNCasts(cfg, whole_blocks, pad)
-    if whole_blocks and norm_weight is None and not (need_dx or need_dw) and ops.few_rows_ok(x2):
+    if (whole_blocks and norm_weight is None and not (need_dx or need_dw)
+            and ops.few_rows_ok(x2, w1.shape[0] + w3.shape[0])):
         (w1q0, _), (w3q0, _), (w2q0, _) = cast.weights((w1, w3, w2), (False, False, False))
         h13 = ops.mx_few_rows(x2, w1q0, cfg.scale_mode, w3q0)
         return ops.mx_gemm_nt(cast.gate(h13, False)[0], w2q0), dict.fromkeys(FFN_SAVED)

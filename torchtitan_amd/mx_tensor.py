@@ -261,7 +261,7 @@ def _linear_forward(x, weight, cfg: MXFP8Config, need_dx: bool, need_dw: bool):
     # rows further apart than they are long, except with cached weight casts, which the fused
     # blocks and the hand-over share without a pitch
     pad = 0 if cfg.cache_weight_casts else ops.CODE_PITCH_PAD
-    if not (need_dx or need_dw) and ops.few_rows_ok(x2):
+    if not (need_dx or need_dw) and ops.few_rows_ok(x2, N):
         wq0, _ = _cast_weight(weight, mode, False, cfg, pitch_pad=pad)
         y = ops.mx_few_rows(x2, wq0, mode)
         return (y if x.dim() == 2 else y.view(*x.shape[:-1], N)), None, None

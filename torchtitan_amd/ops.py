@@ -987,16 +987,18 @@ def _gemm_operands(a: Operand, b: Operand, out: torch.Tensor) -> torch.Tensor:
 
 FEW_ROWS = 32             # rows that `mx_few_rows` takes
 FEW_ROWS_VALUES = 65536   # values of x, rows counted in whole 16s, up to which it is chosen
+FEW_ROWS_COLUMNS = 16384  # columns of all products, up to which it is chosen
 
 
-def few_rows_ok(x: torch.Tensor) -> bool:
-    """`mx_few_rows` runs the products of x: bf16 rows on the GPU in whole blocks of 32, few enough of them,
-    and no dispatch mode that would want to see the GEMM.  Every workgroup casts all of x, so the line is
-    where that costs more than the launch it saves (a cast of its own: 3.7 us on the GPU, about 10 on the
-    host): 16 x 4096 -> 4096 10.7 us in one launch, 3.7 + 7.5 in two; 32 x 2048 -> 6144 12.6, 3.7 + 7.4;
-    32 x 14336 -> 4096 42, 3.8 + 27."""
+def few_rows_ok(x: torch.Tensor, columns: int) -> bool:
+    """`mx_few_rows` runs the products of x with weights of `columns` rows in all: bf16 rows on the GPU in whole
+    blocks of 32, few enough of them, and no dispatch mode that would want to see the GEMM.  Every workgroup
+    casts all of x, so the line is where that costs more than the launch it saves (a cast of its own: 3.7 us
+    on the GPU, about 10 on the host): 16 x 4096 -> 4096 10.7 us in one launch, 3.7 + 7.5 in two; 32 x 2048 ->
+    6144 12.6, 3.7 + 7.4; 32 x 14336 -> 4096 42, 3.8 + 27; and where the workgroups outnumber the CUs: 16 x 2048
+    -> 16384 14.0 and 14.2, -> 2 x 14336 25.8 and 23.5, -> 151936 123 and 80 us."""
     return (x.dtype == torch.bfloat16 and x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= FEW_ROWS
-            and (x.shape[0] + 15 & ~15) * x.shape[1] <= FEW_ROWS_VALUES and x.shape[1] % BLOCK == 0 and x.shape[1] > 0
+            and columns <= FEW_ROWS_COLUMNS and (x.shape[0] + 15 & ~15) * x.shape[1] <= FEW_ROWS_VALUES and x.shape[1] % BLOCK == 0 and x.shape[1] > 0
             and x.stride(1) == 1 and not _watched())
 
 

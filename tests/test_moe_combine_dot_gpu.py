@@ -37,6 +37,23 @@ def test_combine_dot_equals_combine_and_row_dot(device, tokens, k, cols):
     assert out is None and torch.equal(got, dots)
 
 
+@pytest.mark.parametrize("k", [0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 11, 13, 16, 17, 26])
+def test_combine_over_any_number_of_choices(device, k):
+    """Bit-exact against the oracle in every number of rows that are asked for together, of one matrix and of two."""
+    tokens, cols = 37, 264
+    rng = np.random.default_rng(k)
+    rows = tokens * k + 3
+    y, y2 = (bf16_from_bits(randn_bits(rng, (rows, cols)), device) for _ in range(2))
+    pos = rng.permutation(rows)[: tokens * k].astype(np.int64).reshape(tokens, k)
+    if k:
+        pos[0, 0], pos[-1, -1] = rows, -1
+    w = rng.random((tokens, k)).astype(np.float32)
+    tp, tw = torch.from_numpy(pos).to(device), torch.from_numpy(w).to(device)
+    for weights, tweights in ((w, tw), (None, None)):
+        assert np.array_equal(bits_of(ops.moe_combine(y, tp, tweights)), mo.moe_combine(bits_of(y), pos, weights))
+        assert np.array_equal(bits_of(ops.moe_combine(y, tp, tweights, y2)), mo.moe_combine(bits_of(y + y2), pos, weights))
+
+
 def test_no_rows_give_zeros(device):
     x = torch.ones((2, 64), dtype=torch.bfloat16, device=device)
     pos = torch.zeros((2, 3), dtype=torch.int64, device=device)

@@ -159,7 +159,8 @@ def test_gradients_whose_rows_are_one_expanded_row(device, tokens, block):
 
 
 # tile counts around the walk's bands of 32 tile rows and strips of 2 (both forms) and of 2 and 32 (rows alone)
-@pytest.mark.parametrize("tile_rows,tile_cols", [(32, 2), (33, 1), (33, 3), (31, 33), (3, 65), (65, 5)])
+@pytest.mark.parametrize("tile_rows,tile_cols", [(32, 2), (33, 1), (33, 3), (31, 33), (3, 65), (65, 5),
+                                                 (64, 4), (4, 64)])
 def test_every_tile_of_the_walk_is_cast_once(device, tile_rows, tile_cols):
     rows, cols = 128 * tile_rows - 5, 128 * tile_cols - 32
     x = _values(rows, cols, device, tile_rows)

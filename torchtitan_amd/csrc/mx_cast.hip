@@ -448,6 +448,14 @@ struct TileWalk {
   static constexpr uint32_t BY = COL ? MX_CAST_COL_BY : MX_CAST_ROW_BY;
   // tile (bx, by) of a gx x gy grid at place `id` of the walk; id < gx * gy, which fits 31 bits
   static __device__ __forceinline__ void at(uint32_t id, uint32_t gx, uint32_t gy, uint32_t& bx, uint32_t& by) {
+    // whole bands and strips: one division by a number not known here, which a launch of one round feels
+    // (4096 x 4096 13.3 us so, 13.9 with the three below)
+    if (gx % BX == 0 && gy % BY == 0) {
+      const uint32_t block = id / (BX * BY), in = id % (BX * BY), strips = gx / BX;
+      bx = (block % strips) * BX + in / BY;
+      by = (block / strips) * BY + in % BY;
+      return;
+    }
     const uint32_t band = id / (gx * min(BY, gy));
     const uint32_t in_band = id - band * (gx * min(BY, gy)), h = min(BY, gy - band * BY);
     const uint32_t strip = in_band / (BX * h), in = in_band - strip * (BX * h);

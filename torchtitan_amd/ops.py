@@ -765,26 +765,22 @@ def _logprob_splits(rows: int, vocab: int) -> int:
     return max(1, min(-(-256 // rows), vocab // 12288))
 
 
-def _logprob_rows(logits: torch.Tensor) -> torch.Tensor:
-    """bf16 logits [rows, vocab] whose rows follow one another (a copy of expanded ones)."""
-    logits = _check_hp(logits)
-    return logits if logits.stride(0) >= logits.shape[1] else logits.clone(memory_format=torch.contiguous_format)
-
-
 def token_logprob_fwd(logits: torch.Tensor, target: torch.Tensor):
     """(log-probability of target[r] under softmax(logits[r]), log-sum-exp of row r), float32
     [rows], from bf16 logits [rows, vocab] read once."""
-    logits = _logprob_rows(logits)
+    logits = _check_hp(logits)
     if target.dtype != torch.int64 or target.shape != (logits.shape[0],) or target.device != logits.device:
         raise TypeError("target must be int64 [rows] on the logits' device")
     target = target.contiguous()
-    rows, vocab = logits.shape
+    (rows, vocab), ld = logits.shape, logits.stride(0)
+    if ld < vocab:  # rows that overlap
+        logits, ld = logits.clone(memory_format=torch.contiguous_format), vocab
     lp = torch.empty(rows, dtype=torch.float32, device=logits.device)
     lse = torch.empty(rows, dtype=torch.float32, device=logits.device)
     splits = _logprob_splits(rows, vocab) if rows else 1
     partial = torch.empty(2 * rows * splits, dtype=torch.float32, device=logits.device) if splits > 1 else None
     _call("mx_token_logprob_fwd_split", "token_logprob_fwd", logits.device, _ptr(logits), rows, vocab,
-          logits.stride(0), _ptr(target), _ptr(lp), _ptr(lse), splits, _ptr(partial) if splits > 1 else None,
+          ld, _ptr(target), _ptr(lp), _ptr(lse), splits, _ptr(partial) if splits > 1 else None,
           _stream(logits))
     return lp, lse
 
@@ -792,14 +788,16 @@ def token_logprob_fwd(logits: torch.Tensor, target: torch.Tensor):
 def token_logprob_bwd(logits: torch.Tensor, target: torch.Tensor, lse: torch.Tensor,
                       grad_logprob: torch.Tensor) -> torch.Tensor:
     """Gradient of `token_logprob_fwd`'s first output with respect to the logits, bf16."""
-    logits = _logprob_rows(logits)
-    rows, vocab = logits.shape
+    logits = _check_hp(logits)
+    (rows, vocab), ld = logits.shape, logits.stride(0)
+    if ld < vocab:
+        logits, ld = logits.clone(memory_format=torch.contiguous_format), vocab
     g = grad_logprob.to(torch.float32).contiguous()
     lse, target = lse.contiguous(), target.contiguous()
     out = torch.empty((rows, -(-vocab // 8) * 8), dtype=torch.bfloat16, device=logits.device)
     if vocab % 8:
         out = out[:, :vocab]
-    step, ld, ldo = 65535, logits.stride(0), out.stride(0)  # (one grid row per token row)
+    step, ldo = 65535, out.stride(0)  # (one grid row per token row)
     for lo in range(0, rows, step):
         _call("mx_token_logprob_bwd_any", "token_logprob_bwd", logits.device, _ptr(logits) + 2 * lo * ld,
               min(step, rows - lo), vocab, ld, _ptr(target) + 8 * lo, _ptr(lse) + 4 * lo, _ptr(g) + 4 * lo,

@@ -155,3 +155,30 @@ def test_a_cached_cast_is_given_in_the_form_its_caller_wants(no_launches):
         assert type(q) is MXData and torch.equal(q.codes, d.codes) and torch.equal(q.scales, d.scales)
     with pytest.raises(ValueError):
         ops.Operand.of(MXData(_codes(128, 160), torch.zeros(1280, dtype=torch.uint8), MX_SCALES_MFMA))
+
+
+@pytest.mark.parametrize("tokens,dim,hidden,norm", [(64, 128, 256, False), (96, 160, 224, False), (160, 256, 416, True)])
+@pytest.mark.parametrize("need_dx,need_dw", [(True, True), (True, False), (False, True)])
+def test_traced_block_has_the_shapes_that_its_fake_kernel_gives(no_launches, monkeypatch, tokens, dim, hidden, norm, need_dx,
+                                                               need_dw):
+    """The operators' bodies with the launches left out against their fake kernels, forward and backward."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from torchtitan_amd import compiled, mx_blocks
+
+    monkeypatch.setattr(mx_blocks, "_rms_norm_backward",  # (torch's own is for the GPU)
+                        lambda dx, x, rstd, w, need_x, need_w: (dx if need_x else None, w.clone() if need_w else None))
+
+    def run(fwd, bwd):
+        x, w1, w2, w3 = _bf16(tokens, dim), _bf16(hidden, dim), _bf16(dim, hidden), _bf16(hidden, dim)
+        n = torch.ones(dim, dtype=torch.bfloat16) if norm else None
+        out = fwd(x, w1, w2, w3, n, 1e-5, 1, False, need_dx, need_dw)
+        return *out, *bwd(_bf16(tokens, dim), list(out[1:]), x if norm else None, n, 1, need_dx, need_dw, need_dw, need_dw,
+                          norm and need_dx)
+
+    real = run(compiled.mx_ffn_fwd._init_fn, compiled.mx_ffn_bwd._init_fn)
+    with FakeTensorMode():
+        fake = run(torch.ops.torchtitan_amd.mx_ffn_fwd, torch.ops.torchtitan_amd.mx_ffn_bwd)
+    assert [t.shape for t in real] == [t.shape for t in fake] and [t.dtype for t in real] == [t.dtype for t in fake]
+    storages = [t.untyped_storage().data_ptr() for t in real[1:15] if t.numel()]
+    assert len(set(storages)) == len(storages)

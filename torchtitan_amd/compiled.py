@@ -453,12 +453,19 @@ def mx_ffn_fwd(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, w3: torch.Te
     x2 = x.reshape(-1, D)
     if x2.dtype != torch.bfloat16:
         x2 = x2.to(torch.bfloat16)
-    y, saved = mx_blocks.ffn_forward(x2, None, w1, w2, w3, _block_cfg(mode, cache_w), need_dx, need_dw, norm_weight, eps)
-    if cache_w:  # an operator's outputs are its own: not the cache's tensors
-        for name in ("w1", "w2", "w3"):
-            q = saved[name]
-            saved[name] = None if q is None else MXData(q.codes.clone(), q.scales.clone(), MX_SCALES_MFMA)
+    y, saved = mx_blocks.ffn_forward(x2, None, w1, w2, w3, _block_cfg(mode, cache_w), need_dx, need_dw, norm_weight, eps,
+                                     whole_blocks=_ffn_whole_blocks(x2.shape[0], D, w1.shape[0], w2.shape[0]))
+    for name in _FFN_PAIRS:  # an operator's outputs are their own: not the cache's tensors, nor parts of one buffer
+        q = saved[name]
+        if type(q) is ops.Operand or (q is not None and cache_w and name in ("w1", "w2", "w3")):
+            saved[name] = MXData(q.codes.clone(), q.scales.clone(), MX_SCALES_MFMA)
     return (y.view(*x.shape[:-1], w2.shape[0]), *_filled(_ffn_slots(saved), x.device, skip=(11, 13)))
+
+
+def _ffn_whole_blocks(*sizes) -> bool:
+    """Some size is no multiple of 128: the block is cast in whole blocks as the eager one is, so that its products
+    run on the same kernels.  (Otherwise that is the same as the exact sizes, whose casts write tensors of their own.)"""
+    return any(n % ops.WHOLE_BLOCK for n in sizes)
 
 
 # mx_blocks.FFN_SAVED as the operator's 14 tensors: an MXData takes two slots, codes and scales
@@ -473,9 +480,13 @@ def _ffn_slots(saved: dict) -> list:
     return slots + [saved["norm_x"], saved["rstd"], saved["norm_weight"]]
 
 
-def _ffn_saved(slots: list) -> dict:
-    saved = {name: None if slots[1 + 2 * i] is None else MXData(slots[1 + 2 * i], slots[2 + 2 * i], MX_SCALES_MFMA)
-             for i, name in enumerate(_FFN_PAIRS)}
+def _ffn_saved(slots: list, depths: tuple | None) -> dict:
+    """`depths`: in whole blocks, the contraction that each of _FFN_PAIRS was cast from."""
+    saved = {}
+    for i, name in enumerate(_FFN_PAIRS):
+        codes, scales = slots[1 + 2 * i:3 + 2 * i]
+        saved[name] = (None if codes is None else MXData(codes, scales, MX_SCALES_MFMA) if depths is None
+                       else ops.Operand.around(codes, scales, depths[i]))
     return dict(saved, h13=slots[0], norm_x=slots[11], rstd=slots[12], norm_weight=slots[13])
 
 
@@ -487,12 +498,18 @@ def _(x, w1, w2, w3, norm_weight, eps, mode, cache_w, need_dx, need_dw):
                  lambda: "the traced SwiGLU block needs tokens and sizes that are multiples of 32")
     dev = x.device
     s = [_empty(dev) for _ in range(14)]
+    step = ops.WHOLE_BLOCK if _ffn_whole_blocks(M, D, H, O) else 1
+
+    def pair(rows, k):
+        k = -(-k // step) * step
+        return [_u8((rows, k), dev), _mfma(rows, k // 32, dev)]
+
     if need_dx or need_dw:
-        s[0:3] = [torch.empty((2, M, H), dtype=torch.bfloat16, device=dev), _u8((H, O), dev), _mfma(H, O // 32, dev)]
+        s[0:3] = [torch.empty((2, M, H), dtype=torch.bfloat16, device=dev), *pair(H, O)]
     if need_dw:
-        s[3:7] = [_u8((D, M), dev), _mfma(D, M // 32, dev), _u8((H, M), dev), _mfma(H, M // 32, dev)]
+        s[3:7] = [*pair(D, M), *pair(H, M)]
     if need_dx:
-        s[7:11] = [_u8((D, H), dev), _mfma(D, H // 32, dev), _u8((D, H), dev), _mfma(D, H // 32, dev)]
+        s[7:11] = [*pair(D, H), *pair(D, H)]
         if norm_weight is not None:
             s[12] = torch.empty((M,), dtype=torch.float32, device=dev)
     return (x.new_empty((*x.shape[:-1], O), dtype=torch.bfloat16), *s)
@@ -510,8 +527,11 @@ def mx_ffn_bwd(dy: torch.Tensor, saved: list[torch.Tensor], x: torch.Tensor | No
     dy2 = dy.reshape(-1, dy.shape[-1])
     if dy2.dtype != torch.bfloat16:
         dy2 = dy2.to(torch.bfloat16)
-    dx, dw1, dw2, dw3, dnw = mx_blocks.ffn_backward(dy2.contiguous(), _ffn_saved(s), _block_cfg(mode, False), need_x,
-                                                    need_dw1, need_dw2, need_dw3, need_dnw)
+    (M, O), H, D = dy2.shape, s[0].shape[2], (s[7] if s[7] is not None else s[3]).shape[0]
+    whole = _ffn_whole_blocks(M, D, H, O)
+    dx, dw1, dw2, dw3, dnw = mx_blocks.ffn_backward(dy2.contiguous(), _ffn_saved(s, (O, M, M, H, H) if whole else None),
+                                                    _block_cfg(mode, False), need_x, need_dw1, need_dw2, need_dw3,
+                                                    need_dnw, whole_blocks=whole)
     none = lambda: torch.empty((0,), dtype=torch.bfloat16, device=dy.device)
     return (dx if (dx is not None and need_x) else none(), _pack_pair(dw1, dw3, dy.device),
             dw2 if dw2 is not None else none(), dnw if dnw is not None else none())

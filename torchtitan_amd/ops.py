@@ -201,13 +201,15 @@ class Operand:
     whole 128-deep blocks, `depth` how much of it is not zero fill: what the other operand must agree
     with.  One buffer and plain
     numbers instead of two to four tensors and their views: at small sizes making those takes the
-    host longer than the GPU needs for the cast."""
+    host longer than the GPU needs for the cast.  (`scales_buf`: the scales' own buffer, where they have
+    one: an operand `around` two tensors.)"""
 
-    __slots__ = ("buf", "rows", "k", "ld", "at", "scales_at", "depth")
+    __slots__ = ("buf", "rows", "k", "ld", "at", "scales_at", "depth", "scales_buf")
     scale_order = MX_SCALES_MFMA
 
-    def __init__(self, buf: torch.Tensor, layout):
+    def __init__(self, buf: torch.Tensor, layout, scales_buf: torch.Tensor | None = None):
         self.buf = buf
+        self.scales_buf = buf if scales_buf is None else scales_buf
         self.rows, self.k, self.ld, self.at, self.scales_at, self.depth = layout
 
     @property
@@ -221,7 +223,7 @@ class Operand:
 
     @property
     def scales(self) -> torch.Tensor:
-        return self.buf[self.scales_at:self.scales_at + mfma_scale_bytes(self.rows, self.k // BLOCK)]
+        return self.scales_buf[self.scales_at:self.scales_at + mfma_scale_bytes(self.rows, self.k // BLOCK)]
 
     @property
     def codes_ptr(self) -> int:
@@ -229,11 +231,11 @@ class Operand:
 
     @property
     def scales_ptr(self) -> int:
-        return self.buf.data_ptr() + self.scales_at
+        return self.scales_buf.data_ptr() + self.scales_at
 
     def first_rows(self, n: int) -> "Operand":
         """The operand's first n rows (n rounds up to the same multiple of 128)."""
-        return Operand(self.buf, (n, self.k, self.ld, self.at, self.scales_at, self.depth))
+        return Operand(self.buf, (n, self.k, self.ld, self.at, self.scales_at, self.depth), self.scales_buf)
 
     @classmethod
     def of(cls, q: MXData) -> "Operand":
@@ -245,6 +247,12 @@ class Operand:
         out.codes.copy_(q.codes)
         out.scales.copy_(q.scales)
         return out
+
+    @classmethod
+    def around(cls, codes: torch.Tensor, scales: torch.Tensor, depth: int) -> "Operand":
+        """Dense codes [rows, whole blocks] of a contraction of `depth`, and their scales, as they lie."""
+        rows, k = codes.shape
+        return cls(codes, (rows, k, k, 0, 0, depth), scales)
 
     def data(self) -> MXData:
         return MXData(self.codes, self.scales, MX_SCALES_MFMA)

@@ -96,7 +96,7 @@ def test_modules_without_gradients(device, tokens):
 
 
 def test_cached_casts_of_another_form(device):
-    """A dense cached weight cast, as a traced forward leaves it, is used as it is."""
+    """A dense cached weight cast, as a traced forward leaves it, serves an eager forward without gradients."""
     from torchtitan_amd import mx_tensor
 
     cfg = mx_tensor.MXFP8Config(cache_weight_casts=True)

@@ -8,7 +8,9 @@ The eager path of this package calls the HIP library through ``ctypes`` inside
 backward operator registered with ``torch.library`` (schemas, fake kernels for shape
 propagation, an autograd formula), whose bodies run the same casts and GEMMs as the eager
 functions.  A compiled block therefore holds the MXFP8 linears as single nodes with no graph
-break, and its results equal the eager ones bit for bit.
+break, and its results equal the eager ones bit for bit (but for linears of 64 tokens or fewer
+with sizes that are no multiple of 128: eager ones run on whole 128-deep blocks, there on a kernel
+that adds up in another order, and a last bit may differ).
 
 ``torch._grouped_mm`` on a converted 3-D weight traces the same way (the reference compiles MoE
 blocks too, torchtitan/models/llama4/parallelize.py ``apply_compile``): one forward and one

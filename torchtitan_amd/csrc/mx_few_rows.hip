@@ -6,8 +6,8 @@
 // takes 16 to 64 columns of the output and its eight waves take turns along the contraction, fragments
 // straight from memory into registers (a workgroup reads nothing twice, LDS has nothing to share), the next
 // step's on their way while one is multiplied; the eight partial sums meet in LDS.  Codes of 16 / 64
-// rows, us, 128 x 128 tiles and now: 2048 x 6144 13.5 / 14.6, 6.4 / 9.1; 4096 x 4096 23.5 / 24.6, 7.5 / 13.1;
-// 14336 x 4096 83 / 85, 20 / 39.  bf16 rows are cast in registers, with the codes and scales of the
+// rows, us, 128 x 128 tiles and now: 2048 x 6144 13.1 / 14.3, 6.6 / 9.7; 4096 x 4096 23.5 / 24.4, 7.3 / 13.1;
+// 14336 x 4096 83 / 84, 20 / 39.  bf16 rows are cast in registers, with the codes and scales of the
 // casts, and save the launch in front: 16 rows 9.6, 10.7 and 26 us.
 #include "mx_gemm_tile.h"
 

@@ -95,7 +95,7 @@ __global__ __launch_bounds__(THREADS) void token_logprob_fwd_kernel(
       lse_merge(m, s, x, x == -__builtin_inff() ? 0.f : 1.f);
     }
   // across the workgroup: the maximum first, then one rescaling per lane and plain sums (merging
-  // pairs step by step takes two exponentials a step: 2000 rows x 8192 12.5 us that way, 11.1 so)
+  // pairs step by step takes two exponentials a step and an eighth more time at 2000 rows x 8192)
   float top = m;
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off, 64));

@@ -768,8 +768,8 @@ def mx_dequant_many(data) -> list:
 def _logprob_splits(rows: int, vocab: int) -> int:
     """Parts that the forward cuts every row of logits into: enough for one workgroup per CU, none
     of less than 12 288 logits (a workgroup asks for 16 384 at once; smaller parts cost more in
-    reductions than they spread).  Vocabulary 151 936, uncut against so cut: 16 rows 16.0 -> 7.0 us,
-    64 rows 16.6 -> 9.9, 200 rows 20.1 -> 17.8; 300 rows 25.7 -> 23.8 at best, 457 rows 28.7 -> 30.5."""
+    reductions than they spread).  Vocabulary 151 936, uncut against so cut: 16 rows 13.4 -> 6.7 us,
+    64 rows 16.8 -> 9.2, 200 rows 17.5 -> 16.2; 300 rows 23.6 -> 20.2 at best, 457 rows 24.6 -> 27.0."""
     return max(1, min(-(-256 // rows), vocab // 12288))
 
 

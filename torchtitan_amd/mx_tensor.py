@@ -173,7 +173,7 @@ def _cast_weight(w: torch.Tensor, mode: str, need_cols: bool, cfg: MXFP8Config, 
     if cached:
         hit = _weight_cache.get(w, key)
         if hit is not None and (hit[1] is not None or not need_cols or w.shape[-2] % ops.BLOCK):
-            return _in_form(w, key, hit, whole)
+            return hit if (type(hit[0]) is ops.Operand) == whole else _in_form(w, key, hit, whole)
         need_cols = True  # cast once in full, whoever asks first
     wb = (_castable(w) if whole else w if w.dtype == torch.bfloat16 else w.to(torch.bfloat16)).contiguous()
     both = need_cols and (whole or wb.shape[-2] % ops.BLOCK == 0)
@@ -190,12 +190,10 @@ def _cast_weight(w: torch.Tensor, mode: str, need_cols: bool, cfg: MXFP8Config, 
 
 
 def _in_form(w: torch.Tensor, key, hit, whole: bool):
-    """A cached cast in the form its caller wants: operands, or dense `MXData` (views of an operand's buffer).
+    """A cached cast in the other form, which its caller wants: operands, or dense `MXData` (views of an operand's buffer).
     An operand made from a dense entry takes its place, except under graph capture, where it is filled
     by the replay only."""
     rows, cols = hit
-    if w.dim() != 2 or whole == (type(rows) is ops.Operand):
-        return hit
     if not whole:
         return rows.data(), (None if cols is None else cols.data())
     hit = ops.Operand.of(rows), (None if cols is None else ops.Operand.of(cols))

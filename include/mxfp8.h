@@ -368,10 +368,10 @@ int mx_gemm_nt(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b
                const uint8_t* b_scales, void* d, int64_t M, int64_t N, int64_t K, int64_t ldd,
                void* stream);
 
-/* The same GEMM for a caller that can lend scratch memory: shapes with few 256x256 output
- * tiles and a long contraction (the wgrad of a small weight over many tokens,
- * dW[N,K] = dY^T X with M in the tens of thousands) are then split along the contraction over
- * several workgroups per tile, float32 partial sums in `workspace`, one reduction pass.
+/* The same GEMM for a caller that can lend scratch memory: shapes with few output tiles and a
+ * contraction of more than 4096 (the wgrad of a small weight over many tokens, dW[N,K] = dY^T X with M
+ * in the tens of thousands; the down projection of some hundred tokens) are then split along the
+ * contraction over several workgroups per tile, float32 partial sums in `workspace`, one reduction pass.
  * mx_gemm_nt_workspace_bytes: bytes with which the shape would be split on the current device
  * (0: mx_gemm_nt_ws runs exactly what mx_gemm_nt runs).  workspace: device memory, 16-byte
  * aligned, contents undefined before and after; with less than the stated size (or NULL) the

@@ -22,6 +22,12 @@ void mx_debug_force_kernel(int which);
  * (also lowers how many tiles one grouped launch covers); 0: one per CU (default). */
 void mx_debug_set_grid(int workgroups);
 
+/* ta, tb > 0: dense products of the persistent kernel run on tiles of 64 ta x 64 tb (4x4, 3x4, 4x3, 2x4,
+ * 4x2; a split along K not on 3x4 and 4x3), whatever would suit the shape; slices > 0: K is split into as
+ * many slices where mx_gemm_nt_workspace_bytes may split it at all and no slice gets fewer than four
+ * 128-deep blocks.  0: by shape (default). */
+void mx_debug_set_tile(int ta, int tb, int slices);
+
 /* -DMX_TIMING_BUILD only.  Device buffer of 256 * 4 * 8 uint64 that the timing build of the persistent kernel fills with
  * per-wave cycle counts {copy wait, barriers, step body, epilogue, ...}; NULL switches the timing
  * build off (default). */

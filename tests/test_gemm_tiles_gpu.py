@@ -1,0 +1,100 @@
+"""The smaller tiles of the persistent GEMM (192 and 128 rows or columns) and their splits along K: at the
+edges of tiles, 128-row scale groups and 128-deep blocks, against the products of the same codes in float64 and
+against 256 x 256 tiles, whose sums every unsplit tile forms in the same order."""
+import numpy as np
+import pytest
+import torch
+
+from tests.helpers import bf16_from_bits, randn_bits
+from torchtitan_amd import _lib, ops
+
+pytestmark = pytest.mark.gpu
+
+TILES = [(4, 4), (3, 4), (4, 3), (2, 4), (4, 2)]
+
+
+@pytest.fixture
+def hooks():
+    lib = _lib.load()
+    yield lib
+    lib.mx_debug_set_tile(0, 0, 0)
+    lib.mx_debug_set_grid(0)
+
+
+def _operand(device, rng, rows, K, std=1.0):
+    """(pitched operand, what its codes and scales stand for, in float64)"""
+    x = bf16_from_bits(randn_bits(rng, (rows, K), std=std, outliers=1e-3), device)
+    q = ops.to_operands(x, "rceil", cols=False, pitch_pad=128)[0]
+    scales = torch.exp2(ops.scale_unlayout(q.scales.contiguous(), rows, q.k // 32).double() - 127)
+    return q, (q.codes.view(torch.float8_e4m3fn).double().view(rows, -1, 32) * scales[..., None]).view(rows, q.k)
+
+
+def _check(got, want):
+    """`got` is no further from `want` (float64) than its rounding to bf16 by more than 1 %: float32 sums of up to
+    a few thousand terms are off by less than 2^-18 of the terms' norm, a hundredth of the rounding's 2^-9 / sqrt(3) and
+    less, and errors of that size add in squares."""
+    err = lambda t: float((t.double() - want).norm() / want.norm())
+    assert err(got) <= 1.01 * err(want.bfloat16())
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 136, 128),      # less than any tile, one block
+                                   (128, 384, 256), (129, 392, 384),
+                                   (192, 192, 384), (193, 200, 512), (191, 576, 128),
+                                   (385, 1160, 640), (577, 776, 896)])
+def test_every_tile_forms_the_same_sums(device, hooks, M, N, K):
+    rng = np.random.default_rng(M + N + K)
+    (a, ha), (a2, ha2) = _operand(device, rng, M, K), _operand(device, rng, M, K, 0.3)
+    (b, hb), (b2, hb2) = _operand(device, rng, N, K, 0.02), _operand(device, rng, N, K, 0.05)
+    runs = {}
+    for grid in (0, 8):  # 8 workgroups: several tiles each, the ring runs on from one into the next
+        for tile in TILES:
+            hooks.mx_debug_set_grid(grid)
+            hooks.mx_debug_set_tile(*tile, 0)
+            out = torch.full((M, N + 24), 7.0, dtype=torch.bfloat16, device=device)
+            ops._gemm_operands(a, b, out[:, :N])
+            assert bool((out[:, N:] == 7.0).all())
+            got = [out[:, :N].contiguous()]
+            if M > 128:
+                got += [ops.mx_gemm_nt_shared_a(a, b, b2), ops.mx_gemm_nt_shared_b(a, a2, b), ops.mx_gemm_nt_pair(a, b, a2, b2)]
+            runs[grid, tile] = got
+    want = runs[0, (4, 4)]
+    _check(want[0], ha @ hb.T)
+    if M > 128:
+        _check(want[1][1], ha @ hb2.T)
+        _check(want[2][1], ha2 @ hb.T)
+        _check(want[3], ha @ hb.T + ha2 @ hb2.T)
+    for key, got in runs.items():
+        for i, (g, w) in enumerate(zip(got, want, strict=True)):
+            assert torch.equal(g, w), (key, i)
+
+
+@pytest.mark.parametrize("slices", [2, 3, 6])
+@pytest.mark.parametrize("tile", [(4, 4), (2, 4), (4, 2)])
+@pytest.mark.parametrize("M,N,K", [(65, 136, 4096), (200, 392, 4224), (513, 264, 4352)])
+def test_splits_along_k(device, hooks, M, N, K, tile, slices):
+    rng = np.random.default_rng(M + slices)
+    (a, ha), (b, hb) = _operand(device, rng, M, K), _operand(device, rng, N, K, 0.02)
+    hooks.mx_debug_set_tile(*tile, slices)
+    need = int(hooks.mx_gemm_nt_workspace_bytes(M, N, K))
+    assert need == slices * M * N * 4
+    ws = torch.full((need,), 0xFF, dtype=torch.uint8, device=device)  # (NaN)
+    out = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=device)
+    for grid in (0, 8):
+        hooks.mx_debug_set_grid(grid)
+        ops._call("mx_gemm_nt_ld", "gemm_nt_splitk", device, a.codes_ptr, a.scales_ptr, b.codes_ptr, b.scales_ptr,
+                  out.data_ptr(), M, N, a.k, a.ld, N, ws.data_ptr(), need, ops._stream(out))
+        _check(out, ha @ hb.T)
+
+
+def test_shapes_that_are_split(device, hooks):
+    """Which way a shape runs: few rows on their own kernel as long as that is ahead, slices where tiles are few
+    and the contraction is long, and never more partial sums than one 256 x 256 tile per CU but for shapes of
+    more tiles than half of the CUs."""
+    need = lambda M, N, K: int(hooks.mx_gemm_nt_workspace_bytes(M, N, K))
+    with torch.cuda.device(device):
+        assert need(16, 4096, 8192) == 0 and need(64, 4096, 4096) == 0 and need(64, 4096, 8192) > 0
+        assert need(256, 4096, 8192) > 0 and need(2048, 2048, 2048) == 0 and need(4096, 4096, 4096) == 0
+        for M in (65, 200, 1000, 2048):
+            for N in (1024, 4096, 6144):
+                for K in (1024, 4096, 16384, 147456):
+                    assert need(M, N, K) <= 64 << 20 or -(-M // 256) * -(-N // 256) > 128

@@ -31,11 +31,16 @@ __global__ __launch_bounds__(256, 1) void gemm_nt_kernel(DenseArgs p) {
 }
 
 template <int BM, int BN>
+static bool configure_dense() {
+  static std::atomic<bool> configured[kMaxDevices];  // a per-function, per-device setting
+  return raise_lds_limit(reinterpret_cast<const void*>(gemm_nt_kernel<BM, BN>), GemmTile<BM, BN, false, false>::kLdsBytes,
+                         configured);
+}
+template <int BM, int BN>
 static int launch_dense(const DenseArgs& p, hipStream_t st) {
   using Tile = GemmTile<BM, BN, false, false>;
   auto kern = gemm_nt_kernel<BM, BN>;
-  static std::atomic<bool> configured[kMaxDevices];  // a per-function, per-device setting
-  if (!raise_lds_limit(reinterpret_cast<const void*>(kern), Tile::kLdsBytes, configured)) return MX_ERR_LAUNCH;
+  if (!configure_dense<BM, BN>()) return MX_ERR_LAUNCH;
   const int64_t nb = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
   const int64_t grid = (nb + 7) / 8 * 8;
   if (grid > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
@@ -51,15 +56,14 @@ namespace mx {
 int launch_gemm_nt32(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                      const uint8_t* b_scales, void* d, int64_t M, int64_t N, int64_t K,
                      int64_t ldk, int64_t ldd, hipStream_t st);
-}
-namespace mx {
 int launch_few_rows_codes(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                           const uint8_t* b_scales, void* d, int64_t M, int64_t N, int64_t K, int64_t ldk, int64_t ldd,
                           hipStream_t st);
-int splitk_slices(int64_t M, int64_t N, int64_t K);
+GemmPlan plan_dense(int64_t M, int64_t N, int64_t K, bool may_split);
+bool prepare_dense32();
 int launch_gemm_nt32_splitk(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                             const uint8_t* b_scales, void* d, int64_t M, int64_t N, int64_t K,
-                            int64_t ldk, int64_t ldd, int slices, void* workspace, hipStream_t st);
+                            int64_t ldk, int64_t ldd, const GemmPlan& plan, void* workspace, hipStream_t st);
 }
 // Test hooks (include/mxfp8_debug.h), process-wide.
 // 0: pick by shape; 1 / 2: the 16x16x128 tile kernel with 256x256 / 128x128 tiles for every
@@ -68,6 +72,8 @@ static std::atomic<int> force_kernel{0};
 extern "C" void mx_debug_force_kernel(int which) { force_kernel = which; }
 namespace mx { void set_debug_grid(int g); }
 extern "C" void mx_debug_set_grid(int g) { mx::set_debug_grid(g); }
+namespace mx { void set_debug_tile(int ta, int tb, int slices); }
+extern "C" void mx_debug_set_tile(int ta, int tb, int slices) { mx::set_debug_tile(ta, tb, slices); }
 #ifdef MX_TIMING_BUILD
 namespace mx { void set_debug_prof(uint64_t* buf); }
 // device buffer of 256*4*8 uint64 receiving per-wave cycle counts; nullptr switches timing off
@@ -95,6 +101,11 @@ static bool persistent_ok(const void* d, int64_t N, int64_t K, int64_t ldd, int6
            (uint64_t)ldd * 512 > 0x7FFFFFFFull);
 }
 
+// Few rows: a workgroup for every 16 columns and more, its waves along the contraction, while its widest
+// workgroups fit the CUs in one round: 64 rows 2048 -> 16384 13.6 us, 16.4 on tiles; 20480 25.1 and 16.9,
+// 151936 127.8 and 86.8.
+static bool few_rows_shape(int64_t M, int64_t N, int64_t K) { return M <= 64 && K % 128 == 0 && N <= 16384; }
+
 // mx_gemm_nt with operand rows `ldk` bytes apart (ldk >= K, a multiple of 16).
 static int gemm_nt_pitched(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                            const uint8_t* b_scales, void* d, int64_t M, int64_t N, int64_t K, int64_t ldk,
@@ -106,19 +117,20 @@ static int gemm_nt_pitched(const uint8_t* a_codes, const uint8_t* a_scales, cons
   if (256 * ldk > 0x7FFFFFFFll) return MX_ERR_UNSUPPORTED;
   DenseArgs p{a_codes, a_scales, b_codes, b_scales, (uint16_t*)d, M, N, K, ldd, ldk};
   hipStream_t st = (hipStream_t)stream;
-  // Few rows: a workgroup for every 16 columns and more, its waves along the contraction, while its widest
-  // workgroups fit the CUs in one round: 64 rows 2048 -> 16384 13.6 us, 16.4 on tiles; 20480 25.1 and 16.9,
-  // 151936 127.8 and 86.8.
-  if (M <= 64 && K % 128 == 0 && force_kernel == 0 && N <= 16384)
+  if (few_rows_shape(M, N, K) && force_kernel == 0)
     return launch_few_rows_codes(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldk, ldd, st);
-  if (M <= 128 || N <= 128 || force_kernel == 2) return launch_dense<128, 128>(p, st);
-  // Few 256x256 tiles leave most CUs of the persistent kernel idle when the contraction is not
-  // split: up to 3/8 of the CUs' worth of tiles, four times as many 128x128 tiles finish sooner
-  // (measured: 64 tiles 58 vs 71 us at K = 8192; 128 tiles 46 vs 43 us).
-  int num_cus = current_device_cus();
-  if (num_cus == 0) num_cus = 256;
-  const int64_t tiles256 = ((M + 255) / 256) * ((N + 255) / 256);
-  if (force_kernel == 0 && tiles256 * 8 <= (int64_t)num_cus * 3) return launch_dense<128, 128>(p, st);
+  if (N <= 128 || (M <= 128 && force_kernel != 0) || force_kernel == 2) return launch_dense<128, 128>(p, st);
+  if (force_kernel == 0) {
+    if (!persistent_ok(d, N, K, ldd, ldk)) {
+      // (few 256 x 256 tiles: four times as many 128 x 128 ones finish sooner)
+      int num_cus = current_device_cus();
+      if (num_cus == 0) num_cus = 256;
+      const int64_t tiles256 = ((M + 255) / 256) * ((N + 255) / 256);
+      if (M <= 128 || tiles256 * 8 <= (int64_t)num_cus * 3) return launch_dense<128, 128>(p, st);
+      return launch_dense<256, 256>(p, st);
+    }
+    if (plan_dense(M, N, K, false).ta == 0) return launch_dense<128, 128>(p, st);
+  }
   if (force_kernel == 1 || !persistent_ok(d, N, K, ldd, ldk)) return launch_dense<256, 256>(p, st);
   return launch_gemm_nt32(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldk, ldd, st);
 }
@@ -226,10 +238,23 @@ extern "C" int mx_gemm_nt_shared_b(const uint8_t* a_codes, const uint8_t* a_scal
                                 ldd, stream);
 }
 
+// How the shape is split along K by a caller that lends memory for the partial sums (slices == 1: not).
+static GemmPlan split_plan(int64_t M, int64_t N, int64_t K) {
+  constexpr GemmPlan kNone{0, 0, 1};
+  if (M <= 0 || N <= 128 || K <= 0 || N % 8 || (uint64_t)N * 1024 > 0x7FFFFFFFull) return kNone;
+  // Few rows run on their own kernel up to here; behind it slices on tiles are ahead although they
+  // are summed by a second launch (16 x 4096: K 8192 12.8 us, 16.2 in eight slices, K 14336 19.9 and
+  // 20.1; 64 x 4096: K 4096 13.4 and 14.8, K 8192 23.7 and 17.2, K 14336 38 and 22; 64 x 14336, K 4096
+  // 24 and 20).
+  if (few_rows_shape(M, N, K) && ((M + 15) / 16 * 16) * K <= 270000ll * 8192 / (N > 8192 ? N : 8192)) return kNone;
+  return plan_dense(M, N, K, true);
+}
+static int64_t split_bytes(const GemmPlan& plan, int64_t M, int64_t N) {
+  return plan.slices > 1 ? (int64_t)plan.slices * M * N * 4 : 0;
+}
+
 extern "C" int64_t mx_gemm_nt_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  if (M <= 128 || N <= 128 || K <= 0 || N % 8 || (uint64_t)N * 1024 > 0x7FFFFFFFull) return 0;
-  const int s = splitk_slices(M, N, K);
-  return s > 1 ? (int64_t)s * M * N * 4 : 0;
+  return split_bytes(split_plan(M, N, K), M, N);
 }
 
 extern "C" int mx_gemm_nt_ld(const uint8_t* a_codes, const uint8_t* a_scales,
@@ -239,12 +264,12 @@ extern "C" int mx_gemm_nt_ld(const uint8_t* a_codes, const uint8_t* a_scales,
   const int rc = check_dense(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldd);
   if (rc != MX_OK || M == 0 || N == 0) return rc;
   if (ldk < K) return MX_ERR_INVALID_ARG;
-  const int64_t need = force_kernel == 0 ? mx_gemm_nt_workspace_bytes(M, N, K) : 0;
-  if (need == 0 || !workspace || workspace_bytes < need || ((uintptr_t)workspace & 15) ||
-      !persistent_ok(d, N, K, ldd, ldk))
+  GemmPlan plan{0, 0, 1};
+  if (workspace && force_kernel == 0 && persistent_ok(d, N, K, ldd, ldk)) plan = split_plan(M, N, K);
+  if (plan.slices == 1 || workspace_bytes < split_bytes(plan, M, N) || ((uintptr_t)workspace & 15))
     return gemm_nt_pitched(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldk, ldd, stream);
   return launch_gemm_nt32_splitk(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldk, ldd,
-                                 (int)(need / (M * N * 4)), workspace, (hipStream_t)stream);
+                                 plan, workspace, (hipStream_t)stream);
 }
 
 extern "C" int mx_gemm_nt_ws(const uint8_t* a_codes, const uint8_t* a_scales,
@@ -271,6 +296,7 @@ static void* scratch_of_current_device() {
   if (dev < 0) return nullptr;
   std::lock_guard<std::mutex> lock(scratch_mutex);
   if (!scratch_ptr[dev]) {
+    if (!prepare_dense32() || !configure_dense<128, 128>() || !configure_dense<256, 256>()) return nullptr;
     void* ptr = nullptr;
     if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)) != hipSuccess) return nullptr;
     scratch_ptr[dev] = ptr;
@@ -286,12 +312,12 @@ extern "C" int mx_gemm_nt_static(const uint8_t* a_codes, const uint8_t* a_scales
   const int rc = check_dense(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldd);
   if (rc != MX_OK || M == 0 || N == 0) return rc;
   // the size check stands on the shape alone, whatever the test hooks say
-  const int64_t need = mx_gemm_nt_workspace_bytes(M, N, K);
-  if (need > kScratchBytes && persistent_ok(d, N, K, ldd)) return MX_ERR_SCRATCH_TOO_SMALL;
-  if (need == 0 || force_kernel != 0 || !persistent_ok(d, N, K, ldd))  // not split: no scratch involved
-    return mx_gemm_nt(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldd, stream);
+  const GemmPlan plan = split_plan(M, N, K);
+  if (split_bytes(plan, M, N) > kScratchBytes && persistent_ok(d, N, K, ldd)) return MX_ERR_SCRATCH_TOO_SMALL;
   void* ws = scratch_of_current_device();
+  if (plan.slices == 1 || force_kernel != 0 || !persistent_ok(d, N, K, ldd))  // not split: no scratch involved
+    return mx_gemm_nt(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldd, stream);
   if (!ws) return MX_ERR_LAUNCH;
   return launch_gemm_nt32_splitk(a_codes, a_scales, b_codes, b_scales, d, M, N, K, K, ldd,
-                                 (int)(need / (M * N * 4)), ws, (hipStream_t)stream);
+                                 plan, ws, (hipStream_t)stream);
 }

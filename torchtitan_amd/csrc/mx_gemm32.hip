@@ -1,5 +1,5 @@
-// MXFP8 GEMM for large shapes, dense and grouped: persistent 256x256 tiles on the scaled fp8
-// MFMA v_mfma_scale_f32_16x16x128_f8f6f4.
+// MXFP8 GEMM for large shapes, dense and grouped: persistent 256x256 tiles (dense also 192x256,
+// 256x192, 128x256 and 256x128) on the scaled fp8 MFMA v_mfma_scale_f32_16x16x128_f8f6f4.
 //
 //   D[M,N] (bf16) = deq(A)[M,K] * deq(B)[N,K]^T, fp32 accumulate.
 //
@@ -49,12 +49,12 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int kT32 = 256;                        // tile edge (M and N)
 constexpr int kK32 = 64;                         // K per compute step
 constexpr int kKB = 128;                         // K per ring block (= one cache line per row)
-constexpr int kOperand32 = kT32 * kKB;           // 32 KB: 256 rows x 128 B
-constexpr int kCodes32 = 2 * kOperand32;         // A rows then B rows
+constexpr int kCodes32 = 2 * kT32 * kKB;         // A rows then B rows, 256 of 128 B each
 constexpr int kBlock32 = kCodes32 + 3072;        // + scales: groups A0, A1, B0, B1, A2 (+ 512 unused) x 2 steps x 256 B
 constexpr int kRing32 = 2 * kBlock32;            // 134 KB
 constexpr int kPatch32 = 6656;                   // per wave: 4608 B output patch + 2 KB of records / tables
 constexpr int kPatchUsed = 4608;
+constexpr int kPatchPitch = 144;                 // bytes per staged row: 128 + 16, keeps b128 accesses spread
 constexpr uint32_t kRecordsPerPatch = (kPatch32 - kPatchUsed) / 64;
 constexpr uint32_t kMaxTileRecords = 3 * kRecordsPerPatch;  // grouped modes: tile records a workgroup keeps in LDS
 static_assert(kRing32 + 4 * kPatch32 == 160 * 1024, "the kernel's LDS map fills the CU's 160 KB");
@@ -119,6 +119,8 @@ struct Tile32 {
   bool poison;             // grouped modes: the group ends break the alignment contract
   uint32_t rot;            // kGrouped2d3d: 32-row blocks between the tile's first row and the start of
                            // its 128-row scale group (0..3): the A scale bytes are turned by as much
+  uint32_t odd;            // 192-row tiles: bit 0 / 1: the tile begins in the middle of a 128-row scale
+                           // group of A / of B
   uint32_t head, tail;     // kGrouped2d2d: the K range starts `head` 32-deep blocks into its first
                            // 128-deep block and ends `tail` of them into its last (0: at its end)
 };
@@ -184,17 +186,114 @@ __device__ __forceinline__ float acc_read(const V& c) {
 // Fragment sets of four 16-row sub-tiles each, whole 128-deep blocks (a[h][t] =
 // sub-tile 4h + t of the wave's 128 rows of A, b[h][t] likewise for B), the scale dwords of the
 // block being computed (one for the even and one for the odd sub-tiles) and those of the next.
+// The LDS map of a tile of 64 TA x 64 TB: a ring of 128-deep blocks (A rows, B rows, scales of groups A0,
+// A1, B0, B1, A2 of 512 B each) and four waves' output patches.  128 x 256 and 256 x 128 tiles leave
+// room for a third block: theirs is 1024 MFMA cycles, less than it takes the copies from issue
+// to landing, so with one block of lead the matrix cores wait (16384 x 14336, K 4096 829 -> 778 us on
+// 128 x 256, 888 -> 837 on 256 x 128; 4096 x 2048, K 2 x 6144 80 -> 76).  Their patches stage 16 rows
+// instead of 32.  (The two slots of a ring of two stay numbered 0 and 1: offsets that grow by a block
+// cost a dozen more additions between the MFMAs and 1 % of a long launch.)
+template <int TA, int TB>
+struct Lds32 {
+  static constexpr int kStages = TA + TB <= 6 ? 3 : 2;
+  static constexpr int kA = 64 * TA * kKB, kCodes = 64 * (TA + TB) * kKB;
+  static constexpr int kBlock = kCodes + (kStages == 3 ? 2048 : 3072);
+  static constexpr int kRing = kStages * kBlock;
+  static constexpr int kPatchRows = kStages == 3 ? 16 : 32;
+  static constexpr int kPatch = kStages == 3 ? kPatchRows * kPatchPitch : kPatch32;
+  static constexpr int kBytes = kRing + 4 * kPatch;
+  static_assert(kBytes <= 160 * 1024);
+};
+static_assert(Lds32<4, 4>::kRing == kRing32 && Lds32<4, 4>::kBlock == kBlock32, "the grouped modes' tables lie behind it");
+
+template <int TA, int TB>
 struct Frags16 {
-  v8i a[2][4];
-  v8i b[2][4];
+  v8i a[2][TA];
+  v8i b[2][TB];
   uint32_t sa[2], sb[2];
   uint32_t san[2], sbn[2];
-  uint32_t sa_hi[2];  // kGrouped2d3d: as san, of the next 128-row group (see next_scales)
+  uint32_t sa_hi[2], sb_hi[2];  // as san, sbn, of the next 128-row group (see next_scales)
 };
 
-template <int MODE, bool PROF, bool PAIR = false>
+// When a K block's LDS reads and copies are issued: everything is counted in MFMA slots of the
+// block, 4 * TA * TB of them in four quarters (see block_steps).
+template <int TA, int TB>
+struct BlockPlan {
+  static constexpr int kQ = TA * TB;                 // MFMAs of a quarter
+  static constexpr int kCopies = 2 * (TA + TB) + 1;  // copies of a block and wave
+  // quarter 0: the last sub-tile of a[0] (2 reads), then b[1] (2 TB): so many behind each MFMA
+  static constexpr int kReads0 = 2 + 2 * TB;
+  static constexpr int kQuota0 = TA == 4 && TB == 4 ? 1 : TA > 2 ? 2 : 3;
+  // the ring block is released in front of the last sub-tile of a[0], whose data and b[1]'s must have arrived;
+  // with two sub-tiles that is too soon after the reads, and quarter 1 begins first
+  static constexpr int kRelease = TA > 2 ? TB * (TA - 1) : kQ;
+  static constexpr int kFirstCopy = kRelease + 1;
+  static constexpr int copy_slot(int j) { return kFirstCopy + j * (4 * kQ - kFirstCopy) / kCopies; }
+  static constexpr int copy_of(int slot) {  // the copy behind this slot's MFMA (-1: none)
+    for (int j = 0; j < kCopies; ++j)
+      if (copy_slot(j) == slot) return j;
+    return -1;
+  }
+  static constexpr int copies_before(int slot) {
+    int n = 0;
+    for (int j = 0; j < kCopies; ++j) n += copy_slot(j) < slot;
+    return n;
+  }
+  // quarter 2: b[0] of the next block and three scale dwords, in the slots without a copy where
+  // there are enough of those, else evenly
+  static constexpr int kReads2 = 2 * TB + 3;
+  static constexpr bool kFree2 = kQ - (copies_before(3 * kQ) - copies_before(2 * kQ)) >= kReads2;
+  static constexpr int first2(int i) {  // reads of the quarter issued before slot i of it
+    if (!kFree2) return (i * kReads2 + kQ - 1) / kQ;
+    const int n = i - (copies_before(2 * kQ + i) - copies_before(2 * kQ));
+    return n < kReads2 ? n : kReads2;
+  }
+  // quarter 3: reads 0 .. 2 TA - 1 are a[1]'s, 2 TA + j is read j of a[0], whose sub-tile j / 2 is
+  // free behind the first MFMA of the sub-tile after it.  Entry k of the plan, in issue order.
+  static constexpr int kReads3 = 2 * TA + 2 * (TA - 1);
+  static constexpr int kQuota3 = TA * TB >= 2 + kReads3 || (TA == 2 && TB == 4) ? 1 : 2;
+  struct Plan3 {
+    int slot[kReads3], what[kReads3];
+  };
+  static constexpr Plan3 plan3() {
+    Plan3 p{};
+    int k = 0, a1 = 0, a0 = 0;
+    for (int s = 0; s < kQ; ++s)
+      for (int q = 0; q < kQuota3; ++q) {
+        const bool have0 = a0 < 2 * (TA - 1) && s >= TB * (a0 / 2 + 1);
+        if (!have0 && a1 == 2 * TA) continue;
+        p.slot[k] = s;
+        p.what[k++] = have0 ? 2 * TA + a0++ : a1++;
+      }
+    return p;
+  }
+  static constexpr int after_a0(int t) {  // reads of quarter 3 issued after those of a[0][t]
+    const Plan3 p = plan3();
+    for (int k = 0; k < kReads3; ++k)
+      if (p.what[k] == 2 * TA + 2 * t + 1) return kReads3 - 1 - k;
+    return 0;
+  }
+  static constexpr int before0(int slot) { return kQuota0 * slot < kReads0 ? kQuota0 * slot : kReads0; }
+};
+
+// A wave's columns of the tile: sub-tile n begins at column first + 16 n for n < 4 and at
+// second + 16 (n - 4) from there on.  192 wide (TB = 3), the waves share the middle 64 columns and
+// wave 1 takes its own 64 first, so that both write whole 128-byte lines of them.
+template <int TB>
+__device__ __forceinline__ constexpr uint32_t wave_col(uint32_t wn, int n) {
+  if constexpr (TB == 4) return wn * 128 + 16 * n;
+  if constexpr (TB == 2) return wn * 64 + 16 * n;
+  return n < 4 ? wn * 128 + 16 * n : 64 + wn * 32 + 16 * (n - 4);
+}
+
+template <int MODE, bool PROF, bool PAIR = false, int TA = 4, int TB = 4>
 __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  static_assert((TA == 4 && TB == 4) || MODE == kDense || MODE == kSplitK, "grouped tiles are 256 x 256");
+  using Plan = BlockPlan<TA, TB>;
+  using Frags = Frags16<TA, TB>;
+  using Lds = Lds32<TA, TB>;
+  constexpr int kEA = 64 * TA, kEB = 64 * TB;  // tile edges
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -212,7 +311,7 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
   const uint32_t ks_n = K / kK32;    // 64-deep steps per 128-row scale group
   // tile rows / columns of one product, and of the launch (p.two: the second product's tile
   // columns or rows come behind the first's; grouped launches cover columns [tn0, tn0 + tn_cnt))
-  const uint32_t tiles_n1 = (uint32_t)((p.N + kT32 - 1) / kT32), tiles_m1 = (uint32_t)((p.M + kT32 - 1) / kT32);
+  const uint32_t tiles_n1 = (uint32_t)((p.N + kEB - 1) / kEB), tiles_m1 = (uint32_t)((p.M + kEA - 1) / kEA);
   const uint32_t tiles_n = MODE == kDense ? (p.two == kTwoB ? 2 * tiles_n1 : tiles_n1) : (uint32_t)p.tn_cnt;
   const uint32_t tiles_m = p.two == kTwoA ? 2 * tiles_m1 : tiles_m1;
   const uint32_t tn0 = MODE == kDense ? 0u : (uint32_t)p.tn0;
@@ -343,6 +442,7 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
     r.empty = false;
     r.rows_d = 0;
     r.rot = 0;
+    r.odd = 0;
     r.head = 0;
     r.tail = 0;
     const uint8_t* a_codes = (PAIR && seg) ? p.a2_codes : p.a_codes;
@@ -383,14 +483,15 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
       r.a = a_codes + (int64_t)tm * kT32 * K;
       r.b = b_codes + (int64_t)(tn & 3) * kT32 * K;
 #else
-      r.a = a_codes + (int64_t)tm * kT32 * Kt;
-      r.b = b_codes + (int64_t)tn * kT32 * Kt;
+      r.a = a_codes + (int64_t)tm * kEA * Kt;
+      r.b = b_codes + (int64_t)tn * kEB * Kt;
 #endif
-      r.sa = a_scales + (int64_t)(tm * 2) * ks_n * 256;
-      r.sb = b_scales + (int64_t)(tn * 2) * ks_n * 256;
-      r.d = d_base + (int64_t)tm * kT32 * p.ldd + (int64_t)tn * kT32;
-      r.rows_a = p.M - (int64_t)tm * kT32;
-      r.rows_b = p.N - (int64_t)tn * kT32;
+      r.sa = a_scales + (int64_t)(tm * kEA / 128) * ks_n * 256;
+      r.sb = b_scales + (int64_t)(tn * kEB / 128) * ks_n * 256;
+      r.d = d_base + (int64_t)tm * kEA * p.ldd + (int64_t)tn * kEB;
+      r.rows_a = p.M - (int64_t)tm * kEA;
+      r.rows_b = p.N - (int64_t)tn * kEB;
+      r.odd = (tm & 1) | (tn & 1) << 1;
       if (MODE == kGrouped2d3d && p.d_offs) {
         const int64_t left = p.d_rows - (int64_t)tm * kT32;
         r.rows_d = (int32_t)(left < 0 ? 0 : (left > kT32 ? kT32 : left));
@@ -437,15 +538,16 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
       const uint32_t blocks = K / kKB, per = (blocks + G - 1) / G;
       const uint32_t b_lo = g * per, b_hi = b_lo + per < blocks ? b_lo + per : blocks;
       const uint32_t lo = b_lo * kKB;
-      r.a = a_codes + (int64_t)tm * kT32 * Kt + lo;
-      r.b = b_codes + (int64_t)tn * kT32 * Kt + lo;
-      r.sa = a_scales + ((int64_t)(tm * 2) * ks_n + (lo >> 6)) * 256;
-      r.sb = b_scales + ((int64_t)(tn * 2) * ks_n + (lo >> 6)) * 256;
+      r.a = a_codes + (int64_t)tm * kEA * Kt + lo;
+      r.b = b_codes + (int64_t)tn * kEB * Kt + lo;
+      r.sa = a_scales + ((int64_t)(tm * kEA / 128) * ks_n + (lo >> 6)) * 256;
+      r.sb = b_scales + ((int64_t)(tn * kEB / 128) * ks_n + (lo >> 6)) * 256;
       float* part = reinterpret_cast<float*>(p.d) +
-                    ((int64_t)g * p.M + (int64_t)tm * kT32) * p.ldd + (int64_t)tn * kT32;
+                    ((int64_t)g * p.M + (int64_t)tm * kEA) * p.ldd + (int64_t)tn * kEB;
       r.d = reinterpret_cast<uint16_t*>(part);
-      r.rows_a = p.M - (int64_t)tm * kT32;
-      r.rows_b = p.N - (int64_t)tn * kT32;
+      r.rows_a = p.M - (int64_t)tm * kEA;
+      r.rows_b = p.N - (int64_t)tn * kEB;
+      r.odd = (tm & 1) | (tn & 1) << 1;
       r.koff = lo;
       r.nblocks = b_hi - b_lo;
     } else {
@@ -491,6 +593,7 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
   // output patches of waves 1-3 (32 records each; the host splits launches so that a
   // workgroup never has more than kMaxRecords tiles).
   auto record_offset = [&](uint32_t i) -> uint32_t {
+    if constexpr (MODE == kSplitK) return Lds::kRing + i * 64;  // (its output is not staged: the patches are free)
     return kRing32 + (1 + i / kRecordsPerPatch) * kPatch32 + kPatchUsed + (i % kRecordsPerPatch) * 64;
   };
   if constexpr (MODE != kDense) {
@@ -509,7 +612,7 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
       w[2] = (int32_t)t.nblocks;
       w[3] = (int32_t)t.koff;
       w[4] = t.empty ? 1 : 0;
-      w[5] = (int32_t)(t.rot | (t.tail << 8) | (t.head << 16) | ((uint32_t)t.rows_d << 20));
+      w[5] = (int32_t)(t.rot | (t.odd << 4) | (t.tail << 8) | (t.head << 16) | ((uint32_t)t.rows_d << 20));
     }
     __syncthreads();
   }
@@ -544,6 +647,7 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
       t.empty = __builtin_amdgcn_readfirstlane(r3.z) != 0;
       const uint32_t rt = (uint32_t)__builtin_amdgcn_readfirstlane(r3.w);
       t.rot = rt & 3;
+      t.odd = (rt >> 4) & 3;
       t.tail = (rt >> 8) & 3;
       t.head = (rt >> 16) & 3;
       t.rows_d = (int32_t)(rt >> 20);
@@ -568,27 +672,35 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
   // m >> 1: one dword for the even sub-tiles, the one 64 bytes on for the odd ones.
   const uint32_t sw = (li & 2) | ((li & 8) >> 1);
   const uint32_t lane4 = (uint32_t)(lj >> 1) * 256 + (uint32_t)((lj & 1) * 32 + li) * 4;
-  const uint32_t fa0 = (wm * 128 + li) * kKB + ((lj ^ sw) << 4);
-  const uint32_t fb_delta = kOperand32 + (wn - wm) * 128 * kKB;
+  const uint32_t fa0 = (wm * 32 * TA + li) * kKB + ((lj ^ sw) << 4);
+  // sub-tiles 0..3 and 4.. of B (see wave_col), from the place of A's first
+  const uint32_t fb_delta = Lds::kA + (wave_col<TB>(wn, 0) - wm * 32 * TA) * kKB;
+  const uint32_t fb_delta4 = TB == 3 ? Lds::kA + (wave_col<TB>(wn, 4) - 64 - wm * 32 * TA) * kKB : fb_delta;
   // scale copy: lanes 0-31 fetch one 128-row group's 512 bytes of a block, lanes 32-63 the next
   // group's; wave 1 (kGrouped2d3d: a third group of A) has its upper lanes read nothing
   const uint32_t v_scale = (MODE == kGrouped2d3d && wave == 1)
                                ? (lane < 32 ? (uint32_t)lane * 16 : 0x80000000u)
                                : (uint32_t)(lane >> 5) * ks_n * 256 + (lane & 31) * 16;
   // scale groups of a ring block: A0, A1, B0, B1, A2 (512 bytes each, then 512 unused)
-  const uint32_t scale_dst = kCodes32 + ((MODE == kGrouped2d3d && wave == 1) ? 2048u : (uint32_t)(wave >> 1) * 1024u);
-  const uint32_t fsa_s = kCodes32 + wm * 512, fsb_s = kCodes32 + 1024 + wn * 512;
-  const uint32_t fsa_hi_s = kCodes32 + (wm == 0 ? 512 : 2048);
+  const uint32_t scale_dst = Lds::kCodes + ((MODE == kGrouped2d3d && wave == 1) ? 2048u : (uint32_t)(wave >> 1) * 1024u);
+  // 256 rows: a wave has a scale group of its own (kGrouped2d3d: and the next one, see next_scales);
+  // 192: three of the eight bytes of two groups; 128: half of the bytes of one
+  const uint32_t fsa_s = Lds::kCodes + (TA == 4 ? wm * 512 : 0), fsb_s = Lds::kCodes + 1024 + (TB == 4 ? wn * 512 : 0);
+  const uint32_t fsa_hi_s = Lds::kCodes + (TA == 4 && wm != 0 ? 2048 : 512), fsb_hi_s = Lds::kCodes + 1536;
 
   // ---- loader stream: fills ring block `ld_slot` with K block `ld_kb` of tile `ld_tile`
   uint32_t ld_tile = 0, ld_kb = 0, ld_nb = 1;
   int ld_slot = 0;
+  auto next_slot = [](int slot) -> int {
+    if constexpr (Lds::kStages == 2) return slot ^ 1;
+    return slot == Lds::kStages - 1 ? 0 : slot + 1;
+  };
   __amdgpu_buffer_rsrc_t ra, rb, rs;  // codes of A, codes of B, scales this wave copies
   // kGrouped2d3d: a group may start at any multiple of 32 rows, the scales come in 128-row groups
   // of the whole matrix: a tile that starts `rot` 32-row blocks into a group fetches three groups
   // and turns the bytes of every scale dword by `rot` (next_scales).  The rotation belongs to
   // the tile whose block sits in a ring slot.
-  uint32_t ld_rot = 0, slot_rot0 = 0, slot_rot1 = 0;
+  uint32_t ld_rot = 0, slot_rot0 = 0, slot_rot1 = 0;  // (192-row tiles: Tile32::odd)
   // kGrouped2d2d: a K range may start and end at any multiple of 32.  Its first and last
   // 128-deep blocks send the chunks outside the range out of range, so that zeros land in the
   // ring instead of the neighbouring groups' codes and scales.
@@ -609,7 +721,7 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
     if (ld_tile < n_my) {
       const Tile32 t = get_tile(ld_tile);
       ld_nb = t.nblocks;
-      ld_rot = t.rot;
+      ld_rot = MODE == kGrouped2d3d ? t.rot : t.odd;
       ld_head = t.head;
       ld_tail = t.tail;
       // (kGrouped2d2d: the range stops at the end of the operand rows, not of the K range;
@@ -623,7 +735,10 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
       // is cut off by the range and arrives as zeros
       // (kGrouped2d3d: rows counted from the start of the first scale group; wave 1 copies a
       // third group of A when the tile's rows reach into it)
-      const int64_t rows = wave < 2 ? (t.rows_a > 0 ? t.rows_a + 32 * (int64_t)t.rot : 0) : t.rows_b;
+      // (192-row tiles: likewise, 64 rows into the group for every other tile)
+      const int64_t into_a = TA == 3 ? 64 * (int64_t)(t.odd & 1) : 32 * (int64_t)t.rot;
+      const int64_t into_b = TB == 3 ? 64 * (int64_t)(t.odd >> 1) : 0;
+      const int64_t rows = wave < 2 ? (t.rows_a > 0 ? t.rows_a + into_a : 0) : t.rows_b > 0 ? t.rows_b + into_b : 0;
       const uint8_t* sbase = wave < 2 ? t.sa : t.sb;
       if (MODE == kGrouped2d3d && wave == 1)
         rs = make_rsrc(sbase + (int64_t)ks_n * 512, (none || rows <= 256) ? 0 : (int64_t)ld_nb * 512);
@@ -645,26 +760,28 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
 #ifndef MX_LOAD_AUX  // cache policy bits of the operand copies (0: default)
 #define MX_LOAD_AUX 0
 #endif
-  // The 17 copies of a block are issued one at a time, between MFMAs (see block_steps):
-  // piece 0..15 = unit pairs (A unit, B unit alternating), 16 = scales, then advance.
+  // The copies of a block (17 of a 256 x 256 tile) are issued one at a time, between MFMAs (see
+  // block_steps): units of A and of B alternating as long as there are both, scales last, then advance.
   auto issue_piece = [&](auto i_) {
     constexpr int i = decltype(i_)::value;
 #ifdef MX_ABL_DMA_OOB  // timing ablation: every copy is issued with all lanes out of range (zeros land in LDS, nothing is fetched)
     const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.a_codes, 0), rb = ra, rs = ra;
 #endif
 
-    const uint32_t sbase = lds_base + ld_slot * kBlock32;
-    if constexpr (i < 16) {
-      constexpr int q = i >> 1;
-      const int unit = wave * 8 + q;
+    const uint32_t sbase = lds_base + ld_slot * Lds::kBlock;
+    if constexpr (i < 2 * (TA + TB)) {
+      constexpr int kBoth = 4 * (TA < TB ? TA : TB);
+      constexpr bool is_a = i < kBoth ? (i & 1) == 0 : TA > TB;
+      constexpr int q = i < kBoth ? i >> 1 : i - kBoth / 2;
+      const int unit = wave * 2 * (is_a ? TA : TB) + q;
       const uint32_t v = MODE == kGrouped2d2d ? ((q & 1) ? cur_v_odd : cur_v_even)
                                               : ((q & 1) ? (v_even ^ 64) : v_even);
       const uint32_t so = (uint32_t)(unit * 8) * Kp + ld_kb * kKB;
-      if constexpr ((i & 1) == 0)
+      if constexpr (is_a)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void_t*)(uintptr_t)(sbase + unit * 1024), 16, v, so, 0, MX_LOAD_AUX);
       else
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rb, (lds_void_t*)(uintptr_t)(sbase + kOperand32 + unit * 1024), 16, v, so, 0, MX_LOAD_AUX);
+            rb, (lds_void_t*)(uintptr_t)(sbase + Lds::kA + unit * 1024), 16, v, so, 0, MX_LOAD_AUX);
     } else {
       // scales: a group's two 64-deep steps are 512 contiguous bytes, the two groups land behind
       // one another, which is the order the fragment reads expect.  Waves 0 and 2 copy A's and
@@ -677,7 +794,7 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
     }
   };
   auto issue_advance = [&]() {
-    if constexpr (MODE == kGrouped2d3d) {
+    if constexpr (MODE == kGrouped2d3d || TA == 3 || TB == 3) {
       if (ld_slot) slot_rot1 = ld_rot; else slot_rot0 = ld_rot;
     }
     if (++ld_kb == ld_nb) {
@@ -687,10 +804,10 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
     } else {
       set_block_offsets();
     }
-    ld_slot ^= 1;
+    ld_slot = next_slot(ld_slot);
   };
   auto issue_block = [&]() {
-    static_for<0, 17>([&](auto i_) { issue_piece(i_); });
+    static_for<0, Plan::kCopies>([&](auto i_) { issue_piece(i_); });
     issue_advance();
   };
 
@@ -721,24 +838,32 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
   };
   // ---- fragment sets, scale dwords
   // one b128 read of a fragment set: i = 2t + (0: K bytes [16 lj, +16), 1: [64 + 16 lj, +16)) of
-  // sub-tile 4h + t
-  auto read_set_piece = [&](v8i (&set)[4], uint32_t sbase, uint32_t delta, auto h_, auto i_) {
-    constexpr int h = decltype(h_)::value, i = decltype(i_)::value;
-    constexpr int t = i >> 1;
-    constexpr bool hi = i & 1;
+  // the set's sub-tile t, which is sub-tile m of the wave
+  auto read_piece = [&](v8i& dst, uint32_t sbase, uint32_t delta, auto m_, auto i_) {
+    constexpr int m = decltype(m_)::value;
+    constexpr bool hi = decltype(i_)::value & 1;
     const uint32_t base = (fa0 ^ (hi ? 64u : 0u)) + delta;
-    const v4i v = lds_b128(sbase + base, std::integral_constant<int, (4 * h + t) * 2048>{});
-    v8i& dst = set[t];
+    const v4i v = lds_b128(sbase + base, std::integral_constant<int, m * 2048>{});
     if constexpr (hi) {
       dst[4] = v.x; dst[5] = v.y; dst[6] = v.z; dst[7] = v.w;
     } else {
       dst[0] = v.x; dst[1] = v.y; dst[2] = v.z; dst[3] = v.w;
     }
   };
+  auto read_a = [&](Frags& f, uint32_t sbase, auto h_, auto i_) {
+    constexpr int h = decltype(h_)::value, t = decltype(i_)::value >> 1;
+    read_piece(f.a[h][t], sbase, 0u, std::integral_constant<int, TA * h + t>{}, i_);
+  };
+  auto read_b = [&](Frags& f, uint32_t sbase, auto h_, auto i_) {
+    constexpr int h = decltype(h_)::value, t = decltype(i_)::value >> 1, n = TB * h + t;
+    read_piece(f.b[h][t], sbase, n < 4 ? fb_delta : fb_delta4, std::integral_constant<int, n>{}, i_);
+  };
   // the scale dwords of a block, into the "next" registers: piece 0, 1 = A even / odd
-  // sub-tiles, 2, 3 = B, 4, 5 = A of the next 128-row group (kGrouped2d3d)
-  constexpr int kScalePieces = MODE == kGrouped2d3d ? 6 : 4;
-  auto read_scale_piece = [&](Frags16& f, uint32_t sbase, auto i_) {
+  // sub-tiles, 2, 3 = B, then those of the next 128-row group of A (kGrouped2d3d, 192 rows) and of
+  // B (192 columns)
+  constexpr bool kHiA = MODE == kGrouped2d3d || TA == 3, kHiB = TB == 3;
+  constexpr int kScalePieces = 4 + (kHiA ? 2 : 0) + (kHiB ? 2 : 0);
+  auto read_scale_piece = [&](Frags& f, uint32_t sbase, auto i_) {
     constexpr int i = decltype(i_)::value;
     constexpr int e = i & 1;
     if constexpr (i < 2) {
@@ -747,35 +872,46 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
     } else if constexpr (i < 4) {
       const uint32_t ps = sbase + fsb_s + lane4 + e * 64;
       asm volatile("ds_read_b32 %0, %1" : "=v"(f.sbn[e]) : "v"(ps));
-    } else {
+    } else if constexpr (kHiA && i < 6) {
       const uint32_t ps = sbase + fsa_hi_s + lane4 + e * 64;
       asm volatile("ds_read_b32 %0, %1" : "=v"(f.sa_hi[e]) : "v"(ps));
+    } else {
+      const uint32_t ps = sbase + fsb_hi_s + lane4 + e * 64;
+      asm volatile("ds_read_b32 %0, %1" : "=v"(f.sb_hi[e]) : "v"(ps));
     }
   };
-  auto pin_set = [&](v8i (&set)[4]) {
-#pragma unroll
-    for (int t = 0; t < 4; ++t) asm volatile("" : "+v"(set[t]));
+  auto pin_set = [&](auto& set) {
+    for (auto& frag : set) asm volatile("" : "+v"(frag));
   };
   // The next block's scales become the current ones, once their reads have landed.
   // kGrouped2d3d: byte k of an A scale dword becomes the scale of the tile's k-th 32-row block,
   // which is byte (rot + k) of the eight bytes that two neighbouring 128-row groups hold for
   // this lane
-  auto next_scales = [&](Frags16& f, int slot) {
+  // 192 rows: a tile's six 32-row blocks are bytes 0..5 or, every other tile, 2..7 of the eight of
+  // its two groups; three of them, in the order of the wave's sub-tiles, are picked.
+  // 128 rows: the upper wave's two bytes are brought down.
+  auto next_scales = [&](Frags& f, int slot) {
     asm volatile("" : "+v"(f.san[0]), "+v"(f.san[1]), "+v"(f.sbn[0]), "+v"(f.sbn[1]));
-    if constexpr (MODE == kGrouped2d3d) {
-      asm volatile("" : "+v"(f.sa_hi[0]), "+v"(f.sa_hi[1]));
-      const uint32_t rot = slot ? slot_rot1 : slot_rot0;
-      f.sa[0] = __builtin_amdgcn_alignbyte(f.sa_hi[0], f.san[0], rot);
-      f.sa[1] = __builtin_amdgcn_alignbyte(f.sa_hi[1], f.san[1], rot);
-    } else {
-      f.sa[0] = f.san[0];
-      f.sa[1] = f.san[1];
-    }
-    f.sb[0] = f.sbn[0];
-    f.sb[1] = f.sbn[1];
+    if constexpr (kHiA) asm volatile("" : "+v"(f.sa_hi[0]), "+v"(f.sa_hi[1]));
+    if constexpr (kHiB) asm volatile("" : "+v"(f.sb_hi[0]), "+v"(f.sb_hi[1]));
+    const uint32_t rot = slot ? slot_rot1 : slot_rot0;
+    static_for<0, 2>([&](auto e_) {
+      constexpr int e = decltype(e_)::value;
+      if constexpr (MODE == kGrouped2d3d) f.sa[e] = __builtin_amdgcn_alignbyte(f.sa_hi[e], f.san[e], rot);
+      else if constexpr (TA == 3) {
+        const uint32_t sel = (wm ? 0x00050403u : 0x00020100u) + ((rot & 1) ? 0x00020202u : 0u);
+        f.sa[e] = __builtin_amdgcn_perm(f.sa_hi[e], f.san[e], sel);
+      } else if constexpr (TA == 2) f.sa[e] = f.san[e] >> (16 * wm);
+      else f.sa[e] = f.san[e];
+      if constexpr (TB == 3) {
+        const uint32_t sel = (wn ? 0x00030504u : 0x00020100u) + ((rot & 2) ? 0x00020202u : 0u);
+        f.sb[e] = __builtin_amdgcn_perm(f.sb_hi[e], f.sbn[e], sel);
+      } else if constexpr (TB == 2) f.sb[e] = f.sbn[e] >> (16 * wn);
+      else f.sb[e] = f.sbn[e];
+    });
   };
   // ---- compute stream
-  v4f acc[8][8];
+  v4f acc[2 * TA][2 * TB];
   int c_slot = 0;  // ring block holding the K block being computed
   uint64_t prof_vm = 0, prof_bar = 0, prof_body = 0, prof_last = 0, prof_epi = 0;
   uint64_t prof_e_stage = 0, prof_e_wait = 0, prof_e_store = 0;
@@ -786,12 +922,10 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
 #ifndef MX_STORE_AUX
 #define MX_STORE_AUX 2
 #endif
-#ifndef MX_RELEASE16
-#define MX_RELEASE16 12
-#endif
   // A K block is 64 MFMAs, one per 16x16 sub-tile, in four quarters of 16 (512 MFMA cycles each)
   // over the fragment sets a[0], a[1] (rows 0-63, 64-127 of the wave) and b[0], b[1], in an
-  // order that needs every set for two quarters in a row (slots 0-63 = the block's MFMAs):
+  // order that needs every set for two quarters in a row (slots 0-63 = the block's MFMAs; for
+  // the smaller tiles, whose sets hold TA and TB sub-tiles, BlockPlan has the slots):
   //   quarter 0: a[0] x b[0], a[0]'s sub-tiles one after the other.  Read meanwhile, from this
   //              block: the last sub-tile of a[0] (slots 0, 1; used from slot 12) and b[1]
   //              (2-9).  Once every wave has done so (barrier in front of slot kRelease) the
@@ -809,27 +943,22 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
   // cycles and the wave's issue for about half of that: what is issued behind it has to fit
   // the other half, so copies and reads are spread over the slots as evenly as the rules above
   // allow.
-  constexpr int kRelease = MX_RELEASE16;          // slot in front of which the ring block is released
-  constexpr int kFirstCopy = kRelease + 1;        // copy j goes behind the MFMA of slot kFirstCopy + 3j
-  constexpr int kCopiesA = (32 - kFirstCopy + 2) / 3;  // copies issued in quarters 0 and 1
-  static_assert(kRelease >= 12 && kFirstCopy + 3 * 16 < 64, "seventeen copies, three slots apart");
-  auto copy_at = [&](auto slot_) {  // slot 0..63 of the block
+  auto copy_at = [&](auto slot_) {  // slot of the block
 #ifndef MX_ABL_NO_DMA
-    constexpr int sl = decltype(slot_)::value;
-    if constexpr (sl >= kFirstCopy && (sl - kFirstCopy) % 3 == 0 && (sl - kFirstCopy) / 3 < 17)
-      issue_piece(std::integral_constant<int, (sl - kFirstCopy) / 3>{});
+    constexpr int j = Plan::copy_of(decltype(slot_)::value);
+    if constexpr (j >= 0) issue_piece(std::integral_constant<int, j>{});
 #endif
   };
-  // quarter: 16 MFMAs of a[ah] x b[bh]; AMAJOR: a's sub-tiles one after the other (else b's);
+  // quarter: the MFMAs of a[ah] x b[bh]; AMAJOR: a's sub-tiles one after the other (else b's);
   // side(slot, false) runs in front of a slot's MFMA, side(slot, true) behind it
-  auto quarter = [&](Frags16& f, auto first_, auto ah_, auto bh_, auto amajor_, auto&& side) {
+  auto quarter = [&](Frags& f, auto first_, auto ah_, auto bh_, auto amajor_, auto&& side) {
     constexpr bool kFirst = decltype(first_)::value;
     constexpr int ah = decltype(ah_)::value, bh = decltype(bh_)::value;
     constexpr bool kAMajor = decltype(amajor_)::value;
-    static_for<0, 16>([&](auto i_) {
+    static_for<0, Plan::kQ>([&](auto i_) {
       constexpr int i = decltype(i_)::value;
-      constexpr int tm = kAMajor ? i >> 2 : i & 3, tn = kAMajor ? i & 3 : i >> 2;
-      constexpr int m = 4 * ah + tm, n = 4 * bh + tn;
+      constexpr int tm = kAMajor ? i / TB : i % TA, tn = kAMajor ? i % TB : i / TA;
+      constexpr int m = TA * ah + tm, n = TB * bh + tn;
       side(i_, std::false_type{});
       mfma16_asm<(n >> 1), (m >> 1), kFirst>(acc[m][n], f.b[bh][tn], f.a[ah][tm], f.sb[n & 1], f.sa[m & 1]);
       side(i_, std::true_type{});
@@ -840,50 +969,62 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
     asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(kReadsPerPiece * decltype(n_)::value > 15 ? 15 : kReadsPerPiece * decltype(n_)::value) : "memory");
     asm volatile("" : "+v"(frag));
   };
-  auto block_steps = [&](Frags16& f, auto first_) {
+  auto block_steps = [&](Frags& f, auto first_) {
     using H0 = std::integral_constant<int, 0>;
     using H1 = std::integral_constant<int, 1>;
-    const uint32_t s_cur = lds_base + c_slot * kBlock32, s_nxt = lds_base + (c_slot ^ 1) * kBlock32;
-    // quarter 0.  In flight on entry, oldest first: the last two reads of a[1], a[0][1], the
-    // other last two reads of a[1], a[0][2] (see quarter 3)
+    constexpr int kQ = Plan::kQ;
+    const uint32_t s_cur = lds_base + c_slot * Lds::kBlock, s_nxt = lds_base + next_slot(c_slot) * Lds::kBlock;
+    // in front of slot kRelease: this wave's reads of the block are done, and once every wave's are
+    // its place in the ring is free
+    auto release = [&]() {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      asm volatile("" : "+v"(f.a[0][TA - 1]));
+      uint64_t t0 = 0;
+      if constexpr (PROF) t0 = __builtin_readcyclecounter();
+      __builtin_amdgcn_s_barrier();
+      if constexpr (PROF) {
+        const uint64_t t1 = __builtin_readcyclecounter();
+        prof_bar += t1 - t0;
+        prof_last += t1 - t0;  // keep the barrier out of the body figure
+      }
+    };
+    // quarter 0.  In flight on entry: what quarter 3 read after a[0][0], of a[1] and a[0][1] up to a[0][TA - 2]
     quarter(f, first_, H0{}, H0{}, std::true_type{}, [&](auto i_, auto after_) {
       constexpr int i = decltype(i_)::value;
       if constexpr (!decltype(after_)::value) {
-        if constexpr (i == 4) landed(std::integral_constant<int, 4 + 4>{}, f.a[0][1]);
-        if constexpr (i == 8) landed(std::integral_constant<int, 8>{}, f.a[0][2]);
-        if constexpr (i == kRelease) {
-          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's reads of the block are done
-          asm volatile("" : "+v"(f.a[0][3]));
-          uint64_t t0 = 0;
-          if constexpr (PROF) t0 = __builtin_readcyclecounter();
-          __builtin_amdgcn_s_barrier();
-          if constexpr (PROF) {
-            const uint64_t t1 = __builtin_readcyclecounter();
-            prof_bar += t1 - t0;
-            prof_last += t1 - t0;  // keep the barrier out of the body figure
-          }
+        if constexpr (i == Plan::kRelease) release();
+        else if constexpr (i % TB == 0 && i != 0) {
+          constexpr int t = i / TB;  // a sub-tile of a[0] begins
+          // (the last one was read in this quarter's first slots)
+          constexpr int since = t < TA - 1 ? Plan::after_a0(t) + Plan::before0(i) : Plan::before0(i) - 2;
+          landed(std::integral_constant<int, since>{}, f.a[0][t]);
         }
       } else {
 #ifndef MX_ABL_NO_READ
-        if constexpr (i < 2) read_set_piece(f.a[0], s_cur, 0u, H0{}, std::integral_constant<int, 6 + i>{});
-        else if constexpr (i < 10) read_set_piece(f.b[1], s_cur, fb_delta, H1{}, std::integral_constant<int, i - 2>{});
+        static_for<Plan::before0(i), Plan::before0(i + 1)>([&](auto r_) {
+          constexpr int r = decltype(r_)::value;
+          if constexpr (r < 2) read_a(f, s_cur, H0{}, std::integral_constant<int, 2 * (TA - 1) + r>{});
+          else read_b(f, s_cur, H1{}, std::integral_constant<int, r - 2>{});
+        });
 #endif
         copy_at(i_);
       }
     });
+    if constexpr (Plan::kRelease == kQ) release();
     pin_set(f.a[1]);
     pin_set(f.b[1]);
     // quarter 1
     quarter(f, first_, H1{}, H0{}, std::false_type{}, [&](auto i_, auto after_) {
-      if constexpr (decltype(after_)::value) copy_at(std::integral_constant<int, 16 + decltype(i_)::value>{});
+      if constexpr (decltype(after_)::value) copy_at(std::integral_constant<int, kQ + decltype(i_)::value>{});
     });
     uint64_t t0 = 0, t1 = 0;
     if constexpr (PROF) {
       t0 = __builtin_readcyclecounter();
       prof_body += t0 - prof_last;
     }
-    // block b+1 (and any output stores): everything but the copies issued so far in this block
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kCopiesA) : "memory");
+    // block b+1 (and any output stores): everything but the copies issued so far in this block, and
+    // a whole block's where the ring holds three
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(Plan::copies_before(2 * kQ) + (Lds::kStages - 2) * Plan::kCopies) : "memory");
     if constexpr (PROF) {
       t1 = __builtin_readcyclecounter();
       prof_vm += t1 - t0;
@@ -893,45 +1034,46 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
       prof_last = __builtin_readcyclecounter();
       prof_bar += prof_last - t1;
     }
-    // quarter 2: b[0] of block b+1 and its first three scale dwords, in the slots without a copy
+    // quarter 2: b[0] of block b+1 and its first three scale dwords
     quarter(f, first_, H1{}, H1{}, std::false_type{}, [&](auto i_, auto after_) {
-      constexpr int i = decltype(i_)::value, sl = 32 + i;
+      constexpr int i = decltype(i_)::value;
       if constexpr (decltype(after_)::value) {
-        copy_at(std::integral_constant<int, sl>{});
+        copy_at(std::integral_constant<int, 2 * kQ + i>{});
 #ifndef MX_ABL_NO_READ
-        constexpr bool has_copy = sl >= kFirstCopy && (sl - kFirstCopy) % 3 == 0;
-        // free slots of the quarter before this one
-        constexpr int before = i - (sl - kFirstCopy + 2) / 3 + (32 - kFirstCopy + 2) / 3;
-        if constexpr (!has_copy) {
-          if constexpr (before < 8) read_set_piece(f.b[0], s_nxt, fb_delta, H0{}, std::integral_constant<int, before>{});
-          else if constexpr (before < 11) read_scale_piece(f, s_nxt, std::integral_constant<int, before - 8>{});
-        }
+        static_for<Plan::first2(i), Plan::first2(i + 1)>([&](auto r_) {
+          constexpr int r = decltype(r_)::value;
+          if constexpr (r < 2 * TB) read_b(f, s_nxt, H0{}, r_);
+          else read_scale_piece(f, s_nxt, std::integral_constant<int, r - 2 * TB>{});
+        });
 #endif
       }
     });
-    // quarter 3, reads by slot: a[1] 0 (+ the fourth scale dword), 1, 2, 3 (+ the two dwords of
-    // the next scale group, kGrouped2d3d), a[0][0], a[1] 4, 5, a[0][1], a[1] 6, 7, a[0][2]
+    // quarter 3: the other scale dwords before the first read of a[0]; a[1] and a[0] as
+    // BlockPlan::plan3 has them (256 x 256: a[1] 0-3, a[0][0], a[1] 4, 5, a[0][1], a[1] 6, 7, a[0][2], one a slot)
     quarter(f, first_, H0{}, H1{}, std::true_type{}, [&](auto i_, auto after_) {
       constexpr int i = decltype(i_)::value;
       if constexpr (decltype(after_)::value) {
-        copy_at(std::integral_constant<int, 48 + i>{});
+        copy_at(std::integral_constant<int, 3 * kQ + i>{});
 #ifndef MX_ABL_NO_READ
-        if constexpr (i < 4) {
-          read_set_piece(f.a[1], s_nxt, 0u, H1{}, i_);
-          if constexpr (i == 0) read_scale_piece(f, s_nxt, std::integral_constant<int, 3>{});
-          if constexpr (kScalePieces == 6 && i >= 2) read_scale_piece(f, s_nxt, std::integral_constant<int, i + 2>{});
-        } else if constexpr (i < 14) {
-          constexpr int k = i - 4;  // 0, 1: a[0][0]; 2, 3: a[1] 4, 5; 4, 5: a[0][1]; 6, 7: a[1] 6, 7; 8, 9: a[0][2]
-          if constexpr ((k & 3) < 2) read_set_piece(f.a[0], s_nxt, 0u, H0{}, std::integral_constant<int, 2 * (k >> 2) + (k & 1)>{});
-          else read_set_piece(f.a[1], s_nxt, 0u, H1{}, std::integral_constant<int, 4 + 2 * (k >> 2) + (k & 1)>{});
-        }
+        static_for<0, Plan::kReads3>([&](auto k_) {
+          constexpr auto plan = Plan::plan3();
+          constexpr int k = decltype(k_)::value, r = plan.what[k];
+          if constexpr (plan.slot[k] == i) {
+            if constexpr (r < 2 * TA) read_a(f, s_nxt, H1{}, std::integral_constant<int, r>{});
+            else read_a(f, s_nxt, H0{}, std::integral_constant<int, r - 2 * TA>{});
+          }
+        });
+        static_for<3, kScalePieces>([&](auto e_) {
+          if constexpr ((decltype(e_)::value - 3) % TB == i) read_scale_piece(f, s_nxt, e_);
+        });
 #endif
       }
     });
-    c_slot ^= 1;
+    c_slot = next_slot(c_slot);
     // the next block's first MFMAs need its b[0], its scales and the first sub-tile of its
-    // a[0]: everything but the eight reads issued since
-    asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(kReadsPerPiece * 8 > 15 ? 15 : kReadsPerPiece * 8) : "memory");
+    // a[0]: everything but the reads issued since
+    constexpr int since0 = kReadsPerPiece * Plan::after_a0(0);
+    asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(since0 > 15 ? 15 : since0) : "memory");
     pin_set(f.b[0]);
     asm volatile("" : "+v"(f.a[0][0]));
     next_scales(f, c_slot);
@@ -946,8 +1088,7 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
   // Buffer stores: one descriptor per tile bounds the rows, a 32-bit offset per lane, scalar
   // offsets per piece.  Requires N % 8 == 0 and ldd % 8 == 0 (checked on the host).
   // (LDS accesses as assembly, for the reason given at the fragment reads.)
-  constexpr int kPatchPitch = 144;  // bytes per staged row: 128 + 16, keeps b128 accesses spread
-  const uint32_t patch = lds_base + kRing32 + wave * kPatch32;
+  const uint32_t patch = lds_base + Lds::kRing + wave * Lds::kPatch;
   const uint32_t nan_mask = (MODE != kDense && poison) ? 0x7FC07FC0u : 0u;
   auto epilogue = [&](const Tile32& t) {
     // The epilogue's per-lane addresses are worked out here, from a lane number the compiler
@@ -960,17 +1101,17 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
     const uint32_t patch_w = patch + (lane_e & 15) * kPatchPitch + ((lane_e >> 4) & 1) * 32 + (lane_e >> 5) * 16;
     const uint32_t patch_r = patch + (lane_e >> 3) * kPatchPitch + (lane_e & 7) * 16;  // + pass*8 rows
     const int64_t rows_valid = (MODE == kGrouped2d3d && p.d_offs) ? (int64_t)t.rows_d : t.rows_a;
-    const uint32_t cols_valid = (uint32_t)(t.rows_b < kT32 ? t.rows_b : kT32);
+    const uint32_t cols_valid = (uint32_t)(t.rows_b < kEB ? t.rows_b : kEB);
     if constexpr (MODE == kSplitK) {
       // float32 partial sums straight from the accumulators: a lane stores 16 bytes of row li
       // per sub-tile and q; short pieces, but the partial tiles are few and are read back at once
       const uint32_t ld_b = (uint32_t)p.ldd * 4;
-      const __amdgpu_buffer_rsrc_t rp = make_rsrc(t.d, rows_valid * ld_b);
-      const uint32_t row_b = (wm * 128 + li) * ld_b;
+      const __amdgpu_buffer_rsrc_t rp = make_rsrc(t.d, (rows_valid < kEA ? rows_valid : kEA) * ld_b);
+      const uint32_t row_b = (wm * 32 * TA + li) * ld_b;
       // (a lane holds row 16m + li, columns 16n + 4lj + 0..3 of sub-tile (m, n))
-      static_for<0, 64>([&](auto i_) {
-        constexpr int m = decltype(i_)::value >> 3, n = decltype(i_)::value & 7;
-        const uint32_t col = wn * 128 + n * 16 + 4 * lj;
+      static_for<0, 4 * TA * TB>([&](auto i_) {
+        constexpr int m = decltype(i_)::value / (2 * TB), n = decltype(i_)::value % (2 * TB);
+        const uint32_t col = wave_col<TB>(wn, n) + 4 * lj;
         const uint32_t v = col < cols_valid ? row_b + col * 4 : 0x80000000u;
         const u32x4 w = {__float_as_uint(acc_read<0>(acc[m][n])), __float_as_uint(acc_read<1>(acc[m][n])),
                          __float_as_uint(acc_read<2>(acc[m][n])), __float_as_uint(acc_read<3>(acc[m][n]))};
@@ -981,20 +1122,29 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
     const uint32_t ldd_b = (uint32_t)p.ldd * 2;
     const __amdgpu_buffer_rsrc_t rd = make_rsrc(t.d, rows_valid * ldd_b);
     // lane's place in a stored piece: row (lane >> 3) + 8*pass, columns (lane & 7)*8 .. +7
-    const uint32_t colp = wn * 128 + (lane_e & 7) * 8;
-    const uint32_t vrow = (wm * 128 + (lane_e >> 3)) * ldd_b + colp * 2;
-    // Pieces p = 0..7: 32 rows (sub-tile row m = p/2) x 64 columns (sub-tiles n = 2(p%2), +1).
+    const uint32_t colp = wave_col<TB>(wn, 0) + (lane_e & 7) * 8;
+    const uint32_t vrow = (wm * 32 * TA + (lane_e >> 3)) * ldd_b + colp * 2;
+    // ... of a piece of 32 columns: row (lane >> 2) + 16*pass, columns (lane & 3)*8 .. +7
+    const uint32_t patch_r4 = patch + (lane_e >> 2) * kPatchPitch + (lane_e & 3) * 16;
+    const uint32_t colp4 = TB == 3 ? wave_col<TB>(wn, 4) + (lane_e & 3) * 8 : 0;
+    const uint32_t vrow4 = (wm * 32 * TA + (lane_e >> 2)) * ldd_b + colp4 * 2;
+    // Pieces: 32 rows (sub-tile rows m = 2 mp, + 1; 16 where the ring holds three blocks) x 64 columns
+    // (sub-tiles n = 4 np .. + 3), 192-wide tiles' second ones x 32.
     // A wave's LDS instructions execute in order, so a piece's reads may follow its writes
     // without a wait, and the next piece's writes may follow those reads: the only waits are
     // for the read data, with the next piece's conversion and writes already under way.
-    // a lane holds row 16m + li, columns 16n + 4lj + 0..3 of sub-tile (m, n).  Part k of
-    // piece p covers 16 rows x 32 columns: sub-tiles (m, n) and (m, n + 1), m = 2(p / 2) + k / 2,
-    // n = 4(p % 2) + 2(k % 2).  v_permlane16_swap trades the halves of two neighbouring lane
+    // a lane holds row 16m + li, columns 16n + 4lj + 0..3 of sub-tile (m, n).  A part of a
+    // piece covers 16 rows x 32 columns: sub-tiles (m, n) and (m, n + 1).
+    // v_permlane16_swap trades the halves of two neighbouring lane
     // groups: the even groups end up with 8 consecutive columns of sub-tile n, the odd ones with
     // 8 of sub-tile n + 1.
+    constexpr int kNP = (TB + 1) / 2, kSubs = Lds::kPatchRows / 16, kPieces = 2 * TA / kSubs * kNP;
+    constexpr auto col_parts = [](int pc) { return TB == 3 && pc % 2 ? 1 : 2; };
+    constexpr auto parts_of = [col_parts](int pc) { return kSubs * col_parts(pc); };  // parts, and 1 KB stores, of a piece
     auto stage_part = [&](auto p_, auto k_) {
-      constexpr int mp = decltype(p_)::value >> 1, np = decltype(p_)::value & 1, k = decltype(k_)::value;
-      constexpr int m = 2 * mp + (k >> 1), n = 4 * np + 2 * (k & 1);
+      constexpr int mp = decltype(p_)::value / kNP, np = decltype(p_)::value % kNP, k = decltype(k_)::value;
+      constexpr int kc = col_parts(decltype(p_)::value);
+      constexpr int m = kSubs * mp + k / kc, n = 4 * np + 2 * (k % kc);
       const v4f& c0 = acc[m][n];
       const v4f& c1 = acc[m][n + 1];
       const float a[8] = {acc_read<0>(c0), acc_read<1>(c0), acc_read<2>(c0), acc_read<3>(c0),
@@ -1010,36 +1160,39 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
       const u32x2 sx = __builtin_amdgcn_permlane16_swap(x0, x1, false, false);
       const u32x2 sy = __builtin_amdgcn_permlane16_swap(y0, y1, false, false);
       const v4i w = {(int)sx.x, (int)sy.x, (int)sx.y, (int)sy.y};
-      lds_write_b128_hidden<(m & 1) * 16 * kPatchPitch + (k & 1) * 64>(patch_w, w);
+      lds_write_b128_hidden<(k / kc) * 16 * kPatchPitch + (k % kc) * 64>(patch_w, w);
       __builtin_amdgcn_sched_barrier(0);
     };
     v4i r[2][4];
-    static_for<0, 4>([&](auto k_) { stage_part(std::integral_constant<int, 0>{}, k_); });
-    static_for<0, 8>([&](auto p_) {
-      constexpr int pc = decltype(p_)::value, m = pc >> 1, np = pc & 1;
+    static_for<0, parts_of(0)>([&](auto k_) { stage_part(std::integral_constant<int, 0>{}, k_); });
+    static_for<0, kPieces>([&](auto p_) {
+      constexpr int pc = decltype(p_)::value, m = pc / kNP, np = pc % kNP;
+      constexpr int kStores = parts_of(pc), kNext = pc + 1 < kPieces ? parts_of(pc + 1) : 0;
+      constexpr int kEach = (kNext + kStores - 1) / kStores;  // parts of the next piece in front of each store
+      constexpr bool kWide = col_parts(pc) == 2;
+      constexpr int kRows = kWide ? 8 : 16;  // rows of a store
       uint64_t e0 = 0;
       if constexpr (PROF) e0 = __builtin_readcyclecounter();
-      static_for<0, 4>([&](auto q_) {
+      static_for<0, kStores>([&](auto q_) {
         constexpr int q = decltype(q_)::value;
-        r[pc & 1][q] = lds_read_b128_hidden<q * 8 * kPatchPitch>(patch_r);
+        r[pc & 1][q] = lds_read_b128_hidden<q * kRows * kPatchPitch>(kWide ? patch_r : patch_r4);
       });
-      const uint32_t v = (colp + np * 64 < cols_valid) ? vrow + np * 128 : 0x80000000u;
+      const uint32_t v = kWide ? ((colp + np * 64 < cols_valid) ? vrow + np * 128 : 0x80000000u)
+                                      : (colp4 < cols_valid ? vrow4 : 0x80000000u);
       // the next piece's conversion runs between this piece's stores, which drain at the
       // write path's pace
-      static_for<0, 4>([&](auto q_) {
+      static_for<0, kStores>([&](auto q_) {
         constexpr int q = decltype(q_)::value;
-        if constexpr (pc < 7) stage_part(std::integral_constant<int, pc + 1>{}, q_);
-        if constexpr (q == 0) {
-          // the four reads are done once at most the one younger write is outstanding
-          if constexpr (pc < 7) asm volatile("s_waitcnt lgkmcnt(1)" ::: "memory");
-          else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        }
+        static_for<q * kEach, (q + 1) * kEach < kNext ? (q + 1) * kEach : (q * kEach < kNext ? kNext : q * kEach)>(
+            [&](auto k_) { stage_part(std::integral_constant<int, pc + 1>{}, k_); });
+        // the reads are done once at most the younger writes are outstanding
+        if constexpr (q == 0) asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(kEach < kNext ? kEach : kNext) : "memory");
         const v4i rq = pin(r[pc & 1][q]);
         const u32x4 w = {(uint32_t)rq.x, (uint32_t)rq.y, (uint32_t)rq.z, (uint32_t)rq.w};
 #ifdef MX_ABL_STORE_ROWS  // timing ablation: only sub-tile rows below this many are written
-        if constexpr (m < MX_ABL_STORE_ROWS)
+        if constexpr (kSubs * m < 2 * MX_ABL_STORE_ROWS)
 #endif
-        __builtin_amdgcn_raw_buffer_store_b128(w, rd, v, (m * 32 + q * 8) * ldd_b, MX_STORE_AUX);
+        __builtin_amdgcn_raw_buffer_store_b128(w, rd, v, (m * 16 * kSubs + q * kRows) * ldd_b, MX_STORE_AUX);
         __builtin_amdgcn_sched_barrier(0);
       });
       if constexpr (PROF) prof_e_stage += __builtin_readcyclecounter() - e0;
@@ -1050,17 +1203,18 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
   if constexpr (PROF) prof_t0 = __builtin_readcyclecounter();
   // ---- prologue: fill the ring, fetch the first fragments
   loader_open_tile();
-  issue_block();
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll 1
+  for (int i = 0; i < Lds::kStages; ++i) issue_block();
+  // block 0; the others are in flight when the first step starts
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((Lds::kStages - 1) * Plan::kCopies) : "memory");
   __builtin_amdgcn_s_barrier();
-  issue_block();  // block 1: in flight when the first step starts
-  Frags16 f;
+  Frags f;
   {
     using Z = std::integral_constant<int, 0>;
     using O = std::integral_constant<int, 1>;
-    static_for<0, 8>([&](auto i_) { read_set_piece(f.a[0], lds_base, 0u, Z{}, i_); });
-    static_for<0, 8>([&](auto i_) { read_set_piece(f.a[1], lds_base, 0u, O{}, i_); });
-    static_for<0, 8>([&](auto i_) { read_set_piece(f.b[0], lds_base, fb_delta, Z{}, i_); });
+    static_for<0, 2 * TA>([&](auto i_) { read_a(f, lds_base, Z{}, i_); });
+    static_for<0, 2 * TA>([&](auto i_) { read_a(f, lds_base, O{}, i_); });
+    static_for<0, 2 * TB>([&](auto i_) { read_b(f, lds_base, Z{}, i_); });
     static_for<0, kScalePieces>([&](auto i_) { read_scale_piece(f, lds_base, i_); });
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     pin_set(f.a[0]);
@@ -1144,18 +1298,163 @@ static int64_t persistent_grid() {
   return grid;
 }
 
-template <int MODE, bool PROF, bool PAIR = false>
-static int launch32(const Gemm32Args& p, int64_t nb, hipStream_t st) {
-  auto kern = gemm_nt32_kernel<MODE, PROF, PAIR>;
-  constexpr int lds = kRing32 + 4 * kPatch32;  // ring + one output patch per wave = all 160 KB
+template <int MODE, bool PROF, bool PAIR = false, int TA = 4, int TB = 4>
+static bool configure32() {
   static std::atomic<bool> configured[kMaxDevices];
-  if (!raise_lds_limit(reinterpret_cast<const void*>(kern), lds, configured)) return MX_ERR_LAUNCH;
+  return raise_lds_limit(reinterpret_cast<const void*>(gemm_nt32_kernel<MODE, PROF, PAIR, TA, TB>),
+                         Lds32<TA, TB>::kBytes, configured);
+}
+template <int MODE, bool PROF, bool PAIR = false, int TA = 4, int TB = 4>
+static int launch32(const Gemm32Args& p, int64_t nb, hipStream_t st) {
+  auto kern = gemm_nt32_kernel<MODE, PROF, PAIR, TA, TB>;
+  constexpr int lds = Lds32<TA, TB>::kBytes;  // ring + one output patch per wave: most of the CU's 160 KB
+  if (!configure32<MODE, PROF, PAIR, TA, TB>()) return MX_ERR_LAUNCH;
   int64_t grid = persistent_grid();
   if (grid == 0) return MX_ERR_LAUNCH;
   const int64_t need = (nb + 7) / 8 * 8;  // nb: the tile count, or an upper bound of it
   if (need < grid && debug_grid <= 0) grid = need;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, st, p);
   return hipGetLastError() == hipSuccess ? MX_OK : MX_ERR_LAUNCH;
+}
+
+// Test hook: edges of the dense kernels' tiles, 64 ta x 64 tb, and slices (0: by shape).
+static std::atomic<int> debug_tile{0}, debug_slices{0};
+void set_debug_tile(int ta, int tb, int slices) {
+  debug_tile = ta * 16 + tb;
+  debug_slices = slices;
+}
+
+// ---- which tile, and whether to split along K ---------------------------------------------------
+// The dense tiles, and what a 128-deep block of one takes a CU with all CUs busy, in microseconds.
+// Smaller ones cost a little more per flop (operand bytes per flop x 1.17 and 1.5) and leave fewer
+// CUs idle in a launch's last round: 4096 x 2048, K 6144 runs 128 tiles of 256 x 256 in 58 us and
+// 256 of 128 x 256 in 41; 3001 x 4096, K 4096 192 in 49 and 256 of 192 x 256 in 40; with many
+// rounds 256 x 256 stays ahead (16384 x 14336, K 4096: 671 us, 697, 756, 778, 837 in this order).
+struct DenseTile {
+  int ta, tb;
+  double block_us;
+};
+static constexpr DenseTile kDenseTiles[] = {{4, 4, 1.32}, {3, 4, 1.00}, {4, 3, 1.04}, {2, 4, 0.75}, {4, 2, 0.74}};
+
+static int64_t tile_count(const DenseTile& t, int64_t M, int64_t N) {
+  return ((M + 64 * t.ta - 1) / (64 * t.ta)) * ((N + 64 * t.tb - 1) / (64 * t.tb));
+}
+
+// Microseconds that `tiles` tiles of `blocks` blocks each take on `grid` CUs.  Fitted to 240 shapes of
+// 16..16384 rows, 1024..151936 columns and K 256..16384 in every way to run them (residual 5 to 10 %;
+// choosing by it loses 2 % against the best of them): a round costs 3.6 us to fill and up to
+// 1.5 us to drain, and CUs that idle let the others clock higher.
+static double tiles_us(const DenseTile& t, int64_t tiles, int64_t blocks, int64_t grid) {
+  const double area = t.ta * t.tb / 16.0, rest = (double)(tiles % grid) / grid;
+  double us = (double)(tiles / grid) * (blocks * t.block_us + 3.6 + 1.5 * area);
+  if (tiles % grid) us += blocks * t.block_us * (0.68 + 0.32 * rest) + 3.6 + 1.5 * area * rest;
+  return us;
+}
+
+// The tile for `products` products of one launch, their tiles side by side (each with K blocks of
+// its own, or of two operand sets: `blocks` counts both).
+static const DenseTile* best_tile(int64_t M, int64_t N, int64_t blocks, int products, int64_t grid) {
+  const DenseTile* best = nullptr;
+  double best_us = 0;
+  for (const DenseTile& t : kDenseTiles) {
+    if (debug_tile && debug_tile != t.ta * 16 + t.tb) continue;
+    // (a smaller tile has to promise 6 %: over many rounds the power limit leaves less of its gain than
+    // idle CUs cost, 4096 x 14336, K 16384 2 % slower on 192 x 256 where 3 % less was predicted)
+    const double us = (t.ta * t.tb == 16 ? 1.0 : 1.06) * tiles_us(t, products * tile_count(t, M, N), blocks, grid);
+    if (!best || us < best_us) {
+      best = &t;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
+// What a dense product runs on: the persistent kernel with tiles of 64 ta x 64 tb in `slices` slices
+// of K, or (ta == 0) the kernel of one 128 x 128 tile per workgroup.
+//   * That one is ahead for short contractions only: it starts faster (512 x 4096: K 256 6.1 us, 7.4
+//     on the persistent kernel; K 1024 10.2 and 10.2; K 4096 28.5 and 22.7).
+//   * S slices add float32 partial sums, written and read back (3.2 TB/s) by a launch of their own,
+//     and are taken for a predicted gain of 8 %: 256 x 4096, K 8192 40 us unsplit, 23 in four
+//     slices; 512 x 4096, K 14336 85 and 39; 2048 x 2048, K 147456 1270 and 430.  The partial sums stay under 64 MiB,
+//     one 256 x 256 tile per CU; more only for 256 x 256 tiles of a half to one and a half times the CUs
+//     (4352 x 4352, K 147456: 289 tiles, the second round all but empty).
+//     Contractions of up to 4096 stay one chain of sums, as other implementations form them too:
+//     a result that all but cancels moves by several bf16 steps with the order of its sum.
+GemmPlan plan_dense(int64_t M, int64_t N, int64_t K, bool may_split) {
+  const int64_t grid = persistent_grid(), blocks = K / kKB;
+  if (grid == 0 || K % kKB) return {0, 0, 1};
+  const DenseTile* t = best_tile(M, N, blocks, 1, grid);
+  if (!t) return {0, 0, 1};
+  GemmPlan best{t->ta, t->tb, 1};
+  double best_us = tiles_us(*t, tile_count(*t, M, N), blocks, grid) + 2.0;
+  if (!debug_tile) {
+    const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128), rounds = (tiles + grid - 1) / grid;
+    const double us = 4.3 * rounds + (0.28 + 0.47 * rounds) * blocks;
+    if (us < best_us) {
+      best = {0, 0, 1};
+      best_us = us;
+    }
+  }
+  if (!may_split || (blocks <= 32 && !debug_slices)) return best;
+  const double plain_us = best_us;
+  for (const DenseTile& u : kDenseTiles) {
+    if (u.ta * u.tb == 12 || (debug_tile && debug_tile != u.ta * 16 + u.tb)) continue;
+    const int64_t tiles = tile_count(u, M, N);
+    for (int s = 2; s <= 8; ++s) {
+      const int64_t per = (blocks + s - 1) / s;
+      if (per < 4 || (s - 1) * per >= blocks || (debug_slices && s != debug_slices)) continue;
+      const double bytes = 4.0 * s * M * N;
+      const bool large = bytes > (double)(64 << 20);
+      if (large && (u.ta * u.tb < 16 || 2 * tiles <= grid || 2 * tiles >= 3 * grid)) continue;
+      const double us = tiles_us(u, tiles * s, per, grid) + 2.0 + 4.2 + bytes / 3.2e6;
+      if (us < best_us && us <= 0.92 * plain_us || debug_slices) {
+        best = {u.ta, u.tb, s};
+        best_us = us;
+      }
+    }
+  }
+  return best;
+}
+
+// Launches the persistent dense kernel on `p` with tiles of 64 ta x 64 tb.
+template <int MODE, bool PAIR, int TA, int TB>
+static int launch_tile(Gemm32Args p, hipStream_t st) {
+  int64_t tm = (p.M + 64 * TA - 1) / (64 * TA), tn = (p.N + 64 * TB - 1) / (64 * TB);
+  if (p.two == kTwoA) tm *= 2;
+  if (p.two == kTwoB) tn *= 2;
+  if (MODE == kSplitK) p.tn_cnt = (int32_t)tn;
+  return launch32<MODE, false, PAIR, TA, TB>(p, tm * tn * (MODE == kSplitK ? p.G : 1), st);
+}
+template <int MODE, bool PAIR = false>
+static int launch_dense32(const Gemm32Args& p, int ta, int tb, hipStream_t st) {
+  switch (ta * 16 + tb) {
+    case 0x44: return launch_tile<MODE, PAIR, 4, 4>(p, st);
+    case 0x24: return launch_tile<MODE, PAIR, 2, 4>(p, st);
+    case 0x42: return launch_tile<MODE, PAIR, 4, 2>(p, st);
+    default: break;
+  }
+  if constexpr (MODE != kSplitK) {
+    if (ta == 3 && tb == 4) return launch_tile<MODE, PAIR, 3, 4>(p, st);
+    if (ta == 4 && tb == 3) return launch_tile<MODE, PAIR, 4, 3>(p, st);
+  }
+  return MX_ERR_UNSUPPORTED;
+}
+// ... with the tile that suits its shape
+template <bool PAIR = false>
+static int launch_best32(const Gemm32Args& p, hipStream_t st) {
+  const int64_t grid = persistent_grid();
+  if (grid == 0) return MX_ERR_LAUNCH;
+  const DenseTile* t = best_tile(p.M, p.N, (PAIR ? 2 : 1) * p.K / kKB, p.two ? 2 : 1, grid);
+  return t ? launch_dense32<kDense, PAIR>(p, t->ta, t->tb, st) : MX_ERR_UNSUPPORTED;
+}
+
+// Raises the LDS limits of every kernel that a dense product may run on, for a caller that captures
+// products of other shapes than the one it has called.
+bool prepare_dense32() {
+  return configure32<kDense, false, false, 4, 4>() && configure32<kDense, false, false, 3, 4>() &&
+         configure32<kDense, false, false, 4, 3>() && configure32<kDense, false, false, 2, 4>() &&
+         configure32<kDense, false, false, 4, 2>() && configure32<kSplitK, false, false, 4, 4>() &&
+         configure32<kSplitK, false, false, 2, 4>() && configure32<kSplitK, false, false, 4, 2>();
 }
 
 void set_debug_grid(int g) { debug_grid = g; }
@@ -1168,11 +1467,10 @@ int launch_gemm_nt32(const uint8_t* a_codes, const uint8_t* a_scales, const uint
                      int64_t ldk, int64_t ldd, hipStream_t st) {
   Gemm32Args p{a_codes, a_scales, b_codes, b_scales, (uint16_t*)d, M, N, K, ldd, nullptr, 0, 0, 0, debug_prof};
   p.ldk = ldk;
-  const int64_t nb = ((M + kT32 - 1) / kT32) * ((N + kT32 - 1) / kT32);
 #ifdef MX_TIMING_BUILD
-  if (debug_prof) return launch32<kDense, true>(p, nb, st);
+  if (debug_prof) return launch32<kDense, true>(p, ((M + kT32 - 1) / kT32) * ((N + kT32 - 1) / kT32), st);
 #endif
-  return launch32<kDense, false>(p, nb, st);
+  return launch_best32(p, st);
 }
 
 // ---- split along K for shapes whose 256x256 tiles do not fill the CUs ----------------------
@@ -1210,57 +1508,16 @@ int launch_splitk_reduce(const float* part, int slices, int64_t M, int64_t N, vo
   return hipGetLastError() == hipSuccess ? MX_OK : MX_ERR_LAUNCH;
 }
 
-// Number of K slices for a dense shape on the persistent kernel (1: no split), from a cost model
-// in microseconds fitted to measurements on MI355X:
-//   one 128-deep block of a 256x256 tile takes a CU 1.6 us with the whole chip busy (about 10 %
-//   less with idle CUs: the clock is power-bound);
-//   unsplit, up to 3/8 of the CUs' worth of tiles go to the 128x128-tile kernel, 1.3 PFLOP/s
-//   times the share of the CUs its tiles cover;
-//   split, S slices run ceil(tiles * S / CUs) rounds of blocks / S each, then the float32
-//   partial tiles make a round trip through memory (8 bytes per element and slice at 3 TB/s)
-//   plus a second launch.
-// The split is taken when the model promises at least a fifth less time: a 2048 x 2048 weight
-// gradient over 147 456 tokens 1265 -> 559 us, over 32 768 tokens 198 -> 154 us; over 16 384
-// tokens it stays unsplit (105 vs 110 us).
-int splitk_slices(int64_t M, int64_t N, int64_t K) {
-  const int64_t grid = persistent_grid();
-  if (grid == 0 || K % kKB) return 1;
-  const int64_t tiles = ((M + kT32 - 1) / kT32) * ((N + kT32 - 1) / kT32), blocks = K / kKB;
-  if (tiles >= 2 * grid) return 1;
-  const double block_us = 1.6, flops = 2.0 * (double)M * (double)N * (double)K;
-  double plain;
-  if (tiles * 8 <= grid * 3) {
-    const double share = 4.0 * tiles / grid;
-    plain = flops / (1.3e9 * (share < 1.0 ? share : 1.0));  // 1.3e9 flop per microsecond
-  } else {
-    plain = (double)((tiles + grid - 1) / grid) * blocks * block_us * (tiles < grid ? 0.9 : 1.0);
-  }
-  int best = 1;
-  double best_us = plain;
-  for (int s = 2; s <= 8; ++s) {
-    const int64_t per = (blocks + s - 1) / s;
-    if (per < 16 || (int64_t)(s - 1) * per >= blocks) continue;
-    const double us = (double)((tiles * s + grid - 1) / grid) * per * block_us +
-                      (double)s * M * N * 8.0 / 3.0e6 + 8.0;
-    if (us < best_us) {
-      best = s;
-      best_us = us;
-    }
-  }
-  return best_us <= 0.8 * plain ? best : 1;
-}
-
 // D = sum over slices, through `workspace` (S * M * N floats).
 int launch_gemm_nt32_splitk(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                             const uint8_t* b_scales, void* d, int64_t M, int64_t N, int64_t K,
-                            int64_t ldk, int64_t ldd, int slices, void* workspace, hipStream_t st) {
-  const int64_t tiles_n = (N + kT32 - 1) / kT32, tiles = ((M + kT32 - 1) / kT32) * tiles_n;
+                            int64_t ldk, int64_t ldd, const GemmPlan& plan, void* workspace, hipStream_t st) {
   Gemm32Args p{a_codes, a_scales, b_codes, b_scales, (uint16_t*)workspace, M, N, K, N, nullptr,
-               slices, 0, (int32_t)tiles_n, nullptr};
+               plan.slices, 0, 0, nullptr};
   p.ldk = ldk;
-  const int rc = launch32<kSplitK, false>(p, tiles * slices, st);
+  const int rc = launch_dense32<kSplitK>(p, plan.ta, plan.tb, st);
   if (rc != MX_OK) return rc;
-  return launch_splitk_reduce((const float*)workspace, slices, M, N, d, ldd, st);
+  return launch_splitk_reduce((const float*)workspace, plan.slices, M, N, d, ldd, st);
 }
 
 // Grouped forms with every group end a multiple of 32 and all scales in MFMA order
@@ -1316,7 +1573,7 @@ int launch_gemm_nt32_two_b(const uint8_t* a_codes, const uint8_t* a_scales, cons
   p.two = kTwoB;
   p.d2 = (uint16_t*)d2;
   p.ldk = ldk;
-  return launch32<kDense, false>(p, ((M + kT32 - 1) / kT32) * 2 * ((N + kT32 - 1) / kT32), st);
+  return launch_best32(p, st);
 }
 int launch_grouped32_2d3d_two_b(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                                 const uint8_t* b_scales, const uint8_t* b2_codes, const uint8_t* b2_scales,
@@ -1340,7 +1597,7 @@ int launch_gemm_nt32_two_a(const uint8_t* a_codes, const uint8_t* a_scales, cons
   p.two = kTwoA;
   p.d2 = (uint16_t*)d2;
   p.ldk = ldk;
-  return launch32<kDense, false>(p, 2 * ((M + kT32 - 1) / kT32) * ((N + kT32 - 1) / kT32), st);
+  return launch_best32(p, st);
 }
 int launch_grouped32_2d2d_two_a(const uint8_t* at_codes, const uint8_t* at_scales, const uint8_t* at2_codes,
                                 const uint8_t* at2_scales, const uint8_t* bt_codes, const uint8_t* bt_scales,
@@ -1362,8 +1619,7 @@ int launch_gemm_nt32_pair(const uint8_t* a_codes, const uint8_t* a_scales, const
   Gemm32Args p{a_codes, a_scales, b_codes, b_scales, (uint16_t*)d, M, N, K, ldd, nullptr, 0, 0, 0, nullptr,
                a2_codes, a2_scales, b2_codes, b2_scales};
   p.ldk = ldk;
-  const int64_t nb = ((M + kT32 - 1) / kT32) * ((N + kT32 - 1) / kT32);
-  return launch32<kDense, false, true>(p, nb, st);
+  return launch_best32<true>(p, st);
 }
 
 int launch_grouped32_2d3d_pair(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,

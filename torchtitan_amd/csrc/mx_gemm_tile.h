@@ -36,6 +36,12 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
+// How a dense product runs (plan_dense, mx_gemm32.hip): tiles of 64 ta x 64 tb on the persistent kernel,
+// K in `slices` slices; ta == 0: the kernel of one 128 x 128 tile per workgroup.
+struct GemmPlan {
+  int ta, tb, slices;
+};
+
 // One GEMM operand as the tile sees it.
 struct Operand {
   const uint8_t* codes;    // first row of this tile, column 0

@@ -389,6 +389,14 @@ int mx_gemm_nt_ld(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t
                   const uint8_t* b_scales, void* d, int64_t M, int64_t N, int64_t K, int64_t ldk,
                   int64_t ldd, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* mx_gemm_nt_ld with a float32 D: every value is rounded to bf16 as there and written in 4 bytes, which is
+ * what a conversion of that call's result gives (the gradients of float32 parameters and activations under
+ * autocast to bfloat16).  d 16-byte aligned, N and ldd (in floats) multiples of 8, K and ldk of 128, M > 64 and
+ * N > 128: other shapes return MX_ERR_UNSUPPORTED and are the caller's mx_gemm_nt_ld and a conversion. */
+int mx_gemm_nt_f32_ld(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
+                      const uint8_t* b_scales, float* d, int64_t M, int64_t N, int64_t K, int64_t ldk,
+                      int64_t ldd, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* mx_gemm_nt_ws for callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  The
  * float32 partial sums of the split live in a device array built into the library

@@ -1,5 +1,5 @@
 """The smaller tiles of the persistent GEMM (192 and 128 rows or columns) and their splits along K: at the
-edges of tiles, 128-row scale groups and 128-deep blocks, against the products of the same codes in float64 and
+edges of tiles, 128-row scale groups and 128-deep blocks, and their float32 results, against the products of the same codes in float64 and
 against 256 x 256 tiles, whose sums every unsplit tile forms in the same order."""
 import numpy as np
 import pytest
@@ -29,6 +29,17 @@ def _operand(device, rng, rows, K, std=1.0):
     return q, (q.codes.view(torch.float8_e4m3fn).double().view(rows, -1, 32) * scales[..., None]).view(rows, q.k)
 
 
+def _float32(a, b, ld, ws=None):
+    """The product's float32 form, rows `ld` apart."""
+    M, N = a.rows, b.rows
+    out = torch.full((M, ld), 7.0, dtype=torch.float32, device=a.buf.device)
+    ops._call("mx_gemm_nt_f32_ld", "gemm_nt", out.device, a.codes_ptr, a.scales_ptr, b.codes_ptr, b.scales_ptr,
+              out.data_ptr(), M, N, a.k, a.ld, ld, None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
+              ops._stream(out))
+    assert bool((out[:, N:] == 7.0).all())
+    return out[:, :N]
+
+
 def _check(got, want):
     """`got` is no further from `want` (float64) than its rounding to bf16 by more than 1 %: float32 sums of up to
     a few thousand terms are off by less than 2^-18 of the terms' norm, a hundredth of the rounding's 2^-9 / sqrt(3) and
@@ -54,6 +65,7 @@ def test_every_tile_forms_the_same_sums(device, hooks, M, N, K):
             ops._gemm_operands(a, b, out[:, :N])
             assert bool((out[:, N:] == 7.0).all())
             got = [out[:, :N].contiguous()]
+            assert torch.equal(_float32(a, b, N + 24), got[0].float())
             if M > 128:
                 got += [ops.mx_gemm_nt_shared_a(a, b, b2), ops.mx_gemm_nt_shared_b(a, a2, b), ops.mx_gemm_nt_pair(a, b, a2, b2)]
             runs[grid, tile] = got
@@ -84,6 +96,20 @@ def test_splits_along_k(device, hooks, M, N, K, tile, slices):
         ops._call("mx_gemm_nt_ld", "gemm_nt_splitk", device, a.codes_ptr, a.scales_ptr, b.codes_ptr, b.scales_ptr,
                   out.data_ptr(), M, N, a.k, a.ld, N, ws.data_ptr(), need, ops._stream(out))
         _check(out, ha @ hb.T)
+        assert torch.equal(_float32(a, b, N, ws), out.float())
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 136, 128), (256, 1024, 256), (300, 264, 1024)])
+def test_float32_results_of_short_contractions(device, M, N, K):
+    """(these run on the kernel of one 128 x 128 tile per workgroup)"""
+    rng = np.random.default_rng(M)
+    a, b = _operand(device, rng, M, K)[0], _operand(device, rng, N, K, 0.02)[0]
+    want = ops.mx_gemm_nt(a, b)
+    assert torch.equal(_float32(a, b, N + 8), want.float())
+    got = ops.mx_gemm_nt_as(a, b, torch.float32)
+    assert got.dtype == torch.float32 and torch.equal(got, want.float())
+    few = a.first_rows(64)  # no float32 form: the bf16 result, converted
+    assert torch.equal(ops.mx_gemm_nt_as(few, b, torch.float32), ops.mx_gemm_nt(few, b).float())
 
 
 def test_shapes_that_are_split(device, hooks):

@@ -72,6 +72,7 @@ SIGNATURES = {
     "mx_gemm_nt_workspace_bytes": (_I, [_I, _I, _I]),
     "mx_gemm_nt_ws": (c_int, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _P, _I, _P]),
     "mx_gemm_nt_ld": (c_int, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _P]),
+    "mx_gemm_nt_f32_ld": (c_int, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _P]),
     "mx_gemm_nt_static_max_bytes": (_I, []),
     "mx_gemm_nt_static": (c_int, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _P]),
     "mx_gemm_nt_pair": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P]),

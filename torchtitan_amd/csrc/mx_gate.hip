@@ -19,7 +19,8 @@
 
 namespace mx {
 
-int launch_splitk_reduce(const float* part, int slices, int64_t M, int64_t N, void* d, int64_t ldd, hipStream_t st);
+int launch_splitk_reduce(const float* part, int slices, int64_t M, int64_t N, void* d, int64_t ldd, bool f32,
+                         hipStream_t st);
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
@@ -431,5 +432,5 @@ extern "C" int mx_gate_dw(const float* g, const void* x, int64_t ldx, int64_t to
   if (frags == 1) launch(gate_dw_kernel<1>);
   else launch(gate_dw_kernel<2>);
   if (hipGetLastError() != hipSuccess) return MX_ERR_LAUNCH;
-  return launch_splitk_reduce((const float*)workspace, (int)slices, experts, dim, dw, dim, (hipStream_t)stream);
+  return launch_splitk_reduce((const float*)workspace, (int)slices, experts, dim, dw, dim, false, (hipStream_t)stream);
 }

@@ -15,7 +15,7 @@ struct DenseArgs {
   int64_t ldk;  // bytes between operand rows (>= K)
 };
 
-template <int BM, int BN>
+template <int BM, int BN, bool F32 = false>
 __global__ __launch_bounds__(256, 1) void gemm_nt_kernel(DenseArgs p) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   using Tile = GemmTile<BM, BN, false, false>;
@@ -27,20 +27,20 @@ __global__ __launch_bounds__(256, 1) void gemm_nt_kernel(DenseArgs p) {
             p.a_scales + tm * (BM / 128) * ks_n * 256, ks_n};
   Operand B{p.b_codes + tn * BN * p.ldk, p.ldk, p.N - tn * BN,
             p.b_scales + tn * (BN / 128) * ks_n * 256, ks_n};
-  Tile::run(smem, A, B, 0, p.K, p.d + tm * BM * p.ldd + tn * BN, p.ldd);
+  Tile::template run<F32>(smem, A, B, 0, p.K, p.d + ((tm * BM * p.ldd + tn * BN) << (F32 ? 1 : 0)), p.ldd);
 }
 
-template <int BM, int BN>
+template <int BM, int BN, bool F32 = false>
 static bool configure_dense() {
   static std::atomic<bool> configured[kMaxDevices];  // a per-function, per-device setting
-  return raise_lds_limit(reinterpret_cast<const void*>(gemm_nt_kernel<BM, BN>), GemmTile<BM, BN, false, false>::kLdsBytes,
+  return raise_lds_limit(reinterpret_cast<const void*>(gemm_nt_kernel<BM, BN, F32>), GemmTile<BM, BN, false, false>::kLdsBytes,
                          configured);
 }
-template <int BM, int BN>
+template <int BM, int BN, bool F32 = false>
 static int launch_dense(const DenseArgs& p, hipStream_t st) {
   using Tile = GemmTile<BM, BN, false, false>;
-  auto kern = gemm_nt_kernel<BM, BN>;
-  if (!configure_dense<BM, BN>()) return MX_ERR_LAUNCH;
+  auto kern = gemm_nt_kernel<BM, BN, F32>;
+  if (!configure_dense<BM, BN, F32>()) return MX_ERR_LAUNCH;
   const int64_t nb = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
   const int64_t grid = (nb + 7) / 8 * 8;
   if (grid > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
@@ -55,7 +55,7 @@ using namespace mx;
 namespace mx {
 int launch_gemm_nt32(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                      const uint8_t* b_scales, void* d, int64_t M, int64_t N, int64_t K,
-                     int64_t ldk, int64_t ldd, hipStream_t st);
+                     int64_t ldk, int64_t ldd, bool f32, hipStream_t st);
 int launch_few_rows_codes(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                           const uint8_t* b_scales, void* d, int64_t M, int64_t N, int64_t K, int64_t ldk, int64_t ldd,
                           hipStream_t st);
@@ -63,7 +63,8 @@ GemmPlan plan_dense(int64_t M, int64_t N, int64_t K, bool may_split);
 bool prepare_dense32();
 int launch_gemm_nt32_splitk(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                             const uint8_t* b_scales, void* d, int64_t M, int64_t N, int64_t K,
-                            int64_t ldk, int64_t ldd, const GemmPlan& plan, void* workspace, hipStream_t st);
+                            int64_t ldk, int64_t ldd, const GemmPlan& plan, void* workspace, bool f32,
+                            hipStream_t st);
 }
 // Test hooks (include/mxfp8_debug.h), process-wide.
 // 0: pick by shape; 1 / 2: the 16x16x128 tile kernel with 256x256 / 128x128 tiles for every
@@ -132,7 +133,7 @@ static int gemm_nt_pitched(const uint8_t* a_codes, const uint8_t* a_scales, cons
     if (plan_dense(M, N, K, false).ta == 0) return launch_dense<128, 128>(p, st);
   }
   if (force_kernel == 1 || !persistent_ok(d, N, K, ldd, ldk)) return launch_dense<256, 256>(p, st);
-  return launch_gemm_nt32(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldk, ldd, st);
+  return launch_gemm_nt32(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldk, ldd, false, st);
 }
 
 extern "C" int mx_gemm_nt(const uint8_t* a_codes, const uint8_t* a_scales,
@@ -269,7 +270,27 @@ extern "C" int mx_gemm_nt_ld(const uint8_t* a_codes, const uint8_t* a_scales,
   if (plan.slices == 1 || workspace_bytes < split_bytes(plan, M, N) || ((uintptr_t)workspace & 15))
     return gemm_nt_pitched(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldk, ldd, stream);
   return launch_gemm_nt32_splitk(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldk, ldd,
-                                 plan, workspace, (hipStream_t)stream);
+                                 plan, workspace, false, (hipStream_t)stream);
+}
+
+extern "C" int mx_gemm_nt_f32_ld(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
+                                 const uint8_t* b_scales, float* d, int64_t M, int64_t N, int64_t K, int64_t ldk,
+                                 int64_t ldd, void* workspace, int64_t workspace_bytes, void* stream) {
+  const int rc = check_dense(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldd);
+  if (rc != MX_OK || M == 0 || N == 0) return rc;
+  if (ldk < K) return MX_ERR_INVALID_ARG;
+  // (the descriptor of a tile's output spans 256 rows of 4-byte values)
+  if (M <= 64 || N <= 128 || !persistent_ok(d, N, K, ldd, ldk) || (uint64_t)ldd * 1024 > 0x7FFFFFFFull)
+    return MX_ERR_UNSUPPORTED;
+  hipStream_t st = (hipStream_t)stream;
+  if (workspace && !((uintptr_t)workspace & 15)) {
+    const GemmPlan plan = split_plan(M, N, K);
+    if (plan.slices > 1 && workspace_bytes >= split_bytes(plan, M, N))
+      return launch_gemm_nt32_splitk(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldk, ldd, plan, workspace, true, st);
+  }
+  if (plan_dense(M, N, K, false).ta == 0)
+    return launch_dense<128, 128, true>(DenseArgs{a_codes, a_scales, b_codes, b_scales, (uint16_t*)d, M, N, K, ldd, ldk}, st);
+  return launch_gemm_nt32(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldk, ldd, true, st);
 }
 
 extern "C" int mx_gemm_nt_ws(const uint8_t* a_codes, const uint8_t* a_scales,
@@ -319,5 +340,5 @@ extern "C" int mx_gemm_nt_static(const uint8_t* a_codes, const uint8_t* a_scales
     return mx_gemm_nt(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldd, stream);
   if (!ws) return MX_ERR_LAUNCH;
   return launch_gemm_nt32_splitk(a_codes, a_scales, b_codes, b_scales, d, M, N, K, K, ldd,
-                                 plan, ws, (hipStream_t)stream);
+                                 plan, ws, false, (hipStream_t)stream);
 }

@@ -286,7 +286,10 @@ __device__ __forceinline__ constexpr uint32_t wave_col(uint32_t wn, int n) {
   return n < 4 ? wn * 128 + 16 * n : 64 + wn * 32 + 16 * (n - 4);
 }
 
-template <int MODE, bool PROF, bool PAIR = false, int TA = 4, int TB = 4>
+// OUT32 (kDense, one product): D is float32, its values rounded to bf16 first, as a conversion of a bf16 result
+// would give them; ldd counts floats.  (Instances of their own: a branch in front of the bf16 epilogue
+// made 147456 x 2048, K 2048 forward and backward 1.6 % slower.)
+template <int MODE, bool PROF, bool PAIR = false, int TA = 4, int TB = 4, bool OUT32 = false>
 __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   static_assert((TA == 4 && TB == 4) || MODE == kDense || MODE == kSplitK, "grouped tiles are 256 x 256");
@@ -488,7 +491,7 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
 #endif
       r.sa = a_scales + (int64_t)(tm * kEA / 128) * ks_n * 256;
       r.sb = b_scales + (int64_t)(tn * kEB / 128) * ks_n * 256;
-      r.d = d_base + (int64_t)tm * kEA * p.ldd + (int64_t)tn * kEB;
+      r.d = d_base + (((int64_t)tm * kEA * p.ldd + (int64_t)tn * kEB) << (OUT32 ? 1 : 0));
       r.rows_a = p.M - (int64_t)tm * kEA;
       r.rows_b = p.N - (int64_t)tn * kEB;
       r.odd = (tm & 1) | (tn & 1) << 1;
@@ -1163,6 +1166,31 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
       lds_write_b128_hidden<(k / kc) * 16 * kPatchPitch + (k % kc) * 64>(patch_w, w);
       __builtin_amdgcn_sched_barrier(0);
     };
+    if constexpr (OUT32) {
+      // The gradient of a float32 parameter or activation: bf16 values, 4 bytes each.  Written here they cost
+      // 4 bytes per element instead of the 8 of a bf16 matrix and its conversion by a launch of its own.  A store covers
+      // 4 rows of 64 columns (8 of 32), 16 bytes a lane.
+      const uint32_t ld_b = (uint32_t)p.ldd * 4;
+      const __amdgpu_buffer_rsrc_t rf = make_rsrc(t.d, rows_valid * ld_b);
+      static_for<0, kPieces>([&](auto p_) {
+        constexpr int pc = decltype(p_)::value, m = pc / kNP, np = pc % kNP;
+        constexpr int kLanes = col_parts(pc) == 2 ? 16 : 8, kRows = 64 / kLanes, kStores = 16 * kSubs / kRows;
+        static_for<0, parts_of(pc)>([&](auto k_) { stage_part(p_, k_); });
+        const uint32_t row = lane_e / kLanes, col = wave_col<TB>(wn, 4 * np) + (lane_e % kLanes) * 4;
+        const uint32_t from = patch + row * kPatchPitch + (lane_e % kLanes) * 8;
+        const uint32_t v = col < cols_valid ? (wm * 32 * TA + m * 16 * kSubs + row) * ld_b + col * 4 : 0x80000000u;
+        static_for<0, kStores>([&](auto q_) {
+          constexpr int q = decltype(q_)::value;
+          u32x2 x;
+          // (in order behind this wave's writes; waited for on the spot)
+          asm volatile("ds_read_b64 %0, %1 offset:%2\n\ts_waitcnt lgkmcnt(0)"
+                       : "=&v"(x) : "v"(from), "n"(q * kRows * kPatchPitch) : "memory");
+          const u32x4 w = {x.x << 16, x.x & 0xFFFF0000u, x.y << 16, x.y & 0xFFFF0000u};
+          __builtin_amdgcn_raw_buffer_store_b128(w, rf, v, q * kRows * ld_b, MX_STORE_AUX);
+        });
+      });
+      return;
+    }
     v4i r[2][4];
     static_for<0, parts_of(0)>([&](auto k_) { stage_part(std::integral_constant<int, 0>{}, k_); });
     static_for<0, kPieces>([&](auto p_) {
@@ -1298,17 +1326,17 @@ static int64_t persistent_grid() {
   return grid;
 }
 
-template <int MODE, bool PROF, bool PAIR = false, int TA = 4, int TB = 4>
+template <int MODE, bool PROF, bool PAIR = false, int TA = 4, int TB = 4, bool OUT32 = false>
 static bool configure32() {
   static std::atomic<bool> configured[kMaxDevices];
-  return raise_lds_limit(reinterpret_cast<const void*>(gemm_nt32_kernel<MODE, PROF, PAIR, TA, TB>),
+  return raise_lds_limit(reinterpret_cast<const void*>(gemm_nt32_kernel<MODE, PROF, PAIR, TA, TB, OUT32>),
                          Lds32<TA, TB>::kBytes, configured);
 }
-template <int MODE, bool PROF, bool PAIR = false, int TA = 4, int TB = 4>
+template <int MODE, bool PROF, bool PAIR = false, int TA = 4, int TB = 4, bool OUT32 = false>
 static int launch32(const Gemm32Args& p, int64_t nb, hipStream_t st) {
-  auto kern = gemm_nt32_kernel<MODE, PROF, PAIR, TA, TB>;
+  auto kern = gemm_nt32_kernel<MODE, PROF, PAIR, TA, TB, OUT32>;
   constexpr int lds = Lds32<TA, TB>::kBytes;  // ring + one output patch per wave: most of the CU's 160 KB
-  if (!configure32<MODE, PROF, PAIR, TA, TB>()) return MX_ERR_LAUNCH;
+  if (!configure32<MODE, PROF, PAIR, TA, TB, OUT32>()) return MX_ERR_LAUNCH;
   int64_t grid = persistent_grid();
   if (grid == 0) return MX_ERR_LAUNCH;
   const int64_t need = (nb + 7) / 8 * 8;  // nb: the tile count, or an upper bound of it
@@ -1417,35 +1445,35 @@ GemmPlan plan_dense(int64_t M, int64_t N, int64_t K, bool may_split) {
 }
 
 // Launches the persistent dense kernel on `p` with tiles of 64 ta x 64 tb.
-template <int MODE, bool PAIR, int TA, int TB>
+template <int MODE, bool PAIR, bool OUT32, int TA, int TB>
 static int launch_tile(Gemm32Args p, hipStream_t st) {
   int64_t tm = (p.M + 64 * TA - 1) / (64 * TA), tn = (p.N + 64 * TB - 1) / (64 * TB);
   if (p.two == kTwoA) tm *= 2;
   if (p.two == kTwoB) tn *= 2;
   if (MODE == kSplitK) p.tn_cnt = (int32_t)tn;
-  return launch32<MODE, false, PAIR, TA, TB>(p, tm * tn * (MODE == kSplitK ? p.G : 1), st);
+  return launch32<MODE, false, PAIR, TA, TB, OUT32>(p, tm * tn * (MODE == kSplitK ? p.G : 1), st);
 }
-template <int MODE, bool PAIR = false>
+template <int MODE, bool PAIR = false, bool OUT32 = false>
 static int launch_dense32(const Gemm32Args& p, int ta, int tb, hipStream_t st) {
   switch (ta * 16 + tb) {
-    case 0x44: return launch_tile<MODE, PAIR, 4, 4>(p, st);
-    case 0x24: return launch_tile<MODE, PAIR, 2, 4>(p, st);
-    case 0x42: return launch_tile<MODE, PAIR, 4, 2>(p, st);
+    case 0x44: return launch_tile<MODE, PAIR, OUT32, 4, 4>(p, st);
+    case 0x24: return launch_tile<MODE, PAIR, OUT32, 2, 4>(p, st);
+    case 0x42: return launch_tile<MODE, PAIR, OUT32, 4, 2>(p, st);
     default: break;
   }
   if constexpr (MODE != kSplitK) {
-    if (ta == 3 && tb == 4) return launch_tile<MODE, PAIR, 3, 4>(p, st);
-    if (ta == 4 && tb == 3) return launch_tile<MODE, PAIR, 4, 3>(p, st);
+    if (ta == 3 && tb == 4) return launch_tile<MODE, PAIR, OUT32, 3, 4>(p, st);
+    if (ta == 4 && tb == 3) return launch_tile<MODE, PAIR, OUT32, 4, 3>(p, st);
   }
   return MX_ERR_UNSUPPORTED;
 }
 // ... with the tile that suits its shape
-template <bool PAIR = false>
+template <bool PAIR = false, bool OUT32 = false>
 static int launch_best32(const Gemm32Args& p, hipStream_t st) {
   const int64_t grid = persistent_grid();
   if (grid == 0) return MX_ERR_LAUNCH;
   const DenseTile* t = best_tile(p.M, p.N, (PAIR ? 2 : 1) * p.K / kKB, p.two ? 2 : 1, grid);
-  return t ? launch_dense32<kDense, PAIR>(p, t->ta, t->tb, st) : MX_ERR_UNSUPPORTED;
+  return t ? launch_dense32<kDense, PAIR, OUT32>(p, t->ta, t->tb, st) : MX_ERR_UNSUPPORTED;
 }
 
 // Raises the LDS limits of every kernel that a dense product may run on, for a caller that captures
@@ -1464,17 +1492,20 @@ void set_debug_prof(uint64_t* buf) { debug_prof = buf; }
 
 int launch_gemm_nt32(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                      const uint8_t* b_scales, void* d, int64_t M, int64_t N, int64_t K,
-                     int64_t ldk, int64_t ldd, hipStream_t st) {
+                     int64_t ldk, int64_t ldd, bool f32, hipStream_t st) {
   Gemm32Args p{a_codes, a_scales, b_codes, b_scales, (uint16_t*)d, M, N, K, ldd, nullptr, 0, 0, 0, debug_prof};
   p.ldk = ldk;
 #ifdef MX_TIMING_BUILD
   if (debug_prof) return launch32<kDense, true>(p, ((M + kT32 - 1) / kT32) * ((N + kT32 - 1) / kT32), st);
 #endif
+  if (f32) return launch_best32<false, true>(p, st);
   return launch_best32(p, st);
 }
 
 // ---- split along K for shapes whose 256x256 tiles do not fill the CUs ----------------------
-// Sum of the S float32 partial matrices [S][M][N], in slice order, rounded once to bf16.
+// Sum of the S float32 partial matrices [S][M][N], in slice order, rounded once to bf16 (F32: and written as
+// float32).
+template <bool F32>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ part, int S,
                                                             int64_t M, int64_t N,
                                                             uint16_t* __restrict__ d, int64_t ldd) {
@@ -1496,28 +1527,36 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
     acc[0] += lo.x; acc[1] += lo.y; acc[2] += lo.z; acc[3] += lo.w;
     acc[4] += hi.x; acc[5] += hi.y; acc[6] += hi.z; acc[7] += hi.w;
   }
+  if constexpr (F32) {
+    v4f* out = reinterpret_cast<v4f*>(reinterpret_cast<float*>(d) + r * ldd + c);
+    out[0] = v4f{round_bf16(acc[0]), round_bf16(acc[1]), round_bf16(acc[2]), round_bf16(acc[3])};
+    out[1] = v4f{round_bf16(acc[4]), round_bf16(acc[5]), round_bf16(acc[6]), round_bf16(acc[7])};
+    return;
+  }
   const u32x4 w = {pack_bf16(acc[0], acc[1]), pack_bf16(acc[2], acc[3]), pack_bf16(acc[4], acc[5]),
                    pack_bf16(acc[6], acc[7])};
   *reinterpret_cast<u32x4*>(d + r * ldd + c) = w;
 }
 
-int launch_splitk_reduce(const float* part, int slices, int64_t M, int64_t N, void* d, int64_t ldd, hipStream_t st) {
+int launch_splitk_reduce(const float* part, int slices, int64_t M, int64_t N, void* d, int64_t ldd, bool f32,
+                         hipStream_t st) {
   const int64_t threads = M * (N / 8);
-  hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, part, slices, M,
-                     N, (uint16_t*)d, ldd);
+  hipLaunchKernelGGL(f32 ? splitk_reduce_kernel<true> : splitk_reduce_kernel<false>, dim3((unsigned)((threads + 255) / 256)),
+                     dim3(256), 0, st, part, slices, M, N, (uint16_t*)d, ldd);
   return hipGetLastError() == hipSuccess ? MX_OK : MX_ERR_LAUNCH;
 }
 
 // D = sum over slices, through `workspace` (S * M * N floats).
 int launch_gemm_nt32_splitk(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                             const uint8_t* b_scales, void* d, int64_t M, int64_t N, int64_t K,
-                            int64_t ldk, int64_t ldd, const GemmPlan& plan, void* workspace, hipStream_t st) {
+                            int64_t ldk, int64_t ldd, const GemmPlan& plan, void* workspace, bool f32,
+                            hipStream_t st) {
   Gemm32Args p{a_codes, a_scales, b_codes, b_scales, (uint16_t*)workspace, M, N, K, N, nullptr,
                plan.slices, 0, 0, nullptr};
   p.ldk = ldk;
   const int rc = launch_dense32<kSplitK>(p, plan.ta, plan.tb, st);
   if (rc != MX_OK) return rc;
-  return launch_splitk_reduce((const float*)workspace, plan.slices, M, N, d, ldd, st);
+  return launch_splitk_reduce((const float*)workspace, plan.slices, M, N, d, ldd, f32, st);
 }
 
 // Grouped forms with every group end a multiple of 32 and all scales in MFMA order

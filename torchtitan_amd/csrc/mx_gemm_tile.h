@@ -65,6 +65,9 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{lo, hi}, v2bf));
 }
 
+// a float32 rounded to bf16, as float32
+__device__ __forceinline__ float round_bf16(float x) { return __uint_as_float(pack_bf16(x, x) << 16); }
+
 template <int BM, int BN, bool A_ROWMAJOR, bool B_ROWMAJOR>
 struct GemmTile {
   static constexpr int WM = BM / 2, WN = BN / 2;
@@ -78,6 +81,8 @@ struct GemmTile {
 
   // k_begin/k_end: contraction range in elements (multiples of 32); for MFMA-order scales
   // k_begin must be 0.  d points at the tile's first output element.
+  // F32: D is float32, the values rounded to bf16 all the same (N % 8 == 0, ldd % 4 == 0, 16-byte aligned).
+  template <bool F32 = false>
   __device__ __forceinline__ static void run(uint8_t* smem, const Operand& A, const Operand& B, int64_t k_begin,
                              int64_t k_end, uint16_t* __restrict__ d, int64_t ldd) {
     const int tid = threadIdx.x;
@@ -272,6 +277,11 @@ struct GemmTile {
         const int64_t c = wn * WN + n * 16 + lj * 4;
         if (c >= cols_valid) continue;
         const v4f a = acc[m][n];
+        if constexpr (F32) {  // (aligned rows of whole 8s)
+          *reinterpret_cast<v4f*>(reinterpret_cast<float*>(d) + r * ldd + c) =
+              v4f{round_bf16(a.x), round_bf16(a.y), round_bf16(a.z), round_bf16(a.w)};
+          continue;
+        }
         uint16_t* dst = d + r * ldd + c;
         const u32x2 w = {pack_bf16(a.x, a.y), pack_bf16(a.z, a.w)};
         if (vec_ok && c + 3 < cols_valid) {

@@ -292,15 +292,11 @@ class _MXLinear(torch.autograd.Function):
         dyq0, dyq1 = ops.to_operands(dy2, mode, need_dx, need_dw, pad)
         dx = dw = None
         if need_dx:
-            dx = ops.mx_gemm_nt(dyq0, ops.Operand(w_buf, ctx.w_layout))
+            dx = ops.mx_gemm_nt_as(dyq0, ops.Operand(w_buf, ctx.w_layout), ctx.x_dtype)
             if len(ctx.x_shape) != 2:
                 dx = dx.view(ctx.x_shape)
-            if dx.dtype != ctx.x_dtype:
-                dx = dx.to(ctx.x_dtype)
         if need_dw:
-            dw = ops.mx_gemm_nt(dyq1, ops.Operand(x_buf, ctx.x_layout))
-            if dw.dtype != ctx.w_dtype:
-                dw = dw.to(ctx.w_dtype)
+            dw = ops.mx_gemm_nt_as(dyq1, ops.Operand(x_buf, ctx.x_layout), ctx.w_dtype)
         return dx, dw, None
 
 

@@ -991,6 +991,23 @@ def _gemm_operands(a: Operand, b: Operand, out: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def mx_gemm_nt_as(a: MXData, b: MXData, dtype: torch.dtype) -> torch.Tensor:
+    """`mx_gemm_nt` in `dtype`: the bf16 result, for float32 written as such by the product itself where it takes
+    the shape (147456 x 2048 of float32 gradient: 8 of the 12 bytes an element that the product and a
+    conversion move)."""
+    if dtype == torch.float32 and _operands(a, b) and not _watched() and a.depth == b.depth:
+        M, N, K, dev = a.rows, b.rows, a.k, a.buf.device
+        if M > 64 and N > 128 and N % 8 == 0 and max(N * 1024, a.ld * 256) < 1 << 31:
+            out = torch.empty((M, N), dtype=torch.float32, device=dev)
+            ws = _split_workspace(dev, M, N, K)
+            _call("mx_gemm_nt_f32_ld", "gemm_nt" if ws is None else "gemm_nt_splitk", dev, a.codes_ptr, a.scales_ptr,
+                  b.codes_ptr, b.scales_ptr, out.data_ptr(), M, N, K, a.ld, N, None if ws is None else ws.data_ptr(),
+                  0 if ws is None else ws.numel(), _stream(out))
+            return out
+    out = mx_gemm_nt(a, b)
+    return out if out.dtype == dtype else out.to(dtype)
+
+
 FEW_ROWS = 32             # rows that `mx_few_rows` takes
 FEW_ROWS_VALUES = 65536   # values of x, rows counted in whole 16s, up to which it is chosen
 FEW_ROWS_COLUMNS = 16384  # columns of all products, up to which it is chosen

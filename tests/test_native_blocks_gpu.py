@@ -1,0 +1,209 @@
+"""Linears, SwiGLU blocks and routed experts whose launches come from one native call (csrc/host/blocks.cpp) against
+the general path over the forms that the call accepts, and those that it hands back: bit for bit, results and gradients."""
+import pytest
+import torch
+import torch.nn as nn
+
+from tests.test_converter_gpu import _convert
+from torchtitan_amd import _lib, mx_tensor, ops
+from torchtitan_amd.modules import FeedForward, Linear
+from torchtitan_amd.modules.moe import MoE
+
+pytestmark = pytest.mark.gpu
+
+
+class _Counted:
+    """The native module with the calls that it took, by name."""
+
+    def __init__(self, module):
+        self._module, self.taken = module, []
+
+    def __getattr__(self, name):
+        fn = getattr(self._module, name)
+
+        def call(*args):
+            out = fn(*args)
+            if out is not None:
+                self.taken.append(name)
+            return out
+        return call
+
+
+def _both(monkeypatch, fn):
+    """(fn() on native calls, fn() on the general path, names of the native calls taken)."""
+    counted = _Counted(_lib.blocks())
+    mx_tensor.clear_cast_cache()
+    with monkeypatch.context() as m:
+        m.setattr(_lib, "blocks", lambda: counted)
+        native = fn()
+    mx_tensor.clear_cast_cache()
+    with monkeypatch.context() as m:
+        m.setattr(ops, "native_block_ok", lambda *a: False)
+        general = fn()
+    return native, general, counted.taken
+
+
+def _same(a, b):
+    for i, (x, y) in enumerate(zip(a, b, strict=True)):
+        assert x.dtype == y.dtype and x.shape == y.shape, i
+        assert torch.equal(x, y), i
+
+
+def _step(block, params, x, dy, autocast=False, hooks=None):
+    x = x.detach().requires_grad_(True)
+    with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast), hooks() if hooks else torch.enable_grad():
+        y = block(x)
+    return [y.detach(), *torch.autograd.grad(y, [x, *params], dy)]
+
+
+def _holder(module, device, dtype=torch.bfloat16, **kw):
+    holder = nn.Module()
+    holder.block = module
+    holder.to(device).to(dtype)
+    for p in module.parameters():
+        nn.init.normal_(p, 0.0, 0.02)
+    _convert(holder, ["block"], **kw)
+    return module
+
+
+FORMS = {
+    "plain": lambda t, w: torch.randn(t, w),
+    "rows of a wider matrix": lambda t, w: torch.randn(t, w + 64)[:, :w],
+    "rows that are not aligned": lambda t, w: torch.randn(t, w + 3)[:, 3:],
+    "columns first": lambda t, w: torch.randn(w, t).t(),
+    "one row for all": lambda t, w: torch.randn(1, w).expand(t, w),
+    "three dimensions": lambda t, w: torch.randn(1, t, w),
+}
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("tokens,inner,outer", [(1, 160, 256), (33, 256, 160), (129, 512, 384), (300, 160, 144), (700, 384, 1056)])
+@pytest.mark.parametrize("params", ["bfloat16", "float32"])
+def test_linear(device, monkeypatch, form, tokens, inner, outer, params):
+    torch.manual_seed(tokens + inner)
+    dtype = getattr(torch, params)
+    lin = _holder(Linear.Config().build(in_features=inner, out_features=outer), device, dtype)
+    make = lambda w, dt: FORMS[form](tokens, w).to(device).to(dt)
+    x, dy = make(inner, dtype), make(outer, torch.bfloat16)
+    run = lambda: _step(lin, [lin.weight], x, dy, autocast=params == "float32")
+    native, general, taken = _both(monkeypatch, run)
+    _same(native, general)
+    if form in ("plain", "rows of a wider matrix", "three dimensions"):
+        assert "linear_forward" in taken and ("linear_backward" in taken) == (outer % 32 == 0)
+    with torch.no_grad():
+        native, general, taken = _both(monkeypatch, lambda: [lin(x) if params == "bfloat16" else lin(x.bfloat16())])
+    _same(native, general)
+
+
+@pytest.mark.parametrize("tokens", [1, 32, 33, 64, 65, 300])
+@pytest.mark.parametrize("cached", [True, False])
+def test_linear_without_gradients(device, monkeypatch, tokens, cached):
+    lin = _holder(Linear.Config().build(in_features=2176, out_features=288), device, cache=cached)
+    x = torch.randn(tokens, 2176, device=device, dtype=torch.bfloat16)
+    with torch.no_grad():
+        native, general, taken = _both(monkeypatch, lambda: [lin(x), lin(x)])
+    _same(native, general)
+    assert "linear_apply" in taken
+
+
+def test_siblings_and_frozen_weights(device, monkeypatch):
+    """Linears on one activation share its cast whichever path made it; a frozen weight leaves the native call out."""
+    a = _holder(Linear.Config().build(in_features=256, out_features=384), device)
+    b = _holder(Linear.Config().build(in_features=256, out_features=160), device)
+    x0 = torch.randn(130, 256, device=device, dtype=torch.bfloat16)
+
+    def both():
+        x = x0.detach().requires_grad_(True)
+        ya, yb = a(x), b(x)
+        grads = torch.autograd.grad(ya.sum() + yb.sum(), [x, a.weight, b.weight])
+        return [ya.detach(), yb.detach(), *grads]
+    native, general, taken = _both(monkeypatch, both)
+    _same(native, general)
+    assert taken.count("linear_forward") == 1
+    b.weight.requires_grad_(False)
+
+    def frozen():
+        x = x0.detach().requires_grad_(True)
+        y = b(x)
+        return [y.detach(), *torch.autograd.grad(y.float().sum(), [x])]
+    native, general, taken = _both(monkeypatch, frozen)
+    _same(native, general)
+    assert taken == []
+
+
+@pytest.mark.parametrize("form", ["plain", "rows of a wider matrix", "columns first", "three dimensions"])
+@pytest.mark.parametrize("tokens,dim,hidden", [(33, 160, 256), (129, 256, 160), (300, 384, 544)])
+def test_feed_forward(device, monkeypatch, form, tokens, dim, hidden):
+    torch.manual_seed(tokens)
+    ff = _holder(FeedForward.Config(hidden_dim=hidden).build(dim=dim), device)
+    x, dy = (FORMS[form](tokens, dim).to(device).bfloat16() for _ in range(2))
+    run = lambda: _step(ff, list(ff.parameters()), x, dy)
+    native, general, taken = _both(monkeypatch, run)
+    _same(native, general)
+    if form != "columns first":
+        assert taken == ["ffn_forward", "ffn_backward"]
+    # saved tensors that come back as other tensors
+    native, general, taken = _both(monkeypatch, lambda: _step(ff, list(ff.parameters()), x, dy, hooks=lambda: torch.autograd.graph.save_on_cpu()))
+    _same(native, general)
+
+
+@pytest.mark.parametrize("before", [True, False])
+@pytest.mark.parametrize("experts,top_k,shared,tokens", [(1, 1, 0, 40), (8, 2, 1, 200), (16, 4, 0, 37)])
+def test_routed_experts(device, monkeypatch, experts, top_k, shared, tokens, before):
+    torch.manual_seed(tokens)
+    moe = MoE(MoE.Config(num_experts=experts, num_shared_experts=shared, hidden_dim=256, top_k=top_k, score_func="softmax",
+                         score_before_experts=before, route_norm=True), dim=384).to(device).to(torch.bfloat16)
+    moe.init_weights(init_std=0.02, buffer_device=device)
+    holder = nn.Module()
+    holder.moe = moe
+    _convert(holder, ["experts"])
+    x, dy = (torch.randn(1, tokens, 384, device=device, dtype=torch.bfloat16) for _ in range(2))
+
+    def run():
+        moe.tokens_per_expert.zero_()
+        return [*_step(moe, list(moe.parameters()), x, dy), moe.tokens_per_expert.clone()]
+    native, general, taken = _both(monkeypatch, run)
+    _same(native, general)
+    if experts % 8 == 0:  # (the gate's and the router's own kernels, whose choices the call takes)
+        assert "routed_forward" in taken and "routed_backward" in taken
+
+
+def test_capture_and_threads(device):
+    """A captured step of native calls replays on new inputs; two threads on streams of their own."""
+    import threading
+
+    lin = _holder(Linear.Config().build(in_features=256, out_features=384), device)
+    x = torch.randn(200, 256, device=device, dtype=torch.bfloat16, requires_grad=True)
+    dy = torch.randn(200, 384, device=device, dtype=torch.bfloat16)
+    step = lambda: torch.autograd.grad(lin(x), [x, lin.weight], dy)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        for _ in range(2):
+            step()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    for seed in range(3):
+        torch.manual_seed(seed)
+        with torch.no_grad():
+            x.copy_(torch.randn(200, 256, device=device))
+        graph.replay()
+        torch.cuda.synchronize()
+        _same(out, step())
+
+    want, got = [t.clone() for t in step()], {}
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(10):
+                got[i] = step()
+            torch.cuda.current_stream().synchronize()
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for i in range(2):
+        _same(got[i], want)

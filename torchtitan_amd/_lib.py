@@ -116,6 +116,24 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+_blocks = None
+
+
+def blocks():
+    """The native host module (csrc/host/blocks.cpp), bound to the library that `load` has loaded."""
+    global _blocks
+    if _blocks is None:
+        try:
+            from . import _blocks as module
+        except ImportError as ex:
+            raise MXLibraryError("torchtitan_amd/_blocks.so is missing or does not fit this torch: build it with "
+                                 "`python -m torchtitan_amd._build`") from ex
+        lib = load()
+        module.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in SIGNATURES}, check)
+        _blocks = module
+    return _blocks
+
+
 def check(status: int, what: str) -> None:
     if status != 0:
         msg = load().mx_status_string(status).decode()

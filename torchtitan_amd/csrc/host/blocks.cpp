@@ -1,0 +1,462 @@
+// The launches of a converted linear, of the SwiGLU block and of the routed experts, forward and backward, from one
+// native call each.
+//
+// On inputs of up to a few thousand tokens these blocks wait for their host side: between two launches
+// (3.3 us each) Python made operands, asked tensors for their pointers and strides and passed them on, 4 to 8 us
+// a step.  Here the same entry points of the library are called with the same arguments in the same order
+// (ops.py, mx_tensor.py and mx_blocks.py have them step by step); what is allocated is what is allocated there.
+// Nothing is kept between calls, no pointer outlives one.  Every function checks that its inputs are the plain
+// case -- bf16 or float32 matrices on the current GPU whose rows the casts read as they lie -- and returns None
+// otherwise: the caller then takes the general path.
+#include <c10/hip/HIPStream.h>
+#include <torch/extension.h>
+
+#include <array>
+
+#include "mxfp8.h"
+
+namespace py = pybind11;
+using at::Tensor;
+
+namespace {
+
+// ---- the library's entry points: addresses of the symbols that the caller has loaded
+struct Library {
+  decltype(&mx_cast_pad) cast_pad = nullptr;
+  decltype(&mx_cast_pad_many) cast_pad_many = nullptr;
+  decltype(&mx_swiglu_cast_pad) swiglu = nullptr;
+  decltype(&mx_swiglu_bwd_cast_pad) swiglu_bwd = nullptr;
+  decltype(&mx_gemm_nt_workspace_bytes) workspace_bytes = nullptr;
+  decltype(&mx_gemm_nt_ld) gemm = nullptr;
+  decltype(&mx_gemm_nt_f32_ld) gemm_f32 = nullptr;
+  decltype(&mx_gemm_nt_shared_a_ld) shared_a = nullptr;
+  decltype(&mx_gemm_nt_shared_b_ld) shared_b = nullptr;
+  decltype(&mx_gemm_nt_pair_ld) pair = nullptr;
+  decltype(&mx_few_rows) few_rows = nullptr;
+  decltype(&mx_route_fill) route_fill = nullptr;
+  decltype(&mx_cast_rows_gathered) rows_gathered = nullptr;
+  decltype(&mx_swiglu_cast_dim0_dim1_ld) swiglu_dense = nullptr;
+  decltype(&mx_swiglu_bwd_cast_dim0_dim1_ld) swiglu_bwd_dense = nullptr;
+  decltype(&mx_grouped_gemm_2d3d) grouped = nullptr;
+  decltype(&mx_grouped_gemm_2d3d_shared_a) grouped_shared_a = nullptr;
+  decltype(&mx_grouped_gemm_2d3d_pair) grouped_pair = nullptr;
+  decltype(&mx_grouped_gemm_2d2d) grouped_wgrad = nullptr;
+  decltype(&mx_grouped_gemm_2d2d_shared_b) grouped_wgrad_two = nullptr;
+  decltype(&mx_moe_combine) combine = nullptr;
+  decltype(&mx_moe_combine_dot) combine_dot = nullptr;
+} lib;
+PyObject* check_status = nullptr;  // _lib.check, never released
+
+void bind(const py::dict& addresses, const py::object& check) {
+  auto set = [&](const char* name, auto& fn) {
+    fn = reinterpret_cast<std::decay_t<decltype(fn)>>(addresses[name].cast<uintptr_t>());
+  };
+  set("mx_cast_pad", lib.cast_pad);
+  set("mx_cast_pad_many", lib.cast_pad_many);
+  set("mx_swiglu_cast_pad", lib.swiglu);
+  set("mx_swiglu_bwd_cast_pad", lib.swiglu_bwd);
+  set("mx_gemm_nt_workspace_bytes", lib.workspace_bytes);
+  set("mx_gemm_nt_ld", lib.gemm);
+  set("mx_gemm_nt_f32_ld", lib.gemm_f32);
+  set("mx_gemm_nt_shared_a_ld", lib.shared_a);
+  set("mx_gemm_nt_shared_b_ld", lib.shared_b);
+  set("mx_gemm_nt_pair_ld", lib.pair);
+  set("mx_few_rows", lib.few_rows);
+  set("mx_route_fill", lib.route_fill);
+  set("mx_cast_rows_gathered", lib.rows_gathered);
+  set("mx_swiglu_cast_dim0_dim1_ld", lib.swiglu_dense);
+  set("mx_swiglu_bwd_cast_dim0_dim1_ld", lib.swiglu_bwd_dense);
+  set("mx_grouped_gemm_2d3d", lib.grouped);
+  set("mx_grouped_gemm_2d3d_shared_a", lib.grouped_shared_a);
+  set("mx_grouped_gemm_2d3d_pair", lib.grouped_pair);
+  set("mx_grouped_gemm_2d2d", lib.grouped_wgrad);
+  set("mx_grouped_gemm_2d2d_shared_b", lib.grouped_wgrad_two);
+  set("mx_moe_combine", lib.combine);
+  set("mx_moe_combine_dot", lib.combine_dot);
+  check_status = check.ptr();
+  Py_INCREF(check_status);
+}
+
+void checked(int status, const char* name) {
+  if (status) py::reinterpret_borrow<py::object>(check_status)(status, name);  // raises
+}
+
+// ---- operands (ops.Operand): codes [rows, cols up to 128], rows `ld` bytes apart, then the scales
+struct Operand {
+  Tensor buf;
+  int64_t rows, k, ld, at, scales_at, depth;
+  uint8_t* codes() const { return buf.data_ptr<uint8_t>() + at; }
+  uint8_t* scales() const { return buf.data_ptr<uint8_t>() + scales_at; }
+  py::tuple layout() const { return py::make_tuple(rows, k, ld, at, scales_at, depth); }
+};
+
+int64_t up128(int64_t n) { return (n + 127) & ~int64_t{127}; }
+
+// ... around a buffer laid out as `make` lays it out
+Operand around(const Tensor& buf, int64_t rows, int64_t cols, int64_t pad) {
+  const int64_t k = up128(cols), ld = k + pad;
+  return {buf, rows, k, ld, 0, (rows * ld + 255) & ~int64_t{255}, cols};
+}
+Operand make(int64_t rows, int64_t cols, int64_t pad, const Tensor& like) {
+  Operand o = around(Tensor(), rows, cols, pad);
+  o.buf = at::empty({o.scales_at + up128(rows) * (o.k / 32)}, like.options().dtype(at::kByte));
+  return o;
+}
+std::array<Operand, 2> make_pair(int64_t rows, int64_t cols, int64_t pad, const Tensor& like) {
+  Operand a = around(Tensor(), rows, cols, pad), b = a;
+  const int64_t scales = up128(rows) * (a.k / 32);
+  a.scales_at = (2 * rows * a.ld + 255) & ~int64_t{255};
+  b.at = rows * a.ld;
+  b.scales_at = a.scales_at + scales;
+  a.buf = b.buf = at::empty({a.scales_at + 2 * scales}, like.options().dtype(at::kByte));
+  return {a, b};
+}
+
+// A matrix that the casts read as it lies (ops._operand_input returns it unchanged)
+bool plain(const Tensor& t) {
+  if (!t.is_cuda() || t.dim() != 2) return false;
+  const auto type = t.scalar_type();
+  if (type != at::kBFloat16 && type != at::kFloat) return false;
+  const int64_t size = type == at::kFloat ? 4 : 2;
+  return t.size(0) > 0 && t.size(1) > 0 && t.size(1) % 32 == 0 && t.stride(1) == 1 && t.stride(0) >= t.size(1) &&
+         t.stride(0) * size % 16 == 0 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+}
+bool plain_weight(const Tensor& w, const Tensor& x) {
+  return plain(w) && w.is_contiguous() && w.device() == x.device();
+}
+bool on_current_device(const Tensor& t) { return t.device().index() == c10::hip::current_device(); }
+hipStream_t stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+void add_cast(std::array<int64_t, 8 * MX_CAST_PAD_MANY_FIELDS>& table, int64_t& n, const Tensor& x, const Operand& r,
+              const Operand& c) {
+  const int64_t entry[MX_CAST_PAD_MANY_FIELDS] = {
+      reinterpret_cast<int64_t>(x.data_ptr()), x.scalar_type() == at::kFloat, 1, x.size(0), x.size(1), x.stride(0),
+      reinterpret_cast<int64_t>(r.codes()), r.ld, reinterpret_cast<int64_t>(r.scales()),
+      reinterpret_cast<int64_t>(c.codes()), c.ld, reinterpret_cast<int64_t>(c.scales())};
+  std::copy(entry, entry + MX_CAST_PAD_MANY_FIELDS, table.begin() + MX_CAST_PAD_MANY_FIELDS * n++);
+}
+
+// ops._gemm_operands, into rows of `out` (2-D, unit inner stride)
+void gemm_into(const Operand& a, const Operand& b, const Tensor& out, hipStream_t st) {
+  const int64_t need = lib.workspace_bytes(a.rows, b.rows, a.k);
+  const Tensor ws = need ? at::empty({need}, a.buf.options()) : Tensor();
+  checked(lib.gemm(a.codes(), a.scales(), b.codes(), b.scales(), out.data_ptr(), a.rows, b.rows, a.k, a.ld, out.stride(0),
+                   need ? ws.data_ptr() : nullptr, need, st),
+          "mx_gemm_nt_ld");
+}
+// ops.mx_gemm_nt_as
+Tensor gemm(const Operand& a, const Operand& b, const Tensor& like, hipStream_t st, at::ScalarType type = at::kBFloat16) {
+  const int64_t M = a.rows, N = b.rows;
+  if (type == at::kFloat && M > 64 && N > 128 && N % 8 == 0 && std::max(N * 1024, a.ld * 256) < (int64_t{1} << 31)) {
+    Tensor out = at::empty({M, N}, like.options().dtype(at::kFloat));
+    const int64_t need = lib.workspace_bytes(M, N, a.k);
+    const Tensor ws = need ? at::empty({need}, a.buf.options()) : Tensor();
+    checked(lib.gemm_f32(a.codes(), a.scales(), b.codes(), b.scales(), out.data_ptr<float>(), M, N, a.k, a.ld, N,
+                         need ? ws.data_ptr() : nullptr, need, st),
+            "mx_gemm_nt_f32_ld");
+    return out;
+  }
+  Tensor out = at::empty({M, N}, like.options().dtype(at::kBFloat16));
+  gemm_into(a, b, out, st);
+  return type == at::kBFloat16 ? out : out.to(type);
+}
+
+bool persistent_shape(int64_t M, int64_t N) { return M > 128 && N > 128 && N % 8 == 0; }
+
+// ---- the linear ----------------------------------------------------------------------------------
+// (y, row-wise x, column-wise x, column-wise W) of y = x W^T; operands as (buffer, layout)
+py::object linear_forward(const Tensor& x, const Tensor& w, int mode, int64_t pad) {
+  if (!plain(x) || !plain_weight(w, x) || x.size(1) != w.size(1) || !on_current_device(x)) return py::none();
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  hipStream_t st = stream_of(x);
+  const Operand xr = make(M, K, pad, x), xc = make(K, M, pad, x), wr = make(N, K, pad, x), wc = make(K, N, pad, x);
+  std::array<int64_t, 8 * MX_CAST_PAD_MANY_FIELDS> table;
+  int64_t n = 0;
+  add_cast(table, n, x, xr, xc);
+  add_cast(table, n, w, wr, wc);
+  checked(lib.cast_pad_many(n, table.data(), mode, st), "mx_cast_pad_many");
+  const Tensor y = gemm(xr, wr, x, st);
+  return py::make_tuple(y, xr.buf, xr.layout(), xc.buf, xc.layout(), wc.buf, wc.layout());
+}
+
+// (dx, dW) from dy and the buffers of linear_forward's column-wise operands
+py::object linear_backward(const Tensor& dy, const Tensor& x_buf, const Tensor& w_buf, int64_t K, int mode, int64_t pad,
+                           bool dx_f32, bool dw_f32) {
+  if (!plain(dy) || !on_current_device(dy)) return py::none();
+  const int64_t M = dy.size(0), N = dy.size(1);
+  hipStream_t st = stream_of(dy);
+  const Operand r = make(M, N, pad, dy), c = make(N, M, pad, dy);
+  checked(lib.cast_pad(dy.data_ptr(), dy.scalar_type() == at::kFloat, M, N, dy.stride(0), r.codes(), r.ld, r.scales(),
+                       c.codes(), c.ld, c.scales(), mode, st),
+          "mx_cast_pad");
+  const Tensor dx = gemm(r, around(w_buf, K, N, pad), dy, st, dx_f32 ? at::kFloat : at::kBFloat16);
+  const Tensor dw = gemm(c, around(x_buf, K, M, pad), dy, st, dw_f32 ? at::kFloat : at::kBFloat16);
+  return py::make_tuple(dx, dw);
+}
+
+// y = x W^T without gradients, W's row-wise operand given (its buffers and layout): (y, row-wise x or None).
+// `few_rows`, `few_values`, `few_columns`: up to where the product that casts x itself runs (ops.few_rows_ok).
+py::object linear_apply(const Tensor& x, const Tensor& w_buf, const Tensor& w_scales, const std::array<int64_t, 6>& layout,
+                        int mode, int64_t few_rows, int64_t few_values, int64_t few_columns) {
+  const auto [N, k, ld, at, scales_at, depth] = layout;
+  if (!plain(x) || x.size(1) != depth || ld % 128 || w_buf.device() != x.device() || !on_current_device(x)) return py::none();
+  const int64_t M = x.size(0), K = x.size(1);
+  hipStream_t st = stream_of(x);
+  const uint8_t* codes = w_buf.data_ptr<uint8_t>() + at;
+  const uint8_t* scales = w_scales.data_ptr<uint8_t>() + scales_at;
+  if (x.scalar_type() == at::kBFloat16 && M <= few_rows && N <= few_columns && ((M + 15) & ~int64_t{15}) * K <= few_values) {
+    const Tensor y = at::empty({M, N}, x.options());
+    checked(lib.few_rows(x.data_ptr(), M, K, x.stride(0), codes, scales, nullptr, nullptr, N, ld, y.data_ptr(), nullptr, N,
+                         mode, st),
+            "mx_few_rows");
+    return py::make_tuple(y, py::none(), py::none());
+  }
+  const Operand xr = make(M, K, ld - k, x);
+  checked(lib.cast_pad(x.data_ptr(), x.scalar_type() == at::kFloat, M, K, x.stride(0), xr.codes(), xr.ld, xr.scales(), nullptr,
+                       0, nullptr, mode, st),
+          "mx_cast_pad");
+  const Tensor y = at::empty({M, N}, x.options().dtype(at::kBFloat16));
+  const int64_t need = lib.workspace_bytes(M, N, k);
+  const Tensor ws = need ? at::empty({need}, xr.buf.options()) : Tensor();
+  checked(lib.gemm(xr.codes(), xr.scales(), codes, scales, y.data_ptr(), M, N, k, ld, N, need ? ws.data_ptr() : nullptr, need,
+                   st),
+          "mx_gemm_nt_ld");
+  return py::make_tuple(y, xr.buf, xr.layout());
+}
+
+// ---- the SwiGLU block ----------------------------------------------------------------------------
+// (y, h13, then row-wise x and column-wise W2, x, g, W1, W3 as (buffer, layout)) of
+// y = (silu(x W1^T) * (x W3^T)) W2^T
+py::object ffn_forward(const Tensor& x, const Tensor& w1, const Tensor& w3, const Tensor& w2, int mode, int64_t pad) {
+  if (!plain(x) || x.scalar_type() != at::kBFloat16 || !plain_weight(w1, x) || !plain_weight(w3, x) ||
+      !plain_weight(w2, x) || !on_current_device(x))
+    return py::none();
+  const int64_t M = x.size(0), D = x.size(1), H = w1.size(0), O = w2.size(0);
+  if (w1.size(1) != D || w3.size(1) != D || w3.size(0) != H || w2.size(1) != H) return py::none();
+  hipStream_t st = stream_of(x);
+  const Operand xr = make(M, D, pad, x), xc = make(D, M, pad, x);
+  const Operand w1r = make(H, D, pad, x), w1c = make(D, H, pad, x), w3r = make(H, D, pad, x), w3c = make(D, H, pad, x);
+  const Operand w2r = make(O, H, pad, x), w2c = make(H, O, pad, x);
+  std::array<int64_t, 8 * MX_CAST_PAD_MANY_FIELDS> table;
+  int64_t n = 0;
+  add_cast(table, n, x, xr, xc);
+  add_cast(table, n, w1, w1r, w1c);
+  add_cast(table, n, w3, w3r, w3c);
+  add_cast(table, n, w2, w2r, w2c);
+  checked(lib.cast_pad_many(n, table.data(), mode, st), "mx_cast_pad_many");
+  const Tensor h13 = at::empty({2, M, H}, x.options());
+  char* const h1 = static_cast<char*>(h13.data_ptr());
+  char* const h3 = h1 + 2 * M * H;
+  if (persistent_shape(M, H)) {
+    checked(lib.shared_a(xr.codes(), xr.scales(), w1r.codes(), w1r.scales(), w3r.codes(), w3r.scales(), h1, h3, M, H, xr.k,
+                         xr.ld, H, st),
+            "mx_gemm_nt_shared_a_ld");
+  } else {
+    gemm_into(xr, w1r, h13[0], st);
+    gemm_into(xr, w3r, h13[1], st);
+  }
+  const Operand gr = make(M, H, pad, x), gc = make(H, M, pad, x);
+  checked(lib.swiglu(h1, h3, M, H, H, H, gr.codes(), gr.ld, gr.scales(), gc.codes(), gc.ld, gc.scales(), mode, st),
+          "mx_swiglu_cast_pad");
+  const Tensor y = gemm(gr, w2r, x, st);
+  return py::make_tuple(y, h13, xr.buf, xr.layout(), w2c.buf, w2c.layout(), xc.buf, xc.layout(), gc.buf, gc.layout(),
+                        w1c.buf, w1c.layout(), w3c.buf, w3c.layout());
+}
+
+// (dx, dW1, dW2, dW3), bf16, from dy and what ffn_forward returned
+py::object ffn_backward(const Tensor& dy, const Tensor& h13, const Tensor& w2_buf, const Tensor& x_buf, const Tensor& g_buf,
+                        const Tensor& w1_buf, const Tensor& w3_buf, int64_t D, int mode, int64_t pad) {
+  if (!plain(dy) || !on_current_device(dy) || h13.dim() != 3 || !h13.is_contiguous()) return py::none();
+  const int64_t M = dy.size(0), O = dy.size(1), H = h13.size(2);
+  hipStream_t st = stream_of(dy);
+  const Operand r = make(M, O, pad, dy), c = make(O, M, pad, dy);
+  checked(lib.cast_pad(dy.data_ptr(), dy.scalar_type() == at::kFloat, M, O, dy.stride(0), r.codes(), r.ld, r.scales(),
+                       c.codes(), c.ld, c.scales(), mode, st),
+          "mx_cast_pad");
+  const Tensor dg = gemm(r, around(w2_buf, H, O, pad), dy, st);
+  const auto [ra, rb] = make_pair(M, H, pad, dy);
+  const auto [ca, cb] = make_pair(H, M, pad, dy);
+  const char* h1 = static_cast<const char*>(h13.data_ptr());
+  checked(lib.swiglu_bwd(dg.data_ptr(), h1, h1 + 2 * M * H, M, H, H, H, H, ra.codes(), ra.ld, ra.scales(), ca.codes(),
+                         ca.ld, ca.scales(), mode, st),
+          "mx_swiglu_bwd_cast_pad");
+  const Operand x = around(x_buf, D, M, pad), w1 = around(w1_buf, D, H, pad), w3 = around(w3_buf, D, H, pad);
+  const Tensor dw13 = at::empty({2, H, D}, h13.options());
+  if (persistent_shape(H, D)) {
+    char* out = static_cast<char*>(dw13.data_ptr());
+    checked(lib.shared_b(ca.codes(), ca.scales(), cb.codes(), cb.scales(), x.codes(), x.scales(), out, out + 2 * H * D, H, D,
+                         x.k, x.ld, D, st),
+            "mx_gemm_nt_shared_b_ld");
+  } else {
+    gemm_into(ca, x, dw13[0], st);
+    gemm_into(cb, x, dw13[1], st);
+  }
+  const Tensor dw2 = gemm(c, around(g_buf, H, M, pad), dy, st);
+  Tensor dx;
+  if (persistent_shape(M, D)) {
+    dx = at::empty({M, D}, h13.options());
+    checked(lib.pair(ra.codes(), ra.scales(), w1.codes(), w1.scales(), rb.codes(), rb.scales(), w3.codes(), w3.scales(),
+                     dx.data_ptr(), M, D, ra.k, ra.ld, D, st),
+            "mx_gemm_nt_pair_ld");
+  } else {
+    dx = gemm(ra, w1, dy, st) + gemm(rb, w3, dy, st);
+  }
+  return py::make_tuple(dx, dw13.select(0, 0), dw2, dw13.select(0, 1));
+}
+
+// ---- the routed experts --------------------------------------------------------------------------
+// Dense codes [rows, cols] (or a stack of them) and their scales in MFMA order, rows and cols whole 128s but for
+// `rows` of an activation (ops.MXData).
+struct Codes {
+  Tensor codes, scales;
+  const uint8_t* c() const { return codes.data_ptr<uint8_t>(); }
+  const uint8_t* s() const { return scales.data_ptr<uint8_t>(); }
+  uint8_t* c() { return codes.data_ptr<uint8_t>(); }
+  uint8_t* s() { return scales.data_ptr<uint8_t>(); }
+};
+Codes make_codes(int64_t rows, int64_t cols, const Tensor& like) {
+  const auto bytes = like.options().dtype(at::kByte);
+  return {at::empty({rows, cols}, bytes), at::empty({up128(rows) * ((cols / 32 + 1) / 2 * 2)}, bytes)};
+}
+Codes make_stack(int64_t G, int64_t rows, int64_t cols, const Tensor& like) {
+  const auto bytes = like.options().dtype(at::kByte);
+  return {at::empty({G, rows, cols}, bytes), at::empty({G * rows * (cols / 32)}, bytes)};
+}
+void add_stack(std::array<int64_t, 8 * MX_CAST_PAD_MANY_FIELDS>& table, int64_t& n, const Tensor& w, Codes& r, Codes& c) {
+  const int64_t entry[MX_CAST_PAD_MANY_FIELDS] = {
+      reinterpret_cast<int64_t>(w.data_ptr()), w.scalar_type() == at::kFloat, w.size(0), w.size(1), w.size(2), w.size(2),
+      reinterpret_cast<int64_t>(r.c()), w.size(2), reinterpret_cast<int64_t>(r.s()),
+      reinterpret_cast<int64_t>(c.c()), w.size(1), reinterpret_cast<int64_t>(c.s())};
+  std::copy(entry, entry + MX_CAST_PAD_MANY_FIELDS, table.begin() + MX_CAST_PAD_MANY_FIELDS * n++);
+}
+bool plain_stack(const Tensor& w, int64_t G, int64_t rows, int64_t cols, const Tensor& x) {
+  return w.dim() == 3 && w.size(0) == G && w.size(1) == rows && w.size(2) == cols && w.is_contiguous() &&
+         (w.scalar_type() == at::kBFloat16 || w.scalar_type() == at::kFloat) && w.device() == x.device() &&
+         reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0;
+}
+bool plain_list(const Tensor& t, at::ScalarType type, const Tensor& x) {
+  return t.scalar_type() == type && t.is_contiguous() && t.device() == x.device();
+}
+
+// (out, the slots of mx_blocks.ROUTED_SAVED) on x [T, D] for all gradients, from the router's choices; hidden and
+// model size whole 128s.
+py::object routed_forward(const Tensor& x, const Tensor& scores, const Tensor& w1, const Tensor& w3, const Tensor& w2,
+                          const Tensor& selected, const Tensor& block_counts, const Tensor& counts, int64_t alignment,
+                          int64_t multiple, int mode, bool score_before) {
+  if (!plain(x) || x.scalar_type() != at::kBFloat16 || !on_current_device(x) || w1.dim() != 3) return py::none();
+  const int64_t T = x.size(0), D = x.size(1), G = w1.size(0), H = w1.size(1);
+  if (D % 128 || H % 128 || !plain_stack(w1, G, H, D, x) || !plain_stack(w3, G, H, D, x) || !plain_stack(w2, G, D, H, x) ||
+      scores.dim() != 2 || scores.size(0) != T || !plain_list(scores, at::kFloat, x) || !plain_list(selected, at::kLong, x) ||
+      selected.sizes() != scores.sizes() || !plain_list(block_counts, at::kInt, x) || !plain_list(counts, at::kLong, x) ||
+      counts.numel() != G || block_counts.numel() < (T + 15) / 16 * G || alignment % 32 || multiple % 128 || multiple % alignment)
+    return py::none();
+  const int64_t k = scores.size(1);
+  const int64_t R = (T * k + alignment * G + multiple - 1) / multiple * multiple;
+  hipStream_t st = stream_of(x);
+  const Tensor offs = at::empty({G}, x.options().dtype(at::kInt)), src_row = at::empty({R}, x.options().dtype(at::kLong)),
+               row_score = at::empty({R}, x.options().dtype(at::kFloat)),
+               pos = at::empty({T, k}, x.options().dtype(at::kLong));
+  const int32_t* ends = offs.data_ptr<int32_t>();
+  checked(lib.route_fill(selected.data_ptr<int64_t>(), scores.data_ptr<float>(), T, k, G, block_counts.data_ptr<int32_t>(),
+                         counts.data_ptr<int64_t>(), R, alignment, offs.data_ptr<int32_t>(), src_row.data_ptr<int64_t>(),
+                         row_score.data_ptr<float>(), pos.data_ptr<int64_t>(), st),
+          "mx_route_fill");
+  Codes xr = make_codes(R, D, x), xc = make_codes(D, R, x);
+  checked(lib.rows_gathered(x.data_ptr(), src_row.data_ptr<int64_t>(), score_before ? row_score.data_ptr<float>() : nullptr, T,
+                            R, D, x.stride(0), xr.c(), xr.s(), xc.c(), xc.s(), mode, MX_SCALES_MFMA, st),
+          "mx_cast_rows_gathered");
+  Codes w1r = make_stack(G, H, D, x), w1c = make_stack(G, D, H, x), w3r = make_stack(G, H, D, x), w3c = make_stack(G, D, H, x),
+        w2r = make_stack(G, D, H, x), w2c = make_stack(G, H, D, x);
+  std::array<int64_t, 8 * MX_CAST_PAD_MANY_FIELDS> table;
+  int64_t n = 0;
+  add_stack(table, n, w1, w1r, w1c);
+  add_stack(table, n, w3, w3r, w3c);
+  add_stack(table, n, w2, w2r, w2c);
+  checked(lib.cast_pad_many(n, table.data(), mode, st), "mx_cast_pad_many");
+  const Tensor h13 = at::empty({2, R, H}, x.options());
+  char* const h1 = static_cast<char*>(h13.data_ptr());
+  char* const h3 = h1 + 2 * R * H;
+  checked(lib.grouped_shared_a(xr.c(), xr.s(), w1r.c(), w1r.s(), w3r.c(), w3r.s(), ends, h1, h3, R, H, D, G, H, st),
+          "mx_grouped_gemm_2d3d_shared_a");
+  Codes gr = make_codes(R, H, x), gc = make_codes(H, R, x);
+  checked(lib.swiglu_dense(h1, h3, R, H, H, H, gr.c(), H, gr.s(), gc.c(), R, gc.s(), nullptr, mode, MX_SCALES_MFMA, st),
+          "mx_swiglu_cast_dim0_dim1_ld");
+  const Tensor yp = at::empty({R, D}, x.options()), out = at::empty({T, D}, x.options());
+  checked(lib.grouped(gr.c(), gr.s(), w2r.c(), w2r.s(), ends, yp.data_ptr(), R, D, H, G, D, MX_SCALES_MFMA, st),
+          "mx_grouped_gemm_2d3d");
+  checked(lib.combine(yp.data_ptr(), nullptr, R, D, pos.data_ptr<int64_t>(), score_before ? nullptr : scores.data_ptr<float>(),
+                      T, k, D, out.data_ptr(), D, st),
+          "mx_moe_combine");
+  return py::make_tuple(out, py::make_tuple(offs, src_row, row_score, pos, scores, h13, w2c.codes, w2c.scales, xc.codes,
+                                            xc.scales, gc.codes, gc.scales, w1c.codes, w1c.scales, w3c.codes, w3c.scales,
+                                            score_before ? x : yp));
+}
+
+// (dx, d scores, dW1, dW2, dW3) from dout [T, D] and those slots; at most 16 choices a token
+py::object routed_backward(const Tensor& dout, const std::vector<Tensor>& saved, int mode, bool score_before) {
+  const Tensor &offs = saved[0], &src_row = saved[1], &row_score = saved[2], &pos = saved[3], &scores = saved[4],
+               &h13 = saved[5];
+  if (!plain(dout) || dout.scalar_type() != at::kBFloat16 || !dout.is_contiguous() || !on_current_device(dout))
+    return py::none();
+  for (const Tensor& t : saved)
+    if (!t.is_contiguous() || t.device() != dout.device()) return py::none();
+  const int64_t T = dout.size(0), D = dout.size(1), G = offs.numel(), R = h13.size(1), H = h13.size(2), k = pos.size(1);
+  hipStream_t st = stream_of(dout);
+  const int32_t* ends = offs.data_ptr<int32_t>();
+  const int64_t* place = pos.data_ptr<int64_t>();
+  Codes w2{saved[6], saved[7]}, xc{saved[8], saved[9]}, gc{saved[10], saved[11]}, w1{saved[12], saved[13]},
+      w3{saved[14], saved[15]};
+  Codes dr = make_codes(R, D, dout), dc = make_codes(D, R, dout);
+  checked(lib.rows_gathered(dout.data_ptr(), src_row.data_ptr<int64_t>(), score_before ? nullptr : row_score.data_ptr<float>(),
+                            T, R, D, D, dr.c(), dr.s(), dc.c(), dc.s(), mode, MX_SCALES_MFMA, st),
+          "mx_cast_rows_gathered");
+  const Tensor dg = at::empty({R, H}, dout.options());
+  checked(lib.grouped(dr.c(), dr.s(), w2.c(), w2.s(), ends, dg.data_ptr(), R, H, D, G, H, MX_SCALES_MFMA, st),
+          "mx_grouped_gemm_2d3d");
+  // both gradients of the gate, stacked: d(h1) and then d(h3)
+  const auto bytes = dout.options().dtype(at::kByte);
+  const int64_t per_r = up128(R) * (H / 32), per_c = H * (R / 32);
+  const Tensor rows = at::empty({2, R, H}, bytes), cols = at::empty({2, H, R}, bytes), rows_s = at::empty({2 * per_r}, bytes),
+               cols_s = at::empty({2 * per_c}, bytes);
+  uint8_t *r = rows.data_ptr<uint8_t>(), *c = cols.data_ptr<uint8_t>(), *rs = rows_s.data_ptr<uint8_t>(),
+          *cs = cols_s.data_ptr<uint8_t>();
+  const char* h1 = static_cast<const char*>(h13.data_ptr());
+  checked(lib.swiglu_bwd_dense(dg.data_ptr(), h1, h1 + 2 * R * H, R, H, H, H, H, r, H, rs, c, R, cs, nullptr, mode,
+                               MX_SCALES_MFMA, st),
+          "mx_swiglu_bwd_cast_dim0_dim1_ld");
+  const Tensor dw13 = at::empty({2, G, H, D}, dout.options()), dw2 = at::empty({G, D, H}, dout.options());
+  char* dw1 = static_cast<char*>(dw13.data_ptr());
+  checked(lib.grouped_wgrad_two(c, cs, c + H * R, cs + per_c, xc.c(), xc.s(), ends, dw1, dw1 + 2 * G * H * D, R, H, D, G, st),
+          "mx_grouped_gemm_2d2d_shared_b");
+  checked(lib.grouped_wgrad(dc.c(), dc.s(), gc.c(), gc.s(), ends, dw2.data_ptr(), R, D, H, G, MX_SCALES_MFMA, st),
+          "mx_grouped_gemm_2d2d");
+  const Tensor dxp = at::empty({R, D}, dout.options());
+  checked(lib.grouped_pair(r, rs, w1.c(), w1.s(), r + R * H, rs + per_r, w3.c(), w3.s(), ends, dxp.data_ptr(), R, D, H, G, D,
+                           st),
+          "mx_grouped_gemm_2d3d_pair");
+  const Tensor dx = at::empty({T, D}, dout.options()), ds = at::empty({T, k}, scores.options());
+  if (score_before) {
+    checked(lib.combine_dot(dxp.data_ptr(), R, D, place, scores.data_ptr<float>(), saved[16].data_ptr(), D, T, k, D,
+                            dx.data_ptr(), D, ds.data_ptr<float>(), st),
+            "mx_moe_combine_dot");
+  } else {
+    checked(lib.combine_dot(saved[16].data_ptr(), R, D, place, nullptr, dout.data_ptr(), D, T, k, D, nullptr, 0,
+                            ds.data_ptr<float>(), st),
+            "mx_moe_combine_dot");
+    checked(lib.combine(dxp.data_ptr(), nullptr, R, D, place, nullptr, T, k, D, dx.data_ptr(), D, st), "mx_moe_combine");
+  }
+  return py::make_tuple(dx, ds, dw13.select(0, 0), dw2, dw13.select(0, 1));
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_blocks, m) {
+  m.def("bind", &bind);
+  m.def("linear_forward", &linear_forward);
+  m.def("linear_backward", &linear_backward);
+  m.def("linear_apply", &linear_apply);
+  m.def("routed_forward", &routed_forward);
+  m.def("routed_backward", &routed_backward);
+  m.def("ffn_forward", &ffn_forward);
+  m.def("ffn_backward", &ffn_backward);
+}

@@ -10,10 +10,10 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 
-from . import ops
-from .mx_tensor import (MXFP8Config, MXFP8TrainingWeight, _cast_activation, _cast_activation_and_weights,
-                        _cast_cache, _cast_into_groups, _cast_weight, _cast_weights, _castable,
-                        _grouped_2d3d_padded, _pad_plan, _unwrap)
+from . import _lib, ops
+from .mx_tensor import (MXFP8Config, MXFP8TrainingWeight, _cast_activation, _cast_activation_and_weights, _cast_cache,
+                        _cast_into_groups, _cast_weight, _cast_weights, _castable, _grouped_2d3d_padded, _one_launch,
+                        _pad_plan, _unwrap)
 from .ops import MX_SCALES_MFMA, MX_SCALES_ROWMAJOR, MXData
 
 # ----------------------------------------------------------------------------- SwiGLU + linear
@@ -223,11 +223,23 @@ class _MXFeedForward(torch.autograd.Function):
     def forward(ctx, x, w1, w2, w3, cfg: MXFP8Config, norm_weight=None, eps: float = 0.0):
         need_dx = ctx.needs_input_grad[0] or ctx.needs_input_grad[5]
         need_dw = any(ctx.needs_input_grad[1:4])
-        ctx.pad = block_pitch_pad(cfg, need_dx, need_dw)
-        y, saved = ffn_forward(_rows_of(x), x, w1, w2, w3, cfg, need_dx, need_dw, norm_weight, eps, pad=ctx.pad,
-                               whole_blocks=True)
+        ctx.pad = pad = block_pitch_pad(cfg, need_dx, need_dw)
         ctx.cfg, ctx.x_shape = cfg, x.shape
         ctx.w_dtypes = (w1.dtype, w2.dtype, w3.dtype)
+        ctx.native = False
+        if pad and norm_weight is None and all(ctx.needs_input_grad[:4]):
+            x2, key = _rows_of(x), (cfg.scale_mode, pad)
+            if (ops.native_block_ok(x2, x2.shape[1], w1.shape[0], w2.shape[0]) and _one_launch((w1, w3, w2), cfg)
+                    and _cast_cache.get(x, key) is None):
+                out = _lib.blocks().ffn_forward(x2, _castable(w1), _castable(w3), _castable(w2), ops._mode(cfg.scale_mode), pad)
+                if out is not None:
+                    y, h13, xr, xr_layout, *rest = out
+                    _cast_cache.put(x, key, (ops.Operand(xr, xr_layout), ops.Operand(rest[2], rest[3])))
+                    ctx.native, ctx.layouts = True, [None, *rest[1::2], None, None, None]
+                    ctx.save_for_backward(h13, *rest[::2], None, None, None)
+                    return y if x.dim() == 2 else y.view(*x.shape[:-1], w2.shape[0])
+        y, saved = ffn_forward(_rows_of(x), x, w1, w2, w3, cfg, need_dx, need_dw, norm_weight, eps, pad=ctx.pad,
+                               whole_blocks=True)
         ctx.layouts = [q.layout if isinstance(q, ops.Operand) else None for q in saved.values()]
         ctx.save_for_backward(*[q.buf if isinstance(q, ops.Operand) else q for q in saved.values()])
         return y if x.dim() == 2 else y.view(*x.shape[:-1], w2.shape[0])
@@ -236,10 +248,18 @@ class _MXFeedForward(torch.autograd.Function):
     def backward(ctx, dy):
         _cast_cache.clear()  # the forward that shared x's cast with a sibling is over
         need = ctx.needs_input_grad
-        saved = {name: (t if layout is None else ops.Operand(t, layout))
-                 for name, t, layout in zip(FFN_SAVED, ctx.saved_tensors, ctx.layouts)}
-        dx, dw1, dw2, dw3, dnw = ffn_backward(_castable(_rows_of(dy)), saved, ctx.cfg, need[0], need[1], need[2], need[3],
-                                              need[5], pad=ctx.pad, whole_blocks=True)
+        dy2, tensors, out = _castable(_rows_of(dy)), ctx.saved_tensors, None
+        if ctx.native and ops.native_block_ok(dy2, dy2.shape[1]):
+            h13, w2_buf, x_buf, g_buf, w1_buf, w3_buf = tensors[:6]
+            out = _lib.blocks().ffn_backward(dy2, h13, w2_buf, x_buf, g_buf, w1_buf, w3_buf, ctx.x_shape[-1],
+                                             ops._mode(ctx.cfg.scale_mode), ctx.pad)
+        if out is not None:
+            (dx, dw1, dw2, dw3), dnw = out, None
+        else:
+            saved = {name: (t if layout is None else ops.Operand(t, layout))
+                     for name, t, layout in zip(FFN_SAVED, tensors, ctx.layouts)}
+            dx, dw1, dw2, dw3, dnw = ffn_backward(dy2, saved, ctx.cfg, need[0], need[1], need[2], need[3],
+                                                  need[5], pad=ctx.pad, whole_blocks=True)
         cast_back = lambda g, dt: g if g is None or g.dtype == dt else g.to(dt)
         if dx is not None and len(ctx.x_shape) != 2:
             dx = dx.view(ctx.x_shape)
@@ -639,19 +659,32 @@ class _MXRoutedExperts(torch.autograd.Function):
     def forward(ctx, x, top_scores, w1, w2, w3, tok_sorted, counts, score_before: bool, cfg: MXFP8Config, choices=None):
         need_dx, need_ds = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         need_dw = any(ctx.needs_input_grad[2:5])
+        ctx.cfg, ctx.score_before = cfg, score_before
+        ctx.dtypes = (x.dtype, top_scores.dtype, w1.dtype, w2.dtype, w3.dtype)
+        ctx.order, multiple, fast = grouped_layout(x.shape[1], w1.shape[1], w1.shape[0])
+        ctx.native = False
+        if (fast and choices is not None and all(ctx.needs_input_grad[:5]) and top_scores.shape[1] <= ops.MOE_DOT_MAX_TOP_K
+                and ops.native_block_ok(x, x.shape[1], w1.shape[1]) and _one_launch((w1, w3, w2), cfg)):
+            done = _lib.blocks().routed_forward(
+                _bf16(x).contiguous(), top_scores.float().contiguous(), _castable(w1), _castable(w3), _castable(w2),
+                choices[0], choices[1], counts, ops.BLOCK, multiple, ops._mode(cfg.scale_mode), score_before)
+            if done is not None:
+                ctx.native = True
+                ctx.save_for_backward(*done[1])
+                return done[0]
         out, saved = routed_forward(_bf16(x).contiguous(), top_scores, w1, w2, w3, tok_sorted, counts, score_before,
                                     cfg, need_dx, need_ds, need_dw, choices)
-        ctx.cfg, ctx.score_before = cfg, score_before
-        ctx.order = grouped_layout(x.shape[1], w1.shape[1], w1.shape[0])[0]
-        ctx.dtypes = (x.dtype, top_scores.dtype, w1.dtype, w2.dtype, w3.dtype)
         ctx.save_for_backward(*saved)
         return out
 
     @staticmethod
     def backward(ctx, dout):
         need = ctx.needs_input_grad
-        grads = routed_backward(_bf16(dout).contiguous(), list(ctx.saved_tensors), ctx.cfg, ctx.order,
-                                ctx.score_before, need[0], need[1], need[2], need[3], need[4])
+        grads, saved, dout = None, list(ctx.saved_tensors), _bf16(dout).contiguous()
+        if ctx.native and ops.native_block_ok(dout, dout.shape[1]):
+            grads = _lib.blocks().routed_backward(dout, saved, ops._mode(ctx.cfg.scale_mode), ctx.score_before)
+        if grads is None:
+            grads = routed_backward(dout, saved, ctx.cfg, ctx.order, ctx.score_before, *need[:5])
         dx, ds, dw1, dw2, dw3 = (g if g is None or g.dtype == dt else g.to(dt) for g, dt in zip(grads, ctx.dtypes))
         return dx, ds, dw1, dw2, dw3, None, None, None, None, None
 

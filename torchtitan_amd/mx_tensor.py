@@ -21,7 +21,7 @@ import weakref
 import torch
 import torch.nn.functional as F
 
-from . import ops
+from . import _lib, ops
 from .ops import MX_SCALES_MFMA, MX_SCALES_ROWMAJOR, MXData
 
 
@@ -259,10 +259,29 @@ def _linear_forward(x, weight, cfg: MXFP8Config, need_dx: bool, need_dw: bool):
     # rows further apart than they are long, except with cached weight casts, which the fused
     # blocks and the hand-over share without a pitch
     pad = 0 if cfg.cache_weight_casts else ops.CODE_PITCH_PAD
+    if not (need_dx or need_dw) and ops.native_block_ok(x2, K, N):
+        wq0, _ = _cast_weight(weight, mode, False, cfg, pitch_pad=pad)
+        M = x2.shape[0]  # (few rows are cast inside their product, which no sibling shares)
+        few = M <= ops.FEW_ROWS and N <= ops.FEW_ROWS_COLUMNS and (M + 15 & ~15) * K <= ops.FEW_ROWS_VALUES
+        if type(wq0) is ops.Operand and (few or _cast_cache.get(x, (mode, pad)) is None):
+            out = _lib.blocks().linear_apply(x2, wq0.buf, wq0.scales_buf, wq0.layout, ops._mode(mode), ops.FEW_ROWS,
+                                             ops.FEW_ROWS_VALUES, ops.FEW_ROWS_COLUMNS)
+            if out is not None:
+                y, xr, xr_layout = out
+                if xr is not None:
+                    _cast_cache.put(x, (mode, pad), (ops.Operand(xr, xr_layout), None))
+                return (y if x.dim() == 2 else y.view(*x.shape[:-1], N)), None, None
     if not (need_dx or need_dw) and ops.few_rows_ok(x2, N):
         wq0, _ = _cast_weight(weight, mode, False, cfg, pitch_pad=pad)
         y = ops.mx_few_rows(x2, wq0, mode)
         return (y if x.dim() == 2 else y.view(*x.shape[:-1], N)), None, None
+    if need_dx and need_dw and pad and ops.native_block_ok(x2, K, N) and _cast_cache.get(x, (mode, pad)) is None:
+        out = _lib.blocks().linear_forward(x2, _castable(weight), ops._mode(mode), pad)
+        if out is not None:
+            y, xr, xr_layout, xc, xc_layout, wc, wc_layout = out
+            xq1 = ops.Operand(xc, xc_layout)
+            _cast_cache.put(x, (mode, pad), (ops.Operand(xr, xr_layout), xq1))
+            return (y if x.dim() == 2 else y.view(*x.shape[:-1], N)), xq1, ops.Operand(wc, wc_layout)
     (xq0, xq1), (wq0, wq1) = _cast_activation_and_weights(x2, x, (weight,), mode, need_dx, need_dw, cfg, pad)
     y = ops.mx_gemm_nt(xq0, wq0)
     return (y if x.dim() == 2 else y.view(*x.shape[:-1], N)), xq1, wq1
@@ -289,8 +308,17 @@ class _MXLinear(torch.autograd.Function):
         x_buf, w_buf = ctx.saved_tensors
         dy2 = _castable(dy if dy.dim() == 2 else dy.reshape(-1, dy.shape[-1]))
         pad = 0 if ctx.cfg.cache_weight_casts else ops.CODE_PITCH_PAD
-        dyq0, dyq1 = ops.to_operands(dy2, mode, need_dx, need_dw, pad)
         dx = dw = None
+        if need_dx and need_dw and pad and ops.native_block_ok(dy2, dy2.shape[1], ctx.x_shape[-1]):
+            # (operands as both casts of x and W lay them out with this pitch)
+            out = _lib.blocks().linear_backward(dy2, x_buf, w_buf, ctx.x_shape[-1], ops._mode(mode), pad,
+                                                ctx.x_dtype == torch.float32, ctx.w_dtype == torch.float32)
+            if out is not None:
+                dx, dw = out
+                dx = dx if len(ctx.x_shape) == 2 else dx.view(ctx.x_shape)
+                return (dx if dx.dtype == ctx.x_dtype else dx.to(ctx.x_dtype),
+                        dw if dw.dtype == ctx.w_dtype else dw.to(ctx.w_dtype), None)
+        dyq0, dyq1 = ops.to_operands(dy2, mode, need_dx, need_dw, pad)
         if need_dx:
             dx = ops.mx_gemm_nt_as(dyq0, ops.Operand(w_buf, ctx.w_layout), ctx.x_dtype)
             if len(ctx.x_shape) != 2:

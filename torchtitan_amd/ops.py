@@ -1102,6 +1102,14 @@ def _transformed() -> bool:
     return torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0
 
 
+def native_block_ok(x: torch.Tensor, *widths: int) -> bool:
+    """A block on x may run its launches from one native call (`_lib.blocks`): a plain tensor, nobody who would
+    want to see the single steps (a dispatch mode, a function transform, a kernel timer), and no side narrower
+    than a tile of the GEMMs, where other kernels and other combinations of launches run."""
+    return (type(x) is torch.Tensor and x.is_cuda and min(widths) > 128 and _timer is None and not _watched()
+            and not _transformed())
+
+
 def op_sac_save_list() -> set:
     """The dispatcher ops of this package whose outputs a per-op activation-checkpoint policy may
     save (the forward GEMMs): add them to the model's save list

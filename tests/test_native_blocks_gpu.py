@@ -207,3 +207,25 @@ def test_capture_and_threads(device):
         t.join()
     for i in range(2):
         _same(got[i], want)
+
+
+def test_errors_keep_their_types(device, monkeypatch):
+    """Memory that runs out is torch's error on either path; a status of the library is the package's."""
+    lin = _holder(Linear.Config().build(in_features=4096, out_features=4096), device)
+    x = torch.randn(8192, 4096, device=device, dtype=torch.bfloat16, requires_grad=True)
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(device).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(device) + (1 << 20)) / total, device)
+    try:
+        for native in (True, False):
+            with monkeypatch.context() as m:
+                if not native:
+                    m.setattr(ops, "native_block_ok", lambda *a: False)
+                with pytest.raises(torch.OutOfMemoryError):
+                    lin(x)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, device)
+    blocks, w = _lib.blocks(), lin.weight.detach().as_subclass(torch.Tensor)
+    with pytest.raises(_lib.MXLibraryError, match="mx_cast_pad_many"):
+        blocks.linear_forward(x.detach(), w, 7, 128)  # no such scale mode
+    assert torch.isfinite(lin(x)).all()

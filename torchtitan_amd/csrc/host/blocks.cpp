@@ -450,13 +450,14 @@ py::object routed_backward(const Tensor& dout, const std::vector<Tensor>& saved,
 
 }  // namespace
 
+// (errors of torch keep their types: an allocation that fails is a torch.OutOfMemoryError)
 PYBIND11_MODULE(_blocks, m) {
   m.def("bind", &bind);
-  m.def("linear_forward", &linear_forward);
-  m.def("linear_backward", &linear_backward);
-  m.def("linear_apply", &linear_apply);
-  m.def("routed_forward", &routed_forward);
-  m.def("routed_backward", &routed_backward);
-  m.def("ffn_forward", &ffn_forward);
-  m.def("ffn_backward", &ffn_backward);
+  m.def("linear_forward", torch::wrap_pybind_function(linear_forward));
+  m.def("linear_backward", torch::wrap_pybind_function(linear_backward));
+  m.def("linear_apply", torch::wrap_pybind_function(linear_apply));
+  m.def("ffn_forward", torch::wrap_pybind_function(ffn_forward));
+  m.def("ffn_backward", torch::wrap_pybind_function(ffn_backward));
+  m.def("routed_forward", torch::wrap_pybind_function(routed_forward));
+  m.def("routed_backward", torch::wrap_pybind_function(routed_backward));
 }

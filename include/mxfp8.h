@@ -455,6 +455,14 @@ int mx_gemm_nt_pair_ld(const uint8_t* a_codes, const uint8_t* a_scales, const ui
                        const uint8_t* b_scales, const uint8_t* a2_codes, const uint8_t* a2_scales,
                        const uint8_t* b2_codes, const uint8_t* b2_scales, void* d, int64_t M,
                        int64_t N, int64_t K, int64_t ldk, int64_t ldd, void* stream);
+/* mx_gemm_nt_pair_ld for a caller that lends scratch memory, as mx_gemm_nt_ws is to mx_gemm_nt: few output tiles
+ * and a long contraction (the input gradient of a SwiGLU block over some hundred tokens) run in slices of K, half
+ * of them from either product, float32 partial sums in `workspace`, summed in order and rounded once. */
+int64_t mx_gemm_nt_pair_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int mx_gemm_nt_pair_ws(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes, const uint8_t* b_scales,
+                       const uint8_t* a2_codes, const uint8_t* a2_scales, const uint8_t* b2_codes, const uint8_t* b2_scales,
+                       void* d, int64_t M, int64_t N, int64_t K, int64_t ldk, int64_t ldd, void* workspace,
+                       int64_t workspace_bytes, void* stream);
 int mx_gemm_nt_shared_a_ld(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                            const uint8_t* b_scales, const uint8_t* b2_codes, const uint8_t* b2_scales,
                            void* d, void* d2, int64_t M, int64_t N, int64_t K, int64_t ldk,

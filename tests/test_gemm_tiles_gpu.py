@@ -1,6 +1,6 @@
-"""The smaller tiles of the persistent GEMM (192 and 128 rows or columns) and their splits along K: at the
-edges of tiles, 128-row scale groups and 128-deep blocks, and their float32 results, against the products of the same codes in float64 and
-against 256 x 256 tiles, whose sums every unsplit tile forms in the same order."""
+"""The smaller tiles of the persistent GEMM (192 and 128 rows or columns), their splits along K and their float32
+results: at the edges of tiles, 128-row scale groups and 128-deep blocks, against the products of the same codes in
+float64 and against 256 x 256 tiles, whose sums every unsplit tile forms in the same order."""
 import numpy as np
 import pytest
 import torch
@@ -99,6 +99,36 @@ def test_splits_along_k(device, hooks, M, N, K, tile, slices):
         assert torch.equal(_float32(a, b, N, ws), out.float())
 
 
+@pytest.mark.parametrize("slices", [2, 6])
+@pytest.mark.parametrize("tile", [(4, 4), (2, 4), (4, 2)])
+@pytest.mark.parametrize("M,N,K", [(129, 136, 2176), (200, 392, 4224), (513, 264, 1664)])
+def test_splits_of_a_sum_of_two_products(device, hooks, M, N, K, tile, slices):
+    rng = np.random.default_rng(M + slices)
+    (a, ha), (a2, ha2) = _operand(device, rng, M, K), _operand(device, rng, M, K, 0.3)
+    (b, hb), (b2, hb2) = _operand(device, rng, N, K, 0.02), _operand(device, rng, N, K, 0.05)
+    hooks.mx_debug_set_tile(*tile, slices)
+    need = int(hooks.mx_gemm_nt_pair_workspace_bytes(M, N, K))
+    assert need == slices * M * N * 4
+    ws = torch.full((need,), 0xFF, dtype=torch.uint8, device=device)  # (NaN)
+
+    def run(lent):
+        out = torch.full((M, N + 24), 7.0, dtype=torch.bfloat16, device=device)
+        ops._call("mx_gemm_nt_pair_ws", "gemm_nt_pair", device, a.codes_ptr, a.scales_ptr, b.codes_ptr, b.scales_ptr,
+                  a2.codes_ptr, a2.scales_ptr, b2.codes_ptr, b2.scales_ptr, out.data_ptr(), M, N, K, a.ld, N + 24,
+                  ws.data_ptr(), lent, ops._stream(out))
+        assert bool((out[:, N:] == 7.0).all())
+        return out[:, :N]
+
+    for grid in (0, 8):
+        hooks.mx_debug_set_grid(grid)
+        _check(run(need), ha @ hb.T + ha2 @ hb2.T)
+    hooks.mx_debug_set_tile(0, 0, 0)
+    hooks.mx_debug_set_grid(0)
+    ws.fill_(0xFF)
+    _check(run(0), ha @ hb.T + ha2 @ hb2.T)  # too little memory lent: one chain, nothing written there
+    assert bool((ws == 0xFF).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(65, 136, 128), (256, 1024, 256), (300, 264, 1024)])
 def test_float32_results_of_short_contractions(device, M, N, K):
     """(these run on the kernel of one 128 x 128 tile per workgroup)"""
@@ -124,3 +154,10 @@ def test_shapes_that_are_split(device, hooks):
             for N in (1024, 4096, 6144):
                 for K in (1024, 4096, 16384, 147456):
                     assert need(M, N, K) <= 64 << 20 or -(-M // 256) * -(-N // 256) > 128
+        pair = lambda M, N, K: int(hooks.mx_gemm_nt_pair_workspace_bytes(M, N, K))
+        assert pair(256, 4096, 14336) == 8 * 256 * 4096 * 4 and pair(128, 4096, 14336) == pair(300, 1000, 14300) == 0
+        assert pair(256, 4096, 2048) == pair(4096, 2048, 6144) == pair(16384, 4096, 14336) == 0
+        for M in (129, 200, 1000, 2048, 5003):
+            for N in (1024, 4096, 6144):
+                for K in (2176, 6144, 14336, 147456):
+                    assert pair(M, N, K) <= 64 << 20 and pair(M, N, K) % (2 * M * N * 4) == 0

@@ -32,6 +32,8 @@ struct Library {
   decltype(&mx_gemm_nt_shared_a_ld) shared_a = nullptr;
   decltype(&mx_gemm_nt_shared_b_ld) shared_b = nullptr;
   decltype(&mx_gemm_nt_pair_ld) pair = nullptr;
+  decltype(&mx_gemm_nt_pair_workspace_bytes) pair_workspace_bytes = nullptr;
+  decltype(&mx_gemm_nt_pair_ws) pair_split = nullptr;
   decltype(&mx_few_rows) few_rows = nullptr;
   decltype(&mx_route_fill) route_fill = nullptr;
   decltype(&mx_cast_rows_gathered) rows_gathered = nullptr;
@@ -61,6 +63,8 @@ void bind(const py::dict& addresses, const py::object& check) {
   set("mx_gemm_nt_shared_a_ld", lib.shared_a);
   set("mx_gemm_nt_shared_b_ld", lib.shared_b);
   set("mx_gemm_nt_pair_ld", lib.pair);
+  set("mx_gemm_nt_pair_workspace_bytes", lib.pair_workspace_bytes);
+  set("mx_gemm_nt_pair_ws", lib.pair_split);
   set("mx_few_rows", lib.few_rows);
   set("mx_route_fill", lib.route_fill);
   set("mx_cast_rows_gathered", lib.rows_gathered);
@@ -295,9 +299,16 @@ py::object ffn_backward(const Tensor& dy, const Tensor& h13, const Tensor& w2_bu
   Tensor dx;
   if (persistent_shape(M, D)) {
     dx = at::empty({M, D}, h13.options());
-    checked(lib.pair(ra.codes(), ra.scales(), w1.codes(), w1.scales(), rb.codes(), rb.scales(), w3.codes(), w3.scales(),
-                     dx.data_ptr(), M, D, ra.k, ra.ld, D, st),
-            "mx_gemm_nt_pair_ld");
+    if (const int64_t need = lib.pair_workspace_bytes(M, D, ra.k)) {
+      const Tensor ws = at::empty({need}, ra.buf.options());
+      checked(lib.pair_split(ra.codes(), ra.scales(), w1.codes(), w1.scales(), rb.codes(), rb.scales(), w3.codes(),
+                             w3.scales(), dx.data_ptr(), M, D, ra.k, ra.ld, D, ws.data_ptr(), need, st),
+              "mx_gemm_nt_pair_ws");
+    } else {
+      checked(lib.pair(ra.codes(), ra.scales(), w1.codes(), w1.scales(), rb.codes(), rb.scales(), w3.codes(), w3.scales(),
+                       dx.data_ptr(), M, D, ra.k, ra.ld, D, st),
+              "mx_gemm_nt_pair_ld");
+    }
   } else {
     dx = gemm(ra, w1, dy, st) + gemm(rb, w3, dy, st);
   }

@@ -147,6 +147,12 @@ int launch_gemm_nt32_pair(const uint8_t* a_codes, const uint8_t* a_scales, const
                           const uint8_t* b_scales, const uint8_t* a2_codes, const uint8_t* a2_scales,
                           const uint8_t* b2_codes, const uint8_t* b2_scales, void* d, int64_t M,
                           int64_t N, int64_t K, int64_t ldk, int64_t ldd, hipStream_t st);
+GemmPlan plan_pair(int64_t M, int64_t N, int64_t K);
+int launch_gemm_nt32_pair_splitk(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
+                                 const uint8_t* b_scales, const uint8_t* a2_codes, const uint8_t* a2_scales,
+                                 const uint8_t* b2_codes, const uint8_t* b2_scales, void* d, int64_t M, int64_t N,
+                                 int64_t K, int64_t ldk, int64_t ldd, const GemmPlan& plan, void* workspace,
+                                 hipStream_t st);
 }
 
 // The forms over two operand sets exist for the persistent kernel only, dense rows (ldk == K) or
@@ -165,6 +171,29 @@ extern "C" int mx_gemm_nt_pair_ld(const uint8_t* a_codes, const uint8_t* a_scale
     return MX_ERR_UNSUPPORTED;
   return launch_gemm_nt32_pair(a_codes, a_scales, b_codes, b_scales, a2_codes, a2_scales, b2_codes,
                                b2_scales, d, M, N, K, ldk, ldd, (hipStream_t)stream);
+}
+
+extern "C" int64_t mx_gemm_nt_pair_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+  if (M <= 128 || N <= 128 || K <= 0 || N % 8 || (uint64_t)N * 1024 > 0x7FFFFFFFull) return 0;
+  const GemmPlan plan = plan_pair(M, N, K);
+  return plan.slices > 1 ? (int64_t)plan.slices * M * N * 4 : 0;
+}
+
+extern "C" int mx_gemm_nt_pair_ws(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
+                                  const uint8_t* b_scales, const uint8_t* a2_codes, const uint8_t* a2_scales,
+                                  const uint8_t* b2_codes, const uint8_t* b2_scales, void* d, int64_t M, int64_t N,
+                                  int64_t K, int64_t ldk, int64_t ldd, void* workspace, int64_t workspace_bytes,
+                                  void* stream) {
+  int rc = check_dense(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldd);
+  if (rc == MX_OK) rc = check_dense(a2_codes, a2_scales, b2_codes, b2_scales, d, M, N, K, ldd);
+  if (rc != MX_OK || M == 0 || N == 0) return rc;
+  if (ldk < K) return MX_ERR_INVALID_ARG;
+  const int64_t need = force_kernel == 0 && persistent_ok(d, N, K, ldd, ldk) ? mx_gemm_nt_pair_workspace_bytes(M, N, K) : 0;
+  if (need == 0 || !workspace || workspace_bytes < need || ((uintptr_t)workspace & 15))
+    return mx_gemm_nt_pair_ld(a_codes, a_scales, b_codes, b_scales, a2_codes, a2_scales, b2_codes, b2_scales, d, M, N, K,
+                              ldk, ldd, stream);
+  return launch_gemm_nt32_pair_splitk(a_codes, a_scales, b_codes, b_scales, a2_codes, a2_scales, b2_codes, b2_scales, d, M, N,
+                                      K, ldk, ldd, plan_pair(M, N, K), workspace, (hipStream_t)stream);
 }
 
 extern "C" int mx_gemm_nt_pair(const uint8_t* a_codes, const uint8_t* a_scales,

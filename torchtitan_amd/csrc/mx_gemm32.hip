@@ -102,6 +102,8 @@ struct Gemm32Args {
   // as far as A has rows behind its last group.  nullptr: D has A's rows.
   const int32_t* d_offs = nullptr;
   int64_t d_rows = 0;
+  // kSplitK: 2 = the sum of two products (a2 .. b2 as for PAIR), each cut into G / 2 slices
+  int32_t sets = 1;
 };
 enum Gemm32Two { kTwoNone = 0, kTwoB = 1, kTwoA = 2 };
 
@@ -534,12 +536,19 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
       r.nblocks = g < G ? K / kKB : 1;
       r.empty = g >= G;
     } else if (MODE == kSplitK) {
-      // slice g of the K blocks: ceil(blocks / G) each, the host picks G so that none is empty
+      // slice g of the K blocks: ceil(blocks / slices) each, the host picks the number so that none is empty
       const uint32_t per_g = tiles_m * tiles_n;
       const uint32_t g = t / per_g;
       tile_coords(t - g * per_g, tiles_m, tiles_n, tm, tn);
-      const uint32_t blocks = K / kKB, per = (blocks + G - 1) / G;
-      const uint32_t b_lo = g * per, b_hi = b_lo + per < blocks ? b_lo + per : blocks;
+      const uint32_t slices = G / (uint32_t)p.sets, slice = g % slices;
+      if (g >= slices) {
+        a_codes = p.a2_codes;
+        a_scales = p.a2_scales;
+        b_codes = p.b2_codes;
+        b_scales = p.b2_scales;
+      }
+      const uint32_t blocks = K / kKB, per = (blocks + slices - 1) / slices;
+      const uint32_t b_lo = slice * per, b_hi = b_lo + per < blocks ? b_lo + per : blocks;
       const uint32_t lo = b_lo * kKB;
       r.a = a_codes + (int64_t)tm * kEA * Kt + lo;
       r.b = b_codes + (int64_t)tn * kEB * Kt + lo;
@@ -1444,6 +1453,34 @@ GemmPlan plan_dense(int64_t M, int64_t N, int64_t K, bool may_split) {
   return best;
 }
 
+// What the sum of two products over K each runs on: one chain over both (slices == 1), or `slices` slices of
+// which half belong to either, under the conditions above.  One chain of 2 K / 128 blocks per tile bounds few
+// rows: 256 x 4096, K 2 x 14336 takes 189 us so (16 tiles on 256 CUs), 53 in eight slices; 512 rows 189 and 74 in four;
+// 1024 rows 191 and 121 in two; 512 x 2048, K 2 x 6144 57 and 27 in six; 4096 rows 80 and 94 in two: not split.
+GemmPlan plan_pair(int64_t M, int64_t N, int64_t K) {
+  const int64_t grid = persistent_grid(), blocks = K / kKB;
+  GemmPlan best{0, 0, 1};
+  if (grid == 0 || K % kKB || (2 * blocks <= 32 && !debug_slices)) return best;
+  const DenseTile* t = best_tile(M, N, 2 * blocks, 1, grid);
+  if (!t) return best;
+  const double plain_us = tiles_us(*t, tile_count(*t, M, N), 2 * blocks, grid) + 2.0;
+  double best_us = plain_us;
+  for (const DenseTile& u : kDenseTiles) {
+    if (u.ta * u.tb == 12 || (debug_tile && debug_tile != u.ta * 16 + u.tb)) continue;
+    for (int s = 1; s <= 4; ++s) {
+      const int64_t per = (blocks + s - 1) / s;
+      const double bytes = 8.0 * s * M * N;
+      if (per < 4 || (s - 1) * per >= blocks || bytes > (double)(64 << 20) || (debug_slices && 2 * s != debug_slices)) continue;
+      const double us = tiles_us(u, tile_count(u, M, N) * 2 * s, per, grid) + 2.0 + 4.2 + bytes / 3.2e6;
+      if ((us < best_us && us <= 0.92 * plain_us) || debug_slices) {
+        best = {u.ta, u.tb, 2 * s};
+        best_us = us;
+      }
+    }
+  }
+  return best;
+}
+
 // Launches the persistent dense kernel on `p` with tiles of 64 ta x 64 tb.
 template <int MODE, bool PAIR, bool OUT32, int TA, int TB>
 static int launch_tile(Gemm32Args p, hipStream_t st) {
@@ -1659,6 +1696,21 @@ int launch_gemm_nt32_pair(const uint8_t* a_codes, const uint8_t* a_scales, const
                a2_codes, a2_scales, b2_codes, b2_scales};
   p.ldk = ldk;
   return launch_best32<true>(p, st);
+}
+
+// ... in the slices of `plan`, through `workspace` (slices * M * N floats).
+int launch_gemm_nt32_pair_splitk(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
+                                 const uint8_t* b_scales, const uint8_t* a2_codes, const uint8_t* a2_scales,
+                                 const uint8_t* b2_codes, const uint8_t* b2_scales, void* d, int64_t M, int64_t N,
+                                 int64_t K, int64_t ldk, int64_t ldd, const GemmPlan& plan, void* workspace,
+                                 hipStream_t st) {
+  Gemm32Args p{a_codes, a_scales, b_codes, b_scales, (uint16_t*)workspace, M, N, K, N, nullptr, plan.slices, 0, 0, nullptr,
+               a2_codes, a2_scales, b2_codes, b2_scales};
+  p.ldk = ldk;
+  p.sets = 2;
+  const int rc = launch_dense32<kSplitK>(p, plan.ta, plan.tb, st);
+  if (rc != MX_OK) return rc;
+  return launch_splitk_reduce((const float*)workspace, plan.slices, M, N, d, ldd, false, st);
 }
 
 int launch_grouped32_2d3d_pair(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,

@@ -919,7 +919,7 @@ def _as_mfma(d: MXData) -> torch.Tensor:
     return d.scales if d.scale_order == MX_SCALES_MFMA else scale_layout(d.scales)
 
 
-_gemm_workspace: dict = {}  # (device index, M, N, K) -> bytes the library would split with
+_gemm_workspace: dict = {}  # (device index, M, N, K, query) -> bytes the library would split with
 
 
 def _common_pitch(*codes, multiple: int = 128):
@@ -934,14 +934,14 @@ def _common_pitch(*codes, multiple: int = 128):
     return codes, pitch
 
 
-def _split_workspace(device, M: int, N: int, K: int):
+def _split_workspace(device, M: int, N: int, K: int, query: str = "mx_gemm_nt_workspace_bytes"):
     """Float32 partial sums for the shapes whose contraction the library splits (few output tiles, long
     contraction), else None."""
-    key = (device.index, M, N, K)
+    key = (device.index, M, N, K, query)
     need = _gemm_workspace.get(key)
     if need is None:
         with torch.cuda.device(device):
-            need = _gemm_workspace[key] = int(_lib.load().mx_gemm_nt_workspace_bytes(M, N, K))
+            need = _gemm_workspace[key] = int(getattr(_lib.load(), query)(M, N, K))
     return torch.empty(need, dtype=torch.uint8, device=device) if need else None
 
 
@@ -1143,7 +1143,8 @@ def mx_gemm_nt(a: MXData, b: MXData, out: torch.Tensor | None = None) -> torch.T
 def mx_gemm_nt_pair(a: MXData, b: MXData, a2: MXData, b2: MXData) -> torch.Tensor:
     """bf16 deq(a) @ deq(b)^T + deq(a2) @ deq(b2)^T: one GEMM whose output tiles accumulate both
     products before they are rounded and written, where the persistent kernel takes the shape;
-    otherwise two GEMMs and a bf16 add."""
+    otherwise two GEMMs and a bf16 add.  Few tiles and a long contraction run in slices of K, as
+    in `mx_gemm_nt`."""
     if _operands(a, b, a2, b2):
         M, N, K = a.rows, b.rows, a.k
         if a2.rows != M or b2.rows != N or not a.depth == b.depth == a2.depth == b2.depth:
@@ -1151,8 +1152,8 @@ def mx_gemm_nt_pair(a: MXData, b: MXData, a2: MXData, b2: MXData) -> torch.Tenso
         if not _persistent_shape(M, N, K):
             return mx_gemm_nt(a, b) + mx_gemm_nt(a2, b2)
         out = torch.empty((M, N), dtype=torch.bfloat16, device=a.buf.device)
-        _call("mx_gemm_nt_pair_ld", "gemm_nt_pair", out.device, a.codes_ptr, a.scales_ptr, b.codes_ptr, b.scales_ptr,
-              a2.codes_ptr, a2.scales_ptr, b2.codes_ptr, b2.scales_ptr, out.data_ptr(), M, N, K, a.ld, N, _stream(out))
+        _call_pair((a.codes_ptr, a.scales_ptr, b.codes_ptr, b.scales_ptr, a2.codes_ptr, a2.scales_ptr, b2.codes_ptr,
+                    b2.scales_ptr), M, N, K, a.ld, out)
         return out
     M, K = a.codes.shape
     N = b.codes.shape[0]
@@ -1164,9 +1165,17 @@ def mx_gemm_nt_pair(a: MXData, b: MXData, a2: MXData, b2: MXData) -> torch.Tenso
     out = torch.empty((M, N), dtype=torch.bfloat16, device=a.codes.device)
     sa, sb, sa2, sb2 = _as_mfma(a), _as_mfma(b), _as_mfma(a2), _as_mfma(b2)  # kept alive over the launch
     (ac, bc, a2c, b2c), ldk = _common_pitch(a.codes, b.codes, a2.codes, b2.codes)
-    _call("mx_gemm_nt_pair_ld", "gemm_nt_pair", out.device, _ptr(ac), _ptr(sa), _ptr(bc), _ptr(sb),
-          _ptr(a2c), _ptr(sa2), _ptr(b2c), _ptr(sb2), _ptr(out), M, N, K, ldk, N, _stream(out))
+    _call_pair((_ptr(ac), _ptr(sa), _ptr(bc), _ptr(sb), _ptr(a2c), _ptr(sa2), _ptr(b2c), _ptr(sb2)), M, N, K, ldk, out)
     return out
+
+
+def _call_pair(args, M: int, N: int, K: int, ldk: int, out: torch.Tensor) -> None:
+    ws = _split_workspace(out.device, M, N, K, "mx_gemm_nt_pair_workspace_bytes")
+    if ws is None:
+        _call("mx_gemm_nt_pair_ld", "gemm_nt_pair", out.device, *args, out.data_ptr(), M, N, K, ldk, N, _stream(out))
+    else:
+        _call("mx_gemm_nt_pair_ws", "gemm_nt_pair", out.device, *args, out.data_ptr(), M, N, K, ldk, N, ws.data_ptr(),
+              ws.numel(), _stream(out))
 
 
 def _persistent_shape(M: int, N: int, K: int) -> bool:

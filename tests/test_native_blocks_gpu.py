@@ -216,6 +216,13 @@ def test_errors_keep_their_types(device, monkeypatch):
     torch.cuda.empty_cache()
     total = torch.cuda.get_device_properties(device).total_memory
     torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(device) + (1 << 20)) / total, device)
+    held = []  # what earlier tests left in the allocator's cache would serve the linear
+    for size in (1 << 30, 1 << 28, 1 << 26, 1 << 24, 1 << 22, 1 << 20):
+        try:
+            while len(held) < 10000:
+                held.append(torch.empty(size, dtype=torch.uint8, device=device))
+        except torch.OutOfMemoryError:
+            pass
     try:
         for native in (True, False):
             with monkeypatch.context() as m:
@@ -224,6 +231,7 @@ def test_errors_keep_their_types(device, monkeypatch):
                 with pytest.raises(torch.OutOfMemoryError):
                     lin(x)
     finally:
+        held.clear()
         torch.cuda.set_per_process_memory_fraction(1.0, device)
     blocks, w = _lib.blocks(), lin.weight.detach().as_subclass(torch.Tensor)
     with pytest.raises(_lib.MXLibraryError, match="mx_cast_pad_many"):

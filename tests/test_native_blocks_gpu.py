@@ -168,10 +168,8 @@ def test_routed_experts(device, monkeypatch, experts, top_k, shared, tokens, bef
         assert "routed_forward" in taken and "routed_backward" in taken
 
 
-def test_capture_and_threads(device):
-    """A captured step of native calls replays on new inputs; two threads on streams of their own."""
-    import threading
-
+def test_capture(device):
+    """A captured step of native calls replays on new inputs."""
     lin = _holder(Linear.Config().build(in_features=256, out_features=384), device)
     x = torch.randn(200, 256, device=device, dtype=torch.bfloat16, requires_grad=True)
     dy = torch.randn(200, 384, device=device, dtype=torch.bfloat16)
@@ -192,21 +190,81 @@ def test_capture_and_threads(device):
         torch.cuda.synchronize()
         _same(out, step())
 
-    want, got = [t.clone() for t in step()], {}
+
+def test_threads_on_streams_of_their_own(device):
+    """Two threads take the same linears over the same activation, which changes from pass to pass: each orders its
+    stream behind what wrote the activation and no more, so a cast taken over from the other's stream, or memory that it
+    gave back, would show.  Every pass of every thread is compared."""
+    import threading
+
+    a = _holder(Linear.Config().build(in_features=256, out_features=384), device)
+    b = _holder(Linear.Config().build(in_features=256, out_features=160), device)
+    passes, shape = 12, (1000, 256)
+    xs = [torch.randn(shape, device=device, dtype=torch.bfloat16) for _ in range(passes)]
+
+    def step(x):
+        x = x.detach().requires_grad_(True)
+        ya, yb = a(x), b(x)
+        return [ya.detach(), yb.detach(), *torch.autograd.grad((ya, yb), [x, a.weight, b.weight], (ya.detach(), yb.detach()))]
+
+    def forward(x):
+        with torch.no_grad():  # (nothing drops the remembered cast between the threads)
+            return [a(x), b(x)]
+
+    want = [[*step(x), *forward(x)] for x in xs]
+    x, got, failed = torch.empty(shape, device=device, dtype=torch.bfloat16), {}, []
+    written, barrier = torch.cuda.Event(), threading.Barrier(3, timeout=60)
 
     def work(i):
-        with torch.cuda.stream(torch.cuda.Stream()):
-            for _ in range(10):
-                got[i] = step()
-            torch.cuda.current_stream().synchronize()
-    torch.cuda.synchronize()
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                for n in range(passes):
+                    barrier.wait()  # x of this pass is on its way
+                    stream.wait_event(written)
+                    got[n, i] = [*step(x), *forward(x)]
+                    stream.synchronize()
+                    barrier.wait()
+        except Exception as ex:
+            failed.append(ex)
+            barrier.abort()
+
     threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
     for t in threads:
         t.start()
+    try:
+        for n in range(passes):
+            x.copy_(xs[n])
+            written.record()
+            barrier.wait()
+            barrier.wait()
+    except threading.BrokenBarrierError:
+        pass
     for t in threads:
         t.join()
-    for i in range(2):
-        _same(got[i], want)
+    assert not failed, failed
+    for n in range(passes):
+        for i in range(2):
+            _same(got[n, i], want[n])
+
+
+def test_remembered_cast_serves_its_own_stream(device):
+    """A linear on another stream than the one that cast its activation casts again; what was cast there is there."""
+    lin = _holder(Linear.Config().build(in_features=256, out_features=384), device)
+    x, side = torch.randn(200, 256, device=device, dtype=torch.bfloat16), torch.cuda.Stream()
+    key = ("rceil", ops.CODE_PITCH_PAD)
+    with torch.no_grad():
+        mx_tensor.clear_cast_cache()
+        want = lin(x)
+        assert mx_tensor._cast_cache.get(x, key) is not None
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            assert mx_tensor._cast_cache.get(x, key) is None
+            got = lin(x)
+            assert mx_tensor._cast_cache.get(x, key) is not None
+        assert mx_tensor._cast_cache.get(x, key) is None
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(got, want)
 
 
 def test_errors_keep_their_types(device, monkeypatch):

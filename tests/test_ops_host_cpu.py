@@ -182,3 +182,58 @@ def test_traced_block_has_the_shapes_that_its_fake_kernel_gives(no_launches, mon
     assert [t.shape for t in real] == [t.shape for t in fake] and [t.dtype for t in real] == [t.dtype for t in fake]
     storages = [t.untyped_storage().data_ptr() for t in real[1:15] if t.numel()]
     assert len(set(storages)) == len(storages)
+
+
+def test_remembered_activation_cast_stays_on_its_stream(no_launches, monkeypatch):
+    """A sibling on the stream that cast the activation takes the codes; one on another stream, whose work is not
+    ordered behind that launch, or on the other side of a graph capture casts again."""
+    from torchtitan_amd import mx_tensor
+
+    place = (0x10, False)
+    monkeypatch.setattr(mx_tensor, "_place", lambda t: place, raising=False)
+    x = _bf16(200, 256)
+    cast = lambda: mx_tensor._cast_activation(x, x, "rceil", True)
+    first = cast()
+    assert cast() is first
+    for place in ((0x20, False), (0x20, True), (0x10, True)):
+        again = cast()
+        assert again is not first and cast() is again
+        first = again
+    x.add_(1)
+    assert cast() is not first
+
+
+def test_remembered_activation_cast_is_read_and_dropped_as_a_whole(no_launches):
+    """Threads that remember, look up and drop entries: a lookup gives the cast of its own tensor or nothing."""
+    import sys
+    import threading
+
+    from torchtitan_amd import mx_tensor
+
+    cache, wrong = mx_tensor._ActivationCastCache(), []
+
+    def work(i):
+        xs = [_bf16(1, 32) for _ in range(4)]
+        try:
+            for n in range(20000):
+                x = xs[n % 4]
+                cache.put(x, i, (i, n % 4))
+                got = cache.get(x, i)
+                if got not in (None, (i, n % 4)):
+                    wrong.append(got)
+                if n % 3 == 0:
+                    cache.clear()
+        except Exception as ex:  # (a thread's own exception would pass unnoticed)
+            wrong.append(ex)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(1e-6)  # between any two steps of a lookup
+    try:
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        sys.setswitchinterval(interval)
+    assert not wrong

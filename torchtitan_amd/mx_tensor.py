@@ -48,49 +48,53 @@ class MXFP8Config:
 
 
 # ----------------------------------------------------------------------------- cast reuse
+def _place(x: torch.Tensor):
+    """Where work on x goes now: the current stream of its GPU, and whether that is being captured."""
+    if not x.is_cuda:
+        return None
+    return ops._stream(x), torch.cuda.is_current_stream_capturing()
+
+
 class _ActivationCastCache:
     """Remembers the fused cast of the last activation tensor.
 
     w1(x) and w3(x) of a SwiGLU block, or wq/wk/wv of attention, receive the same tensor object;
     the second and third linear reuse the codes instead of re-reading x.  The entry is keyed on
-    object identity, the tensor's version counter and its address, and holds only a weak
-    reference to the activation.
+    object identity, the tensor's version counter and its address, on the stream that the cast was
+    launched on, and holds only a weak reference to the activation.
 
     What keeps a hit from being stale: an entry lives for one forward at most.  It is dropped at
-    the start of every backward of a converted linear, whenever the stream's graph-capture state
-    changes (an entry made by an eager warm-up is never reused under capture, so the cast is
-    always recorded into the graph, and an entry made under capture is never reused by eager
-    code), and by `clear_cast_cache()`.  Writes through this package's `out=` arguments bump the
-    destination's version counter.  A caller that overwrites an activation behind autograd's back
-    (`.data`, a foreign kernel) between two forwards without a backward in between must call
-    `clear_cast_cache()`.
+    the start of every backward of a converted linear and by `clear_cast_cache()`, and serves
+    neither another stream, whose work is not ordered behind the cast and which the codes' memory
+    does not belong to, nor the other state of graph capture (an entry made by an eager warm-up is
+    never reused under capture, so the cast is always recorded into the graph, and an entry made
+    under capture is never reused by eager code).  Writes through this package's `out=` arguments
+    bump the destination's version counter.  A caller that overwrites an activation behind
+    autograd's back (`.data`, a foreign kernel) between two forwards without a backward in between
+    must call `clear_cast_cache()`.
+
+    There is one entry for all threads, replaced and dropped as a whole: two threads cost each other
+    their hits, and autograd's own threads drop the forward's entry.
     """
 
     def __init__(self):
-        self._ref = None
-        self._key = None
-        self._value = None
-        self._capturing = False
+        self._entry = None  # (weak reference to the activation, key, cast)
 
-    def _sync_capture_state(self, x: torch.Tensor):
-        capturing = x.is_cuda and torch.cuda.is_current_stream_capturing()
-        if capturing != self._capturing:
-            self.clear()
-            self._capturing = capturing
+    @staticmethod
+    def _key(x: torch.Tensor, mode):
+        return x._version, mode, x.data_ptr(), _place(x)
 
     def get(self, x: torch.Tensor, mode):
-        self._sync_capture_state(x)
-        if self._ref is not None and self._ref() is x and self._key == (x._version, mode, x.data_ptr()):
-            return self._value
+        entry = self._entry
+        if entry is not None and entry[0]() is x and entry[1] == self._key(x, mode):
+            return entry[2]
         return None
 
     def put(self, x: torch.Tensor, mode, value):
-        self._ref = weakref.ref(x)
-        self._key = (x._version, mode, x.data_ptr())
-        self._value = value
+        self._entry = weakref.ref(x), self._key(x, mode), value
 
     def clear(self):
-        self._ref = self._key = self._value = None
+        self._entry = None
 
 
 _cast_cache = _ActivationCastCache()

@@ -129,3 +129,36 @@ def test_single_linear_captured_after_a_warm_up_on_the_same_static_input(device)
                 assert torch.equal(y, want), rep
                 # eager calls on the same static tensor between replays see its new contents too
                 assert torch.equal(holder.proj(x), want)
+
+
+def test_two_graphs_captured_on_the_same_static_input(device):
+    """Linears on one static input in a graph of their own each, captured one after the other: each graph casts the
+    input itself, so either replays alone on what the input holds then."""
+    torch.manual_seed(43)
+    holder = nn.Module()
+    holder.a = Linear.Config().build(in_features=256, out_features=384)
+    holder.b = Linear.Config().build(in_features=256, out_features=160)
+    holder.to(device).to(torch.bfloat16)
+    for lin in (holder.a, holder.b):
+        lin.init_weights(init_std=0.05)
+    _convert(holder, ["a", "b"])
+    inputs = [torch.randn(4, 64, 256, device=device, dtype=torch.bfloat16) for _ in range(3)]
+    x = torch.zeros_like(inputs[0])
+    with torch.no_grad():
+        eager = [(holder.a(xi), holder.b(xi)) for xi in inputs]
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            holder.a(x), holder.b(x)
+        torch.cuda.current_stream().wait_stream(side)
+        graphs, outs = [torch.cuda.CUDAGraph() for _ in range(2)], []
+        for lin, graph in zip((holder.a, holder.b), graphs):
+            with torch.cuda.graph(graph):
+                outs.append(lin(x))
+        for rep in range(2):
+            for xi, want in zip(inputs, eager):
+                x.copy_(xi)
+                for i in (1, 0):
+                    graphs[i].replay()
+                    torch.cuda.synchronize()
+                    assert torch.equal(outs[i], want[i]), (rep, i)

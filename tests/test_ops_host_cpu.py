@@ -186,16 +186,16 @@ def test_traced_block_has_the_shapes_that_its_fake_kernel_gives(no_launches, mon
 
 def test_remembered_activation_cast_stays_on_its_stream(no_launches, monkeypatch):
     """A sibling on the stream that cast the activation takes the codes; one on another stream, whose work is not
-    ordered behind that launch, or on the other side of a graph capture casts again."""
+    ordered behind that launch, or in another graph capture casts again."""
     from torchtitan_amd import mx_tensor
 
-    place = (0x10, False)
+    place = (0x10, 0)
     monkeypatch.setattr(mx_tensor, "_place", lambda t: place, raising=False)
     x = _bf16(200, 256)
     cast = lambda: mx_tensor._cast_activation(x, x, "rceil", True)
     first = cast()
     assert cast() is first
-    for place in ((0x20, False), (0x20, True), (0x10, True)):
+    for place in ((0x20, 0), (0x20, 1), (0x20, 2), (0x10, 2), (0x10, 0)):
         again = cast()
         assert again is not first and cast() is again
         first = again

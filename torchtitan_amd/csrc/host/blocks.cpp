@@ -5,7 +5,7 @@
 // (3.3 us each) Python made operands, asked tensors for their pointers and strides and passed them on, 4 to 8 us
 // a step.  Here the same entry points of the library are called with the same arguments in the same order
 // (ops.py, mx_tensor.py and mx_blocks.py have them step by step); what is allocated is what is allocated there.
-// Nothing is kept between calls, no pointer outlives one.  Every function checks that its inputs are the plain
+// Nothing is kept between calls, no pointer outlives one.  Every block's function checks that its inputs are the plain
 // case -- bf16 or float32 matrices on the current GPU whose rows the casts read as they lie -- and returns None
 // otherwise: the caller then takes the general path.
 #include <c10/hip/HIPStream.h>
@@ -459,11 +459,21 @@ py::object routed_backward(const Tensor& dout, const std::vector<Tensor>& saved,
   return py::make_tuple(dx, ds, dw13.select(0, 0), dw2, dw13.select(0, 1));
 }
 
+// The capture that `stream` is part of, a number of its own for every capture (0: none).
+unsigned long long capture_id(uintptr_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  const hipError_t rc = hipStreamGetCaptureInfo(reinterpret_cast<hipStream_t>(stream), &status, &id);
+  TORCH_CHECK(rc == hipSuccess, "hipStreamGetCaptureInfo: ", hipGetErrorString(rc));
+  return status == hipStreamCaptureStatusNone ? 0 : id;
+}
+
 }  // namespace
 
 // (errors of torch keep their types: an allocation that fails is a torch.OutOfMemoryError)
 PYBIND11_MODULE(_blocks, m) {
   m.def("bind", &bind);
+  m.def("capture_id", torch::wrap_pybind_function(capture_id));
   m.def("linear_forward", torch::wrap_pybind_function(linear_forward));
   m.def("linear_backward", torch::wrap_pybind_function(linear_backward));
   m.def("linear_apply", torch::wrap_pybind_function(linear_apply));

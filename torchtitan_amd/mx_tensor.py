@@ -49,10 +49,11 @@ class MXFP8Config:
 
 # ----------------------------------------------------------------------------- cast reuse
 def _place(x: torch.Tensor):
-    """Where work on x goes now: the current stream of its GPU, and whether that is being captured."""
+    """Where work on x goes now: the current stream of its GPU, and the graph capture that it is part of (0: none)."""
     if not x.is_cuda:
         return None
-    return ops._stream(x), torch.cuda.is_current_stream_capturing()
+    stream = ops._stream(x)
+    return stream, _lib.blocks().capture_id(stream) if torch.cuda.is_current_stream_capturing() else 0
 
 
 class _ActivationCastCache:
@@ -66,9 +67,9 @@ class _ActivationCastCache:
     What keeps a hit from being stale: an entry lives for one forward at most.  It is dropped at
     the start of every backward of a converted linear and by `clear_cast_cache()`, and serves
     neither another stream, whose work is not ordered behind the cast and which the codes' memory
-    does not belong to, nor the other state of graph capture (an entry made by an eager warm-up is
-    never reused under capture, so the cast is always recorded into the graph, and an entry made
-    under capture is never reused by eager code).  Writes through this package's `out=` arguments
+    does not belong to, nor anything outside the graph capture that it was made in (an entry made by
+    an eager warm-up or in another capture is never reused under capture, so every graph records the
+    casts that it needs, and an entry made under capture is never reused by eager code).  Writes through this package's `out=` arguments
     bump the destination's version counter.  A caller that overwrites an activation behind
     autograd's back (`.data`, a foreign kernel) between two forwards without a backward in between
     must call `clear_cast_cache()`.

@@ -11,6 +11,7 @@ import pytest
 import torch
 import torch.nn as nn
 
+from tests.test_converter_gpu import _convert as _convert_with
 from torchtitan_amd.modules import FeedForward, Linear, MoE
 from torchtitan_amd.protocols import ModelConvertersContainer
 from torchtitan_amd.quantization.mx import MXFP8Converter
@@ -162,3 +163,34 @@ def test_two_graphs_captured_on_the_same_static_input(device):
                     graphs[i].replay()
                     torch.cuda.synchronize()
                     assert torch.equal(outs[i], want[i]), (rep, i)
+
+
+@pytest.mark.parametrize("first_user", ["eager", "graph"])
+def test_cached_weight_casts_of_a_capture_stay_in_it(device, first_user):
+    """With cached weight casts, a capture is the first to cast a weight: its codes exist only once the graph has run,
+    so eager calls before that and other graphs cast for themselves."""
+    torch.manual_seed(47)
+    holder = nn.Module()
+    holder.plain, holder.cached = (Linear.Config().build(in_features=256, out_features=384) for _ in range(2))
+    holder.to(device).to(torch.bfloat16)
+    holder.plain.init_weights(init_std=0.05)
+    x = torch.randn(200, 256, device=device, dtype=torch.bfloat16)
+    with torch.no_grad():
+        holder.cached.weight.copy_(holder.plain.weight)
+        _convert(holder, ["plain"])
+        _convert_with(holder, ["cached"], cache=True)
+        want = holder.plain(x)
+        graphs, outs = [torch.cuda.CUDAGraph() for _ in range(2)], []
+        for graph in graphs:
+            with torch.cuda.graph(graph):
+                outs.append(holder.cached(x))
+        if first_user == "eager":
+            assert torch.equal(holder.cached(x), want)
+        for rep in range(2):
+            for i in (1, 0):
+                graphs[i].replay()
+                torch.cuda.synchronize()
+                assert torch.equal(outs[i], want), (rep, i)
+                assert torch.equal(holder.cached(x), want), (rep, i)
+            x.normal_()
+            want = holder.plain(x)

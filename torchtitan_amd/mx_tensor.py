@@ -48,12 +48,16 @@ class MXFP8Config:
 
 
 # ----------------------------------------------------------------------------- cast reuse
+def _capture(x: torch.Tensor) -> int:
+    """The graph capture that work on x is part of now (0: none)."""
+    if not x.is_cuda or not torch.cuda.is_current_stream_capturing():
+        return 0
+    return _lib.blocks().capture_id(ops._stream(x))
+
+
 def _place(x: torch.Tensor):
-    """Where work on x goes now: the current stream of its GPU, and the graph capture that it is part of (0: none)."""
-    if not x.is_cuda:
-        return None
-    stream = ops._stream(x)
-    return stream, _lib.blocks().capture_id(stream) if torch.cuda.is_current_stream_capturing() else 0
+    """Where work on x goes now: the current stream of its GPU, and the graph capture that it is part of."""
+    return (ops._stream(x), _capture(x)) if x.is_cuda else None
 
 
 class _ActivationCastCache:
@@ -126,7 +130,8 @@ class _WeightCastCache:
     accumulation, several forwards per step, or a hand-over of the weights in MXFP8 form, the
     casts after the first are repeats.  An entry is keyed on the weight's memory (address, shape,
     strides) and valid while that storage is alive and its version counter is unchanged: every
-    in-place update (optimizer step, ``copy_``, init) invalidates it.  Off unless the converter
+    in-place update (optimizer step, ``copy_``, init) invalidates it.  A cast made under graph capture
+    exists once that graph has run: its entry serves that capture only.  Off unless the converter
     is built with ``cache_weight_casts=True``; holds 2 bytes per weight element."""
 
     def __init__(self):
@@ -140,8 +145,8 @@ class _WeightCastCache:
         e = self._entries.get(self._key(w, mode))
         if e is None:
             return None
-        ref, version, rows, cols = e
-        if ref.expired() or version != w._version:
+        ref, version, capture, rows, cols = e
+        if ref.expired() or version != w._version or (capture and capture != _capture(w)):
             return None
         return rows, cols
 
@@ -151,7 +156,7 @@ class _WeightCastCache:
         dead = [k for k, e in self._entries.items() if e[0].expired()]
         for k in dead:
             del self._entries[k]
-        self._entries[self._key(w, mode)] = (StorageWeakRef(w.untyped_storage()), w._version, rows, cols)
+        self._entries[self._key(w, mode)] = (StorageWeakRef(w.untyped_storage()), w._version, _capture(w), rows, cols)
 
     def clear(self):
         self._entries.clear()
@@ -197,7 +202,7 @@ def _cast_weight(w: torch.Tensor, mode: str, need_cols: bool, cfg: MXFP8Config, 
 def _in_form(w: torch.Tensor, key, hit, whole: bool):
     """A cached cast in the other form, which its caller wants: operands, or dense `MXData` (views of an operand's buffer).
     An operand made from a dense entry takes its place, except under graph capture, where it is filled
-    by the replay only."""
+    by the replay only and the entry may serve others."""
     rows, cols = hit
     if not whole:
         return rows.data(), (None if cols is None else cols.data())

@@ -267,6 +267,29 @@ def test_remembered_cast_serves_its_own_stream(device):
     assert torch.equal(got, want)
 
 
+def test_cached_weight_cast_on_another_stream(device):
+    """A cached weight cast that is still queued when another stream asks for it: that stream waits for it."""
+    plain = _holder(Linear.Config().build(in_features=2176, out_features=288), device)
+    lin = _holder(Linear.Config().build(in_features=2176, out_features=288), device, cache=True)
+    x, side = torch.randn(300, 2176, device=device, dtype=torch.bfloat16), torch.cuda.Stream()
+    with torch.no_grad():
+        for p, q in zip(lin.parameters(), plain.parameters()):
+            p.copy_(q)
+        want = plain(x)
+        torch.cuda.synchronize()
+        torch.cuda._sleep(100_000_000)  # some 50 ms in front of the cast
+        first = lin(x)
+        with torch.cuda.stream(side):
+            got = lin(x)
+            side.synchronize()
+        for p in lin.parameters():
+            p.mul_(1)  # (a new version: the entry is replaced)
+        again = lin(x)
+    torch.cuda.synchronize()
+    for y in (first, got, again):
+        assert torch.equal(y, want)
+
+
 def test_errors_keep_their_types(device, monkeypatch):
     """Memory that runs out is torch's error on either path; a status of the library is the package's."""
     lin = _holder(Linear.Config().build(in_features=4096, out_features=4096), device)

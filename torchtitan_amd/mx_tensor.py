@@ -123,6 +123,20 @@ def _cast_activation(x2: torch.Tensor, src: torch.Tensor, mode: str, need_cols: 
 
 
 # ----------------------------------------------------------------------------- weight casts
+def _follow(done: torch.cuda.Event, *casts) -> None:
+    """Orders the current stream behind `done`, an event behind the casts, and keeps their memory until the stream has
+    read them.  (Not under capture, which begins with the device idle and cannot wait for work outside it.)"""
+    if torch.cuda.is_current_stream_capturing():
+        return
+    for q in casts:
+        if q is None:
+            continue
+        for t in (q.buf, q.scales_buf) if type(q) is ops.Operand else (q.codes, q.scales):
+            here = torch.cuda.current_stream(t.device)
+            here.wait_event(done)
+            t.record_stream(here)
+
+
 class _WeightCastCache:
     """MXFP8 forms of weights that have not changed since they were cast.
 
@@ -131,7 +145,8 @@ class _WeightCastCache:
     casts after the first are repeats.  An entry is keyed on the weight's memory (address, shape,
     strides) and valid while that storage is alive and its version counter is unchanged: every
     in-place update (optimizer step, ``copy_``, init) invalidates it.  A cast made under graph capture
-    exists once that graph has run: its entry serves that capture only.  Off unless the converter
+    exists once that graph has run: its entry serves that capture only.  A hit on another stream than the
+    one that cast orders that stream behind the cast.  Off unless the converter
     is built with ``cache_weight_casts=True``; holds 2 bytes per weight element."""
 
     def __init__(self):
@@ -145,9 +160,11 @@ class _WeightCastCache:
         e = self._entries.get(self._key(w, mode))
         if e is None:
             return None
-        ref, version, capture, rows, cols = e
+        ref, version, capture, stream, done, rows, cols = e
         if ref.expired() or version != w._version or (capture and capture != _capture(w)):
             return None
+        if done is not None and stream != ops._stream(w):
+            _follow(done, rows, cols)
         return rows, cols
 
     def put(self, w: torch.Tensor, mode, rows: MXData, cols):
@@ -156,7 +173,10 @@ class _WeightCastCache:
         dead = [k for k, e in self._entries.items() if e[0].expired()]
         for k in dead:
             del self._entries[k]
-        self._entries[self._key(w, mode)] = (StorageWeakRef(w.untyped_storage()), w._version, _capture(w), rows, cols)
+        capture, stream, done = _capture(w), None, None
+        if w.is_cuda and not capture:
+            stream, done = ops._stream(w), torch.cuda.current_stream(w.device).record_event()
+        self._entries[self._key(w, mode)] = (StorageWeakRef(w.untyped_storage()), w._version, capture, stream, done, rows, cols)
 
     def clear(self):
         self._entries.clear()

@@ -66,14 +66,18 @@ def _holder(module, device, dtype=torch.bfloat16, **kw):
     return module
 
 
-FORMS = {
-    "plain": lambda t, w: torch.randn(t, w),
-    "rows of a wider matrix": lambda t, w: torch.randn(t, w + 64)[:, :w],
-    "rows that are not aligned": lambda t, w: torch.randn(t, w + 3)[:, 3:],
-    "columns first": lambda t, w: torch.randn(w, t).t(),
-    "one row for all": lambda t, w: torch.randn(1, w).expand(t, w),
-    "three dimensions": lambda t, w: torch.randn(1, t, w),
+FORMS = {  # from randn(*shape), which has the device and the type: a copy to either would lay the rows out anew
+    "plain": lambda randn, t, w: randn(t, w),
+    "rows of a wider matrix": lambda randn, t, w: randn(t, w + 64)[:, :w],
+    "rows that are not aligned": lambda randn, t, w: randn(t, w + 3)[:, 3:],
+    "columns first": lambda randn, t, w: randn(w, t).t(),
+    "one row for all": lambda randn, t, w: randn(1, w).expand(t, w),
+    "three dimensions": lambda randn, t, w: randn(1, t, w),
 }
+
+
+def _form(form, device, dtype, tokens, width):
+    return FORMS[form](lambda *shape: torch.randn(shape, device=device, dtype=dtype), tokens, width)
 
 
 @pytest.mark.parametrize("form", FORMS)
@@ -83,8 +87,7 @@ def test_linear(device, monkeypatch, form, tokens, inner, outer, params):
     torch.manual_seed(tokens + inner)
     dtype = getattr(torch, params)
     lin = _holder(Linear.Config().build(in_features=inner, out_features=outer), device, dtype)
-    make = lambda w, dt: FORMS[form](tokens, w).to(device).to(dt)
-    x, dy = make(inner, dtype), make(outer, torch.bfloat16)
+    x, dy = _form(form, device, dtype, tokens, inner), _form(form, device, torch.bfloat16, tokens, outer)
     run = lambda: _step(lin, [lin.weight], x, dy, autocast=params == "float32")
     native, general, taken = _both(monkeypatch, run)
     _same(native, general)
@@ -104,6 +107,23 @@ def test_linear_without_gradients(device, monkeypatch, tokens, cached):
         native, general, taken = _both(monkeypatch, lambda: [lin(x), lin(x)])
     _same(native, general)
     assert "linear_apply" in taken
+
+
+@pytest.mark.parametrize("tokens,dtype", [(16, torch.float32), (16, torch.bfloat16), (200, torch.bfloat16)])
+@pytest.mark.parametrize("form", ["plain", "rows that are not aligned"])
+def test_siblings_without_gradients(device, monkeypatch, tokens, dtype, form):
+    """Linears on one activation cast it once, but for the few bf16 rows that are cast inside their products, and their
+    weights once each."""
+    lins = [_holder(Linear.Config().build(in_features=256, out_features=n), device) for n in (384, 160, 160)]
+    x, weights = _form(form, device, dtype, tokens, 256), []
+    cast = mx_tensor._cast_weight
+    monkeypatch.setattr(mx_tensor, "_cast_weight", lambda w, *args, **kw: weights.append(w.shape[0]) or cast(w, *args, **kw))
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16, enabled=dtype == torch.float32):
+        native, general, taken = _both(monkeypatch, lambda: [lin(x) for lin in lins])
+    _same(native, general)
+    assert weights == 2 * [384, 160, 160]
+    few = tokens <= ops.FEW_ROWS and dtype == torch.bfloat16
+    assert taken == (["linear_apply"] * (3 if few else 1) if form == "plain" else [])
 
 
 def test_siblings_and_frozen_weights(device, monkeypatch):
@@ -136,7 +156,7 @@ def test_siblings_and_frozen_weights(device, monkeypatch):
 def test_feed_forward(device, monkeypatch, form, tokens, dim, hidden):
     torch.manual_seed(tokens)
     ff = _holder(FeedForward.Config(hidden_dim=hidden).build(dim=dim), device)
-    x, dy = (FORMS[form](tokens, dim).to(device).bfloat16() for _ in range(2))
+    x, dy = (_form(form, device, torch.bfloat16, tokens, dim) for _ in range(2))
     run = lambda: _step(ff, list(ff.parameters()), x, dy)
     native, general, taken = _both(monkeypatch, run)
     _same(native, general)

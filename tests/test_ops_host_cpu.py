@@ -237,3 +237,27 @@ def test_remembered_activation_cast_is_read_and_dropped_as_a_whole(no_launches):
     finally:
         sys.setswitchinterval(interval)
     assert not wrong
+
+
+@pytest.mark.parametrize("cached", [False, True])
+def test_a_forward_without_gradients_casts_each_operand_once(no_launches, monkeypatch, cached):
+    """... also where the native call hands its input back, and where a sibling linear has cast the activation."""
+    from torchtitan_amd import _lib, mx_tensor
+
+    class Blocks:
+        handed_back = 0
+
+        def linear_apply(self, *args):
+            self.handed_back += 1
+
+    blocks, casts = Blocks(), []
+    monkeypatch.setattr(_lib, "blocks", lambda: blocks)
+    monkeypatch.setattr(ops, "native_block_ok", lambda *args: True)
+    monkeypatch.setattr(ops, "_call", lambda name, tag, device, *args: casts.append((name, args[0])))
+    cfg = mx_tensor.MXFP8Config(cache_weight_casts=cached)
+    x, weights = _bf16(200, 256), [_bf16(384, 256), _bf16(160, 256)]
+    for w in weights:
+        mx_tensor._linear_forward(x, w, cfg, False, False)
+    casts = [pointer for name, pointer in casts if name == "mx_cast_pad" or name.startswith("mx_cast_dim")]
+    assert blocks.handed_back == 1  # (the second linear takes the activation's cast as it is)
+    assert sorted(casts) == sorted(t.data_ptr() for t in (x, *weights))

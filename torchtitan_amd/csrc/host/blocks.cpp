@@ -199,16 +199,16 @@ py::object linear_backward(const Tensor& dy, const Tensor& x_buf, const Tensor& 
 }
 
 // y = x W^T without gradients, W's row-wise operand given (its buffers and layout): (y, row-wise x or None).
-// `few_rows`, `few_values`, `few_columns`: up to where the product that casts x itself runs (ops.few_rows_ok).
+// `few`: by the product that casts x itself (ops.few_rows_ok).
 py::object linear_apply(const Tensor& x, const Tensor& w_buf, const Tensor& w_scales, const std::array<int64_t, 6>& layout,
-                        int mode, int64_t few_rows, int64_t few_values, int64_t few_columns) {
+                        int mode, bool few) {
   const auto [N, k, ld, at, scales_at, depth] = layout;
   if (!plain(x) || x.size(1) != depth || ld % 128 || w_buf.device() != x.device() || !on_current_device(x)) return py::none();
   const int64_t M = x.size(0), K = x.size(1);
   hipStream_t st = stream_of(x);
   const uint8_t* codes = w_buf.data_ptr<uint8_t>() + at;
   const uint8_t* scales = w_scales.data_ptr<uint8_t>() + scales_at;
-  if (x.scalar_type() == at::kBFloat16 && M <= few_rows && N <= few_columns && ((M + 15) & ~int64_t{15}) * K <= few_values) {
+  if (few) {
     const Tensor y = at::empty({M, N}, x.options());
     checked(lib.few_rows(x.data_ptr(), M, K, x.stride(0), codes, scales, nullptr, nullptr, N, ld, y.data_ptr(), nullptr, N,
                          mode, st),

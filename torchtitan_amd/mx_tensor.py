@@ -282,6 +282,26 @@ def _castable(t: torch.Tensor) -> torch.Tensor:
     return t if t.dtype in (torch.bfloat16, torch.float32) else t.to(torch.bfloat16)
 
 
+def _linear_apply(x2: torch.Tensor, src: torch.Tensor, weight: torch.Tensor, cfg: MXFP8Config, pad: int):
+    """x2 W^T without gradients.  The activation's cast is shared with sibling linears on `src`, but for few rows, which are
+    cast inside their product; the weight is cast once, whichever way the product runs."""
+    mode, (K, N) = cfg.scale_mode, (x2.shape[1], weight.shape[0])
+    few = ops.few_rows_ok(x2, N)
+    remembered = None if few else _cast_cache.get(src, (mode, pad))
+    wq0, _ = _cast_weight(weight, mode, False, cfg, pitch_pad=pad)
+    if remembered is None and type(wq0) is ops.Operand and ops.native_block_ok(x2, K, N):
+        out = _lib.blocks().linear_apply(x2, wq0.buf, wq0.scales_buf, wq0.layout, ops._mode(mode), few)
+        if out is not None:
+            y, xr, xr_layout = out
+            if xr is not None:
+                _cast_cache.put(src, (mode, pad), (ops.Operand(xr, xr_layout), None))
+            return y
+    if few:
+        return ops.mx_few_rows(x2, wq0, mode)
+    xq0, _ = _cast_activation(x2, src, mode, need_cols=False, pitch_pad=pad)
+    return ops.mx_gemm_nt(xq0, wq0)
+
+
 def _linear_forward(x, weight, cfg: MXFP8Config, need_dx: bool, need_dw: bool):
     """(y, column-wise x or None, column-wise W or None) of the converted linear."""
     mode, K, N = cfg.scale_mode, x.shape[-1], weight.shape[0]
@@ -289,21 +309,8 @@ def _linear_forward(x, weight, cfg: MXFP8Config, need_dx: bool, need_dw: bool):
     # rows further apart than they are long, except with cached weight casts, which the fused
     # blocks and the hand-over share without a pitch
     pad = 0 if cfg.cache_weight_casts else ops.CODE_PITCH_PAD
-    if not (need_dx or need_dw) and ops.native_block_ok(x2, K, N):
-        wq0, _ = _cast_weight(weight, mode, False, cfg, pitch_pad=pad)
-        M = x2.shape[0]  # (few rows are cast inside their product, which no sibling shares)
-        few = M <= ops.FEW_ROWS and N <= ops.FEW_ROWS_COLUMNS and (M + 15 & ~15) * K <= ops.FEW_ROWS_VALUES
-        if type(wq0) is ops.Operand and (few or _cast_cache.get(x, (mode, pad)) is None):
-            out = _lib.blocks().linear_apply(x2, wq0.buf, wq0.scales_buf, wq0.layout, ops._mode(mode), ops.FEW_ROWS,
-                                             ops.FEW_ROWS_VALUES, ops.FEW_ROWS_COLUMNS)
-            if out is not None:
-                y, xr, xr_layout = out
-                if xr is not None:
-                    _cast_cache.put(x, (mode, pad), (ops.Operand(xr, xr_layout), None))
-                return (y if x.dim() == 2 else y.view(*x.shape[:-1], N)), None, None
-    if not (need_dx or need_dw) and ops.few_rows_ok(x2, N):
-        wq0, _ = _cast_weight(weight, mode, False, cfg, pitch_pad=pad)
-        y = ops.mx_few_rows(x2, wq0, mode)
+    if not (need_dx or need_dw):
+        y = _linear_apply(x2, x, weight, cfg, pad)
         return (y if x.dim() == 2 else y.view(*x.shape[:-1], N)), None, None
     if need_dx and need_dw and pad and ops.native_block_ok(x2, K, N) and _cast_cache.get(x, (mode, pad)) is None:
         out = _lib.blocks().linear_forward(x2, _castable(weight), ops._mode(mode), pad)

@@ -75,3 +75,33 @@ def test_static_scratch_gemm_rejects_what_does_not_fit(device):
         assert st == 5 and b"scratch" in lib.mx_status_string(st)
     torch.cuda.synchronize(device)
     assert bool((out == 7.0).all()), "nothing was launched"
+
+
+# Splits of more than the array holds, before tiles that fill more than 5/7 of a round of the CUs were left unsplit:
+# 190, 195 and 204 of them.  Such shapes run; one of 130 tiles is refused.
+@pytest.mark.parametrize("M,N,K,taken", [(4864, 2560, 98304, True), (4864, 2560, 147456, True), (592, 16416, 147456, True),
+                                         (3072, 4352, 262144, True), (1280, 6656, 131072, False)])
+def test_static_scratch_gemm_of_long_contractions(device, M, N, K, taken):
+    lib = _lib.load()
+    lib.mx_debug_force_kernel(0)
+    lib.mx_debug_set_grid(0)
+    lib.mx_debug_set_tile(0, 0, 0)
+    with torch.cuda.device(device):
+        assert (int(lib.mx_gemm_nt_workspace_bytes(M, N, K)) <= 64 << 20) == taken
+    # e4m3 codes of either sign up to 1.875 (0x3F), all scales 1
+    g = torch.Generator(device).manual_seed(M)
+    a, b = (torch.randint(0, 64, (rows, K), dtype=torch.uint8, device=device, generator=g) for rows in (M, N))
+    a[:, ::2] |= 0x80
+    scales = lambda rows: torch.full((int(lib.mx_scales_mfma_bytes(rows, K // 32)),), 127, dtype=torch.uint8, device=device)
+    sa, sb = scales(M), scales(N)
+    want, got = (torch.full((M, N), 7.0, dtype=torch.bfloat16, device=device) for _ in range(2))
+    args = (ops._ptr(a), ops._ptr(sa), ops._ptr(b), ops._ptr(sb))
+    with torch.cuda.device(device):
+        st = lib.mx_gemm_nt_static(*args, ops._ptr(got), M, N, K, N, ops._stream(got))
+    assert st == (0 if taken else 5)
+    torch.cuda.synchronize(device)
+    if not taken:
+        assert bool((got == 7.0).all())
+        return
+    ops._call("mx_gemm_nt", "gemm_nt", device, *args, ops._ptr(want), M, N, K, N, ops._stream(want))
+    assert torch.equal(got, want)  # one chain of sums

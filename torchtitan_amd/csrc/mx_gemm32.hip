@@ -1413,8 +1413,11 @@ static const DenseTile* best_tile(int64_t M, int64_t N, int64_t blocks, int prod
 //   * S slices add float32 partial sums, written and read back (3.2 TB/s) by a launch of their own,
 //     and are taken for a predicted gain of 8 %: 256 x 4096, K 8192 40 us unsplit, 23 in four
 //     slices; 512 x 4096, K 14336 85 and 39; 2048 x 2048, K 147456 1270 and 430.  The partial sums stay under 64 MiB,
-//     one 256 x 256 tile per CU; more only for 256 x 256 tiles of a half to one and a half times the CUs
-//     (4352 x 4352, K 147456: 289 tiles, the second round all but empty).
+//     one 256 x 256 tile per CU; more only where 256 x 256 tiles leave a good part of their rounds empty: half to 5/7 of
+//     the CUs (1280 x 6656, K 131072: 130 tiles, 1050 us unsplit, 940 in five slices; 2304 x 4096, K 147456: 144,
+//     1511 and 1405), or one to one and a half times (4352 x 4352, K 147456: 289, 3045 and 2777).  In
+//     between the promise is not kept: 592 x 16416, K 147456: 195 tiles, 1470 unsplit and 1577 in five
+//     slices; 4864 x 2560: 190 tiles, K 98304 1215 and 1244 in four, K 147456 1743 and 1641.
 //     Contractions of up to 4096 stay one chain of sums, as other implementations form them too:
 //     a result that all but cancels moves by several bf16 steps with the order of its sum.
 GemmPlan plan_dense(int64_t M, int64_t N, int64_t K, bool may_split) {
@@ -1442,7 +1445,8 @@ GemmPlan plan_dense(int64_t M, int64_t N, int64_t K, bool may_split) {
       if (per < 4 || (s - 1) * per >= blocks || (debug_slices && s != debug_slices)) continue;
       const double bytes = 4.0 * s * M * N;
       const bool large = bytes > (double)(64 << 20);
-      if (large && (u.ta * u.tb < 16 || 2 * tiles <= grid || 2 * tiles >= 3 * grid)) continue;
+      if (large && (u.ta * u.tb < 16 || 2 * tiles <= grid || (7 * tiles > 5 * grid && tiles <= grid) || 2 * tiles >= 3 * grid))
+        continue;
       const double us = tiles_us(u, tiles * s, per, grid) + 2.0 + 4.2 + bytes / 3.2e6;
       if (us < best_us && us <= 0.92 * plain_us || debug_slices) {
         best = {u.ta, u.tb, s};

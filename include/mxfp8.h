@@ -408,8 +408,9 @@ int mx_gemm_nt_f32_ld(const uint8_t* a_codes, const uint8_t* a_scales, const uin
  * launches nothing (to know beforehand: mx_gemm_nt_workspace_bytes(M, N, K) against
  * mx_gemm_nt_static_max_bytes(); such a shape runs through mx_gemm_nt unsplit, or through
  * mx_gemm_nt_ws with memory of the caller's).  The first call on a GPU looks up that GPU's copy
- * of the array and raises the LDS limit of every dense kernel, neither of which belongs into a graph capture:
- * make one call per GPU (any shape) before capturing.  All calls on one GPU share that GPU's array: calls that overlap in time on
+ * of the array, which does not belong into a graph capture: make one call per GPU (any shape) before
+ * capturing.  (Likewise for the other dense products: the first one on a GPU of more than 64 rows raises the LDS
+ * limits of the kernels of all of them, whatever its form and shape.)  All calls on one GPU share that GPU's array: calls that overlap in time on
  * the same GPU (two streams, two threads) race on it.  Nothing in the array needs clearing between
  * calls: every partial tile is written in full before the reduction reads it. */
 int64_t mx_gemm_nt_static_max_bytes(void);

@@ -28,6 +28,9 @@ void mx_debug_set_grid(int workgroups);
  * 128-deep blocks.  0: by shape (default). */
 void mx_debug_set_tile(int ta, int tb, int slices);
 
+/* How many kernels have had their LDS limit raised, counted once per kernel and GPU. */
+int mx_debug_lds_limits_raised(void);
+
 /* -DMX_TIMING_BUILD only.  Device buffer of 256 * 4 * 8 uint64 that the timing build of the persistent kernel fills with
  * per-wave cycle counts {copy wait, barriers, step body, epilogue, ...}; NULL switches the timing
  * build off (default). */

@@ -161,3 +161,36 @@ def test_shapes_that_are_split(device, hooks):
             for N in (1024, 4096, 6144):
                 for K in (2176, 6144, 14336, 147456):
                     assert pair(M, N, K) <= 64 << 20 and pair(M, N, K) % (2 * M * N * 4) == 0
+
+
+def test_one_product_prepares_all_others_for_capture(device, hooks):
+    """The first dense product on tiles raises the LDS limits of every tile and form, so that a graph may capture others
+    than the one that the program warmed up on: nothing is left to raise, and captured products replay as eager ones."""
+    rng = np.random.default_rng(5)
+    M, N, K = 200, 264, 4352
+    (a, a2), (b, b2) = [[_operand(device, rng, rows, K, std)[0] for _ in range(2)] for rows, std in ((M, 1.0), (N, 0.02))]
+    ops.mx_gemm_nt(a, b)
+    raised = hooks.mx_debug_lds_limits_raised()
+    assert raised >= 3 * len(TILES) + 3 + 3  # plain, float32 and sum of two; slices of K; one tile a workgroup
+
+    def products():
+        out = []
+        for tile in TILES:
+            for slices in (0, 2) if tile[0] * tile[1] != 12 else (0,):
+                hooks.mx_debug_set_tile(*tile, slices)
+                ops._gemm_workspace.clear()
+                out += [ops.mx_gemm_nt(a, b), ops.mx_gemm_nt_as(a, b, torch.float32), ops.mx_gemm_nt_pair(a, b, a2, b2),
+                        ops.mx_gemm_nt_shared_a(a, b, b2), ops.mx_gemm_nt_shared_b(a, a2, b)]
+        hooks.mx_debug_set_tile(0, 0, 0)
+        ops._gemm_workspace.clear()
+        return out
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = products()
+    assert hooks.mx_debug_lds_limits_raised() == raised
+    for std in (1.0, 3.0):
+        a.buf.copy_(_operand(device, rng, M, K, std)[0].buf)
+        graph.replay()
+        torch.cuda.synchronize()
+        for i, (x, y) in enumerate(zip(got, products(), strict=True)):
+            assert torch.equal(x, y), i

@@ -125,6 +125,8 @@ inline int current_device_cus() {
   return n;
 }
 
+inline std::atomic<int> lds_limits_raised{0};  // (include/mxfp8_debug.h)
+
 // Raises a kernel's dynamic-LDS limit once per device.  `done` is the kernel's own table
 // (a function-local static of the launcher, one per template instance).
 inline bool raise_lds_limit(const void* kernel, int bytes, std::atomic<bool> (&done)[kMaxDevices]) {
@@ -132,7 +134,7 @@ inline bool raise_lds_limit(const void* kernel, int bytes, std::atomic<bool> (&d
   if (dev < 0) return false;
   if (!done[dev].load(std::memory_order_acquire)) {
     if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) return false;
-    done[dev].store(true, std::memory_order_release);
+    if (!done[dev].exchange(true, std::memory_order_acq_rel)) ++lds_limits_raised;
   }
   return true;
 }

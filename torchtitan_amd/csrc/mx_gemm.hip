@@ -36,11 +36,28 @@ static bool configure_dense() {
   return raise_lds_limit(reinterpret_cast<const void*>(gemm_nt_kernel<BM, BN, F32>), GemmTile<BM, BN, false, false>::kLdsBytes,
                          configured);
 }
+// Raises the LDS limit of every kernel on tiles that a dense product of any shape and form may run on, in front of the
+// first such launch on a GPU: limits are not to be raised under graph capture, and which tile a captured shape takes
+// is not the caller's business.
+bool prepare_dense32();
+bool prepare_dense() {
+  static std::atomic<bool> prepared[kMaxDevices];
+  const int dev = current_device();
+  if (dev < 0) return false;
+  if (!prepared[dev].load(std::memory_order_acquire)) {
+    if (!prepare_dense32() || !configure_dense<128, 128>() || !configure_dense<256, 256>() ||
+        !configure_dense<128, 128, true>())
+      return false;
+    prepared[dev].store(true, std::memory_order_release);
+  }
+  return true;
+}
+
 template <int BM, int BN, bool F32 = false>
 static int launch_dense(const DenseArgs& p, hipStream_t st) {
   using Tile = GemmTile<BM, BN, false, false>;
   auto kern = gemm_nt_kernel<BM, BN, F32>;
-  if (!configure_dense<BM, BN, F32>()) return MX_ERR_LAUNCH;
+  if (!prepare_dense()) return MX_ERR_LAUNCH;
   const int64_t nb = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
   const int64_t grid = (nb + 7) / 8 * 8;
   if (grid > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
@@ -60,7 +77,6 @@ int launch_few_rows_codes(const uint8_t* a_codes, const uint8_t* a_scales, const
                           const uint8_t* b_scales, void* d, int64_t M, int64_t N, int64_t K, int64_t ldk, int64_t ldd,
                           hipStream_t st);
 GemmPlan plan_dense(int64_t M, int64_t N, int64_t K, bool may_split);
-bool prepare_dense32();
 int launch_gemm_nt32_splitk(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                             const uint8_t* b_scales, void* d, int64_t M, int64_t N, int64_t K,
                             int64_t ldk, int64_t ldd, const GemmPlan& plan, void* workspace, bool f32,
@@ -73,6 +89,7 @@ static std::atomic<int> force_kernel{0};
 extern "C" void mx_debug_force_kernel(int which) { force_kernel = which; }
 namespace mx { void set_debug_grid(int g); }
 extern "C" void mx_debug_set_grid(int g) { mx::set_debug_grid(g); }
+extern "C" int mx_debug_lds_limits_raised(void) { return mx::lds_limits_raised; }
 namespace mx { void set_debug_tile(int ta, int tb, int slices); }
 extern "C" void mx_debug_set_tile(int ta, int tb, int slices) { mx::set_debug_tile(ta, tb, slices); }
 #ifdef MX_TIMING_BUILD
@@ -346,7 +363,7 @@ static void* scratch_of_current_device() {
   if (dev < 0) return nullptr;
   std::lock_guard<std::mutex> lock(scratch_mutex);
   if (!scratch_ptr[dev]) {
-    if (!prepare_dense32() || !configure_dense<128, 128>() || !configure_dense<256, 256>()) return nullptr;
+    if (!prepare_dense()) return nullptr;
     void* ptr = nullptr;
     if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)) != hipSuccess) return nullptr;
     scratch_ptr[dev] = ptr;

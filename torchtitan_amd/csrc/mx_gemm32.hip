@@ -1341,11 +1341,13 @@ static bool configure32() {
   return raise_lds_limit(reinterpret_cast<const void*>(gemm_nt32_kernel<MODE, PROF, PAIR, TA, TB, OUT32>),
                          Lds32<TA, TB>::kBytes, configured);
 }
+bool prepare_dense();
 template <int MODE, bool PROF, bool PAIR = false, int TA = 4, int TB = 4, bool OUT32 = false>
 static int launch32(const Gemm32Args& p, int64_t nb, hipStream_t st) {
   auto kern = gemm_nt32_kernel<MODE, PROF, PAIR, TA, TB, OUT32>;
   constexpr int lds = Lds32<TA, TB>::kBytes;  // ring + one output patch per wave: most of the CU's 160 KB
-  if (!configure32<MODE, PROF, PAIR, TA, TB, OUT32>()) return MX_ERR_LAUNCH;
+  constexpr bool kDenseForm = !PROF && (MODE == kDense || MODE == kSplitK);
+  if (!(kDenseForm ? prepare_dense() : configure32<MODE, PROF, PAIR, TA, TB, OUT32>())) return MX_ERR_LAUNCH;
   int64_t grid = persistent_grid();
   if (grid == 0) return MX_ERR_LAUNCH;
   const int64_t need = (nb + 7) / 8 * 8;  // nb: the tile count, or an upper bound of it
@@ -1517,12 +1519,15 @@ static int launch_best32(const Gemm32Args& p, hipStream_t st) {
   return t ? launch_dense32<kDense, PAIR, OUT32>(p, t->ta, t->tb, st) : MX_ERR_UNSUPPORTED;
 }
 
-// Raises the LDS limits of every kernel that a dense product may run on, for a caller that captures
-// products of other shapes than the one it has called.
+// Raises the LDS limit of every persistent kernel that a dense product may run on (prepare_dense).
+template <int TA, int TB>
+static bool prepare_tile() {
+  return configure32<kDense, false, false, TA, TB>() && configure32<kDense, false, true, TA, TB>() &&
+         configure32<kDense, false, false, TA, TB, true>();
+}
 bool prepare_dense32() {
-  return configure32<kDense, false, false, 4, 4>() && configure32<kDense, false, false, 3, 4>() &&
-         configure32<kDense, false, false, 4, 3>() && configure32<kDense, false, false, 2, 4>() &&
-         configure32<kDense, false, false, 4, 2>() && configure32<kSplitK, false, false, 4, 4>() &&
+  return prepare_tile<4, 4>() && prepare_tile<3, 4>() && prepare_tile<4, 3>() && prepare_tile<2, 4>() &&
+         prepare_tile<4, 2>() && configure32<kSplitK, false, false, 4, 4>() &&
          configure32<kSplitK, false, false, 2, 4>() && configure32<kSplitK, false, false, 4, 2>();
 }
 

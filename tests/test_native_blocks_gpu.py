@@ -188,6 +188,45 @@ def test_routed_experts(device, monkeypatch, experts, top_k, shared, tokens, bef
         assert "routed_forward" in taken and "routed_backward" in taken
 
 
+def _block(kind, device):
+    if kind == "linear":
+        return _holder(Linear.Config().build(in_features=256, out_features=384), device)
+    if kind == "feed forward":
+        return _holder(FeedForward.Config(hidden_dim=384).build(dim=256), device)
+    moe = MoE(MoE.Config(num_experts=8, num_shared_experts=0, hidden_dim=256, top_k=2, score_func="softmax"),
+              dim=256).to(device).to(torch.bfloat16)
+    moe.init_weights(init_std=0.02, buffer_device=device)
+    holder = nn.Module()
+    holder.moe = moe
+    _convert(holder, ["experts"])
+    return moe
+
+
+@pytest.mark.parametrize("kind", ["linear", "feed forward", "experts"])
+def test_saved_tensors_that_hooks_return_as_others(device, monkeypatch, kind):
+    """Hooks may give a backward its saved tensors with other strides; on another device, or with less in them, is an
+    error on either path."""
+    torch.manual_seed(1)
+    block = _block(kind, device)
+    x, dy = (torch.randn(1, 200, n, device=device, dtype=torch.bfloat16) for n in (256, 384 if kind == "linear" else 256))
+    pack = lambda t: t
+    strided = lambda t: torch.stack((t, t), -1)[..., 0]
+    moved = lambda t: t.cpu()
+    short = lambda t: t.view(-1)[:t.numel() // 2].clone() if t.dtype == torch.uint8 and t.dim() == 1 else t
+    step = lambda unpack: _step(block, list(block.parameters()), x, dy,
+                                hooks=lambda: torch.autograd.graph.saved_tensors_hooks(pack, unpack))
+    want = step(lambda t: t)
+    native, general, taken = _both(monkeypatch, lambda: step(strided))
+    assert any(name.endswith("_forward") for name in taken) and not any(name.endswith("_backward") for name in taken)
+    _same(native, want)
+    _same(general, want)
+    with pytest.raises((RuntimeError, TypeError)):
+        step(moved)
+    if kind != "experts":  # (whose codes and scales are tensors with shapes of their own)
+        with pytest.raises(RuntimeError, match="saved MXFP8 operand"):
+            step(short)
+
+
 def test_capture(device):
     """A captured step of native calls replays on new inputs."""
     lin = _holder(Linear.Config().build(in_features=256, out_features=384), device)

@@ -96,24 +96,34 @@ struct Operand {
 
 int64_t up128(int64_t n) { return (n + 127) & ~int64_t{127}; }
 
-// ... around a buffer laid out as `make` lays it out
-Operand around(const Tensor& buf, int64_t rows, int64_t cols, int64_t pad) {
+Operand layout_of(int64_t rows, int64_t cols, int64_t pad) {
   const int64_t k = up128(cols), ld = k + pad;
-  return {buf, rows, k, ld, 0, (rows * ld + 255) & ~int64_t{255}, cols};
+  return {Tensor(), rows, k, ld, 0, (rows * ld + 255) & ~int64_t{255}, cols};
 }
 Operand make(int64_t rows, int64_t cols, int64_t pad, const Tensor& like) {
-  Operand o = around(Tensor(), rows, cols, pad);
+  Operand o = layout_of(rows, cols, pad);
   o.buf = at::empty({o.scales_at + up128(rows) * (o.k / 32)}, like.options().dtype(at::kByte));
   return o;
 }
 std::array<Operand, 2> make_pair(int64_t rows, int64_t cols, int64_t pad, const Tensor& like) {
-  Operand a = around(Tensor(), rows, cols, pad), b = a;
+  Operand a = layout_of(rows, cols, pad), b = a;
   const int64_t scales = up128(rows) * (a.k / 32);
   a.scales_at = (2 * rows * a.ld + 255) & ~int64_t{255};
   b.at = rows * a.ld;
   b.scales_at = a.scales_at + scales;
   a.buf = b.buf = at::empty({a.scales_at + 2 * scales}, like.options().dtype(at::kByte));
   return {a, b};
+}
+
+// A saved operand of `rows` rows and a contraction of `cols`, from the buffer that a backward gets back (hooks on
+// saved tensors may have made it anew) and the layout that the forward kept: false unless it is what the products
+// of this call take, on the GPU of `like`.  (ops.saved_operand has the general case.)
+using Layout = std::array<int64_t, 6>;
+bool saved_operand(Operand& o, const Tensor& buf, const Layout& layout, int64_t rows, int64_t cols, int64_t pad, const Tensor& like) {
+  const auto [r, k, ld, at, scales_at, depth] = layout;
+  o = {buf, r, k, ld, at, scales_at, depth};
+  return r == rows && depth == cols && k == up128(cols) && ld == k + pad && buf.scalar_type() == at::kByte &&
+         buf.device() == like.device() && buf.is_contiguous() && buf.numel() >= scales_at + up128(rows) * (k / 32);
 }
 
 // A matrix that the casts read as it lies (ops._operand_input returns it unchanged)
@@ -183,24 +193,26 @@ py::object linear_forward(const Tensor& x, const Tensor& w, int mode, int64_t pa
   return py::make_tuple(y, xr.buf, xr.layout(), xc.buf, xc.layout(), wc.buf, wc.layout());
 }
 
-// (dx, dW) from dy and the buffers of linear_forward's column-wise operands
-py::object linear_backward(const Tensor& dy, const Tensor& x_buf, const Tensor& w_buf, int64_t K, int mode, int64_t pad,
-                           bool dx_f32, bool dw_f32) {
+// (dx, dW) from dy and linear_forward's column-wise operands
+py::object linear_backward(const Tensor& dy, const Tensor& x_buf, const Layout& x_layout, const Tensor& w_buf,
+                           const Layout& w_layout, int mode, int64_t pad, bool dx_f32, bool dw_f32) {
   if (!plain(dy) || !on_current_device(dy)) return py::none();
-  const int64_t M = dy.size(0), N = dy.size(1);
+  const int64_t M = dy.size(0), N = dy.size(1), K = x_layout[0];
+  Operand x, w;
+  if (!saved_operand(x, x_buf, x_layout, K, M, pad, dy) || !saved_operand(w, w_buf, w_layout, K, N, pad, dy)) return py::none();
   hipStream_t st = stream_of(dy);
   const Operand r = make(M, N, pad, dy), c = make(N, M, pad, dy);
   checked(lib.cast_pad(dy.data_ptr(), dy.scalar_type() == at::kFloat, M, N, dy.stride(0), r.codes(), r.ld, r.scales(),
                        c.codes(), c.ld, c.scales(), mode, st),
           "mx_cast_pad");
-  const Tensor dx = gemm(r, around(w_buf, K, N, pad), dy, st, dx_f32 ? at::kFloat : at::kBFloat16);
-  const Tensor dw = gemm(c, around(x_buf, K, M, pad), dy, st, dw_f32 ? at::kFloat : at::kBFloat16);
+  const Tensor dx = gemm(r, w, dy, st, dx_f32 ? at::kFloat : at::kBFloat16);
+  const Tensor dw = gemm(c, x, dy, st, dw_f32 ? at::kFloat : at::kBFloat16);
   return py::make_tuple(dx, dw);
 }
 
 // y = x W^T without gradients, W's row-wise operand given (its buffers and layout): (y, row-wise x or None).
 // `few`: by the product that casts x itself (ops.few_rows_ok).
-py::object linear_apply(const Tensor& x, const Tensor& w_buf, const Tensor& w_scales, const std::array<int64_t, 6>& layout,
+py::object linear_apply(const Tensor& x, const Tensor& w_buf, const Tensor& w_scales, const Layout& layout,
                         int mode, bool few) {
   const auto [N, k, ld, at, scales_at, depth] = layout;
   if (!plain(x) || x.size(1) != depth || ld % 128 || w_buf.device() != x.device() || !on_current_device(x)) return py::none();
@@ -267,24 +279,30 @@ py::object ffn_forward(const Tensor& x, const Tensor& w1, const Tensor& w3, cons
                         w1c.buf, w1c.layout(), w3c.buf, w3c.layout());
 }
 
-// (dx, dW1, dW2, dW3), bf16, from dy and what ffn_forward returned
-py::object ffn_backward(const Tensor& dy, const Tensor& h13, const Tensor& w2_buf, const Tensor& x_buf, const Tensor& g_buf,
-                        const Tensor& w1_buf, const Tensor& w3_buf, int64_t D, int mode, int64_t pad) {
-  if (!plain(dy) || !on_current_device(dy) || h13.dim() != 3 || !h13.is_contiguous()) return py::none();
+// (dx, dW1, dW2, dW3), bf16, from dy and what ffn_forward returned: h13 and the column-wise W2, x, g, W1, W3
+py::object ffn_backward(const Tensor& dy, const Tensor& h13, const std::array<Tensor, 5>& bufs,
+                        const std::array<Layout, 5>& layouts, int64_t D, int mode, int64_t pad) {
+  if (!plain(dy) || !on_current_device(dy) || h13.dim() != 3 || !h13.is_contiguous() || h13.scalar_type() != at::kBFloat16 ||
+      h13.device() != dy.device() || h13.size(0) != 2 || h13.size(1) != dy.size(0))
+    return py::none();
   const int64_t M = dy.size(0), O = dy.size(1), H = h13.size(2);
+  const std::array<std::array<int64_t, 2>, 5> sides{{{H, O}, {D, M}, {H, M}, {D, H}, {D, H}}};
+  std::array<Operand, 5> saved;
+  for (int i = 0; i < 5; ++i)
+    if (!saved_operand(saved[i], bufs[i], layouts[i], sides[i][0], sides[i][1], pad, dy)) return py::none();
+  const auto& [w2, x, g, w1, w3] = saved;
   hipStream_t st = stream_of(dy);
   const Operand r = make(M, O, pad, dy), c = make(O, M, pad, dy);
   checked(lib.cast_pad(dy.data_ptr(), dy.scalar_type() == at::kFloat, M, O, dy.stride(0), r.codes(), r.ld, r.scales(),
                        c.codes(), c.ld, c.scales(), mode, st),
           "mx_cast_pad");
-  const Tensor dg = gemm(r, around(w2_buf, H, O, pad), dy, st);
+  const Tensor dg = gemm(r, w2, dy, st);
   const auto [ra, rb] = make_pair(M, H, pad, dy);
   const auto [ca, cb] = make_pair(H, M, pad, dy);
   const char* h1 = static_cast<const char*>(h13.data_ptr());
   checked(lib.swiglu_bwd(dg.data_ptr(), h1, h1 + 2 * M * H, M, H, H, H, H, ra.codes(), ra.ld, ra.scales(), ca.codes(),
                          ca.ld, ca.scales(), mode, st),
           "mx_swiglu_bwd_cast_pad");
-  const Operand x = around(x_buf, D, M, pad), w1 = around(w1_buf, D, H, pad), w3 = around(w3_buf, D, H, pad);
   const Tensor dw13 = at::empty({2, H, D}, h13.options());
   if (persistent_shape(H, D)) {
     char* out = static_cast<char*>(dw13.data_ptr());
@@ -295,7 +313,7 @@ py::object ffn_backward(const Tensor& dy, const Tensor& h13, const Tensor& w2_bu
     gemm_into(ca, x, dw13[0], st);
     gemm_into(cb, x, dw13[1], st);
   }
-  const Tensor dw2 = gemm(c, around(g_buf, H, M, pad), dy, st);
+  const Tensor dw2 = gemm(c, g, dy, st);
   Tensor dx;
   if (persistent_shape(M, D)) {
     dx = at::empty({M, D}, h13.options());
@@ -405,13 +423,23 @@ py::object routed_forward(const Tensor& x, const Tensor& scores, const Tensor& w
 
 // (dx, d scores, dW1, dW2, dW3) from dout [T, D] and those slots; at most 16 choices a token
 py::object routed_backward(const Tensor& dout, const std::vector<Tensor>& saved, int mode, bool score_before) {
+  TORCH_CHECK(saved.size() == 17, "17 saved tensors expected");
   const Tensor &offs = saved[0], &src_row = saved[1], &row_score = saved[2], &pos = saved[3], &scores = saved[4],
                &h13 = saved[5];
   if (!plain(dout) || dout.scalar_type() != at::kBFloat16 || !dout.is_contiguous() || !on_current_device(dout))
     return py::none();
   for (const Tensor& t : saved)
     if (!t.is_contiguous() || t.device() != dout.device()) return py::none();
+  if (h13.dim() != 3 || h13.size(0) != 2 || pos.dim() != 2 || h13.scalar_type() != at::kBFloat16 ||
+      saved[16].scalar_type() != at::kBFloat16)
+    return py::none();
   const int64_t T = dout.size(0), D = dout.size(1), G = offs.numel(), R = h13.size(1), H = h13.size(2), k = pos.size(1);
+  const int64_t weight = G * D * H, tokens_d = up128(D) * (R / 32), tokens_h = up128(H) * (R / 32);
+  const int64_t sizes[] = {G, R, R, T * k, T * k, 2 * R * H, weight, weight / 32, D * R, tokens_d, H * R, tokens_h,
+                           weight, weight / 32, weight, weight / 32, (score_before ? T : R) * D};
+  for (size_t i = 0; i < std::size(sizes); ++i)
+    TORCH_CHECK(saved[i].numel() == sizes[i], "saved tensor ", i, " came back with ", saved[i].numel(), " elements, ",
+                sizes[i], " expected");
   hipStream_t st = stream_of(dout);
   const int32_t* ends = offs.data_ptr<int32_t>();
   const int64_t* place = pos.data_ptr<int64_t>();

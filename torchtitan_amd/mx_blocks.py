@@ -45,13 +45,13 @@ class _MXSwiGLULinear(torch.autograd.Function):
         dyq0, dyq1 = ops.to_operands(_castable(_rows_of(dy)), mode, need_dh, need_dw)
         dh1 = dh3 = dw = None
         if need_dh:
-            dg = ops.mx_gemm_nt(dyq0, ops.Operand(w_buf, ctx.w_layout)).view(h1.shape)
+            dg = ops.mx_gemm_nt(dyq0, ops.saved_operand(w_buf, ctx.w_layout, dy.device)).view(h1.shape)
             if ctx.needs_input_grad[1]:
                 dh3 = dg * F.silu(h1)
             if ctx.needs_input_grad[0]:
                 dh1 = torch.ops.aten.silu_backward(dg * h3, h1)
         if need_dw:
-            dw = ops.mx_gemm_nt(dyq1, ops.Operand(g_buf, ctx.g_layout))
+            dw = ops.mx_gemm_nt(dyq1, ops.saved_operand(g_buf, ctx.g_layout, dy.device))
             if dw.dtype != ctx.w_dtype:
                 dw = dw.to(ctx.w_dtype)
         return dh1, dh3, dw, None
@@ -250,13 +250,12 @@ class _MXFeedForward(torch.autograd.Function):
         need = ctx.needs_input_grad
         dy2, tensors, out = _castable(_rows_of(dy)), ctx.saved_tensors, None
         if ctx.native and ops.native_block_ok(dy2, dy2.shape[1]):
-            h13, w2_buf, x_buf, g_buf, w1_buf, w3_buf = tensors[:6]
-            out = _lib.blocks().ffn_backward(dy2, h13, w2_buf, x_buf, g_buf, w1_buf, w3_buf, ctx.x_shape[-1],
+            out = _lib.blocks().ffn_backward(dy2, tensors[0], tensors[1:6], ctx.layouts[1:6], ctx.x_shape[-1],
                                              ops._mode(ctx.cfg.scale_mode), ctx.pad)
         if out is not None:
             (dx, dw1, dw2, dw3), dnw = out, None
         else:
-            saved = {name: (t if layout is None else ops.Operand(t, layout))
+            saved = {name: (t if layout is None else ops.saved_operand(t, layout, dy2.device))
                      for name, t, layout in zip(FFN_SAVED, tensors, ctx.layouts)}
             dx, dw1, dw2, dw3, dnw = ffn_backward(dy2, saved, ctx.cfg, need[0], need[1], need[2], need[3],
                                                   need[5], pad=ctx.pad, whole_blocks=True)
@@ -348,7 +347,7 @@ class _MXNormLinears(torch.autograd.Function):
         mode = ctx.cfg.scale_mode
         saved = list(ctx.saved_tensors)
         x2, rstd, norm_weight = saved[:3]
-        hq1, *wqs = (ops.Operand(buf, layout) for buf, layout in zip(saved[3:], ctx.layouts))
+        hq1, *wqs = (ops.saved_operand(buf, layout, x2.device) for buf, layout in zip(saved[3:], ctx.layouts))
         dh, dws = None, []
         for i, dy in enumerate(dys):
             need_dw = ctx.needs_input_grad[4 + i]
@@ -684,6 +683,7 @@ class _MXRoutedExperts(torch.autograd.Function):
         if ctx.native and ops.native_block_ok(dout, dout.shape[1]):
             grads = _lib.blocks().routed_backward(dout, saved, ops._mode(ctx.cfg.scale_mode), ctx.score_before)
         if grads is None:
+            saved = [ops.saved_matrix(t, dout.device) for t in saved]
             grads = routed_backward(dout, saved, ctx.cfg, ctx.order, ctx.score_before, *need[:5])
         dx, ds, dw1, dw2, dw3 = (g if g is None or g.dtype == dt else g.to(dt) for g, dt in zip(grads, ctx.dtypes))
         return dx, ds, dw1, dw2, dw3, None, None, None, None, None

@@ -347,8 +347,7 @@ class _MXLinear(torch.autograd.Function):
         pad = 0 if ctx.cfg.cache_weight_casts else ops.CODE_PITCH_PAD
         dx = dw = None
         if need_dx and need_dw and pad and ops.native_block_ok(dy2, dy2.shape[1], ctx.x_shape[-1]):
-            # (operands as both casts of x and W lay them out with this pitch)
-            out = _lib.blocks().linear_backward(dy2, x_buf, w_buf, ctx.x_shape[-1], ops._mode(mode), pad,
+            out = _lib.blocks().linear_backward(dy2, x_buf, ctx.x_layout, w_buf, ctx.w_layout, ops._mode(mode), pad,
                                                 ctx.x_dtype == torch.float32, ctx.w_dtype == torch.float32)
             if out is not None:
                 dx, dw = out
@@ -357,11 +356,11 @@ class _MXLinear(torch.autograd.Function):
                         dw if dw.dtype == ctx.w_dtype else dw.to(ctx.w_dtype), None)
         dyq0, dyq1 = ops.to_operands(dy2, mode, need_dx, need_dw, pad)
         if need_dx:
-            dx = ops.mx_gemm_nt_as(dyq0, ops.Operand(w_buf, ctx.w_layout), ctx.x_dtype)
+            dx = ops.mx_gemm_nt_as(dyq0, ops.saved_operand(w_buf, ctx.w_layout, dy2.device), ctx.x_dtype)
             if len(ctx.x_shape) != 2:
                 dx = dx.view(ctx.x_shape)
         if need_dw:
-            dw = ops.mx_gemm_nt_as(dyq1, ops.Operand(x_buf, ctx.x_layout), ctx.w_dtype)
+            dw = ops.mx_gemm_nt_as(dyq1, ops.saved_operand(x_buf, ctx.x_layout, dy2.device), ctx.w_dtype)
         return dx, dw, None
 
 

@@ -258,6 +258,25 @@ class Operand:
         return MXData(self.codes, self.scales, MX_SCALES_MFMA)
 
 
+def saved_operand(buf: torch.Tensor, layout, device) -> Operand:
+    """An operand from the buffer that a backward gets back and the layout that its forward kept.  The buffer may have
+    been through hooks on saved tensors: strides that the kernels would not follow are laid out anew, another device,
+    type or size is an error."""
+    rows, k, _, _, scales_at, _ = layout
+    need = scales_at + mfma_scale_bytes(rows, k // BLOCK)
+    if buf.device != device or buf.dtype != torch.uint8 or buf.numel() < need:
+        raise RuntimeError(f"a saved MXFP8 operand came back as {buf.dtype} x {buf.numel()} on {buf.device}; "
+                           f"expected torch.uint8 x {need} on {device}")
+    return Operand(buf if buf.is_contiguous() else buf.contiguous(), layout)
+
+
+def saved_matrix(t: torch.Tensor | None, device) -> torch.Tensor | None:
+    """`t`, which a backward gets back, as the kernels read it: dense, on `device` (see `saved_operand`)."""
+    if t is not None and t.device != device:
+        raise RuntimeError(f"a saved tensor came back on {t.device}; expected {device}")
+    return t if t is None else t.contiguous()
+
+
 def _new_operand(rows: int, cols: int, pad: int, device) -> Operand:
     """An operand of `rows` rows with a contraction of `cols` rounded up to whole 128-deep blocks."""
     k = -(-cols // WHOLE_BLOCK) * WHOLE_BLOCK
@@ -589,7 +608,9 @@ def route_topk_bwd(logits: torch.Tensor, selected: torch.Tensor, dtop: torch.Ten
                    scale: float) -> torch.Tensor:
     """Gradient of `route_topk`'s weights with respect to the logits, float32 [T, E]."""
     T, E = logits.shape
-    logits, dtop = logits.contiguous(), dtop.contiguous()
+    if selected.device != logits.device or dtop.device != logits.device:
+        raise ValueError("operands on different devices")
+    logits, selected, dtop = logits.contiguous(), selected.contiguous(), dtop.contiguous()
     out = torch.empty((T, E), dtype=torch.float32, device=logits.device)
     _call("mx_route_topk_bwd", "route_topk_bwd", logits.device, _ptr(logits), T, E, selected.shape[1], int(softmax),
           int(norm), scale, _ptr(selected), _ptr(dtop), _ptr(out), _stream(logits))

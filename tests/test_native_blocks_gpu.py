@@ -250,6 +250,37 @@ def test_capture(device):
         _same(out, step())
 
 
+def test_other_threads_run_during_native_calls(device, monkeypatch):
+    """The library is called with the interpreter lock released: every entry point is replaced by a function that says
+    whether its caller holds it (1: an error status), and launches nothing."""
+    import ctypes
+
+    blocks = [_block(kind, device) for kind in ("linear", "feed forward", "experts")]
+    counted, called = _Counted(_lib.blocks()), []
+
+    def held(status, name):
+        called.append(name)
+        raise AssertionError(f"{name} was called with the interpreter lock held")
+
+    address = ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value
+    _lib.blocks().bind({name: address for name in _lib.SIGNATURES}, held)
+    try:
+        with monkeypatch.context() as m:
+            m.setattr(_lib, "blocks", lambda: counted)
+            for block, outer in zip(blocks, (384, 256, 256)):
+                x, dy = (torch.zeros(1, 200, n, device=device, dtype=torch.bfloat16) for n in (256, outer))
+                _step(block, list(block.parameters()), x, dy)
+            with torch.no_grad():
+                for tokens in (16, 200):
+                    blocks[0](torch.zeros(tokens, 256, device=device, dtype=torch.bfloat16))
+    finally:
+        _lib._blocks = None
+        _lib.blocks()  # bound to the library again
+    assert not called
+    assert {"linear_forward", "linear_backward", "linear_apply", "ffn_forward", "ffn_backward", "routed_forward",
+            "routed_backward"} <= set(counted.taken)
+
+
 def test_threads_on_streams_of_their_own(device):
     """Two threads take the same linears over the same activation, which changes from pass to pass: each orders its
     stream behind what wrote the activation and no more, so a cast taken over from the other's stream, or memory that it

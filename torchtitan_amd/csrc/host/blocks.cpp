@@ -12,6 +12,7 @@
 #include <torch/extension.h>
 
 #include <array>
+#include <optional>
 
 #include "mxfp8.h"
 
@@ -81,8 +82,14 @@ void bind(const py::dict& addresses, const py::object& check) {
   Py_INCREF(check_status);
 }
 
+// Python's other threads run while a call allocates and launches, as they do under ctypes: a launch waits where the
+// queue is full.  Reset before Python objects are made.
+using Unlocked = std::optional<py::gil_scoped_release>;
+
 void checked(int status, const char* name) {
-  if (status) py::reinterpret_borrow<py::object>(check_status)(status, name);  // raises
+  if (!status) return;
+  py::gil_scoped_acquire locked;
+  py::reinterpret_borrow<py::object>(check_status)(status, name);  // raises
 }
 
 // ---- operands (ops.Operand): codes [rows, cols up to 128], rows `ld` bytes apart, then the scales
@@ -183,6 +190,7 @@ py::object linear_forward(const Tensor& x, const Tensor& w, int mode, int64_t pa
   if (!plain(x) || !plain_weight(w, x) || x.size(1) != w.size(1) || !on_current_device(x)) return py::none();
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
   hipStream_t st = stream_of(x);
+  Unlocked unlocked(std::in_place);
   const Operand xr = make(M, K, pad, x), xc = make(K, M, pad, x), wr = make(N, K, pad, x), wc = make(K, N, pad, x);
   std::array<int64_t, 8 * MX_CAST_PAD_MANY_FIELDS> table;
   int64_t n = 0;
@@ -190,6 +198,7 @@ py::object linear_forward(const Tensor& x, const Tensor& w, int mode, int64_t pa
   add_cast(table, n, w, wr, wc);
   checked(lib.cast_pad_many(n, table.data(), mode, st), "mx_cast_pad_many");
   const Tensor y = gemm(xr, wr, x, st);
+  unlocked.reset();
   return py::make_tuple(y, xr.buf, xr.layout(), xc.buf, xc.layout(), wc.buf, wc.layout());
 }
 
@@ -201,12 +210,14 @@ py::object linear_backward(const Tensor& dy, const Tensor& x_buf, const Layout& 
   Operand x, w;
   if (!saved_operand(x, x_buf, x_layout, K, M, pad, dy) || !saved_operand(w, w_buf, w_layout, K, N, pad, dy)) return py::none();
   hipStream_t st = stream_of(dy);
+  Unlocked unlocked(std::in_place);
   const Operand r = make(M, N, pad, dy), c = make(N, M, pad, dy);
   checked(lib.cast_pad(dy.data_ptr(), dy.scalar_type() == at::kFloat, M, N, dy.stride(0), r.codes(), r.ld, r.scales(),
                        c.codes(), c.ld, c.scales(), mode, st),
           "mx_cast_pad");
   const Tensor dx = gemm(r, w, dy, st, dx_f32 ? at::kFloat : at::kBFloat16);
   const Tensor dw = gemm(c, x, dy, st, dw_f32 ? at::kFloat : at::kBFloat16);
+  unlocked.reset();
   return py::make_tuple(dx, dw);
 }
 
@@ -218,6 +229,7 @@ py::object linear_apply(const Tensor& x, const Tensor& w_buf, const Tensor& w_sc
   if (!plain(x) || x.size(1) != depth || ld % 128 || w_buf.device() != x.device() || !on_current_device(x)) return py::none();
   const int64_t M = x.size(0), K = x.size(1);
   hipStream_t st = stream_of(x);
+  Unlocked unlocked(std::in_place);
   const uint8_t* codes = w_buf.data_ptr<uint8_t>() + at;
   const uint8_t* scales = w_scales.data_ptr<uint8_t>() + scales_at;
   if (few) {
@@ -225,6 +237,7 @@ py::object linear_apply(const Tensor& x, const Tensor& w_buf, const Tensor& w_sc
     checked(lib.few_rows(x.data_ptr(), M, K, x.stride(0), codes, scales, nullptr, nullptr, N, ld, y.data_ptr(), nullptr, N,
                          mode, st),
             "mx_few_rows");
+    unlocked.reset();
     return py::make_tuple(y, py::none(), py::none());
   }
   const Operand xr = make(M, K, ld - k, x);
@@ -237,6 +250,7 @@ py::object linear_apply(const Tensor& x, const Tensor& w_buf, const Tensor& w_sc
   checked(lib.gemm(xr.codes(), xr.scales(), codes, scales, y.data_ptr(), M, N, k, ld, N, need ? ws.data_ptr() : nullptr, need,
                    st),
           "mx_gemm_nt_ld");
+  unlocked.reset();
   return py::make_tuple(y, xr.buf, xr.layout());
 }
 
@@ -250,6 +264,7 @@ py::object ffn_forward(const Tensor& x, const Tensor& w1, const Tensor& w3, cons
   const int64_t M = x.size(0), D = x.size(1), H = w1.size(0), O = w2.size(0);
   if (w1.size(1) != D || w3.size(1) != D || w3.size(0) != H || w2.size(1) != H) return py::none();
   hipStream_t st = stream_of(x);
+  Unlocked unlocked(std::in_place);
   const Operand xr = make(M, D, pad, x), xc = make(D, M, pad, x);
   const Operand w1r = make(H, D, pad, x), w1c = make(D, H, pad, x), w3r = make(H, D, pad, x), w3c = make(D, H, pad, x);
   const Operand w2r = make(O, H, pad, x), w2c = make(H, O, pad, x);
@@ -275,6 +290,7 @@ py::object ffn_forward(const Tensor& x, const Tensor& w1, const Tensor& w3, cons
   checked(lib.swiglu(h1, h3, M, H, H, H, gr.codes(), gr.ld, gr.scales(), gc.codes(), gc.ld, gc.scales(), mode, st),
           "mx_swiglu_cast_pad");
   const Tensor y = gemm(gr, w2r, x, st);
+  unlocked.reset();
   return py::make_tuple(y, h13, xr.buf, xr.layout(), w2c.buf, w2c.layout(), xc.buf, xc.layout(), gc.buf, gc.layout(),
                         w1c.buf, w1c.layout(), w3c.buf, w3c.layout());
 }
@@ -292,6 +308,7 @@ py::object ffn_backward(const Tensor& dy, const Tensor& h13, const std::array<Te
     if (!saved_operand(saved[i], bufs[i], layouts[i], sides[i][0], sides[i][1], pad, dy)) return py::none();
   const auto& [w2, x, g, w1, w3] = saved;
   hipStream_t st = stream_of(dy);
+  Unlocked unlocked(std::in_place);
   const Operand r = make(M, O, pad, dy), c = make(O, M, pad, dy);
   checked(lib.cast_pad(dy.data_ptr(), dy.scalar_type() == at::kFloat, M, O, dy.stride(0), r.codes(), r.ld, r.scales(),
                        c.codes(), c.ld, c.scales(), mode, st),
@@ -330,6 +347,7 @@ py::object ffn_backward(const Tensor& dy, const Tensor& h13, const std::array<Te
   } else {
     dx = gemm(ra, w1, dy, st) + gemm(rb, w3, dy, st);
   }
+  unlocked.reset();
   return py::make_tuple(dx, dw13.select(0, 0), dw2, dw13.select(0, 1));
 }
 
@@ -382,6 +400,7 @@ py::object routed_forward(const Tensor& x, const Tensor& scores, const Tensor& w
   const int64_t k = scores.size(1);
   const int64_t R = (T * k + alignment * G + multiple - 1) / multiple * multiple;
   hipStream_t st = stream_of(x);
+  Unlocked unlocked(std::in_place);
   const Tensor offs = at::empty({G}, x.options().dtype(at::kInt)), src_row = at::empty({R}, x.options().dtype(at::kLong)),
                row_score = at::empty({R}, x.options().dtype(at::kFloat)),
                pos = at::empty({T, k}, x.options().dtype(at::kLong));
@@ -416,6 +435,7 @@ py::object routed_forward(const Tensor& x, const Tensor& scores, const Tensor& w
   checked(lib.combine(yp.data_ptr(), nullptr, R, D, pos.data_ptr<int64_t>(), score_before ? nullptr : scores.data_ptr<float>(),
                       T, k, D, out.data_ptr(), D, st),
           "mx_moe_combine");
+  unlocked.reset();
   return py::make_tuple(out, py::make_tuple(offs, src_row, row_score, pos, scores, h13, w2c.codes, w2c.scales, xc.codes,
                                             xc.scales, gc.codes, gc.scales, w1c.codes, w1c.scales, w3c.codes, w3c.scales,
                                             score_before ? x : yp));
@@ -441,6 +461,7 @@ py::object routed_backward(const Tensor& dout, const std::vector<Tensor>& saved,
     TORCH_CHECK(saved[i].numel() == sizes[i], "saved tensor ", i, " came back with ", saved[i].numel(), " elements, ",
                 sizes[i], " expected");
   hipStream_t st = stream_of(dout);
+  Unlocked unlocked(std::in_place);
   const int32_t* ends = offs.data_ptr<int32_t>();
   const int64_t* place = pos.data_ptr<int64_t>();
   Codes w2{saved[6], saved[7]}, xc{saved[8], saved[9]}, gc{saved[10], saved[11]}, w1{saved[12], saved[13]},
@@ -484,6 +505,7 @@ py::object routed_backward(const Tensor& dout, const std::vector<Tensor>& saved,
             "mx_moe_combine_dot");
     checked(lib.combine(dxp.data_ptr(), nullptr, R, D, place, nullptr, T, k, D, dx.data_ptr(), D, st), "mx_moe_combine");
   }
+  unlocked.reset();
   return py::make_tuple(dx, ds, dw13.select(0, 0), dw2, dw13.select(0, 1));
 }
 

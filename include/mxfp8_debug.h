@@ -14,8 +14,8 @@ extern "C" {
 #endif
 
 /* 0: pick the dense GEMM kernel by shape (default); 1 / 2: the one-tile-per-workgroup kernel with
- * 256x256 / 128x128 tiles for every shape; 3: the persistent kernel for every shape it can take,
- * however few tiles there are. */
+ * 256x256 / 128x128 tiles for every shape (float32 results: 128x128 either way); 3: the persistent
+ * kernel for every shape it can take, however few tiles there are. */
 void mx_debug_force_kernel(int which);
 
 /* > 0: number of persistent workgroups of the persistent kernel, rounded up to a multiple of 8

@@ -19,6 +19,7 @@ def hooks():
     yield lib
     lib.mx_debug_set_tile(0, 0, 0)
     lib.mx_debug_set_grid(0)
+    lib.mx_debug_force_kernel(0)
 
 
 def _operand(device, rng, rows, K, std=1.0):
@@ -194,3 +195,17 @@ def test_one_product_prepares_all_others_for_capture(device, hooks):
         torch.cuda.synchronize()
         for i, (x, y) in enumerate(zip(got, products(), strict=True)):
             assert torch.equal(x, y), i
+
+
+@pytest.mark.parametrize("kernel", [1, 2, 3])
+def test_float32_results_on_a_forced_kernel(device, hooks, kernel):
+    """A forced kernel is not split, whatever is lent, and gives the bf16 product's values on that kernel."""
+    rng = np.random.default_rng(kernel)
+    M, N, K = 200, 392, 8192
+    (a, _), (b, _) = _operand(device, rng, M, K), _operand(device, rng, N, K, 0.02)
+    need = int(hooks.mx_gemm_nt_workspace_bytes(M, N, K))
+    assert need > 0
+    ws = torch.full((need,), 0xFF, dtype=torch.uint8, device=device)
+    hooks.mx_debug_force_kernel(kernel)
+    assert torch.equal(_float32(a, b, N, ws), ops.mx_gemm_nt(a, b).float())
+    assert bool((ws == 0xFF).all())

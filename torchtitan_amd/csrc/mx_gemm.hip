@@ -329,12 +329,12 @@ extern "C" int mx_gemm_nt_f32_ld(const uint8_t* a_codes, const uint8_t* a_scales
   if (M <= 64 || N <= 128 || !persistent_ok(d, N, K, ldd, ldk) || (uint64_t)ldd * 1024 > 0x7FFFFFFFull)
     return MX_ERR_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
-  if (workspace && !((uintptr_t)workspace & 15)) {
+  if (workspace && force_kernel == 0 && !((uintptr_t)workspace & 15)) {
     const GemmPlan plan = split_plan(M, N, K);
     if (plan.slices > 1 && workspace_bytes >= split_bytes(plan, M, N))
       return launch_gemm_nt32_splitk(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldk, ldd, plan, workspace, true, st);
   }
-  if (plan_dense(M, N, K, false).ta == 0)
+  if (force_kernel == 1 || force_kernel == 2 || (force_kernel == 0 && plan_dense(M, N, K, false).ta == 0))
     return launch_dense<128, 128, true>(DenseArgs{a_codes, a_scales, b_codes, b_scales, (uint16_t*)d, M, N, K, ldd, ldk}, st);
   return launch_gemm_nt32(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldk, ldd, true, st);
 }

@@ -163,7 +163,7 @@ class _WeightCastCache:
         ref, version, capture, stream, done, rows, cols = e
         if ref.expired() or version != w._version or (capture and capture != _capture(w)):
             return None
-        if done is not None and stream != ops._stream(w):
+        if done is not None and stream[1] != ops._raw_stream(stream[0]):
             _follow(done, rows, cols)
         return rows, cols
 
@@ -175,7 +175,7 @@ class _WeightCastCache:
             del self._entries[k]
         capture, stream, done = _capture(w), None, None
         if w.is_cuda and not capture:
-            stream, done = ops._stream(w), torch.cuda.current_stream(w.device).record_event()
+            stream, done = (w.device.index, ops._stream(w)), torch.cuda.current_stream(w.device).record_event()
         self._entries[self._key(w, mode)] = (StorageWeakRef(w.untyped_storage()), w._version, capture, stream, done, rows, cols)
 
     def clear(self):
@@ -282,21 +282,25 @@ def _castable(t: torch.Tensor) -> torch.Tensor:
     return t if t.dtype in (torch.bfloat16, torch.float32) else t.to(torch.bfloat16)
 
 
-def _linear_apply(x2: torch.Tensor, src: torch.Tensor, weight: torch.Tensor, cfg: MXFP8Config, pad: int):
+def _linear_apply(x2: torch.Tensor, src: torch.Tensor, weight: torch.Tensor, cfg: MXFP8Config, K: int, N: int, pad: int):
     """x2 W^T without gradients.  The activation's cast is shared with sibling linears on `src`, but for few rows, which are
     cast inside their product; the weight is cast once, whichever way the product runs."""
-    mode, (K, N) = cfg.scale_mode, (x2.shape[1], weight.shape[0])
-    few = ops.few_rows_ok(x2, N)
-    remembered = None if few else _cast_cache.get(src, (mode, pad))
+    mode = cfg.scale_mode
+    native = ops.native_block_ok(x2, K, N)
+    if native:  # (what else `few_rows_ok` asks for, the native call checks itself)
+        few = x2.dtype == torch.bfloat16 and ops.few_rows_size(x2.shape[0], K, N)
+        native = few or _cast_cache.get(src, (mode, pad)) is None
+    else:
+        few = ops.few_rows_ok(x2, N)
     wq0, _ = _cast_weight(weight, mode, False, cfg, pitch_pad=pad)
-    if remembered is None and type(wq0) is ops.Operand and ops.native_block_ok(x2, K, N):
+    if native and type(wq0) is ops.Operand:
         out = _lib.blocks().linear_apply(x2, wq0.buf, wq0.scales_buf, wq0.layout, ops._mode(mode), few)
         if out is not None:
             y, xr, xr_layout = out
             if xr is not None:
                 _cast_cache.put(src, (mode, pad), (ops.Operand(xr, xr_layout), None))
             return y
-    if few:
+    if few and ops.few_rows_ok(x2, N):
         return ops.mx_few_rows(x2, wq0, mode)
     xq0, _ = _cast_activation(x2, src, mode, need_cols=False, pitch_pad=pad)
     return ops.mx_gemm_nt(xq0, wq0)
@@ -310,7 +314,7 @@ def _linear_forward(x, weight, cfg: MXFP8Config, need_dx: bool, need_dw: bool):
     # blocks and the hand-over share without a pitch
     pad = 0 if cfg.cache_weight_casts else ops.CODE_PITCH_PAD
     if not (need_dx or need_dw):
-        y = _linear_apply(x2, x, weight, cfg, pad)
+        y = _linear_apply(x2, x, weight, cfg, K, N, pad)
         return (y if x.dim() == 2 else y.view(*x.shape[:-1], N)), None, None
     if need_dx and need_dw and pad and ops.native_block_ok(x2, K, N) and _cast_cache.get(x, (mode, pad)) is None:
         out = _lib.blocks().linear_forward(x2, _castable(weight), ops._mode(mode), pad)

@@ -1034,6 +1034,11 @@ FEW_ROWS_VALUES = 65536   # values of x, rows counted in whole 16s, up to which 
 FEW_ROWS_COLUMNS = 16384  # columns of all products, up to which it is chosen
 
 
+def few_rows_size(rows: int, cols: int, columns: int) -> bool:
+    """The sizes of x and of all products' columns that `few_rows_ok` allows."""
+    return 0 < rows <= FEW_ROWS and columns <= FEW_ROWS_COLUMNS and (rows + 15 & ~15) * cols <= FEW_ROWS_VALUES
+
+
 def few_rows_ok(x: torch.Tensor, columns: int) -> bool:
     """`mx_few_rows` runs the products of x with weights of `columns` rows in all: bf16 rows on the GPU in whole
     blocks of 32, few enough of them, and no dispatch mode that would want to see the GEMM.  Every workgroup
@@ -1041,9 +1046,8 @@ def few_rows_ok(x: torch.Tensor, columns: int) -> bool:
     on the GPU, about 10 on the host): 16 x 4096 -> 4096 10.7 us in one launch, 3.7 + 7.5 in two; 32 x 2048 ->
     6144 12.6, 3.7 + 7.4; 32 x 14336 -> 4096 42, 3.8 + 27; and where the workgroups outnumber the CUs: 16 x 2048
     -> 16384 14.0 and 14.2, -> 2 x 14336 25.8 and 23.5, -> 151936 123 and 80 us."""
-    return (x.dtype == torch.bfloat16 and x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= FEW_ROWS
-            and columns <= FEW_ROWS_COLUMNS and (x.shape[0] + 15 & ~15) * x.shape[1] <= FEW_ROWS_VALUES and x.shape[1] % BLOCK == 0 and x.shape[1] > 0
-            and x.stride(1) == 1 and not _watched())
+    return (x.dtype == torch.bfloat16 and x.is_cuda and x.dim() == 2 and few_rows_size(*x.shape, columns)
+            and x.shape[1] % BLOCK == 0 and x.shape[1] > 0 and x.stride(1) == 1 and not _watched())
 
 
 def mx_few_rows(x: torch.Tensor, w: Operand, mode="floor", w2: Operand | None = None) -> torch.Tensor:

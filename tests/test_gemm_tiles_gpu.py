@@ -209,3 +209,42 @@ def test_float32_results_on_a_forced_kernel(device, hooks, kernel):
     hooks.mx_debug_force_kernel(kernel)
     assert torch.equal(_float32(a, b, N, ws), ops.mx_gemm_nt(a, b).float())
     assert bool((ws == 0xFF).all())
+
+
+@pytest.mark.parametrize("slices", [2, 6])
+@pytest.mark.parametrize("tile", [(4, 4), (2, 4), (4, 2)])
+@pytest.mark.parametrize("M,N,K", [(1, 136, 16896), (16, 264, 16896), (33, 392, 5760), (64, 136, 4352)])
+def test_splits_of_few_rows(device, hooks, M, N, K, tile, slices):
+    """Up to 64 rows, of contractions behind the line up to which their own kernel runs."""
+    rng = np.random.default_rng(M + slices)
+    (a, ha), (b, hb) = _operand(device, rng, M, K), _operand(device, rng, N, K, 0.02)
+    hooks.mx_debug_set_tile(*tile, slices)
+    need = int(hooks.mx_gemm_nt_workspace_bytes(M, N, K))
+    assert need == slices * M * N * 4
+    ws = torch.full((need,), 0xFF, dtype=torch.uint8, device=device)  # (NaN)
+    out = torch.full((M, N + 24), 7.0, dtype=torch.bfloat16, device=device)
+    for grid in (0, 8):
+        hooks.mx_debug_set_grid(grid)
+        ops._call("mx_gemm_nt_ld", "gemm_nt_splitk", device, a.codes_ptr, a.scales_ptr, b.codes_ptr, b.scales_ptr,
+                  out.data_ptr(), M, N, a.k, a.ld, N + 24, ws.data_ptr(), need, ops._stream(out))
+        _check(out[:, :N], ha @ hb.T)
+        assert bool((out[:, N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 4096, 8192), (33, 1024, 14336), (16, 4096, 17408)])
+def test_few_rows_that_are_split_by_shape(device, M, N, K):
+    rng = np.random.default_rng(M)
+    (a, ha), (b, hb) = _operand(device, rng, M, K), _operand(device, rng, N, K, 0.02)
+    with torch.cuda.device(device):
+        assert int(_lib.load().mx_gemm_nt_workspace_bytes(M, N, K)) > 0
+    _check(ops.mx_gemm_nt(a, b), ha @ hb.T)
+
+
+@pytest.mark.parametrize("N,K", [(1024, 2048), (4096, 4096), (392, 384)])
+def test_rows_do_not_depend_on_how_many_there_are(device, N, K):
+    """More than 64 rows of a contraction of up to 4096: one chain of sums in one order on every kernel and tile."""
+    rng = np.random.default_rng(N)
+    a, b = _operand(device, rng, 3001, K)[0], _operand(device, rng, N, K, 0.02)[0]
+    want = ops.mx_gemm_nt(a, b)
+    for M in (65, 128, 129, 200, 1000, 2048):
+        assert torch.equal(ops.mx_gemm_nt(a.first_rows(M), b), want[:M]), M

@@ -8,9 +8,13 @@
 // blocks, so the loads of the next tile's first blocks are already in flight while a tile is
 // written out.
 //
+// (Numbers here and below are those of the 256x256 tile where nothing else is said: a wave owns half of
+// either edge of any tile, Lds32 and BlockPlan have what follows from that.)
+//
 // Global -> LDS moves whole 128-byte rows (buffer_load_dwordx4 ... lds, 8 rows per instruction:
 // full cache lines, which the texture path delivers about twice as fast as 64-byte pieces), so
-// the ring holds two 128-deep blocks of 64 KB codes + 2 KB scales.  Two barriers per block: one
+// the ring holds two 128-deep blocks of 64 KB codes + 2 KB scales (128x256 and 256x128 tiles: three of
+// 48 + 2 KB).  Two barriers per block: one
 // releases the ring block whose last fragments have just been read (its refill starts there,
 // spread thinly because the copy path is the scarce resource), one makes sure the next block
 // has landed.
@@ -185,9 +189,6 @@ __device__ __forceinline__ float acc_read(const V& c) {
   return x;
 }
 
-// Fragment sets of four 16-row sub-tiles each, whole 128-deep blocks (a[h][t] =
-// sub-tile 4h + t of the wave's 128 rows of A, b[h][t] likewise for B), the scale dwords of the
-// block being computed (one for the even and one for the odd sub-tiles) and those of the next.
 // The LDS map of a tile of 64 TA x 64 TB: a ring of 128-deep blocks (A rows, B rows, scales of groups A0,
 // A1, B0, B1, A2 of 512 B each) and four waves' output patches.  128 x 256 and 256 x 128 tiles leave
 // room for a third block: theirs is 1024 MFMA cycles, less than it takes the copies from issue
@@ -208,6 +209,9 @@ struct Lds32 {
 };
 static_assert(Lds32<4, 4>::kRing == kRing32 && Lds32<4, 4>::kBlock == kBlock32, "the grouped modes' tables lie behind it");
 
+// Two fragment sets a side, whole 128-deep blocks: a[h][t] is sub-tile TA h + t of the wave's 32 TA rows of
+// A (16 rows each), b[h][t] likewise for B; the scale dwords of the block being computed (one for the even
+// and one for the odd sub-tiles) and those of the next.
 template <int TA, int TB>
 struct Frags16 {
   v8i a[2][TA];
@@ -934,7 +938,7 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
 #ifndef MX_STORE_AUX
 #define MX_STORE_AUX 2
 #endif
-  // A K block is 64 MFMAs, one per 16x16 sub-tile, in four quarters of 16 (512 MFMA cycles each)
+  // A K block of a 256x256 tile is 64 MFMAs, one per 16x16 sub-tile, in four quarters of 16 (512 MFMA cycles each)
   // over the fragment sets a[0], a[1] (rows 0-63, 64-127 of the wave) and b[0], b[1], in an
   // order that needs every set for two quarters in a row (slots 0-63 = the block's MFMAs; for
   // the smaller tiles, whose sets hold TA and TB sub-tiles, BlockPlan has the slots):
@@ -1414,14 +1418,17 @@ static const DenseTile* best_tile(int64_t M, int64_t N, int64_t blocks, int prod
 //     on the persistent kernel; K 1024 10.2 and 10.2; K 4096 28.5 and 22.7).
 //   * S slices add float32 partial sums, written and read back (3.2 TB/s) by a launch of their own,
 //     and are taken for a predicted gain of 8 %: 256 x 4096, K 8192 40 us unsplit, 23 in four
-//     slices; 512 x 4096, K 14336 85 and 39; 2048 x 2048, K 147456 1270 and 430.  The partial sums stay under 64 MiB,
+//     slices; 512 x 4096, K 14336 85 and 39; 2048 x 2048, K 147456 976 and 427 (rows 128 bytes further apart than
+//     they are long; dense rows 1300 and 537).  The partial sums stay under 64 MiB,
 //     one 256 x 256 tile per CU; more only where 256 x 256 tiles leave a good part of their rounds empty: half to 5/7 of
 //     the CUs (1280 x 6656, K 131072: 130 tiles, 1050 us unsplit, 940 in five slices; 2304 x 4096, K 147456: 144,
 //     1511 and 1405), or one to one and a half times (4352 x 4352, K 147456: 289, 3045 and 2777).  In
 //     between the promise is not kept: 592 x 16416, K 147456: 195 tiles, 1470 unsplit and 1577 in five
 //     slices; 4864 x 2560: 190 tiles, K 98304 1215 and 1244 in four, K 147456 1743 and 1641.
-//     Contractions of up to 4096 stay one chain of sums, as other implementations form them too:
-//     a result that all but cancels moves by several bf16 steps with the order of its sum.
+//     Contractions of up to 4096 stay one chain of sums.  Up to 2048 slices gain nothing (256 x 1024, K 2048 13.9 us
+//     and 13.9 in four; 256 x 2048, K 1024 9.6 and 13.1 in two; 2048 x 2048, K 2048 15.3 and 26.9); at 4096 they would
+//     (256 x 1024 22.9 and 16.1 in four, 256 x 4096 23.2 and 17.9), which is given up so that at these
+//     widths a row's result of more than 64 rows does not depend on how many there are: all tiles add in one order.
 GemmPlan plan_dense(int64_t M, int64_t N, int64_t K, bool may_split) {
   const int64_t grid = persistent_grid(), blocks = K / kKB;
   if (grid == 0 || K % kKB) return {0, 0, 1};

@@ -216,8 +216,10 @@ class _MXFeedForward(torch.autograd.Function):
     Forward: one cast of x, the gate inside the cast that feeds W2.  Backward: the gate's
     gradients inside the cast that feeds the dgrad / wgrad GEMMs of W1 and W3.  Neither g nor
     dh1 / dh3 is written to memory; kept for backward are h1, h3 and the column-wise MXFP8 forms
-    of x, g and the weights.  Results are bit-identical to the three converted linears around
-    bf16 ``F.silu`` and ``*`` (torchtitan/models/common/feed_forward.py:61-62)."""
+    of x, g and the weights.  y and the weights' gradients are bit-identical to those of the three converted
+    linears around bf16 ``F.silu`` and ``*`` (torchtitan/models/common/feed_forward.py:61-62) where no
+    product is split along K (`ops.mx_gemm_nt`; W1's and W3's products are not split here), else up to the
+    order of float32 sums; x's gradient is summed in float32 and rounded once."""
 
     @staticmethod
     def forward(ctx, x, w1, w2, w3, cfg: MXFP8Config, norm_weight=None, eps: float = 0.0):

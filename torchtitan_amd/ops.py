@@ -1209,8 +1209,8 @@ def _persistent_shape(M: int, N: int, K: int) -> bool:
 
 def mx_gemm_nt_shared_a(a: MXData, b: MXData, b2: MXData) -> torch.Tensor:
     """bf16 [2, M, N]: deq(a) @ deq(b)^T and deq(a) @ deq(b2)^T.  One launch in which the panels
-    of `a` are fetched once for both products where the persistent kernel takes the shape,
-    otherwise two GEMMs; bit-identical either way."""
+    of `a` are fetched once for both products where the persistent kernel takes the shape (never split
+    along K: bit-identical to `mx_gemm_nt` where that is not split either), otherwise two GEMMs."""
     if _operands(a, b, b2) and not _watched():
         M, N, K = a.rows, b.rows, a.k
         if b2.rows != N or not a.depth == b.depth == b2.depth:

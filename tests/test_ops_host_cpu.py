@@ -261,3 +261,13 @@ def test_a_forward_without_gradients_casts_each_operand_once(no_launches, monkey
     casts = [pointer for name, pointer in casts if name == "mx_cast_pad" or name.startswith("mx_cast_dim")]
     assert blocks.handed_back == 1  # (the second linear takes the activation's cast as it is)
     assert sorted(casts) == sorted(t.data_ptr() for t in (x, *weights))
+
+
+@pytest.mark.parametrize("pairs", [0, 1, 96, 127, 128, 129, 352, 383, 384, 385, 480, 481, 131072, 12983 * 8])
+@pytest.mark.parametrize("experts", [1, 8, 128])
+def test_padded_layouts_of_whole_blocks_are_no_whole_512s(pairs, experts):
+    """A bound of the aligned groups, at most two blocks beyond it, whose rows of column-wise codes do not lie 4 KB apart."""
+    need, got = pairs + 32 * experts, ops.plan_length(pairs, experts, 32, 128)
+    assert got % 128 == 0 and got % 512 and need <= got < need + 256
+    assert got < need + 128 or (got - 128) % 512 == 0
+    assert ops.plan_length(pairs, experts, 32) == need + -need % 32

@@ -157,9 +157,9 @@ def _grouped_layout(T: int, K: int, N: int, G: int, pad: bool):
     choices ``_MXGroupedMM.forward`` makes, as a function of the static sizes."""
     fast = K % 128 == 0 and N % 128 == 0 and G <= ops.FAST_MAX_GROUPS
     padded = pad or fast
-    step = ops.FAST_LENGTH_MULTIPLE if fast else ops.BLOCK
-    Tp = -(-(T + ops.BLOCK * G) // step) * step if padded else T
-    return (MX_SCALES_MFMA if fast else MX_SCALES_ROWMAJOR), padded, Tp, (ops.FAST_LENGTH_MULTIPLE if fast else 1)
+    multiple = ops.FAST_LENGTH_MULTIPLE if fast else 1
+    Tp = ops.plan_length(T, G, ops.BLOCK, multiple) if padded else T
+    return (MX_SCALES_MFMA if fast else MX_SCALES_ROWMAJOR), padded, Tp, multiple
 
 
 def _fake_scales(rows: int, nblk: int, order: int, device):
@@ -615,9 +615,7 @@ def _grouped_ffn_sizes(T, D, H, G, pad):
 
     order, multiple, fast = mx_blocks.grouped_layout(D, H, G)
     padded = pad or fast
-    step = max(ops.BLOCK, multiple)
-    Tp = -(-(T + ops.BLOCK * G) // step) * step if padded else T
-    return order, padded, Tp
+    return order, padded, ops.plan_length(T, G, ops.BLOCK, multiple) if padded else T
 
 
 @mx_grouped_ffn_fwd.register_fake
@@ -724,8 +722,7 @@ def _(x, top_scores, w1, w2, w3, tok_sorted, counts, score_before, mode, cache_w
     G, H, _ = w1.shape
     torch._check(D % 32 == 0 and H % 32 == 0, lambda: "the traced routed experts need sizes that are multiples of 32")
     order, multiple, _ = mx_blocks.grouped_layout(D, H, G)
-    step = max(ops.BLOCK, multiple)
-    Tp = -(-(T * k + ops.BLOCK * G) // step) * step
+    Tp = ops.plan_length(T * k, G, ops.BLOCK, multiple)
     dev = x.device
     s = [_empty(dev) for _ in range(17)]
     s[0] = torch.empty((G,), dtype=torch.int32, device=dev)

@@ -394,13 +394,11 @@ def _pad_plan(offs: torch.Tensor, T: int, align: int = 32, length_multiple: int 
     the way back).  The way back is, for every original row, its row in the padded layout or the
     index of an appended zero row (int64 [T]: a gather) -- or, with `direct`, a copy of the
     unpadded group ends (int32 [G]) for a grouped GEMM that writes the unpadded rows itself.
-    No host synchronisation: the padded length is the static bound round_up(T + align G, align),
-    rounded up further to `length_multiple` (a multiple of align) when one is given.
+    No host synchronisation: the padded length is the static bound `ops.plan_length`.
     """
     G = offs.numel()
     sizes = torch.diff(offs, prepend=offs.new_zeros(1))
-    step = max(align, length_multiple)
-    max_len = -(-(T + align * G) // step) * step
+    max_len = ops.plan_length(T, G, align, length_multiple)
     perm, _, m_offsets = ops.group_offsets_pad(sizes, G, 1, max_len, align)
     if direct:
         return perm, m_offsets, offs.to(torch.int32).clone()

@@ -479,8 +479,7 @@ def moe_route_plan(counts: torch.Tensor, order: torch.Tensor, scores: torch.Tens
     """(padded inclusive group ends int32 [E], token of every padded row int64 [max_len] (-1 =
     padding), score of every padded row float32 [max_len], padded row of every (token, choice)
     pair int64 [pairs]) for tokens-per-expert `counts` and the expert-sorted pair order; the
-    padded length is the static bound round_up(pairs + alignment * E, alignment), rounded up
-    further to `length_multiple` (a multiple of the alignment) when one is given."""
+    padded length is the static bound `plan_length`."""
     if not counts.is_cuda:
         raise _lib.MXLibraryError("moe_route_plan runs on the GPU only")
     dev = counts.device
@@ -493,7 +492,7 @@ def moe_route_plan(counts: torch.Tensor, order: torch.Tensor, scores: torch.Tens
         if scores.dtype != torch.float32 or scores.numel() != R or scores.device != dev:
             raise TypeError("scores must be float32 with one entry per pair")
         scores = scores.contiguous()
-    max_len = _plan_length(R, E, alignment, length_multiple)
+    max_len = plan_length(R, E, alignment, length_multiple)
     offs = torch.empty(E, dtype=torch.int32, device=dev)
     src_row = torch.empty(max_len, dtype=torch.int64, device=dev)
     row_score = torch.empty(max_len, dtype=torch.float32, device=dev)
@@ -617,11 +616,20 @@ def route_topk_bwd(logits: torch.Tensor, selected: torch.Tensor, dtop: torch.Ten
     return out
 
 
-def _plan_length(pairs: int, experts: int, alignment: int, length_multiple: int) -> int:
+def plan_length(pairs, experts: int, alignment: int, length_multiple: int = 1):
+    """Rows of the padded layout of `pairs` rows in groups aligned to `alignment`: a static bound, in multiples of
+    `length_multiple`, and one more where its 128s (the persistent kernel's layout) come to whole 512s.  The column-wise
+    codes have rows of this many bytes, and a weight gradient reads 128-byte pieces of 512 of them at a time: where rows
+    lie a whole number of 4 KB apart those fall on few channels of the L2 (128 experts 768 x 2048 and 2048 x 768 over
+    131 072 pairs: 265 and 267 us with 135168 rows = 33 x 4096; with 1024 more 251 and 256, 512 more 240 and 245, 256
+    more 238 and 240, 128 more 235 and 240).  (Without a branch on the length, which may be symbolic.)"""
     step = max(alignment, length_multiple)
     if step % alignment:
         raise ValueError("length_multiple must be a multiple of the alignment")
-    return -(-(pairs + alignment * experts) // step) * step
+    rows = -(-(pairs + alignment * experts) // step) * step
+    if length_multiple != WHOLE_BLOCK:
+        return rows
+    return rows + step * ((3 - rows // step % 4) // 3)
 
 
 def route_fill(selected: torch.Tensor, scores: torch.Tensor, counts: torch.Tensor, block_counts: torch.Tensor,
@@ -629,7 +637,7 @@ def route_fill(selected: torch.Tensor, scores: torch.Tensor, counts: torch.Tenso
     """The plan of `moe_route_plan` (same outputs, pos [T, k]) from `route_topk`'s, without a sort."""
     T, k = selected.shape
     E, dev = counts.numel(), selected.device
-    max_len = _plan_length(T * k, E, alignment, length_multiple)
+    max_len = plan_length(T * k, E, alignment, length_multiple)
     scores = scores.contiguous()
     offs = torch.empty(E, dtype=torch.int32, device=dev)
     src_row = torch.empty(max_len, dtype=torch.int64, device=dev)

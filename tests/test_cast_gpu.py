@@ -506,3 +506,32 @@ def test_gate_and_norm_casts_with_row_pitches_write_the_same_codes(device, R, C,
                                                ops._ptr(ct), R + pad, ops._ptr(st_), None, 1, L, ops._stream(a)) != 0
         assert lib.mx_swiglu_cast_dim0_dim1_ld(ops._ptr(a), ops._ptr(b), R, C, C, C, ops._ptr(c), C + 8, ops._ptr(s),
                                                ops._ptr(ct), R + pad, ops._ptr(st_), None, 1, L, ops._stream(a)) != 0
+
+
+@pytest.mark.parametrize("mode", ["floor", "rceil"])
+@pytest.mark.parametrize("R,C", [(32, 32), (160, 288), (224, 4992), (4096, 2048), (4096, 2080), (4096, 3072), (4096, 3104)])
+def test_gate_casts_of_few_tiles_equal_those_of_many(device, mode, R, C):
+    """Up to some hundred tiles a lane holds fewer rows, and a 32-row block's maxima come from several waves: codes and scales
+    are those of the row-major form, which always holds eight; an infinity and a NaN in one wave's rows of a block reach the
+    scales of the others."""
+    g = torch.Generator(device=device).manual_seed(R + C)
+    a, b, dg = (torch.randn(R, C, device=device, generator=g).to(torch.bfloat16) for _ in range(3))
+    a[3, 5], b[19, 7], dg[30, 9] = float("inf"), float("nan"), float("-inf")
+    L, M = ops.MX_SCALES_ROWMAJOR, ops.MX_SCALES_MFMA
+
+    def check(want, got):
+        rows, nblk = want.scales.shape
+        assert torch.equal(got.codes[:, :want.codes.shape[1]], want.codes)
+        assert torch.equal(ops.scale_unlayout(got.scales.contiguous(), rows, nblk), want.scales)
+
+    want = ops.swiglu_to_mx_dim0_dim1(a, b, mode, L)[:2]
+    for w, q in zip(want, ops.swiglu_to_mx_dim0_dim1(a, b, mode, M)[:2]):
+        check(w, q)
+    for cols in (True, False):
+        row = ops.swiglu_to_operands(a, b, mode, cols=cols)[0]
+        assert torch.equal(row.codes[:, :C], want[0].codes)
+        assert torch.equal(ops.scale_unlayout(row.scales, R, row.k // 32)[:, :C // 32], want[0].scales)
+    want, got = ops.swiglu_bwd_to_mx_dim0_dim1(dg, a, b, mode, L)[:2], ops.swiglu_bwd_to_mx_dim0_dim1(dg, a, b, mode, M)[:2]
+    for ws, qs in zip(want, got):
+        for w, q in zip(ws, qs):
+            check(w, q)

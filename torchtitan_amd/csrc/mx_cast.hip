@@ -296,6 +296,8 @@ __global__ __launch_bounds__(256) void cast_dim0_dim1_kernel(
 //                transposed tile, which leaves as 32*WAVES-byte rows.
 // All scale bytes of the tile are staged in LDS in their final order and leave as dwords
 // (whole 256-byte groups in MFMA order, padding entries included as zeros).
+// KR: rows that a lane holds, 8 as above; with 4 or 2 a wave owns 4 KR rows, the tile has as many more
+// waves, and those of a 32-row block exchange their column maxima through LDS (see with_lane_rows).
 // ------------------------------------------------------------------------------------
 __device__ __forceinline__ uint32_t lane_xor(uint32_t v, int lane, int mask) {
   return (uint32_t)__builtin_amdgcn_ds_bpermute((lane ^ mask) << 2, (int)v);
@@ -330,17 +332,17 @@ __device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w 
 
 // Quantize one lane's 8x8 patch.  FINITE = no Inf / NaN anywhere in the wave's patches: the
 // straight-line path; otherwise the general path with per-block NaN handling and clamps.
-template <int MODE, int ORDER, bool ROW, bool COL, int WAVES, bool FINITE>
-__device__ __forceinline__ void quantize_patch(u32x4 (&v)[8], const uint32_t (&mr)[8],
+template <int MODE, int ORDER, bool ROW, bool COL, int WAVES, bool FINITE, int KR>
+__device__ __forceinline__ void quantize_patch(u32x4 (&v)[KR], const uint32_t (&mr)[KR],
                                                const uint32_t (&mc)[4], uint8_t* codes_row,
                                                int64_t cols, int rows_left, bool col_ok,
                                                uint8_t* lds_codes, uint8_t* lds_st,
                                                uint8_t* lds_sr, int wave, int lane, int rl0) {
   constexpr int PITCH = 32 * WAVES + 16;
-  const int g = lane >> 4, q = lane & 15;
+  const int g = lane >> 4, q = lane & 15, band = wave * KR / 8;
   if (ROW) {
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
+    for (int k = 0; k < KR; ++k) {
       const u32x4 w = v[k];
       uint32_t sb;
       float mult;
@@ -382,43 +384,54 @@ __device__ __forceinline__ void quantize_patch(u32x4 (&v)[8], const uint32_t (&m
       const uint32_t amax = (j & 1) ? (mc[j >> 1] >> 16) : (mc[j >> 1] & 0xFFFFu);
       uint32_t sb;
       float mu;
-      u32x2 d;
+      uint32_t d[(KR + 3) / 4];  // the column's codes, row by row
       if (FINITE) {
         finite_scale<MODE>(amax, sb, mu);
-        float f[8];
+        float f[KR];
 #pragma unroll
-        for (int k = 0; k < 8; ++k)
+        for (int k = 0; k < KR; ++k)
           f[k] = ((j & 1) ? bf16_hi(v[k][j >> 1]) : bf16_lo(v[k][j >> 1])) * mu;
-        d.x = cvt2_finite<MODE, true>(f[2], f[3], cvt2_finite<MODE, false>(f[0], f[1], 0));
-        d.y = cvt2_finite<MODE, true>(f[6], f[7], cvt2_finite<MODE, false>(f[4], f[5], 0));
+#pragma unroll
+        for (int k = 0; k < KR; k += 4) {
+          const uint32_t half = cvt2_finite<MODE, false>(f[k], f[k + 1], 0);
+          if constexpr (KR >= 4) d[k / 4] = cvt2_finite<MODE, true>(f[k + 2], f[k + 3], half);
+          else d[k / 4] = half;
+        }
       } else {
         sb = scale_byte<MODE>(amax);
         mu = scale_multiplier<MODE>(sb);
-        uint32_t e[8];
+        uint32_t e[KR];
 #pragma unroll
-        for (int k = 0; k < 8; ++k)
+        for (int k = 0; k < KR; ++k)
           e[k] = (j & 1) ? (v[k][j >> 1] >> 16) : (v[k][j >> 1] & 0xFFFFu);
         if (sb != 255) {
-          float f[8];
+          float f[KR];
 #pragma unroll
-          for (int k = 0; k < 8; ++k) f[k] = __uint_as_float(e[k] << 16) * mu;
-          d.x = cvt2f<true>(f[2], f[3], cvt2f<false>(f[0], f[1], 0));
-          d.y = cvt2f<true>(f[6], f[7], cvt2f<false>(f[4], f[5], 0));
+          for (int k = 0; k < KR; ++k) f[k] = __uint_as_float(e[k] << 16) * mu;
+#pragma unroll
+          for (int k = 0; k < KR; k += 4) {
+            d[k / 4] = cvt2f<false>(f[k], f[k + 1], 0);
+            if constexpr (KR >= 4) d[k / 4] = cvt2f<true>(f[k + 2], f[k + 3], d[k / 4]);
+          }
         } else {
-          d.x = nan_block_code(e[0]) | (nan_block_code(e[1]) << 8) |
-                (nan_block_code(e[2]) << 16) | (nan_block_code(e[3]) << 24);
-          d.y = nan_block_code(e[4]) | (nan_block_code(e[5]) << 8) |
-                (nan_block_code(e[6]) << 16) | (nan_block_code(e[7]) << 24);
+#pragma unroll
+          for (int k = 0; k < KR; k += 4) {
+            d[k / 4] = nan_block_code(e[k]) | (nan_block_code(e[k + 1]) << 8);
+            if constexpr (KR >= 4) d[k / 4] |= (nan_block_code(e[k + 2]) << 16) | (nan_block_code(e[k + 3]) << 24);
+          }
         }
       }
       const int cl = 8 * q + j;
-      *reinterpret_cast<u32x2*>(lds_codes + cl * PITCH + wave * 32 + 8 * g) = d;
-      if (g == 0) {
+      uint8_t* const to = lds_codes + cl * PITCH + KR * (4 * wave + g);
+      if constexpr (KR == 8) *reinterpret_cast<u32x2*>(to) = u32x2{d[0], d[1]};
+      else if constexpr (KR == 4) *reinterpret_cast<uint32_t*>(to) = d[0];
+      else *reinterpret_cast<uint16_t*>(to) = (uint16_t)d[0];
+      if (g == 0 && (KR == 8 || wave % (8 / KR) == 0)) {
         if (ORDER == MX_SCALES_MFMA)
-          lds_st[((wave >> 1) << 8) + ((((wave & 1) << 5) + (cl & 31)) << 2) + (cl >> 5)] =
+          lds_st[((band >> 1) << 8) + ((((band & 1) << 5) + (cl & 31)) << 2) + (cl >> 5)] =
               (uint8_t)sb;
         else
-          lds_st[cl * WAVES + wave] = (uint8_t)sb;
+          lds_st[cl * WAVES + band] = (uint8_t)sb;
       }
     }
   }
@@ -517,12 +530,13 @@ __device__ __forceinline__ void swiglu_bwd2(uint32_t dg2, uint32_t a2, uint32_t 
   db2 = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f_t{db_lo, db_hi}, v2bf_t));
 }
 
-// 8 rows x 16 bytes of a bf16 matrix per lane; rows past `rows_left` and lanes past the last
+// KR rows x 16 bytes of a bf16 matrix per lane; rows past `rows_left` and lanes past the last
 // column read as zero.
-__device__ __forceinline__ void load_patch(u32x4 (&v)[8], const uint16_t* src, int64_t ld,
+template <int KR>
+__device__ __forceinline__ void load_patch(u32x4 (&v)[KR], const uint16_t* src, int64_t ld,
                                            bool col_ok, int rows_left) {
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
+  for (int k = 0; k < KR; ++k) {
     v[k] = u32x4{0, 0, 0, 0};
     if (col_ok && k < rows_left)
       v[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src + k * ld));
@@ -537,11 +551,12 @@ __device__ __forceinline__ uint32_t pack_f32(uint32_t lo, uint32_t hi) {
   const float b = __uint_as_float((hi & 0x7FFFFFFFu) > 0x7F800000u ? 0x7FC00000u : hi);
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f_t{a, b}, v2bf_t));
 }
-__device__ __forceinline__ void load_patch_f32(u32x4 (&v)[8], const float* src, int64_t ld, bool col_ok,
+template <int KR>
+__device__ __forceinline__ void load_patch_f32(u32x4 (&v)[KR], const float* src, int64_t ld, bool col_ok,
                                                int rows_left) {
-  u32x4 w[8][2];
+  u32x4 w[KR][2];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
+  for (int k = 0; k < KR; ++k) {
     w[k][0] = w[k][1] = u32x4{0, 0, 0, 0};
     if (col_ok && k < rows_left) {
       w[k][0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src + k * ld));
@@ -549,31 +564,34 @@ __device__ __forceinline__ void load_patch_f32(u32x4 (&v)[8], const float* src, 
     }
   }
 #pragma unroll
-  for (int k = 0; k < 8; ++k)
+  for (int k = 0; k < KR; ++k)
     v[k] = u32x4{pack_f32(w[k][0].x, w[k][0].y), pack_f32(w[k][0].z, w[k][0].w), pack_f32(w[k][1].x, w[k][1].y),
                  pack_f32(w[k][1].z, w[k][1].w)};
 }
 
+// Threads of a tile of 32 WAVES rows whose lanes hold KR rows each.
+__device__ __host__ constexpr int cast_threads(int waves, int kr) { return 64 * waves * 8 / kr; }
+
 // Second half of the tile kernel: block maxima, quantization and the stores of one 8 x 8 patch
 // per lane.  Ends with every wave past its reads of the shared staging buffers only after the
 // caller's next barrier.
-template <int MODE, int ORDER, bool ROW, bool COL, int WAVES>
+template <int MODE, int ORDER, bool ROW, bool COL, int WAVES, int KR>
 __device__ __forceinline__ void emit_tile(
-    u32x4 (&v)[8], uint8_t* __restrict__ codes, uint8_t* __restrict__ scales,
+    u32x4 (&v)[KR], uint8_t* __restrict__ codes, uint8_t* __restrict__ scales,
     uint8_t* __restrict__ codes_t, uint8_t* __restrict__ scales_t, uint8_t* lds_codes,
-    uint8_t* lds_st, uint8_t* lds_sr, int64_t rows, int64_t cols, int64_t nblk, int64_t ks_n,
+    uint8_t* lds_st, uint8_t* lds_sr, u32x4* lds_mc, int64_t rows, int64_t cols, int64_t nblk, int64_t ks_n,
     int64_t nblk_t, int64_t ks_n_t, int64_t r0, int64_t c0, int64_t c, int rl0, int rows_left,
     int tid, int wave, int lane, int64_t ldc, int64_t ldct, int64_t cols_out, int64_t rows_out) {
   // ldc / ldct: bytes between rows of the row-wise / column-wise codes (>= cols_out / rows_out);
   // what lies beyond the matrix was loaded as zeros and quantizes to zero codes and zero scales
   const bool col_ok = c < cols_out;
-  constexpr int TR = 32 * WAVES, TC = 128, PITCH = TR + 16;
+  constexpr int TR = 32 * WAVES, TC = 128, PITCH = TR + 16, NT = cast_threads(WAVES, KR);
   // block maxima first: they also tell whether the wave holds any Inf / NaN
-  uint32_t mr[8] = {0, 0, 0, 0, 0, 0, 0, 0}, mc[4] = {0, 0, 0, 0};
+  uint32_t mr[KR] = {}, mc[4] = {0, 0, 0, 0};
   uint32_t top = 0;
   if (ROW) {
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
+    for (int k = 0; k < KR; ++k) {
       const u32x4 w = v[k];
       uint32_t m = pk_max_u16(pk_max_u16(w.x & 0x7FFF7FFFu, w.y & 0x7FFF7FFFu),
                               pk_max_u16(w.z & 0x7FFF7FFFu, w.w & 0x7FFF7FFFu));
@@ -586,7 +604,7 @@ __device__ __forceinline__ void emit_tile(
   }
   if (COL) {
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
+    for (int k = 0; k < KR; ++k) {
       mc[0] = pk_max_u16(mc[0], v[k].x & 0x7FFF7FFFu);
       mc[1] = pk_max_u16(mc[1], v[k].y & 0x7FFF7FFFu);
       mc[2] = pk_max_u16(mc[2], v[k].z & 0x7FFF7FFFu);
@@ -597,20 +615,32 @@ __device__ __forceinline__ void emit_tile(
       mc[i] = pk_max_u16(mc[i], lane_xor(mc[i], lane, 16));
       mc[i] = pk_max_u16(mc[i], lane_xor(mc[i], lane, 32));
     }
-    if (!ROW) {
+    if constexpr (KR < 8) {  // a 32-row block's maxima are those of its 8 / KR waves
+      constexpr int PER = 8 / KR;
+      const int q = lane & 15;
+      if (lane < 16) lds_mc[wave * 16 + q] = u32x4{mc[0], mc[1], mc[2], mc[3]};
+      __syncthreads();
+#pragma unroll
+      for (int p = 0; p < PER; ++p) {
+        const u32x4 o = lds_mc[(wave / PER * PER + p) * 16 + q];
+        mc[0] = pk_max_u16(mc[0], o.x);
+        mc[1] = pk_max_u16(mc[1], o.y);
+        mc[2] = pk_max_u16(mc[2], o.z);
+        mc[3] = pk_max_u16(mc[3], o.w);
+      }
+    }
+    if (!ROW || KR < 8) {
       const uint32_t t = pk_max_u16(pk_max_u16(mc[0], mc[1]), pk_max_u16(mc[2], mc[3]));
-      top = max(t & 0xFFFFu, t >> 16);
+      top = max(top, max(t & 0xFFFFu, t >> 16));
     }
   }
   uint8_t* codes_row = ROW ? codes + (r0 + rl0) * ldc + c : nullptr;
   if (__builtin_amdgcn_ballot_w64(top >= 0x7F80u) == 0)
-    quantize_patch<MODE, ORDER, ROW, COL, WAVES, true>(v, mr, mc, codes_row, ldc, rows_left,
-                                                       col_ok, lds_codes, lds_st, lds_sr, wave,
-                                                       lane, rl0);
+    quantize_patch<MODE, ORDER, ROW, COL, WAVES, true, KR>(v, mr, mc, codes_row, ldc, rows_left, col_ok, lds_codes,
+                                                           lds_st, lds_sr, wave, lane, rl0);
   else
-    quantize_patch<MODE, ORDER, ROW, COL, WAVES, false>(v, mr, mc, codes_row, ldc, rows_left,
-                                                        col_ok, lds_codes, lds_st, lds_sr, wave,
-                                                        lane, rl0);
+    quantize_patch<MODE, ORDER, ROW, COL, WAVES, false, KR>(v, mr, mc, codes_row, ldc, rows_left, col_ok, lds_codes,
+                                                            lds_st, lds_sr, wave, lane, rl0);
   __syncthreads();
 
   if (ROW && tid < TR) {
@@ -634,8 +664,8 @@ __device__ __forceinline__ void emit_tile(
     constexpr int SEGS = TR / 16;  // 16-byte pieces of one transposed row
     const int seg = tid % SEGS;
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const int o = p * 32 + tid / SEGS;
+    for (int p = 0; p < TC * SEGS / NT; ++p) {
+      const int o = p * (NT / SEGS) + tid / SEGS;
       if (c0 + o < cols && r0 + seg * 16 < rows_out) {
         const u32x4 t = *reinterpret_cast<const u32x4*>(lds_codes + o * PITCH + seg * 16);
 #ifdef MX_ABL_COL_UNTRANSPOSED  // timing ablation: the column-wise codes go out as rows of the input
@@ -679,30 +709,31 @@ __device__ __forceinline__ void emit_tile(
 __device__ __forceinline__ uint32_t scale2(uint32_t w, float s) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f_t{bf16_lo(w) * s, bf16_hi(w) * s}, v2bf_t));
 }
-__device__ __forceinline__ void load_patch_rows(u32x4 (&v)[8], const uint16_t* x, int64_t ld,
+template <int KR>
+__device__ __forceinline__ void load_patch_rows(u32x4 (&v)[KR], const uint16_t* x, int64_t ld,
                                                 int64_t c, const int64_t* row_idx, int64_t src_rows,
                                                 const float* row_scale, bool col_ok, int rows_left) {
   if (!col_ok || rows_left <= 0 || src_rows <= 0) {
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = u32x4{0, 0, 0, 0};
+    for (int k = 0; k < KR; ++k) v[k] = u32x4{0, 0, 0, 0};
     return;
   }
-  int64_t r[8];
-  float s[8];
-  bool in[8];
+  int64_t r[KR];
+  float s[KR];
+  bool in[KR];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
+  for (int k = 0; k < KR; ++k) {
     const int at = k < rows_left ? k : 0;
     r[k] = row_idx[at];
     s[k] = row_scale ? row_scale[at] : 1.0f;
   }
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
+  for (int k = 0; k < KR; ++k) {
     in[k] = k < rows_left && r[k] >= 0 && r[k] < src_rows;
     v[k] = *reinterpret_cast<const u32x4*>(x + (in[k] ? r[k] : 0) * ld + c);
   }
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
+  for (int k = 0; k < KR; ++k) {
     if (row_scale)
       v[k] = u32x4{scale2(v[k].x, s[k]), scale2(v[k].y, s[k]), scale2(v[k].z, s[k]), scale2(v[k].w, s[k])};
     if (!in[k]) v[k] = u32x4{0, 0, 0, 0};
@@ -727,8 +758,8 @@ struct TileExtras {
 };
 
 // The gate-backward variant is bound by vector ALU work: four workgroups per CU (128 VGPRs).
-template <int MODE, int ORDER, bool ROW, bool COL, int WAVES, int GATE, bool GATHER, bool F32 = false>
-__global__ __launch_bounds__(64 * WAVES, GATE == 2 ? 4 : 1) void cast_tile_kernel(
+template <int MODE, int ORDER, bool ROW, bool COL, int WAVES, int GATE, bool GATHER, bool F32 = false, int KR = 8>
+__global__ __launch_bounds__(cast_threads(WAVES, KR), GATE == 2 && KR == 8 ? 4 : 1) void cast_tile_kernel(
     const uint16_t* __restrict__ x, int64_t rows, int64_t cols, int64_t ldx,
     uint8_t* __restrict__ codes, uint8_t* __restrict__ scales, int64_t nblk, int64_t ks_n,
     uint8_t* __restrict__ codes_t, uint8_t* __restrict__ scales_t, int64_t nblk_t,
@@ -743,7 +774,8 @@ __global__ __launch_bounds__(64 * WAVES, GATE == 2 ? 4 : 1) void cast_tile_kerne
   __shared__ __attribute__((aligned(16))) uint8_t lds_st[COL ? TC * WAVES : 16];
   __shared__ __attribute__((aligned(16))) uint8_t lds_sr[ROW ? TR * 4 : 16];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, q = lane & 15;
-  const int rl0 = wave * 32 + 8 * g;  // first tile-local row of this lane
+  __shared__ u32x4 lds_mc[COL && KR < 8 ? cast_threads(WAVES, KR) / 4 : 1];
+  const int rl0 = KR * (4 * wave + g);  // first tile-local row of this lane
 
   // a batch of independent [rows, cols] matrices is walked as one stack of gy * batch tile rows
   uint32_t bx, by_all;
@@ -765,9 +797,9 @@ __global__ __launch_bounds__(64 * WAVES, GATE == 2 ? 4 : 1) void cast_tile_kerne
   const int64_t c = c0 + 8 * q;
   const bool col_ok = c < cols;
   const int64_t left64 = rows - (r0 + rl0);
-  const int rows_left = left64 > 8 ? 8 : (left64 < 0 ? 0 : (int)left64);
+  const int rows_left = left64 > KR ? KR : (left64 < 0 ? 0 : (int)left64);
 
-  u32x4 v[8];
+  u32x4 v[KR];
   if constexpr (GATHER)
     load_patch_rows(v, x, ldx, c, ex.row_idx + r0 + rl0, ex.src_rows,
                     ex.row_scale ? ex.row_scale + r0 + rl0 : nullptr, col_ok, rows_left);
@@ -776,10 +808,10 @@ __global__ __launch_bounds__(64 * WAVES, GATE == 2 ? 4 : 1) void cast_tile_kerne
   else
     load_patch(v, x + (r0 + rl0) * ldx + c, ldx, col_ok, rows_left);
   if constexpr (GATE == 1) {  // x = gate input a, x3 = b: quantize g = silu(a) * b
-    u32x4 b[8];
+    u32x4 b[KR];
     load_patch(b, x3 + (r0 + rl0) * ldx3 + c, ldx3, col_ok, rows_left);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
+    for (int k = 0; k < KR; ++k) {
       v[k] = u32x4{swiglu2(v[k].x, b[k].x), swiglu2(v[k].y, b[k].y), swiglu2(v[k].z, b[k].z),
                    swiglu2(v[k].w, b[k].w)};
       if (g_out && col_ok && k < rows_left)
@@ -794,7 +826,7 @@ __global__ __launch_bounds__(64 * WAVES, GATE == 2 ? 4 : 1) void cast_tile_kerne
     const float w8[8] = {bf16_lo(wv.x), bf16_hi(wv.x), bf16_lo(wv.y), bf16_hi(wv.y),
                          bf16_lo(wv.z), bf16_hi(wv.z), bf16_lo(wv.w), bf16_hi(wv.w)};
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
+    for (int k = 0; k < KR; ++k) {
       if (col_ok && k < rows_left) {
         const float rs = ex.row_scale[r0 + rl0 + k];
         const uint32_t d[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
@@ -810,13 +842,13 @@ __global__ __launch_bounds__(64 * WAVES, GATE == 2 ? 4 : 1) void cast_tile_kerne
   }
   if constexpr (GATE == 2) {
     // backward of the gate: x = a, x3 = b, x4 = dg; two stacked outputs, d/da then d/db
-    u32x4 w[8];
+    u32x4 w[KR];
     {
-      u32x4 b[8], dg[8];
+      u32x4 b[KR], dg[KR];
       load_patch(b, x3 + (r0 + rl0) * ldx3 + c, ldx3, col_ok, rows_left);
       load_patch(dg, x4 + (r0 + rl0) * ldx4 + c, ldx4, col_ok, rows_left);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
+      for (int k = 0; k < KR; ++k) {
         uint32_t da[4], db[4];
         swiglu_bwd2(dg[k].x, v[k].x, b[k].x, da[0], db[0]);
         swiglu_bwd2(dg[k].y, v[k].y, b[k].y, da[1], db[1]);
@@ -831,7 +863,7 @@ __global__ __launch_bounds__(64 * WAVES, GATE == 2 ? 4 : 1) void cast_tile_kerne
       }
     }
     emit_tile<MODE, ORDER, ROW, COL, WAVES>(w, codes, scales, codes_t, scales_t, lds_codes, lds_st,
-                                            lds_sr, rows, cols, nblk, ks_n, nblk_t, ks_n_t, r0, c0,
+                                            lds_sr, lds_mc, rows, cols, nblk, ks_n, nblk_t, ks_n_t, r0, c0,
                                             c, rl0, rows_left, tid, wave, lane, ldc, ldct, cols_out, rows_out);
     __syncthreads();  // the staging buffers are reused by the second output
     if (ROW) {
@@ -844,7 +876,7 @@ __global__ __launch_bounds__(64 * WAVES, GATE == 2 ? 4 : 1) void cast_tile_kerne
     }
   }
   emit_tile<MODE, ORDER, ROW, COL, WAVES>(v, codes, scales, codes_t, scales_t, lds_codes, lds_st,
-                                          lds_sr, rows, cols, nblk, ks_n, nblk_t, ks_n_t, r0, c0, c,
+                                          lds_sr, lds_mc, rows, cols, nblk, ks_n, nblk_t, ks_n_t, r0, c0, c,
                                           rl0, rows_left, tid, wave, lane, ldc, ldct, cols_out, rows_out);
 }
 
@@ -895,7 +927,7 @@ __global__ __launch_bounds__(64 * WAVES) void cast_list_kernel(CastList list, in
   const int64_t nblk = cols_out / 32, nblk_t = rows_out / 32;
   emit_tile<MODE, MX_SCALES_MFMA, true, true, WAVES>(
       v, e.codes + bz * rows * e.ldc, e.scales + bz * e.s_bstride, e.codes_t + bz * cols * e.ldct,
-      e.scales_t + bz * e.st_bstride, lds_codes, lds_st, lds_sr, rows, cols, nblk, nblk / 2, nblk_t, nblk_t / 2, r0, c0,
+      e.scales_t + bz * e.st_bstride, lds_codes, lds_st, lds_sr, nullptr, rows, cols, nblk, nblk / 2, nblk_t, nblk_t / 2, r0, c0,
       c, rl0, rows_left, tid, wave, lane, e.ldc, e.ldct, cols_out, rows_out);
 }
 
@@ -964,24 +996,49 @@ using namespace mx;
 #define MX_CAST_WAVES 4
 #endif
 #define MX_DISPATCH_TILE(ROW, COL, GATE, GATHER, ...)                                                         \
-  do {                                                                                           \
-    if (scale_mode == MX_SCALE_FLOOR && scale_order == MX_SCALES_ROWMAJOR)                       \
-      hipLaunchKernelGGL(                                                                        \
-          (cast_tile_kernel<MX_SCALE_FLOOR, MX_SCALES_ROWMAJOR, ROW, COL, MX_CAST_WAVES, GATE, GATHER>), grid, \
-          block, 0, st, __VA_ARGS__);                                                            \
-    else if (scale_mode == MX_SCALE_FLOOR)                                                       \
-      hipLaunchKernelGGL(                                                                        \
-          (cast_tile_kernel<MX_SCALE_FLOOR, MX_SCALES_MFMA, ROW, COL, MX_CAST_WAVES, GATE, GATHER>), grid,     \
-          block, 0, st, __VA_ARGS__);                                                            \
-    else if (scale_order == MX_SCALES_ROWMAJOR)                                                  \
-      hipLaunchKernelGGL(                                                                        \
-          (cast_tile_kernel<MX_SCALE_RCEIL, MX_SCALES_ROWMAJOR, ROW, COL, MX_CAST_WAVES, GATE, GATHER>), grid, \
-          block, 0, st, __VA_ARGS__);                                                            \
-    else                                                                                         \
-      hipLaunchKernelGGL(                                                                        \
-          (cast_tile_kernel<MX_SCALE_RCEIL, MX_SCALES_MFMA, ROW, COL, MX_CAST_WAVES, GATE, GATHER>), grid,     \
-          block, 0, st, __VA_ARGS__);                                                            \
+  do {                                                                                                        \
+    with_lane_rows<GATE, COL>(scale_order == MX_SCALES_MFMA ? (int64_t)grid.x : INT64_MAX, [&](auto kr) {          \
+      constexpr int KR = decltype(kr)::value;                                                                 \
+      block = dim3(cast_threads(MX_CAST_WAVES, KR));                                                          \
+      if constexpr (KR == 8) {                                                                                \
+        if (scale_order == MX_SCALES_ROWMAJOR) {                                                              \
+          if (scale_mode == MX_SCALE_FLOOR)                                                                   \
+            hipLaunchKernelGGL((cast_tile_kernel<MX_SCALE_FLOOR, MX_SCALES_ROWMAJOR, ROW, COL, MX_CAST_WAVES, \
+                                                 GATE, GATHER>), grid, block, 0, st, __VA_ARGS__);            \
+          else                                                                                                \
+            hipLaunchKernelGGL((cast_tile_kernel<MX_SCALE_RCEIL, MX_SCALES_ROWMAJOR, ROW, COL, MX_CAST_WAVES, \
+                                                 GATE, GATHER>), grid, block, 0, st, __VA_ARGS__);            \
+          return;                                                                                             \
+        }                                                                                                     \
+      }                                                                                                       \
+      if (scale_mode == MX_SCALE_FLOOR)                                                                       \
+        hipLaunchKernelGGL((cast_tile_kernel<MX_SCALE_FLOOR, MX_SCALES_MFMA, ROW, COL, MX_CAST_WAVES, GATE,   \
+                                             GATHER, false, KR>), grid, block, 0, st, __VA_ARGS__);           \
+      else                                                                                                    \
+        hipLaunchKernelGGL((cast_tile_kernel<MX_SCALE_RCEIL, MX_SCALES_MFMA, ROW, COL, MX_CAST_WAVES, GATE,   \
+                                             GATHER, false, KR>), grid, block, 0, st, __VA_ARGS__);           \
+    });                                                                                                       \
   } while (0)
+
+// Calls `launch` with the rows that a lane holds (8, 4 or 2 of a tile's 128 x 128 values over 4, 8 or 16 waves), by the
+// tiles of the launch.  A gate is a chain of some hundred instructions a value: with a tile or two per CU its SIMDs
+// wait for one wave's chain, which more and shorter waves fill.  us, 8 rows and fewer (bf16, after other kernels):
+//   tiles          both directions, forward   backward       row-wise alone
+//   32             9.0   7.8                  15.0   13.0     7.7   5.5
+//   512           15.8  14.0                  26.4   23.7    13.6  10.1
+//   768           19.3  18.1                  33.2   33.5    16.7  15.0
+//   1024          25.8  26.9                  43.9   49.4    20.8  19.1
+//   1536          35.2  36.0                  60.6   62.8    28.6  27.3
+//   14336          264   264                   475    514     209   225
+// Beyond that bandwidth decides, and fewer bytes are asked for at a time.  (The plain casts gain nothing: 5.2 us and 5.3
+// of 256 x 2048; nor does one copy of the backward's code for both outputs, in a loop: 13 -> 27 us, spilled.)
+template <int GATE, bool COL, class F>
+static inline void with_lane_rows(int64_t tiles, F launch) {
+  if constexpr (GATE == 1 || GATE == 2) {
+    if (tiles <= (!COL ? 2048 : GATE == 1 ? 768 : 512)) return launch(std::integral_constant<int, COL ? 4 : 2>{});
+  }
+  launch(std::integral_constant<int, 8>{});
+}
 
 // The tile kernel loads 16 bytes (8 columns) per lane.
 static inline bool tile_ok(const void* x, int64_t cols, int64_t ldx) {
@@ -1040,7 +1097,7 @@ extern "C" int mx_cast_dim0(const void* x, int64_t rows, int64_t cols, int64_t l
   const int64_t tgx = (cols + kT - 1) / kT, tgy = (rows + kTileRows - 1) / kTileRows;
   if (scale_order == MX_SCALES_MFMA && tile_grid_x(tgx, tgy) <= 0x7FFFFFFF) {
     // scattered scale bytes cost more than the tiled read: stage them through LDS
-    dim3 grid = tile_grid(tgx, tgy, 1), block(64 * MX_CAST_WAVES);
+    dim3 grid = tile_grid(tgx, tgy, 1), block;
     MX_DISPATCH_TILE(true, false, 0, false, (const uint16_t*)x, rows, cols, ldx, codes, scales, nblk,
                      ks_n, (uint8_t*)nullptr, (uint8_t*)nullptr, (int64_t)0, (int64_t)0, (int64_t)0,
                      (int64_t)0, (int64_t)0, (uint32_t)tgx, (uint32_t)tgy, TileExtras{});
@@ -1074,7 +1131,7 @@ extern "C" int mx_cast_dim1_batched(const void* x, int64_t batch, int64_t rows, 
   hipStream_t st = (hipStream_t)stream;
   const int64_t tgy = (rows + kTileRows - 1) / kTileRows;
   if (tile_ok(x, cols, ldx) && tile_grid_x(gx, tgy * batch) <= 0x7FFFFFFF) {
-    dim3 grid = tile_grid(gx, tgy, batch), block(64 * MX_CAST_WAVES);
+    dim3 grid = tile_grid(gx, tgy, batch), block;
     MX_DISPATCH_TILE(false, true, 0, false, (const uint16_t*)x, rows, cols, ldx, (uint8_t*)nullptr,
                      (uint8_t*)nullptr, (int64_t)0, (int64_t)0, codes_t, scales_t, nblk_t, ks_n_t,
                      rows * ldx, (int64_t)0, st_b, (uint32_t)gx, (uint32_t)tgy,
@@ -1116,7 +1173,7 @@ extern "C" int mx_cast_dim0_dim1_batched(const void* x, int64_t batch, int64_t r
   const int64_t tgy = (rows + kTileRows - 1) / kTileRows;
   if (tile_ok(x, cols, ldx) && ((uintptr_t)codes & 7) == 0 && ((uintptr_t)scales & 3) == 0 &&
       tile_grid_x(gx, tgy * batch) <= 0x7FFFFFFF) {
-    dim3 grid = tile_grid(gx, tgy, batch), block(64 * MX_CAST_WAVES);
+    dim3 grid = tile_grid(gx, tgy, batch), block;
     MX_DISPATCH_TILE(true, true, 0, false, (const uint16_t*)x, rows, cols, ldx, codes, scales, nblk,
                      ks_n, codes_t, scales_t, nblk_t, ks_n_t, rows * ldx, s_b, st_b, (uint32_t)gx,
                      (uint32_t)tgy, tile_batch(batch));
@@ -1158,7 +1215,7 @@ extern "C" int mx_cast_dim0_dim1_ld(const void* x, int64_t rows, int64_t cols, i
   // only the tile kernel knows pitches: inputs it does not take are the caller's dense cast
   if (!tile_ok(x, cols, ldx) || tile_grid_x(gx, tgy) > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
-  dim3 grid = tile_grid(gx, tgy, 1), block(64 * MX_CAST_WAVES);
+  dim3 grid = tile_grid(gx, tgy, 1), block;
   TileExtras ex = tile_batch(1);
   ex.ldc = ld_codes;
   ex.ldct = ld_codes_t;
@@ -1225,7 +1282,7 @@ extern "C" int mx_cast_rows_gathered(const void* x, const int64_t* row_index,
   const int64_t gx = (cols + kT - 1) / kT, tgy = (rows + kTileRows - 1) / kTileRows;
   if (tile_grid_x(gx, tgy) > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
-  dim3 grid = tile_grid(gx, tgy, 1), block(64 * MX_CAST_WAVES);
+  dim3 grid = tile_grid(gx, tgy, 1), block;
   TileExtras ex;
   ex.row_idx = row_index;
   ex.src_rows = src_rows;
@@ -1298,7 +1355,7 @@ extern "C" int mx_rmsnorm_cast_dim0_dim1_ld(const void* x, const void* weight, f
   hipStream_t st = (hipStream_t)stream;
   hipLaunchKernelGGL(rms_rstd_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st,
                      (const uint16_t*)x, rows, cols, ldx, eps, rstd);
-  dim3 grid = tile_grid(gx, tgy, 1), block(64 * MX_CAST_WAVES);
+  dim3 grid = tile_grid(gx, tgy, 1), block;
   TileExtras ex;
   ex.x3 = (const uint16_t*)weight;
   ex.g_out = (uint16_t*)y;
@@ -1340,7 +1397,7 @@ extern "C" int mx_swiglu_cast_dim0_dim1_ld(const void* a, const void* b, int64_t
   const int64_t gx = (cols + kT - 1) / kT, tgy = (rows + kTileRows - 1) / kTileRows;
   if (tile_grid_x(gx, tgy) > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
-  dim3 grid = tile_grid(gx, tgy, 1), block(64 * MX_CAST_WAVES);
+  dim3 grid = tile_grid(gx, tgy, 1), block;
   TileExtras ex{(const uint16_t*)b, ldb, (uint16_t*)g, nullptr, 0, nullptr, 0};
   ex.ldc = ld_codes;
   ex.ldct = ld_codes_t;
@@ -1383,7 +1440,7 @@ extern "C" int mx_swiglu_bwd_cast_dim0_dim1_ld(const void* dg, const void* a, co
   const int64_t gx = (cols + kT - 1) / kT, tgy = (rows + kTileRows - 1) / kTileRows;
   if (tile_grid_x(gx, tgy) > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
-  dim3 grid = tile_grid(gx, tgy, 1), block(64 * MX_CAST_WAVES);
+  dim3 grid = tile_grid(gx, tgy, 1), block;
   TileExtras ex{(const uint16_t*)b, ldb, (uint16_t*)dab, (const uint16_t*)dg, lddg, nullptr, 0};
   ex.ldc = ld_codes;
   ex.ldct = ld_codes_t;
@@ -1427,7 +1484,7 @@ struct PadOut {
 
 struct PadPlan {
   int64_t nblk, ks_n, nblk_t, ks_n_t, gx, gy;
-  dim3 grid, block;
+  dim3 grid;
   TileExtras ex;
 };
 
@@ -1446,7 +1503,6 @@ int pad_plan(int64_t rows, int64_t cols, const PadOut& o, PadPlan& p) {
   p.gy = (rows + kTileRows - 1) / kTileRows;
   if (tile_grid_x(p.gx, p.gy) > 0x7FFFFFFF) return MX_ERR_UNSUPPORTED;
   p.grid = tile_grid(p.gx, p.gy, 1);
-  p.block = dim3(64 * MX_CAST_WAVES);
   p.ex = tile_batch(1);
   p.ex.ldc = o.ld;
   p.ex.ldct = o.ld_t;
@@ -1459,15 +1515,18 @@ template <bool ROW, bool COL, int GATE, bool F32 = false>
 int launch_pad(const void* x, int64_t rows, int64_t cols, int64_t ldx, const PadOut& o, const PadPlan& p,
                int scale_mode, hipStream_t st) {
   const int64_t s_b = mfma_scale_bytes(rows, p.nblk), st_b = mfma_scale_bytes(cols, p.nblk_t);
-  auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, p.grid, p.block, 0, st, (const uint16_t*)x, rows, cols, ldx, o.codes, o.scales, p.nblk,
+  auto go = [&](auto kern, int threads) {
+    hipLaunchKernelGGL(kern, p.grid, dim3(threads), 0, st, (const uint16_t*)x, rows, cols, ldx, o.codes, o.scales, p.nblk,
                        p.ks_n, o.codes_t, o.scales_t, p.nblk_t, p.ks_n_t, (int64_t)0, s_b, st_b, (uint32_t)p.gx,
                        (uint32_t)p.gy, p.ex);
   };
-  if (scale_mode == MX_SCALE_FLOOR)
-    go(cast_tile_kernel<MX_SCALE_FLOOR, MX_SCALES_MFMA, ROW, COL, MX_CAST_WAVES, GATE, false, F32>);
-  else
-    go(cast_tile_kernel<MX_SCALE_RCEIL, MX_SCALES_MFMA, ROW, COL, MX_CAST_WAVES, GATE, false, F32>);
+  with_lane_rows<GATE, COL>(p.gx * p.gy, [&](auto kr) {
+    constexpr int KR = decltype(kr)::value, kThreads = cast_threads(MX_CAST_WAVES, KR);
+    if (scale_mode == MX_SCALE_FLOOR)
+      go(cast_tile_kernel<MX_SCALE_FLOOR, MX_SCALES_MFMA, ROW, COL, MX_CAST_WAVES, GATE, false, F32, KR>, kThreads);
+    else
+      go(cast_tile_kernel<MX_SCALE_RCEIL, MX_SCALES_MFMA, ROW, COL, MX_CAST_WAVES, GATE, false, F32, KR>, kThreads);
+  });
   return launch_status();
 }
 

@@ -1061,3 +1061,52 @@ def test_blocks_of_any_size_under_torch_compile_equal_eager(device, tokens, dim,
             results.append([y.detach(), *(torch.autograd.grad(y, ins, dy) if ins else ())])
         assert all(torch.equal(a, b) for a, b in zip(*results, strict=True)), wanted
     torch._dynamo.reset()
+
+
+@pytest.mark.parametrize("dim,hidden", [(1024, 2048), (160, 224)])
+@pytest.mark.parametrize("tokens", [5, 96, 384])
+def test_frozen_cached_weights_are_cast_once_with_rows_apart(device, dim, hidden, tokens):
+    """Forwards without gradients on frozen weights read the entry that the hook made, eagerly and (whole blocks) traced,
+    with the outputs of weights that are not cached; the hand-over and a training step behind them find what they need."""
+    import torch._dynamo
+    from torchtitan_amd import mx_tensor
+    from torchtitan_amd.quantization.mx import export_mxfp8_state_dict
+
+    mx_tensor._weight_cache.clear()
+    holders, boxes = [], []
+    for cache in (False, True):
+        holder = nn.Module()
+        holder.ff = FeedForward.Config(hidden_dim=hidden).build(dim=dim).to(device).to(torch.bfloat16)
+        if holders:
+            holder.load_state_dict(holders[0].state_dict())
+        else:
+            holder.ff.init_weights(init_std=0.05)
+        boxes.append(_convert(holder, ["ff"], cache=cache))
+        holders.append(holder.requires_grad_(False))
+    plain, cached = (h.ff for h in holders)
+    boxes[1].post_optimizer_hook(holders[1])
+    entries = lambda: {k: id(e[5]) for k, e in mx_tensor._weight_cache._entries.items()}
+    made = entries()
+    assert len(made) == 3 and all(e[5].ld == e[5].k + ops.CODE_PITCH_PAD and e[6] is None
+                                  for e in mx_tensor._weight_cache._entries.values())
+    x = torch.randn(tokens, dim, device=device).to(torch.bfloat16)
+    with torch.no_grad():
+        assert torch.equal(cached(x), plain(x)) and torch.equal(cached.w1(x), plain.w1(x))
+        if dim % 128 == 0 and tokens % 32 == 0:
+            torch._dynamo.reset()
+            compiled = torch.compile(lambda t: (cached(t), cached.w1(t)), backend="aot_eager", fullgraph=True)
+            y, h = compiled(x)
+            assert torch.equal(y, plain(x)) and torch.equal(h, plain.w1(x))
+            torch._dynamo.reset()
+    want, got = export_mxfp8_state_dict(holders[0]), export_mxfp8_state_dict(holders[1])
+    for name in want:
+        assert got[name]["codes"].is_contiguous()
+        assert torch.equal(got[name]["codes"], want[name]["codes"]) and torch.equal(got[name]["scales"], want[name]["scales"])
+    assert entries() == made  # nothing was cast again
+    outs = []
+    for h in holders:
+        xs = x.clone().requires_grad_(True)
+        y = h.requires_grad_(True).ff(xs)
+        outs.append((y, *torch.autograd.grad(y, [xs, *h.parameters()], torch.ones_like(y))))
+    assert all(torch.equal(a, b) for a, b in zip(*outs, strict=True))
+    mx_tensor._weight_cache.clear()

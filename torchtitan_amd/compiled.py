@@ -54,7 +54,7 @@ def mx_linear_fwd(x: torch.Tensor, weight: torch.Tensor, mode: int, need_dx: boo
     (codes [K, M], MFMA-order scales; empty unless `need_dw`) and of W (codes [K, N], MFMA-order
     scales; empty unless `need_dx`).  Without gradients only the row-wise casts run.  `cache_w`:
     the weight's casts come from, and go to, the cache of unchanged weights."""
-    from .mx_tensor import _cast_weight
+    from .mx_tensor import _cast_weight, _rounded_up, frozen_rows
 
     M, K, N = _dims(x, weight)
     name = _MODE_NAMES[mode]
@@ -62,6 +62,10 @@ def mx_linear_fwd(x: torch.Tensor, weight: torch.Tensor, mode: int, need_dx: boo
     if x2.dtype != torch.bfloat16:
         x2 = x2.to(torch.bfloat16)
     x2 = x2.contiguous()
+    frozen = frozen_rows(weight, name) if cache_w and not (need_dx or need_dw or _rounded_up(weight)) else None
+    if frozen is not None:
+        y = ops.mx_gemm_nt(ops.to_operands(x2, name, True, False, frozen.ld - frozen.k)[0], frozen)
+        return (y.view(*x.shape[:-1], N), *(_empty(x.device) for _ in range(4)))
     if need_dw:
         xq0, xq1 = ops.to_mx_dim0_dim1(x2, name, MX_SCALES_MFMA)
     else:

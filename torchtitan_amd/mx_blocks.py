@@ -13,7 +13,7 @@ import torch.nn.functional as F
 from . import _lib, ops
 from .mx_tensor import (MXFP8Config, MXFP8TrainingWeight, _cast_activation, _cast_activation_and_weights, _cast_cache,
                         _cast_into_groups, _cast_weight, _cast_weights, _castable, _grouped_2d3d_padded, _one_launch,
-                        _pad_plan, _unwrap)
+                        _pad_plan, _rounded_up, _unwrap, frozen_rows, rows_apart)
 from .ops import MX_SCALES_MFMA, MX_SCALES_ROWMAJOR, MXData
 
 # ----------------------------------------------------------------------------- SwiGLU + linear
@@ -150,6 +150,9 @@ def ffn_forward(x2, x_src, w1, w2, w3, cfg: MXFP8Config, need_dx: bool, need_dw:
     with sibling linears); `pad`: the row pitch padding of every code matrix (the saved ones
     carry it into the backward); `whole_blocks`: see `_FFNCasts`.  The eager autograd function and
     the traced operator both run this."""
+    if (x_src is None and cfg.cache_weight_casts and not (need_dx or need_dw)
+            and not any(_rounded_up(w) or frozen_rows(w, cfg.scale_mode) is None for w in (w1, w2, w3))):
+        whole_blocks, pad = True, ops.CODE_PITCH_PAD  # (traced, behind a hook that has cast frozen weights)
     cast = _FFNCasts(cfg, whole_blocks, pad)
     if (whole_blocks and norm_weight is None and not (need_dx or need_dw)
             and ops.few_rows_ok(x2, w1.shape[0] + w3.shape[0])):
@@ -301,8 +304,9 @@ def _feed_forward(x, w1, w2, w3, bias2, norm_weight, eps: float):
         if torch.is_grad_enabled() or ops._transformed():
             y = _MXFeedForward.apply(x, w1, w2, w3, w2.mx_config, norm_weight, eps)
         else:  # nothing is kept for a backward
-            y, _ = ffn_forward(_rows_of(x), x, w1, w2, w3, w2.mx_config, False, False, norm_weight, eps,
-                               whole_blocks=True)
+            cfg = w2.mx_config
+            pad = rows_apart(cfg, not (w1.requires_grad or w2.requires_grad or w3.requires_grad))
+            y, _ = ffn_forward(_rows_of(x), x, w1, w2, w3, cfg, False, False, norm_weight, eps, pad=pad, whole_blocks=True)
             y = y if x.dim() == 2 else y.view(*x.shape[:-1], w2.shape[0])
         if bias2 is not None:
             y = y + bias2.to(y.dtype)

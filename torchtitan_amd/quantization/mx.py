@@ -20,7 +20,7 @@ import torch.nn as nn
 
 from .. import _lib
 from ..modules.linear import Linear
-from ..mx_tensor import MXFP8Config, MXFP8TrainingWeight, _cast_weight, wrap_parameter
+from ..mx_tensor import MXFP8Config, MXFP8TrainingWeight, _cast_weight, frozen_rows, rows_apart, wrap_parameter
 from . import QuantizationConverter
 from .module_utils import capture_module_attrs, inject_module_protocol, verify_module_protocol
 from .utils import module_filter_fn
@@ -185,8 +185,10 @@ class MXFP8Converter(QuantizationConverter):
         for m in model if isinstance(model, (list, tuple)) else [model]:
             for p in m.parameters():
                 if isinstance(p, MXFP8TrainingWeight) and p.is_cuda:
+                    # frozen weights for forwards without gradients alone: row-wise, rows apart
+                    pad = rows_apart(p.mx_config, not p.requires_grad) if p.dim() == 2 else 0
                     with torch.no_grad():
-                        _cast_weight(p.as_subclass(torch.Tensor), p.mx_config.scale_mode, True, p.mx_config)
+                        _cast_weight(p.as_subclass(torch.Tensor), p.mx_config.scale_mode, not pad, p.mx_config, pad)
 
 
 MXFP8_PAYLOAD_FORMAT = "mxfp8:e4m3fn+e8m0:block32:dim-1"
@@ -230,7 +232,9 @@ def _rows_from_cache(p: torch.Tensor, cfg: MXFP8Config):
     is none)."""
     from .. import ops
 
-    rows, _ = _cast_weight(p, cfg.scale_mode, False, cfg)
+    rows = frozen_rows(p, cfg.scale_mode) if not p.requires_grad else None
+    if rows is None:
+        rows, _ = _cast_weight(p, cfg.scale_mode, False, cfg)
     codes, laid = rows.codes, rows.scales
     lead, K = p.shape[:-1], p.shape[-1]
     nblk = K // 32

@@ -408,3 +408,40 @@ def test_errors_keep_their_types(device, monkeypatch):
     with pytest.raises(_lib.MXLibraryError, match="mx_cast_pad_many"):
         blocks.linear_forward(x.detach(), w, 7, 128)  # no such scale mode
     assert torch.isfinite(lin(x)).all()
+
+
+@pytest.mark.parametrize("form", ["plain", "rows of a wider matrix", "rows that are not aligned", "columns first"])
+def test_single_launches(device, monkeypatch, form):
+    """The gate, the routing, the log-probabilities and the hand-over's lists through the native module and step by step:
+    the same outputs for operands that it takes and for those that it hands back."""
+    torch.manual_seed(3)
+    T, D, E, k, V = 33, 256, 16, 4, 1003
+    bf, f32 = torch.bfloat16, torch.float32
+    x, w, base = (_form(form, device, bf, rows, D) for rows in (T, E, T))
+    dlogits, logits = _form(form, device, f32, T, E), _form(form, device, f32, T, E)
+    bias, dtop = torch.randn(E, device=device), _form(form, device, f32, T, k)
+    vocab, grad = _form(form, device, bf, T, V), torch.randn(2 * T, device=device)[::2]
+    target = torch.randint(0, V, (T,), device=device)
+    listed = [_form(form, device, t, 7, 96) for t in (bf, f32)] + [torch.randn(2, 5, 64, device=device)]
+
+    def run():
+        out = [ops.gate_logits(x, w), ops.gate_dx(dlogits, w), ops.gate_dx(dlogits, w, base), ops.gate_dw(dlogits, x)]
+        for softmax in (True, False):
+            top, selected, counts, blocks = ops.route_topk(logits, bias if softmax else None, k, softmax, True, 2.5)
+            out += [top, selected, counts, blocks, ops.route_topk_bwd(logits, selected, dtop, softmax, True, 2.5)]
+        lp, lse = ops.token_logprob_fwd(vocab, target)
+        out += [lp, lse, ops.token_logprob_bwd(vocab, target, lse, grad), ops.token_logprob_bwd(vocab, target, lse, lp)]
+        sent = ops.to_mx_rows_many(listed, "rceil")
+        return out + [t for q in sent for t in (q.codes, q.scales)] + ops.mx_dequant_many(sent)
+
+    counted = _Counted(_lib.blocks())
+    with monkeypatch.context() as m:
+        m.setattr(_lib, "blocks", lambda: counted)
+        native = run()
+    with monkeypatch.context() as m:
+        m.setattr(ops, "_single", lambda x: False)
+        general = run()
+    _same(native, general)
+    if form == "plain":
+        assert {"gate_logits", "gate_dx", "gate_dw", "route_topk", "route_topk_bwd", "token_logprob_fwd", "token_logprob_bwd",
+                "rows_many", "dequant_many"} <= set(counted.taken)

@@ -83,6 +83,12 @@ def _call(name: str, tag: str, device, *args) -> None:
         _lib.check(st, name)
 
 
+def _single(x: torch.Tensor) -> bool:
+    """A launch on x may go through the native module, which makes the outputs and passes the pointers on in a third of
+    the time (8 to 10 us a launch here); it returns None for operands that are not plain."""
+    return x.is_cuda and _timer is None and not _watched()
+
+
 def _mode(mode) -> int:
     if isinstance(mode, str):
         return SCALE_MODES[mode]
@@ -533,6 +539,8 @@ def _gate_check(x: torch.Tensor, experts: int, *others: torch.Tensor) -> None:
 
 def gate_logits(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """float32 [tokens, experts] = x w^T for bf16 x [tokens, dim], w [experts, dim], as a float32 matmul."""
+    if _single(x) and (out := _lib.blocks().gate_logits(x, w)) is not None:
+        return out
     x, w = _gate_rows(x), _gate_rows(w)
     if w.shape[1] != x.shape[1]:
         raise ValueError(f"column mismatch: {x.shape[1]} vs {w.shape[1]}")
@@ -553,6 +561,8 @@ def _gate_grad(dlogits: torch.Tensor, T: int, E: int) -> torch.Tensor:
 
 def gate_dx(dlogits: torch.Tensor, w: torch.Tensor, base: torch.Tensor | None = None) -> torch.Tensor:
     """bf16 [tokens, dim] = dlogits w, summed in float32; with `base` (bf16 of that shape) the bf16 sum of both."""
+    if _single(w) and (out := _lib.blocks().gate_dx(dlogits, w, base)) is not None:
+        return out
     w = _gate_rows(w)
     (E, D), T = w.shape, dlogits.shape[0]
     dlogits = _gate_grad(dlogits, T, E)
@@ -570,6 +580,8 @@ def gate_dx(dlogits: torch.Tensor, w: torch.Tensor, base: torch.Tensor | None = 
 
 def gate_dw(dlogits: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """bf16 [experts, dim] = dlogits^T x, summed in float32."""
+    if _single(x) and (out := _lib.blocks().gate_dw(dlogits, x)) is not None:
+        return out
     x = _gate_rows(x)
     (T, D), E = x.shape, dlogits.shape[1]
     dlogits = _gate_grad(dlogits, T, E)
@@ -585,6 +597,8 @@ def route_topk(logits: torch.Tensor, bias: torch.Tensor | None, top_k: int, soft
     """Token-choice routing from float32 logits [T, E] (`mx_route_topk`): (weights of the chosen experts
     float32 [T, k], the experts int64 [T, k] in falling order of score + bias, pairs per expert int64
     [E], and what `route_fill` needs to place the pairs)."""
+    if _single(logits) and (out := _lib.blocks().route_topk(logits, bias, top_k, bool(softmax), bool(norm), scale)) is not None:
+        return out
     T, E = logits.shape
     dev = logits.device
     if logits.dtype != torch.float32 or not logits.is_cuda:
@@ -606,6 +620,10 @@ def route_topk(logits: torch.Tensor, bias: torch.Tensor | None, top_k: int, soft
 def route_topk_bwd(logits: torch.Tensor, selected: torch.Tensor, dtop: torch.Tensor, softmax: bool, norm: bool,
                    scale: float) -> torch.Tensor:
     """Gradient of `route_topk`'s weights with respect to the logits, float32 [T, E]."""
+    if _single(logits):
+        out = _lib.blocks().route_topk_bwd(logits, selected, dtop, bool(softmax), bool(norm), scale)
+        if out is not None:
+            return out
     T, E = logits.shape
     if selected.device != logits.device or dtop.device != logits.device:
         raise ValueError("operands on different devices")
@@ -751,6 +769,9 @@ def _host_table(values, kind):
 def to_mx_rows_many(tensors, mode="floor"):
     """Row-wise `MXData` (codes of the tensor's shape, row-major scales [..., last/32]) of every tensor in the
     list -- bf16 or float32, one device, last dimension a multiple of 32 -- in one launch."""
+    tensors = list(tensors)
+    if tensors and _single(tensors[0]) and (out := _lib.blocks().rows_many(tensors, _mode(mode))) is not None:
+        return [MXData(codes, scales, MX_SCALES_ROWMAJOR) for codes, scales in out]
     tensors = [t.contiguous() if t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
                for t in tensors]
     if not tensors:
@@ -777,6 +798,11 @@ def to_mx_rows_many(tensors, mode="floor"):
 
 def mx_dequant_many(data) -> list:
     """bf16 values of every row-wise `MXData` with row-major scales in the list (any shapes), in one launch."""
+    data = list(data)
+    if data and _single(data[0].codes) and all(q.scale_order == MX_SCALES_ROWMAJOR for q in data):
+        out = _lib.blocks().dequant_many([q.codes for q in data], [q.scales for q in data])
+        if out is not None:
+            return out
     data = [MXData(q.codes.contiguous(), q.scales.contiguous(), q.scale_order) for q in data]
     if not data:
         return []
@@ -805,6 +831,10 @@ def _logprob_splits(rows: int, vocab: int) -> int:
 def token_logprob_fwd(logits: torch.Tensor, target: torch.Tensor):
     """(log-probability of target[r] under softmax(logits[r]), log-sum-exp of row r), float32
     [rows], from bf16 logits [rows, vocab] read once."""
+    if logits.dim() == 2 and logits.shape[0] and _single(logits):
+        out = _lib.blocks().token_logprob_fwd(logits, target, _logprob_splits(*logits.shape))
+        if out is not None:
+            return out
     logits = _check_hp(logits)
     if target.dtype != torch.int64 or target.shape != (logits.shape[0],) or target.device != logits.device:
         raise TypeError("target must be int64 [rows] on the logits' device")
@@ -825,6 +855,8 @@ def token_logprob_fwd(logits: torch.Tensor, target: torch.Tensor):
 def token_logprob_bwd(logits: torch.Tensor, target: torch.Tensor, lse: torch.Tensor,
                       grad_logprob: torch.Tensor) -> torch.Tensor:
     """Gradient of `token_logprob_fwd`'s first output with respect to the logits, bf16."""
+    if _single(logits) and (out := _lib.blocks().token_logprob_bwd(logits, target, lse, grad_logprob)) is not None:
+        return out
     logits = _check_hp(logits)
     (rows, vocab), ld = logits.shape, logits.stride(0)
     if ld < vocab:

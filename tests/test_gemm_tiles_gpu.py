@@ -248,3 +248,38 @@ def test_rows_do_not_depend_on_how_many_there_are(device, N, K):
     want = ops.mx_gemm_nt(a, b)
     for M in (65, 128, 129, 200, 1000, 2048):
         assert torch.equal(ops.mx_gemm_nt(a.first_rows(M), b), want[:M]), M
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 136, 128), (64, 200, 640), (128, 384, 256), (129, 392, 768), (192, 136, 896),
+                                   (321, 200, 1024), (200, 328, 2176), (577, 776, 1152)])
+@pytest.mark.parametrize("pad", [0, 128])
+def test_tiles_of_the_few_tiles_kernel_form_the_same_sums(device, hooks, M, N, K, pad):
+    """64 x 64 and 128 x 64 tiles against 256 x 256 ones: rows and columns that end inside a tile or a half of a scale
+    group, contractions shorter, as long and longer than the ring, and the sum of two whose second one begins inside it."""
+    rng = np.random.default_rng(M + N + K)
+    (a, ha), (a2, _) = _operand(device, rng, M, K), _operand(device, rng, M, K, 0.3)
+    (b, hb), (b2, _) = _operand(device, rng, N, K, 0.02), _operand(device, rng, N, K, 0.05)
+    if pad == 0:
+        a, a2, b, b2 = (ops.Operand.of(q.data()._replace(codes=q.codes.contiguous())) for q in (a, a2, b, b2))
+
+    def run(tile):
+        hooks.mx_debug_set_tile(*tile, 0)
+        out = torch.full((M, N + 24), 7.0, dtype=torch.bfloat16, device=device)
+        ops._call("mx_gemm_nt_ld", "gemm_nt", device, a.codes_ptr, a.scales_ptr, b.codes_ptr, b.scales_ptr, out.data_ptr(), M, N,
+                  a.k, a.ld, N + 24, None, 0, ops._stream(out))
+        assert bool((out[:, N:] == 7.0).all())
+        got = [out[:, :N].contiguous()]
+        if M > 64:
+            got.append(_float32(a, b, N + 24))
+        if M > 128:
+            got += [ops.mx_gemm_nt_shared_a(a, b, b2), ops.mx_gemm_nt_shared_b(a, a2, b), ops.mx_gemm_nt_pair(a, b, a2, b2)]
+        return got
+
+    hooks.mx_debug_force_kernel(3)
+    want = run((4, 4))
+    hooks.mx_debug_force_kernel(0)
+    _check(want[0], ha @ hb.T)
+    for tile in ((1, 1), (2, 1)):
+        for i, (g, w) in enumerate(zip(run(tile), want, strict=True)):
+            if M > 64 or i:  # (up to 64 rows have a kernel of their own, with sums in another order)
+                assert torch.equal(g, w), (tile, i)

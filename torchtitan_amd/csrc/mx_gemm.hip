@@ -40,12 +40,13 @@ static bool configure_dense() {
 // first such launch on a GPU: limits are not to be raised under graph capture, and which tile a captured shape takes
 // is not the caller's business.
 bool prepare_dense32();
+bool prepare_ring();
 bool prepare_dense() {
   static std::atomic<bool> prepared[kMaxDevices];
   const int dev = current_device();
   if (dev < 0) return false;
   if (!prepared[dev].load(std::memory_order_acquire)) {
-    if (!prepare_dense32() || !configure_dense<128, 128>() || !configure_dense<256, 256>() ||
+    if (!prepare_dense32() || !prepare_ring() || !configure_dense<128, 128>() || !configure_dense<256, 256>() ||
         !configure_dense<128, 128, true>())
       return false;
     prepared[dev].store(true, std::memory_order_release);
@@ -77,6 +78,8 @@ int launch_few_rows_codes(const uint8_t* a_codes, const uint8_t* a_scales, const
                           const uint8_t* b_scales, void* d, int64_t M, int64_t N, int64_t K, int64_t ldk, int64_t ldd,
                           hipStream_t st);
 GemmPlan plan_dense(int64_t M, int64_t N, int64_t K, bool may_split);
+GemmPlan plan_ring(int64_t M, int64_t N, int64_t blocks, int products);
+int launch_ring(const RingArgs& p, int ta, int tb, hipStream_t st);
 int launch_gemm_nt32_splitk(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                             const uint8_t* b_scales, void* d, int64_t M, int64_t N, int64_t K,
                             int64_t ldk, int64_t ldd, const GemmPlan& plan, void* workspace, bool f32,
@@ -147,7 +150,11 @@ static int gemm_nt_pitched(const uint8_t* a_codes, const uint8_t* a_scales, cons
       if (M <= 128 || tiles256 * 8 <= (int64_t)num_cus * 3) return launch_dense<128, 128>(p, st);
       return launch_dense<256, 256>(p, st);
     }
-    if (plan_dense(M, N, K, false).ta == 0) return launch_dense<128, 128>(p, st);
+    const GemmPlan plan = plan_dense(M, N, K, false);
+    if (plan.ta == 0) return launch_dense<128, 128>(p, st);
+    if (plan.ring())
+      return launch_ring({a_codes, a_scales, b_codes, b_scales, nullptr, nullptr, nullptr, nullptr, d, nullptr, M, N, K, ldk, ldd,
+                          0, 0, 0}, plan.ta, plan.tb, st);
   }
   if (force_kernel == 1 || !persistent_ok(d, N, K, ldd, ldk)) return launch_dense<256, 256>(p, st);
   return launch_gemm_nt32(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldk, ldd, false, st);
@@ -186,6 +193,10 @@ extern "C" int mx_gemm_nt_pair_ld(const uint8_t* a_codes, const uint8_t* a_scale
   if (ldk < K) return MX_ERR_INVALID_ARG;
   if (M <= 128 || N <= 128 || !persistent_ok(d, N, K, ldd, ldk) || force_kernel == 1 || force_kernel == 2)
     return MX_ERR_UNSUPPORTED;
+  const GemmPlan plan = force_kernel == 0 ? plan_ring(M, N, 2 * (K / 128), 1) : GemmPlan{0, 0, 1};
+  if (plan.ring())
+    return launch_ring({a_codes, a_scales, b_codes, b_scales, a2_codes, a2_scales, b2_codes, b2_scales, d, nullptr, M, N, K, ldk,
+                        ldd, 0, 1, 0}, plan.ta, plan.tb, (hipStream_t)stream);
   return launch_gemm_nt32_pair(a_codes, a_scales, b_codes, b_scales, a2_codes, a2_scales, b2_codes,
                                b2_scales, d, M, N, K, ldk, ldd, (hipStream_t)stream);
 }
@@ -247,6 +258,10 @@ extern "C" int mx_gemm_nt_shared_a_ld(const uint8_t* a_codes, const uint8_t* a_s
   if (M <= 128 || N <= 128 || !persistent_ok(d, N, K, ldd, ldk) || !persistent_ok(d2, N, K, ldd, ldk) ||
       force_kernel == 1 || force_kernel == 2)
     return MX_ERR_UNSUPPORTED;
+  const GemmPlan plan = force_kernel == 0 ? plan_ring(M, N, K / 128, 2) : GemmPlan{0, 0, 1};
+  if (plan.ring())
+    return launch_ring({a_codes, a_scales, b_codes, b_scales, nullptr, nullptr, b2_codes, b2_scales, d, d2, M, N, K, ldk, ldd, 1,
+                        0, 0}, plan.ta, plan.tb, (hipStream_t)stream);
   return launch_gemm_nt32_two_b(a_codes, a_scales, b_codes, b_scales, b2_codes, b2_scales, d, d2, M, N,
                                 K, ldk, ldd, (hipStream_t)stream);
 }
@@ -272,6 +287,10 @@ extern "C" int mx_gemm_nt_shared_b_ld(const uint8_t* a_codes, const uint8_t* a_s
   if (M <= 128 || N <= 128 || !persistent_ok(d, N, K, ldd, ldk) || !persistent_ok(d2, N, K, ldd, ldk) ||
       force_kernel == 1 || force_kernel == 2)
     return MX_ERR_UNSUPPORTED;
+  const GemmPlan plan = force_kernel == 0 ? plan_ring(M, N, K / 128, 2) : GemmPlan{0, 0, 1};
+  if (plan.ring())
+    return launch_ring({a_codes, a_scales, b_codes, b_scales, a2_codes, a2_scales, nullptr, nullptr, d, d2, M, N, K, ldk, ldd, 2,
+                        0, 0}, plan.ta, plan.tb, (hipStream_t)stream);
   return launch_gemm_nt32_two_a(a_codes, a_scales, a2_codes, a2_scales, b_codes, b_scales, d, d2, M, N,
                                 K, ldk, ldd, (hipStream_t)stream);
 }
@@ -334,7 +353,11 @@ extern "C" int mx_gemm_nt_f32_ld(const uint8_t* a_codes, const uint8_t* a_scales
     if (plan.slices > 1 && workspace_bytes >= split_bytes(plan, M, N))
       return launch_gemm_nt32_splitk(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldk, ldd, plan, workspace, true, st);
   }
-  if (force_kernel == 1 || force_kernel == 2 || (force_kernel == 0 && plan_dense(M, N, K, false).ta == 0))
+  const GemmPlan plan = force_kernel == 0 ? plan_dense(M, N, K, false) : GemmPlan{4, 4, 1};
+  if (plan.ring())
+    return launch_ring({a_codes, a_scales, b_codes, b_scales, nullptr, nullptr, nullptr, nullptr, d, nullptr, M, N, K, ldk, ldd,
+                        0, 0, 1}, plan.ta, plan.tb, st);
+  if (force_kernel == 1 || force_kernel == 2 || plan.ta == 0)
     return launch_dense<128, 128, true>(DenseArgs{a_codes, a_scales, b_codes, b_scales, (uint16_t*)d, M, N, K, ldd, ldk}, st);
   return launch_gemm_nt32(a_codes, a_scales, b_codes, b_scales, d, M, N, K, ldk, ldd, true, st);
 }

@@ -48,8 +48,6 @@
 
 namespace mx {
 
-typedef float v4f __attribute__((ext_vector_type(4)));
-
 constexpr int kT32 = 256;                        // tile edge (M and N)
 constexpr int kK32 = 64;                         // K per compute step
 constexpr int kKB = 128;                         // K per ring block (= one cache line per row)
@@ -159,25 +157,6 @@ __device__ __forceinline__ v4i lds_read_b128_hidden(uint32_t addr) {
 __device__ __forceinline__ v4i pin(v4i v) {
   asm volatile("" : "+v"(v));
   return v;
-}
-
-// One scaled MFMA, C = 0 (FIRST) or accumulate.  Written as assembly: left as builtins, the
-// compiler gathers all MFMAs of a tile's first block behind the block's copies, reads and
-// barriers instead of leaving them interleaved.  op_sel / op_sel_hi pick the scale byte of the
-// lane's scale dword: NB for the first operand, MB for the second.
-template <int NB, int MB, bool FIRST>
-__device__ __forceinline__ void mfma16_asm(v4f& c, const v8i& b, const v8i& a, uint32_t sb,
-                                           uint32_t sa) {
-  if constexpr (FIRST)
-    asm volatile(
-        "v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, 0, %3, %4 op_sel:[%5,%6,0] op_sel_hi:[%7,%8,0]"
-        : "=a"(c)
-        : "v"(b), "v"(a), "v"(sb), "v"(sa), "n"(NB & 1), "n"(MB & 1), "n"(NB >> 1), "n"(MB >> 1));
-  else
-    asm volatile(
-        "v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel:[%5,%6,0] op_sel_hi:[%7,%8,0]"
-        : "+a"(c)
-        : "v"(b), "v"(a), "v"(sb), "v"(sa), "n"(NB & 1), "n"(MB & 1), "n"(NB >> 1), "n"(MB >> 1));
 }
 
 // One accumulator register into a VGPR, where the caller says (as assembly: the compiler's own
@@ -1412,6 +1391,35 @@ static const DenseTile* best_tile(int64_t M, int64_t N, int64_t blocks, int prod
   return best;
 }
 
+// The tiles of the kernel of few tiles, and the microseconds that `tiles` of `blocks` blocks each take on it, fitted to the
+// 225 shapes of 72..2048 rows, 512..10240 columns and K 256..10240 for which it may be chosen (residual 4 %).
+struct RingTile {
+  int ta, tb;
+  double start_us, block_us, part_us, share_us, round_us;
+};
+static constexpr RingTile kRingTiles[] = {{1, 1, 1.74, 0.289, 0.242, 0.038, 2.88}, {2, 1, 1.26, 0.436, 0.350, 0.087, 3.73}};
+static double ring_us(const RingTile& t, int64_t tiles, int64_t blocks, int64_t grid) {
+  const double rest = (double)(tiles % grid) / grid;
+  double us = t.start_us + (double)(tiles / grid) * (blocks * t.block_us + t.round_us);
+  if (tiles % grid) us += blocks * (t.part_us + t.share_us * rest) + t.round_us;
+  return us;
+}
+// The one of them that promises 3 % over `us`, which then becomes its time.  (Over those shapes the choice takes 0.81 of
+// the time without it, the best one of either 0.81; none of them got slower by more than 3 %.)
+static const RingTile* better_ring(int64_t M, int64_t N, int64_t blocks, int products, int64_t grid, double& us) {
+  const RingTile* best = nullptr;
+  for (const RingTile& t : kRingTiles) {
+    if (debug_tile && debug_tile != t.ta * 16 + t.tb) continue;
+    const int64_t tiles = products * ((M + 64 * t.ta - 1) / (64 * t.ta)) * ((N + 64 * t.tb - 1) / (64 * t.tb));
+    const double mine = ring_us(t, tiles, blocks, grid);
+    if (mine < (best ? us : 0.97 * us) || debug_tile) {
+      best = &t;
+      us = mine;
+    }
+  }
+  return best;
+}
+
 // What a dense product runs on: the persistent kernel with tiles of 64 ta x 64 tb in `slices` slices
 // of K, or (ta == 0) the kernel of one 128 x 128 tile per workgroup.
 //   * That one is ahead for short contractions only: it starts faster (512 x 4096: K 256 6.1 us, 7.4
@@ -1433,7 +1441,11 @@ GemmPlan plan_dense(int64_t M, int64_t N, int64_t K, bool may_split) {
   const int64_t grid = persistent_grid(), blocks = K / kKB;
   if (grid == 0 || K % kKB) return {0, 0, 1};
   const DenseTile* t = best_tile(M, N, blocks, 1, grid);
-  if (!t) return {0, 0, 1};
+  if (!t) {
+    double us = 0;
+    const RingTile* r = better_ring(M, N, blocks, 1, grid, us);
+    return r ? GemmPlan{r->ta, r->tb, 1} : GemmPlan{0, 0, 1};
+  }
   GemmPlan best{t->ta, t->tb, 1};
   double best_us = tiles_us(*t, tile_count(*t, M, N), blocks, grid) + 2.0;
   if (!debug_tile) {
@@ -1444,25 +1456,30 @@ GemmPlan plan_dense(int64_t M, int64_t N, int64_t K, bool may_split) {
       best_us = us;
     }
   }
-  if (!may_split || (blocks <= 32 && !debug_slices)) return best;
   const double plain_us = best_us;
-  for (const DenseTile& u : kDenseTiles) {
-    if (u.ta * u.tb == 12 || (debug_tile && debug_tile != u.ta * 16 + u.tb)) continue;
-    const int64_t tiles = tile_count(u, M, N);
-    for (int s = 2; s <= 8; ++s) {
-      const int64_t per = (blocks + s - 1) / s;
-      if (per < 4 || (s - 1) * per >= blocks || (debug_slices && s != debug_slices)) continue;
-      const double bytes = 4.0 * s * M * N;
-      const bool large = bytes > (double)(64 << 20);
-      if (large && (u.ta * u.tb < 16 || 2 * tiles <= grid || (7 * tiles > 5 * grid && tiles <= grid) || 2 * tiles >= 3 * grid))
-        continue;
-      const double us = tiles_us(u, tiles * s, per, grid) + 2.0 + 4.2 + bytes / 3.2e6;
-      if (us < best_us && us <= 0.92 * plain_us || debug_slices) {
-        best = {u.ta, u.tb, s};
-        best_us = us;
+  if (may_split && (blocks > 32 || debug_slices)) {
+    for (const DenseTile& u : kDenseTiles) {
+      if (u.ta * u.tb == 12 || (debug_tile && debug_tile != u.ta * 16 + u.tb)) continue;
+      const int64_t tiles = tile_count(u, M, N);
+      for (int s = 2; s <= 8; ++s) {
+        const int64_t per = (blocks + s - 1) / s;
+        if (per < 4 || (s - 1) * per >= blocks || (debug_slices && s != debug_slices)) continue;
+        const double bytes = 4.0 * s * M * N;
+        const bool large = bytes > (double)(64 << 20);
+        if (large && (u.ta * u.tb < 16 || 2 * tiles <= grid || (7 * tiles > 5 * grid && tiles <= grid) || 2 * tiles >= 3 * grid))
+          continue;
+        const double us = tiles_us(u, tiles * s, per, grid) + 2.0 + 4.2 + bytes / 3.2e6;
+        if (us < best_us && us <= 0.92 * plain_us || debug_slices) {
+          best = {u.ta, u.tb, s};
+          best_us = us;
+        }
       }
     }
   }
+  // Few tiles, not split: 64-wide ones (up to 64 rows have a kernel of their own).  Where a split is to be had it is as fast
+  // or faster: 256 x 4096, K 6144 17.7 us and 17.6 in one chain; 512 x 512, K 10240 18.7 and 25.2.
+  if (best.slices == 1 && !debug_tile && M > 64)
+    if (const RingTile* r = better_ring(M, N, blocks, 1, grid, best_us)) best = {r->ta, r->tb, 1};
   return best;
 }
 
@@ -1492,6 +1509,18 @@ GemmPlan plan_pair(int64_t M, int64_t N, int64_t K) {
     }
   }
   return best;
+}
+
+// Whether two products of one launch (products == 2), or one over the K blocks of two operand sets (`blocks` counts both),
+// run on the kernel of few tiles: ring() then.
+GemmPlan plan_ring(int64_t M, int64_t N, int64_t blocks, int products) {
+  const int64_t grid = persistent_grid();
+  if (grid == 0) return {0, 0, 1};
+  const DenseTile* t = best_tile(M, N, blocks, products, grid);
+  double us = t ? tiles_us(*t, products * tile_count(*t, M, N), blocks, grid) + 2.0 : 0;
+  if (t && debug_tile) return {0, 0, 1};
+  const RingTile* r = better_ring(M, N, blocks, products, grid, us);
+  return r ? GemmPlan{r->ta, r->tb, 1} : GemmPlan{0, 0, 1};
 }
 
 // Launches the persistent dense kernel on `p` with tiles of 64 ta x 64 tb.

@@ -37,9 +37,20 @@ __device__ __forceinline__ void static_for(F&& f) {
 }
 
 // How a dense product runs (plan_dense, mx_gemm32.hip): tiles of 64 ta x 64 tb on the persistent kernel,
-// K in `slices` slices; ta == 0: the kernel of one 128 x 128 tile per workgroup.
+// K in `slices` slices, or, 64 x 64 and 128 x 64, on the kernel of few tiles (mx_gemm_ring.hip); ta == 0: the kernel of one
+// 128 x 128 tile per workgroup.
 struct GemmPlan {
   int ta, tb, slices;
+  bool ring() const { return ta * tb == 1 || ta * tb == 2; }
+};
+
+// A product, or two, on the kernel of few tiles (mx_gemm_ring.hip).  The second operand set: `pair` D = A B^T + A2 B2^T;
+// `two` == 1 D2 = A B2^T, == 2 D2 = A2 B^T.
+struct RingArgs {
+  const uint8_t *a_codes, *a_scales, *b_codes, *b_scales, *a2_codes, *a2_scales, *b2_codes, *b2_scales;
+  void *d, *d2;
+  int64_t M, N, K, ldk, ldd;
+  int32_t two, pair, f32;
 };
 
 // One GEMM operand as the tile sees it.
@@ -59,6 +70,24 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, int64
 
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+
+// One scaled MFMA, C = 0 (FIRST) or accumulate.  Written as assembly: left as builtins, the
+// compiler gathers MFMAs behind copies, reads and barriers instead of leaving them interleaved.  op_sel / op_sel_hi pick the scale byte of the
+// lane's scale dword: NB for the first operand, MB for the second.
+template <int NB, int MB, bool FIRST>
+__device__ __forceinline__ void mfma16_asm(v4f& c, const v8i& b, const v8i& a, uint32_t sb,
+                                           uint32_t sa) {
+  if constexpr (FIRST)
+    asm volatile(
+        "v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, 0, %3, %4 op_sel:[%5,%6,0] op_sel_hi:[%7,%8,0]"
+        : "=a"(c)
+        : "v"(b), "v"(a), "v"(sb), "v"(sa), "n"(NB & 1), "n"(MB & 1), "n"(NB >> 1), "n"(MB >> 1));
+  else
+    asm volatile(
+        "v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel:[%5,%6,0] op_sel_hi:[%7,%8,0]"
+        : "+a"(c)
+        : "v"(b), "v"(a), "v"(sb), "v"(sa), "n"(NB & 1), "n"(MB & 1), "n"(NB >> 1), "n"(MB >> 1));
+}
 
 // two floats -> two bf16 (round to nearest even) in one dword: v_cvt_pk_bf16_f32
 __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {

@@ -473,6 +473,17 @@ int mx_gemm_nt_shared_b_ld(const uint8_t* a_codes, const uint8_t* a_scales, cons
                            void* d, void* d2, int64_t M, int64_t N, int64_t K, int64_t ldk,
                            int64_t ldd, void* stream);
 
+/* The row-wise MXFP8 cast of bf16(bf16(silu(A B^T)) * A B2^T), both products rounded to bf16, in one launch: what
+ * mx_gemm_nt_shared_a_ld and mx_swiglu_cast_pad without column-wise outputs give, the same bits, without the two products
+ * in memory.  codes [M, N up to 128] with rows ld_codes bytes apart (a multiple of 16), scales in MFMA order.  M > 128,
+ * N > 128, N % 8 and K % 128, else MX_ERR_UNSUPPORTED.  mx_gemm_nt_swiglu_planned: 1 where this one launch is
+ * predicted to be done before the two. */
+int mx_gemm_nt_swiglu_planned(int64_t M, int64_t N, int64_t K);
+int mx_gemm_nt_swiglu_ld(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
+                         const uint8_t* b_scales, const uint8_t* b2_codes, const uint8_t* b2_scales,
+                         uint8_t* codes, int64_t ld_codes, uint8_t* scales, int64_t M, int64_t N, int64_t K,
+                         int64_t ldk, int scale_mode, void* stream);
+
 /* Grouped GEMM, 2D x 3D: for group g with rows [offs[g-1], offs[g]) of A:
  * D[rows, :] = deq(A[rows, :]) * deq(B[g])^T.  a_codes [T,K]; b_codes [G,N,K];
  * b_scales G consecutive MFMA-order blocks, each for [N, K/32].

@@ -283,3 +283,25 @@ def test_tiles_of_the_few_tiles_kernel_form_the_same_sums(device, hooks, M, N, K
         for i, (g, w) in enumerate(zip(run(tile), want, strict=True)):
             if M > 64 or i:  # (up to 64 rows have a kernel of their own, with sums in another order)
                 assert torch.equal(g, w), (tile, i)
+
+
+@pytest.mark.parametrize("M,N,K", [(129, 136, 128), (256, 256, 384), (300, 392, 640), (385, 200, 2016), (512, 1000, 4096)])
+@pytest.mark.parametrize("mode", ["floor", "rceil"])
+@pytest.mark.parametrize("pad", [0, 128])
+def test_gate_in_the_product_gives_the_bits_of_the_gate_behind_it(device, M, N, K, mode, pad):
+    """Rows and columns that end inside a tile, a scale group and a 32-column block; sizes of the factors from where
+    the gate is linear to where it overflows, blocks of zeros, infinities and NaN."""
+    rng = np.random.default_rng(M + N + K)
+    x = bf16_from_bits(randn_bits(rng, (M, K), std=1.0, outliers=1e-3), device)
+    x[1:60:7] = 0
+    x[2], x[67], x[3, 5], x[70, 9] = 1e30, -1e30, float("nan"), float("inf")
+    w, w2 = (bf16_from_bits(randn_bits(rng, (N, K), std=s, outliers=1e-3), device) for s in (0.05, 2.0))
+    w[:64], w2[64:96] = w[:64] * 1e-12, 0
+    a, b, b2 = (ops.to_operands(t, mode, cols=False, pitch_pad=pad)[0] for t in (x, w, w2))
+    h = ops.mx_gemm_nt_shared_a(a, b, b2)
+    want = ops.swiglu_to_operands(h[0], h[1], mode, False, pad)[0]
+    got = ops.mx_gemm_nt_swiglu(a, b, b2, mode, planned=True)
+    assert (got.k, got.ld, got.depth) == (want.k, want.ld, want.depth)
+    wrong = (got.codes != want.codes).nonzero().tolist()
+    assert not wrong, (len(wrong), wrong[:8])
+    assert torch.equal(*(ops.scale_unlayout(q.scales.contiguous(), M, q.k // 32) for q in (got, want)))

@@ -81,6 +81,8 @@ SIGNATURES = {
     "mx_gemm_nt_pair_ws": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _P]),
     "mx_gemm_nt_shared_a_ld": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     "mx_gemm_nt_shared_b_ld": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
+    "mx_gemm_nt_swiglu_ld": (c_int, [_P, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, c_int, _P]),
+    "mx_gemm_nt_swiglu_planned": (c_int, [_I, _I, _I]),
     "mx_gemm_nt_shared_a": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P]),
     "mx_gemm_nt_shared_b": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P]),
     "mx_grouped_gemm_2d3d_shared_a": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),

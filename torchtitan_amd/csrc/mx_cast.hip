@@ -325,10 +325,6 @@ __device__ __forceinline__ uint32_t cvt2_finite(float lo, float hi, uint32_t old
   return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(lo, hi, (int)old, HIGH);
 }
 
-typedef float v2f_t __attribute__((ext_vector_type(2)));
-typedef __bf16 v2bf_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
-__device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }
 
 // Quantize one lane's 8x8 patch.  FINITE = no Inf / NaN anywhere in the wave's patches: the
 // straight-line path; otherwise the general path with per-block NaN handling and clamps.
@@ -476,26 +472,6 @@ struct TileWalk {
     by = band * BY + in % h;
   }
 };
-
-// SwiGLU gate in front of the cast: g = bf16(bf16(silu(a)) * b) per element, each step rounded
-// to bf16 like the unfused bf16 tensor ops.  silu follows the float32 formula a / (1 + exp(-a))
-// with a correctly rounded quotient (hardware reciprocal plus one Newton step on the
-// remainder): the bf16 result equals torch's GPU silu for every one of the 65536 bf16 inputs.
-__device__ __forceinline__ float silu_f32(float a) {
-  // Numerator and denominator come scaled by 1/4: the hardware reciprocal flushes a denormal result, and a quarter of
-  // a finite denominator has none.  The remainder is NaN where the product itself is the answer (a = +inf; an
-  // infinite denominator, whose reciprocal is 0): as 1 it adds nothing to either.  It is subtracted so that a = -0
-  // keeps its sign.
-  const float ds = __builtin_fmaf(__expf(-a), 0.25f, 0.25f), r = __builtin_amdgcn_rcpf(ds);
-  const float as = 0.25f * a, q = as * r;
-  return __builtin_fmaf(-fminf(__builtin_fmaf(q, ds, -as), 1.0f), r, q);
-}
-__device__ __forceinline__ uint32_t swiglu2(uint32_t a2, uint32_t b2) {
-  const float s_lo = silu_f32(bf16_lo(a2)), s_hi = silu_f32(bf16_hi(a2));
-  const uint32_t s2 = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f_t{s_lo, s_hi}, v2bf_t));
-  const float g_lo = bf16_lo(s2) * bf16_lo(b2), g_hi = bf16_hi(s2) * bf16_hi(b2);
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f_t{g_lo, g_hi}, v2bf_t));
-}
 
 // Backward of g = silu(a) * b under bf16 autograd, tensor op by tensor op:
 //   d/db = bf16(dg * bf16(silu(a)))

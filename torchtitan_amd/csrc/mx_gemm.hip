@@ -266,6 +266,34 @@ extern "C" int mx_gemm_nt_shared_a_ld(const uint8_t* a_codes, const uint8_t* a_s
                                 K, ldk, ldd, (hipStream_t)stream);
 }
 
+namespace mx {
+bool plan_gated(int64_t M, int64_t N, int64_t K);
+int launch_gemm_nt32_gated(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes, const uint8_t* b_scales,
+                           const uint8_t* b2_codes, const uint8_t* b2_scales, uint8_t* codes, uint8_t* scales, int64_t M,
+                           int64_t N, int64_t K, int64_t ldk, int64_t ld_codes, int scale_mode, hipStream_t st);
+}
+
+extern "C" int mx_gemm_nt_swiglu_planned(int64_t M, int64_t N, int64_t K) {
+  return M > 128 && N > 128 && K > 0 && N % 8 == 0 && K % 128 == 0 && force_kernel == 0 && plan_gated(M, N, K);
+}
+
+extern "C" int mx_gemm_nt_swiglu_ld(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
+                                    const uint8_t* b_scales, const uint8_t* b2_codes, const uint8_t* b2_scales,
+                                    uint8_t* codes, int64_t ld_codes, uint8_t* scales, int64_t M, int64_t N, int64_t K,
+                                    int64_t ldk, int scale_mode, void* stream) {
+  int rc = check_dense(a_codes, a_scales, b_codes, b_scales, codes, M, N, K, N);
+  if (rc == MX_OK) rc = check_dense(a_codes, a_scales, b2_codes, b2_scales, codes, M, N, K, N);
+  if (rc != MX_OK || M == 0 || N == 0) return rc;
+  if (ldk < K || ld_codes < (N + 127) / 128 * 128 || !scales || (scale_mode != MX_SCALE_FLOOR && scale_mode != MX_SCALE_RCEIL))
+    return MX_ERR_INVALID_ARG;
+  if (ld_codes % 16 || ((uintptr_t)codes & 15) || ((uintptr_t)scales & 3)) return MX_ERR_ALIGNMENT;
+  if (M <= 128 || N <= 128 || K % 128 || ldk % 128 || (uint64_t)ldk * 256 > 0x7FFFFFFFull || N % 8 ||
+      (uint64_t)ld_codes * 256 > 0x7FFFFFFFull)
+    return MX_ERR_UNSUPPORTED;
+  return launch_gemm_nt32_gated(a_codes, a_scales, b_codes, b_scales, b2_codes, b2_scales, codes, scales, M, N, K, ldk, ld_codes,
+                                scale_mode, (hipStream_t)stream);
+}
+
 extern "C" int mx_gemm_nt_shared_a(const uint8_t* a_codes, const uint8_t* a_scales,
                                    const uint8_t* b_codes, const uint8_t* b_scales,
                                    const uint8_t* b2_codes, const uint8_t* b2_scales, void* d,

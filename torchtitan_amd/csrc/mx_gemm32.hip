@@ -106,6 +106,8 @@ struct Gemm32Args {
   int64_t d_rows = 0;
   // kSplitK: 2 = the sum of two products (a2 .. b2 as for PAIR), each cut into G / 2 slices
   int32_t sets = 1;
+  // GATE: how the gated product is scaled (d its codes, ldd bytes between their rows, d2 their scales)
+  int32_t scale_mode = 0;
 };
 enum Gemm32Two { kTwoNone = 0, kTwoB = 1, kTwoA = 2 };
 
@@ -125,6 +127,7 @@ struct Tile32 {
                            // its 128-row scale group (0..3): the A scale bytes are turned by as much
   uint32_t odd;            // 192-row tiles: bit 0 / 1: the tile begins in the middle of a 128-row scale
                            // group of A / of B
+  uint32_t tm, tn;         // GATE: its row and column
   uint32_t head, tail;     // kGrouped2d2d: the K range starts `head` 32-deep blocks into its first
                            // 128-deep block and ends `tail` of them into its last (0: at its end)
 };
@@ -274,14 +277,22 @@ __device__ __forceinline__ constexpr uint32_t wave_col(uint32_t wn, int n) {
 // OUT32 (kDense, one product): D is float32, its values rounded to bf16 first, as a conversion of a bf16 result
 // would give them; ldd counts floats.  (Instances of their own: a branch in front of the bf16 epilogue
 // made 147456 x 2048, K 2048 forward and backward 1.6 % slower.)
-template <int MODE, bool PROF, bool PAIR = false, int TA = 4, int TB = 4, bool OUT32 = false>
+// GATE (kDense, 256 x 256): G = silu(A B^T) * (A B2^T), every step rounded to bf16 as the tensor operations round, leaves
+// as the row-wise MXFP8 operand of the next product: of a forward without gradients nothing else is read again.  A
+// tile is 256 rows of 128 columns of G: a wave's sub-tiles 0 .. 3 come from B, 4 .. 7 from the same rows of B2, so that a lane
+// holds both factors of its values; waves 0 and 2 copy B's rows into the ring, 1 and 3 those of B2.  What the
+// gate adds to the epilogue (8 K vector instructions a wave, about 5 us a round, matrix cores idle) is less than the
+// 8 bytes a value that are not written and read again, and the launch: 512 x 14336, K 4096 59.9 us in two launches, 53.0 in
+// this one; 1024 x 14336 113 and 101 (plan_gated for where it is not).
+template <int MODE, bool PROF, bool PAIR = false, int TA = 4, int TB = 4, bool OUT32 = false, bool GATE = false>
 __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  static_assert(!GATE || (MODE == kDense && TA == 4 && TB == 4 && !PAIR && !OUT32));
   static_assert((TA == 4 && TB == 4) || MODE == kDense || MODE == kSplitK, "grouped tiles are 256 x 256");
   using Plan = BlockPlan<TA, TB>;
   using Frags = Frags16<TA, TB>;
   using Lds = Lds32<TA, TB>;
-  constexpr int kEA = 64 * TA, kEB = 64 * TB;  // tile edges
+  constexpr int kEA = 64 * TA, kEB = GATE ? 128 : 64 * TB;  // tile edges
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -431,6 +442,7 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
     r.rows_d = 0;
     r.rot = 0;
     r.odd = 0;
+    r.tm = r.tn = 0;
     r.head = 0;
     r.tail = 0;
     const uint8_t* a_codes = (PAIR && seg) ? p.a2_codes : p.a_codes;
@@ -480,6 +492,10 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
       r.rows_a = p.M - (int64_t)tm * kEA;
       r.rows_b = p.N - (int64_t)tn * kEB;
       r.odd = (tm & 1) | (tn & 1) << 1;
+      if constexpr (GATE) {
+        r.tm = tm;
+        r.tn = tn;
+      }
       if (MODE == kGrouped2d3d && p.d_offs) {
         const int64_t left = p.d_rows - (int64_t)tm * kT32;
         r.rows_d = (int32_t)(left < 0 ? 0 : (left > kT32 ? kT32 : left));
@@ -673,15 +689,16 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
   const uint32_t fb_delta4 = TB == 3 ? Lds::kA + (wave_col<TB>(wn, 4) - 64 - wm * 32 * TA) * kKB : fb_delta;
   // scale copy: lanes 0-31 fetch one 128-row group's 512 bytes of a block, lanes 32-63 the next
   // group's; wave 1 (kGrouped2d3d: a third group of A) has its upper lanes read nothing
-  const uint32_t v_scale = (MODE == kGrouped2d3d && wave == 1)
+  const uint32_t v_scale = (MODE == kGrouped2d3d && wave == 1) || (GATE && wave >= 2)
                                ? (lane < 32 ? (uint32_t)lane * 16 : 0x80000000u)
                                : (uint32_t)(lane >> 5) * ks_n * 256 + (lane & 31) * 16;
   // scale groups of a ring block: A0, A1, B0, B1, A2 (512 bytes each, then 512 unused)
-  const uint32_t scale_dst = Lds::kCodes + ((MODE == kGrouped2d3d && wave == 1) ? 2048u : (uint32_t)(wave >> 1) * 1024u);
+  // (GATE: B's group in place of B0, B2's in place of A2, zeros behind either)
+  const uint32_t scale_dst = Lds::kCodes + ((MODE == kGrouped2d3d && wave == 1) || (GATE && wave == 3) ? 2048u : (uint32_t)(wave >> 1) * 1024u);
   // 256 rows: a wave has a scale group of its own (kGrouped2d3d: and the next one, see next_scales);
   // 192: three of the eight bytes of two groups; 128: half of the bytes of one
-  const uint32_t fsa_s = Lds::kCodes + (TA == 4 ? wm * 512 : 0), fsb_s = Lds::kCodes + 1024 + (TB == 4 ? wn * 512 : 0);
-  const uint32_t fsa_hi_s = Lds::kCodes + (TA == 4 && wm != 0 ? 2048 : 512), fsb_hi_s = Lds::kCodes + 1536;
+  const uint32_t fsa_s = Lds::kCodes + (TA == 4 ? wm * 512 : 0), fsb_s = Lds::kCodes + 1024 + (TB == 4 && !GATE ? wn * 512 : 0);
+  const uint32_t fsa_hi_s = Lds::kCodes + (TA == 4 && wm != 0 ? 2048 : 512), fsb_hi_s = Lds::kCodes + (GATE ? 2048 : 1536);
 
   // ---- loader stream: fills ring block `ld_slot` with K block `ld_kb` of tile `ld_tile`
   uint32_t ld_tile = 0, ld_kb = 0, ld_nb = 1;
@@ -724,7 +741,11 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
       // its one block arrives as zeros, scales included.
       const bool none = MODE != kDense && t.empty;
       ra = make_rsrc(t.a, none ? 0 : t.rows_a * (int64_t)Kp - t.koff);
-      rb = make_rsrc(t.b, none ? 0 : t.rows_b * (int64_t)Kp - t.koff);
+      if constexpr (GATE) {  // this wave's 64 rows: of B or of B2
+        const uint8_t* from = (wave & 1 ? p.b2_codes + (t.b - p.b_codes) : t.b) + (int64_t)(wave >> 1) * 64 * Kp;
+        rb = make_rsrc(from, (t.rows_b - (wave >> 1) * 64) * (int64_t)Kp);
+      } else
+        rb = make_rsrc(t.b, none ? 0 : t.rows_b * (int64_t)Kp - t.koff);
       // wave 0 copies the scales of A's two 128-row groups, wave 2 those of B's (one copy per
       // block each: lanes 0-31 fetch group 0, lanes 32-63 group 1); a group beyond the operand
       // is cut off by the range and arrives as zeros
@@ -734,7 +755,7 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
       const int64_t into_a = TA == 3 ? 64 * (int64_t)(t.odd & 1) : 32 * (int64_t)t.rot;
       const int64_t into_b = TB == 3 ? 64 * (int64_t)(t.odd >> 1) : 0;
       const int64_t rows = wave < 2 ? (t.rows_a > 0 ? t.rows_a + into_a : 0) : t.rows_b > 0 ? t.rows_b + into_b : 0;
-      const uint8_t* sbase = wave < 2 ? t.sa : t.sb;
+      const uint8_t* sbase = wave < 2 ? t.sa : GATE && wave == 3 ? p.b2_scales + (t.sb - p.b_scales) : t.sb;
       if (MODE == kGrouped2d3d && wave == 1)
         rs = make_rsrc(sbase + (int64_t)ks_n * 512, (none || rows <= 256) ? 0 : (int64_t)ld_nb * 512);
       else
@@ -771,7 +792,7 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
       const int unit = wave * 2 * (is_a ? TA : TB) + q;
       const uint32_t v = MODE == kGrouped2d2d ? ((q & 1) ? cur_v_odd : cur_v_even)
                                               : ((q & 1) ? (v_even ^ 64) : v_even);
-      const uint32_t so = (uint32_t)(unit * 8) * Kp + ld_kb * kKB;
+      const uint32_t so = (uint32_t)((GATE && !is_a ? q : unit) * 8) * Kp + ld_kb * kKB;
       if constexpr (is_a)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void_t*)(uintptr_t)(sbase + unit * 1024), 16, v, so, 0, MX_LOAD_AUX);
       else
@@ -856,7 +877,7 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
   // the scale dwords of a block, into the "next" registers: piece 0, 1 = A even / odd
   // sub-tiles, 2, 3 = B, then those of the next 128-row group of A (kGrouped2d3d, 192 rows) and of
   // B (192 columns)
-  constexpr bool kHiA = MODE == kGrouped2d3d || TA == 3, kHiB = TB == 3;
+  constexpr bool kHiA = MODE == kGrouped2d3d || TA == 3, kHiB = TB == 3 || GATE;
   constexpr int kScalePieces = 4 + (kHiA ? 2 : 0) + (kHiB ? 2 : 0);
   auto read_scale_piece = [&](Frags& f, uint32_t sbase, auto i_) {
     constexpr int i = decltype(i_)::value;
@@ -901,6 +922,8 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
       if constexpr (TB == 3) {
         const uint32_t sel = (wn ? 0x00030504u : 0x00020100u) + ((rot & 2) ? 0x00020202u : 0u);
         f.sb[e] = __builtin_amdgcn_perm(f.sb_hi[e], f.sbn[e], sel);
+      } else if constexpr (GATE) {  // sub-tiles 0 .. 3: two of B's four 32-row blocks, 4 .. 7: the same two of B2's
+        f.sb[e] = __builtin_amdgcn_perm(f.sb_hi[e], f.sbn[e], wn ? 0x07060302u : 0x05040100u);
       } else if constexpr (TB == 2) f.sb[e] = f.sbn[e] >> (16 * wn);
       else f.sb[e] = f.sbn[e];
     });
@@ -1114,6 +1137,67 @@ __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
       });
       return;
     }
+    if constexpr (GATE) {
+      // A lane holds, of row 16 m + li, columns 16 n + 4 lj .. + 3 of both factors.  A 32-column block's maximum is over two
+      // n and the four lanes of a row; four dwords of codes are turned around among those lanes, so that each stores 16
+      // consecutive bytes; the wave's 128 rows of two blocks are one whole 256-byte group of scales, lane 32 b + r
+      // its dword of rows r, r + 32, r + 64, r + 96 of block b.
+      const uint32_t gi = lane_e & 15, gj = lane_e >> 4, ldc = (uint32_t)p.ldd;
+      const bool rceil = p.scale_mode == MX_SCALE_RCEIL;
+      const __amdgpu_buffer_rsrc_t rc = make_rsrc(reinterpret_cast<uint8_t*>(p.d) + (int64_t)t.tm * kEA * p.ldd + t.tn * kEB,
+                                                  (rows_valid < kEA ? rows_valid : kEA) * (int64_t)ldc - t.tn * kEB);
+      const uint32_t v = (wm * 128 + gi) * ldc + wn * 64 + gj * 16;
+      auto rows_max = [](uint32_t x) -> uint32_t {  // over the four lanes of a row
+        const u32x2 a = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        const uint32_t y = max(a.x, a.y);
+        const u32x2 b = __builtin_amdgcn_permlane32_swap(y, y, false, false);
+        return max(b.x, b.y);
+      };
+      uint32_t scales = 0, inside[4];  // (columns of the fill are zeros, also where the row's sums are NaN)
+      static_for<0, 4>([&](auto n_) {
+        inside[decltype(n_)::value] = wn * 64 + 16 * decltype(n_)::value + 4 * gj < cols_valid ? ~0u : 0u;
+      });
+      static_for<0, 8>([&](auto m_) {
+        constexpr int m = decltype(m_)::value;
+        uint32_t g[4][2], top[2] = {0, 0};
+        static_for<0, 4>([&](auto n_) {
+          constexpr int n = decltype(n_)::value;
+          const v4f &c = acc[m][n], &c2 = acc[m][n + 4];
+          const uint32_t a0 = pack_bf16(acc_read<0>(c), acc_read<1>(c)), a1 = pack_bf16(acc_read<2>(c), acc_read<3>(c));
+          const uint32_t b0 = pack_bf16(acc_read<0>(c2), acc_read<1>(c2)), b1 = pack_bf16(acc_read<2>(c2), acc_read<3>(c2));
+          g[n][0] = swiglu2(a0, b0) & inside[n];
+          g[n][1] = swiglu2(a1, b1) & inside[n];
+          top[n >> 1] = pk_max_u16(top[n >> 1], pk_max_u16(g[n][0] & 0x7FFF7FFFu, g[n][1] & 0x7FFF7FFFu));
+          __builtin_amdgcn_sched_barrier(0);
+        });
+        uint32_t sb[2];
+        float mult[2];
+        static_for<0, 2>([&](auto b_) {
+          constexpr int b = decltype(b_)::value;
+          const uint32_t amax = rows_max(max(top[b] & 0xFFFFu, top[b] >> 16));
+          sb[b] = rceil ? scale_byte<MX_SCALE_RCEIL>(amax) : scale_byte<MX_SCALE_FLOOR>(amax);
+          mult[b] = rceil ? scale_multiplier<MX_SCALE_RCEIL>(sb[b]) : scale_multiplier<MX_SCALE_FLOOR>(sb[b]);
+        });
+        uint32_t d[4];
+        static_for<0, 4>([&](auto n_) {
+          constexpr int n = decltype(n_)::value;
+          d[n] = cvt2<true>(g[n][1], mult[n >> 1], cvt2<false>(g[n][0], mult[n >> 1], 0));
+          if (sb[n >> 1] == 255) d[n] = nan_block_codes2(g[n][0]) | (nan_block_codes2(g[n][1]) << 16);
+        });
+        const u32x2 e0 = __builtin_amdgcn_permlane16_swap(d[0], d[1], false, false);
+        const u32x2 e1 = __builtin_amdgcn_permlane16_swap(d[2], d[3], false, false);
+        const u32x2 f0 = __builtin_amdgcn_permlane32_swap(e0.x, e1.x, false, false);
+        const u32x2 f1 = __builtin_amdgcn_permlane32_swap(e0.y, e1.y, false, false);
+        __builtin_amdgcn_raw_buffer_store_b128(u32x4{f0.x, f1.x, f0.y, f1.y}, rc, v, m * 16 * ldc, 0);
+        if ((gj & 1) == (m & 1)) scales |= (gj >> 1 ? sb[1] : sb[0]) << (8 * (m >> 1));
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      if ((int64_t)t.tm * kEA + wm * 128 < p.M) {
+        const int64_t steps = (p.N + 127) / 128 * 2;
+        reinterpret_cast<uint32_t*>(p.d2)[(((int64_t)t.tm * 2 + wm) * steps + t.tn * 2 + wn) * 64 + lane_e] = scales;
+      }
+      return;
+    }
     const uint32_t ldd_b = (uint32_t)p.ldd * 2;
     const __amdgpu_buffer_rsrc_t rd = make_rsrc(t.d, rows_valid * ldd_b);
     // lane's place in a stored piece: row (lane >> 3) + 8*pass, columns (lane & 7)*8 .. +7
@@ -1318,16 +1402,16 @@ static int64_t persistent_grid() {
   return grid;
 }
 
-template <int MODE, bool PROF, bool PAIR = false, int TA = 4, int TB = 4, bool OUT32 = false>
+template <int MODE, bool PROF, bool PAIR = false, int TA = 4, int TB = 4, bool OUT32 = false, bool GATE = false>
 static bool configure32() {
   static std::atomic<bool> configured[kMaxDevices];
-  return raise_lds_limit(reinterpret_cast<const void*>(gemm_nt32_kernel<MODE, PROF, PAIR, TA, TB, OUT32>),
+  return raise_lds_limit(reinterpret_cast<const void*>(gemm_nt32_kernel<MODE, PROF, PAIR, TA, TB, OUT32, GATE>),
                          Lds32<TA, TB>::kBytes, configured);
 }
 bool prepare_dense();
-template <int MODE, bool PROF, bool PAIR = false, int TA = 4, int TB = 4, bool OUT32 = false>
+template <int MODE, bool PROF, bool PAIR = false, int TA = 4, int TB = 4, bool OUT32 = false, bool GATE = false>
 static int launch32(const Gemm32Args& p, int64_t nb, hipStream_t st) {
-  auto kern = gemm_nt32_kernel<MODE, PROF, PAIR, TA, TB, OUT32>;
+  auto kern = gemm_nt32_kernel<MODE, PROF, PAIR, TA, TB, OUT32, GATE>;
   constexpr int lds = Lds32<TA, TB>::kBytes;  // ring + one output patch per wave: most of the CU's 160 KB
   constexpr bool kDenseForm = !PROF && (MODE == kDense || MODE == kSplitK);
   if (!(kDenseForm ? prepare_dense() : configure32<MODE, PROF, PAIR, TA, TB, OUT32>())) return MX_ERR_LAUNCH;
@@ -1563,7 +1647,7 @@ static bool prepare_tile() {
 }
 bool prepare_dense32() {
   return prepare_tile<4, 4>() && prepare_tile<3, 4>() && prepare_tile<4, 3>() && prepare_tile<2, 4>() &&
-         prepare_tile<4, 2>() && configure32<kSplitK, false, false, 4, 4>() &&
+         prepare_tile<4, 2>() && configure32<kDense, false, false, 4, 4, false, true>() && configure32<kSplitK, false, false, 4, 4>() &&
          configure32<kSplitK, false, false, 2, 4>() && configure32<kSplitK, false, false, 4, 2>();
 }
 
@@ -1741,6 +1825,34 @@ int launch_gemm_nt32_pair(const uint8_t* a_codes, const uint8_t* a_scales, const
                a2_codes, a2_scales, b2_codes, b2_scales};
   p.ldk = ldk;
   return launch_best32<true>(p, st);
+}
+
+// Whether the gated product of [M, K] with two weights of N rows leaves its product as codes: where that is predicted to be
+// done before the two products and the cast of their gate.  Fitted to 68 shapes of 129..4096 rows, 1024..14336 columns and
+// K 512..5120 (none got slower, none left more than 4 % behind): 4 us a round for the gate against a launch and its bytes.
+// Full rounds win (3001 x 8192, K 1024 77.9 and 66.3 us; 4096 x 6144, K 2048 107 and 95.5; 1500 x 4992, K 2016 37.5 and
+// 33.0), tiles that leave half of the CUs idle lose to the smaller ones of the two launches (512 x 8192, K 3072 31.6 and 37.4).
+bool plan_gated(int64_t M, int64_t N, int64_t K) {
+  const int64_t grid = persistent_grid(), blocks = K / kKB;
+  if (grid == 0) return false;
+  const DenseTile* t = best_tile(M, N, blocks, 2, grid);
+  if (!t) return false;
+  double us = tiles_us(*t, 2 * tile_count(*t, M, N), blocks, grid) + 2.0;
+  better_ring(M, N, blocks, 2, grid, us);
+  const int64_t tiles = ((M + 255) / 256) * ((N + 127) / 128);
+  const double gated = tiles_us(kDenseTiles[0], tiles, blocks, grid) + 1.0 + 4.0 * ((tiles + grid - 1) / grid);
+  return gated < us + M * N / 0.75e6;
+}
+int launch_gemm_nt32_gated(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes, const uint8_t* b_scales,
+                           const uint8_t* b2_codes, const uint8_t* b2_scales, uint8_t* codes, uint8_t* scales, int64_t M,
+                           int64_t N, int64_t K, int64_t ldk, int64_t ld_codes, int scale_mode, hipStream_t st) {
+  Gemm32Args p{a_codes, a_scales, b_codes, b_scales, (uint16_t*)codes, M, N, K, ld_codes, nullptr, 0, 0, 0, nullptr};
+  p.b2_codes = b2_codes;
+  p.b2_scales = b2_scales;
+  p.d2 = (uint16_t*)scales;
+  p.ldk = ldk;
+  p.scale_mode = scale_mode;
+  return launch32<kDense, false, false, 4, 4, false, true>(p, ((M + 255) / 256) * ((N + 127) / 128), st);
 }
 
 // ... in the slices of `plan`, through `workspace` (slices * M * N floats).

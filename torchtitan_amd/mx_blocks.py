@@ -172,6 +172,10 @@ def ffn_forward(x2, x_src, w1, w2, w3, cfg: MXFP8Config, need_dx: bool, need_dw:
                     else _cast_activation(x2, x_src, cfg.scale_mode, need_cols=need_dw, pitch_pad=pad))
         wqs = cast.weights(ws, ws_cols)
     (w1q0, w1q1), (w3q0, w3q1), (w2q0, w2q1) = wqs
+    if not (need_dx or need_dw):  # nobody reads h1 and h3 again: the gate may run in the product's launch
+        gq0 = ops.mx_gemm_nt_swiglu(xq0, w1q0, w3q0, cfg.scale_mode)
+        if gq0 is not None:
+            return ops.mx_gemm_nt(gq0, w2q0), dict.fromkeys(FFN_SAVED)
     h13 = ops.mx_gemm_nt_shared_a(xq0, w1q0, w3q0)  # one launch: x's panels fetched once for both
     gq0, gq1 = cast.gate(h13, need_dw)
     y = ops.mx_gemm_nt(gq0, w2q0)

@@ -1282,6 +1282,21 @@ def mx_gemm_nt_shared_a(a: MXData, b: MXData, b2: MXData) -> torch.Tensor:
     return out
 
 
+def mx_gemm_nt_swiglu(a: MXData, b: MXData, b2: MXData, mode="floor", planned: bool = False):
+    """The row-wise operand of ``silu(deq(a) @ deq(b)^T) * (deq(a) @ deq(b2)^T)`` in one launch, the same bits as
+    `swiglu_to_operands` makes of `mx_gemm_nt_shared_a`'s products; None where those two launches are predicted to be faster
+    (`planned`: not asked) or the operands are not for it."""
+    if not _operands(a, b, b2) or _watched() or a.depth != b.depth or a.depth != b2.depth or b.rows != b2.rows:
+        return None
+    M, N = a.rows, b.rows
+    if M <= 128 or N <= 128 or N % 8 or not (planned or _lib.load().mx_gemm_nt_swiglu_planned(M, N, a.k)):
+        return None
+    out = _new_operand(M, N, a.ld - a.k, a.buf.device)
+    _call("mx_gemm_nt_swiglu_ld", "gemm_nt_swiglu", out.buf.device, a.codes_ptr, a.scales_ptr, b.codes_ptr, b.scales_ptr,
+          b2.codes_ptr, b2.scales_ptr, out.codes_ptr, out.ld, out.scales_ptr, M, N, a.k, a.ld, _mode(mode), _stream(out.buf))
+    return out
+
+
 def mx_gemm_nt_shared_b(a: MXData, a2: MXData, b: MXData) -> torch.Tensor:
     """bf16 [2, M, N]: deq(a) @ deq(b)^T and deq(a2) @ deq(b)^T, as `mx_gemm_nt_shared_a` with the
     roles of the operands swapped."""

@@ -184,6 +184,24 @@ def test_traced_block_has_the_shapes_that_its_fake_kernel_gives(no_launches, mon
     assert len(set(storages)) == len(storages)
 
 
+@pytest.mark.parametrize("need_dx,need_dw", [(True, True), (True, False), (False, True)])
+def test_traced_linear_has_the_shapes_that_its_fake_kernel_gives(no_launches, need_dx, need_dw):
+    """... also where the weight is frozen, or the input takes no gradient: what is not kept comes to the backward empty."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from torchtitan_amd import compiled
+
+    def run(fwd, bwd):
+        out = fwd(_bf16(2, 96, 160), _bf16(224, 160), 1, need_dx, need_dw, False)
+        return *out, *bwd(_bf16(2, 96, 224), *out[1:], 1, need_dx, need_dw)
+
+    real = run(compiled.mx_linear_fwd._init_fn, compiled.mx_linear_bwd._init_fn)
+    with FakeTensorMode():
+        fake = run(torch.ops.torchtitan_amd.mx_linear_fwd, torch.ops.torchtitan_amd.mx_linear_bwd)
+    assert [t.shape for t in real] == [t.shape for t in fake] and [t.dtype for t in real] == [t.dtype for t in fake]
+    assert real[5].shape == ((192, 160) if need_dx else (0,)) and real[6].shape == ((224, 160) if need_dw else (0,))
+
+
 def test_remembered_activation_cast_stays_on_its_stream(no_launches, monkeypatch):
     """A sibling on the stream that cast the activation takes the codes; one on another stream, whose work is not
     ordered behind that launch, or in another graph capture casts again."""

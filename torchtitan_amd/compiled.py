@@ -90,13 +90,18 @@ def _(x, weight, mode, need_dx=True, need_dw=True, cache_w=False):
             _u8((K, N), dev) if need_dx else _empty(dev), _mfma(K, N // 32, dev) if need_dx else _empty(dev))
 
 
+def _linear_sizes(dy, x_codes_t, w_codes_t, need_dx: bool):
+    """M, K, N of the linear: an operand that no gradient asks for was not kept and is empty."""
+    N = dy.shape[-1]
+    return dy.numel() // N, (w_codes_t if need_dx else x_codes_t).shape[0], N
+
+
 @torch.library.custom_op("torchtitan_amd::mx_linear_bwd", mutates_args=())
 def mx_linear_bwd(dy: torch.Tensor, x_codes_t: torch.Tensor, x_scales_t: torch.Tensor, w_codes_t: torch.Tensor,
                   w_scales_t: torch.Tensor, mode: int, need_dx: bool, need_dw: bool) -> tuple[torch.Tensor, torch.Tensor]:
     """(dX [M, K], dW [N, K]) in bf16 from dY and the saved column-wise forms; an output that is
     not needed comes back empty."""
-    K, M = x_codes_t.shape
-    N = w_codes_t.shape[1]
+    M, K, N = _linear_sizes(dy, x_codes_t, w_codes_t, need_dx)
     name = _MODE_NAMES[mode]
     dy2 = dy.reshape(M, N)
     if dy2.dtype != torch.bfloat16:
@@ -115,8 +120,7 @@ def mx_linear_bwd(dy: torch.Tensor, x_codes_t: torch.Tensor, x_scales_t: torch.T
 
 @mx_linear_bwd.register_fake
 def _(dy, x_codes_t, x_scales_t, w_codes_t, w_scales_t, mode, need_dx, need_dw):
-    K, M = x_codes_t.shape
-    N = w_codes_t.shape[1]
+    M, K, N = _linear_sizes(dy, x_codes_t, w_codes_t, need_dx)
     bf = dict(dtype=torch.bfloat16, device=dy.device)
     return (torch.empty((M, K) if need_dx else (0,), **bf), torch.empty((N, K) if need_dw else (0,), **bf))
 

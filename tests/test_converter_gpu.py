@@ -1110,3 +1110,93 @@ def test_frozen_cached_weights_are_cast_once_with_rows_apart(device, dim, hidden
         outs.append((y, *torch.autograd.grad(y, [xs, *h.parameters()], torch.ones_like(y))))
     assert all(torch.equal(a, b) for a, b in zip(*outs, strict=True))
     mx_tensor._weight_cache.clear()
+
+
+@pytest.mark.parametrize("dim,hidden", [(256, 384), (160, 224)])
+@pytest.mark.parametrize("trained", ["nothing", "an adapter"])
+@pytest.mark.parametrize("first", ["hook", "without gradients", "with gradients", "export", "traced"])
+def test_frozen_weights_with_gradients_through_them(device, dim, hidden, trained, first):
+    """Frozen weights whose casts are cached, read by every kind of caller in turn, whoever is first: the values of weights
+    that are not cached, one entry a weight (in whole 128s, where traced and eager callers share it), and a graph that reads
+    an entry is right after the entry has got its column-wise codes."""
+    import torch._dynamo
+    from torchtitan_amd import mx_blocks, mx_tensor
+    from torchtitan_amd.quantization.mx import export_mxfp8_state_dict
+
+    mx_tensor._weight_cache.clear()
+    gen = torch.Generator(device=device).manual_seed(11)
+    x, dy = (torch.randn(160, dim, generator=gen, device=device).to(torch.bfloat16) for _ in range(2))
+    norm = (torch.randn(dim, generator=gen, device=device) * 0.1 + 1).to(torch.bfloat16)
+    holders, boxes = [], []
+    for cache in (False, True):
+        holder = nn.Module()
+        holder.ff = FeedForward.Config(hidden_dim=hidden).build(dim=dim).to(device).to(torch.bfloat16)
+        if holders:
+            holder.load_state_dict(holders[0].state_dict())
+        else:
+            holder.ff.init_weights(init_std=0.05)
+        boxes.append(_convert(holder, ["ff"], cache=cache, norm=True))
+        holders.append(holder.requires_grad_(False))
+    if trained == "an adapter":
+        holders[1].adapter = nn.Parameter(torch.zeros(4, device=device))
+    entries = lambda: {k[0]: (id(e[5]), id(e[6])) for k, e in mx_tensor._weight_cache._entries.items()}
+
+    def norm_block(ff, t):
+        return mx_blocks.mx_norm_feed_forward(t, norm, 1e-5, ff.w1.weight, ff.w2.weight, ff.w3.weight)
+
+    def norm_linears(ff, t):
+        return torch.cat(mx_blocks.mx_norm_linears(t, norm, 1e-5, (ff.w1.weight, ff.w3.weight)), 1)
+
+    def read(holder, way):
+        torch._dynamo.reset()
+        if way == "export":
+            sent = export_mxfp8_state_dict(nn.ModuleDict({"ff": holder.ff}))
+            return [t for v in sent.values() for t in (v["codes"], v["scales"])]
+        outs = []
+        programs = [lambda t: holder.ff(t), lambda t: holder.ff.w1(t), lambda t: norm_block(holder.ff, t)]
+        if way != "traced":  # (an eager function only)
+            programs.append(lambda t: norm_linears(holder.ff, t))
+        for fn in programs:
+            run = torch.compile(fn, backend="aot_eager", fullgraph=True) if way == "traced" else fn
+            if way != "with gradients":
+                with torch.no_grad():
+                    outs.append(run(x))
+            if way in ("with gradients", "traced"):
+                t = x.clone().requires_grad_(True)
+                y = run(t)
+                outs += [y.detach(), *torch.autograd.grad(y, t, dy.repeat(1, -(-y.shape[1] // dim))[:, :y.shape[1]])]
+            if way == "without gradients":
+                outs.append(run(x))  # (a grad mode in which nothing takes gradients)
+        return outs
+
+    ways = ["without gradients", "with gradients", "export", "traced"]
+    want = {way: read(holders[0], way) for way in ways}
+    if first == "hook":
+        boxes[1].post_optimizer_hook(holders[1])
+        rows_only = trained == "nothing"
+        assert all((e[6] is None) == rows_only for e in mx_tensor._weight_cache._entries.values())
+        ways = [None] + ways
+    else:
+        ways.remove(first)
+        ways.insert(0, first)
+    graph = y = None
+    for turn in range(2):
+        for way in ways:
+            if way is not None:
+                got = read(holders[1], way)
+                assert len(got) == len(want[way]) and all(torch.equal(a, b) for a, b in zip(got, want[way])), (turn, way)
+            if graph is None:  # behind the first reader
+                torch.cuda.synchronize()
+                graph = torch.cuda.CUDAGraph()
+                with torch.no_grad(), torch.cuda.graph(graph):
+                    y = holders[1].ff(x)
+            y.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, want["without gradients"][0]), (turn, way)
+        if turn == 0:
+            made = entries()
+    if dim % 128 == 0:
+        assert len(mx_tensor._weight_cache) == 3
+    assert entries() == made  # the second time nothing was cast
+    mx_tensor._weight_cache.clear()

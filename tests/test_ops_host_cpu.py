@@ -289,3 +289,93 @@ def test_padded_layouts_of_whole_blocks_are_no_whole_512s(pairs, experts):
     assert got % 128 == 0 and got % 512 and need <= got < need + 256
     assert got < need + 128 or (got - 128) % 512 == 0
     assert ops.plan_length(pairs, experts, 32) == need + -need % 32
+
+
+def _frozen_readers(path, weights, norm):
+    """The ways in which a program reads the frozen weights of a linear, of a SwiGLU block or of linears behind a norm:
+    calls that take whether gradients flow through the weights."""
+    from torchtitan_amd import compiled, mx_blocks, mx_tensor
+
+    w1, w2, w3 = weights
+    (H, D), mode = w1.shape, ops.SCALE_MODES["rceil"]
+    plain = [w.as_subclass(torch.Tensor) for w in weights]
+
+    def x(grad, cols=D):
+        return _bf16(160, cols).requires_grad_(grad)
+
+    def block_of_norm(grad):
+        return mx_blocks.mx_norm_feed_forward(x(grad), norm, 1e-5, w1, w2, w3)
+
+    return {
+        "linear": ((w1,), lambda grad: mx_tensor.mx_linear(x(grad), plain[0], None, w1.mx_config, True),
+                   lambda grad: compiled.mx_linear_fwd._init_fn(x(False), plain[0], mode, grad, False, True)),
+        "block": (weights, lambda grad: mx_blocks.mx_feed_forward(x(grad), w1, w2, w3), block_of_norm,
+                  lambda grad: compiled.mx_ffn_fwd._init_fn(x(False), *plain, None, 1e-5, mode, True, grad, False),
+                  lambda grad: compiled.mx_ffn_fwd._init_fn(x(False), *plain, norm, 1e-5, mode, True, grad, False)),
+        "norm and linears": ((w1, w3), lambda grad: mx_blocks.mx_norm_linears(x(grad), norm, 1e-5, (w1, w3)),
+                             lambda grad: mx_tensor.mx_linear(x(grad), plain[0], None, w1.mx_config, True)),
+        "gate and linear": ((w2,), lambda grad: mx_blocks.mx_swiglu_linear(x(grad, H), x(grad, H), w2)),
+    }[path]
+
+
+@pytest.mark.parametrize("path,reader", [("linear", 0), ("linear", 1), ("block", 0), ("block", 1), ("block", 2), ("block", 3),
+                                         ("norm and linears", 0), ("gate and linear", 0)])
+@pytest.mark.parametrize("grad", [False, True])
+def test_a_frozen_weight_is_cast_once_whoever_reads_it(no_launches, monkeypatch, path, reader, grad):
+    """Every forward on cached casts of frozen weights takes the entry that another one has made, with gradients through
+    it or without: each form of a weight is cast once, and no weight has two entries."""
+    from torchtitan_amd import mx_tensor
+
+    cfg = mx_tensor.MXFP8Config(cache_weight_casts=True)
+    weights = [mx_tensor.MXFP8TrainingWeight(_bf16(*shape), cfg) for shape in ((256, 384), (384, 256), (256, 384))]
+    used, *readers = _frozen_readers(path, weights, torch.ones(384, dtype=torch.bfloat16))
+    casts = []
+
+    def call(name, tag, device, *args):
+        if name == "mx_cast_pad":
+            casts.extend((args[0], form) for form, at in (("rows", 5), ("columns", 8)) if args[at] is not None)
+        elif name in ("mx_cast_dim0", "mx_cast_dim0_dim1", "mx_cast_dim0_dim1_ld"):
+            casts.extend((args[0], form) for form in ("rows", "columns")[:1 if name == "mx_cast_dim0" else 2])
+
+    def read(i, grad):
+        with torch.set_grad_enabled(grad):
+            return readers[i](grad)
+
+    monkeypatch.setattr(ops, "_call", call)
+    read(reader, grad)
+    for again in (False, True, False):
+        for i in range(len(readers)):
+            read(i, again)
+    own = {w.data_ptr() for w in used}
+    assert sorted(c for c in casts if c[0] in own) == sorted((p, form) for p in own for form in ("rows", "columns"))
+    assert len(mx_tensor._weight_cache) == len(used)
+    with torch.no_grad():  # (an update leaves no entry of the old values behind)
+        for w in used:
+            w.add_(1)
+    read(0, True), read(0, False)
+    assert len(mx_tensor._weight_cache) == len(used)
+
+
+def test_operands_of_a_frozen_weight_agree_on_their_pitch(no_launches):
+    """... so that no product makes copies of them: forward and backward through an entry with rows apart."""
+    from torchtitan_amd import mx_blocks, mx_tensor
+
+    cfg, seen = mx_tensor.MXFP8Config(cache_weight_casts=True), []
+    weights = [mx_tensor.MXFP8TrainingWeight(_bf16(*shape), cfg) for shape in ((256, 384), (384, 256), (256, 384))]
+    product = ops._operands
+    try:
+        ops._operands = lambda *qs: seen.append(product(*qs)) or seen[-1]
+        with torch.no_grad():  # (makes the entries)
+            mx_blocks.mx_feed_forward(_bf16(160, 384), *weights)
+        h = torch.zeros(160, 256, dtype=torch.bfloat16, requires_grad=True)
+        for run in (lambda x: mx_blocks.mx_feed_forward(x, *weights),
+                    lambda x: mx_tensor.mx_linear(x, weights[0].as_subclass(torch.Tensor), None, cfg, True),
+                    lambda x: mx_blocks.mx_swiglu_linear(h, h, weights[1])):
+            x = torch.zeros(160, 384, dtype=torch.bfloat16, requires_grad=True)
+            y = run(x)
+            y.backward(torch.zeros_like(y))
+    finally:
+        ops._operands = product
+    assert seen and all(seen)
+    assert all(e[5].ld == e[5].k + ops.CODE_PITCH_PAD and e[6].ld == e[6].k + ops.CODE_PITCH_PAD
+               for e in mx_tensor._weight_cache._entries.values())

@@ -54,7 +54,7 @@ def mx_linear_fwd(x: torch.Tensor, weight: torch.Tensor, mode: int, need_dx: boo
     (codes [K, M], MFMA-order scales; empty unless `need_dw`) and of W (codes [K, N], MFMA-order
     scales; empty unless `need_dx`).  Without gradients only the row-wise casts run.  `cache_w`:
     the weight's casts come from, and go to, the cache of unchanged weights."""
-    from .mx_tensor import _cast_weight, _rounded_up, frozen_rows
+    from .mx_tensor import _cast_weight, _rounded_up, rows_apart
 
     M, K, N = _dims(x, weight)
     name = _MODE_NAMES[mode]
@@ -62,10 +62,12 @@ def mx_linear_fwd(x: torch.Tensor, weight: torch.Tensor, mode: int, need_dx: boo
     if x2.dtype != torch.bfloat16:
         x2 = x2.to(torch.bfloat16)
     x2 = x2.contiguous()
-    frozen = frozen_rows(weight, name) if cache_w and not (need_dx or need_dw or _rounded_up(weight)) else None
-    if frozen is not None:
-        y = ops.mx_gemm_nt(ops.to_operands(x2, name, True, False, frozen.ld - frozen.k)[0], frozen)
-        return (y.view(*x.shape[:-1], N), *(_empty(x.device) for _ in range(4)))
+    if cache_w and not need_dw and not _rounded_up(weight) and rows_apart(weight, name):
+        wq0, wq1 = _cast_weight(weight, name, need_dx, _block_cfg(mode, cache_w), ops.CODE_PITCH_PAD)
+        y = ops.mx_gemm_nt(ops.to_operands(x2, name, True, False, ops.CODE_PITCH_PAD)[0], wq0)
+        e = lambda: _empty(x.device)
+        return (y.view(*x.shape[:-1], N), e(), e(), wq1.codes.clone() if need_dx else e(),
+                wq1.scales.clone() if need_dx else e())
     if need_dw:
         xq0, xq1 = ops.to_mx_dim0_dim1(x2, name, MX_SCALES_MFMA)
     else:
@@ -458,13 +460,19 @@ def mx_ffn_fwd(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, w3: torch.Te
     """(y, 14 tensors for the backward) of the SwiGLU block w2(silu(w1 x) * w3 x), RMSNorm in front
     when `norm_weight` is given."""
     from . import mx_blocks
+    from .mx_tensor import rows_apart
 
     D = x.shape[-1]
     x2 = x.reshape(-1, D)
     if x2.dtype != torch.bfloat16:
         x2 = x2.to(torch.bfloat16)
-    y, saved = mx_blocks.ffn_forward(x2, None, w1, w2, w3, _block_cfg(mode, cache_w), need_dx, need_dw, norm_weight, eps,
-                                     whole_blocks=_ffn_whole_blocks(x2.shape[0], D, w1.shape[0], w2.shape[0]))
+    cfg, wqs, pad = _block_cfg(mode, cache_w), None, 0
+    whole = _ffn_whole_blocks(x2.shape[0], D, w1.shape[0], w2.shape[0])
+    if cache_w and not need_dw and all(rows_apart(w, cfg.scale_mode) for w in (w1, w2, w3)):
+        whole = True
+        wqs, pad = mx_blocks.cached_ffn_weights(w1, w2, w3, cfg, need_dx, need_dw, frozen=True)
+    y, saved = mx_blocks.ffn_forward(x2, None, w1, w2, w3, cfg, need_dx, need_dw, norm_weight, eps, pad=pad,
+                                     whole_blocks=whole, wqs=wqs)
     for name in _FFN_PAIRS:  # an operator's outputs are their own: not the cache's tensors, nor parts of one buffer
         q = saved[name]
         if type(q) is ops.Operand or (q is not None and cache_w and name in ("w1", "w2", "w3")):

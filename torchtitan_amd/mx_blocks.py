@@ -13,8 +13,16 @@ import torch.nn.functional as F
 from . import _lib, ops
 from .mx_tensor import (MXFP8Config, MXFP8TrainingWeight, _cast_activation, _cast_activation_and_weights, _cast_cache,
                         _cast_into_groups, _cast_weight, _cast_weights, _castable, _grouped_2d3d_padded, _one_launch,
-                        _pad_plan, _rounded_up, _unwrap, frozen_rows, rows_apart)
+                        _pad_plan, _unwrap, cached_weights)
 from .ops import MX_SCALES_MFMA, MX_SCALES_ROWMAJOR, MXData
+
+
+def _weights_and_pitch(ws, need_cols: bool, cfg: MXFP8Config):
+    """(casts of the matrices, bytes between the rows of their codes) for a function without a pitch of its own."""
+    if cfg.cache_weight_casts:
+        return cached_weights(ws, cfg.scale_mode, [need_cols] * len(ws), cfg)
+    return [_cast_weight(w, cfg.scale_mode, need_cols, cfg) for w in ws], 0
+
 
 # ----------------------------------------------------------------------------- SwiGLU + linear
 class _MXSwiGLULinear(torch.autograd.Function):
@@ -28,10 +36,10 @@ class _MXSwiGLULinear(torch.autograd.Function):
         mode = cfg.scale_mode
         H, N = h1.shape[-1], weight.shape[0]
         need_dh, need_dw = ctx.needs_input_grad[0] or ctx.needs_input_grad[1], ctx.needs_input_grad[2]
-        gq0, gq1 = ops.swiglu_to_operands(h1.reshape(-1, H), h3.reshape(-1, H), mode, need_dw)
-        wq0, wq1 = _cast_weight(weight, mode, need_dh, cfg)
+        ((wq0, wq1),), pad = _weights_and_pitch((weight,), need_dh, cfg)
+        gq0, gq1 = ops.swiglu_to_operands(h1.reshape(-1, H), h3.reshape(-1, H), mode, need_dw, pad)
         y = ops.mx_gemm_nt(gq0, wq0)
-        ctx.cfg, ctx.w_dtype = cfg, weight.dtype
+        ctx.cfg, ctx.w_dtype, ctx.pad = cfg, weight.dtype, pad
         ctx.g_layout, ctx.w_layout = (gq1.layout if need_dw else None), (wq1.layout if need_dh else None)
         ctx.save_for_backward(h1, h3, gq1.buf if need_dw else None, wq1.buf if need_dh else None)
         return y.view(*h1.shape[:-1], N)
@@ -42,7 +50,7 @@ class _MXSwiGLULinear(torch.autograd.Function):
         need_dh = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
         need_dw = ctx.needs_input_grad[2]
         h1, h3, g_buf, w_buf = ctx.saved_tensors
-        dyq0, dyq1 = ops.to_operands(_castable(_rows_of(dy)), mode, need_dh, need_dw)
+        dyq0, dyq1 = ops.to_operands(_castable(_rows_of(dy)), mode, need_dh, need_dw, ctx.pad)
         dh1 = dh3 = dw = None
         if need_dh:
             dg = ops.mx_gemm_nt(dyq0, ops.saved_operand(w_buf, ctx.w_layout, dy.device)).view(h1.shape)
@@ -103,8 +111,8 @@ FFN_SAVED = ("h13", "w2", "x", "g", "w1", "w3", "norm_x", "rstd", "norm_weight")
 
 def block_pitch_pad(cfg: MXFP8Config, need_dx: bool, need_dw: bool) -> int:
     """Bytes the eager SwiGLU block leaves between the rows of its MXFP8 codes: ops.CODE_PITCH_PAD
-    in a training step; none with cached weight casts, whose entries other callers read as dense
-    codes."""
+    in a training step; none of its own with cached weight casts, whose pitch it takes
+    (`cached_weights`)."""
     return ops.CODE_PITCH_PAD if need_dx and need_dw and not cfg.cache_weight_casts else 0
 
 
@@ -143,20 +151,22 @@ class _FFNCasts:
         return ops.rms_norm_to_mx(x2, _bf16(weight), eps, self.mode, MX_SCALES_MFMA)[:3]
 
 
+def cached_ffn_weights(w1, w2, w3, cfg: MXFP8Config, need_dx: bool, need_dw: bool, frozen: bool = False):
+    """`cached_weights` of w1, w3 and w2 as `ffn_forward` takes them."""
+    return cached_weights((w1, w3, w2), cfg.scale_mode, (need_dx, need_dx, need_dx or need_dw), cfg, frozen)
+
+
 def ffn_forward(x2, x_src, w1, w2, w3, cfg: MXFP8Config, need_dx: bool, need_dw: bool, norm_weight=None,
-                eps: float = 0.0, pad: int = 0, whole_blocks: bool = False):
+                eps: float = 0.0, pad: int = 0, whole_blocks: bool = False, wqs=None):
     """Forward of the SwiGLU block on a 2-D bf16 activation: (y [M, out], dict of what FFN_SAVED names).
     `x_src` is the tensor the activation-cast cache is keyed on (None: no sharing of x's cast
     with sibling linears); `pad`: the row pitch padding of every code matrix (the saved ones
-    carry it into the backward); `whole_blocks`: see `_FFNCasts`.  The eager autograd function and
-    the traced operator both run this."""
-    if (x_src is None and cfg.cache_weight_casts and not (need_dx or need_dw)
-            and not any(_rounded_up(w) or frozen_rows(w, cfg.scale_mode) is None for w in (w1, w2, w3))):
-        whole_blocks, pad = True, ops.CODE_PITCH_PAD  # (traced, behind a hook that has cast frozen weights)
+    carry it into the backward); `whole_blocks`: see `_FFNCasts`; `wqs`: the casts of w1, w3 and w2, where the caller
+    has them, with the pitch `pad`.  The eager autograd function and the traced operator both run this."""
     cast = _FFNCasts(cfg, whole_blocks, pad)
     if (whole_blocks and norm_weight is None and not (need_dx or need_dw)
             and ops.few_rows_ok(x2, w1.shape[0] + w3.shape[0])):
-        (w1q0, _), (w3q0, _), (w2q0, _) = cast.weights((w1, w3, w2), (False, False, False))
+        (w1q0, _), (w3q0, _), (w2q0, _) = wqs or cast.weights((w1, w3, w2), (False, False, False))
         h13 = ops.mx_few_rows(x2, w1q0, cfg.scale_mode, w3q0)
         return ops.mx_gemm_nt(cast.gate(h13, False)[0], w2q0), dict.fromkeys(FFN_SAVED)
     rstd = None
@@ -164,13 +174,13 @@ def ffn_forward(x2, x_src, w1, w2, w3, cfg: MXFP8Config, need_dx: bool, need_dw:
     if norm_weight is not None:  # RMSNorm in front: normalised inside the cast, rstd kept for its backward
         x2 = x2.contiguous()
         xq0, xq1, rstd = cast.norm(x2, norm_weight, eps)
-        wqs = cast.weights(ws, ws_cols)
-    elif x_src is not None and need_dx:
+        wqs = wqs or cast.weights(ws, ws_cols)
+    elif x_src is not None and need_dx and wqs is None:
         (xq0, xq1), *wqs = _cast_activation_and_weights(x2, x_src, ws, cfg.scale_mode, need_dx, need_dw, cfg, pad)
     else:
         xq0, xq1 = (cast.plain(x2, need_dw) if x_src is None
                     else _cast_activation(x2, x_src, cfg.scale_mode, need_cols=need_dw, pitch_pad=pad))
-        wqs = cast.weights(ws, ws_cols)
+        wqs = wqs or cast.weights(ws, ws_cols)
     (w1q0, w1q1), (w3q0, w3q1), (w2q0, w2q1) = wqs
     if not (need_dx or need_dw):  # nobody reads h1 and h3 again: the gate may run in the product's launch
         gq0 = ops.mx_gemm_nt_swiglu(xq0, w1q0, w3q0, cfg.scale_mode)
@@ -247,8 +257,11 @@ class _MXFeedForward(torch.autograd.Function):
                     ctx.native, ctx.layouts = True, [None, *rest[1::2], None, None, None]
                     ctx.save_for_backward(h13, *rest[::2], None, None, None)
                     return y if x.dim() == 2 else y.view(*x.shape[:-1], w2.shape[0])
+        wqs = None
+        if cfg.cache_weight_casts:
+            wqs, ctx.pad = cached_ffn_weights(w1, w2, w3, cfg, need_dx, need_dw)
         y, saved = ffn_forward(_rows_of(x), x, w1, w2, w3, cfg, need_dx, need_dw, norm_weight, eps, pad=ctx.pad,
-                               whole_blocks=True)
+                               whole_blocks=True, wqs=wqs)
         ctx.layouts = [q.layout if isinstance(q, ops.Operand) else None for q in saved.values()]
         ctx.save_for_backward(*[q.buf if isinstance(q, ops.Operand) else q for q in saved.values()])
         return y if x.dim() == 2 else y.view(*x.shape[:-1], w2.shape[0])
@@ -310,9 +323,12 @@ def _feed_forward(x, w1, w2, w3, bias2, norm_weight, eps: float):
         if torch.is_grad_enabled() or ops._transformed():
             y = _MXFeedForward.apply(x, w1, w2, w3, w2.mx_config, norm_weight, eps)
         else:  # nothing is kept for a backward
-            cfg = w2.mx_config
-            pad = rows_apart(cfg, not (w1.requires_grad or w2.requires_grad or w3.requires_grad))
-            y, _ = ffn_forward(_rows_of(x), x, w1, w2, w3, cfg, False, False, norm_weight, eps, pad=pad, whole_blocks=True)
+            cfg, wqs, pad = w2.mx_config, None, ops.CODE_PITCH_PAD
+            if cfg.cache_weight_casts:
+                frozen = not (w1.requires_grad or w2.requires_grad or w3.requires_grad)
+                wqs, pad = cached_ffn_weights(w1, w2, w3, cfg, False, False, frozen)
+            y, _ = ffn_forward(_rows_of(x), x, w1, w2, w3, cfg, False, False, norm_weight, eps, pad=pad, whole_blocks=True,
+                               wqs=wqs)
             y = y if x.dim() == 2 else y.view(*x.shape[:-1], w2.shape[0])
         if bias2 is not None:
             y = y + bias2.to(y.dtype)
@@ -340,11 +356,11 @@ class _MXNormLinears(torch.autograd.Function):
         mode = cfg.scale_mode
         D = x.shape[-1]
         x2 = x.reshape(-1, D).contiguous()
-        hq0, hq1, rstd = ops.rms_norm_to_operands(x2, _bf16(norm_weight), eps, mode)
         need_dh = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
+        wqs, ctx.pad = _weights_and_pitch(weights, need_dh, cfg)
+        hq0, hq1, rstd = ops.rms_norm_to_operands(x2, _bf16(norm_weight), eps, mode, ctx.pad)
         outs, saved, ctx.layouts = [], [x2, rstd, norm_weight, hq1.buf], [hq1.layout]
-        for w in weights:
-            wq0, wq1 = _cast_weight(w, mode, need_dh, cfg)
+        for w, (wq0, wq1) in zip(weights, wqs):
             outs.append(ops.mx_gemm_nt(hq0, wq0).view(*x.shape[:-1], w.shape[0]))
             if need_dh:
                 saved.append(wq1.buf)
@@ -366,7 +382,7 @@ class _MXNormLinears(torch.autograd.Function):
             if dy is None or not (ctx.need_dh or need_dw):
                 dws.append(None)
                 continue
-            dyq0, dyq1 = ops.to_operands(_castable(_rows_of(dy)), mode, ctx.need_dh, need_dw)
+            dyq0, dyq1 = ops.to_operands(_castable(_rows_of(dy)), mode, ctx.need_dh, need_dw, ctx.pad)
             if ctx.need_dh:
                 part = ops.mx_gemm_nt(dyq0, wqs[i])
                 dh = part if dh is None else dh + part

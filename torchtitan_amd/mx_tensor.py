@@ -147,7 +147,8 @@ class _WeightCastCache:
     in-place update (optimizer step, ``copy_``, init) invalidates it.  A cast made under graph capture
     exists once that graph has run: its entry serves that capture only.  A hit on another stream than the
     one that cast orders that stream behind the cast.  Off unless the converter
-    is built with ``cache_weight_casts=True``; holds 2 bytes per weight element."""
+    is built with ``cache_weight_casts=True``; holds 2 bytes per weight element, 1 where only forwards without gradients
+    have read a frozen weight (`cached_weights`)."""
 
     def __init__(self):
         self._entries = {}
@@ -170,13 +171,15 @@ class _WeightCastCache:
     def put(self, w: torch.Tensor, mode, rows: MXData, cols):
         from torch.multiprocessing.reductions import StorageWeakRef
 
-        dead = [k for k, e in self._entries.items() if e[0].expired()]
+        own = self._key(w, mode)
+        dead = [k for k, e in self._entries.items()  # (also the form with another pitch of a weight since updated)
+                if e[0].expired() or (e[1] != w._version and k[:4] == own[:4] and k[4][::2] == mode[::2])]
         for k in dead:
-            del self._entries[k]
+            self._entries.pop(k, None)
         capture, stream, done = _capture(w), None, None
         if w.is_cuda and not capture:
             stream, done = (w.device.index, ops._stream(w)), torch.cuda.current_stream(w.device).record_event()
-        self._entries[self._key(w, mode)] = (StorageWeakRef(w.untyped_storage()), w._version, capture, stream, done, rows, cols)
+        self._entries[own] = (StorageWeakRef(w.untyped_storage()), w._version, capture, stream, done, rows, cols)
 
     def clear(self):
         self._entries.clear()
@@ -194,8 +197,8 @@ def _cast_weight(w: torch.Tensor, mode: str, need_cols: bool, cfg: MXFP8Config, 
     scale order.  2-D weights: GEMM operands as `ops.to_operands` makes them (the contraction in whole
     128-deep blocks, `pitch_pad` bytes between the rows); with `whole_blocks` off the dense form
     over exactly N and K.  The column-wise form of a stack or a dense form exists when asked for and
-    N is a multiple of 32.  Cached, both forms are made for whoever asks first, but of padded rows, which forwards
-    without gradients alone read (`rows_apart`)."""
+    N is a multiple of 32.  Cached, both forms are made for whoever asks first, but with padded rows: there the
+    column-wise one joins the entry when it is first asked for (see `cached_weights`)."""
     cached = cfg.cache_weight_casts
     whole = whole_blocks and w.dim() == 2
     # the cache keeps padded, rounded-up and dense casts apart; where nothing is rounded the last two have the
@@ -203,8 +206,8 @@ def _cast_weight(w: torch.Tensor, mode: str, need_cols: bool, cfg: MXFP8Config, 
     key = (mode, pitch_pad, whole and _rounded_up(w))
     if cached:
         hit = _weight_cache.get(w, key)
-        if hit is not None and (hit[1] is not None or not need_cols or w.shape[-2] % ops.BLOCK):
-            return hit if (type(hit[0]) is ops.Operand) == whole else _in_form(w, key, hit, whole)
+        if hit is not None and (hit[1] is not None or not need_cols or whole or w.shape[-2] % ops.BLOCK):
+            return _as_asked(w, key, hit, need_cols, whole)
         need_cols = need_cols or not pitch_pad  # cast once in full, whoever asks first
     wb = (_castable(w) if whole else w if w.dtype == torch.bfloat16 else w.to(torch.bfloat16)).contiguous()
     both = need_cols and (whole or wb.shape[-2] % ops.BLOCK == 0)
@@ -220,26 +223,56 @@ def _cast_weight(w: torch.Tensor, mode: str, need_cols: bool, cfg: MXFP8Config, 
     return q
 
 
-def rows_apart(cfg: MXFP8Config, frozen: bool) -> int:
-    """Bytes that a forward without gradients leaves between the rows of its codes: none where the cast of a weight that
-    is being trained is cached, whose dense entry the training steps, traced callers and the hand-over share.  A `frozen`
-    weight's entry is for such forwards only.  Rows a whole number of KB long lie on few channels of the L2 and of the
-    memory: 512 tokens 4096 -> 2 x 14336 59.7 us on dense rows from memory, 52.0 on these; 14336 -> 4096 52.0 and 47.7."""
-    return 0 if cfg.cache_weight_casts and not frozen else ops.CODE_PITCH_PAD
+def cached_weights(ws, mode: str, need_cols, cfg: MXFP8Config, frozen: bool = False):
+    """(`_cast_weight` of every matrix as whole-block operands, bytes between the rows of their codes) for an eager forward
+    on cached casts: all operands of a product have one pitch, so the forward casts its activations with this one.
+
+    The casts that are there are taken as they lie, whoever made them, so that a weight is cast once and kept in one
+    form; column-wise codes that a backward needs join an entry that has none.  Where there are none yet, a forward
+    without gradients on `frozen` weights leaves rows apart and casts row-wise only (as `post_optimizer_hook` does on a
+    model that takes no gradients at all), anyone else makes the dense form, which traced callers share.
+    Rows a whole number of KB long lie on few channels of the L2 and of the memory: 512 tokens 4096 -> 2 x 14336
+    59.7 us on dense rows from memory, 52.0 on rows apart; 14336 -> 4096 52.0 and 47.7."""
+    dense = False
+    for pad in ((ops.CODE_PITCH_PAD, 0) if frozen else (0, ops.CODE_PITCH_PAD)):
+        found = []
+        for w in ws:
+            key = (mode, pad, _rounded_up(w))
+            hit = _weight_cache.get(w, key)
+            if hit is not None:
+                found.append((w, key, hit))
+            elif pad:
+                break
+        if len(found) == len(ws):
+            return [_as_asked(*each, need, True) for each, need in zip(found, need_cols)], pad
+        dense = dense or (pad == 0 and len(found) > 0)
+    pad = ops.CODE_PITCH_PAD if frozen and not dense else 0
+    return [_cast_weight(w, mode, need, cfg, pad) for w, need in zip(ws, need_cols)], pad
 
 
-def frozen_rows(w: torch.Tensor, mode: str):
-    """The cached row-wise operand, rows apart, of a frozen weight, where there is one: for traced forwards without
-    gradients and the hand-over, so that they do not cast what `post_optimizer_hook` has cast."""
-    if w.dim() != 2 or not ops.CODE_PITCH_PAD:
-        return None
-    hit = _weight_cache.get(w, (mode, ops.CODE_PITCH_PAD, _rounded_up(w)))
-    return None if hit is None else hit[0]
+def rows_apart(w: torch.Tensor, mode: str) -> bool:
+    """The cache holds operands of the matrix with rows apart: for traced callers, so that they do not cast what
+    `post_optimizer_hook` or a forward without gradients has cast."""
+    return (w.dim() == 2 and ops.CODE_PITCH_PAD > 0
+            and _weight_cache.get(w, (mode, ops.CODE_PITCH_PAD, _rounded_up(w))) is not None)
 
 
 def _rounded_up(w: torch.Tensor) -> bool:
     """Whole-block operands of the matrix are larger than dense ones."""
     return bool(w.shape[0] % ops.WHOLE_BLOCK or w.shape[1] % ops.WHOLE_BLOCK)
+
+
+def _as_asked(w: torch.Tensor, key, hit, need_cols: bool, whole: bool):
+    """A cached cast as its caller wants it: in its form, with the column-wise codes.  Those that are cast now join the entry,
+    whose row-wise codes stay where they lie (a graph may read them), except under graph capture, where only the replay
+    fills them."""
+    if (type(hit[0]) is ops.Operand) != whole:
+        hit = _in_form(w, key, hit, whole)
+    if need_cols and whole and hit[1] is None:
+        hit = hit[0], ops.to_operands(_castable(w).contiguous(), key[0], False, True, hit[0].ld - hit[0].k)[1]
+        if not (w.is_cuda and torch.cuda.is_current_stream_capturing()):
+            _weight_cache.put(w, key, *hit)
+    return hit
 
 
 def _in_form(w: torch.Tensor, key, hit, whole: bool):
@@ -305,17 +338,25 @@ def _castable(t: torch.Tensor) -> torch.Tensor:
     return t if t.dtype in (torch.bfloat16, torch.float32) else t.to(torch.bfloat16)
 
 
-def _linear_apply(x2: torch.Tensor, src: torch.Tensor, weight: torch.Tensor, cfg: MXFP8Config, K: int, N: int, pad: int):
+def _linear_apply(x2: torch.Tensor, src: torch.Tensor, weight: torch.Tensor, cfg: MXFP8Config, K: int, N: int, frozen: bool):
     """x2 W^T without gradients.  The activation's cast is shared with sibling linears on `src`, but for few rows, which are
     cast inside their product; the weight is cast once, whichever way the product runs."""
-    mode = cfg.scale_mode
+    mode, pad = cfg.scale_mode, ops.CODE_PITCH_PAD
+    if cfg.cache_weight_casts:
+        for pad in ((pad, 0) if frozen else (0, pad)):  # (what `cached_weights` finds, 1.5 us sooner)
+            wq0, _ = _weight_cache.get(weight, (mode, pad, _rounded_up(weight))) or (None, None)
+            if type(wq0) is ops.Operand:
+                break
+        else:
+            ((wq0, _),), pad = cached_weights((weight,), mode, (False,), cfg, frozen)
+    else:
+        wq0, _ = _cast_weight(weight, mode, False, cfg, pitch_pad=pad)
     native = ops.native_block_ok(x2, K, N)
     if native:  # (what else `few_rows_ok` asks for, the native call checks itself)
         few = x2.dtype == torch.bfloat16 and ops.few_rows_size(x2.shape[0], K, N)
         native = few or _cast_cache.get(src, (mode, pad)) is None
     else:
         few = ops.few_rows_ok(x2, N)
-    wq0, _ = _cast_weight(weight, mode, False, cfg, pitch_pad=pad)
     if native and type(wq0) is ops.Operand:
         out = _lib.blocks().linear_apply(x2, wq0.buf, wq0.scales_buf, wq0.layout, ops._mode(mode), few)
         if out is not None:
@@ -330,23 +371,26 @@ def _linear_apply(x2: torch.Tensor, src: torch.Tensor, weight: torch.Tensor, cfg
 
 
 def _linear_forward(x, weight, cfg: MXFP8Config, need_dx: bool, need_dw: bool, frozen: bool = False):
-    """(y, column-wise x or None, column-wise W or None) of the converted linear; `frozen`: see `rows_apart`."""
+    """(y, column-wise x or None, column-wise W or None) of the converted linear; `frozen`: see `cached_weights`."""
     mode, K, N = cfg.scale_mode, x.shape[-1], weight.shape[0]
     x2 = _castable(x if x.dim() == 2 else x.reshape(-1, K))
-    # rows further apart than they are long, except with cached weight casts, which the fused
-    # blocks and the hand-over share without a pitch
-    pad = 0 if cfg.cache_weight_casts else ops.CODE_PITCH_PAD
     if not (need_dx or need_dw):
-        y = _linear_apply(x2, x, weight, cfg, K, N, rows_apart(cfg, frozen))
+        y = _linear_apply(x2, x, weight, cfg, K, N, frozen)
         return (y if x.dim() == 2 else y.view(*x.shape[:-1], N)), None, None
-    if need_dx and need_dw and pad and ops.native_block_ok(x2, K, N) and _cast_cache.get(x, (mode, pad)) is None:
+    # rows further apart than they are long, except with cached weight casts, which have a pitch of their own
+    cached, pad = cfg.cache_weight_casts, ops.CODE_PITCH_PAD
+    if need_dx and need_dw and pad and not cached and ops.native_block_ok(x2, K, N) and _cast_cache.get(x, (mode, pad)) is None:
         out = _lib.blocks().linear_forward(x2, _castable(weight), ops._mode(mode), pad)
         if out is not None:
             y, xr, xr_layout, xc, xc_layout, wc, wc_layout = out
             xq1 = ops.Operand(xc, xc_layout)
             _cast_cache.put(x, (mode, pad), (ops.Operand(xr, xr_layout), xq1))
             return (y if x.dim() == 2 else y.view(*x.shape[:-1], N)), xq1, ops.Operand(wc, wc_layout)
-    (xq0, xq1), (wq0, wq1) = _cast_activation_and_weights(x2, x, (weight,), mode, need_dx, need_dw, cfg, pad)
+    if cached:
+        ((wq0, wq1),), pad = cached_weights((weight,), mode, (need_dx,), cfg)
+        xq0, xq1 = _cast_activation(x2, x, mode, need_cols=need_dw, pitch_pad=pad)
+    else:
+        (xq0, xq1), (wq0, wq1) = _cast_activation_and_weights(x2, x, (weight,), mode, need_dx, need_dw, cfg, pad)
     y = ops.mx_gemm_nt(xq0, wq0)
     return (y if x.dim() == 2 else y.view(*x.shape[:-1], N)), xq1, wq1
 
@@ -361,6 +405,9 @@ class _MXLinear(torch.autograd.Function):
         ctx.x_dtype = x.dtype
         ctx.w_dtype = weight.dtype
         ctx.x_layout, ctx.w_layout = (xq1.layout if need_dw else None), (wq1.layout if need_dx else None)
+        if need_dx or need_dw:  # the backward's casts take the pitch of the operands that they meet
+            kept = wq1 if need_dx else xq1
+            ctx.pad = kept.ld - kept.k
         ctx.save_for_backward(xq1.buf if need_dw else None, wq1.buf if need_dx else None)
         return y
 
@@ -371,7 +418,7 @@ class _MXLinear(torch.autograd.Function):
         need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         x_buf, w_buf = ctx.saved_tensors
         dy2 = _castable(dy if dy.dim() == 2 else dy.reshape(-1, dy.shape[-1]))
-        pad = 0 if ctx.cfg.cache_weight_casts else ops.CODE_PITCH_PAD
+        pad = ctx.pad
         dx = dw = None
         if need_dx and need_dw and pad and ops.native_block_ok(dy2, dy2.shape[1], ctx.x_shape[-1]):
             out = _lib.blocks().linear_backward(dy2, x_buf, ctx.x_layout, w_buf, ctx.w_layout, ops._mode(mode), pad,

@@ -20,7 +20,7 @@ import torch.nn as nn
 
 from .. import _lib
 from ..modules.linear import Linear
-from ..mx_tensor import MXFP8Config, MXFP8TrainingWeight, _cast_weight, frozen_rows, rows_apart, wrap_parameter
+from ..mx_tensor import MXFP8Config, MXFP8TrainingWeight, _cast_weight, cached_weights, wrap_parameter
 from . import QuantizationConverter
 from .module_utils import capture_module_attrs, inject_module_protocol, verify_module_protocol
 from .utils import module_filter_fn
@@ -97,7 +97,8 @@ class MXFP8Converter(QuantizationConverter):
 
         cache_weight_casts: bool = False
         """Not in the reference's Config.  Keep the MXFP8 forms of a converted weight until the
-        weight is next updated in place (2 extra bytes per weight element): `post_optimizer_hook`
+        weight is next updated in place (2 extra bytes per weight element; 1 in a model that takes no
+        gradients, until one is asked for through it): `post_optimizer_hook`
         then casts every converted weight once per optimizer step, and every forward until the
         next step (gradient accumulation, evaluation, several micro-batches) and
         `export_mxfp8_state_dict` reuse those codes."""
@@ -182,13 +183,18 @@ class MXFP8Converter(QuantizationConverter):
         optimizer step, for the forwards that follow and for a hand-over in MXFP8 form."""
         if not self.enabled or not self.config.cache_weight_casts:
             return
-        for m in model if isinstance(model, (list, tuple)) else [model]:
-            for p in m.parameters():
+        params = [p for m in (model if isinstance(model, (list, tuple)) else [model]) for p in m.parameters()]
+        # Nothing is trained: forwards without gradients alone, row-wise casts.  A frozen weight among trained ones
+        # (adapters, a partly frozen model) is cast in both forms: gradients go through it.
+        trained = any(p.requires_grad for p in params)
+        with torch.no_grad():
+            for p in params:
                 if isinstance(p, MXFP8TrainingWeight) and p.is_cuda:
-                    # frozen weights for forwards without gradients alone: row-wise, rows apart
-                    pad = rows_apart(p.mx_config, not p.requires_grad) if p.dim() == 2 else 0
-                    with torch.no_grad():
-                        _cast_weight(p.as_subclass(torch.Tensor), p.mx_config.scale_mode, not pad, p.mx_config, pad)
+                    w, cfg = p.as_subclass(torch.Tensor), p.mx_config
+                    if p.dim() == 2:
+                        cached_weights((w,), cfg.scale_mode, (trained,), cfg, not trained)
+                    else:
+                        _cast_weight(w, cfg.scale_mode, True, cfg)
 
 
 MXFP8_PAYLOAD_FORMAT = "mxfp8:e4m3fn+e8m0:block32:dim-1"
@@ -232,8 +238,9 @@ def _rows_from_cache(p: torch.Tensor, cfg: MXFP8Config):
     is none)."""
     from .. import ops
 
-    rows = frozen_rows(p, cfg.scale_mode) if not p.requires_grad else None
-    if rows is None:
+    if p.dim() == 2:
+        ((rows, _),), _ = cached_weights((p,), cfg.scale_mode, (False,), cfg)
+    else:
         rows, _ = _cast_weight(p, cfg.scale_mode, False, cfg)
     codes, laid = rows.codes, rows.scales
     lead, K = p.shape[:-1], p.shape[-1]

@@ -192,8 +192,13 @@ __global__ __launch_bounds__(256, 1) void gemm_ring_kernel(RingArgs p) {
   }
   if (s < total) step(f0, f1);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the copies behind the last block
-  // (the compiler does not know the assembly above for MFMAs: what reads the accumulators waits for the last one's passes)
+  // The compiler does not know the assembly above for MFMAs: what reads the accumulators waits for the last one's passes,
+  // and comes from here, so that no copy out of them is placed ahead of the wait.
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+  for (int m = 0; m < TM; ++m)
+#pragma unroll
+    for (int n = 0; n < TN; ++n) asm volatile("" : "+a"(acc[m][n]));
 
   // ---- out: a lane holds row 16 m + li, columns 16 n + 4 lj .. + 3 of sub-tile (m, n)
   const int size = p.f32 ? 4 : 2;

@@ -188,6 +188,23 @@ def test_routed_experts(device, monkeypatch, experts, top_k, shared, tokens, bef
         assert "routed_forward" in taken and "routed_backward" in taken
 
 
+@pytest.mark.parametrize("tokens,rows", [(127, 512), (128, 512), (640, 1664), (641, 1664), (896, 2048)])
+def test_routed_experts_lay_out_the_planned_rows(device, monkeypatch, tokens, rows):
+    """The padded layout of the native call has the rows of the general one, also where its bound is a whole number of 512."""
+    torch.manual_seed(tokens)
+    moe = _block("experts", device)
+    x, dy = (torch.randn(1, tokens, 256, device=device, dtype=torch.bfloat16) for _ in range(2))
+
+    def run():
+        sizes = []
+        pack = lambda t: sizes.append(torch.tensor(t.shape)) or t
+        out = _step(moe, list(moe.parameters()), x, dy, hooks=lambda: torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t))
+        return [*out, torch.tensor(sorted(int(n) for s in sizes for n in s))]
+    native, general, taken = _both(monkeypatch, run)
+    _same(native, general)
+    assert "routed_forward" in taken and rows in native[-1].tolist() and rows == ops.plan_length(2 * tokens, 8, 32, 128)
+
+
 def _block(kind, device):
     if kind == "linear":
         return _holder(Linear.Config().build(in_features=256, out_features=384), device)

@@ -184,6 +184,22 @@ def test_traced_block_has_the_shapes_that_its_fake_kernel_gives(no_launches, mon
     assert len(set(storages)) == len(storages)
 
 
+@pytest.mark.parametrize("T,rows", [(192, 512), (704, 1664), (705, 1664), (1984, 4096), (4032, 8192), (6080, 12416)])
+def test_traced_experts_have_the_padded_length_of_the_plan(T, rows):
+    """The fake kernels' layouts at bounds of whole 512s: an additional block, but for powers of two."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    A, D, H, G, k = torch.ops.torchtitan_amd, 128, 256, 4, 2
+    with FakeTensorMode():
+        x, e1, e2 = _bf16(T, D), torch.empty(G, H, D), torch.empty(G, D, H)
+        scores, order, counts = torch.empty(T, k), torch.empty(T * k, dtype=torch.int64), torch.empty(G, dtype=torch.int64)
+        out = A.mx_routed_experts_fwd(x, scores, e1, e2, e1, order, counts, True, 1, False, True, True, True)
+        assert out[6].shape == (2, rows, H)
+        offs, pairs = torch.empty(G, dtype=torch.int32), _bf16(T * k, D)
+        assert A.mx_grouped_ffn_fwd(pairs, e1, e2, e1, offs, 1, True, False, True, True)[4].shape == (2, rows, H)
+        assert A.mx_grouped_mm_fwd(pairs, e1, offs, 1, True)[4].shape == (D, rows)
+
+
 @pytest.mark.parametrize("need_dx,need_dw", [(True, True), (True, False), (False, True)])
 def test_traced_linear_has_the_shapes_that_its_fake_kernel_gives(no_launches, need_dx, need_dw):
     """... also where the weight is frozen, or the input takes no gradient: what is not kept comes to the backward empty."""
@@ -284,11 +300,19 @@ def test_a_forward_without_gradients_casts_each_operand_once(no_launches, monkey
 @pytest.mark.parametrize("pairs", [0, 1, 96, 127, 128, 129, 352, 383, 384, 385, 480, 481, 131072, 12983 * 8])
 @pytest.mark.parametrize("experts", [1, 8, 128])
 def test_padded_layouts_of_whole_blocks_are_no_whole_512s(pairs, experts):
-    """A bound of the aligned groups, at most two blocks beyond it, whose rows of column-wise codes do not lie 4 KB apart."""
+    """A bound of the aligned groups, at most two blocks beyond it, whose rows of column-wise codes do not lie 4 KB apart,
+    unless they are a power of two below 65536 (where the additional block costs more than it gives)."""
     need, got = pairs + 32 * experts, ops.plan_length(pairs, experts, 32, 128)
-    assert got % 128 == 0 and got % 512 and need <= got < need + 256
+    power = got in (512, 1024, 2048, 4096, 8192, 16384, 32768)
+    assert got % 128 == 0 and (got % 512 or power) and need <= got < need + 256
     assert got < need + 128 or (got - 128) % 512 == 0
     assert ops.plan_length(pairs, experts, 32) == need + -need % 32
+
+
+@pytest.mark.parametrize("need,rows", [(384, 384), (385, 512), (512, 512), (1536, 1664), (4000, 4096), (8192, 8192),
+                                       (12288, 12416), (32768, 32768), (65536, 65664), (135168, 135296)])
+def test_padded_lengths_by_the_bound_of_their_groups(need, rows):
+    assert ops.plan_length(need - 32 * 4, 4, 32, 128) == rows
 
 
 def _frozen_readers(path, weights, norm):

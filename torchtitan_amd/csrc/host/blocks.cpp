@@ -473,7 +473,7 @@ py::object routed_forward(const Tensor& x, const Tensor& scores, const Tensor& w
     return py::none();
   const int64_t k = scores.size(1);
   int64_t R = (T * k + alignment * G + multiple - 1) / multiple * multiple;  // ops.plan_length
-  if (multiple == 128 && R % 512 == 0) R += multiple;
+  if (multiple == 128 && R % 512 == 0 && ((R & (R - 1)) != 0 || R >= 65536)) R += multiple;
   hipStream_t st = stream_of(x);
   Unlocked unlocked(std::in_place);
   const Tensor offs = at::empty({G}, x.options().dtype(at::kInt)), src_row = at::empty({R}, x.options().dtype(at::kLong)),

@@ -636,18 +636,28 @@ def route_topk_bwd(logits: torch.Tensor, selected: torch.Tensor, dtop: torch.Ten
 
 def plan_length(pairs, experts: int, alignment: int, length_multiple: int = 1):
     """Rows of the padded layout of `pairs` rows in groups aligned to `alignment`: a static bound, in multiples of
-    `length_multiple`, and one more where its 128s (the persistent kernel's layout) come to whole 512s.  The column-wise
-    codes have rows of this many bytes, and a weight gradient reads 128-byte pieces of 512 of them at a time: where rows
-    lie a whole number of 4 KB apart those fall on few channels of the L2 (128 experts 768 x 2048 and 2048 x 768 over
-    131 072 pairs: 265 and 267 us with 135168 rows = 33 x 4096; with 1024 more 251 and 256, 512 more 240 and 245, 256
-    more 238 and 240, 128 more 235 and 240).  (Without a branch on the length, which may be symbolic.)"""
+    `length_multiple`, and one more where its 128s (the persistent kernel's layout) come to whole 512s, but for the
+    powers of two below 65536.  The column-wise codes have rows of this many bytes, and a weight gradient reads 128-byte
+    pieces of 512 of them at a time: where rows lie a whole number of KB apart those fall on few channels of the L2 (128
+    experts 768 x 2048 and 2048 x 768 over 131 072 pairs: 265 and 267 us with 135168 rows = 33 x 4096; with 1024 more 251
+    and 256, 512 more 240 and 245, 256 more 238 and 240, 128 more 235 and 240).  Rows a power of two apart spread better,
+    and the additional row of tiles opens another round of launches that fill theirs: below 65536 that costs more.
+    All GPU work of the experts forward and backward, 1536 to 135680 rows, five sets of experts (8 to 128 of 1024 x 512 ..
+    2048 x 1024), time without the additional rows over the time with them:
+        odd 512s              0.99 .. 1.03, about 1.00 below 65536      odd 1024s, 2048s   0.99 .. 1.04
+        multiples of 3 x 4096  1.00 .. 1.08 (24576, 32 experts of 2048 x 768: 776 and 731 us)
+        2048                  1.00 .. 1.01                              4096               0.96 .. 1.00
+        8192                  0.94 .. 1.01                              16384              0.96 .. 1.00
+        32768                 0.97 .. 1.02                              65536, 131072      1.00 .. 1.04
+    (Without a branch on the length, which may be symbolic.)"""
     step = max(alignment, length_multiple)
     if step % alignment:
         raise ValueError("length_multiple must be a multiple of the alignment")
     rows = -(-(pairs + alignment * experts) // step) * step
     if length_multiple != WHOLE_BLOCK:
         return rows
-    return rows + step * ((3 - rows // step % 4) // 3)
+    whole_512s = (3 - rows // step % 4) // 3
+    return rows + step * whole_512s * torch.sym_min(1, (rows & (rows - 1)) + rows // 65536)
 
 
 def route_fill(selected: torch.Tensor, scores: torch.Tensor, counts: torch.Tensor, block_counts: torch.Tensor,

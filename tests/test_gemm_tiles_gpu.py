@@ -305,3 +305,51 @@ def test_gate_in_the_product_gives_the_bits_of_the_gate_behind_it(device, M, N, 
     wrong = (got.codes != want.codes).nonzero().tolist()
     assert not wrong, (len(wrong), wrong[:8])
     assert torch.equal(*(ops.scale_unlayout(q.scales.contiguous(), M, q.k // 32) for q in (got, want)))
+
+
+@pytest.mark.parametrize("M,N,K", [(700, 1000, 128), (1025, 520, 256), (700, 1000, 640), (2048, 776, 384), (520, 2056, 2016)])
+@pytest.mark.parametrize("mode", ["floor", "rceil"])
+def test_gate_in_the_product_over_several_tiles_a_workgroup(device, hooks, M, N, K, mode):
+    """Eight workgroups take three tiles and more each, the last rows and columns ragged, over one, two and an odd number of
+    blocks: the next tile's copies are in flight while a tile is gated, and the waves change between both weights."""
+    rng = np.random.default_rng(M + N + K)
+    x, w, w2 = (bf16_from_bits(randn_bits(rng, (rows, K), std=s, outliers=1e-3), device)
+                for rows, s in ((M, 1.0), (N, 0.05), (N, 0.5)))
+    a, b, b2 = (ops.to_operands(t, mode, cols=False, pitch_pad=128)[0] for t in (x, w, w2))
+    h = ops.mx_gemm_nt_shared_a(a, b, b2)
+    want = ops.swiglu_to_operands(h[0], h[1], mode, False, 128)[0]
+    for grid in (8, 16):
+        hooks.mx_debug_set_grid(grid)
+        assert -(-M // 256) * -(-N // 128) > grid
+        got = ops.mx_gemm_nt_swiglu(a, b, b2, mode, planned=True)
+        wrong = (got.codes != want.codes).nonzero().tolist()
+        assert not wrong, (grid, len(wrong), wrong[:8])
+        assert torch.equal(*(ops.scale_unlayout(q.scales.contiguous(), M, q.k // 32) for q in (got, want))), grid
+
+
+@pytest.mark.parametrize("norm", [False, True])
+def test_feed_forward_without_gradients_gates_in_the_product(device, monkeypatch, norm):
+    """A block of two rounds of tiles takes the gated launch by itself, behind a norm or not, and gives the bits of the
+    two launches."""
+    from torchtitan_amd import mx_blocks
+    from torchtitan_amd.mx_tensor import MXFP8Config, MXFP8TrainingWeight
+
+    M, D, H = 4096, 2048, 6144
+    g = torch.Generator(device=device).manual_seed(3)
+    rn = lambda *shape, std=1.0: (torch.randn(shape, generator=g, device=device) * std).to(torch.bfloat16)
+    cfg = MXFP8Config(fuse_rmsnorm_cast=norm)
+    x, n = rn(M, D), (rn(D) * 0.1 + 1).to(torch.bfloat16)
+    w1, w2, w3 = (MXFP8TrainingWeight(rn(*shape, std=0.02), cfg) for shape in ((H, D), (D, H), (H, D)))
+    run = (lambda: mx_blocks.mx_norm_feed_forward(x, n, 1e-5, w1, w2, w3)) if norm else (
+        lambda: mx_blocks.mx_feed_forward(x, w1, w2, w3))
+    calls, call = [], ops._call
+    assert _lib.load().mx_gemm_nt_swiglu_planned(M, H, D)
+    with torch.no_grad():
+        with monkeypatch.context() as m:
+            m.setattr(ops, "_call", lambda name, *args: calls.append(name) or call(name, *args))
+            got = run()
+        assert calls.count("mx_gemm_nt_swiglu_ld") == 1 and "mx_gemm_nt_shared_a_ld" not in calls
+        with monkeypatch.context() as m:
+            m.setattr(ops, "mx_gemm_nt_swiglu", lambda *args: None)
+            want = run()
+    assert torch.equal(got, want) and bool(torch.isfinite(got).all())

@@ -296,8 +296,8 @@ __global__ __launch_bounds__(256) void cast_dim0_dim1_kernel(
 //                transposed tile, which leaves as 32*WAVES-byte rows.
 // All scale bytes of the tile are staged in LDS in their final order and leave as dwords
 // (whole 256-byte groups in MFMA order, padding entries included as zeros).
-// KR: rows that a lane holds, 8 as above; with 4 or 2 a wave owns 4 KR rows, the tile has as many more
-// waves, and those of a 32-row block exchange their column maxima through LDS (see with_lane_rows).
+// KR: rows that a lane holds, 8 as above; with 4, or 2 of the row-wise form alone, a wave owns 4 KR rows, the tile has
+// as many more waves, and those of a 32-row block exchange their column maxima through LDS (see with_lane_rows).
 // ------------------------------------------------------------------------------------
 __device__ __forceinline__ uint32_t lane_xor(uint32_t v, int lane, int mask) {
   return (uint32_t)__builtin_amdgcn_ds_bpermute((lane ^ mask) << 2, (int)v);
@@ -325,8 +325,7 @@ __device__ __forceinline__ uint32_t cvt2_finite(float lo, float hi, uint32_t old
   return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(lo, hi, (int)old, HIGH);
 }
 
-
-// Quantize one lane's 8x8 patch.  FINITE = no Inf / NaN anywhere in the wave's patches: the
+// Quantize one lane's KR x 8 patch.  FINITE = no Inf / NaN anywhere in the wave's patches: the
 // straight-line path; otherwise the general path with per-block NaN handling and clamps.
 template <int MODE, int ORDER, bool ROW, bool COL, int WAVES, bool FINITE, int KR>
 __device__ __forceinline__ void quantize_patch(u32x4 (&v)[KR], const uint32_t (&mr)[KR],
@@ -374,13 +373,14 @@ __device__ __forceinline__ void quantize_patch(u32x4 (&v)[KR], const uint32_t (&
       }
     }
   }
-  if (COL) {
+  if constexpr (COL) {
+    static_assert(KR >= 4, "a column's codes leave as whole dwords (with_lane_rows)");
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const uint32_t amax = (j & 1) ? (mc[j >> 1] >> 16) : (mc[j >> 1] & 0xFFFFu);
       uint32_t sb;
       float mu;
-      uint32_t d[(KR + 3) / 4];  // the column's codes, row by row
+      uint32_t d[KR / 4];  // the column's codes, row by row
       if (FINITE) {
         finite_scale<MODE>(amax, sb, mu);
         float f[KR];
@@ -390,8 +390,7 @@ __device__ __forceinline__ void quantize_patch(u32x4 (&v)[KR], const uint32_t (&
 #pragma unroll
         for (int k = 0; k < KR; k += 4) {
           const uint32_t half = cvt2_finite<MODE, false>(f[k], f[k + 1], 0);
-          if constexpr (KR >= 4) d[k / 4] = cvt2_finite<MODE, true>(f[k + 2], f[k + 3], half);
-          else d[k / 4] = half;
+          d[k / 4] = cvt2_finite<MODE, true>(f[k + 2], f[k + 3], half);
         }
       } else {
         sb = scale_byte<MODE>(amax);
@@ -407,21 +406,20 @@ __device__ __forceinline__ void quantize_patch(u32x4 (&v)[KR], const uint32_t (&
 #pragma unroll
           for (int k = 0; k < KR; k += 4) {
             d[k / 4] = cvt2f<false>(f[k], f[k + 1], 0);
-            if constexpr (KR >= 4) d[k / 4] = cvt2f<true>(f[k + 2], f[k + 3], d[k / 4]);
+            d[k / 4] = cvt2f<true>(f[k + 2], f[k + 3], d[k / 4]);
           }
         } else {
 #pragma unroll
           for (int k = 0; k < KR; k += 4) {
             d[k / 4] = nan_block_code(e[k]) | (nan_block_code(e[k + 1]) << 8);
-            if constexpr (KR >= 4) d[k / 4] |= (nan_block_code(e[k + 2]) << 16) | (nan_block_code(e[k + 3]) << 24);
+            d[k / 4] |= (nan_block_code(e[k + 2]) << 16) | (nan_block_code(e[k + 3]) << 24);
           }
         }
       }
       const int cl = 8 * q + j;
       uint8_t* const to = lds_codes + cl * PITCH + KR * (4 * wave + g);
       if constexpr (KR == 8) *reinterpret_cast<u32x2*>(to) = u32x2{d[0], d[1]};
-      else if constexpr (KR == 4) *reinterpret_cast<uint32_t*>(to) = d[0];
-      else *reinterpret_cast<uint16_t*>(to) = (uint16_t)d[0];
+      else *reinterpret_cast<uint32_t*>(to) = d[0];
       if (g == 0 && (KR == 8 || wave % (8 / KR) == 0)) {
         if (ORDER == MX_SCALES_MFMA)
           lds_st[((band >> 1) << 8) + ((((band & 1) << 5) + (cl & 31)) << 2) + (cl >> 5)] =
@@ -481,7 +479,8 @@ struct TileWalk {
 // quotient.  Scaled and guarded as in silu_f32.  The kernel is bound by vector instructions: without selects
 // around the exponential, the scaling and the remainder 2048 x 1408 .. 5003 x 6144 take 2 to 5 % less (71.3 -> 67.7 us).
 //
-// exp(-a) as 2^n 2^f, f the rounded rest of -a log2(e) in two parts: within a step of the hardware's exponential (its
+// exp(-a) as 2^n 2^f by Cody and Waite's reduction (Software Manual for the Elementary Functions, 1980): f what is left of
+// -a log2(e), the constant in two parts, so that its rounding does not enter f.  Within a step of the hardware's exponential (its
 // argument unreduced moves a few results in a million by one bf16 step).  The clamp keeps every step finite; NaN
 // comes out as some number, and from the caller's factor a as NaN again.
 __device__ __forceinline__ float exp_neg(float a) {
@@ -1000,8 +999,8 @@ using namespace mx;
   } while (0)
 
 // Calls `launch` with the rows that a lane holds (8, 4 or 2 of a tile's 128 x 128 values over 4, 8 or 16 waves), by the
-// tiles of the launch.  A gate is a chain of some hundred instructions a value: with a tile or two per CU its SIMDs
-// wait for one wave's chain, which more and shorter waves fill.  us, 8 rows and fewer (bf16, after other kernels):
+// tiles that the launch has for a CU.  A gate is a chain of some hundred instructions a value: with a tile or two per CU its SIMDs
+// wait for one wave's chain, which more and shorter waves fill.  us on 256 CUs, 8 rows and fewer (bf16, after other kernels):
 //   tiles          both directions, forward   backward       row-wise alone
 //   32             9.0   7.8                  15.0   13.0     7.7   5.5
 //   512           15.8  14.0                  26.4   23.7    13.6  10.1
@@ -1014,7 +1013,9 @@ using namespace mx;
 template <int GATE, bool COL, class F>
 static inline void with_lane_rows(int64_t tiles, F launch) {
   if constexpr (GATE == 1 || GATE == 2) {
-    if (tiles <= (!COL ? 2048 : GATE == 1 ? 768 : 512)) return launch(std::integral_constant<int, COL ? 4 : 2>{});
+    const int cus = current_device_cus();
+    const int64_t per_cu = !COL ? 8 : GATE == 1 ? 3 : 2;
+    if (tiles <= per_cu * (cus ? cus : 256)) return launch(std::integral_constant<int, COL ? 4 : 2>{});
   }
   launch(std::integral_constant<int, 8>{});
 }

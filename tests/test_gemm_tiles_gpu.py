@@ -327,6 +327,16 @@ def test_gate_in_the_product_over_several_tiles_a_workgroup(device, hooks, M, N,
         assert torch.equal(*(ops.scale_unlayout(q.scales.contiguous(), M, q.k // 32) for q in (got, want))), grid
 
 
+@pytest.mark.parametrize("M,N,K,gated", [(4096, 6144, 2048, 1), (3001, 8192, 1024, 1), (512, 14336, 4096, 1), (1500, 4992, 2048, 1),
+                                         (2270, 4096, 1536, 0), (1409, 6080, 768, 0), (3533, 4736, 1920, 0),
+                                         (2048, 5632, 2048, 0), (512, 8192, 3072, 0)])
+def test_gate_in_the_product_is_chosen_where_it_is_ahead(device, M, N, K, gated):
+    """Full rounds of tiles, not a last round of few (measured: 7 to 15 % behind the two launches) nor half of the CUs."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the line is for 256 CUs")
+    assert _lib.load().mx_gemm_nt_swiglu_planned(M, N, K) == gated
+
+
 @pytest.mark.parametrize("norm", [False, True])
 def test_feed_forward_without_gradients_gates_in_the_product(device, monkeypatch, norm):
     """A block of two rounds of tiles takes the gated launch by itself, behind a norm or not, and gives the bits of the

@@ -281,9 +281,9 @@ __device__ __forceinline__ constexpr uint32_t wave_col(uint32_t wn, int n) {
 // as the row-wise MXFP8 operand of the next product: of a forward without gradients nothing else is read again.  A
 // tile is 256 rows of 128 columns of G: a wave's sub-tiles 0 .. 3 come from B, 4 .. 7 from the same rows of B2, so that a lane
 // holds both factors of its values; waves 0 and 2 copy B's rows into the ring, 1 and 3 those of B2.  What the
-// gate adds to the epilogue (8 K vector instructions a wave, about 5 us a round, matrix cores idle) is less than the
-// 8 bytes a value that are not written and read again, and the launch: 512 x 14336, K 4096 59.9 us in two launches, 53.0 in
-// this one; 1024 x 14336 113 and 101 (plan_gated for where it is not).
+// gate adds to the epilogue (8 K vector instructions a wave, matrix cores idle; 5 to 6.7 us a round over two products on the
+// same tiles with their stores) is less than the 8 bytes a value that are not written and read again, and the launch: 512 x
+// 14336, K 4096 59.7 us in two launches, 55.2 in this one; 1024 x 14336 108 and 102 (plan_gated for where it is not).
 template <int MODE, bool PROF, bool PAIR = false, int TA = 4, int TB = 4, bool OUT32 = false, bool GATE = false>
 __global__ __launch_bounds__(256, 1) void gemm_nt32_kernel(Gemm32Args p) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
@@ -1828,10 +1828,13 @@ int launch_gemm_nt32_pair(const uint8_t* a_codes, const uint8_t* a_scales, const
 }
 
 // Whether the gated product of [M, K] with two weights of N rows leaves its product as codes: where that is predicted to be
-// done before the two products and the cast of their gate.  Fitted to 68 shapes of 129..4096 rows, 1024..14336 columns and
-// K 512..5120 (none got slower, none left more than 4 % behind): 4 us a round for the gate against a launch and its bytes.
-// Full rounds win (3001 x 8192, K 1024 77.9 and 66.3 us; 4096 x 6144, K 2048 107 and 95.5; 1500 x 4992, K 2016 37.5 and
-// 33.0), tiles that leave half of the CUs idle lose to the smaller ones of the two launches (512 x 8192, K 3072 31.6 and 37.4).
+// done before the two products and the cast of their gate.  The gate costs 6 us a round, also a last one of few tiles,
+// which then does not pay: 288 tiles of 12 blocks (2270 x 4096, K 1536) 45 us in two launches and 50 gated, 352 of 16 (2048 x 5632,
+// K 2048) 58 and 63, 518 of 15 (3533 x 4736, K 1920) 79 and 86.  Full rounds win (3001 x 8192, K 1024 75 and 65 us; 4096 x 6144,
+// K 2048 105 and 96; 1500 x 4992, K 2048 38 and 35), tiles that leave half of the CUs idle lose to the smaller ones of the
+// two launches (512 x 8192, K 3072 34 and 42).  Fitted to 228 shapes of 129..4600 rows, 1024..14336 columns and K 512..5400, on
+// operands from the cache and from memory: of the 107 that it chooses none is slower, and the choice takes 0.1 % more than
+// the better of both each time.  (4 us a round chose 134 of them, 19 slower by 3 to 13 %.)
 bool plan_gated(int64_t M, int64_t N, int64_t K) {
   const int64_t grid = persistent_grid(), blocks = K / kKB;
   if (grid == 0) return false;
@@ -1840,8 +1843,8 @@ bool plan_gated(int64_t M, int64_t N, int64_t K) {
   double us = tiles_us(*t, 2 * tile_count(*t, M, N), blocks, grid) + 2.0;
   better_ring(M, N, blocks, 2, grid, us);
   const int64_t tiles = ((M + 255) / 256) * ((N + 127) / 128);
-  const double gated = tiles_us(kDenseTiles[0], tiles, blocks, grid) + 1.0 + 4.0 * ((tiles + grid - 1) / grid);
-  return gated < us + M * N / 0.75e6;
+  const double gated = tiles_us(kDenseTiles[0], tiles, blocks, grid) + 1.0 + 6.0 * ((tiles + grid - 1) / grid);
+  return gated < us + 2.0 + M * N / 1e6;
 }
 int launch_gemm_nt32_gated(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes, const uint8_t* b_scales,
                            const uint8_t* b2_codes, const uint8_t* b2_scales, uint8_t* codes, uint8_t* scales, int64_t M,

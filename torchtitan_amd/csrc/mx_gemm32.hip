@@ -1560,8 +1560,11 @@ GemmPlan plan_dense(int64_t M, int64_t N, int64_t K, bool may_split) {
       }
     }
   }
-  // Few tiles, not split: 64-wide ones (up to 64 rows have a kernel of their own).  Where a split is to be had it is as fast
-  // or faster: 256 x 4096, K 6144 17.7 us and 17.6 in one chain; 512 x 512, K 10240 18.7 and 25.2.
+  // Few tiles, not split: 64-wide ones (up to 64 rows have a kernel of their own).  A split is not compared with them.  Of
+  // 151 shapes that are split (72..1024 rows, 512..4096 columns) the better 64-wide tile in one chain takes, over the split's
+  // time, 0.72 to 0.89 with 34 blocks (1024 x 1024 14.8 and 20.6 us), 0.81 to 1.07 with 48, 0.89 to 1.30 with 64, 0.97 to 1.49
+  // with 80 and 1.10 to 1.57 with 112 (256 x 512 33.5 and 22.3).  Sums of two products, which plan_pair splits (83 shapes): 0.91 to
+  // 1.33 with 2 x 32 blocks, 1.05 to 1.52 with 2 x 48, 1.37 to 2.18 with 2 x 112.
   if (best.slices == 1 && !debug_tile && M > 64)
     if (const RingTile* r = better_ring(M, N, blocks, 1, grid, best_us)) best = {r->ta, r->tb, 1};
   return best;

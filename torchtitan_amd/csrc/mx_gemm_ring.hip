@@ -5,9 +5,10 @@
 //
 // A product of some hundred rows has too few 256-wide tiles for the CUs, and each of them waits for its operands: a block
 // takes 0.5 to 0.75 us where its MFMAs take 0.2 to 0.4.  Here the tiles are small, so that more CUs have one, and a ring
-// of eight (64 x 64) or six (128 x 64) blocks hides the latency: a block takes 0.24 and 0.36 us, bound by the fragment
-// reads (256 and 375 cycles of a CU's LDS) and their latency, with many CUs by what they get out of the L2.  us on the
-// GPU, before and now: 256 x 1024, K 2048 14.0 and 8.1; 512 x 1024, K 1024 9.7 and 6.8; 200 x 2560, K 4096 23.4 and 13.1;
+// of eight (64 x 64) or six (128 x 64) blocks hides the latency: a block takes 0.24 and 0.35 us on few CUs, 0.28 and 0.44
+// with a tile on each.  That is about 580 and 840 cycles, of which the fragment reads fill 256 and 384 of the LDS's (32 and 48 KB
+// at 128 B): what bounds it is the chain of a block, barrier, reads and their latency, MFMAs and waits, which nothing
+// else on the CU overlaps, and with many CUs what they get out of the L2.  us on the GPU, before and now: 256 x 1024, K 2048 14.0 and 8.1; 512 x 1024, K 1024 9.7 and 6.8; 200 x 2560, K 4096 23.4 and 13.1;
 // 768 x 1024, K 4096 23.4 and 13.4; 128 x 10240, K 3072 19.7 and 14.7.  (128 x 128 tiles with four blocks gain nothing over
 // the persistent kernel anywhere: 14.2 us in the first of these.)
 //

@@ -477,7 +477,7 @@ struct TileWalk {
 // with the float32 formula of the unfused silu backward op.  silu(a) = a / (1 + exp(-a)) shares
 // the denominator: a * s corrected by one Newton step on the remainder is the correctly rounded
 // quotient.  Scaled and guarded as in silu_f32.  The kernel is bound by vector instructions: without selects
-// around the exponential, the scaling and the remainder 2048 x 1408 .. 5003 x 6144 take 2 to 5 % less (71.3 -> 67.7 us).
+// around the exponential, the scaling and the remainder 2048 x 1408 .. 5003 x 6144 take 2 to 5 % less (71.3 -> 67.7 us, alone).
 //
 // exp(-a) as 2^n 2^f by Cody and Waite's reduction (Software Manual for the Elementary Functions, 1980): f what is left of
 // -a log2(e), the constant in two parts, so that its rounding does not enter f.  Within a step of the hardware's exponential (its

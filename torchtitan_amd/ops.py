@@ -656,8 +656,8 @@ def plan_length(pairs, experts: int, alignment: int, length_multiple: int = 1):
     rows = -(-(pairs + alignment * experts) // step) * step
     if length_multiple != WHOLE_BLOCK:
         return rows
-    whole_512s = (3 - rows // step % 4) // 3
-    return rows + step * whole_512s * torch.sym_min(1, (rows & (rows - 1)) + rows // 65536)
+    whole_512s, least = (3 - rows // step % 4) // 3, min if type(rows) is int else torch.sym_min
+    return rows + step * whole_512s * least(1, (rows & (rows - 1)) + rows // 65536)
 
 
 def route_fill(selected: torch.Tensor, scores: torch.Tensor, counts: torch.Tensor, block_counts: torch.Tensor,
